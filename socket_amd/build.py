@@ -20,7 +20,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libsocket_hip.so")
 CORE_PATH = os.path.join(HERE, "libsocket_core.so")
-CORE_SOURCES = ["common.hip", "attend.hip", "decode_ops.hip", "rows.hip", "chunk_attend.hip", "latent.hip",
+CORE_SOURCES = ["common.hip", "attend.hip", "decode_ops.hip", "rows.hip", "chunk_attend.hip", "prompt_attend.hip", "latent.hip",
                 "recurrence.hip"]
 SOURCES = ["score.hip", "collide.hip", "topk.hip", "hash.hip", "softhash.hip", "block_sparse.hip"]
 ARCH = "gfx950"
@@ -38,6 +38,7 @@ FLAGS = [
 FILE_FLAGS = {
     "block_sparse.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "attend.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],     # the MFMA dense flash-decode, for the same reason
+    "prompt_attend.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "chunk_attend.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "latent.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "recurrence.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

@@ -11,6 +11,10 @@
 // may be shared by all heads, and the output may be gated.
 #include "elem.h"
 
+// prompt_attend.hip
+bool prompt_attend_fits(const socket_chunk_attention& a);
+int prompt_attend_launch(const socket_chunk_attention& a, bool weights16, hipStream_t s);
+
 namespace {
 
 // Work items of a token: V elements of the first rotated half of a head with the V that
@@ -484,7 +488,7 @@ __global__ __launch_bounds__(256, NK == 32 ? 2 : 1) void chunk_attend_mma_kernel
 }
 
 bool mma_fits(const socket_chunk_attention& a) {
-  if (a.force_simple || a.pos || a.dtype != SOCKET_BF16 || a.D % 8 != 0 || a.D + a.D2 > 256) return false;
+  if (a.force_simple || a.pos || a.D % 8 != 0 || a.D + a.D2 > 256) return false;
   if (a.k2 ? a.Dv > 256 || a.softcap > 0.f : a.Dv != a.D || a.gate) return false;
   if (a.Dv % 8 != 0 || a.D2 % 8 != 0) return false;
   const int64_t strides[] = {a.q_stride_b, a.q_stride_t, a.q_stride_h, a.k_stride_b, a.k_stride_t, a.k_stride_g,
@@ -580,21 +584,41 @@ extern "C" int socket_chunk_ring_store(const void* k, int64_t k_sb, int64_t k_st
   return SOCKET_OK;
 }
 
-extern "C" int socket_chunk_attend(const socket_chunk_attention* args, void* stream) {
-  SOCKET_REQUIRE(args && args->q && args->out, SOCKET_ERR_NULL);
-  socket_chunk_attention a = *args;
-  if (a.Dv == 0) a.Dv = a.D;
+namespace {
+int check_attention(const socket_chunk_attention& a) {
   SOCKET_REQUIRE((a.k_ring && a.v_ring) || (!a.pos && a.k_from == 0), SOCKET_ERR_NULL);
   SOCKET_REQUIRE(a.pos || (a.k_from >= 0 && a.k_from <= a.pos0), SOCKET_ERR_SHAPE);
   SOCKET_REQUIRE(a.k2 ? (a.D2 > 0 && !a.pos && a.k_from == 0) : a.D2 == 0, SOCKET_ERR_SHAPE);
   SOCKET_REQUIRE(a.Dv > 0 && (a.D + a.D2 + 64) * 4 * kSimpleWaves <= 48 * 1024, SOCKET_ERR_UNSUPPORTED);
   SOCKET_REQUIRE(a.pos || (a.k_new && a.v_new), SOCKET_ERR_NULL);
-  SOCKET_REQUIRE(a.dtype == SOCKET_F32 || a.dtype == SOCKET_BF16, SOCKET_ERR_UNSUPPORTED);
   SOCKET_REQUIRE(a.B > 0 && a.B <= 65535 && a.T > 0 && a.H > 0 && a.G > 0 && a.H % a.G == 0, SOCKET_ERR_SHAPE);
   SOCKET_REQUIRE(a.chunk > 0 && (!a.pos || a.T == 1) && a.pos0 >= 0, SOCKET_ERR_SHAPE);
   SOCKET_REQUIRE(a.D > 0 && a.Dv <= 64 * kSimpleDims, SOCKET_ERR_UNSUPPORTED);
+  return SOCKET_OK;
+}
+}  // namespace
+
+extern "C" int socket_prompt_attention(const socket_chunk_attention* args, int weights16, void* stream) {
+  SOCKET_REQUIRE(args && args->q && args->out, SOCKET_ERR_NULL);
+  socket_chunk_attention a = *args;
+  if (a.Dv == 0) a.Dv = a.D;
+  const int st = check_attention(a);
+  if (st != SOCKET_OK) return st;
+  SOCKET_REQUIRE(a.dtype == SOCKET_F16 || a.dtype == SOCKET_BF16, SOCKET_ERR_UNSUPPORTED);
+  SOCKET_REQUIRE(mma_fits(a) && prompt_attend_fits(a), SOCKET_ERR_UNSUPPORTED);
+  return prompt_attend_launch(a, weights16 != 0, (hipStream_t)stream);
+}
+
+extern "C" int socket_chunk_attend(const socket_chunk_attention* args, void* stream) {
+  SOCKET_REQUIRE(args && args->q && args->out, SOCKET_ERR_NULL);
+  socket_chunk_attention a = *args;
+  if (a.Dv == 0) a.Dv = a.D;
+  const int st = check_attention(a);
+  if (st != SOCKET_OK) return st;
+  SOCKET_REQUIRE(a.dtype == SOCKET_F32 || a.dtype == SOCKET_BF16, SOCKET_ERR_UNSUPPORTED);
   hipStream_t s = (hipStream_t)stream;
-  if (mma_fits(a)) {
+  if (a.dtype == SOCKET_BF16 && mma_fits(a)) {
+    if (prompt_attend_fits(a)) return prompt_attend_launch(a, false, s);
     if (a.k2) {
       const int dq = a.D + a.D2;
       if (dq <= 64 && a.Dv <= 64) return launch_mma<64, 64, 2, true>(a, s);
