@@ -118,7 +118,7 @@ CORE_SIGNATURES = {
     "socket_rope_half_rows": (_I, [POINTER(RopeHalf), _P]),
     "socket_chunk_ring_store": (_I, [_P, _L, _L, _L, _P, _L, _L, _L, _P, _P, _L, _L, _L, _I, _I, _I, _I, _I, _I, _L, _P]),
     "socket_chunk_attend": (_I, [POINTER(ChunkAttention), _P]),
-    "socket_prompt_attention": (_I, [POINTER(ChunkAttention), _I, _P]),
+    "socket_prompt_attention": (_I, [POINTER(ChunkAttention), _P, _I, _P]),
     "socket_dense_decode_capped_workspace_bytes": (_Z, [_I, _I, _I]),
     "socket_dense_decode_capped": (_I, [_P, _P, _P, _I] + [_L] * 8 + [_P, _P, _L, _L, _P, _Z, _I, _I, _I, _I, _I, _F, _F, _P]),
     "socket_recurrence_step": (_I, [POINTER(Recurrence), _P]),

@@ -13,7 +13,7 @@
 
 // prompt_attend.hip
 bool prompt_attend_fits(const socket_chunk_attention& a);
-int prompt_attend_launch(const socket_chunk_attention& a, bool weights16, hipStream_t s);
+int prompt_attend_launch(const socket_chunk_attention& a, const int64_t* positions, bool weights16, hipStream_t s);
 
 namespace {
 
@@ -598,7 +598,7 @@ int check_attention(const socket_chunk_attention& a) {
 }
 }  // namespace
 
-extern "C" int socket_prompt_attention(const socket_chunk_attention* args, int weights16, void* stream) {
+extern "C" int socket_prompt_attention(const socket_chunk_attention* args, const int64_t* positions, int weights16, void* stream) {
   SOCKET_REQUIRE(args && args->q && args->out, SOCKET_ERR_NULL);
   socket_chunk_attention a = *args;
   if (a.Dv == 0) a.Dv = a.D;
@@ -606,7 +606,9 @@ extern "C" int socket_prompt_attention(const socket_chunk_attention* args, int w
   if (st != SOCKET_OK) return st;
   SOCKET_REQUIRE(a.dtype == SOCKET_F16 || a.dtype == SOCKET_BF16, SOCKET_ERR_UNSUPPORTED);
   SOCKET_REQUIRE(mma_fits(a) && prompt_attend_fits(a), SOCKET_ERR_UNSUPPORTED);
-  return prompt_attend_launch(a, weights16 != 0, (hipStream_t)stream);
+  // (with positions of its own a token may see any key: one endless chunk, all keys in k_new)
+  SOCKET_REQUIRE(!positions || (a.chunk == INT32_MAX && a.k_from == 0 && a.softcap == 0.f && !a.k2), SOCKET_ERR_UNSUPPORTED);
+  return prompt_attend_launch(a, positions, weights16 != 0, (hipStream_t)stream);
 }
 
 extern "C" int socket_chunk_attend(const socket_chunk_attention* args, void* stream) {
@@ -618,7 +620,7 @@ extern "C" int socket_chunk_attend(const socket_chunk_attention* args, void* str
   SOCKET_REQUIRE(a.dtype == SOCKET_F32 || a.dtype == SOCKET_BF16, SOCKET_ERR_UNSUPPORTED);
   hipStream_t s = (hipStream_t)stream;
   if (a.dtype == SOCKET_BF16 && mma_fits(a)) {
-    if (prompt_attend_fits(a)) return prompt_attend_launch(a, false, s);
+    if (prompt_attend_fits(a)) return prompt_attend_launch(a, nullptr, false, s);
     if (a.k2) {
       const int dq = a.D + a.D2;
       if (dq <= 64 && a.Dv <= 64) return launch_mma<64, 64, 2, true>(a, s);

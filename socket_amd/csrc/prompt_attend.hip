@@ -120,9 +120,10 @@ __device__ __forceinline__ void pa_copy_tile(const char* first, int64_t stride, 
 // D: key dims, D2: dims of a second key segment that all heads share (with it the output may be gated),
 // DV: value dims.  SPLIT: weights enter the second product as a sum of two 16-bit numbers.  CAPPED:
 // scores pass softcap tanh(s / softcap), which bounds them, so that exp(score) needs no running
-// maximum: p = exp(cap - 2 cap / (exp(2 s / cap) + 1)).
-template <class DT, int D, int D2, int DV, bool SPLIT, bool CAPPED>
-__global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_chunk_attention a) {
+// maximum: p = exp(cap - 2 cap / (exp(2 s / cap) + 1)).  POS: token t sees the keys up to positions[t]
+// instead of pos0 + t (one endless chunk, a.k_from = 0).
+template <class DT, int D, int D2, int DV, bool SPLIT, bool CAPPED, bool POS>
+__global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_chunk_attention a, const int64_t* positions) {
   constexpr int CK = D / 8, CK2 = D2 / 8, CV = DV / 8;            // 16-byte pieces per row
   constexpr int KS = D / 16, KS2 = D2 / 16, DB = DV / 32;
   constexpr int kK2 = kPaKeys * D * 2, kV = kK2 + kPaKeys * D2 * 2, kStage = kV + kPaKeys * DV * 2;   // places in a stage
@@ -139,11 +140,11 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
   const int col = lane & 31, half = lane >> 5;
 
   // (positions as 32-bit offsets from the first key of the tile's first chunk)
-  const int64_t base = (a.pos0 + r0 / Gq) / a.chunk * a.chunk;
-  const int end = (int)(a.pos0 + min(r0 + kPaRows - 1, R - 1) / Gq - base) + 1;   // keys [0, end)
+  const int64_t base = POS ? 0 : (a.pos0 + r0 / Gq) / a.chunk * a.chunk;
   const int64_t wr0 = min(r0 + wave * 32, R - 1), wr1 = min(r0 + wave * 32 + 31, R - 1);
-  const int iw0 = (int)(a.pos0 + wr0 / Gq - base), iw1 = (int)(a.pos0 + wr1 / Gq - base);
-  const int cw0 = iw0 / a.chunk * a.chunk, cw1 = iw1 / a.chunk * a.chunk;         // (base is a chunk's start)
+  int end = (int)(a.pos0 + min(r0 + kPaRows - 1, R - 1) / Gq - base) + 1;   // keys [0, end)
+  int iw0 = (int)(a.pos0 + wr0 / Gq - base), iw1 = (int)(a.pos0 + wr1 / Gq - base);
+  const int cw0 = iw0 / a.chunk * a.chunk, cw1 = iw1 / a.chunk * a.chunk;   // (base is a chunk's start)
   const bool wave_live = r0 + wave * 32 < R;
 
   const char* k_new = (const char*)a.k_new + (b * a.k_stride_b + g * a.k_stride_g) * 2;
@@ -160,7 +161,8 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
     const bool live = r < R;
     const int64_t t = (live ? r : 0) / Gq;
     row_i = live ? (int)(a.pos0 + t - base) : -1;
-    row_c = live ? row_i / a.chunk * a.chunk : 0;
+    if (POS && live) row_i = (int)max((int64_t)-1, min(positions[t], a.pos0 + a.T - 1));
+    row_c = live && !POS ? row_i / a.chunk * a.chunk : 0;
     const uint16_t* q = (const uint16_t*)a.q + b * a.q_stride_b + t * a.q_stride_t + (g * Gq + (live ? r : 0) % Gq) * a.q_stride_h;
 #pragma unroll
     for (int ks = 0; ks < KS + KS2; ++ks) qf[ks] = live ? *reinterpret_cast<const uint4*>(q + 16 * ks + 8 * half) : make_uint4(0, 0, 0, 0);
@@ -169,6 +171,23 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
   // do not include the copies and would drain them on every trip)
 #pragma unroll
   for (int ks = 0; ks < KS + KS2; ++ks) asm volatile("" ::"v"(qf[ks].x), "v"(qf[ks].y), "v"(qf[ks].z), "v"(qf[ks].w));
+
+  if constexpr (POS) {      // what the tile's and the wave's rows see, from the positions themselves
+    int* ends = reinterpret_cast<int*>(pa_lds);
+    int lo = row_i < 0 && r >= R ? INT32_MAX : row_i, hi = row_i;
+#pragma unroll
+    for (int step = 32; step > 0; step >>= 1) {
+      lo = min(lo, __shfl_xor(lo, step, 64));
+      hi = max(hi, __shfl_xor(hi, step, 64));
+    }
+    iw0 = __builtin_amdgcn_readfirstlane(lo);
+    iw1 = __builtin_amdgcn_readfirstlane(hi);
+    if (lane == 0) ends[wave] = hi + 1;
+    __syncthreads();
+    end = __builtin_amdgcn_readfirstlane(max(max(ends[0], ends[1]), max(ends[2], ends[3])));
+    __syncthreads();        // (the places are the first tile's)
+  }
+  static_assert(kPaWaves == 4, "ends");
 
   pa_f32x16 o[DB];
 #pragma unroll
@@ -202,7 +221,7 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
   const int k_swz = pa_swizzle<CK>(col);
   const int v_key = 4 * half + ((lane >> 2) & 3), v_piece = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1), v_byte = (lane & 1) * 8;
 
-  copy_keys(0, 0);
+  if (end > 0) copy_keys(0, 0);
   int stage = 0;
   for (int j0 = 0; j0 < end; j0 += kPaKeys, stage ^= 1) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -319,7 +338,7 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
 
   l += lane_xor32(l);
   if (r >= R) return;
-  const float inv = 1.f / l;
+  const float inv = l > 0.f || l != l ? 1.f / l : 0.f;     // (a row that sees nothing is zero)
   const int64_t t = r / Gq, h = g * Gq + r % Gq;
   uint16_t* out = (uint16_t*)a.out + (((int64_t)b * a.T + t) * a.H + h) * DV;
   const int64_t g0 = b * a.gate_stride_b + t * a.gate_stride_t + h * DV;
@@ -341,38 +360,41 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
     }
 }
 
-template <class DT, int D, int D2, int DV, bool SPLIT, bool CAPPED>
-int pa_launch(const socket_chunk_attention& a, hipStream_t s) {
+template <class DT, int D, int D2, int DV, bool SPLIT, bool CAPPED, bool POS = false>
+int pa_launch(const socket_chunk_attention& a, const int64_t* positions, hipStream_t s) {
   const int64_t rows = (int64_t)a.T * (a.H / a.G);
   const int64_t n = (rows + kPaRows - 1) / kPaRows * a.G * a.B;
   SOCKET_REQUIRE(n < (1LL << 31), SOCKET_ERR_SHAPE);
   constexpr int lds = 2 * kPaKeys * (D + D2 + DV) * 2;
-  auto kern = prompt_attend_kernel<DT, D, D2, DV, SPLIT, CAPPED>;
+  auto kern = prompt_attend_kernel<DT, D, D2, DV, SPLIT, CAPPED, POS>;
   if constexpr (lds > 65536) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
       return SOCKET_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64 * kPaWaves), lds, s, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64 * kPaWaves), lds, s, a, positions);
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
 }
 
-}  // namespace
+template <class DT, int D>
+int pa_plain(const socket_chunk_attention& a, const int64_t* positions, bool weights16, hipStream_t s) {
+  if constexpr (DT::kEnum == SOCKET_BF16) {
+    if (a.softcap > 0.f) return pa_launch<DT, D, 0, D, true, true>(a, nullptr, s);
+  }
+  if (weights16)
+    return positions ? pa_launch<DT, D, 0, D, false, false, true>(a, positions, s) : pa_launch<DT, D, 0, D, false, false>(a, nullptr, s);
+  return positions ? pa_launch<DT, D, 0, D, true, false, true>(a, positions, s) : pa_launch<DT, D, 0, D, true, false>(a, nullptr, s);
+}
 
 template <class DT>
-static int pa_run(const socket_chunk_attention& a, bool weights16, hipStream_t s) {
-  if (a.k2) {
-    if constexpr (DT::kEnum == SOCKET_BF16) return pa_launch<DT, 128, 64, 128, true, false>(a, s);
-    return SOCKET_ERR_UNSUPPORTED;
-  }
+int pa_run(const socket_chunk_attention& a, const int64_t* positions, bool weights16, hipStream_t s) {
   if constexpr (DT::kEnum == SOCKET_BF16) {
-    if (a.softcap > 0.f)
-      return a.D == 64 ? pa_launch<DT, 64, 0, 64, true, true>(a, s) : pa_launch<DT, 128, 0, 128, true, true>(a, s);
+    if (a.k2) return pa_launch<DT, 128, 64, 128, true, false>(a, nullptr, s);
   }
-  if (a.D == 64)
-    return weights16 ? pa_launch<DT, 64, 0, 64, false, false>(a, s) : pa_launch<DT, 64, 0, 64, true, false>(a, s);
-  return weights16 ? pa_launch<DT, 128, 0, 128, false, false>(a, s) : pa_launch<DT, 128, 0, 128, true, false>(a, s);
+  return a.D == 64 ? pa_plain<DT, 64>(a, positions, weights16, s) : pa_plain<DT, 128>(a, positions, weights16, s);
 }
+
+}  // namespace
 
 // Whether the shape is one of this file's; alignment and the checks of the entry points are the caller's.
 bool prompt_attend_fits(const socket_chunk_attention& a) {
@@ -386,6 +408,6 @@ bool prompt_attend_fits(const socket_chunk_attention& a) {
   return (a.D == 64 || a.D == 128) && a.Dv == a.D && !a.gate;
 }
 
-int prompt_attend_launch(const socket_chunk_attention& a, bool weights16, hipStream_t s) {
-  return a.dtype == SOCKET_F16 ? pa_run<DType_f16>(a, weights16, s) : pa_run<DType_bf16>(a, weights16, s);
+int prompt_attend_launch(const socket_chunk_attention& a, const int64_t* positions, bool weights16, hipStream_t s) {
+  return a.dtype == SOCKET_F16 ? pa_run<DType_f16>(a, positions, weights16, s) : pa_run<DType_bf16>(a, positions, weights16, s);
 }

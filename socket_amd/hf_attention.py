@@ -38,7 +38,7 @@ import torch
 import torch.nn as nn
 from torch.nn import functional as F
 
-from . import hash_cache
+from . import hash_cache, layer_ops
 from .socket_kernels import dense_decode_fwd
 
 
@@ -216,6 +216,9 @@ class SocketLlamaAttention(nn.Module):
             if attention_mask is not None:
                 y = F.scaled_dot_product_attention(q, k, v, attn_mask=attention_mask, scale=self.scaling,
                                                    enable_gqa=H != Hkv)
+            elif T_q > 1 and T_q == T_k and layer_ops.prompt_attend_fits(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)):
+                y = layer_ops.prompt_attend(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), 0, self.scaling,
+                                            weights16=True).transpose(1, 2)
             else:
                 y = F.scaled_dot_product_attention(q, k, v, is_causal=T_q > 1 and T_q == T_k, scale=self.scaling,
                                                    enable_gqa=H != Hkv)

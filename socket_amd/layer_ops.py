@@ -330,6 +330,45 @@ def causal_attend(q: Tensor, k: Tensor, k_shared: Tensor, v: Tensor, pos0: int, 
     return out
 
 
+def prompt_attend_fits(q: Tensor, k: Tensor, v: Tensor) -> bool:
+    """Whether `prompt_attend` takes q [B,T,H,D], k / v [B,S,G,D]: plain 16-bit device tensors of 64 or 128
+    dims in rows a 16-byte load can read, that nothing differentiates, transforms or traces."""
+    D = q.shape[-1]
+    if not q.is_cuda or q.dtype not in (torch.bfloat16, torch.float16) or D not in (64, 128) or q.shape[1] < 1:
+        return False
+    if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.maybe_current_level() is not None:
+        return False
+    for t in (q, k, v):
+        if type(t) is not Tensor or t.dtype != q.dtype or t.device != q.device or t.shape[-1] != D or t.stride(-1) != 1:
+            return False
+        if (torch.is_grad_enabled() and t.requires_grad) or t.data_ptr() % 16 != 0 or any(st % 8 != 0 for st in t.stride()[:3]):
+            return False
+    return (k.shape == v.shape and k.shape[0] == q.shape[0] and q.shape[0] <= 65535 and q.shape[2] % k.shape[2] == 0
+            and k.shape[1] < 2 ** 30 and max(k.stride(1), v.stride(1)) < 2 ** 24 and min(k.stride() + v.stride()) >= 0)
+
+
+@torch.no_grad()
+def prompt_attend(q: Tensor, k: Tensor, v: Tensor, pos0: int, scale: float, positions: Optional[Tensor] = None,
+                  weights16: bool = False) -> Tensor:
+    """Causal attention of queries q [B,T,H,D] at positions pos0 .. over k / v [B,S,G,D], S = pos0 + T, of every
+    position (any strides): [B,T,H,D].  `positions` (int64 [T], on the device): token t sees the keys up to
+    positions[t] instead.  `weights16`: the weights enter the second product rounded to the inputs' type, as flash
+    attention kernels have it, instead of in two terms."""
+    B, T, H, D = q.shape
+    assert k.shape[1] == v.shape[1] == pos0 + T
+    out = torch.empty(B, T, H, D, dtype=q.dtype, device=q.device)
+    a = ChunkAttention(q=q.data_ptr(), q_stride_b=q.stride(0), q_stride_t=q.stride(1), q_stride_h=q.stride(2),
+                       dtype=dtype_enum(q.dtype), B=B, T=T, H=H, G=k.shape[2], D=D, chunk=ENDLESS, pos0=pos0, k_from=0,
+                       scale=scale, out=out.data_ptr())
+    a.k_new, (a.k_stride_b, a.k_stride_t, a.k_stride_g) = k.data_ptr(), k.stride()[:3]
+    a.v_new, (a.v_stride_b, a.v_stride_t, a.v_stride_g) = v.data_ptr(), v.stride()[:3]
+    if positions is not None:
+        assert positions.dtype == torch.int64 and positions.is_cuda and positions.numel() == T and positions.is_contiguous()
+    check("socket_prompt_attention", core().socket_prompt_attention(ctypes.byref(a), ptr(positions), int(weights16),
+                                                                    stream_ptr(q.device)))
+    return out
+
+
 def _latent_args(src: Optional[Tensor], cache, dim: int, H: int, B: int, T: int, cos_sin: Tensor, pos0: int,
                  pos: Optional[Tensor], eps: float) -> Latent:
     a = Latent(dtype=dtype_enum(cache.rows.dtype), B=B, T=T, H=H, dim=dim, rot=cache.rot, rank=cache.rank, eps=eps,

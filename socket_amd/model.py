@@ -15,8 +15,9 @@ walks its state:
     back to the host (the reference syncs at model.py:211-212,228,483) and the
     whole step can be recorded into a HIP graph;
   * no per-step code relayout (model.py:490-509), no K/V prefix copies
-    (:541-542), no T x T boolean mask (:279-281): prefill attends causally
-    through torch's flash SDPA, decode through the HIP kernels.
+    (:541-542), no T x T boolean mask (:279-281): a 16-bit prompt attends causally
+    through the HIP kernel of csrc/prompt_attend.hip (other types and head widths, and
+    anything that is differentiated, through torch's SDPA), decode through the HIP kernels.
 
 Everything outside the attention hook (embedding, linears, norms, rotary) is
 plain torch: it is plumbing around the path, not part of it.
@@ -32,7 +33,7 @@ import torch.nn as nn
 from torch import Tensor
 from torch.nn import functional as F
 
-from . import decode_ops, hash_cache
+from . import decode_ops, hash_cache, layer_ops
 from .socket_kernels import dense_decode_fwd
 
 
@@ -560,12 +561,20 @@ class Attention(nn.Module):
         itself (dense in both modes, as GPT-FAST/model.py:466-481)."""
         gqa = self.n_head != self.n_local_heads
         qh = q.transpose(1, 2)
-        if self.kv_cache is None or pos0 == 0:
+        alone = self.kv_cache is None or pos0 == 0
+        if not alone:
+            end = pos0 + q.shape[1]
+            kc, vc = self.kv_cache.k_cache[:, :, :end], self.kv_cache.v_cache[:, :, :end]
+        kt, vt = (k, v) if alone else (kc.transpose(1, 2), vc.transpose(1, 2))
+        if layer_ops.prompt_attend_fits(q, kt, vt):
+            # (a block by itself is attended to as the library's flash kernels do it, weights in the model's
+            # type; over the cache the masked form kept them in 32 bits, and a token sees what its position says)
+            return layer_ops.prompt_attend(q, kt, vt, 0 if alone else pos0, self.head_dim ** -0.5,
+                                           positions=None if alone else input_pos, weights16=alone)
+        if alone:
             y = F.scaled_dot_product_attention(qh, k.transpose(1, 2), v.transpose(1, 2), is_causal=True,
                                                enable_gqa=gqa)
         else:
-            end = pos0 + q.shape[1]
-            kc, vc = self.kv_cache.k_cache[:, :, :end], self.kv_cache.v_cache[:, :, :end]
             mask = torch.arange(end, device=q.device)[None, :] <= input_pos[:, None]      # [S,end]
             y = F.scaled_dot_product_attention(qh, kc, vc, attn_mask=mask, enable_gqa=gqa)
         return y.transpose(1, 2)

@@ -74,3 +74,52 @@ def test_scores_of_any_size():
         got = layer_ops.chunk_attend(q, k, v, ChunkRing(B, T, 2, D, T, torch.bfloat16, DEV), 0, 1.0, 0.0)
         assert torch.isfinite(got).all()
         close(got, softmax_attention(q, k, v, 0, T, 1.0), 2 ** -8 if gain < 1e3 else 2 ** -6)
+
+
+@pytest.mark.parametrize("B,T,first,H,G,D,dt,w16", [
+    (2, 65, 0, 8, 2, 128, torch.bfloat16, True), (1, 257, 0, 6, 6, 64, torch.float16, True), (1, 128, 190, 4, 1, 128, torch.float16, False),
+    (3, 2, 63, 8, 8, 64, torch.bfloat16, False), (2, 300, 37, 7, 7, 128, torch.bfloat16, False)])
+def test_causal_over_a_cache(B, T, first, H, G, D, dt, w16):
+    """Keys and values as a cache holds them ([B,G,S,D]), the portion's positions given or counted."""
+    g = torch.Generator(device=DEV).manual_seed(T)
+    q = torch.randn(B, T, H, D, generator=g, device=DEV).to(dt)
+    k, v = (torch.randn(B, G, first + T + 5, D, generator=g, device=DEV).to(dt)[:, :, :first + T].transpose(1, 2) for _ in range(2))
+    assert layer_ops.prompt_attend_fits(q, k, v)
+    want = softmax_attention(q, k, v, first, 1 << 30, D ** -0.5)
+    unit = 2 ** -8 if dt == torch.bfloat16 else 2 ** -11
+    close(layer_ops.prompt_attend(q, k, v, first, D ** -0.5, weights16=w16), want, unit)
+    pos = torch.arange(first, first + T, device=DEV)
+    close(layer_ops.prompt_attend(q, k, v, first, D ** -0.5, pos, w16), want, unit)
+
+
+def test_positions_that_are_no_run():
+    """A token sees the keys up to its own position, wherever it stands; none for a position before the first."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    T, first, H, D = 150, 40, 4, 64
+    q = torch.randn(1, T, H, D, generator=g, device=DEV).bfloat16()
+    k, v = (torch.randn(1, first + T, H, D, generator=g, device=DEV).bfloat16() for _ in range(2))
+    pos = torch.randint(0, first + T + 20, (T,), generator=g, device=DEV)
+    got = layer_ops.prompt_attend(q, k, v, first, 0.1, pos)
+    s = torch.einsum("bthd,bshd->bhts", q.double(), k.double()) * 0.1
+    s = s.masked_fill(torch.arange(first + T, device=DEV)[None] > pos[:, None], -math.inf)
+    close(got, torch.einsum("bhts,bshd->bthd", torch.softmax(s, -1), v.double()), 2 ** -8)
+    pos[7] = -1
+    assert (layer_ops.prompt_attend(q, k, v, first, 0.1, pos)[:, 7] == 0).all()
+
+
+def test_what_it_leaves_to_the_library():
+    q = torch.randn(1, 8, 4, 64, device=DEV).bfloat16()
+    assert layer_ops.prompt_attend_fits(q, q, q)
+    assert not layer_ops.prompt_attend_fits(q.float(), q.float(), q.float())
+    assert not layer_ops.prompt_attend_fits(q[..., :40], q[..., :40], q[..., :40])
+    assert not layer_ops.prompt_attend_fits(q, q[:, :, :3], q[:, :, :3])
+    assert not layer_ops.prompt_attend_fits(q[..., 1:], q[..., 1:], q[..., 1:])
+    grad = q.clone().requires_grad_()
+    assert not layer_ops.prompt_attend_fits(grad, q, q)
+    with torch.no_grad():
+        assert layer_ops.prompt_attend_fits(grad, q, q)
+    seen = []
+    torch.vmap(lambda x: (seen.append(layer_ops.prompt_attend_fits(x, x, x)), x)[1])(q[None])
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(layer_ops.prompt_attend_fits(q, q, q))
+    assert seen == [False, False]
