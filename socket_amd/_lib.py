@@ -138,6 +138,7 @@ CORE_SIGNATURES = {
     "socket_rope_append": (_I, [_P, _I, _L, _P, _I, _L, _P, _I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _I, _I, _I, _I,
                                 _L, _P]),
     "socket_add_rmsnorm": (_I, [_P, _P, _P, _P, _P, _I, _L, _I, c_float, _P]),
+    "socket_rope_rows": (_I, [_P, _I, _L, _L, _P, _I, _P, _P, _P, _L, _L, _L, _L, _I, _I, _I, _I, _I, _L, _P]),
     "socket_silu_mul": (_I, [_P, _P, _P, _I, _L, _P]),
     "socket_gemv_bf16": (_I, [_P, _L, _P, _P, _P, _L, _I, _I, _I, _P]),
     "socket_norm_gemv_bf16": (_I, [_P, _P, _P, c_float, _P, _P, _P, _P, _I, _I, _I, _P]),
@@ -261,3 +262,12 @@ def require_device(*tensors) -> None:
     for t in tensors:
         if t is not None and not t.is_cuda:
             raise AssertionError("expected a tensor on the HIP device")
+
+
+def plain_tensors(*tensors) -> bool:
+    """True for device tensors that nothing differentiates, transforms or traces, which a kernel may
+    therefore read and write by address in place of torch operations."""
+    if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.maybe_current_level() is not None:
+        return False
+    grad = torch.is_grad_enabled()
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and not (grad and t.requires_grad) for t in tensors)

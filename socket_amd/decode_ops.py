@@ -8,7 +8,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from ._lib import check, dtype_enum, lib, ptr, stream_ptr
+from ._lib import check, dtype_enum, lib, plain_tensors, ptr, stream_ptr
 
 
 @torch.no_grad()
@@ -43,6 +43,41 @@ def rope_append(qkv: torch.Tensor, freqs_cis: torch.Tensor, input_pos: torch.Ten
     if return_new:
         return q_out, k_new, v_new
     return q_out
+
+
+def rope_rows_fits(qkv: torch.Tensor, freqs: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor) -> bool:
+    """Whether `rope_rows` takes the projected rows qkv [B,S,N] and these caches."""
+    per = 16 // qkv.element_size()
+    D = k_cache.shape[-1]
+    return (qkv.is_cuda and plain_tensors(qkv, freqs, k_cache, v_cache) and qkv.dtype in (torch.bfloat16, torch.float16, torch.float32)
+            and k_cache.dtype == v_cache.dtype == qkv.dtype and k_cache.shape[0] == qkv.shape[0] <= 65535 and 0 < qkv.shape[1] <= 65535 * 8
+            and k_cache.stride() == v_cache.stride() and k_cache.stride(-1) == qkv.stride(-1) == 1 and D % per == 0 and D % 2 == 0
+            and all(st % per == 0 for st in qkv.stride()[:2] + k_cache.stride()[:3])
+            and all(t.data_ptr() % 16 == 0 for t in (qkv, k_cache, v_cache))
+            and freqs.dtype in (torch.bfloat16, torch.float32) and freqs.is_contiguous() and tuple(freqs.shape) == (qkv.shape[1], D // 2, 2))
+
+
+@torch.no_grad()
+def rope_rows(qkv: torch.Tensor, freqs: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, t0: int, n_heads: int,
+              n_kv_heads: int) -> torch.Tensor:
+    """The prompt rows qkv [B,S,(Hq+2Hkv)*D] -> rotated queries [B,S,Hq,D]; rotated keys and values go into rows
+    t0 .. t0 + S of the caches [B,Hkv,Tcap,D].  freqs [S,D/2,2]: the rows' angles.  One launch with the results of
+    apply_rotary_emb on q and k (GPT-FAST/model.py:626-639) and the cache writes (:215-217)."""
+    B, S, N = qkv.shape
+    D = k_cache.shape[-1]
+    assert N == (n_heads + 2 * n_kv_heads) * D and k_cache.shape[1] == n_kv_heads
+    q = torch.empty((B, S, n_heads, D), dtype=qkv.dtype, device=qkv.device)
+    check("socket_rope_rows", lib().socket_rope_rows(
+        ptr(qkv), dtype_enum(qkv.dtype), qkv.stride(0), qkv.stride(1), ptr(freqs), dtype_enum(freqs.dtype), ptr(q),
+        ptr(k_cache), ptr(v_cache), *k_cache.stride()[:3], int(t0), B, S, n_heads, n_kv_heads, D, k_cache.shape[2],
+        stream_ptr(qkv.device)))
+    return q
+
+
+def pointwise_fits(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether `add_rmsnorm` and `silu_mul` may stand for torch's operations on these two."""
+    return (plain_tensors(a, b) and a.dtype == b.dtype and a.dtype in (torch.bfloat16, torch.float16, torch.float32)
+            and a.is_contiguous() and b.is_contiguous())
 
 
 @torch.no_grad()

@@ -17,7 +17,8 @@ import torch
 from torch import Tensor
 from torch.nn import functional as F
 
-from ._lib import (ChunkAttention, DepthMix, Latent, LatentAttend, Recurrence, Residual, RopeHalf, RowsLinear, check, core, dtype_enum, ptr, stream_ptr)
+from ._lib import (ChunkAttention, DepthMix, Latent, LatentAttend, Recurrence, Residual, RopeHalf, RowsLinear, check, core, dtype_enum, plain_tensors, ptr,
+                   stream_ptr)
 
 MAX_GEMV_ROWS = 4
 GATED_UNITS = {"clamped": 1, "silu": 2}
@@ -332,16 +333,14 @@ def causal_attend(q: Tensor, k: Tensor, k_shared: Tensor, v: Tensor, pos0: int, 
 
 def prompt_attend_fits(q: Tensor, k: Tensor, v: Tensor) -> bool:
     """Whether `prompt_attend` takes q [B,T,H,D], k / v [B,S,G,D]: plain 16-bit device tensors of 64 or 128
-    dims in rows a 16-byte load can read, that nothing differentiates, transforms or traces."""
+    dims in rows a 16-byte load can read."""
     D = q.shape[-1]
-    if not q.is_cuda or q.dtype not in (torch.bfloat16, torch.float16) or D not in (64, 128) or q.shape[1] < 1:
-        return False
-    if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.maybe_current_level() is not None:
+    if not q.is_cuda or q.dtype not in (torch.bfloat16, torch.float16) or D not in (64, 128) or q.shape[1] < 1 or not plain_tensors(q, k, v):
         return False
     for t in (q, k, v):
-        if type(t) is not Tensor or t.dtype != q.dtype or t.device != q.device or t.shape[-1] != D or t.stride(-1) != 1:
+        if t.dtype != q.dtype or t.device != q.device or t.shape[-1] != D or t.stride(-1) != 1:
             return False
-        if (torch.is_grad_enabled() and t.requires_grad) or t.data_ptr() % 16 != 0 or any(st % 8 != 0 for st in t.stride()[:3]):
+        if t.data_ptr() % 16 != 0 or any(st % 8 != 0 for st in t.stride()[:3]):
             return False
     return (k.shape == v.shape and k.shape[0] == q.shape[0] and q.shape[0] <= 65535 and q.shape[2] % k.shape[2] == 0
             and k.shape[1] < 2 ** 30 and max(k.stride(1), v.stride(1)) < 2 ** 24 and min(k.stride() + v.stride()) >= 0)

@@ -204,6 +204,20 @@ class KVCache(nn.Module):
         self.lens.fill_(hi + 1)
         return self.k_cache, self.v_cache
 
+    @torch.no_grad()
+    def update_projected(self, qkv: Tensor, freqs_cis: Tensor, n_heads: int, pos0: int, hash_keys: bool = False):
+        """`update` for the projected rows qkv [B,S,(Hq+2Hkv)*D] of a prompt at pos0, with the rotary embedding
+        (freqs_cis [S,D/2,2]) in the same launch; returns the rotated queries [B,S,Hq,D] and the new rows of
+        keys and values as [B,S,Hkv,D] views of the cache."""
+        S = qkv.shape[1]
+        self._bounds(pos0, S)
+        q = decode_ops.rope_rows(qkv, freqs_cis, self.k_cache, self.v_cache, pos0, n_heads, self.k_cache.size(1))
+        k, v = (c[:, :, pos0:pos0 + S].transpose(1, 2) for c in (self.k_cache, self.v_cache))
+        if hash_keys:
+            _hash_rows(self, k, v, t0=pos0)
+        self.lens.fill_(pos0 + S)
+        return q, k, v
+
     def _write_run(self, pos0: int, k_val: Tensor, v_val: Tensor, v_norm: Optional[Tensor],
                    k_hard: Optional[Tensor], hash_keys: bool) -> None:
         """Rows [pos0, pos0 + S) of every buffer from k_val / v_val [B,S,H,D]."""
@@ -488,14 +502,19 @@ class Attention(nn.Module):
     def _run(self, x: Tensor, freqs_cis: Tensor, input_pos: Tensor, sparse: bool, pos0: Optional[int]) -> Tensor:
         bsz, seqlen, _ = x.shape
         kv_size = self.n_local_heads * self.head_dim
-        q, k, v = self.wqkv(x).split([self.dim, kv_size, kv_size], dim=-1)
+        qkv = self.wqkv(x)
+        cache = self.kv_cache
+        if seqlen > 1 and pos0 is not None and type(cache) is KVCache and decode_ops.rope_rows_fits(qkv, freqs_cis, cache.k_cache, cache.v_cache):
+            # a prompt on the device: rotated and appended in one launch, attended to where it lies
+            q, k, v = cache.update_projected(qkv, freqs_cis, self.n_head, pos0, hash_keys=sparse)
+            return self.wo(self._prefill_attention(q, k, v, input_pos, pos0).reshape(bsz, seqlen, self.dim))
+        q, k, v = qkv.split([self.dim, kv_size, kv_size], dim=-1)
         q = q.view(bsz, seqlen, self.n_head, self.head_dim)
         k = k.view(bsz, seqlen, self.n_local_heads, self.head_dim)
         v = v.view(bsz, seqlen, self.n_local_heads, self.head_dim)
         q = apply_rotary_emb(q, freqs_cis)
         k = apply_rotary_emb(k, freqs_cis)
 
-        cache = self.kv_cache
         if sparse:
             assert cache is not None, "Call setup_caches() first so kv_cache exists"
         if cache is not None:
@@ -598,7 +617,10 @@ class FeedForward(nn.Module):
         self.w2 = nn.Linear(config.intermediate_size, config.dim, bias=False)
 
     def forward(self, x: Tensor) -> Tensor:
-        return self.w2(F.silu(self.w1(x)) * self.w3(x))
+        a, b = self.w1(x), self.w3(x)
+        if a.is_cuda and a.numel() > 0 and decode_ops.pointwise_fits(a, b) and a.shape == b.shape:
+            return self.w2(decode_ops.silu_mul(a, b))
+        return self.w2(F.silu(a) * b)
 
 
 class RMSNorm(nn.Module):
@@ -608,6 +630,8 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(dim))
 
     def forward(self, x: Tensor) -> Tensor:
+        if x.is_cuda and x.numel() > 0 and decode_ops.pointwise_fits(x, self.weight) and x.shape[-1] == self.weight.numel():
+            return decode_ops.add_rmsnorm(x, self.weight, self.eps)[1]
         xf = x.float()
         return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps)).type_as(x) * self.weight
 
