@@ -85,6 +85,21 @@ int socket_hash_keys(const void* k, const void* v, int dtype,
                      const int32_t* pos_b, int t0,
                      int B, int Hkv, int S, int D, int L, int P, int64_t Tcap,
                      void* stream);
+/* The same for rows of D <= 128 elements, D a multiple of 8, against planes padded with zeros to 128. */
+int socket_hash_rows(const void* k, const void* v, int dtype, int64_t k_stride_b, int64_t k_stride_h,
+                     int64_t k_stride_s, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_s,
+                     const void* planes_words, uint32_t* codes, uint16_t* v_norm, const int32_t* pos_b, int t0, int B,
+                     int Hkv, int S, int D, int L, int P, int64_t Tcap, void* stream);
+/* An append: the S new rows of keys and values go into rows t0 .. t0 + S - 1 of the caches (element strides b, h, s;
+ * unit-stride last dim; whole 16-byte pieces throughout) as socket_hash_rows takes them into codes and v_norm, and
+ * lens [B] (may be NULL) becomes t0 + S.  Replaces KVCache.update (GPT-FAST/model.py:187-229) with its hashing
+ * (:449-450). */
+int socket_cache_append(const void* k, const void* v, int dtype, int64_t k_stride_b, int64_t k_stride_h,
+                        int64_t k_stride_s, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_s,
+                        const void* planes_words, void* k_cache, void* v_cache, int64_t cache_stride_b,
+                        int64_t cache_stride_h, int64_t cache_stride_s, uint32_t* codes, uint16_t* v_norm, int32_t* lens,
+                        int t0, int B, int Hkv, int S, int D, int L, int P, int64_t Tcap, void* stream);
+
 
 /* Packed words -> int16 codes with arbitrary output strides (elements) over
  * (b, h, l, t) for tokens [t0, t0+T).  out[b,h,l,t-t0].  Gives the reference's

@@ -168,6 +168,9 @@ SIGNATURES = {
     "socket_permute_planes": (_I, [_P, _I, _I, _I, _I, _P, _P]),
     "socket_hash_keys": (_I, [_P, _P, _I, _L, _L, _L, _L, _L, _L, _P, _P, _P, _P, _I,
                               _I, _I, _I, _I, _I, _I, _L, _P]),
+    "socket_hash_rows": (_I, [_P, _P, _I, _L, _L, _L, _L, _L, _L, _P, _P, _P, _P, _I,
+                              _I, _I, _I, _I, _I, _I, _L, _P]),
+    "socket_cache_append": (_I, [_P, _P, _I] + [_L] * 6 + [_P, _P, _P, _L, _L, _L, _P, _P, _P] + [_I] * 7 + [_L, _P]),
     "socket_unpack_codes": (_I, [_P, _P, _I, _I, _I, _I, _I, _I, _L, _L, _L, _L, _L, _P]),
     "socket_pack_codes": (_I, [_P, _L, _L, _L, _L, _P, _I, _I, _I, _I, _I, _I, _L, _P]),
     "socket_score_range_parts": (_I, [_I, _I, _I, _I, _I, _I, _I, _I]),

@@ -115,7 +115,7 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
     int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
     const uint16_t* __restrict__ planes_words,  // bf16 [NW*32, 128]
     uint32_t* __restrict__ codes, uint16_t* __restrict__ v_norm,
-    const int32_t* __restrict__ pos_b, int t0, int Hkv, int S, int L, int P, int NW, int64_t Tcap,
+    const int32_t* __restrict__ pos_b, int t0, int Hkv, int S, int D, int L, int P, int NW, int64_t Tcap,
     int tiles_per_row, int n_tiles, int wc, int words_per_wg) {
   typedef typename DT::storage ST;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -175,8 +175,8 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
         const bool ok = srow < S;
 #pragma unroll
         for (int ks = 0; ks < kKSteps; ++ks) {
-          dst[nb][ks].u = ok ? load_frag8<DT>(base + (int64_t)srow * ss + ks * 32 + (lane >> 4) * 8)
-                             : make_uint4(0, 0, 0, 0);
+          const int d = ks * 32 + (lane >> 4) * 8;      // (a narrower head's row ends in zeros)
+          dst[nb][ks].u = ok && d < D ? load_frag8<DT>(base + (int64_t)srow * ss + d) : make_uint4(0, 0, 0, 0);
         }
       }
     };
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
         for (int g = 0; g < kKeysPerWave / 4; ++g) {
           const int srow = s0 + g * 4 + sub;
-          ss[g] = (srow < S) ? sumsq8<DT>(vbase + (int64_t)srow * v_ss + part * 8) : 0.f;
+          ss[g] = (srow < S && part * 8 < D) ? sumsq8<DT>(vbase + (int64_t)srow * v_ss + part * 8) : 0.f;
         }
 #pragma unroll
         for (int g = 0; g < kKeysPerWave / 4; ++g) {
@@ -336,18 +336,28 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
 // lanes of a fragment read (sixteen consecutive rows, one chunk) hit sixteen
 // different slots.
 constexpr int kStreamTile = 128;                       // keys per tile
-constexpr int kStreamTileBytes = kStreamTile * kD * 2;  // 32 KB
-constexpr int kStreamStageBytes = 2 * kStreamTileBytes; // keys | values
+constexpr int stream_stage_bytes(int D) { return 2 * kStreamTile * D * 2; }   // keys | values
 constexpr int kStreamWordsPerWave = 3;
 constexpr int kStreamMaxWords = kStreamWordsPerWave * kHashWaves;
 
+// D: 128, or 64 (half the contraction: the planes' other half is zero).  STORE: the tile's rows also go on
+// into k_cache / v_cache (element strides c_sb, c_sh, c_ss) at their positions, from LDS: an append then
+// reads its keys and values once.
+template <int D, bool STORE>
 __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void hash_keys_stream_kernel(
     const uint16_t* __restrict__ k_, const uint16_t* __restrict__ v_, int64_t k_sb, int64_t k_sh,
     int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
     const uint16_t* __restrict__ planes_words,  // bf16 [NW*32, 128]
     uint32_t* __restrict__ codes, uint16_t* __restrict__ v_norm,
     const int32_t* __restrict__ pos_b, int t0, int Hkv, int S, int L, int P, int NW, int64_t Tcap,
-    int tiles_per_row, int n_tiles) {
+    int tiles_per_row, int n_tiles, uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache, int64_t c_sb,
+    int64_t c_sh, int64_t c_ss) {
+  constexpr int kKSteps = D / 32, CH = D / 8, kRows = 64 / CH;      // k-steps; 16-byte pieces of a row; rows of a 1 KB copy
+  constexpr int kStreamTileBytes = kStreamTile * D * 2, kStreamStageBytes = stream_stage_bytes(D);
+  constexpr int kPieces = kStreamTile / kRows / kHashWaves;
+  // where piece c of row r goes: sixteen consecutive rows at one piece must hit sixteen different 16-byte
+  // slots of the banks (rows of 128 bytes start half a bank line apart by the row's parity)
+  auto place = [](int r, int c) { return c ^ (CH == 16 ? (r & 15) : ((r >> 1) & 7)); };
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   // (the wave index as a scalar: every address that depends on it -- this wave's
   // words of the code cache above all -- then stays out of the vector registers;
@@ -373,12 +383,14 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb) {
           const int col = w * 32 + pbit0 - 4 * mb;
-          preg[j][ks][mb].u = w < NW ? planes16[(int64_t)col * 16 + ks * 4 + quarter] : make_uint4(0, 0, 0, 0);
+          preg[j][ks][mb].u = w < NW ? planes16[(int64_t)col * (kD / 8) + ks * 4 + quarter] : make_uint4(0, 0, 0, 0);
         }
     }
   }
   const uint32_t sel1 = (quarter & 1) ? 0x03070105u : 0x06020400u;
   const uint32_t sel2 = (quarter & 2) ? 0x03020706u : 0x05040100u;
+  // (a copy's rows are all the same modulo 16, so a lane's piece is too)
+  const int lane_at = lane / CH * (int)(c_ss / 8) + place(kRows * wave + lane / CH, lane % CH);
 
   // this wave's four 1 KB pieces of a tile (rows 4p .. 4p+3 of piece p), keys and values
   auto issue_tile = [&](int tile, int stage) {
@@ -389,11 +401,11 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
     const uint16_t* vbase = with_values ? v_ + b * v_sb + h * v_sh : nullptr;
     unsigned char* dst = lds_raw + (size_t)stage * kStreamStageBytes;
 #pragma unroll
-    for (int q = 0; q < kStreamTile / 4 / kHashWaves; ++q) {
+    for (int q = 0; q < kPieces; ++q) {
       const int p = wave + kHashWaves * q;
-      const int row = 4 * p + quarter;
+      const int row = kRows * p + lane / CH;
       const int srow = min(s0 + row, S - 1);  // rows past the end re-read the last one; never stored
-      const int chunk = prow ^ (row & 15);
+      const int chunk = place(kRows * wave + lane / CH, lane % CH);
       lds_dma16_stream(kbase + (int64_t)srow * k_ss + chunk * 8, dst + p * 1024);
       if (with_values) lds_dma16_stream(vbase + (int64_t)srow * v_ss + chunk * 8, dst + kStreamTileBytes + p * 1024);
     }
@@ -417,7 +429,19 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
     const uint4* ktile = reinterpret_cast<const uint4*>(lds_raw + (size_t)stage * kStreamStageBytes);
     const uint4* vtile = ktile + kStreamTileBytes / 16;
     // chunk c of row r of a tile (r & 15 == prow for every row this lane reads)
-    auto frag_at = [&](const uint4* t, int r, int c) { return t[r * 16 + (c ^ prow)]; };
+    auto frag_at = [&](const uint4* t, int r, int c) { return t[r * CH + place(prow, c)]; };
+
+    if constexpr (STORE) {
+      // this wave's pieces of the tile on into the caches, whole rows of 256 (128) bytes
+      const int64_t c0 = (int64_t)(pair / Hkv) * c_sb + (pair % Hkv) * c_sh + (int64_t)(pos0 + s0 + kRows * wave) * c_ss;
+#pragma unroll
+      for (int q = 0; q < kPieces; ++q)
+        if (s0 + kRows * (wave + kHashWaves * q) + lane / CH < S) {
+          const int64_t at = c0 + (int64_t)(kRows * kHashWaves * q) * c_ss;
+          reinterpret_cast<uint4*>(k_cache + at)[lane_at] = ktile[(wave + kHashWaves * q) * 64 + lane];
+          reinterpret_cast<uint4*>(v_cache + at)[lane_at] = vtile[(wave + kHashWaves * q) * 64 + lane];
+        }
+    }
 
     if (with_values) {
       // ||v||^2 = diagonal of V V^T (see hash_keys_kernel), key block `wave` of the tile
@@ -505,6 +529,42 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
     if (my_words == 3) tile_body(std::integral_constant<int, 3>{});
     else if (my_words == 2) tile_body(std::integral_constant<int, 2>{});
     else if (my_words == 1) tile_body(std::integral_constant<int, 1>{});
+  }
+}
+
+// Keys and values [B,Hkv,S,D] (any strides, whole 16-byte pieces) into rows t0 .. of the caches; the lengths
+// become t0 + S.  A lane moves kCopyPieces pieces of each, requested together; a wave's stores are whole rows.
+constexpr int kCopyPieces = 4;
+template <class DT>
+__global__ __launch_bounds__(256) void copy_rows_kernel(const void* __restrict__ k, const void* __restrict__ v, int64_t k_sb,
+                                                        int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
+                                                        void* __restrict__ k_cache, void* __restrict__ v_cache, int64_t c_sb,
+                                                        int64_t c_sh, int64_t c_ss, int32_t* __restrict__ lens, int t0, int B,
+                                                        int Hkv, int S, int D, int copy) {
+  typedef typename DT::storage ST;
+  constexpr int E = DT::kPer16B;
+  if (lens && blockIdx.x == 0 && blockIdx.y == 0)
+    for (int b = threadIdx.x; b < B; b += 256) lens[b] = t0 + S;
+  if (!copy) return;
+  const int b = blockIdx.y / Hkv, h = blockIdx.y % Hkv, per = D / E;
+  const ST* kp = (const ST*)k + b * k_sb + h * k_sh;
+  const ST* vp = (const ST*)v + b * v_sb + h * v_sh;
+  const int64_t c0 = b * c_sb + h * c_sh, n = (int64_t)S * per, i0 = (int64_t)blockIdx.x * 256 * kCopyPieces + threadIdx.x;
+  uint4 x[kCopyPieces], y[kCopyPieces];
+#pragma unroll
+  for (int u = 0; u < kCopyPieces; ++u) {
+    const int64_t i = min(i0 + u * 256, n - 1);
+    const int s = (int)(i / per), d = (int)(i % per) * E;
+    x[u] = *reinterpret_cast<const uint4*>(kp + s * k_ss + d);
+    y[u] = *reinterpret_cast<const uint4*>(vp + s * v_ss + d);
+  }
+#pragma unroll
+  for (int u = 0; u < kCopyPieces; ++u) {
+    const int64_t i = i0 + u * 256;
+    if (i >= n) break;
+    const int64_t at = c0 + (t0 + i / per) * c_ss + i % per * E;
+    *reinterpret_cast<uint4*>((ST*)k_cache + at) = x[u];
+    *reinterpret_cast<uint4*>((ST*)v_cache + at) = y[u];
   }
 }
 
@@ -601,56 +661,52 @@ extern "C" int socket_permute_planes(const void* planes, int planes_dtype, int L
   return SOCKET_OK;
 }
 
-extern "C" int socket_hash_keys(const void* k, const void* v, int dtype, int64_t k_stride_b,
-                                int64_t k_stride_h, int64_t k_stride_s, int64_t v_stride_b,
-                                int64_t v_stride_h, int64_t v_stride_s, const void* planes_words,
-                                uint32_t* codes, uint16_t* v_norm, const int32_t* pos_b, int t0,
-                                int B, int Hkv, int S, int D, int L, int P, int64_t Tcap,
-                                void* stream) {
-  SOCKET_REQUIRE(k && planes_words && codes, SOCKET_ERR_NULL);
-  SOCKET_REQUIRE(v == nullptr || v_norm != nullptr, SOCKET_ERR_NULL);
-  SOCKET_REQUIRE(D == kD, SOCKET_ERR_UNSUPPORTED);
-  const int NW = words_per_key(L, P);
-  SOCKET_REQUIRE(NW > 0 && B > 0 && Hkv > 0 && S > 0, SOCKET_ERR_SHAPE);
-  SOCKET_REQUIRE(t0 >= 0 && (pos_b != nullptr || (int64_t)t0 + S <= Tcap), SOCKET_ERR_SHAPE);
-  const int eb = socket_dtype_bytes(dtype);
-  SOCKET_REQUIRE(eb != 0, SOCKET_ERR_UNSUPPORTED);
-  const int per16 = 16 / eb;
-  SOCKET_REQUIRE(socket_aligned16(k) && socket_aligned16(planes_words) &&
-                     k_stride_b % per16 == 0 && k_stride_h % per16 == 0 && k_stride_s % per16 == 0,
-                 SOCKET_ERR_ALIGN);
-  if (v) {
-    SOCKET_REQUIRE(socket_aligned16(v) && v_stride_b % per16 == 0 && v_stride_h % per16 == 0 &&
-                       v_stride_s % per16 == 0,
-                   SOCKET_ERR_ALIGN);
-  }
-  const SocketDeviceLimits& lim = socket_device_limits();
-  hipStream_t s = (hipStream_t)stream;
-  {
-    // enough 128-key tiles to keep every CU streaming: the variant with the planes in registers
-    const int tiles_per_row = (S + kStreamTile - 1) / kStreamTile;
-    const int64_t n_tiles64 = (int64_t)B * Hkv * tiles_per_row;
-    SOCKET_REQUIRE(n_tiles64 < (1LL << 30), SOCKET_ERR_SHAPE);  // tile + grid size stays an int
-    if (dtype == SOCKET_BF16 && NW <= kStreamMaxWords && n_tiles64 >= lim.cu_count &&
-        2 * kStreamStageBytes <= lim.max_lds_per_block) {
-      const size_t lds = 2 * (size_t)kStreamStageBytes;
-      auto kern = hash_keys_stream_kernel;
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)lds) != hipSuccess)
-        return SOCKET_ERR_LAUNCH;
-      const int n_wg = (int)(n_tiles64 < lim.cu_count ? n_tiles64 : lim.cu_count);
-      hipLaunchKernelGGL(kern, dim3(n_wg), dim3(kHashThreads), lds, s, (const uint16_t*)k, (const uint16_t*)v,
-                         k_stride_b, k_stride_h, k_stride_s, v_stride_b, v_stride_h, v_stride_s,
-                         (const uint16_t*)planes_words, codes, v_norm, pos_b, t0, Hkv, S, L, P, NW, Tcap,
-                         tiles_per_row, (int)n_tiles64);
-      SOCKET_LAUNCH_CHECK();
-      return SOCKET_OK;
-    }
-  }
-  const int tiles_per_row = (S + kKeysPerWave - 1) / kKeysPerWave;
-  const int64_t n_tiles64 = (int64_t)B * Hkv * tiles_per_row;
+namespace {
+
+// Keys (and values) as hash_keys and cache_append have them; k_cache: the rows also go there.
+struct HashRows {
+  const void *k, *v;
+  int dtype;
+  int64_t k_sb, k_sh, k_ss, v_sb, v_sh, v_ss;
+  const void* planes_words;
+  uint32_t* codes;
+  uint16_t* v_norm;
+  const int32_t* pos_b;
+  int t0, B, Hkv, S, D, L, P, NW;
+  int64_t Tcap;
+  void *k_cache, *v_cache;
+  int64_t c_sb, c_sh, c_ss;
+};
+
+// Enough 128-key tiles to keep every CU streaming: the variant with the planes in registers.
+bool streams(const HashRows& a, const SocketDeviceLimits& lim) {
+  const int64_t tiles = (int64_t)a.B * a.Hkv * ((a.S + kStreamTile - 1) / kStreamTile);
+  return a.dtype == SOCKET_BF16 && (a.D == 128 || a.D == 64) && a.NW <= kStreamMaxWords && tiles >= lim.cu_count &&
+         2 * stream_stage_bytes(a.D) <= lim.max_lds_per_block;
+}
+
+template <int D, bool STORE>
+int launch_stream(const HashRows& a, const SocketDeviceLimits& lim, hipStream_t s) {
+  const int tiles_per_row = (a.S + kStreamTile - 1) / kStreamTile;
+  const int64_t n_tiles64 = (int64_t)a.B * a.Hkv * tiles_per_row;
+  const size_t lds = 2 * (size_t)stream_stage_bytes(D);
+  auto kern = hash_keys_stream_kernel<D, STORE>;
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    return SOCKET_ERR_LAUNCH;
+  const int n_wg = (int)(n_tiles64 < lim.cu_count ? n_tiles64 : lim.cu_count);
+  hipLaunchKernelGGL(kern, dim3(n_wg), dim3(kHashThreads), lds, s, (const uint16_t*)a.k, (const uint16_t*)a.v, a.k_sb, a.k_sh,
+                     a.k_ss, a.v_sb, a.v_sh, a.v_ss, (const uint16_t*)a.planes_words, a.codes, a.v_norm, a.pos_b, a.t0, a.Hkv,
+                     a.S, a.L, a.P, a.NW, a.Tcap, tiles_per_row, (int)n_tiles64, (uint16_t*)a.k_cache, (uint16_t*)a.v_cache,
+                     a.c_sb, a.c_sh, a.c_ss);
+  SOCKET_LAUNCH_CHECK();
+  return SOCKET_OK;
+}
+
+int launch_staged(const HashRows& a, const SocketDeviceLimits& lim, hipStream_t s) {
+  const int tiles_per_row = (a.S + kKeysPerWave - 1) / kKeysPerWave;
+  const int64_t n_tiles64 = (int64_t)a.B * a.Hkv * tiles_per_row;
   SOCKET_REQUIRE(n_tiles64 < (1LL << 31), SOCKET_ERR_SHAPE);
-  const int n_tiles = (int)n_tiles64;
+  const int n_tiles = (int)n_tiles64, NW = a.NW;
   // plane slice: every word when they all fit in LDS (one slice, loaded once per
   // workgroup), else as many as fit; one persistent workgroup per CU
   int wc = lim.max_lds_per_block / (32 * kD * 2);
@@ -673,17 +729,107 @@ extern "C" int socket_hash_keys(const void* k, const void* v, int dtype, int64_t
         hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                                   \
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)   \
       return SOCKET_ERR_LAUNCH;                                                                    \
-    hipLaunchKernelGGL(kern, grid, dim3(kHashThreads), lds, s, k, v, k_stride_b, k_stride_h,       \
-                       k_stride_s, v_stride_b, v_stride_h, v_stride_s,                             \
-                       (const uint16_t*)planes_words, codes, v_norm, pos_b, t0, Hkv, S, L, P, NW,  \
-                       Tcap, tiles_per_row, n_tiles, wc, words_per_wg);                            \
+    hipLaunchKernelGGL(kern, grid, dim3(kHashThreads), lds, s, a.k, a.v, a.k_sb, a.k_sh, a.k_ss,   \
+                       a.v_sb, a.v_sh, a.v_ss, (const uint16_t*)a.planes_words, a.codes, a.v_norm, \
+                       a.pos_b, a.t0, a.Hkv, a.S, a.D, a.L, a.P, NW, a.Tcap, tiles_per_row, n_tiles, \
+                       wc, words_per_wg);                                                          \
   } while (0)
-  if (dtype == SOCKET_BF16) SOCKET_HASH_LAUNCH(DType_bf16);
-  else if (dtype == SOCKET_F16) SOCKET_HASH_LAUNCH(DType_f16);
+  if (a.dtype == SOCKET_BF16) SOCKET_HASH_LAUNCH(DType_bf16);
+  else if (a.dtype == SOCKET_F16) SOCKET_HASH_LAUNCH(DType_f16);
   else SOCKET_HASH_LAUNCH(DType_f32);
 #undef SOCKET_HASH_LAUNCH
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
+}
+
+int check_hash_rows(const HashRows& a) {
+  SOCKET_REQUIRE(a.k && a.planes_words && a.codes, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(a.v == nullptr || a.v_norm != nullptr, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(a.NW > 0 && a.B > 0 && a.Hkv > 0 && a.S > 0, SOCKET_ERR_SHAPE);
+  SOCKET_REQUIRE(a.t0 >= 0 && (a.pos_b != nullptr || (int64_t)a.t0 + a.S <= a.Tcap), SOCKET_ERR_SHAPE);
+  const int eb = socket_dtype_bytes(a.dtype);
+  SOCKET_REQUIRE(eb != 0, SOCKET_ERR_UNSUPPORTED);
+  const int per16 = 16 / eb;
+  SOCKET_REQUIRE(socket_aligned16(a.k) && socket_aligned16(a.planes_words) && a.k_sb % per16 == 0 && a.k_sh % per16 == 0 &&
+                     a.k_ss % per16 == 0,
+                 SOCKET_ERR_ALIGN);
+  if (a.v)
+    SOCKET_REQUIRE(socket_aligned16(a.v) && a.v_sb % per16 == 0 && a.v_sh % per16 == 0 && a.v_ss % per16 == 0, SOCKET_ERR_ALIGN);
+  // (tile + grid size stays an int)
+  SOCKET_REQUIRE((int64_t)a.B * a.Hkv * ((a.S + kStreamTile - 1) / kStreamTile) < (1LL << 30), SOCKET_ERR_SHAPE);
+  return SOCKET_OK;
+}
+
+}  // namespace
+
+extern "C" int socket_hash_keys(const void* k, const void* v, int dtype, int64_t k_stride_b,
+                                int64_t k_stride_h, int64_t k_stride_s, int64_t v_stride_b,
+                                int64_t v_stride_h, int64_t v_stride_s, const void* planes_words,
+                                uint32_t* codes, uint16_t* v_norm, const int32_t* pos_b, int t0,
+                                int B, int Hkv, int S, int D, int L, int P, int64_t Tcap,
+                                void* stream) {
+  SOCKET_REQUIRE(k && planes_words && codes, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(v == nullptr || v_norm != nullptr, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(D == kD, SOCKET_ERR_UNSUPPORTED);
+  const HashRows a = {k, v, dtype, k_stride_b, k_stride_h, k_stride_s, v_stride_b, v_stride_h, v_stride_s, planes_words, codes,
+                      v_norm, pos_b, t0, B, Hkv, S, D, L, P, words_per_key(L, P), Tcap, nullptr, nullptr, 0, 0, 0};
+  const int st = check_hash_rows(a);
+  if (st != SOCKET_OK) return st;
+  const SocketDeviceLimits& lim = socket_device_limits();
+  return streams(a, lim) ? launch_stream<kD, false>(a, lim, (hipStream_t)stream) : launch_staged(a, lim, (hipStream_t)stream);
+}
+
+extern "C" int socket_hash_rows(const void* k, const void* v, int dtype, int64_t k_stride_b, int64_t k_stride_h,
+                                int64_t k_stride_s, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_s,
+                                const void* planes_words, uint32_t* codes, uint16_t* v_norm, const int32_t* pos_b, int t0,
+                                int B, int Hkv, int S, int D, int L, int P, int64_t Tcap, void* stream) {
+  SOCKET_REQUIRE(D > 0 && D <= kD && D % 8 == 0, SOCKET_ERR_UNSUPPORTED);
+  const HashRows a = {k, v, dtype, k_stride_b, k_stride_h, k_stride_s, v_stride_b, v_stride_h, v_stride_s, planes_words, codes,
+                      v_norm, pos_b, t0, B, Hkv, S, D, L, P, words_per_key(L, P), Tcap, nullptr, nullptr, 0, 0, 0};
+  const int st = check_hash_rows(a);
+  if (st != SOCKET_OK) return st;
+  hipStream_t s = (hipStream_t)stream;
+  const SocketDeviceLimits& lim = socket_device_limits();
+  if (!streams(a, lim)) return launch_staged(a, lim, s);
+  return D == 64 ? launch_stream<64, false>(a, lim, s) : launch_stream<128, false>(a, lim, s);
+}
+
+extern "C" int socket_cache_append(const void* k, const void* v, int dtype, int64_t k_stride_b, int64_t k_stride_h,
+                                   int64_t k_stride_s, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_s,
+                                   const void* planes_words, void* k_cache, void* v_cache, int64_t cache_stride_b,
+                                   int64_t cache_stride_h, int64_t cache_stride_s, uint32_t* codes, uint16_t* v_norm,
+                                   int32_t* lens, int t0, int B, int Hkv, int S, int D, int L, int P, int64_t Tcap,
+                                   void* stream) {
+  SOCKET_REQUIRE(k && v && k_cache && v_cache, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(D > 0 && D <= kD && D % 8 == 0, SOCKET_ERR_UNSUPPORTED);
+  HashRows a = {k, v, dtype, k_stride_b, k_stride_h, k_stride_s, v_stride_b, v_stride_h, v_stride_s, planes_words, codes,
+                v_norm, nullptr, t0, B, Hkv, S, D, L, P, words_per_key(L, P), Tcap, k_cache, v_cache, cache_stride_b,
+                cache_stride_h, cache_stride_s};
+  const int st = check_hash_rows(a);
+  if (st != SOCKET_OK) return st;
+  const int per16 = 16 / socket_dtype_bytes(dtype);
+  SOCKET_REQUIRE(socket_aligned16(k_cache) && socket_aligned16(v_cache) && cache_stride_b % per16 == 0 &&
+                     cache_stride_h % per16 == 0 && cache_stride_s % per16 == 0,
+                 SOCKET_ERR_ALIGN);
+  SOCKET_REQUIRE((int64_t)B * Hkv <= 65535 && cache_stride_s >= 0 && cache_stride_s < (1 << 28), SOCKET_ERR_SHAPE);
+  hipStream_t s = (hipStream_t)stream;
+  const SocketDeviceLimits& lim = socket_device_limits();
+  const bool streamed = streams(a, lim);
+  // the rows' copy (all of it where the hash does not pass them on) and the lengths
+  if (!streamed || lens) {
+    const int64_t pieces = streamed ? 1 : (int64_t)S * (D / per16);
+    const dim3 grid((unsigned)((pieces + 256 * kCopyPieces - 1) / (256 * kCopyPieces)), (unsigned)(streamed ? 1 : B * Hkv));
+#define SOCKET_COPY(DT)                                                                                                    \
+  hipLaunchKernelGGL((copy_rows_kernel<DT>), grid, dim3(256), 0, s, k, v, k_stride_b, k_stride_h, k_stride_s, v_stride_b,  \
+                     v_stride_h, v_stride_s, k_cache, v_cache, cache_stride_b, cache_stride_h, cache_stride_s, lens, t0, B, \
+                     Hkv, S, D, streamed ? 0 : 1)
+    if (dtype == SOCKET_F32) SOCKET_COPY(DType_f32);
+    else SOCKET_COPY(DType_bf16);      // (16-bit rows are moved as they are)
+#undef SOCKET_COPY
+    SOCKET_LAUNCH_CHECK();
+  }
+  if (!streamed) return launch_staged(a, lim, s);
+  return D == 64 ? launch_stream<64, true>(a, lim, s) : launch_stream<128, true>(a, lim, s);
 }
 
 extern "C" int socket_unpack_codes(const uint32_t* codes, int16_t* out, int B, int Hkv, int L, int P,

@@ -22,7 +22,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from ._lib import check, dtype_enum, lib, ptr, stream_ptr
+from ._lib import check, dtype_enum, lib, plain_tensors, ptr, stream_ptr
 from .socket_kernels import prefers_one_launch, sparse_attention_fwd, sparse_attention_fwd_static
 from .sparse import select_list
 
@@ -74,7 +74,10 @@ def hash_keys_into(k: torch.Tensor, v: Optional[torch.Tensor], planes_words: tor
     else:
         raise ValueError(layout)
     assert k.stride(-1) == 1 and (v is None or (v.stride(-1) == 1 and v.shape == k.shape and v.dtype == k.dtype))
-    if D < HASH_DIM and planes_words.shape[1] == HASH_DIM and S > 0:
+    per = 16 // k.element_size()
+    narrow = D < HASH_DIM and planes_words.shape[1] == HASH_DIM and S > 0
+    fits = narrow and D % 8 == 0 and all(t is None or t.data_ptr() % 16 == 0 for t in (k, v)) and all(st % per == 0 for st in ks + vs)
+    if narrow and not fits:
         # a narrower head: the new rows are padded with zeros to the kernel's 128 coordinates
         # (same sign bits, same value norms); strides are then those of the padded copies
         k = torch.nn.functional.pad(k, (0, HASH_DIM - D))
@@ -95,7 +98,8 @@ def hash_keys_into(k: torch.Tensor, v: Optional[torch.Tensor], planes_words: tor
         assert pos_b.dtype == torch.int32 and pos_b.is_cuda and pos_b.numel() == B
     if S == 0:
         return
-    check("socket_hash_keys", lib().socket_hash_keys(
+    entry = lib().socket_hash_rows if fits else lib().socket_hash_keys       # (a narrower head the kernel reads as it is)
+    check("socket_hash_keys", entry(
         ptr(k), ptr(v), dtype_enum(k.dtype), *ks, *vs, ptr(planes_words), ptr(codes), ptr(v_norm),
         ptr(pos_b), int(t0), B, Hkv, S, D, int(L), int(P), Tcap, stream_ptr(k.device)))
 
@@ -482,8 +486,28 @@ class SocketHashCache:
         if pos0 < 0 or pos0 + S > self.Tcap:
             raise RuntimeError(
                 f"KVCache.update out-of-bounds: positions [{pos0},{pos0 + S - 1}] but cache T={self.Tcap}")
+        if self._append_fits(k_bshd, v_bshd):
+            kc = self.k_cache
+            check("socket_cache_append", lib().socket_cache_append(
+                ptr(k_bshd), ptr(v_bshd), dtype_enum(kc.dtype), k_bshd.stride(0), k_bshd.stride(2), k_bshd.stride(1),
+                v_bshd.stride(0), v_bshd.stride(2), v_bshd.stride(1), ptr(self.planes_words), ptr(kc), ptr(self.v_cache),
+                kc.stride(0), kc.stride(1), kc.stride(2), ptr(self.codes), ptr(self.v_norm), ptr(self.lens), int(pos0), B, H, S, D,
+                self.L, self.P, self.Tcap, stream_ptr(kc.device)))
+            return
         self.k_cache[:, :, pos0:pos0 + S].copy_(k_bshd.permute(0, 2, 1, 3))
         self.v_cache[:, :, pos0:pos0 + S].copy_(v_bshd.permute(0, 2, 1, 3))
         hash_keys_into(self.k_cache[:, :, pos0:pos0 + S], self.v_cache[:, :, pos0:pos0 + S],
                        self.planes_words, self.codes, self.v_norm, self.L, self.P, t0=pos0)
         self.lens.fill_(pos0 + S)      # the cached length follows the position
+
+    def _append_fits(self, k: torch.Tensor, v: torch.Tensor) -> bool:
+        """Whether one call of the library copies and hashes these rows (else: torch's copies, then the hash)."""
+        kc, per = self.k_cache, 16 // self.k_cache.element_size()
+        own = (kc, self.v_cache, self.codes, self.v_norm, self.lens, self.planes_words)
+        return (plain_tensors(k, v, *own) and k.dtype == v.dtype == kc.dtype == self.v_cache.dtype and k.device == v.device == kc.device
+                and kc.dtype in (torch.bfloat16, torch.float16, torch.float32)
+                and k.shape == v.shape and tuple(k.shape[2:]) == (kc.shape[1], kc.shape[3]) and k.shape[1] > 0
+                and k.shape[3] % 8 == 0 and k.shape[3] <= HASH_DIM and self.planes_words.shape[1] == HASH_DIM and kc.shape[0] * kc.shape[1] <= 65535
+                and all(t.is_contiguous() for t in own) and k.stride(3) == v.stride(3) == 1
+                and all(st % per == 0 for st in k.stride()[:3] + v.stride()[:3])
+                and all(t.data_ptr() % 16 == 0 for t in (k, v, kc, self.v_cache)))
