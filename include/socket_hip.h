@@ -502,6 +502,25 @@ int socket_block_sparse_attention(const void* q, const void* k, const void* v, i
                                   int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_m,
                                   int B, int H, int T, int D, int num_rows, int klist,
                                   int block_m, int block_n, void* stream);
+/* The same with rows at or past seqlens[b] set to zero. */
+int socket_block_sparse_attention_cleared(const void* q, const void* k, const void* v, int dtype,
+                                  int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_m,
+                                  int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n,
+                                  int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_n,
+                                  const int32_t* seqlens, const int32_t* block_index, void* out,
+                                  int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_m,
+                                  int B, int H, int T, int D, int num_rows, int klist,
+                                  int block_m, int block_n, void* stream);
+/* Block lists from block scores [B,R,C] (element strides b, r): per row the forced blocks -- 0, the diagonal (row r's
+ * first query r * block_m lies in block r * block_m / block_n) with `diagonal`, `window` blocks up to it -- and the K
+ * best-scoring others, none past the block of the row's last query (of Tq) with `causal`; the lower block first among
+ * equal scores (each raised by 1e-6 * block / C), scores of -inf never.  out [B,R,K] int32, ascending: repeats of n_slots
+ * slots (the most forced blocks any row has, plus K) count as block 0, the K smallest stay, one 0 makes way for the
+ * diagonal (_assemble in block_sparse_flash_attention.py; kernels/block_sparse_flash_attention.py:11-222).
+ * C <= 4096, else SOCKET_ERR_UNSUPPORTED. */
+int socket_block_lists(const float* scores, int64_t stride_b, int64_t stride_r, int32_t* out, int B, int R, int C, int K,
+                       int n_slots, int block_m, int block_n, int Tq, int causal, int diagonal, int window, void* stream);
+
 
 /* ------------------------------------------------------------------------
  * Layers of decoders with a 32-bit residual stream, chunked attention and

@@ -195,6 +195,8 @@ SIGNATURES = {
     "socket_decode_prologue": (_I, [_P, _I, _L, _P, _I, _L, _P, _I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _P, _P, _P, _P,
                                     _I, _I, _I, _I, _I, _I, _I, _I, _I, _L, c_float, c_float, _P]),
     "socket_block_sparse_attention": (_I, [_P, _P, _P, _I] + [_L] * 9 + [_P, _P, _P] + [_L] * 3 + [_I] * 8 + [_P]),
+    "socket_block_sparse_attention_cleared": (_I, [_P, _P, _P, _I] + [_L] * 9 + [_P, _P, _P] + [_L] * 3 + [_I] * 8 + [_P]),
+    "socket_block_lists": (_I, [_P, _L, _L, _P] + [_I] * 11 + [_P]),
 }
 
 _lib = None

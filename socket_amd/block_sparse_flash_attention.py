@@ -3,8 +3,9 @@
 Counterpart of kernels/block_sparse_flash_attention.py (index builders :11-274,
 Triton kernel `random_walk_fwd` :280-367, launcher :370-437, convenience wrapper
 :440-453) with the same function names, arguments and results.  The index
-builders are host-side tensor logic and stay in torch; the attention itself is
-one HIP kernel of libsocket_hip (`socket_block_sparse_attention`) -- there is no
+builders are one HIP launch for float32 scores on the device (`socket_block_lists`)
+and torch operations for other types, on the host and for very long rows; the attention
+itself is one HIP kernel of libsocket_hip (`socket_block_sparse_attention`) -- there is no
 other route, a missing library raises.
 
 How a block list comes about (both builders): every row block has a set of
@@ -22,17 +23,52 @@ sorted ascending (tests check it against a literal restatement of the pipeline).
 """
 from __future__ import annotations
 
+import functools
 from typing import Optional
 
 import torch
 import torch.nn.functional as F
 
-from ._lib import check, dtype_enum, lib, ptr, stream_ptr
+from ._lib import check, dtype_enum, lib, plain_tensors, ptr, stream_ptr
 
 __all__ = [
     "random_walk_indices", "random_walk_indices_from_block_probs", "expand_block_index_to_heads",
     "block_mask_to_indices", "random_walk_sparse_attention", "build_and_run_rw_sparse_attn",
 ]
+
+
+LIST_MAX_BLOCKS, LIST_MAX_PICKS = 4096, 256      # what one launch takes; longer lists are sorted by torch
+
+
+@functools.lru_cache(maxsize=256)
+def _most_forced(R: int, C: int, block_m: int, block_n: int, Tq: int, causal: bool, diagonal: bool, window: int) -> int:
+    """The largest number of forced blocks any row has (a function of the shape alone)."""
+    most = 0
+    for r in range(R):
+        d = r * block_m // block_n
+        last = min(C - 1, min((r + 1) * block_m - 1, Tq - 1) // block_n) if causal else C - 1
+        lo, hi = (max(0, d - (window - 1)), min(d, last)) if window > 0 else (1, 0)
+        rest = {0} | ({min(d, C - 1)} if diagonal else set())
+        most = max(most, max(0, hi - lo + 1) + sum(c <= last and not lo <= c <= hi for c in rest))
+    return most
+
+
+def _lists(scores: torch.Tensor, K: int, block_m: int, block_n: int, Tq: int, causal: bool, diagonal: bool,
+           window: Optional[int]) -> Optional[torch.Tensor]:
+    """`_assemble` as one launch, for float32 scores on the device; None for what it does not take."""
+    B, R, C = scores.shape
+    k = min(K, C)
+    if not (scores.is_cuda and scores.dtype == torch.float32 and 0 < C <= LIST_MAX_BLOCKS and k <= LIST_MAX_PICKS and 0 < B <= 65535
+            and R > 0 and (R + 1) * block_m < 2 ** 31 and plain_tensors(scores)):
+        return None
+    w = 0 if window is None else max(0, int(window))
+    scores = scores if scores.stride(2) == 1 else scores.contiguous()
+    out = torch.empty((B, R, k), dtype=torch.int32, device=scores.device)
+    slots = _most_forced(R, C, block_m, block_n, Tq, bool(causal), bool(diagonal), min(w, R * block_m // block_n + 1)) + k
+    check("socket_block_lists", lib().socket_block_lists(
+        ptr(scores), scores.stride(0), scores.stride(1), ptr(out), B, R, C, k, slots, block_m, block_n, Tq, int(bool(causal)),
+        int(bool(diagonal)), min(w, 2 ** 30), stream_ptr(scores.device)))
+    return out
 
 
 def _assemble(scores: torch.Tensor, valid: torch.Tensor, forced: torch.Tensor, K: int,
@@ -80,6 +116,9 @@ def random_walk_indices(random_walk_probs: torch.Tensor, block_m: int, block_n: 
     R, C = -(-T_q // block_m), -(-T_k // block_n)
     x = F.pad(random_walk_probs, (0, C * block_n - T_k, 0, R * block_m - T_q))
     scores = x.view(B, R, block_m, C, block_n).sum(dim=(2, 4))
+    out = _lists(scores, K, block_m, block_n, T_q, enforce_causal_blocks, force_include_diagonal, window_blocks)
+    if out is not None:
+        return out
     rows = torch.arange(R, device=device)
     cols = torch.arange(C, device=device)
     if enforce_causal_blocks:
@@ -109,6 +148,9 @@ def random_walk_indices_from_block_probs(random_walk_probs_blk: torch.Tensor, K:
     assert random_walk_probs_blk.dim() == 3
     B, R, C = random_walk_probs_blk.shape
     assert K > 0
+    out = _lists(random_walk_probs_blk, K, 1, 1, R, enforce_causal_blocks, force_include_diagonal, window_blocks)
+    if out is not None:
+        return out
     device = random_walk_probs_blk.device
     rows = torch.arange(R, device=device)
     cols = torch.arange(C, device=device)
@@ -188,8 +230,8 @@ def random_walk_sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tens
     q, k, v = (t if t.stride(-1) == 1 else t.contiguous() for t in (q, k, v))
     block_index = block_index.contiguous()
     seqlens = seqlens.contiguous()
-    out = torch.zeros((B, H, T, D), dtype=q.dtype, device=q.device)
-    check("socket_block_sparse_attention", lib().socket_block_sparse_attention(
+    out = torch.empty((B, H, T, D), dtype=q.dtype, device=q.device)
+    check("socket_block_sparse_attention", lib().socket_block_sparse_attention_cleared(
         ptr(q), ptr(k), ptr(v), dtype_enum(q.dtype),
         q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
         v.stride(0), v.stride(1), v.stride(2), ptr(seqlens), ptr(block_index), ptr(out),

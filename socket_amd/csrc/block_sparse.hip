@@ -24,7 +24,7 @@
 // 8-byte reads: rows of 72 elements, the sixteen 4-key groups of a row placed at
 // group ^ (dim / 8 % 16), which keeps both the transposing stores and the
 // fragment reads at the two LDS passes their 512 bytes need.
-#include "socket_common.h"
+#include "mma_tiles.h"
 
 namespace {
 
@@ -94,35 +94,198 @@ __device__ __forceinline__ float bs_xor32(float v, bool upper_half) {
   return __uint_as_float(upper_half ? r[0] : r[1]);
 }
 
+// Zeros into rows [from, to) of an output head.
+template <int D>
+__device__ __forceinline__ void bs_clear_rows(uint16_t* out, int64_t stride, int from, int to) {
+  for (int i = threadIdx.x; i < (to - from) * (D / 4); i += kBsThreads)
+    *reinterpret_cast<uint2*>(out + (int64_t)(from + i / (D / 4)) * stride + i % (D / 4) * 4) = make_uint2(0, 0);
+}
+
+// The row block and head of this workgroup.  Workgroups are dealt to the 8 XCDs round-robin by linear
+// id.  Renumbered so that each XCD walks one contiguous eighth of the (head, row block) space in
+// order: neighbouring row blocks share their window tiles, which then come from that XCD's L2 instead
+// of being fetched once per XCD.
+__device__ __forceinline__ void bs_place(int num_rows, int& start_m, int& bh) {
+  start_m = blockIdx.x;
+  bh = blockIdx.y;
+  const int64_t total = (int64_t)gridDim.x * gridDim.y;
+  if (total % 8 == 0) {
+    const int64_t n = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+    const int64_t id = (n % 8) * (total / 8) + n / 8;
+    start_m = (int)(id % num_rows);
+    bh = (int)(id / num_rows);
+  }
+}
+
+// Head widths of 64 and 128.  Two waves share a half of the row block (32 rows each) and take the
+// upper and the lower 32 keys of every listed block, with a softmax of their own that is merged at
+// the end; products, tile copies and the reads of V are the prompt attention's (mma_tiles.h).  The
+// next block's K and V are copied into the other stage of LDS while this one is worked on, without
+// registers: a list of eight blocks is bound by the delivery of its tiles (114 flop per byte), and
+// the kernel below, which asked for a tile when it wanted it, waited a memory latency for each.
+template <class DT, int D>
+__global__ __launch_bounds__(kBsThreads, 2) void block_sparse_tiles_kernel(
+    const uint16_t* __restrict__ q_, const uint16_t* __restrict__ k_, const uint16_t* __restrict__ v_,
+    int64_t q_sb, int64_t q_sh, int64_t q_sm, int64_t k_sb, int64_t k_sh, int64_t k_sn, int64_t v_sb,
+    int64_t v_sh, int64_t v_sn, const int32_t* __restrict__ seqlens, const int32_t* __restrict__ block_index,
+    uint16_t* __restrict__ out, int64_t o_sb, int64_t o_sh, int64_t o_sm, int H, int T, int num_rows, int klist,
+    int num_cols, float scale_log2, int clear_past) {
+  static_assert(kBsBlock == kPaKeys && kBsThreads == 64 * kPaWaves, "a listed block is one tile");
+  constexpr int CH = D / 8, KS = D / 16, DB = D / 32, kTile = kPaKeys * D * 2, kStage = 2 * kTile;
+  extern __shared__ __attribute__((aligned(16))) unsigned char bs_lds[];
+  int start_m, bh;
+  bs_place(num_rows, start_m, bh);
+  const int b = bh / H, h = bh % H;
+  const int seqlen = min(seqlens[b], T);
+  if (clear_past) bs_clear_rows<D>(out + b * o_sb + h * o_sh, o_sm, max(seqlen, start_m * kBsBlock), min(T, (start_m + 1) * kBsBlock));
+  if (start_m * kBsBlock >= seqlen) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, half = lane >> 5, rows_of = wave & 1, keys_of = wave >> 1;
+  const int row0 = start_m * kBsBlock + 32 * rows_of, row = row0 + col;      // (the row is the N index of every product)
+  const bool row_ok = row < seqlen;
+
+  const uint16_t* qb = q_ + b * q_sb + h * q_sh;
+  const char* kb = (const char*)(k_ + b * k_sb + h * k_sh);
+  const char* vb = (const char*)(v_ + b * v_sb + h * v_sh);
+  uint4 qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+    qf[ks] = row_ok ? *reinterpret_cast<const uint4*>(qb + (int64_t)row * q_sm + 16 * ks + 8 * half) : make_uint4(0, 0, 0, 0);
+  // (the fragments must have arrived before the first copy is issued, see prompt_attend.hip)
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(qf[ks].x), "v"(qf[ks].y), "v"(qf[ks].z), "v"(qf[ks].w));
+
+  const int32_t* blocks = block_index + ((int64_t)bh * num_rows + start_m) * klist;
+  auto first_of = [&](int j) __attribute__((always_inline)) {   // (the lists hold valid ids; a stray one must not fault)
+    return __builtin_amdgcn_readfirstlane(min(max(blocks[j], 0), num_cols - 1)) * kBsBlock;
+  };
+  const int64_t far = 1 << 24;      // (strides that 32-bit offsets inside a tile cannot span)
+  auto copy_block = [&](int first, int stage) __attribute__((always_inline)) {
+    unsigned char* st = bs_lds + stage * kStage;
+    if (first + kBsBlock <= seqlen && k_sn >= 0 && k_sn < far && v_sn >= 0 && v_sn < far) {
+      pa_copy_tile<CH>(kb + (int64_t)first * k_sn * 2, k_sn * 2, st, wave, lane);
+      pa_copy_tile<CH>(vb + (int64_t)first * v_sn * 2, v_sn * 2, st + kTile, wave, lane);
+    } else {                        // keys past the sequence are copies of its last (masked below)
+      pa_copy_rows<CH>([&](int key) { return kb + (int64_t)min(first + key, seqlen - 1) * k_sn * 2; }, st, wave, lane);
+      pa_copy_rows<CH>([&](int key) { return vb + (int64_t)min(first + key, seqlen - 1) * v_sn * 2; }, st + kTile, wave, lane);
+    }
+  };
+
+  pa_f32x16 o[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) o[db] = pa_f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  float l = 0.f, m = -INFINITY;
+  const int k_at = (32 * keys_of + col) * CH, k_swz = pa_swizzle<CH>(col);
+
+  int next = first_of(0);
+  copy_block(next, 0);
+  for (int j = 0; j < klist; ++j) {
+    const int start_n = next;
+    if (j + 1 < klist) next = first_of(j + 1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();     // this block has landed for every wave, the other stage has been consumed
+    if (j + 1 < klist) copy_block(next, (j + 1) & 1);
+    const int key0 = start_n + 32 * keys_of;
+    if (key0 > row0 + 31 || row0 >= seqlen) continue;     // (wave-uniform: nothing visible)
+    const uint4* kt = reinterpret_cast<const uint4*>(bs_lds + (j & 1) * kStage);
+    const unsigned char* vt = bs_lds + (j & 1) * kStage + kTile;
+
+    pa_f32x16 s = pa_f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) s = PaType<DT>::mfma(kt[k_at + ((2 * ks + half) ^ k_swz)], qf[ks], s);
+    // register i: key key0 + 8 (i / 4) + 4 half + i % 4
+    if (!(key0 + 31 <= row0 && row0 + 31 < seqlen)) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (!(row_ok && key0 + 4 * half + 8 * (i >> 2) + (i & 3) <= row)) s[i] = -INFINITY;
+    }
+    float mb = s[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mb = fmaxf(mb, s[i]);
+    mb = fmaxf(mb, lane_xor32(mb)) * scale_log2;
+    // (accumulators rescaled when a maximum has grown by more than 2^8, and large scores: see prompt_attend.hip)
+    if (__builtin_amdgcn_ballot_w64(mb > m + 8.f || (m == -INFINITY && mb > m)) != 0) {
+      const float mn = fmaxf(m, mb);
+      const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
+    }
+    const float shift = m == -INFINITY ? 0.f : m;
+    if (__builtin_amdgcn_ballot_w64(fabsf(shift) > 1048576.f) == 0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], scale_log2, -shift));
+        l += s[i];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        s[i] = __builtin_amdgcn_exp2f(pa_scaled_minus(s[i], scale_log2, shift));
+        l += s[i];
+      }
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      uint4 p;
+      uint32_t* w = &p.x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = PaType<DT>::pack2(s[8 * kk + 2 * i], s[8 * kk + 2 * i + 1]);
+#pragma unroll
+      for (int db = 0; db < DB; ++db) o[db] = PaType<DT>::mfma(pa_values<CH>(vt, 32 * keys_of + 16 * kk, db, lane), p, o[db]);
+    }
+  }
+
+  // merge the two key halves of a row half through LDS
+  l += lane_xor32(l);
+  __syncthreads();
+  float* mine = reinterpret_cast<float*>(bs_lds) + rows_of * (DB * 16 + 2) * 64 + lane;
+  if (keys_of == 1) {
+    mine[0] = m;
+    mine[64] = l;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mine[(2 + db * 16 + i) * 64] = o[db][i];
+  }
+  __syncthreads();
+  if (keys_of == 1 || !row_ok) return;
+  const float m1 = mine[0], top = fmaxf(m, m1);
+  const float a0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - top), a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - top);
+  const float inv = 1.f / (l * a0 + mine[64] * a1 + 1e-9f);
+  uint16_t* orow = out + b * o_sb + h * o_sh + (int64_t)row * o_sm;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+      float x[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = (o[db][i + e] * a0 + mine[(2 + db * 16 + i + e) * 64] * a1) * inv;
+      *reinterpret_cast<uint2*>(orow + db * 32 + 2 * i + 4 * half) = make_uint2(PaType<DT>::pack2(x[0], x[1]), PaType<DT>::pack2(x[2], x[3]));
+    }
+}
+
 template <class DT, int D>
 __global__ __launch_bounds__(kBsThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void block_sparse_fwd_kernel(
     const uint16_t* __restrict__ q_, const uint16_t* __restrict__ k_, const uint16_t* __restrict__ v_,
     int64_t q_sb, int64_t q_sh, int64_t q_sm, int64_t k_sb, int64_t k_sh, int64_t k_sn, int64_t v_sb,
     int64_t v_sh, int64_t v_sn, const int32_t* __restrict__ seqlens, const int32_t* __restrict__ block_index,
     uint16_t* __restrict__ out, int64_t o_sb, int64_t o_sh, int64_t o_sm, int H, int T, int num_rows, int klist,
-    int num_cols, float scale_log2) {
+    int num_cols, float scale_log2, int clear_past) {
   constexpr int CH = D / 8;                 // 16-byte chunks per row
   constexpr int KS = (D + 31) / 32;         // k-steps of the first product
   constexpr int DB = D / 16;                // 16-dim blocks of the output
   __shared__ __attribute__((aligned(16))) uint4 k_lds[kBsBlock * CH];
   __shared__ __attribute__((aligned(16))) uint16_t vt_lds[D * kBsVtStride];
 
-  // Workgroups are dealt to the 8 XCDs round-robin by linear id.  Renumbered so
-  // that each XCD walks one contiguous eighth of the (head, row block) space in
-  // order: neighbouring row blocks share their window tiles, which then come from
-  // that XCD's L2 instead of being fetched once per XCD.
-  int start_m = blockIdx.x, bh = blockIdx.y;
-  {
-    const int64_t total = (int64_t)gridDim.x * gridDim.y;
-    if (total % 8 == 0) {
-      const int64_t n = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-      const int64_t id = (n % 8) * (total / 8) + n / 8;
-      start_m = (int)(id % num_rows);
-      bh = (int)(id / num_rows);
-    }
-  }
+  int start_m, bh;
+  bs_place(num_rows, start_m, bh);
   const int b = bh / H, h = bh % H;
   const int seqlen = min(seqlens[b], T);
+  if (clear_past) bs_clear_rows<D>(out + b * o_sb + h * o_sh, o_sm, max(seqlen, start_m * kBsBlock), min(T, (start_m + 1) * kBsBlock));
   if (start_m * kBsBlock >= seqlen) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int prow = lane & 15, quarter = lane >> 4;
@@ -309,23 +472,114 @@ __global__ __launch_bounds__(kBsThreads) __attribute__((amdgpu_waves_per_eu(4, 4
   }
 }
 
+// ---- block lists ---------------------------------------------------------------------------------
+//
+// One wave per row of block scores: the forced blocks (block 0, the diagonal, the window behind it), the K
+// best-scoring other causal blocks, and the closed form of the reference's de-duplication: with U the
+// distinct chosen blocks, n_slots - |U| + 1 zeros (at most K), then the smallest members of U up to K
+// entries, and one zero makes way for the diagonal.  A lane keeps N scores of its own (columns lane, lane +
+// 64, ...) as ordered integers in registers and 64 columns of the chosen set as bits; a pick is a
+// wave maximum over (score, lower column first).  In place of some sixty torch launches, sorts and a host
+// read among them: 330 us of a 32700-token call, now one launch of 10 us (512 rows of 512 blocks, K = 8).
+constexpr int kListWaves = 4;
+constexpr int kListMaxCols = 4096;     // bits of a wave's set: 64 lanes x 64
+
+// the score with a bonus for recent blocks, rounded operation by operation as torch evaluates it
+__device__ __forceinline__ float list_score(float score, int col, float inv_c) {
+#pragma clang fp contract(off)
+  const float x = (float)col * inv_c;
+  const float y = x * 1e-6f;
+  return score + y;
+}
+
+template <int N>
+__global__ __launch_bounds__(64 * kListWaves) void block_lists_kernel(const float* __restrict__ scores, int64_t sb, int64_t sr,
+                                                                      int32_t* __restrict__ out, int R, int C, int K, int n_slots,
+                                                                      int block_m, int block_n, int Tq, int causal, int diagonal,
+                                                                      int window) {
+  const int lane = threadIdx.x & 63, r = blockIdx.x * kListWaves + (threadIdx.x >> 6), b = blockIdx.y;
+  if (r >= R) return;                    // (wave-uniform; no barrier below)
+  const int d = r * block_m / block_n, diag = min(d, C - 1);
+  const int last = causal ? min(C - 1, min((r + 1) * block_m - 1, Tq - 1) / block_n) : C - 1;      // last valid block
+  const int w0 = window > 0 ? max(0, d - (window - 1)) : 1, w1 = window > 0 ? d : 0;
+  auto forced = [&](int c) { return c == 0 || (diagonal && c == diag) || (c >= w0 && c <= w1); };
+  const float inv_c = 1.f / (float)C;
+
+  uint32_t key[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    const int c = e * 64 + lane;
+    key[e] = 0;
+    if (c <= last && !forced(c)) key[e] = score_to_key(list_score(scores[b * sb + r * sr + c], c, inv_c));
+  }
+  uint64_t set = 0;                      // chosen blocks 64 lane .. + 63
+  for (int i = 0; i < 64; ++i) {
+    const int c = lane * 64 + i;
+    if (c <= last && forced(c)) set |= 1ull << i;
+  }
+  const uint32_t none = score_to_key(-INFINITY);      // (a score of -inf is no candidate)
+  for (int k = 0; k < K; ++k) {
+    uint32_t best = 0;
+    int at = 0;
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+      if (key[e] > best) {
+        best = key[e];
+        at = e;
+      }
+    uint64_t v = ((uint64_t)best << 32) | (uint32_t)~(at * 64 + lane);
+#pragma unroll
+    for (int step = 32; step > 0; step >>= 1) {
+      const uint64_t o = __shfl_xor((unsigned long long)v, step, 64);
+      v = o > v ? o : v;
+    }
+    if ((uint32_t)(v >> 32) <= none) break;            // (wave-uniform)
+    const int c = (int)~(uint32_t)v;
+    if (lane == c >> 6) set |= 1ull << (c & 63);
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+      if (e * 64 + lane == c) key[e] = 0;
+  }
+  int distinct = __popcll(set);
+#pragma unroll
+  for (int step = 32; step > 0; step >>= 1) distinct += __shfl_xor(distinct, step, 64);
+  const int zeros = min(K, n_slots - distinct + 1), keep = K - zeros, lead = zeros - (diagonal ? 1 : 0);
+  if (lane == 0) set &= ~1ull;
+  const int mine = __popcll(set), before = wave_incl_scan(mine) - mine;
+  int32_t* row = out + ((int64_t)b * R + r) * K;
+  for (int i = lane; i < lead; i += 64) row[i] = 0;
+  int below = 0;                         // members under the diagonal
+  for (int i = 0, rank = before; i < 64; ++i) {
+    if (!((set >> i) & 1)) continue;
+    const int c = lane * 64 + i;
+    if (rank < keep) {
+      row[lead + rank + (diagonal && c >= diag ? 1 : 0)] = c;
+      if (c < diag) ++below;
+    }
+    ++rank;
+  }
+#pragma unroll
+  for (int step = 32; step > 0; step >>= 1) below += __shfl_xor(below, step, 64);
+  if (diagonal && lane == 0) row[lead + below] = diag;
+}
+
 template <class DT>
 int launch_block_sparse(const void* q, const void* k, const void* v, int64_t q_sb, int64_t q_sh, int64_t q_sm,
                         int64_t k_sb, int64_t k_sh, int64_t k_sn, int64_t v_sb, int64_t v_sh, int64_t v_sn,
                         const int32_t* seqlens, const int32_t* block_index, void* out, int64_t o_sb, int64_t o_sh,
-                        int64_t o_sm, int B, int H, int T, int D, int num_rows, int klist, hipStream_t s) {
+                        int64_t o_sm, int B, int H, int T, int D, int num_rows, int klist, int clear_past, hipStream_t s) {
   const int num_cols = (T + kBsBlock - 1) / kBsBlock;
   const float scale_log2 = 1.44269504f / sqrtf((float)D);
   const dim3 grid(num_rows, B * H);
-#define SOCKET_BS(DD)                                                                                        \
-  hipLaunchKernelGGL((block_sparse_fwd_kernel<DT, DD>), grid, dim3(kBsThreads), 0, s, (const uint16_t*)q,    \
+#define SOCKET_BS(KERN, LDS)                                                                                 \
+  hipLaunchKernelGGL(KERN, grid, dim3(kBsThreads), LDS, s, (const uint16_t*)q,                               \
                      (const uint16_t*)k, (const uint16_t*)v, q_sb, q_sh, q_sm, k_sb, k_sh, k_sn, v_sb, v_sh, \
                      v_sn, seqlens, block_index, (uint16_t*)out, o_sb, o_sh, o_sm, H, T, num_rows, klist,    \
-                     num_cols, scale_log2)
-  if (D == 128) SOCKET_BS(128);
-  else if (D == 64) SOCKET_BS(64);
-  else if (D == 32) SOCKET_BS(32);
-  else SOCKET_BS(16);
+                     num_cols, scale_log2, clear_past)
+  if (D == 128) SOCKET_BS((block_sparse_tiles_kernel<DT, 128>), 4 * kPaKeys * 128 * 2);
+  else if (D == 64) SOCKET_BS((block_sparse_tiles_kernel<DT, 64>), 4 * kPaKeys * 64 * 2);
+  else if (D == 32) SOCKET_BS((block_sparse_fwd_kernel<DT, 32>), 0);
+  else SOCKET_BS((block_sparse_fwd_kernel<DT, 16>), 0);
 #undef SOCKET_BS
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
@@ -333,14 +587,14 @@ int launch_block_sparse(const void* q, const void* k, const void* v, int64_t q_s
 
 }  // namespace
 
-extern "C" int socket_block_sparse_attention(const void* q, const void* k, const void* v, int dtype,
+static int block_sparse_run(const void* q, const void* k, const void* v, int dtype,
                                              int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_m,
                                              int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n,
                                              int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_n,
                                              const int32_t* seqlens, const int32_t* block_index, void* out,
                                              int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_m, int B,
                                              int H, int T, int D, int num_rows, int klist, int block_m,
-                                             int block_n, void* stream) {
+                                             int block_n, int clear_past, void* stream) {
   SOCKET_REQUIRE(q && k && v && seqlens && block_index && out, SOCKET_ERR_NULL);
   SOCKET_REQUIRE(dtype == SOCKET_BF16 || dtype == SOCKET_F16, SOCKET_ERR_UNSUPPORTED);
   SOCKET_REQUIRE(D == 16 || D == 32 || D == 64 || D == 128, SOCKET_ERR_UNSUPPORTED);
@@ -357,8 +611,43 @@ extern "C" int socket_block_sparse_attention(const void* q, const void* k, const
   if (dtype == SOCKET_BF16)
     return launch_block_sparse<DType_bf16>(q, k, v, q_stride_b, q_stride_h, q_stride_m, k_stride_b, k_stride_h,
                                            k_stride_n, v_stride_b, v_stride_h, v_stride_n, seqlens, block_index,
-                                           out, o_stride_b, o_stride_h, o_stride_m, B, H, T, D, num_rows, klist, s);
+                                           out, o_stride_b, o_stride_h, o_stride_m, B, H, T, D, num_rows, klist,
+                                           clear_past, s);
   return launch_block_sparse<DType_f16>(q, k, v, q_stride_b, q_stride_h, q_stride_m, k_stride_b, k_stride_h,
                                         k_stride_n, v_stride_b, v_stride_h, v_stride_n, seqlens, block_index, out,
-                                        o_stride_b, o_stride_h, o_stride_m, B, H, T, D, num_rows, klist, s);
+                                        o_stride_b, o_stride_h, o_stride_m, B, H, T, D, num_rows, klist,
+                                           clear_past, s);
+}
+
+#define SOCKET_BS_ARGS                                                                                                      \
+  const void *q, const void *k, const void *v, int dtype, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_m,       \
+      int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n, int64_t v_stride_b, int64_t v_stride_h,                   \
+      int64_t v_stride_n, const int32_t *seqlens, const int32_t *block_index, void *out, int64_t o_stride_b,                \
+      int64_t o_stride_h, int64_t o_stride_m, int B, int H, int T, int D, int num_rows, int klist, int block_m, int block_n
+#define SOCKET_BS_PASS                                                                                                      \
+  q, k, v, dtype, q_stride_b, q_stride_h, q_stride_m, k_stride_b, k_stride_h, k_stride_n, v_stride_b, v_stride_h,           \
+      v_stride_n, seqlens, block_index, out, o_stride_b, o_stride_h, o_stride_m, B, H, T, D, num_rows, klist, block_m, block_n
+extern "C" int socket_block_sparse_attention(SOCKET_BS_ARGS, void* stream) { return block_sparse_run(SOCKET_BS_PASS, 0, stream); }
+extern "C" int socket_block_sparse_attention_cleared(SOCKET_BS_ARGS, void* stream) { return block_sparse_run(SOCKET_BS_PASS, 1, stream); }
+#undef SOCKET_BS_ARGS
+#undef SOCKET_BS_PASS
+
+extern "C" int socket_block_lists(const float* scores, int64_t stride_b, int64_t stride_r, int32_t* out, int B, int R, int C, int K,
+                                  int n_slots, int block_m, int block_n, int Tq, int causal, int diagonal, int window, void* stream) {
+  SOCKET_REQUIRE(scores && out, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(B > 0 && B <= 65535 && R > 0 && C > 0 && K > 0 && K <= C && n_slots >= K && block_m > 0 && block_n > 0 && Tq > 0,
+                 SOCKET_ERR_SHAPE);
+  SOCKET_REQUIRE((int64_t)(R + 1) * block_m < INT32_MAX, SOCKET_ERR_SHAPE);
+  SOCKET_REQUIRE(C <= kListMaxCols, SOCKET_ERR_UNSUPPORTED);
+  const dim3 grid((unsigned)((R + kListWaves - 1) / kListWaves), (unsigned)B), block(64 * kListWaves);
+  hipStream_t s = (hipStream_t)stream;
+#define SOCKET_LISTS(N)                                                                                                    \
+  hipLaunchKernelGGL((block_lists_kernel<N>), grid, block, 0, s, scores, stride_b, stride_r, out, R, C, K, n_slots, block_m, \
+                     block_n, Tq, causal, diagonal, window)
+  if (C <= 256) SOCKET_LISTS(4);
+  else if (C <= 1024) SOCKET_LISTS(16);
+  else SOCKET_LISTS(64);
+#undef SOCKET_LISTS
+  SOCKET_LAUNCH_CHECK();
+  return SOCKET_OK;
 }

@@ -21,101 +21,12 @@
 // chunk_attend.hip's kernel): 32 heads over 8 kv heads of 128, cap 30, 8000 tokens 835 against 1209 us
 // (628 TFLOP/s); 32 heads of 128 + 64 shared dims, 8000 tokens 864 against 1849 us (759); without a cap
 // 6001 tokens 475 us (621), with weights rounded to 16 bits 325 us (909).
-#include "elem.h"
+#include "mma_tiles.h"
 
 namespace {
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 pa_bf16x8;
-typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 pa_f16x8;
-typedef float pa_f32x16 __attribute__((ext_vector_type(16)));
-typedef short pa_s16x4 __attribute__((ext_vector_type(4)));
-
-template <class DT>
-struct PaType;
-template <>
-struct PaType<DType_bf16> {
-  static __device__ __forceinline__ pa_f32x16 mfma(const uint4& a, const uint4& b, pa_f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(pa_bf16x8, a), __builtin_bit_cast(pa_bf16x8, b), c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{lo, hi}, bf2));
-  }
-  static __device__ __forceinline__ float low(uint32_t w) { return __uint_as_float(w << 16); }
-  static __device__ __forceinline__ float high(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-};
-template <>
-struct PaType<DType_f16> {
-  static __device__ __forceinline__ pa_f32x16 mfma(const uint4& a, const uint4& b, pa_f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(pa_f16x8, a), __builtin_bit_cast(pa_f16x8, b), c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{lo, hi}, h2));
-  }
-  static __device__ __forceinline__ float low(uint32_t w) { return f16_bits_to_f32((uint16_t)(w & 0xffffu)); }
-  static __device__ __forceinline__ float high(uint32_t w) { return f16_bits_to_f32((uint16_t)(w >> 16)); }
-};
-
-constexpr int kPaKeys = 64;      // keys of a tile
-constexpr int kPaWaves = 4;
 constexpr int kPaRows = 32 * kPaWaves;
-constexpr float kPaLog2e = 1.4426950408889634f;
 constexpr float kPaMaxCap = 60.f;   // exp(60) * 2^31 keys < 3.4e38, exp(-60) > 1.2e-38
-
-// x * c rounded, then less m: not contracted, so that the largest score gives exactly zero.
-__device__ __forceinline__ float pa_scaled_minus(float x, float c, float m) {
-#pragma clang fp contract(off)
-  const float y = x * c;
-  return y - m;
-}
-
-// Where a row's 16-byte pieces go (CH of them): piece ^ pa_swizzle(key).  Sixteen keys at one piece
-// must fall on sixteen 16-byte bank groups (rows of 128 bytes start half a bank line apart by the
-// key's parity), and the four keys x 64 bytes of a transposing read on all of them.
-template <int CH>
-__device__ __forceinline__ int pa_swizzle(int key) {
-  if constexpr (CH == 16) return ((key & 3) << 2) | ((key >> 2) & 3);
-  else return (((key >> 1) & 1) << 2) | (((key >> 2) & 1) << 1) | ((key >> 3) & 1);
-}
-
-// 16 bytes per lane from base + off into LDS (see lds_dma16); `base` is the same for the whole wave.
-__device__ __forceinline__ void pa_dma16(const char* base, uint32_t off, void* lds_dst) {
-  const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds_dst);
-  uint32_t saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %3\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(off), "s"(at), "s"(base)
-      : "memory");
-}
-
-// A tile of CH-piece rows into LDS: wave `wave` of kPaWaves issues its share of the copies.  row(key)
-// tells where a key's row starts, or the rows are `stride` bytes apart from `first` on.
-template <int CH, class ROW>
-__device__ __forceinline__ void pa_copy_rows(ROW row, unsigned char* tile, int wave, int lane) {
-  constexpr int N = kPaKeys * CH / 64 / kPaWaves;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const int s = (wave * N + i) * 64 + lane, key = s / CH, piece = s % CH ^ pa_swizzle<CH>(key);
-    lds_dma16(row(key) + piece * 16, tile + (wave * N + i) * 1024);
-  }
-}
-template <int CH>
-__device__ __forceinline__ void pa_copy_tile(const char* first, int64_t stride, unsigned char* tile, int wave, int lane) {
-  constexpr int N = kPaKeys * CH / 64 / kPaWaves;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const int s = (wave * N + i) * 64 + lane, key = s / CH, piece = s % CH ^ pa_swizzle<CH>(key);
-    pa_dma16(first, (uint32_t)(key * (int)stride + piece * 16), tile + (wave * N + i) * 1024);
-  }
-}
 
 // D: key dims, D2: dims of a second key segment that all heads share (with it the output may be gated),
 // DV: value dims.  SPLIT: weights enter the second product as a sum of two 16-bit numbers.  CAPPED:
@@ -216,10 +127,7 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
     }
   };
 
-  // Fragment addresses: K row `col` of a 32-key block, piece 2 ks + half; V: lane i of a group of 16
-  // names key i / 4 and dims 4 (i % 4), groups are (dims 0-15 | 16-31) x (keys 0-3 | 4-7).
-  const int k_swz = pa_swizzle<CK>(col);
-  const int v_key = 4 * half + ((lane >> 2) & 3), v_piece = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1), v_byte = (lane & 1) * 8;
+  const int k_swz = pa_swizzle<CK>(col);      // (of K row `col` of a 32-key block)
 
   if (end > 0) copy_keys(0, 0);
   int stage = 0;
@@ -321,15 +229,7 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
       }
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        pa_s16x4 v[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const int key = 16 * kk + 8 * e + v_key;
-          const int at = key * CV * 16 + (((4 * db + v_piece) ^ pa_swizzle<CV>(key)) << 4) + v_byte;
-          v[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pa_s16x4*)(vt + at));
-        }
-        const uint2 v0 = __builtin_bit_cast(uint2, v[0]), v1 = __builtin_bit_cast(uint2, v[1]);
-        const uint4 vf = make_uint4(v0.x, v0.y, v1.x, v1.y);
+        const uint4 vf = pa_values<CV>(vt, 16 * kk, db, lane);
         o[db] = PaType<DT>::mfma(vf, ph, o[db]);
         if constexpr (SPLIT) o[db] = PaType<DT>::mfma(vf, pl, o[db]);
       }
