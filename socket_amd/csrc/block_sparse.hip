@@ -117,22 +117,24 @@ __device__ __forceinline__ void bs_place(int num_rows, int& start_m, int& bh) {
   }
 }
 
-// Head widths of 64 and 128.  Two waves share a half of the row block (32 rows each) and take the
-// upper and the lower 32 keys of every listed block, with a softmax of their own that is merged at
-// the end; products, tile copies and the reads of V are the prompt attention's (mma_tiles.h).  The
-// next block's K and V are copied into the other stage of LDS while this one is worked on, without
-// registers: a list of eight blocks is bound by the delivery of its tiles (114 flop per byte), and
-// the kernel below, which asked for a tile when it wanted it, waited a memory latency for each.
+// Head widths of 64 and 128: the same products with K and V tiles copied from global memory straight
+// into LDS (mma_tiles.h) and V^T fragments by transposing reads, so that no lane spends registers or
+// vector operations on staging.  A workgroup holds one tile of each at a time (32 KB); four of them
+// share a CU, and while one waits for its tiles the others work.  32700 tokens x 32 heads x 8 random
+// blocks: 450 us, 41 us per listed block (the register-staged form: 498), the same with every block
+// in the L2, so what bounds it is the chain of a tile -- copy, product, softmax, product -- at four waves
+// a SIMD.  Slower: 32x32 products with two waves sharing rows and merging key halves (505), a ring of
+// five tiles ahead (550), persistent workgroups that prefetch the next row block (580).
 template <class DT, int D>
-__global__ __launch_bounds__(kBsThreads, 2) void block_sparse_tiles_kernel(
+__global__ __launch_bounds__(kBsThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void block_sparse_tiles_kernel(
     const uint16_t* __restrict__ q_, const uint16_t* __restrict__ k_, const uint16_t* __restrict__ v_,
     int64_t q_sb, int64_t q_sh, int64_t q_sm, int64_t k_sb, int64_t k_sh, int64_t k_sn, int64_t v_sb,
     int64_t v_sh, int64_t v_sn, const int32_t* __restrict__ seqlens, const int32_t* __restrict__ block_index,
     uint16_t* __restrict__ out, int64_t o_sb, int64_t o_sh, int64_t o_sm, int H, int T, int num_rows, int klist,
     int num_cols, float scale_log2, int clear_past) {
   static_assert(kBsBlock == kPaKeys && kBsThreads == 64 * kPaWaves, "a listed block is one tile");
-  constexpr int CH = D / 8, KS = D / 16, DB = D / 32, kTile = kPaKeys * D * 2, kStage = 2 * kTile;
-  extern __shared__ __attribute__((aligned(16))) unsigned char bs_lds[];
+  constexpr int CH = D / 8, KS = D / 32, DB = D / 16, kTile = kPaKeys * D * 2;
+  __shared__ __attribute__((aligned(16))) unsigned char tiles[2 * kTile];
   int start_m, bh;
   bs_place(num_rows, start_m, bh);
   const int b = bh / H, h = bh % H;
@@ -140,68 +142,64 @@ __global__ __launch_bounds__(kBsThreads, 2) void block_sparse_tiles_kernel(
   if (clear_past) bs_clear_rows<D>(out + b * o_sb + h * o_sh, o_sm, max(seqlen, start_m * kBsBlock), min(T, (start_m + 1) * kBsBlock));
   if (start_m * kBsBlock >= seqlen) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col = lane & 31, half = lane >> 5, rows_of = wave & 1, keys_of = wave >> 1;
-  const int row0 = start_m * kBsBlock + 32 * rows_of, row = row0 + col;      // (the row is the N index of every product)
+  const int prow = lane & 15, quarter = lane >> 4;
+  const int row0 = start_m * kBsBlock + wave * 16, row = row0 + prow;   // (the row is the N index of every product)
   const bool row_ok = row < seqlen;
 
   const uint16_t* qb = q_ + b * q_sb + h * q_sh;
   const char* kb = (const char*)(k_ + b * k_sb + h * k_sh);
   const char* vb = (const char*)(v_ + b * v_sb + h * v_sh);
+  const int32_t* blocks = block_index + ((int64_t)bh * num_rows + start_m) * klist;
+  constexpr int64_t far = 1 << 24;      // (strides that 32-bit offsets inside a tile cannot span)
+  auto copy_rows = [&](const char* rows, int64_t st, int first, unsigned char* at) __attribute__((always_inline)) {
+    if (first + kBsBlock <= seqlen && st >= 0 && st < far) pa_copy_tile<CH>(rows + first * st * 2, st * 2, at, wave, lane);
+    else pa_copy_rows<CH>([&](int r) { return rows + min(first + r, seqlen - 1) * st * 2; }, at, wave, lane);   // (past the end: the last key, masked)
+  };
+
   uint4 qf[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
-    qf[ks] = row_ok ? *reinterpret_cast<const uint4*>(qb + (int64_t)row * q_sm + 16 * ks + 8 * half) : make_uint4(0, 0, 0, 0);
-  // (the fragments must have arrived before the first copy is issued, see prompt_attend.hip)
+    qf[ks] = row_ok ? *reinterpret_cast<const uint4*>(qb + (int64_t)row * q_sm + 32 * ks + 8 * quarter) : make_uint4(0, 0, 0, 0);
+  bs_f32x4 o[DB];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(qf[ks].x), "v"(qf[ks].y), "v"(qf[ks].z), "v"(qf[ks].w));
+  for (int db = 0; db < DB; ++db) o[db] = bs_f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  const uint4* kt = reinterpret_cast<const uint4*>(tiles);
+  const int k_swz = pa_swizzle<CH>(prow);
+  // V: lane i of a quarter names key 4 quarter + i / 4 (of 16) and dims 4 (i % 4) .. + 3 of 16
+  const int v_key = 4 * quarter + (prow >> 2), v_swz = pa_swizzle<CH>(v_key);
+  const unsigned char* vt = tiles + kTile + v_key * CH * 16 + (prow & 1) * 8;
 
-  const int32_t* blocks = block_index + ((int64_t)bh * num_rows + start_m) * klist;
-  auto first_of = [&](int j) __attribute__((always_inline)) {   // (the lists hold valid ids; a stray one must not fault)
-    return __builtin_amdgcn_readfirstlane(min(max(blocks[j], 0), num_cols - 1)) * kBsBlock;
-  };
-  const int64_t far = 1 << 24;      // (strides that 32-bit offsets inside a tile cannot span)
-  auto copy_block = [&](int first, int stage) __attribute__((always_inline)) {
-    unsigned char* st = bs_lds + stage * kStage;
-    if (first + kBsBlock <= seqlen && k_sn >= 0 && k_sn < far && v_sn >= 0 && v_sn < far) {
-      pa_copy_tile<CH>(kb + (int64_t)first * k_sn * 2, k_sn * 2, st, wave, lane);
-      pa_copy_tile<CH>(vb + (int64_t)first * v_sn * 2, v_sn * 2, st + kTile, wave, lane);
-    } else {                        // keys past the sequence are copies of its last (masked below)
-      pa_copy_rows<CH>([&](int key) { return kb + (int64_t)min(first + key, seqlen - 1) * k_sn * 2; }, st, wave, lane);
-      pa_copy_rows<CH>([&](int key) { return vb + (int64_t)min(first + key, seqlen - 1) * v_sn * 2; }, st + kTile, wave, lane);
-    }
-  };
-
-  pa_f32x16 o[DB];
-#pragma unroll
-  for (int db = 0; db < DB; ++db) o[db] = pa_f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  float l = 0.f, m = -INFINITY;
-  const int k_at = (32 * keys_of + col) * CH, k_swz = pa_swizzle<CH>(col);
-
-  int next = first_of(0);
-  copy_block(next, 0);
   for (int j = 0; j < klist; ++j) {
-    const int start_n = next;
-    if (j + 1 < klist) next = first_of(j + 1);
+    const int start_n = __builtin_amdgcn_readfirstlane(min(max(blocks[j], 0), num_cols - 1)) * kBsBlock;   // (a stray id must not fault)
+    __syncthreads();  // the previous tiles have been consumed
+    copy_rows(kb, k_sn, start_n, tiles);
+    copy_rows(vb, v_sn, start_n, tiles + kTile);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();     // this block has landed for every wave, the other stage has been consumed
-    if (j + 1 < klist) copy_block(next, (j + 1) & 1);
-    const int key0 = start_n + 32 * keys_of;
-    if (key0 > row0 + 31 || row0 >= seqlen) continue;     // (wave-uniform: nothing visible)
-    const uint4* kt = reinterpret_cast<const uint4*>(bs_lds + (j & 1) * kStage);
-    const unsigned char* vt = bs_lds + (j & 1) * kStage + kTile;
+    __syncthreads();
+    if (start_n > row0 + 15 || row0 >= seqlen) continue;     // (wave-uniform: nothing visible)
 
-    pa_f32x16 s = pa_f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    // S^T = K . Q^T: register r of block nb is key nb * 16 + 4 * quarter + r against row `row`
+    bs_f32x4 s[4];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) s = PaType<DT>::mfma(kt[k_at + ((2 * ks + half) ^ k_swz)], qf[ks], s);
-    // register i: key key0 + 8 (i / 4) + 4 half + i % 4
-    if (!(key0 + 31 <= row0 && row0 + 31 < seqlen)) {
+    for (int nb = 0; nb < 4; ++nb) s[nb] = bs_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (!(row_ok && key0 + 4 * half + 8 * (i >> 2) + (i & 3) <= row)) s[i] = -INFINITY;
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) s[nb] = BsType<DT>::mfma(kt[(nb * 16 + prow) * CH + ((4 * ks + quarter) ^ k_swz)], qf[ks], s[nb]);
+    if (!(start_n + kBsBlock - 1 <= row0 && row0 + 15 < seqlen)) {
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (!(row_ok && start_n + nb * 16 + 4 * quarter + r <= row)) s[nb][r] = -INFINITY;
     }
-    float mb = s[0];
+    float mb = s[0][0];
 #pragma unroll
-    for (int i = 1; i < 16; ++i) mb = fmaxf(mb, s[i]);
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mb = fmaxf(mb, s[nb][r]);
+    mb = fmaxf(mb, lane_xor16(mb));
     mb = fmaxf(mb, lane_xor32(mb)) * scale_log2;
     // (accumulators rescaled when a maximum has grown by more than 2^8, and large scores: see prompt_attend.hip)
     if (__builtin_amdgcn_ballot_w64(mb > m + 8.f || (m == -INFINITY && mb > m)) != 0) {
@@ -212,60 +210,55 @@ __global__ __launch_bounds__(kBsThreads, 2) void block_sparse_tiles_kernel(
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
+        for (int r = 0; r < 4; ++r) o[db][r] *= alpha;
     }
     const float shift = m == -INFINITY ? 0.f : m;
     if (__builtin_amdgcn_ballot_w64(fabsf(shift) > 1048576.f) == 0) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], scale_log2, -shift));
-        l += s[i];
-      }
+      for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[nb][r] = __builtin_amdgcn_exp2f(fmaf(s[nb][r], scale_log2, -shift));
+          l += s[nb][r];
+        }
     } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        s[i] = __builtin_amdgcn_exp2f(pa_scaled_minus(s[i], scale_log2, shift));
-        l += s[i];
-      }
+      for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          s[nb][r] = __builtin_amdgcn_exp2f(pa_scaled_minus(s[nb][r], scale_log2, shift));
+          l += s[nb][r];
+        }
     }
+    // O^T += V^T . P^T, slots 0..3: keys 32c + 4q + r, slots 4..7: keys 32c + 16 + 4q + r
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
+    for (int c = 0; c < 2; ++c) {
       uint4 p;
-      uint32_t* w = &p.x;
+      p.x = BsType<DT>::pack2(s[2 * c][0], s[2 * c][1]);
+      p.y = BsType<DT>::pack2(s[2 * c][2], s[2 * c][3]);
+      p.z = BsType<DT>::pack2(s[2 * c + 1][0], s[2 * c + 1][1]);
+      p.w = BsType<DT>::pack2(s[2 * c + 1][2], s[2 * c + 1][3]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = PaType<DT>::pack2(s[8 * kk + 2 * i], s[8 * kk + 2 * i + 1]);
+      for (int db = 0; db < DB; ++db) {
+        uint2 v[2];
 #pragma unroll
-      for (int db = 0; db < DB; ++db) o[db] = PaType<DT>::mfma(pa_values<CH>(vt, 32 * keys_of + 16 * kk, db, lane), p, o[db]);
+        for (int e = 0; e < 2; ++e)      // (16 keys further on the pieces lie the same way)
+          v[e] = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pa_s16x4*)(
+              vt + (32 * c + 16 * e) * CH * 16 + (((2 * db + ((prow >> 1) & 1)) ^ v_swz) << 4))));
+        o[db] = BsType<DT>::mfma(make_uint4(v[0].x, v[0].y, v[1].x, v[1].y), p, o[db]);
+      }
     }
   }
 
-  // merge the two key halves of a row half through LDS
+  l += lane_xor16(l);
   l += lane_xor32(l);
-  __syncthreads();
-  float* mine = reinterpret_cast<float*>(bs_lds) + rows_of * (DB * 16 + 2) * 64 + lane;
-  if (keys_of == 1) {
-    mine[0] = m;
-    mine[64] = l;
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) mine[(2 + db * 16 + i) * 64] = o[db][i];
-  }
-  __syncthreads();
-  if (keys_of == 1 || !row_ok) return;
-  const float m1 = mine[0], top = fmaxf(m, m1);
-  const float a0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - top), a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - top);
-  const float inv = 1.f / (l * a0 + mine[64] * a1 + 1e-9f);
+  if (!row_ok) return;
+  const float inv = 1.f / (l + 1e-9f);
   uint16_t* orow = out + b * o_sb + h * o_sh + (int64_t)row * o_sm;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int i = 0; i < 16; i += 4) {
-      float x[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = (o[db][i + e] * a0 + mine[(2 + db * 16 + i + e) * 64] * a1) * inv;
-      *reinterpret_cast<uint2*>(orow + db * 32 + 2 * i + 4 * half) = make_uint2(PaType<DT>::pack2(x[0], x[1]), PaType<DT>::pack2(x[2], x[3]));
-    }
+    *reinterpret_cast<uint2*>(orow + db * 16 + 4 * quarter) =
+        make_uint2(BsType<DT>::pack2(o[db][0] * inv, o[db][1] * inv), BsType<DT>::pack2(o[db][2] * inv, o[db][3] * inv));
 }
 
 template <class DT, int D>
@@ -480,7 +473,7 @@ __global__ __launch_bounds__(kBsThreads) __attribute__((amdgpu_waves_per_eu(4, 4
 // entries, and one zero makes way for the diagonal.  A lane keeps N scores of its own (columns lane, lane +
 // 64, ...) as ordered integers in registers and 64 columns of the chosen set as bits; a pick is a
 // wave maximum over (score, lower column first).  In place of some sixty torch launches, sorts and a host
-// read among them: 330 us of a 32700-token call, now one launch of 10 us (512 rows of 512 blocks, K = 8).
+// read among them: 350 us of a 32700-token call, now one launch of 12.6 us (511 rows of 511 blocks, K = 8).
 constexpr int kListWaves = 4;
 constexpr int kListMaxCols = 4096;     // bits of a wave's set: 64 lanes x 64
 
@@ -490,6 +483,19 @@ __device__ __forceinline__ float list_score(float score, int col, float inv_c) {
   const float x = (float)col * inv_c;
   const float y = x * 1e-6f;
   return score + y;
+}
+
+// The largest x of the wave, in every lane (see wave_reduce_to_last).
+__device__ __forceinline__ uint32_t list_max(uint32_t x) {
+#define SOCKET_STEP(ctrl, rows) x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctrl, rows, 0xf, false));
+  SOCKET_STEP(0x111, 0xf)
+  SOCKET_STEP(0x112, 0xf)
+  SOCKET_STEP(0x114, 0xf)
+  SOCKET_STEP(0x118, 0xf)
+  SOCKET_STEP(0x142, 0xa)
+  SOCKET_STEP(0x143, 0xc)
+#undef SOCKET_STEP
+  return __builtin_amdgcn_readlane(x, 63);
 }
 
 template <int N>
@@ -512,11 +518,13 @@ __global__ __launch_bounds__(64 * kListWaves) void block_lists_kernel(const floa
     key[e] = 0;
     if (c <= last && !forced(c)) key[e] = score_to_key(list_score(scores[b * sb + r * sr + c], c, inv_c));
   }
-  uint64_t set = 0;                      // chosen blocks 64 lane .. + 63
-  for (int i = 0; i < 64; ++i) {
-    const int c = lane * 64 + i;
-    if (c <= last && forced(c)) set |= 1ull << i;
-  }
+  // chosen blocks 64 lane .. + 63, as bits: first the forced ones
+  auto bits = [&](int lo, int hi) -> uint64_t {      // of columns lo .. hi that are this lane's and valid
+    lo = max(lo - lane * 64, 0);
+    hi = min(min(hi, last) - lane * 64, 63);
+    return lo > hi ? 0 : (~0ull << lo) & (~0ull >> (63 - hi));
+  };
+  uint64_t set = bits(0, 0) | bits(w0, w1) | (diagonal ? bits(diag, diag) : 0);
   const uint32_t none = score_to_key(-INFINITY);      // (a score of -inf is no candidate)
   for (int k = 0; k < K; ++k) {
     uint32_t best = 0;
@@ -527,39 +535,30 @@ __global__ __launch_bounds__(64 * kListWaves) void block_lists_kernel(const floa
         best = key[e];
         at = e;
       }
-    uint64_t v = ((uint64_t)best << 32) | (uint32_t)~(at * 64 + lane);
-#pragma unroll
-    for (int step = 32; step > 0; step >>= 1) {
-      const uint64_t o = __shfl_xor((unsigned long long)v, step, 64);
-      v = o > v ? o : v;
-    }
-    if ((uint32_t)(v >> 32) <= none) break;            // (wave-uniform)
-    const int c = (int)~(uint32_t)v;
+    const uint32_t top = list_max(best);
+    if (top <= none) break;                            // (wave-uniform)
+    const int c = (int)~list_max(best == top ? ~(uint32_t)(at * 64 + lane) : 0u);      // the lowest column of that score
     if (lane == c >> 6) set |= 1ull << (c & 63);
+    if (lane == (c & 63)) {
 #pragma unroll
-    for (int e = 0; e < N; ++e)
-      if (e * 64 + lane == c) key[e] = 0;
+      for (int e = 0; e < N; ++e)
+        if (e == c >> 6) key[e] = 0;
+    }
   }
-  int distinct = __popcll(set);
-#pragma unroll
-  for (int step = 32; step > 0; step >>= 1) distinct += __shfl_xor(distinct, step, 64);
+  const int members = wave_incl_scan((int)__popcll(set));
+  const int distinct = __builtin_amdgcn_readlane(members, 63);
   const int zeros = min(K, n_slots - distinct + 1), keep = K - zeros, lead = zeros - (diagonal ? 1 : 0);
+  int rank = members - (int)__popcll(set) - (lane == 0 ? 0 : 1);      // (block 0 is always chosen and is no non-zero member)
   if (lane == 0) set &= ~1ull;
-  const int mine = __popcll(set), before = wave_incl_scan(mine) - mine;
   int32_t* row = out + ((int64_t)b * R + r) * K;
   for (int i = lane; i < lead; i += 64) row[i] = 0;
-  int below = 0;                         // members under the diagonal
-  for (int i = 0, rank = before; i < 64; ++i) {
-    if (!((set >> i) & 1)) continue;
-    const int c = lane * 64 + i;
-    if (rank < keep) {
-      row[lead + rank + (diagonal && c >= diag ? 1 : 0)] = c;
-      if (c < diag) ++below;
-    }
-    ++rank;
+  int below = 0;                         // kept members under the diagonal
+  for (; set != 0 && rank < keep; set &= set - 1, ++rank) {
+    const int c = lane * 64 + __ffsll((unsigned long long)set) - 1;
+    row[lead + rank + (diagonal && c >= diag ? 1 : 0)] = c;
+    if (c < diag) ++below;
   }
-#pragma unroll
-  for (int step = 32; step > 0; step >>= 1) below += __shfl_xor(below, step, 64);
+  below = __builtin_amdgcn_readlane(wave_incl_scan(below), 63);
   if (diagonal && lane == 0) row[lead + below] = diag;
 }
 
@@ -571,15 +570,15 @@ int launch_block_sparse(const void* q, const void* k, const void* v, int64_t q_s
   const int num_cols = (T + kBsBlock - 1) / kBsBlock;
   const float scale_log2 = 1.44269504f / sqrtf((float)D);
   const dim3 grid(num_rows, B * H);
-#define SOCKET_BS(KERN, LDS)                                                                                 \
-  hipLaunchKernelGGL(KERN, grid, dim3(kBsThreads), LDS, s, (const uint16_t*)q,                               \
+#define SOCKET_BS(KERN)                                                                                      \
+  hipLaunchKernelGGL(KERN, grid, dim3(kBsThreads), 0, s, (const uint16_t*)q,                                 \
                      (const uint16_t*)k, (const uint16_t*)v, q_sb, q_sh, q_sm, k_sb, k_sh, k_sn, v_sb, v_sh, \
                      v_sn, seqlens, block_index, (uint16_t*)out, o_sb, o_sh, o_sm, H, T, num_rows, klist,    \
                      num_cols, scale_log2, clear_past)
-  if (D == 128) SOCKET_BS((block_sparse_tiles_kernel<DT, 128>), 4 * kPaKeys * 128 * 2);
-  else if (D == 64) SOCKET_BS((block_sparse_tiles_kernel<DT, 64>), 4 * kPaKeys * 64 * 2);
-  else if (D == 32) SOCKET_BS((block_sparse_fwd_kernel<DT, 32>), 0);
-  else SOCKET_BS((block_sparse_fwd_kernel<DT, 16>), 0);
+  if (D == 128) SOCKET_BS((block_sparse_tiles_kernel<DT, 128>));
+  else if (D == 64) SOCKET_BS((block_sparse_tiles_kernel<DT, 64>));
+  else if (D == 32) SOCKET_BS((block_sparse_fwd_kernel<DT, 32>));
+  else SOCKET_BS((block_sparse_fwd_kernel<DT, 16>));
 #undef SOCKET_BS
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
