@@ -218,6 +218,16 @@ int socket_score_packed_grouped(const void* q_table, int q_dtype, const uint32_t
 int socket_soft_hash_collision(const float* q_probs, const int16_t* key_buckets,
                                const uint8_t* allowed, const float* v_hist, float* out,
                                int B, int H, int L, int R, int T, void* stream);
+/* The same with a table and value norms of any of the three types (widened to fp32, which changes no value). */
+int socket_soft_hash_collision_typed(const void* q_probs, int q_dtype, const int16_t* key_buckets, const uint8_t* allowed,
+                                     const void* v_hist, int v_dtype, float* out, int B, int H, int L, int R, int T,
+                                     void* stream);
+/* The list assembly of build_sparse_list_decode (GPT-FAST/kernels/sparse.py:62-95) around the `heavy` top-k entries that
+ * already stand at the end of each of `rows` rows: positions 0 .. sink - 1 and max(T - window, sink) .. T - 1 before them
+ * (T - 1 if that is none), -1 wherever allowed [rows,T] is false; list_len [rows] becomes the row's width. */
+int socket_finish_list(int32_t* list, int32_t* list_len, const uint8_t* allowed, int rows, int T, int sink, int window,
+                       int heavy, void* stream);
+
 
 /* fp16 variant: q_probs f16 [B,H,L,R], v_norm f16 [B,H,T], any L.
  * Replaces soft_hash_score, GPT-FAST/kernels/soft_hash_score/soft_hash_score_bindings.cpp:10-36

@@ -26,8 +26,19 @@ constexpr int kTokensPerThread = 8;
 constexpr int kAhead = 6;   // tables whose codes are in flight per lane
 constexpr size_t kCollideLdsSlack = 1024;
 
+struct Bf16Entry {
+  uint16_t bits;
+};
 __device__ __forceinline__ float entry_to_f32(float x) { return x; }
 __device__ __forceinline__ float entry_to_f32(uint16_t x) { return f16_bits_to_f32(x); }
+__device__ __forceinline__ float entry_to_f32(Bf16Entry x) { return bf16_bits_to_f32(x.bits); }
+
+// Value norm i of an array of any of the three types (widening changes no value).
+__device__ __forceinline__ float norm_at(const void* v, int dtype, int64_t i) {
+  if (dtype == SOCKET_F32) return ((const float*)v)[i];
+  const uint16_t u = ((const uint16_t*)v)[i];
+  return dtype == SOCKET_F16 ? f16_bits_to_f32(u) : bf16_bits_to_f32(u);
+}
 
 // ct: tables per LDS slice.  INLDS false: a single table exceeds LDS, gather from global memory.
 // VEC: rows are 16-byte aligned (T % 8 == 0 and aligned bases): 16-byte code loads.
@@ -41,7 +52,7 @@ __device__ __forceinline__ float entry_to_f32(uint16_t x) { return f16_bits_to_f
 template <typename QT, int THREADS, bool VEC, bool INLDS, bool STREAM>
 __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
     const QT* __restrict__ q_probs, const int16_t* __restrict__ key_buckets,
-    const uint8_t* __restrict__ allowed, const QT* __restrict__ v_hist, float* __restrict__ out,
+    const uint8_t* __restrict__ allowed, const void* __restrict__ v_hist, int v_dtype, float* __restrict__ out,
     int L, int R, int T, int ct, int chunks) {
   extern __shared__ __attribute__((aligned(16))) unsigned char collide_lds[];
   QT* table = reinterpret_cast<QT*>(collide_lds);
@@ -94,19 +105,15 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
       const uint2 aw = *reinterpret_cast<const uint2*>(allowed + o);
       const uint32_t ab[2] = {aw.x, aw.y};
       float vh[TPT];
-      if (sizeof(QT) == 4) {
-        const float4 v0 = *reinterpret_cast<const float4*>(v_hist + o);
-        const float4 v1 = *reinterpret_cast<const float4*>(v_hist + o + 4);
+      if (v_dtype == SOCKET_F32) {      // (uniform)
+        const float4 v0 = *reinterpret_cast<const float4*>((const float*)v_hist + o);
+        const float4 v1 = *reinterpret_cast<const float4*>((const float*)v_hist + o + 4);
         vh[0] = v0.x, vh[1] = v0.y, vh[2] = v0.z, vh[3] = v0.w;
         vh[4] = v1.x, vh[5] = v1.y, vh[6] = v1.z, vh[7] = v1.w;
       } else {
-        const uint4 w = *reinterpret_cast<const uint4*>(v_hist + o);
-        const uint32_t u[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          vh[2 * i] = f16_bits_to_f32((uint16_t)(u[i] & 0xffffu));
-          vh[2 * i + 1] = f16_bits_to_f32((uint16_t)(u[i] >> 16));
-        }
+        const uint4 w = *reinterpret_cast<const uint4*>((const uint16_t*)v_hist + o);
+        if (v_dtype == SOCKET_F16) unpack16<DType_f16>(w, vh);
+        else unpack16<DType_bf16>(w, vh);
       }
       float res[TPT];
 #pragma unroll
@@ -117,7 +124,7 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
     } else {
 #pragma unroll
       for (int i = 0; i < TPT; ++i) {
-        if (t0 + i < T) out[o + i] = allowed[o + i] ? sum[i] * entry_to_f32(v_hist[o + i]) : -INFINITY;
+        if (t0 + i < T) out[o + i] = allowed[o + i] ? sum[i] * norm_at(v_hist, v_dtype, o + i) : -INFINITY;
       }
     }
   };
@@ -185,7 +192,7 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
 
 template <typename QT>
 int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const uint8_t* allowed,
-                         const QT* v_hist, float* out, int B, int H, int L, int R, int T,
+                         const void* v_hist, int v_dtype, float* out, int B, int H, int L, int R, int T,
                          hipStream_t stream) {
   const SocketDeviceLimits& lim = socket_device_limits();
   const size_t per_table = (size_t)R * sizeof(QT);
@@ -198,10 +205,19 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
   }
   const size_t lds = (size_t)ct * per_table;
   const bool vec = T % 8 == 0 && (((uintptr_t)key_buckets | (uintptr_t)allowed | (uintptr_t)v_hist | (uintptr_t)out) & 15) == 0;
-  // short rows: a quarter of the threads, so that a tile is not mostly idle lanes
-  const bool small = T <= 256 * kTokensPerThread;
-  const int threads = small ? 256 : 1024;
-  const int tiles = (T + threads * kTokensPerThread - 1) / (threads * kTokensPerThread);
+  // The widest workgroup that still leaves one to every CU (each pulls the whole table through LDS, and its
+  // waves are all that a CU has in flight): 32 heads x 32768 tokens, L60 x R1024, 1024 lanes on half the CUs with
+  // an fp32 table in two slices 43.6 us, 512 lanes with the bf16 table in one 33.7.  Short rows take a quarter, so
+  // that a tile is not mostly idle lanes.
+  auto tiles_of = [&](int th) { return (T + th * kTokensPerThread - 1) / (th * kTokensPerThread); };
+  int threads = 256;
+  if (T > 256 * kTokensPerThread)
+    for (int th : {1024, 512})
+      if ((int64_t)tiles_of(th) * B * H >= lim.cu_count) {
+        threads = th;
+        break;
+      }
+  const int tiles = tiles_of(threads);
   // tiles per workgroup: as many as leave two workgroups per CU (they amortise the
   // slices a workgroup pulls through LDS), at most 8
   int chunks = (int)((int64_t)tiles * B * H / (2 * (int64_t)lim.cu_count));
@@ -222,7 +238,7 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
         granted.store(budget, std::memory_order_release);                                             \
       }                                                                                               \
     }                                                                                                 \
-    hipLaunchKernelGGL(kern, grid, dim3(TH), lds, stream, q_probs, key_buckets, allowed, v_hist, out, L, R, T, ct, chunks); \
+    hipLaunchKernelGGL(kern, grid, dim3(TH), lds, stream, q_probs, key_buckets, allowed, v_hist, v_dtype, out, L, R, T, ct, chunks); \
   } while (0)
 #define SOCKET_COLLIDE_V(TH, LD)         \
   do {                                   \
@@ -231,16 +247,33 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
     else SOCKET_COLLIDE(TH, false, LD, false);  \
   } while (0)
   if (ct > 0) {
-    if (small) SOCKET_COLLIDE_V(256, true);
+    if (threads == 256) SOCKET_COLLIDE_V(256, true);
+    else if (threads == 512) SOCKET_COLLIDE_V(512, true);
     else SOCKET_COLLIDE_V(1024, true);
   } else {
-    if (small) SOCKET_COLLIDE_V(256, false);
+    if (threads == 256) SOCKET_COLLIDE_V(256, false);
+    else if (threads == 512) SOCKET_COLLIDE_V(512, false);
     else SOCKET_COLLIDE_V(1024, false);
   }
 #undef SOCKET_COLLIDE_V
 #undef SOCKET_COLLIDE
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
+}
+
+// The rest of a row [sink | window | heavy] whose heavy entries are in place: the sink and window positions
+// (the last position if there are none), -1 for every position that is not allowed, and the length.
+__global__ __launch_bounds__(256) void finish_list_kernel(int32_t* __restrict__ list, int32_t* __restrict__ list_len,
+                                                          const uint8_t* __restrict__ allowed, int T, int sink, int window,
+                                                          int heavy) {
+  const int start = max(T - window, sink), nwin = window > 0 && start < T ? T - start : 0, base = sink + nwin > 0 ? sink + nwin : 1;
+  int32_t* row = list + (int64_t)blockIdx.x * (base + heavy);
+  const uint8_t* ok = allowed + (int64_t)blockIdx.x * T;
+  for (int i = threadIdx.x; i < base + heavy; i += 256) {
+    const int at = i >= base ? row[i] : sink + nwin == 0 ? T - 1 : i < sink ? i : start + (i - sink);
+    row[i] = ok[min(max(at, 0), T - 1)] ? at : -1;
+  }
+  if (threadIdx.x == 0) list_len[blockIdx.x] = base + heavy;
 }
 
 }  // namespace
@@ -251,8 +284,33 @@ extern "C" int socket_soft_hash_collision(const float* q_probs, const int16_t* k
   SOCKET_REQUIRE(q_probs && key_buckets && allowed && v_hist && out, SOCKET_ERR_NULL);
   SOCKET_REQUIRE(B > 0 && H > 0 && L > 0 && R > 0 && T > 0, SOCKET_ERR_SHAPE);
   SOCKET_REQUIRE((int64_t)B * H <= 65535, SOCKET_ERR_SHAPE);
-  return launch_collision_i16<float>(q_probs, key_buckets, allowed, v_hist, out, B, H, L, R, T,
+  return launch_collision_i16<float>(q_probs, key_buckets, allowed, v_hist, SOCKET_F32, out, B, H, L, R, T,
                                      (hipStream_t)stream);
+}
+
+extern "C" int socket_soft_hash_collision_typed(const void* q_probs, int q_dtype, const int16_t* key_buckets,
+                                                const uint8_t* allowed, const void* v_hist, int v_dtype, float* out,
+                                                int B, int H, int L, int R, int T, void* stream) {
+  SOCKET_REQUIRE(q_probs && key_buckets && allowed && v_hist && out, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(socket_dtype_bytes(q_dtype) != 0 && socket_dtype_bytes(v_dtype) != 0, SOCKET_ERR_UNSUPPORTED);
+  SOCKET_REQUIRE(B > 0 && H > 0 && L > 0 && R > 0 && T > 0, SOCKET_ERR_SHAPE);
+  SOCKET_REQUIRE((int64_t)B * H <= 65535, SOCKET_ERR_SHAPE);
+  hipStream_t s = (hipStream_t)stream;
+  if (q_dtype == SOCKET_F32)
+    return launch_collision_i16<float>((const float*)q_probs, key_buckets, allowed, v_hist, v_dtype, out, B, H, L, R, T, s);
+  if (q_dtype == SOCKET_F16)
+    return launch_collision_i16<uint16_t>((const uint16_t*)q_probs, key_buckets, allowed, v_hist, v_dtype, out, B, H, L, R, T, s);
+  return launch_collision_i16<Bf16Entry>((const Bf16Entry*)q_probs, key_buckets, allowed, v_hist, v_dtype, out, B, H, L, R, T, s);
+}
+
+extern "C" int socket_finish_list(int32_t* list, int32_t* list_len, const uint8_t* allowed, int rows, int T, int sink, int window,
+                                  int heavy, void* stream) {
+  SOCKET_REQUIRE(list && list_len && allowed, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(rows > 0 && T > 0 && sink >= 0 && window >= 0 && sink <= T && window <= T && heavy >= 0, SOCKET_ERR_SHAPE);
+  hipLaunchKernelGGL(finish_list_kernel, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, list, list_len, allowed, T, sink,
+                     window, heavy);
+  SOCKET_LAUNCH_CHECK();
+  return SOCKET_OK;
 }
 
 extern "C" int socket_soft_hash_score_f16(const uint16_t* q_probs, const int16_t* key_buckets,
@@ -261,6 +319,6 @@ extern "C" int socket_soft_hash_score_f16(const uint16_t* q_probs, const int16_t
   SOCKET_REQUIRE(q_probs && key_buckets && allowed && v_norm && out, SOCKET_ERR_NULL);
   SOCKET_REQUIRE(B > 0 && H > 0 && L > 0 && R > 0 && T > 0, SOCKET_ERR_SHAPE);
   SOCKET_REQUIRE((int64_t)B * H <= 65535, SOCKET_ERR_SHAPE);
-  return launch_collision_i16<uint16_t>(q_probs, key_buckets, allowed, v_norm, out, B, H, L, R, T,
+  return launch_collision_i16<uint16_t>(q_probs, key_buckets, allowed, v_norm, SOCKET_F16, out, B, H, L, R, T,
                                         (hipStream_t)stream);
 }

@@ -16,7 +16,7 @@ import collections
 
 import torch
 
-from ._lib import SOCKET_TOPK_MAX_M, check, lib, ptr, stream_ptr
+from ._lib import SOCKET_TOPK_MAX_M, check, dtype_enum, lib, ptr, stream_ptr
 from .socket_kernels import (  # noqa: F401  (re-exported, as in the reference module)
     attention_mask_to_allowed_prob,
     sparse_attention_fwd,
@@ -114,6 +114,16 @@ def select_list(scores: torch.Tensor, sink: int, window: int, M: int, *, lens=No
     sparse_len = torch.empty((B, H), dtype=torch.int32, device=scores.device)
     if list_width == 0:
         return sparse_list, sparse_len.zero_()
+    _select_into(scores, sink, window, M, lens, budgets, write_base, row_range, split, sparse_list, sparse_len)
+    return sparse_list, sparse_len
+
+
+def _select_into(scores, sink: int, window: int, M: int, lens, budgets, write_base: bool, row_range, split: bool,
+                 sparse_list: torch.Tensor, sparse_len: torch.Tensor) -> None:
+    """The selection's launch into the rows of `sparse_list` [B,H,width] (any stride between rows)."""
+    B, H, T = scores.shape
+    width = sparse_list.shape[2]
+    assert sparse_list.stride(2) == 1 and sparse_list.stride(0) == H * sparse_list.stride(1)
     L = lib()
     ws, ws_bytes = None, L.socket_select_workspace_bytes(B, H, T, M) if split else 0
     if ws_bytes:
@@ -122,12 +132,38 @@ def select_list(scores: torch.Tensor, sink: int, window: int, M: int, *, lens=No
         check("socket_select_list", L.socket_select_list(
             ptr(scores), scores.stride(1), ptr(lens), ptr(budgets), ptr(row_range),
             0 if row_range is None else row_range.shape[2], B, H, T, M, int(sink), int(window),
-            1 if write_base else 0, ptr(sparse_list), list_width, list_width, ptr(sparse_len),
+            1 if write_base else 0, ptr(sparse_list), sparse_list.stride(1), width, ptr(sparse_len),
             ptr(ws), ws_bytes, stream_ptr(scores.device)))
     except RuntimeError:
         if ws is not None:
             reset_select_workspaces()
         raise
+
+
+def _build_in_place(q_probs, k_hard, v_norm, allowed, sink: int, window: int, M: int):
+    """`build_sparse_list_decode` in three launches: scores from the operands in their own types, the top-k straight
+    into the list, and the positions and -1 entries around it.  None for operands it does not take."""
+    B, H, L, R = q_probs.shape
+    T = k_hard.shape[3]
+    types = (torch.float16, torch.bfloat16, torch.float32)
+    if (min(B, H, T, L, R, M) < 1 or B * H > 65535 or v_norm.dtype not in types or k_hard.dtype != torch.int16
+            or tuple(k_hard.shape[:2]) != (B, H) or tuple(v_norm.shape) != (B, H, T) or tuple(allowed.shape) != (B, H, T)
+            or not all(t.device == q_probs.device for t in (k_hard, v_norm, allowed))):
+        return None
+    if M > SOCKET_TOPK_MAX_M:
+        raise RuntimeError(f"top-k budget {M} exceeds the supported maximum {SOCKET_TOPK_MAX_M}")
+    q_probs, k_hard, v_norm, allowed = (t.contiguous() for t in (q_probs, k_hard, v_norm, allowed))
+    sink, window = max(0, min(sink, T)), max(0, min(window, T))
+    base = max(1, sink + (T - max(T - window, sink) if window > 0 else 0))
+    scores = torch.empty((B, H, T), dtype=torch.float32, device=q_probs.device)
+    sparse_list = torch.empty((B, H, base + M), dtype=torch.int32, device=q_probs.device)
+    sparse_len = torch.empty((B, H), dtype=torch.int32, device=q_probs.device)
+    s = stream_ptr(q_probs.device)
+    check("socket_soft_hash_collision", lib().socket_soft_hash_collision_typed(
+        ptr(q_probs), dtype_enum(q_probs.dtype), ptr(k_hard), ptr(allowed), ptr(v_norm), dtype_enum(v_norm.dtype), ptr(scores),
+        B, H, L, R, T, s))
+    _select_into(scores, 0, 0, M, None, None, False, None, True, sparse_list[:, :, base:], sparse_len)
+    check("socket_finish_list", lib().socket_finish_list(ptr(sparse_list), ptr(sparse_len), ptr(allowed), B * H, T, sink, window, M, s))
     return sparse_list, sparse_len
 
 
@@ -155,6 +191,10 @@ def build_sparse_list_decode(
     assert L2 == L
     device = q_probs.device
     M_eff = min(M, T)
+    built = _build_in_place(q_probs, k_hard_bhlt if k_hard_bhlt.dtype == torch.int16 else k_hard_bhlt.to(torch.int16),
+                            v_norm_bht, allowed_bht, int(sink), int(window), int(M_eff))
+    if built is not None:
+        return built
     if M_eff > 0:
         ext = _get_soft_hash_ext()
         q_probs_f32 = q_probs.float().unsqueeze(2).contiguous()
