@@ -47,10 +47,10 @@ __device__ __forceinline__ void store16<DType_f32>(void* base, int64_t idx, cons
 template <>
 __device__ __forceinline__ void store16<DType_bf16>(void* base, int64_t idx, const float* v) {
   uint4 w;
-  w.x = (uint32_t)f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16);
-  w.y = (uint32_t)f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16);
-  w.z = (uint32_t)f32_to_bf16_bits(v[4]) | ((uint32_t)f32_to_bf16_bits(v[5]) << 16);
-  w.w = (uint32_t)f32_to_bf16_bits(v[6]) | ((uint32_t)f32_to_bf16_bits(v[7]) << 16);
+  w.x = f32x2_to_bf16_bits(v[0], v[1]);
+  w.y = f32x2_to_bf16_bits(v[2], v[3]);
+  w.z = f32x2_to_bf16_bits(v[4], v[5]);
+  w.w = f32x2_to_bf16_bits(v[6], v[7]);
   *reinterpret_cast<uint4*>((uint16_t*)base + idx) = w;
 }
 template <>

@@ -44,7 +44,7 @@ __device__ __forceinline__ void store_vec(void* p, int64_t i, const float* v) {
     uint32_t w[N / 2];
 #pragma unroll
     for (int k = 0; k < N / 2; ++k)
-      w[k] = (uint32_t)f32_to_bf16_bits(v[2 * k]) | ((uint32_t)f32_to_bf16_bits(v[2 * k + 1]) << 16);
+      w[k] = f32x2_to_bf16_bits(v[2 * k], v[2 * k + 1]);
     if constexpr (N == 8) *reinterpret_cast<uint4*>((uint16_t*)p + i) = make_uint4(w[0], w[1], w[2], w[3]);
     else *reinterpret_cast<uint2*>((uint16_t*)p + i) = make_uint2(w[0], w[1]);
   }

@@ -56,10 +56,10 @@ __device__ __forceinline__ uint4 load_frag8<DType_f32>(const float* p) {
   const float4 a = *reinterpret_cast<const float4*>(p);
   const float4 c = *reinterpret_cast<const float4*>(p + 4);
   uint4 r;
-  r.x = (uint32_t)f32_to_bf16_bits(a.x) | ((uint32_t)f32_to_bf16_bits(a.y) << 16);
-  r.y = (uint32_t)f32_to_bf16_bits(a.z) | ((uint32_t)f32_to_bf16_bits(a.w) << 16);
-  r.z = (uint32_t)f32_to_bf16_bits(c.x) | ((uint32_t)f32_to_bf16_bits(c.y) << 16);
-  r.w = (uint32_t)f32_to_bf16_bits(c.z) | ((uint32_t)f32_to_bf16_bits(c.w) << 16);
+  r.x = f32x2_to_bf16_bits(a.x, a.y);
+  r.y = f32x2_to_bf16_bits(a.z, a.w);
+  r.z = f32x2_to_bf16_bits(c.x, c.y);
+  r.w = f32x2_to_bf16_bits(c.z, c.w);
   return r;
 }
 template <>
@@ -68,10 +68,10 @@ __device__ __forceinline__ uint4 load_frag8<DType_f16>(const uint16_t* p) {
   float f[8];
   unpack16<DType_f16>(raw, f);
   uint4 r;
-  r.x = (uint32_t)f32_to_bf16_bits(f[0]) | ((uint32_t)f32_to_bf16_bits(f[1]) << 16);
-  r.y = (uint32_t)f32_to_bf16_bits(f[2]) | ((uint32_t)f32_to_bf16_bits(f[3]) << 16);
-  r.z = (uint32_t)f32_to_bf16_bits(f[4]) | ((uint32_t)f32_to_bf16_bits(f[5]) << 16);
-  r.w = (uint32_t)f32_to_bf16_bits(f[6]) | ((uint32_t)f32_to_bf16_bits(f[7]) << 16);
+  r.x = f32x2_to_bf16_bits(f[0], f[1]);
+  r.y = f32x2_to_bf16_bits(f[2], f[3]);
+  r.z = f32x2_to_bf16_bits(f[4], f[5]);
+  r.w = f32x2_to_bf16_bits(f[6], f[7]);
   return r;
 }
 

@@ -86,8 +86,8 @@ __device__ __forceinline__ void sh_store4<DType_f32>(void* p, int64_t i, const f
 template <>
 __device__ __forceinline__ void sh_store4<DType_bf16>(void* p, int64_t i, const float (&v)[4]) {
   *reinterpret_cast<uint2*>((uint16_t*)p + i) =
-      make_uint2((uint32_t)f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16),
-                 (uint32_t)f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16));
+      make_uint2(f32x2_to_bf16_bits(v[0], v[1]),
+                 f32x2_to_bf16_bits(v[2], v[3]));
 }
 template <>
 __device__ __forceinline__ void sh_store4<DType_f16>(void* p, int64_t i, const float (&v)[4]) {
@@ -366,8 +366,8 @@ __device__ __forceinline__ void soft_hash_block(
             *reinterpret_cast<float4*>((float*)out + o) = make_float4(lg[g][0], lg[g][1], lg[g][2], lg[g][3]);
           } else {
             uint2 w;
-            w.x = (uint32_t)f32_to_bf16_bits(lg[g][0]) | ((uint32_t)f32_to_bf16_bits(lg[g][1]) << 16);
-            w.y = (uint32_t)f32_to_bf16_bits(lg[g][2]) | ((uint32_t)f32_to_bf16_bits(lg[g][3]) << 16);
+            w.x = f32x2_to_bf16_bits(lg[g][0], lg[g][1]);
+            w.y = f32x2_to_bf16_bits(lg[g][2], lg[g][3]);
             *reinterpret_cast<uint2*>((uint16_t*)out + o) = w;
           }
         }
@@ -394,7 +394,7 @@ __device__ __forceinline__ void soft_hash_block(
             uint32_t w[2 * W];
 #pragma unroll
             for (int c = 0; c < 2 * W; ++c)
-              w[c] = (uint32_t)f32_to_bf16_bits(v[2 * c]) | ((uint32_t)f32_to_bf16_bits(v[2 * c + 1]) << 16);
+              w[c] = f32x2_to_bf16_bits(v[2 * c], v[2 * c + 1]);
             uint16_t* dst = (uint16_t*)out + o;
             if constexpr (W == 4) {
               *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
@@ -549,7 +549,7 @@ __global__ __launch_bounds__(kSHThreads) void decode_prologue_kernel(
         for (int j = 0; j < 4; ++j) {
           float re, im;
           rotate_pair(x[2 * j], x[2 * j + 1], f[ks][2 * j], f[ks][2 * j + 1], re, im);
-          o[j] = (uint32_t)f32_to_bf16_bits(re) | ((uint32_t)f32_to_bf16_bits(im) << 16);
+          o[j] = f32x2_to_bf16_bits(re, im);
         }
         kf[ks].u = make_uint4(o[0], o[1], o[2], o[3]);
       } else {
