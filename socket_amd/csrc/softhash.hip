@@ -86,14 +86,273 @@ __device__ __forceinline__ void sh_store4<DType_f32>(void* p, int64_t i, const f
 template <>
 __device__ __forceinline__ void sh_store4<DType_bf16>(void* p, int64_t i, const float (&v)[4]) {
   *reinterpret_cast<uint2*>((uint16_t*)p + i) =
-      make_uint2(f32x2_to_bf16_bits(v[0], v[1]),
-                 f32x2_to_bf16_bits(v[2], v[3]));
+      make_uint2(f32x2_to_bf16_bits(v[0], v[1]), f32x2_to_bf16_bits(v[2], v[3]));
 }
 template <>
 __device__ __forceinline__ void sh_store4<DType_f16>(void* p, int64_t i, const float (&v)[4]) {
   *reinterpret_cast<uint2*>((uint16_t*)p + i) =
       make_uint2((uint32_t)f32_to_f16_bits(v[0]) | ((uint32_t)f32_to_f16_bits(v[1]) << 16),
                  (uint32_t)f32_to_f16_bits(v[2]) | ((uint32_t)f32_to_f16_bits(v[3]) << 16));
+}
+
+// ---------------------------------------------------------------------------
+// bf16 queries and planes of 128 dims, K = 10, R = 1024 (whatever the group): both products on the
+// matrix cores, sixteen heads of one table to a workgroup.
+//
+//   proj^T[plane, head] = planes . q^T          v_mfma_f32_16x16x32_bf16, exact products, fp32 sums
+//   logit^T[bucket, head] = protos . t          t in three bf16 terms (hi, mid, lo: all 24 bits), so that
+//                                               two products of 16 x 16 x 32 keep what fp32 keeps
+// In both the head is the N index: lane x holds head x % 16 in all its registers, the planes of lane
+// quarter q are 4 q .. + 3, and the terms a lane splits off its own projections are the operand it
+// has to supply.  Bucket order inside a product is free: block ii of a 64-bucket chunk takes buckets
+// 4 m + ii for row m, so that a lane's prototypes are runs of four (8-byte loads) and its results runs of
+// sixteen.  A wave has 256 buckets; maxima and sums meet in 512 bytes of LDS.  Logits are made in
+// base-2 units (log2 e goes into t) for the hardware's exponential.
+// The scalar form below spends ten multiply-adds and a library exponential per (head, bucket) and is bound by
+// the vector ALU: with it the decode prologue takes 23 us for 4 x 32 heads x 60 tables and 56 us for
+// 16 x 28 x 48; with this one 13 us and 25 us, and 7.7 us instead of 10.4 us for one sequence of 32 x 60
+// (dependent trips to memory and a launch).
+//
+// W: heads of a unit (the scorer's grouped layout [unit, L, R, W]; 1 for the reference's [B,Hq,L,R], whose
+// units are heads).  OT: float or uint16_t (bf16).  FT: void, or the element type of a rotary table, as above.
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 sh_bf16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float sh_f32x4;
+union ShFrag {
+  uint4 u;
+  sh_bf16x8 v;
+};
+__device__ __forceinline__ sh_f32x4 sh_mfma(const uint4& a, const uint4& b, sh_f32x4 c) {
+  ShFrag x, y;
+  x.u = a;
+  y.u = b;
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.v, y.v, c, 0, 0, 0);
+}
+__device__ __forceinline__ uint32_t sh_dpp_xor1(uint32_t x) { return __builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, false); }
+__device__ __forceinline__ uint32_t sh_dpp_xor2(uint32_t x) { return __builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, false); }
+
+// eight consecutive table entries (cos, sin of four pairs) as floats
+template <class FT>
+__device__ __forceinline__ void sh_load8(const void* p, int64_t i, float (&o)[8]);
+template <>
+__device__ __forceinline__ void sh_load8<DType_bf16>(const void* p, int64_t i, float (&o)[8]) {
+  unpack16<DType_bf16>(*reinterpret_cast<const uint4*>((const uint16_t*)p + i), o);
+}
+template <>
+__device__ __forceinline__ void sh_load8<DType_f32>(const void* p, int64_t i, float (&o)[8]) {
+  const float4 a = *reinterpret_cast<const float4*>((const float*)p + i);
+  const float4 c = *reinterpret_cast<const float4*>((const float*)p + i + 4);
+  o[0] = a.x, o[1] = a.y, o[2] = a.z, o[3] = a.w, o[4] = c.x, o[5] = c.y, o[6] = c.z, o[7] = c.w;
+}
+
+constexpr int kMxHeads = 16, kMxD = 128, kMxK = 10, kMxR = 1024;
+
+// Which heads the units are: `parts` units of W heads to a kv head's G (0: a unit is a head of Hq).
+struct MxUnits {
+  int count, parts, Hq, Hkv, G;
+};
+
+template <class FT, int W, class OT>
+__device__ __forceinline__ void soft_hash_mx_block(const int l, const int group, const MxUnits& units, const uint16_t* __restrict__ q,
+                                                   int64_t q_sb, int64_t q_sh, const uint16_t* __restrict__ planes,
+                                                   const uint16_t* __restrict__ protos_T, OT* __restrict__ out, int L, float scale,
+                                                   const void* __restrict__ freqs, const int64_t* __restrict__ pos, int pos_stride,
+                                                   int64_t n_pos, uint16_t* __restrict__ q_out) {
+  constexpr bool kRope = !std::is_void<FT>::value;
+  __shared__ float red[2][kSHWaves][kMxHeads];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 15, quarter = lane >> 4;
+  const int unit = group * (kMxHeads / W) + n / W;
+  const bool in_units = unit < units.count;
+  const int u = in_units ? unit : 0;
+  const int per_seq = units.parts > 0 ? units.Hkv * units.parts : units.Hq;
+  const int b = u / per_seq, at = u % per_seq;
+  const int member = units.parts > 0 ? at % units.parts * W + n % W : 0;       // of the kv head's group
+  const bool live = in_units && (units.parts == 0 || member < units.G);
+  const int head = units.parts > 0 ? at / units.parts * units.G + (live ? member : 0) : at;
+
+  // everything is asked for first: queries, angles, planes, prototypes
+  const uint16_t* qrow = q + b * q_sb + head * q_sh;
+  int64_t p = 0;
+  bool turn = false;
+  if constexpr (kRope) {
+    p = pos[(int64_t)b * pos_stride];
+    turn = p >= 0 && p < n_pos;
+  }
+  uint4 qf[4], pl[4];
+  uint2 pr[4][4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    qf[ks] = *reinterpret_cast<const uint4*>(qrow + 32 * ks + 8 * quarter);
+    pl[ks] = *reinterpret_cast<const uint4*>(planes + ((int64_t)l * kMxK + min(n, kMxK - 1)) * kMxD + 32 * ks + 8 * quarter);
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      pr[c][r] = *reinterpret_cast<const uint2*>(protos_T + min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c + 4 * n);
+  if (quarter >= 2) {         // (no prototype past the tenth: zeros, whatever the tenth is)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * quarter + r >= kMxK) pr[c][r] = make_uint2(0, 0);
+  }
+  if constexpr (kRope) {
+    // (angles of row 0 for a position outside the table: a load under a condition is waited for at once)
+    float f[4][8];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) sh_load8<FT>(freqs, (turn ? p : 0) * kMxD + 32 * ks + 8 * quarter, f[ks]);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (turn) {
+        float x[8];
+        unpack16<DType_bf16>(qf[ks], x);
+        uint32_t w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          float re, im;
+          rotate_pair(x[2 * j], x[2 * j + 1], f[ks][2 * j], f[ks][2 * j + 1], re, im);
+          w[j] = f32x2_to_bf16_bits(re, im);
+        }
+        qf[ks] = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+      if (l == 0 && wave == 0 && live)
+        *reinterpret_cast<uint4*>(q_out + ((int64_t)b * units.Hq + head) * kMxD + 32 * ks + 8 * quarter) = qf[ks];
+    }
+  }
+
+  // register r: plane 4 quarter + r of head n (planes past the tenth repeat it and are dropped)
+  sh_f32x4 proj = sh_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) proj = sh_mfma(pl[ks], qf[ks], proj);
+  float hi[4], mid[4], lo[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float t = 4 * quarter + r < kMxK ? tanhf(proj[r]) * scale : 0.f;
+    hi[r] = sh_round<DType_bf16>(t);
+    mid[r] = sh_round<DType_bf16>(t - hi[r]);
+    lo[r] = t - hi[r] - mid[r];
+  }
+  const uint4 t_high = make_uint4(f32x2_to_bf16_bits(hi[0], hi[1]), f32x2_to_bf16_bits(hi[2], hi[3]),
+                                  f32x2_to_bf16_bits(mid[0], mid[1]), f32x2_to_bf16_bits(mid[2], mid[3]));
+  const uint4 t_low = make_uint4(f32x2_to_bf16_bits(lo[0], lo[1]), f32x2_to_bf16_bits(lo[2], lo[3]), 0, 0);
+
+  // lg[c][ii][r]: bucket 256 wave + 64 c + 4 (4 quarter + r) + ii of head n
+  sh_f32x4 lg[4][4];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) {
+      const uint32_t sel = (ii & 1) ? 0x07060302u : 0x05040100u;
+      auto word = [&](int r) { return ii < 2 ? pr[c][r].x : pr[c][r].y; };
+      const uint32_t a0 = __builtin_amdgcn_perm(word(1), word(0), sel), a1 = __builtin_amdgcn_perm(word(3), word(2), sel);
+      lg[c][ii] = sh_mfma(make_uint4(a0, a1, 0, 0), t_low, sh_f32x4{0.f, 0.f, 0.f, 0.f});
+      lg[c][ii] = sh_mfma(make_uint4(a0, a1, a0, a1), t_high, lg[c][ii]);
+    }
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, lg[c][ii][r]);
+  mx = fmaxf(mx, lane_xor16(mx));
+  mx = fmaxf(mx, lane_xor32(mx));
+  if (quarter == 0) red[0][wave][n] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(red[0][0][n], red[0][1][n]), fmaxf(red[0][2][n], red[0][3][n]));
+  float sum = 0.f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        lg[c][ii][r] = __builtin_amdgcn_exp2f(lg[c][ii][r] - mx);
+        sum += lg[c][ii][r];
+      }
+  sum += lane_xor16(sum);
+  sum += lane_xor32(sum);
+  if (quarter == 0) red[1][wave][n] = sum;
+  __syncthreads();
+  sum = (red[1][0][n] + red[1][1][n]) + (red[1][2][n] + red[1][3][n]);
+  const float inv = live ? 1.f / sum : 0.f;          // (heads that only fill a unit up are zero)
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) lg[c][ii][r] *= inv;
+  if (!in_units) return;      // (whole groups of W lanes)
+
+  OT* base = out + ((int64_t)unit * L + l) * kMxR * W;
+  if constexpr (std::is_same<OT, float>::value) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) base[(wave * 256 + 64 * c + 16 * quarter + 4 * r + ii) * W + n % W] = lg[c][ii][r];
+  } else if constexpr (W == 1) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      uint32_t w[8];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        w[2 * r] = f32x2_to_bf16_bits(lg[c][0][r], lg[c][1][r]);
+        w[2 * r + 1] = f32x2_to_bf16_bits(lg[c][2][r], lg[c][3][r]);
+      }
+      uint4* to = reinterpret_cast<uint4*>(base + wave * 256 + 64 * c + 16 * quarter);
+      to[0] = make_uint4(w[0], w[1], w[2], w[3]);
+      to[1] = make_uint4(w[4], w[5], w[6], w[7]);
+    }
+  } else {
+    // heads of a unit lie on neighbouring lanes: exchanges between lanes x ^ 1 (and x ^ 2) leave lane j of the
+    // unit with the heads of bucket j (and j + 2) of four, a run of four buckets over ii
+    const uint32_t sel = (lane & 1) ? 0x03020706u : 0x05040100u;
+    const bool upper = (lane >> 1) & 1;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      uint32_t x[4], y[4];
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) {
+        const uint32_t w0 = f32x2_to_bf16_bits(lg[c][ii][0], lg[c][ii][1]);
+        const uint32_t w1 = f32x2_to_bf16_bits(lg[c][ii][2], lg[c][ii][3]);
+        const uint32_t a = __builtin_amdgcn_perm(sh_dpp_xor1(w0), w0, sel);       // two heads of bucket row (lane & 1)
+        const uint32_t d = __builtin_amdgcn_perm(sh_dpp_xor1(w1), w1, sel);       // ... and of row 2 + (lane & 1)
+        if constexpr (W == 2) {
+          x[ii] = a;
+          y[ii] = d;
+        } else {
+          const uint32_t got = sh_dpp_xor2(upper ? a : d), own = upper ? d : a;
+          x[ii] = upper ? got : own;
+          y[ii] = upper ? own : got;
+        }
+      }
+      const int row = wave * 256 + 64 * c + 16 * quarter;
+      if constexpr (W == 2) {
+        *reinterpret_cast<uint4*>(base + (row + 4 * (lane & 1)) * 2) = make_uint4(x[0], x[1], x[2], x[3]);
+        *reinterpret_cast<uint4*>(base + (row + 8 + 4 * (lane & 1)) * 2) = make_uint4(y[0], y[1], y[2], y[3]);
+      } else {
+        uint4* to = reinterpret_cast<uint4*>(base + (row + 4 * (lane & 3)) * 4);
+        to[0] = make_uint4(x[0], y[0], x[1], y[1]);
+        to[1] = make_uint4(x[2], y[2], x[3], y[3]);
+      }
+    }
+  }
+}
+
+__host__ __device__ __forceinline__ float mx_scale(float tanh_scale, float inv_temperature) {
+  return tanh_scale * inv_temperature * 1.4426950408889634f;
+}
+
+template <int W, class OT>
+__global__ __launch_bounds__(kSHThreads) void soft_hash_mx_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_sh,
+                                                                  const uint16_t* __restrict__ planes,
+                                                                  const uint16_t* __restrict__ protos_T, OT* __restrict__ out,
+                                                                  MxUnits units, int L, float scale) {
+  soft_hash_mx_block<void, W, OT>(blockIdx.x, blockIdx.y, units, q, q_sb, q_sh, planes, protos_T, out, L, scale, nullptr, nullptr, 0, 0,
+                                  nullptr);
 }
 
 // GC: heads per group the registers are sized for (4 or 8).  KC: K when known at
@@ -448,30 +707,10 @@ __global__ __launch_bounds__(kSHThreads) void soft_hash_kernel(
 // The key's sign bits come from the same matrix-core contraction as the cache
 // hashing kernel's (planes the M operand, the key column 0 of the N operand, the
 // k-steps in the same order), so both give the same bits for the same key.
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 sh_bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float sh_f32x4;
-union ShFrag {
-  uint4 u;
-  sh_bf16x8 v;
-};
-
-// eight consecutive table entries (cos, sin of four pairs) as floats
-template <class FT>
-__device__ __forceinline__ void sh_load8(const void* p, int64_t i, float (&o)[8]);
-template <>
-__device__ __forceinline__ void sh_load8<DType_bf16>(const void* p, int64_t i, float (&o)[8]) {
-  unpack16<DType_bf16>(*reinterpret_cast<const uint4*>((const uint16_t*)p + i), o);
-}
-template <>
-__device__ __forceinline__ void sh_load8<DType_f32>(const void* p, int64_t i, float (&o)[8]) {
-  const float4 a = *reinterpret_cast<const float4*>((const float*)p + i);
-  const float4 c = *reinterpret_cast<const float4*>((const float*)p + i + 4);
-  o[0] = a.x, o[1] = a.y, o[2] = a.z, o[3] = a.w, o[4] = c.x, o[5] = c.y, o[6] = c.z, o[7] = c.w;
-}
-
 constexpr int kPrologueD = 128;
 
-template <int GC, class FT>
+// GC: as in soft_hash_block, or 0: soft_hash_mx_block with units of W heads, OT the output's elements.
+template <int GC, class FT, int W, class OT>
 __global__ __launch_bounds__(kSHThreads) void decode_prologue_kernel(
     const uint16_t* __restrict__ qkv, int64_t qkv_sb, const void* __restrict__ freqs,
     const int64_t* __restrict__ pos, int pos_stride, int64_t n_pos, uint16_t* __restrict__ q_out,
@@ -480,17 +719,23 @@ __global__ __launch_bounds__(kSHThreads) void decode_prologue_kernel(
     uint16_t* __restrict__ v_norm, int NW, int64_t Tcap, const void* __restrict__ planes,
     const void* __restrict__ protos_T, void* __restrict__ q_table, int out_dtype, int Hq, int Hkv, int G, int L,
     int K, int R, float tanh_scale, float inv_temperature, int parts, int width, int word_blocks,
-    int n_key_blocks) {
+    int n_key_blocks, MxUnits units) {
   constexpr int D = kPrologueD;
   const int bx = blockIdx.x;
   if (bx >= n_key_blocks) {
     const int i = bx - n_key_blocks;
     const int l = i % L, pair = i / L;
+    if constexpr (GC == 0) {
+      soft_hash_mx_block<FT, W, OT>(l, pair, units, qkv, qkv_sb, D, (const uint16_t*)planes, (const uint16_t*)protos_T, (OT*)q_table, L,
+                                    mx_scale(tanh_scale, inv_temperature), freqs, pos, pos_stride, n_pos, q_out);
+      return;
+    } else {
     const int64_t p = pos[(int64_t)(pair / Hkv) * pos_stride];
     soft_hash_block<DType_bf16, GC, 10, FT>(l, pair, qkv, qkv_sb, D, planes, protos_T, q_table, out_dtype, Hq, Hkv,
                                             G, D, L, K, R, tanh_scale, inv_temperature, parts, width, 0, 1, freqs, p,
                                             p >= 0 && p < n_pos, q_out);
     return;
+    }
   }
   const int pair = bx / word_blocks, part = bx % word_blocks;
   const int b = pair / Hkv, kvh = pair % Hkv;
@@ -603,6 +848,14 @@ __global__ __launch_bounds__(kSHThreads) void decode_prologue_kernel(
 
 namespace {
 
+// The matrix-core form takes one prototype table size, the one the models have; its bits depend on neither the
+// group nor the layout, so that every way to a table gives the same one.
+bool mx_serves(int D, int K, int R) { return D == kMxD && K == kMxK && R == kMxR; }
+
+MxUnits mx_units(int B, int Hq, int Hkv, int parts) {
+  return {parts > 0 ? B * Hkv * parts : B * Hq, parts, Hq, Hkv, Hq / Hkv};
+}
+
 int soft_hash_entry(const void* q, int dtype, int64_t q_stride_b, int64_t q_stride_h, const void* planes,
                     const void* protos_T, void* out, int out_dtype, int B, int Hq, int Hkv, int D, int L, int K,
                     int R, float tanh_scale, float inv_temperature, void* stream, int grouped) {
@@ -628,6 +881,28 @@ int soft_hash_entry(const void* q, int dtype, int64_t q_stride_b, int64_t q_stri
                          ? 1
                          : 0;
   const int G = Hq / Hkv;
+  if (dtype == SOCKET_BF16 && mx_serves(D, K, R) && vec_ok && q_stride_b % 8 == 0 && q_stride_h % 8 == 0) {
+    const MxUnits units = mx_units(B, Hq, Hkv, parts);
+    const int W = grouped ? width : 1, per = kMxHeads / W;
+    const dim3 mx_grid(L, (units.count + per - 1) / per);
+    SOCKET_REQUIRE(mx_grid.y <= 65535, SOCKET_ERR_SHAPE);
+    const float scale = mx_scale(tanh_scale, inv_temperature);
+#define SOCKET_MX(WV)                                                                                                         \
+  do {                                                                                                                        \
+    if (out_dtype == SOCKET_F32)                                                                                              \
+      hipLaunchKernelGGL((soft_hash_mx_kernel<WV, float>), mx_grid, dim3(kSHThreads), 0, s, (const uint16_t*)q, q_stride_b,   \
+                         q_stride_h, (const uint16_t*)planes, (const uint16_t*)protos_T, (float*)out, units, L, scale);       \
+    else                                                                                                                      \
+      hipLaunchKernelGGL((soft_hash_mx_kernel<WV, uint16_t>), mx_grid, dim3(kSHThreads), 0, s, (const uint16_t*)q, q_stride_b, \
+                         q_stride_h, (const uint16_t*)planes, (const uint16_t*)protos_T, (uint16_t*)out, units, L, scale);    \
+  } while (0)
+    if (W == 4) SOCKET_MX(4);
+    else if (W == 2) SOCKET_MX(2);
+    else SOCKET_MX(1);
+#undef SOCKET_MX
+    SOCKET_LAUNCH_CHECK();
+    return SOCKET_OK;
+  }
   // K = 10 with a single sweep (R <= 4 buckets per lane) and vector loads: the
   // prototypes go from global memory straight into registers.  Otherwise they go
   // to LDS as fp32 when they fit in 64 KB, else they are read from global memory
@@ -728,20 +1003,40 @@ extern "C" int socket_decode_prologue(const void* qkv, int dtype, int64_t qkv_st
                                kSHWaves * GC + 3) / 4) * 4;
   const size_t dyn_lds = head_floats * sizeof(float);
   hipStream_t s = (hipStream_t)stream;
-#define SOCKET_DP(GCV, FT)                                                                                      \
-  hipLaunchKernelGGL((decode_prologue_kernel<GCV, FT>), dim3((unsigned)n_blocks), dim3(kSHThreads), dyn_lds, s, \
+  const bool mx = mx_serves(D, K, R);
+  const MxUnits units = mx_units(B, Hq, Hkv, parts);
+  const int W = grouped ? width : 1, per = kMxHeads / W;
+  const int64_t blocks = mx ? n_key_blocks + (int64_t)((units.count + per - 1) / per) * L : n_blocks;
+#define SOCKET_DP(GCV, FT, WV, OT)                                                                              \
+  hipLaunchKernelGGL((decode_prologue_kernel<GCV, FT, WV, OT>), dim3((unsigned)blocks), dim3(kSHThreads), mx ? 0 : dyn_lds, s, \
                      (const uint16_t*)qkv, qkv_stride_b, freqs_cis, pos, pos_stride, n_pos, (uint16_t*)q_out,   \
                      (uint16_t*)k_cache, (uint16_t*)v_cache, cache_stride_b, cache_stride_h, cache_stride_s,    \
                      lens, (const uint16_t*)planes_words, (uint32_t*)codes, (uint16_t*)v_norm, NW, Tcap,        \
                      planes, protos_T, q_table, out_dtype, Hq, Hkv, G, L, K, R, tanh_scale, inv_temperature,    \
-                     parts, width, word_blocks, (int)n_key_blocks)
-  if (GC == 4) {
-    if (freqs_dtype == SOCKET_F32) SOCKET_DP(4, DType_f32);
-    else SOCKET_DP(4, DType_bf16);
+                     parts, width, word_blocks, (int)n_key_blocks, units)
+#define SOCKET_DP_MX(FT)                                                     \
+  do {                                                                       \
+    if (out_dtype == SOCKET_F32) {                                           \
+      if (W == 4) SOCKET_DP(0, FT, 4, float);                                \
+      else if (W == 2) SOCKET_DP(0, FT, 2, float);                           \
+      else SOCKET_DP(0, FT, 1, float);                                       \
+    } else {                                                                 \
+      if (W == 4) SOCKET_DP(0, FT, 4, uint16_t);                             \
+      else if (W == 2) SOCKET_DP(0, FT, 2, uint16_t);                        \
+      else SOCKET_DP(0, FT, 1, uint16_t);                                    \
+    }                                                                        \
+  } while (0)
+  if (mx) {
+    if (freqs_dtype == SOCKET_F32) SOCKET_DP_MX(DType_f32);
+    else SOCKET_DP_MX(DType_bf16);
+  } else if (GC == 4) {
+    if (freqs_dtype == SOCKET_F32) SOCKET_DP(4, DType_f32, 1, float);
+    else SOCKET_DP(4, DType_bf16, 1, float);
   } else {
-    if (freqs_dtype == SOCKET_F32) SOCKET_DP(8, DType_f32);
-    else SOCKET_DP(8, DType_bf16);
+    if (freqs_dtype == SOCKET_F32) SOCKET_DP(8, DType_f32, 1, float);
+    else SOCKET_DP(8, DType_bf16, 1, float);
   }
+#undef SOCKET_DP_MX
 #undef SOCKET_DP
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;

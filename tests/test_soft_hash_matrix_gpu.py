@@ -1,0 +1,62 @@
+"""The matrix-core soft hash (bf16, 128 dims, K = 10, R = 1024) against float64: every width of a unit, padded groups, units
+that do not fill a workgroup's sixteen heads, both output types, and one head's NaN kept to itself."""
+import math
+
+import pytest
+import torch
+
+from socket_amd import hash_cache
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def exact(q, planes, protos, temperature):
+    t = torch.tanh(torch.einsum("bhd,lkd->bhlk", q.double(), planes.double())) / math.sqrt(q.shape[-1])
+    return torch.softmax(torch.einsum("bhlk,kr->bhlr", t, protos.double()) / temperature, -1)
+
+
+def inputs(B, Hq, L, seed, cube):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    q = torch.randn(B, Hq, 128, generator=g, device=DEV).bfloat16()
+    planes = (torch.randn(L, 10, 128, generator=g, device=DEV) * (1.0 if cube else 0.1)).bfloat16()
+    r, k = torch.arange(1024, device=DEV)[None], torch.arange(10, device=DEV)[:, None]
+    protos = (((r >> (9 - k)) & 1) * 2 - 1).bfloat16() if cube else torch.randn(10, 1024, generator=g, device=DEV).bfloat16()
+    return q, planes, protos
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,cube,temp", [(1, 1, 1, 1, True, 0.3), (3, 6, 3, 5, False, 0.3), (1, 28, 4, 3, True, 0.3),
+                                                  (2, 15, 5, 4, False, 1.0), (5, 40, 8, 2, True, 1.0), (1, 7, 7, 3, False, 0.02)])
+def test_tables_of_every_layout(B, Hq, Hkv, L, cube, temp):
+    q, planes, protos = inputs(B, Hq, L, B + Hq, cube)
+    want = exact(q, planes, protos, temp)
+    parts, width = hash_cache.group_shape(Hq, Hkv)
+    G = Hq // Hkv
+    plain = hash_cache.soft_hash(q, planes, protos, temp, Hkv)
+    wide = hash_cache.soft_hash(q, planes, protos, temp, Hkv, out_dtype=torch.float32)
+    # (ten fp32 products and sums of logits up to 0.9 / temp, an exponential and a normalisation to an ulp or two)
+    unit = 2 ** -23 * (16 + 16 * 0.9 / temp)
+    assert ((wide.double() - want).abs() <= unit * want).all()
+    # (bfloat16 has eight significant bits: a rounding is off by up to 2^-8 of its result)
+    assert ((plain.double() - want).abs() <= (2 ** -8 + 2 * unit) * want).all()
+    for got, flat in ((hash_cache.soft_hash(q, planes, protos, temp, Hkv, grouped=True), plain),
+                      (hash_cache.soft_hash(q, planes, protos, temp, Hkv, out_dtype=torch.float32, grouped=True), wide)):
+        for h in range(Hq):
+            kv, g = h // G, h % G
+            assert torch.equal(got[:, kv * parts + g // width, :, :, g % width], flat[:, h])
+        for g in range(G, parts * width):
+            assert (got.view(B, Hkv, parts, L, 1024, width)[:, :, g // width, :, :, g % width] == 0).all()
+    assert torch.equal(plain, hash_cache.soft_hash(q, planes, protos, temp, None))
+
+
+def test_a_head_of_nan_stays_alone():
+    q, planes, protos = inputs(2, 8, 2, 1, True)
+    clean = hash_cache.soft_hash(q, planes, protos, 0.3, 2)
+    q[1, 3, 17] = float("nan")
+    q[0, 2, 5] = float("inf")
+    got = hash_cache.soft_hash(q, planes, protos, 0.3, 2)
+    keep = torch.ones(2, 8, dtype=torch.bool, device=DEV)
+    keep[1, 3] = keep[0, 2] = False
+    assert torch.equal(got[keep], clean[keep]) and got[1, 3].isnan().all()
+    # an infinite coordinate saturates every plane it meets
+    assert torch.allclose(got[0, 2].double(), exact(q, planes, protos, 0.3)[0, 2], rtol=2 ** -8)
