@@ -471,6 +471,10 @@ int socket_add_rmsnorm(const void* x, const void* residual, const void* weight, 
 /* out = round(silu(a)) * b elementwise over n elements (FeedForward, GPT-FAST/model.py:599-600). */
 int socket_silu_mul(const void* a, const void* b, void* out, int dtype, int64_t n, void* stream);
 
+/* tok[b] = the first index of the greatest of logits[b, 0 .. V) (rows `stride` elements apart; a NaN counts as the
+ * greatest), and pos[0] += 1 unless pos is NULL: the end of a greedy decode step (GPT-FAST/generate.py:127-132). */
+int socket_greedy(const void* logits, int dtype, int64_t stride, int B, int V, int32_t* tok, int64_t* pos, void* stream);
+
 /* y[m,n] = sum_k x[m,k] * w[n,k]: the linear layers of a single-token step as matrix-vector
  * products (M <= 4 rows, bf16, fp32 accumulation; K a multiple of 2048; x rows `x_stride`
  * elements apart, y rows `y_stride`; w [N,K] contiguous).  With w_gate (another [N,K]):

@@ -10,6 +10,8 @@
 //  * add_rmsnorm_kernel: optional residual add + RMSNorm (model.py:603-614 and
 //    the `x + ...` of TransformerBlock :340-342).
 //  * silu_mul_kernel: silu(a) * b of the feed-forward (model.py:599-600).
+//  * greedy_kernel: the next token (the first of the greatest logits, GPT-FAST/generate.py:127-132) and the
+//    position after it.
 #include "socket_common.h"
 
 namespace {
@@ -575,6 +577,92 @@ extern "C" int socket_rope_rows(const void* qkv, int dtype, int64_t qkv_stride_b
   else SOCKET_ROWS_F(DType_f16);
 #undef SOCKET_ROWS_F
 #undef SOCKET_ROWS
+  SOCKET_LAUNCH_CHECK();
+  return SOCKET_OK;
+}
+
+namespace {
+
+// The first index of a row's greatest value (a NaN counts as the greatest, as in torch.argmax), one workgroup to a
+// row; workgroup 0 also advances the position.  The row comes from L2 (the product before has just written it) and
+// one CU reads 128 KB of it in about a microsecond, so splitting it over workgroups would only add a pass: 32000
+// logits take 5 us with the launch, where torch's reduction, its cast to int, the copy to the token
+// buffer and the position's add took 26 us in four launches.
+constexpr int kGreedyThreads = 1024;
+
+template <class DT, bool VEC>
+__global__ __launch_bounds__(kGreedyThreads) void greedy_kernel(const void* __restrict__ logits, int64_t stride, int V,
+                                                               int32_t* __restrict__ tok, int64_t* __restrict__ pos) {
+  constexpr int E = VEC ? DT::kPer16B : 1, U = 8;      // elements of a load, loads in flight
+  __shared__ uint64_t red[kGreedyThreads / 64];
+  const int64_t row = blockIdx.x * stride;
+  uint32_t best = 0;
+  int at = 0;
+  const int pieces = V / E;
+  auto take = [&](uint32_t key, int i) {
+    if (key > best) best = key, at = i;                // (a lane's indices rise: the first of equals stays)
+  };
+  for (int p0 = 0; p0 < pieces; p0 += U * kGreedyThreads) {
+    uint4 w[VEC ? U : 1];
+    float x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = min(p0 + u * kGreedyThreads + (int)threadIdx.x, pieces - 1);
+      if constexpr (VEC) w[u] = *reinterpret_cast<const uint4*>((const typename DT::storage*)logits + row + (int64_t)p * E);
+      else x[u] = ld<DT>(logits, row + p);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int p = p0 + u * kGreedyThreads + threadIdx.x;
+      if (p >= pieces) continue;
+      if constexpr (VEC) {
+        float f[E];
+        unpack16<DT>(w[u], f);
+#pragma unroll
+        for (int e = 0; e < E; ++e) take(score_to_key(f[e]), p * E + e);
+      } else {
+        take(score_to_key(x[u]), p);
+      }
+    }
+  }
+  if (VEC && (int)threadIdx.x < V - pieces * E) {
+    const int i = pieces * E + threadIdx.x;
+    take(score_to_key(ld<DT>(logits, row + i)), i);
+  }
+  uint64_t m = ((uint64_t)best << 32) | (0xffffffffu - (uint32_t)at);
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint64_t o = __shfl_xor(m, d, 64);
+    m = o > m ? o : m;
+  }
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < kGreedyThreads / 64; ++w) m = red[w] > m ? red[w] : m;
+    tok[blockIdx.x] = (int32_t)(0xffffffffu - (uint32_t)m);
+    if (pos && blockIdx.x == 0) pos[0] += 1;
+  }
+}
+
+}  // namespace
+
+extern "C" int socket_greedy(const void* logits, int dtype, int64_t stride, int B, int V, int32_t* tok, int64_t* pos,
+                             void* stream) {
+  SOCKET_REQUIRE(logits && tok, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(socket_dtype_bytes(dtype) != 0, SOCKET_ERR_UNSUPPORTED);
+  SOCKET_REQUIRE(B > 0 && V > 0 && V < (1 << 30) && stride >= V, SOCKET_ERR_SHAPE);
+  const bool vec = socket_aligned16(logits) && stride * socket_dtype_bytes(dtype) % 16 == 0 && V >= 16;
+  hipStream_t s = (hipStream_t)stream;
+#define SOCKET_GREEDY_LAUNCH(DT)                                                                                       \
+  do {                                                                                                                 \
+    if (vec) hipLaunchKernelGGL((greedy_kernel<DT, true>), dim3(B), dim3(kGreedyThreads), 0, s, logits, stride, V, tok, pos);  \
+    else hipLaunchKernelGGL((greedy_kernel<DT, false>), dim3(B), dim3(kGreedyThreads), 0, s, logits, stride, V, tok, pos);     \
+  } while (0)
+  if (dtype == SOCKET_F32) SOCKET_GREEDY_LAUNCH(DType_f32);
+  else if (dtype == SOCKET_BF16) SOCKET_GREEDY_LAUNCH(DType_bf16);
+  else SOCKET_GREEDY_LAUNCH(DType_f16);
+#undef SOCKET_GREEDY_LAUNCH
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
 }

@@ -110,6 +110,28 @@ def silu_mul(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
 
 
 @torch.no_grad()
+def greedy_tokens(logits: torch.Tensor, out: Optional[torch.Tensor] = None, pos: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """argmax over the last dimension of logits [B,V] as int32 [B,1], into `out` if given; with `pos` (int64, one
+    element) the position is raised by one as well.  One launch (GPT-FAST/generate.py:127-132)."""
+    B, V = logits.shape
+    others = [t for t in (out, pos) if t is not None]
+    if (plain_tensors(logits, *others) and logits.dtype in (torch.float32, torch.bfloat16, torch.float16) and logits.stride(1) == 1
+            and logits.stride(0) >= V and 0 < V < 1 << 30 and B > 0
+            and (out is None or (out.dtype == torch.int32 and out.is_contiguous() and out.numel() == B))
+            and (pos is None or (pos.dtype == torch.int64 and pos.numel() == 1))):
+        tok = torch.empty((B, 1), dtype=torch.int32, device=logits.device) if out is None else out
+        check("socket_greedy", lib().socket_greedy(ptr(logits), dtype_enum(logits.dtype), logits.stride(0), B, V, ptr(tok),
+                                                   ptr(pos), stream_ptr(logits.device)))
+        return tok
+    tok = torch.argmax(logits, dim=-1, keepdim=True).to(torch.int32)
+    if out is not None:
+        out.copy_(tok)
+    if pos is not None:
+        pos.add_(1)
+    return tok if out is None else out
+
+
+@torch.no_grad()
 def linear_rows(x: torch.Tensor, weight: torch.Tensor, gate_weight: torch.Tensor = None) -> torch.Tensor:
     """x @ weight.T for the few rows of a decode step (nn.Linear without bias,
     GPT-FAST/model.py:436, :476), or with `gate_weight` silu(x @ weight.T) * (x @ gate_weight.T)

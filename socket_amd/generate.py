@@ -27,7 +27,7 @@ from typing import Callable, List, Optional, Tuple
 
 import torch
 
-from . import hash_cache, registry
+from . import decode_ops, hash_cache, registry
 from .hybrid import HybridArgs
 from .model import ModelArgs, Transformer
 from .socket_kernels import sparse_attention_fwd
@@ -117,11 +117,13 @@ class DecodeGraph:
                 t.copy_(old)
         return put_back
 
-    def _step(self):
+    def _logits(self):
         fwd = self.model.forward if self.decode_type == "dense" else self.model.sparse_forward
-        logits = fwd(self.tok, self.pos)
-        nxt = torch.argmax(logits[:, -1], dim=-1, keepdim=True).to(torch.int)
-        return logits, nxt
+        return fwd(self.tok, self.pos)
+
+    def _step(self):
+        logits = self._logits()
+        return logits, decode_ops.greedy_tokens(logits[:, -1])
 
     @torch.no_grad()
     def capture(self, tok: torch.Tensor, pos: int) -> None:
@@ -140,9 +142,8 @@ class DecodeGraph:
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(self.graph):
-            self.logits, nxt = self._step()
-            self.tok.copy_(nxt)
-            self.pos.add_(1)
+            self.logits = self._logits()
+            decode_ops.greedy_tokens(self.logits[:, -1], out=self.tok, pos=self.pos)
 
     @torch.no_grad()
     def check(self, tok: torch.Tensor, pos: int, replays: int = 3) -> dict:
