@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
   const int cpw = 32 / P;
 
   // gridDim.y splits the packed words between workgroups when there are too
-  // few key tiles to occupy the chip (the per-step append of a handful of keys)
+  // few key tiles to occupy the chip
   const int word_begin = blockIdx.y * words_per_wg;
   const int word_end = min(NW, word_begin + words_per_wg);
 
@@ -532,6 +532,163 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
   }
 }
 
+// ---------------------------------------------------------------------------
+// Direct variant for few rows (a decode step's, a short block's): nothing in LDS, no wave waits for another.
+//
+// The rows of all (b, kv head) pairs are numbered through and cut into tiles of NB 16-row blocks, so that a
+// decode step's handful shares one contraction whatever pairs it belongs to.  A wave makes ONE packed word of a
+// tile: its plane fragments and its keys are requested together, straight into registers, and the whole kernel is
+// one trip to memory, 8 NB products and a store.  (The staged kernel above pays a trip for the planes, a barrier, a trip
+// for the keys, and reads the planes' LDS image through for every tile.)  The last row of the grid has the values' norms
+// and, where `k_cache` is given, the rows' copies and the lengths.
+// A decode step's 8 rows, 32 tables of 8 planes: 3.5 us where the staged kernel takes 6.4 (float32); 512 rows of 60 x
+// 10: 3.5 against 10.8 (bf16).
+// Same k-steps in the same order on the same fragments as above: the bits are equal.
+constexpr int kDirectWaves = 4, kDirectThreads = kDirectWaves * SOCKET_WAVE;
+
+template <class DT, int NB>
+__global__ __launch_bounds__(kDirectThreads) void hash_keys_direct_kernel(
+    const void* __restrict__ k_, const void* __restrict__ v_, int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh,
+    int64_t v_ss, const uint16_t* __restrict__ planes_words, uint32_t* __restrict__ codes, uint16_t* __restrict__ v_norm,
+    const int32_t* __restrict__ pos_b, int t0, int Hkv, int S, int D, int L, int P, int NW, int64_t Tcap, int n_rows,
+    int word_groups, void* __restrict__ k_cache, void* __restrict__ v_cache, int64_t c_sb, int64_t c_sh, int64_t c_ss,
+    int32_t* __restrict__ lens, int B) {
+  typedef typename DT::storage ST;
+  constexpr int kTile = 16 * NB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int prow = lane & 15, quarter = lane >> 4;
+  const int row0 = blockIdx.x * kTile;
+  struct Where {
+    int b, h, s;
+  };
+  auto where = [&](int row) {
+    const unsigned r = min(row, n_rows - 1), pair = r / (unsigned)S;
+    return Where{(int)(pair / (unsigned)Hkv), (int)(pair % (unsigned)Hkv), (int)(r - pair * S)};
+  };
+  auto start = [&](const void* base, const Where& at, int64_t sb, int64_t sh, int64_t ss) {
+    return (const ST*)base + at.b * sb + at.h * sh + at.s * ss;
+  };
+  auto fragments = [&](const ST* row, Frag (&dst)[kKSteps]) {
+#pragma unroll
+    for (int ks = 0; ks < kKSteps; ++ks) {
+      const int d = ks * 32 + quarter * 8;           // (a narrower head's row ends in zeros)
+      dst[ks].u = make_uint4(0, 0, 0, 0);
+      if (ks * 32 < D) {                             // (the same for every lane)
+        const uint4 x = load_frag8<DT>(row + min(d, D - 8));
+        if (d < D) dst[ks].u = x;
+      }
+    }
+  };
+
+  if ((int)blockIdx.y == word_groups) {
+    constexpr bool kNormByMfma = DT::kEnum == SOCKET_BF16;
+    if (v_ && kNormByMfma) {                         // (the Gram diagonal, as in the kernel above)
+      for (int nb = wave; nb < NB; nb += kDirectWaves) {
+        const int row = row0 + nb * 16 + prow;
+        const Where at = where(row);
+        Frag vf[kKSteps];
+        fragments(start(v_, at, v_sb, v_sh, v_ss), vf);
+        f32x4 g = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < kKSteps; ++ks) g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[ks].v, vf[ks].v, g, 0, 0, 0);
+        const int r = prow - 4 * quarter, pos = (pos_b ? pos_b[at.b] : t0) + at.s;
+        const float d = r == 0 ? g[0] : r == 1 ? g[1] : r == 2 ? g[2] : g[3];
+        if (r >= 0 && r < 4 && row < n_rows && in_cache(pos, Tcap))
+          v_norm[((int64_t)at.b * Hkv + at.h) * Tcap + pos] = f32_to_f16_bits(sqrtf(d));
+      }
+    } else if (v_) {
+      float ss[NB];
+#pragma unroll
+      for (int g = 0; g < NB; ++g) {
+        const ST* row = start(v_, where(row0 + (wave * NB + g) * 4 + quarter), v_sb, v_sh, v_ss);
+        const float x = sumsq8<DT>(row + min(prow * 8, D - 8));
+        ss[g] = prow * 8 < D ? x : 0.f;
+      }
+#pragma unroll
+      for (int g = 0; g < NB; ++g) {
+        const int row = row0 + (wave * NB + g) * 4 + quarter;
+        const Where at = where(row);
+        float t = ss[g];
+#pragma unroll
+        for (int x = 1; x < 16; x <<= 1) t += __shfl_xor(t, x, SOCKET_WAVE);
+        const int pos = (pos_b ? pos_b[at.b] : t0) + at.s;
+        if (prow == 0 && row < n_rows && in_cache(pos, Tcap))
+          v_norm[((int64_t)at.b * Hkv + at.h) * Tcap + pos] = f32_to_f16_bits(sqrtf(t));
+      }
+    }
+    if (k_cache) {
+      if (lens && blockIdx.x == 0)
+        for (int b = tid; b < B; b += kDirectThreads) lens[b] = t0 + S;
+      constexpr int E = DT::kPer16B, U = 2;
+      const int per = D / E, n = min(kTile, n_rows - row0) * per;
+      for (int i0 = tid; i0 < n; i0 += U * kDirectThreads) {
+        uint4 x[U], y[U];
+        int64_t to[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int i = min(i0 + u * kDirectThreads, n - 1), d = i % per * E;
+          const Where at = where(row0 + i / per);
+          x[u] = *reinterpret_cast<const uint4*>(start(k_, at, k_sb, k_sh, k_ss) + d);
+          y[u] = *reinterpret_cast<const uint4*>(start(v_, at, v_sb, v_sh, v_ss) + d);
+          to[u] = at.b * c_sb + at.h * c_sh + (t0 + at.s) * c_ss + d;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (i0 + u * kDirectThreads >= n) break;
+          *reinterpret_cast<uint4*>((ST*)k_cache + to[u]) = x[u];
+          *reinterpret_cast<uint4*>((ST*)v_cache + to[u]) = y[u];
+        }
+      }
+    }
+    return;
+  }
+
+  const int w = blockIdx.y * kDirectWaves + wave;
+  if (w >= NW) return;
+  const int pbit0 = 8 * (prow >> 2) + 7 - (prow & 3);      // (plane row of each accumulator register: see above)
+  Frag pf[kKSteps][2], kf[NB][kKSteps];
+#pragma unroll
+  for (int ks = 0; ks < kKSteps; ++ks)
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+      pf[ks][mb].u = reinterpret_cast<const uint4*>(planes_words)[(int64_t)(w * 32 + pbit0 - 4 * mb) * 16 + ks * 4 + quarter];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) fragments(start(k_, where(row0 + nb * 16 + prow), k_sb, k_sh, k_ss), kf[nb]);
+  const int row = row0 + (NB == 4 ? lane : prow);          // whose word this lane stores
+  const Where at = where(row);
+  const int pos = (pos_b ? pos_b[at.b] : t0) + at.s;
+  uint32_t neg = 0;
+#pragma unroll
+  for (int nb = NB - 1; nb >= 0; --nb) {
+    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int ks = 0; ks < kKSteps; ++ks)
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb)
+        acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[ks][mb].v, kf[nb][ks].v, acc[mb], 0, 0, 0);
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) neg = __builtin_amdgcn_alignbit(neg, __float_as_uint(acc[mb][r]), 31);
+  }
+  uint32_t word;
+  if constexpr (NB == 4) {                                 // (the byte transpose of the kernel above)
+    const uint32_t t = lane_xor16(neg, quarter & 1);
+    const uint32_t x = __builtin_amdgcn_perm(t, neg, (quarter & 1) ? 0x03070105u : 0x06020400u);
+    const uint32_t u = lane_xor32(x, quarter & 2);
+    word = __builtin_amdgcn_perm(u, x, (quarter & 2) ? 0x03020706u : 0x05040100u);
+  } else {
+    static_assert(NB == 1, "one block, or four whose bytes fill a word");
+    word = neg << (8 * quarter);
+    word |= lane_xor16(word, quarter & 1);
+    word |= lane_xor32(word, quarter & 2);
+  }
+  const int cpw = 32 / P, nbits = min(cpw, L - w * cpw) * P;
+  const uint32_t valid = nbits >= 32 ? 0xffffffffu : ((1u << nbits) - 1u);
+  if ((NB == 4 || quarter == 0) && row < n_rows && in_cache(pos, Tcap))
+    codes[(((int64_t)at.b * Hkv + at.h) * NW + w) * Tcap + pos] = ~word & valid;
+}
+
 // Keys and values [B,Hkv,S,D] (any strides, whole 16-byte pieces) into rows t0 .. of the caches; the lengths
 // become t0 + S.  A lane moves kCopyPieces pieces of each, requested together; a wave's stores are whole rows.
 constexpr int kCopyPieces = 4;
@@ -702,6 +859,43 @@ int launch_stream(const HashRows& a, const SocketDeviceLimits& lim, hipStream_t 
   return SOCKET_OK;
 }
 
+// Few enough rows for the direct variant.  Its time grows with rows x words, since a wave fetches its tile's keys and
+// its word's planes for itself; the others' hardly does below a few tiles per CU.  Hashing 8 pairs' rows with 20
+// words, bf16 of 128 dims, direct / staged: 8192 rows 10.4 / 11.8 us, 12288 13.5 / 12.1; with 8 words 24576 rows 11.3 / 12.0.
+// The lines cross between 180k (float32) and 260k words; with the copy in the same launch (one fewer) between 270k and
+// 400k: 12288 rows of 64 dims in 16 bits 12.1 / 15.6 us, 16384 of 128 bf16 dims 18.5 / 17.4.  Where the streamed kernel
+// has at least half of every tile it is ahead of both (32768 rows, 8 words: 7.0 against 14.5 direct).
+bool goes_direct(const HashRows& a, bool streamed) {
+  const int64_t rows = (int64_t)a.B * a.Hkv * a.S, tiles = (int64_t)a.B * a.Hkv * ((a.S + kStreamTile - 1) / kStreamTile);
+  if (streamed && 2 * rows >= tiles * kStreamTile) return false;
+  return rows * a.NW <= (a.k_cache ? 256 : 176) * 1024 && a.NW <= 65536;      // (a grid's y)
+}
+
+int launch_direct(const HashRows& a, const SocketDeviceLimits& lim, int32_t* lens, hipStream_t s) {
+  const int n_rows = a.B * a.Hkv * a.S, groups = (a.NW + kDirectWaves - 1) / kDirectWaves;
+  const int rows_of = (a.v || a.k_cache) ? 1 : 0;
+  // four blocks to a tile once that still gives every CU a workgroup
+  const bool wide = (int64_t)((n_rows + 63) / 64) * groups >= lim.cu_count;
+  const int tile = wide ? 64 : 16;
+  const dim3 grid((n_rows + tile - 1) / tile, groups + rows_of);
+#define SOCKET_DIRECT(DT, NB)                                                                                             \
+  hipLaunchKernelGGL((hash_keys_direct_kernel<DT, NB>), grid, dim3(kDirectThreads), 0, s, a.k, a.v, a.k_sb, a.k_sh, a.k_ss, \
+                     a.v_sb, a.v_sh, a.v_ss, (const uint16_t*)a.planes_words, a.codes, a.v_norm, a.pos_b, a.t0, a.Hkv, a.S, \
+                     a.D, a.L, a.P, a.NW, a.Tcap, n_rows, groups, a.k_cache, a.v_cache, a.c_sb, a.c_sh, a.c_ss, lens, a.B)
+#define SOCKET_DIRECT_DT(DT)           \
+  do {                                 \
+    if (wide) SOCKET_DIRECT(DT, 4);    \
+    else SOCKET_DIRECT(DT, 1);         \
+  } while (0)
+  if (a.dtype == SOCKET_BF16) SOCKET_DIRECT_DT(DType_bf16);
+  else if (a.dtype == SOCKET_F16) SOCKET_DIRECT_DT(DType_f16);
+  else SOCKET_DIRECT_DT(DType_f32);
+#undef SOCKET_DIRECT_DT
+#undef SOCKET_DIRECT
+  SOCKET_LAUNCH_CHECK();
+  return SOCKET_OK;
+}
+
 int launch_staged(const HashRows& a, const SocketDeviceLimits& lim, hipStream_t s) {
   const int tiles_per_row = (a.S + kKeysPerWave - 1) / kKeysPerWave;
   const int64_t n_tiles64 = (int64_t)a.B * a.Hkv * tiles_per_row;
@@ -776,7 +970,9 @@ extern "C" int socket_hash_keys(const void* k, const void* v, int dtype, int64_t
   const int st = check_hash_rows(a);
   if (st != SOCKET_OK) return st;
   const SocketDeviceLimits& lim = socket_device_limits();
-  return streams(a, lim) ? launch_stream<kD, false>(a, lim, (hipStream_t)stream) : launch_staged(a, lim, (hipStream_t)stream);
+  const bool streamed = streams(a, lim);
+  if (goes_direct(a, streamed)) return launch_direct(a, lim, nullptr, (hipStream_t)stream);
+  return streamed ? launch_stream<kD, false>(a, lim, (hipStream_t)stream) : launch_staged(a, lim, (hipStream_t)stream);
 }
 
 extern "C" int socket_hash_rows(const void* k, const void* v, int dtype, int64_t k_stride_b, int64_t k_stride_h,
@@ -790,7 +986,9 @@ extern "C" int socket_hash_rows(const void* k, const void* v, int dtype, int64_t
   if (st != SOCKET_OK) return st;
   hipStream_t s = (hipStream_t)stream;
   const SocketDeviceLimits& lim = socket_device_limits();
-  if (!streams(a, lim)) return launch_staged(a, lim, s);
+  const bool streamed = streams(a, lim);
+  if (goes_direct(a, streamed)) return launch_direct(a, lim, nullptr, s);
+  if (!streamed) return launch_staged(a, lim, s);
   return D == 64 ? launch_stream<64, false>(a, lim, s) : launch_stream<128, false>(a, lim, s);
 }
 
@@ -815,6 +1013,7 @@ extern "C" int socket_cache_append(const void* k, const void* v, int dtype, int6
   hipStream_t s = (hipStream_t)stream;
   const SocketDeviceLimits& lim = socket_device_limits();
   const bool streamed = streams(a, lim);
+  if (goes_direct(a, streamed)) return launch_direct(a, lim, lens, s);
   // the rows' copy (all of it where the hash does not pass them on) and the lengths
   if (!streamed || lens) {
     const int64_t pieces = streamed ? 1 : (int64_t)S * (D / per16);
