@@ -432,11 +432,12 @@ int socket_rope_append(const void* qkv, int dtype, int64_t qkv_stride_b, const v
 
 /* The same for the S rows of a prompt: qkv [B,S,(Hq+2Hkv)*D] (element strides b, s; unit-stride last dim) -> q_out
  * [B,S,Hq,D] contiguous, rotated keys and values into rows t0 .. t0 + S - 1 of the caches.  freqs [S, D/2, 2]: (cos, sin)
- * of the rows, bf16 or f32.  Pointers and strides must be multiples of 16 bytes (SOCKET_ERR_ALIGN). */
+ * of the rows, bf16 or f32.  lens [B] (or NULL) becomes t0 + S.  Pointers and strides must be multiples of 16 bytes
+ * (SOCKET_ERR_ALIGN). */
 int socket_rope_rows(const void* qkv, int dtype, int64_t qkv_stride_b, int64_t qkv_stride_s, const void* freqs,
                      int freqs_dtype, void* q_out, void* k_cache, void* v_cache, int64_t cache_stride_b,
-                     int64_t cache_stride_h, int64_t cache_stride_s, int64_t t0, int B, int S, int Hq, int Hkv, int D,
-                     int64_t Tcap, void* stream);
+                     int64_t cache_stride_h, int64_t cache_stride_s, int32_t* lens, int64_t t0, int B, int S, int Hq,
+                     int Hkv, int D, int64_t Tcap, void* stream);
 
 /* The head of a single-token decode step in ONE launch: what socket_rope_append,
  * socket_hash_keys on the new key and socket_soft_hash (out_dtype / grouped as

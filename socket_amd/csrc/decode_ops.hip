@@ -128,9 +128,10 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(const void* __restrict__
                                                         const void* __restrict__ freqs, void* __restrict__ q_out,
                                                         void* __restrict__ k_cache, void* __restrict__ v_cache, int64_t c_sb,
                                                         int64_t c_sh, int64_t c_ss, int64_t t0, int s0, int S, int Hq, int Hkv,
-                                                        int D) {
+                                                        int D, int32_t* __restrict__ lens) {
   constexpr int E = DT::kPer16B;
   typedef typename DT::storage ST;
+  if (lens && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) lens[blockIdx.z] = (int32_t)(t0 + S);
   const int pieces = D / E, per_row = (Hq + 2 * Hkv) * pieces;
   const int w = blockIdx.x * 256 + threadIdx.x, s = s0 + blockIdx.y, b = blockIdx.z;
   if (w >= per_row) return;
@@ -548,8 +549,8 @@ extern "C" int socket_add_rmsnorm(const void* x, const void* residual, const voi
 
 extern "C" int socket_rope_rows(const void* qkv, int dtype, int64_t qkv_stride_b, int64_t qkv_stride_s, const void* freqs,
                                 int freqs_dtype, void* q_out, void* k_cache, void* v_cache, int64_t cache_stride_b,
-                                int64_t cache_stride_h, int64_t cache_stride_s, int64_t t0, int B, int S, int Hq, int Hkv, int D,
-                                int64_t Tcap, void* stream) {
+                                int64_t cache_stride_h, int64_t cache_stride_s, int32_t* lens, int64_t t0, int B, int S, int Hq,
+                                int Hkv, int D, int64_t Tcap, void* stream) {
   SOCKET_REQUIRE(qkv && freqs && q_out && k_cache && v_cache, SOCKET_ERR_NULL);
   SOCKET_REQUIRE(socket_dtype_bytes(dtype) != 0 && (freqs_dtype == SOCKET_F32 || freqs_dtype == SOCKET_BF16), SOCKET_ERR_UNSUPPORTED);
   SOCKET_REQUIRE(B > 0 && B <= 65535 && S > 0 && S <= 65535 * 8 && Hq > 0 && Hkv > 0 && D > 0, SOCKET_ERR_SHAPE);
@@ -565,7 +566,7 @@ extern "C" int socket_rope_rows(const void* qkv, int dtype, int64_t qkv_stride_b
     const int n = S - s0 < 65535 ? S - s0 : 65535;                                                                       \
     const dim3 grid((unsigned)(((Hq + 2 * Hkv) * (D / per) + 255) / 256), (unsigned)n, (unsigned)B);                     \
     hipLaunchKernelGGL((rope_rows_kernel<DT, FT>), grid, block, 0, st, qkv, qkv_stride_b, qkv_stride_s, freqs, q_out,    \
-                       k_cache, v_cache, cache_stride_b, cache_stride_h, cache_stride_s, t0, s0, S, Hq, Hkv, D);         \
+                       k_cache, v_cache, cache_stride_b, cache_stride_h, cache_stride_s, t0, s0, S, Hq, Hkv, D, lens);   \
   }
 #define SOCKET_ROWS_F(DT)                                          \
   do {                                                             \

@@ -59,17 +59,19 @@ def rope_rows_fits(qkv: torch.Tensor, freqs: torch.Tensor, k_cache: torch.Tensor
 
 @torch.no_grad()
 def rope_rows(qkv: torch.Tensor, freqs: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, t0: int, n_heads: int,
-              n_kv_heads: int) -> torch.Tensor:
+              n_kv_heads: int, lens: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The prompt rows qkv [B,S,(Hq+2Hkv)*D] -> rotated queries [B,S,Hq,D]; rotated keys and values go into rows
-    t0 .. t0 + S of the caches [B,Hkv,Tcap,D].  freqs [S,D/2,2]: the rows' angles.  One launch with the results of
+    t0 .. t0 + S of the caches [B,Hkv,Tcap,D].  freqs [S,D/2,2]: the rows' angles;
+    lens (int32 [B]) becomes t0 + S.  One launch with the results of
     apply_rotary_emb on q and k (GPT-FAST/model.py:626-639) and the cache writes (:215-217)."""
     B, S, N = qkv.shape
     D = k_cache.shape[-1]
     assert N == (n_heads + 2 * n_kv_heads) * D and k_cache.shape[1] == n_kv_heads
+    assert lens is None or (lens.dtype == torch.int32 and lens.is_contiguous() and lens.numel() == B)
     q = torch.empty((B, S, n_heads, D), dtype=qkv.dtype, device=qkv.device)
     check("socket_rope_rows", lib().socket_rope_rows(
         ptr(qkv), dtype_enum(qkv.dtype), qkv.stride(0), qkv.stride(1), ptr(freqs), dtype_enum(freqs.dtype), ptr(q),
-        ptr(k_cache), ptr(v_cache), *k_cache.stride()[:3], int(t0), B, S, n_heads, n_kv_heads, D, k_cache.shape[2],
+        ptr(k_cache), ptr(v_cache), *k_cache.stride()[:3], ptr(lens), int(t0), B, S, n_heads, n_kv_heads, D, k_cache.shape[2],
         stream_ptr(qkv.device)))
     return q
 

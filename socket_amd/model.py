@@ -26,7 +26,7 @@ from __future__ import annotations
 
 import math
 from dataclasses import dataclass
-from typing import Optional, Sequence
+from typing import Optional, Sequence, Tuple
 
 import torch
 import torch.nn as nn
@@ -211,11 +211,10 @@ class KVCache(nn.Module):
         keys and values as [B,S,Hkv,D] views of the cache."""
         S = qkv.shape[1]
         self._bounds(pos0, S)
-        q = decode_ops.rope_rows(qkv, freqs_cis, self.k_cache, self.v_cache, pos0, n_heads, self.k_cache.size(1))
+        q = decode_ops.rope_rows(qkv, freqs_cis, self.k_cache, self.v_cache, pos0, n_heads, self.k_cache.size(1), self.lens)
         k, v = (c[:, :, pos0:pos0 + S].transpose(1, 2) for c in (self.k_cache, self.v_cache))
         if hash_keys:
             _hash_rows(self, k, v, t0=pos0)
-        self.lens.fill_(pos0 + S)
         return q, k, v
 
     def _write_run(self, pos0: int, k_val: Tensor, v_val: Tensor, v_norm: Optional[Tensor],
@@ -374,13 +373,13 @@ class Transformer(nn.Module):
                                           self.output.weight)
         # (a decode step's position is unchecked on the host: keep the table lookup in range)
         freqs_cis = self.freqs_cis[input_pos if pos0 is not None else input_pos.clamp(0, self.freqs_cis.size(0) - 1)]
+        ffn = None
         for layer in self.layers:
-            x = layer._run(x, input_pos, freqs_cis, sparse, pos0)
-        if rows is not None:
-            x = x[:, list(rows)]
-        elif last_only:
-            x = x[:, -1:]
-        return self.output(self.norm(x))
+            x, ffn = layer._run_pending(x, ffn, input_pos, freqs_cis, sparse, pos0)
+        pick = list(rows) if rows is not None else slice(-1, None) if last_only else slice(None)
+        if rows is not None or last_only:           # (the last sum only where it is wanted)
+            x, ffn = x[:, pick], None if ffn is None else ffn[:, pick]
+        return self.output(self.norm.add(x, ffn)[1])
 
     def forward(self, idx: Tensor, input_pos: Optional[Tensor] = None, *, pos0: Optional[int] = None,
                 last_only: bool = False, rows: Optional[Sequence[int]] = None) -> Tensor:
@@ -408,8 +407,14 @@ class TransformerBlock(nn.Module):
         self.attention_norm = RMSNorm(config.dim, config.norm_eps)
 
     def _run(self, x, input_pos, freqs_cis, sparse: bool, pos0):
-        h = x + self.attention._run(self.attention_norm(x), freqs_cis, input_pos, sparse, pos0)
-        return h + self.feed_forward(self.ffn_norm(h))
+        h, ffn = self._run_pending(x, None, input_pos, freqs_cis, sparse, pos0)
+        return h + ffn
+
+    def _run_pending(self, x, pending, input_pos, freqs_cis, sparse: bool, pos0):
+        """The block on x + pending (None: x); returns its residual stream and its feed-forward output, not yet added."""
+        x, n = self.attention_norm.add(x, pending)
+        h, n = self.ffn_norm.add(x, self.attention._run(n, freqs_cis, input_pos, sparse, pos0))
+        return h, self.feed_forward(n)
 
     def _run_fused(self, x, pending, input_pos, sparse: bool, step: "DecodeStep"):
         """One token through the block.  The block's input is x + pending (`pending`:
@@ -634,6 +639,18 @@ class RMSNorm(nn.Module):
             return decode_ops.add_rmsnorm(x, self.weight, self.eps)[1]
         xf = x.float()
         return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps)).type_as(x) * self.weight
+
+    def add(self, x: Tensor, residual: Optional[Tensor]) -> Tuple[Tensor, Tensor]:
+        """(x + residual, its norm), the add and the norm by one launch where the kernel takes both."""
+        if residual is None:
+            return x, self(x)
+        if (x.is_cuda and x.numel() > 0 and x.shape == residual.shape and x.shape[-1] == self.weight.numel()
+                and decode_ops.pointwise_fits(x, residual) and decode_ops.pointwise_fits(x, self.weight)
+                and type(self) is RMSNorm and not self._forward_hooks and not self._forward_pre_hooks
+                and not nn.modules.module._has_any_global_hook()):
+            return tuple(decode_ops.add_rmsnorm(x, self.weight, self.eps, residual=residual))
+        h = x + residual
+        return h, self(h)
 
 
 def precompute_freqs_cis(seq_len: int, n_elem: int, base: float = 10000, dtype=torch.bfloat16) -> Tensor:
