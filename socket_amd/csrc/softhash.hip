@@ -12,8 +12,10 @@
 // one launch computing in fp32 from the inputs as stored and rounding once, to
 // the output dtype.
 //
-// One workgroup per (table l, batch b, KV head): the K planes of the table and
-// the G query heads of the group sit in LDS, G*K lanes take the projections,
+// Three forms: on the matrix cores (bf16, 128 dims, K = 10, R = 1024), a wave to a
+// head (R <= 256), and the general one.  In that, one workgroup per (table l, batch b,
+// KV head): the K planes of the table and the G query heads of the group sit in LDS,
+// four lanes to a projection,
 // then every lane owns runs of four buckets and makes three sweeps over them
 // (maximum, sum of exponentials, normalised write), recomputing the K-term
 // logits each time rather than holding R/64 of them per head in registers.
