@@ -382,6 +382,94 @@ __global__ __launch_bounds__(kAttThreads) void sparse_stage1_kernel(
   }
 }
 
+// fp32 rows with short lists (at most row_entries(D)): a workgroup of sixteen waves takes a (b, h) row's whole list in one
+// pass, every entry requested at once, and writes the output itself.  The list's few hundred KB come through one CU at its
+// L2 rate in about the time a second launch takes: 32 rows x 196 entries of 128 dims 6.3 us where splits and their merge
+// take 7.4 (8 rows 5.4 / 6.2, 256 rows 11.3 / 14.3).  Past one pass a lone CU is behind (32 rows x 400: 10.1 / 8.4), and
+// 16-bit rows gain nothing (196 entries 6.8 / 6.1).
+constexpr int kRowWaves = 16, kRowUnroll = 8;
+constexpr int row_entries(int D) { return kRowWaves * (SOCKET_WAVE / (D / 4)) * kRowUnroll; }
+
+template <int D>
+__global__ __launch_bounds__(kRowWaves * SOCKET_WAVE) void sparse_row_kernel(
+    const float* __restrict__ q_, const float* __restrict__ k_, const float* __restrict__ v_, int64_t q_sb, int64_t q_sh,
+    int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, const int32_t* __restrict__ sparse_list,
+    int64_t list_sb, int64_t list_sh, const int32_t* __restrict__ sparse_len, int64_t len_sb, int64_t len_sh, int G, int kv_rows,
+    int list_width, float sm_scale, float* __restrict__ out, int64_t out_sb, int64_t out_sh) {
+  constexpr int LPR = D / 4, RPW = SOCKET_WAVE / LPR;
+  __shared__ float lds[kRowWaves][D + 2];
+  const int h = blockIdx.x, b = blockIdx.y, kvh = h / G;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int slot = lane / LPR, chunk = lane % LPR;
+  const float* kbase = k_ + b * k_sb + kvh * k_sh + chunk * 4;
+  const float* vbase = v_ + b * v_sb + kvh * v_sh + chunk * 4;
+  const int32_t* list = sparse_list + b * list_sb + h * list_sh;
+  const int len = min(sparse_len[b * len_sb + h * len_sh], list_width);
+  const float4 qf = *reinterpret_cast<const float4*>(q_ + b * q_sb + h * q_sh + chunk * 4);
+  int idx[kRowUnroll];
+#pragma unroll
+  for (int u = 0; u < kRowUnroll; ++u) {         // (past the list: its last entry, not live)
+    const int e = (u * kRowWaves + wave) * RPW + slot;
+    idx[u] = list[min(e, list_width - 1)];
+    if (e >= len || idx[u] >= kv_rows) idx[u] = -1;
+  }
+  float4 kr[kRowUnroll], vr[kRowUnroll];
+#pragma unroll
+  for (int u = 0; u < kRowUnroll; ++u) {
+    kr[u] = vr[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (idx[u] >= 0) {
+      kr[u] = *reinterpret_cast<const float4*>(kbase + (int64_t)idx[u] * k_ss);
+      vr[u] = *reinterpret_cast<const float4*>(vbase + (int64_t)idx[u] * v_ss);
+    }
+  }
+  float sc[kRowUnroll], m[1] = {-INFINITY}, l[1] = {0.f}, acc[1][4] = {{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int u = 0; u < kRowUnroll; ++u) {
+    const float d = group_sum<LPR>(qf.x * kr[u].x + qf.y * kr[u].y + qf.z * kr[u].z + qf.w * kr[u].w);
+    sc[u] = idx[u] >= 0 ? d * sm_scale : -INFINITY;
+    m[0] = fmaxf(m[0], sc[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < kRowUnroll; ++u) {
+    const float p = idx[u] >= 0 ? fast_exp(sc[u] - m[0]) : 0.f;
+    l[0] += p;
+    acc[0][0] += p * vr[u].x;
+    acc[0][1] += p * vr[u].y;
+    acc[0][2] += p * vr[u].z;
+    acc[0][3] += p * vr[u].w;
+  }
+  // row slots inside the wave, then the waves through LDS
+#pragma unroll
+  for (int d = LPR; d < SOCKET_WAVE; d <<= 1) {
+    auto partner = [&](float x) { return d == 16 ? lane_xor16(x) : d == 32 ? lane_xor32(x) : __shfl_xor(x, d, SOCKET_WAVE); };
+    const float m2 = partner(m[0]), l2 = partner(l[0]);
+    float a2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a2[i] = partner(acc[0][i]);
+    merge_state<4>(m[0], l[0], acc[0], m2, l2, a2);
+  }
+  if (lane < LPR) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lds[wave][chunk * 4 + i] = acc[0][i];
+    if (chunk == 0) {
+      lds[wave][D] = m[0];
+      lds[wave][D + 1] = l[0];
+    }
+  }
+  __syncthreads();
+  if (tid >= D) return;
+  float M = -INFINITY, sum = 0.f, val = 0.f;
+#pragma unroll
+  for (int w = 0; w < kRowWaves; ++w) M = fmaxf(M, lds[w][D]);
+#pragma unroll
+  for (int w = 0; w < kRowWaves; ++w) {
+    const float f = lds[w][D] == M ? 1.f : fast_exp(lds[w][D] - M);
+    sum += lds[w][D + 1] * f;
+    val += lds[w][tid] * f;
+  }
+  out[b * out_sb + h * out_sh + tid] = val / sum;      // (0/0 -> NaN when nothing was attended, as the reference)
+}
+
 // Dense flash-decode: rows [s*rows_per_split, ...) of one kv head, all G heads
 // of the group computed from a single read of each K and V row.
 template <class DT, int D, int GP>
@@ -1051,6 +1139,33 @@ extern "C" size_t socket_sparse_attention_workspace_bytes(int B, int Hq, int D, 
 
 namespace {
 
+// A workgroup to a row (sparse_row_kernel, where both sides' times are): fp32, lists of one pass, no more rows than CUs.
+bool one_row_each(int B, int Hq, int D, int max_len, int dtype) {
+  return dtype == SOCKET_F32 && (D == 16 || D == 32 || D == 64 || D == 128) && max_len <= row_entries(D) &&
+         (int64_t)B * Hq <= socket_device_limits().cu_count;
+}
+
+int launch_rows(const AttArgs& a, const int32_t* list, int64_t list_sb, int64_t list_sh, const int32_t* len, int64_t len_sb,
+                int64_t len_sh, void* out, int64_t out_sb, int64_t out_sh, int B, int Hq, int Hkv, int D, int kv_rows,
+                int list_width, hipStream_t s) {
+  const int st = check_common(a, B, Hq, Hkv, D);
+  if (st != SOCKET_OK) return st;
+  SOCKET_REQUIRE(list && len, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(kv_rows > 0, SOCKET_ERR_SHAPE);
+#define SOCKET_ROW(DD)                                                                                                        \
+  hipLaunchKernelGGL((sparse_row_kernel<DD>), dim3(Hq, B), dim3(kRowWaves * SOCKET_WAVE), 0, s, (const float*)a.q,            \
+                     (const float*)a.k, (const float*)a.v, a.q_sb, a.q_sh, a.k_sb, a.k_sh, a.k_ss, a.v_sb, a.v_sh, a.v_ss, list, \
+                     list_sb, list_sh, len, len_sb, len_sh, Hq / Hkv, kv_rows, list_width, 1.0f / sqrtf((float)D), (float*)out, \
+                     out_sb, out_sh)
+  if (D == 128) SOCKET_ROW(128);
+  else if (D == 64) SOCKET_ROW(64);
+  else if (D == 32) SOCKET_ROW(32);
+  else SOCKET_ROW(16);
+#undef SOCKET_ROW
+  SOCKET_LAUNCH_CHECK();
+  return SOCKET_OK;
+}
+
 int sparse_attention_on(void* workspace, const void* q, const void* k, const void* v, int dtype,
                         int64_t q_stride_b, int64_t q_stride_h, int64_t k_stride_b, int64_t k_stride_h,
                         int64_t k_stride_s, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_s,
@@ -1058,6 +1173,10 @@ int sparse_attention_on(void* workspace, const void* q, const void* k, const voi
                         const int32_t* sparse_len, int64_t len_stride_b, int64_t len_stride_h, void* out,
                         int64_t out_stride_b, int64_t out_stride_h, int B, int Hq, int Hkv, int D,
                         int kv_rows, int max_len, void* stream) {
+  if (one_row_each(B, Hq, D, max_len, dtype))
+    return launch_rows({q, k, v, dtype, q_stride_b, q_stride_h, k_stride_b, k_stride_h, k_stride_s, v_stride_b, v_stride_h, v_stride_s},
+                       sparse_list, list_stride_b, list_stride_h, sparse_len, len_stride_b, len_stride_h, out, out_stride_b,
+                       out_stride_h, B, Hq, Hkv, D, kv_rows, max_len, (hipStream_t)stream);
   const int bs = socket_sparse_attention_block_seq(B, Hq, max_len);
   const int nsplit = (max_len + bs - 1) / bs;
   float* mid_o = (float*)workspace;
@@ -1160,6 +1279,10 @@ extern "C" int socket_sparse_attention_static(const void* q, const void* k, cons
   unsigned int* arrive = nullptr;
   const int st = static_scratch(&ws, &arrive);
   if (st != SOCKET_OK) return st;
+  if (one_row_each(B, Hq, D, max_len, dtype))
+    return launch_rows({q, k, v, dtype, q_stride_b, q_stride_h, k_stride_b, k_stride_h, k_stride_s, v_stride_b, v_stride_h, v_stride_s},
+                       sparse_list, list_stride_b, list_stride_h, sparse_len, len_stride_b, len_stride_h, out, out_stride_b,
+                       out_stride_h, B, Hq, Hkv, D, kv_rows, max_len, (hipStream_t)stream);
   // Nothing in the partials array has to start at zero: a row's merge reads only the
   // splits the same launch wrote (the first ceil(len / split size) of the row).  One
   // launch: the workgroup that finishes a row's last split merges the row.
