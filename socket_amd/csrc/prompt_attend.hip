@@ -17,10 +17,11 @@
 // What bounds it: the matrix pipes and, per score, one exponential (three with a soft cap) and some
 // five other vector operations on the same SIMD; two workgroups per CU (64 KB of LDS each, at most
 // 256 registers) let one's softmax run beside the other's products.  32 rows per wave: a K fragment
-// of 1 KB feeds one 32-cycle product, which is what the LDS delivers.  Measured (causal, bf16, against
-// chunk_attend.hip's kernel): 32 heads over 8 kv heads of 128, cap 30, 8000 tokens 835 against 1209 us
-// (628 TFLOP/s); 32 heads of 128 + 64 shared dims, 8000 tokens 864 against 1849 us (759); without a cap
-// 6001 tokens 475 us (621), with weights rounded to 16 bits 325 us (909).
+// of 1 KB feeds one 32-cycle product, which is what the LDS delivers.  Measured (causal, bf16, repeated calls; in
+// brackets chunk_attend.hip's kernel): 32 heads over 8 kv heads of 128, cap 30, 8000 tokens 788 (1209) us, 666 TFLOP/s;
+// 32 heads of 128 + 64 shared dims, 8000 tokens 792 (1849) us, 828; without a cap 6001 tokens 399 us (740), with
+// weights rounded to 16 bits 307 us (961).  A rescale that waits until a maximum has grown by 2^8 takes 297 us, but then a
+// row's largest weight is rounded (error against float64 2.08e-3 instead of 2.02e-3) and depends on the wave's other rows.
 #include "mma_tiles.h"
 
 namespace {
@@ -185,10 +186,10 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
 #pragma unroll
         for (int i = 0; i < 16; ++i) mb = fmaxf(mb, s[nb][i]);
       mb = fmaxf(mb, lane_xor32(mb)) * c1;      // (c1 > 0)
-      // The accumulators are rescaled only when a row's maximum has grown by more than a factor of 2^8
-      // since the last time: weights up to 2^8 round as well as weights up to 1.
-      if (__builtin_amdgcn_ballot_w64(mb > m + 8.f || (m == -INFINITY && mb > m)) != 0) {
-        const float mn = fmaxf(m, mb);
+      // The shift is the row's own maximum so far, whatever the wave's other rows do: the largest weight is 1, which
+      // rounds exactly, and lanes whose maximum stays multiply by 1.
+      const float mn = fmaxf(m, mb);
+      if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {
         const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
         m = mn;
         l *= alpha;
@@ -198,23 +199,23 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
           for (int i = 0; i < 16; ++i) o[db][i] *= alpha;
       }
       const float shift = m == -INFINITY ? 0.f : m;
-      if (__builtin_amdgcn_ballot_w64(fabsf(shift) > 1048576.f) == 0) {
+      const bool large = fabsf(shift) > 1048576.f;
+      if (__builtin_amdgcn_ballot_w64(large) == 0) {
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            s[nb][i] = __builtin_amdgcn_exp2f(fmaf(s[nb][i], c1, -shift));
-            l += s[nb][i];
-          }
+          for (int i = 0; i < 16; ++i) s[nb][i] = __builtin_amdgcn_exp2f(fmaf(s[nb][i], c1, -shift));
       } else {        // scores so large that the product's rounding matters: round it as the maximum's was
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            s[nb][i] = __builtin_amdgcn_exp2f(pa_scaled_minus(s[nb][i], c1, shift));
-            l += s[nb][i];
-          }
+          for (int i = 0; i < 16; ++i)
+            s[nb][i] = __builtin_amdgcn_exp2f(large ? pa_scaled_minus(s[nb][i], c1, shift) : fmaf(s[nb][i], c1, -shift));
       }
+#pragma unroll
+      for (int nb = 0; nb < 2; ++nb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) l += s[nb][i];
     }
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {          // 16 keys: registers 8 (kk % 2) .. + 7 of block kk / 2
