@@ -704,7 +704,8 @@ int socket_chunk_attend(const socket_chunk_attention* args, void* stream);
 /* The same for prompts of 64 or 128 dims (or 128 value dims beside 192 key dims, the last ones shared) in bf16 or fp16 on
  * the matrix cores; other shapes, strides that are not multiples of 8 elements and unaligned tensors:
  * SOCKET_ERR_UNSUPPORTED.  `weights16`: the attention weights enter the second product rounded to the type instead of as
- * a sum of two numbers of it.  `positions` [T] (device, may be NULL): token t sees the keys up to positions[t] instead
+ * a sum of three numbers of it, which holds all bits of a 32-bit weight (two with a soft cap or shared key dims, whatever
+ * `weights16` is).  `positions` [T] (device, may be NULL): token t sees the keys up to positions[t] instead
  * of pos0 + t; needs one endless chunk, k_from = 0, no soft cap and no second key segment. */
 int socket_prompt_attention(const socket_chunk_attention* args, const int64_t* positions, int weights16, void* stream);
 

@@ -13,7 +13,7 @@
 
 // prompt_attend.hip
 bool prompt_attend_fits(const socket_chunk_attention& a);
-int prompt_attend_launch(const socket_chunk_attention& a, const int64_t* positions, bool weights16, hipStream_t s);
+int prompt_attend_launch(const socket_chunk_attention& a, const int64_t* positions, int terms, hipStream_t s);
 
 namespace {
 
@@ -608,7 +608,7 @@ extern "C" int socket_prompt_attention(const socket_chunk_attention* args, const
   SOCKET_REQUIRE(mma_fits(a) && prompt_attend_fits(a), SOCKET_ERR_UNSUPPORTED);
   // (with positions of its own a token may see any key: one endless chunk, all keys in k_new)
   SOCKET_REQUIRE(!positions || (a.chunk == INT32_MAX && a.k_from == 0 && a.softcap == 0.f && !a.k2), SOCKET_ERR_UNSUPPORTED);
-  return prompt_attend_launch(a, positions, weights16 != 0, (hipStream_t)stream);
+  return prompt_attend_launch(a, positions, weights16 ? 1 : 3, (hipStream_t)stream);
 }
 
 extern "C" int socket_chunk_attend(const socket_chunk_attention* args, void* stream) {
@@ -620,7 +620,7 @@ extern "C" int socket_chunk_attend(const socket_chunk_attention* args, void* str
   SOCKET_REQUIRE(a.dtype == SOCKET_F32 || a.dtype == SOCKET_BF16, SOCKET_ERR_UNSUPPORTED);
   hipStream_t s = (hipStream_t)stream;
   if (a.dtype == SOCKET_BF16 && mma_fits(a)) {
-    if (prompt_attend_fits(a)) return prompt_attend_launch(a, nullptr, false, s);
+    if (prompt_attend_fits(a)) return prompt_attend_launch(a, nullptr, 2, s);
     if (a.k2) {
       const int dq = a.D + a.D2;
       if (dq <= 64 && a.Dv <= 64) return launch_mma<64, 64, 2, true>(a, s);

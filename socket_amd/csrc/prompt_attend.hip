@@ -18,10 +18,11 @@
 // five other vector operations on the same SIMD; two workgroups per CU (64 KB of LDS each, at most
 // 256 registers) let one's softmax run beside the other's products.  32 rows per wave: a K fragment
 // of 1 KB feeds one 32-cycle product, which is what the LDS delivers.  Measured (causal, bf16, repeated calls; in
-// brackets chunk_attend.hip's kernel): 32 heads over 8 kv heads of 128, cap 30, 8000 tokens 788 (1209) us, 666 TFLOP/s;
-// 32 heads of 128 + 64 shared dims, 8000 tokens 792 (1849) us, 828; without a cap 6001 tokens 399 us (740), with
-// weights rounded to 16 bits 307 us (961).  A rescale that waits until a maximum has grown by 2^8 takes 297 us, but then a
-// row's largest weight is rounded (error against float64 2.08e-3 instead of 2.02e-3) and depends on the wave's other rows.
+// brackets chunk_attend.hip's kernel): 32 heads over 8 kv heads of 128, cap 30, 8000 tokens 795 (1017) us, 660 TFLOP/s;
+// 32 heads of 128 + 64 shared dims, 8000 tokens 798 (1538) us, 821; without a cap 6001 tokens 307 us (961) with weights
+// rounded to 16 bits, 399 (740) in two terms, 495 (596) in three.  A rescale that waits until a maximum has grown by 2^8
+// takes 297 us instead of 307, but then a row's largest weight is rounded (error against float64 2.08e-3 instead of
+// 2.02e-3) and depends on the wave's other rows.
 #include "mma_tiles.h"
 
 namespace {
@@ -30,11 +31,11 @@ constexpr int kPaRows = 32 * kPaWaves;
 constexpr float kPaMaxCap = 60.f;   // exp(60) * 2^31 keys < 3.4e38, exp(-60) > 1.2e-38
 
 // D: key dims, D2: dims of a second key segment that all heads share (with it the output may be gated),
-// DV: value dims.  SPLIT: weights enter the second product as a sum of two 16-bit numbers.  CAPPED:
-// scores pass softcap tanh(s / softcap), which bounds them, so that exp(score) needs no running
+// DV: value dims.  TERMS: weights enter the second product as a sum of so many 16-bit numbers; three of bf16 hold all
+// 24 bits of a 32-bit weight.  CAPPED: scores pass softcap tanh(s / softcap), which bounds them, so that exp(score) needs no running
 // maximum: p = exp(cap - 2 cap / (exp(2 s / cap) + 1)).  POS: token t sees the keys up to positions[t]
 // instead of pos0 + t (one endless chunk, a.k_from = 0).
-template <class DT, int D, int D2, int DV, bool SPLIT, bool CAPPED, bool POS>
+template <class DT, int D, int D2, int DV, int TERMS, bool CAPPED, bool POS>
 __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_chunk_attention a, const int64_t* positions) {
   constexpr int CK = D / 8, CK2 = D2 / 8, CV = DV / 8;            // 16-byte pieces per row
   constexpr int KS = D / 16, KS2 = D2 / 16, DB = DV / 32;
@@ -105,6 +106,8 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
 #pragma unroll
   for (int db = 0; db < DB; ++db) o[db] = pa_f32x16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   float l = 0.f, m = -INFINITY;
+  // (the largest weight: the later terms of small weights would leave fp16's range if it were 1)
+  constexpr float kUnit = DT::kEnum == SOCKET_F16 && TERMS > 1 ? 16384.f : 1.f;
   const float c1 = CAPPED ? 2.f * kPaLog2e * a.scale / a.softcap : a.scale * kPaLog2e;
   const float c2 = a.softcap * kPaLog2e;
 
@@ -186,7 +189,7 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
 #pragma unroll
         for (int i = 0; i < 16; ++i) mb = fmaxf(mb, s[nb][i]);
       mb = fmaxf(mb, lane_xor32(mb)) * c1;      // (c1 > 0)
-      // The shift is the row's own maximum so far, whatever the wave's other rows do: the largest weight is 1, which
+      // The shift is the row's own maximum so far, whatever the wave's other rows do: the largest weight is a power of two, which
       // rounds exactly, and lanes whose maximum stays multiply by 1.
       const float mn = fmaxf(m, mb);
       if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {
@@ -204,13 +207,13 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) s[nb][i] = __builtin_amdgcn_exp2f(fmaf(s[nb][i], c1, -shift));
+          for (int i = 0; i < 16; ++i) s[nb][i] = __builtin_amdgcn_exp2f(fmaf(s[nb][i], c1, -shift)) * kUnit;
       } else {        // scores so large that the product's rounding matters: round it as the maximum's was
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
           for (int i = 0; i < 16; ++i)
-            s[nb][i] = __builtin_amdgcn_exp2f(large ? pa_scaled_minus(s[nb][i], c1, shift) : fmaf(s[nb][i], c1, -shift));
+            s[nb][i] = __builtin_amdgcn_exp2f(large ? pa_scaled_minus(s[nb][i], c1, shift) : fmaf(s[nb][i], c1, -shift)) * kUnit;
       }
 #pragma unroll
       for (int nb = 0; nb < 2; ++nb)
@@ -219,20 +222,23 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
     }
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {          // 16 keys: registers 8 (kk % 2) .. + 7 of block kk / 2
-      uint4 ph, pl;
-      uint32_t* h = &ph.x;
-      uint32_t* lo = &pl.x;
+      uint4 p[TERMS];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float x = s[kk >> 1][8 * (kk & 1) + 2 * i], y = s[kk >> 1][8 * (kk & 1) + 2 * i + 1];
-        h[i] = PaType<DT>::pack2(x, y);
-        if constexpr (SPLIT) lo[i] = PaType<DT>::pack2(x - PaType<DT>::low(h[i]), y - PaType<DT>::high(h[i]));
+        float x = s[kk >> 1][8 * (kk & 1) + 2 * i], y = s[kk >> 1][8 * (kk & 1) + 2 * i + 1];
+#pragma unroll
+        for (int n = 0; n < TERMS; ++n) {     // (what is left after a term is exact)
+          const uint32_t w = PaType<DT>::pack2(x, y);
+          (&p[n].x)[i] = w;
+          x -= PaType<DT>::low(w);
+          y -= PaType<DT>::high(w);
+        }
       }
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         const uint4 vf = pa_values<CV>(vt, 16 * kk, db, lane);
-        o[db] = PaType<DT>::mfma(vf, ph, o[db]);
-        if constexpr (SPLIT) o[db] = PaType<DT>::mfma(vf, pl, o[db]);
+#pragma unroll
+        for (int n = 0; n < TERMS; ++n) o[db] = PaType<DT>::mfma(vf, p[n], o[db]);
       }
     }
   }
@@ -261,13 +267,13 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
     }
 }
 
-template <class DT, int D, int D2, int DV, bool SPLIT, bool CAPPED, bool POS = false>
+template <class DT, int D, int D2, int DV, int TERMS, bool CAPPED, bool POS = false>
 int pa_launch(const socket_chunk_attention& a, const int64_t* positions, hipStream_t s) {
   const int64_t rows = (int64_t)a.T * (a.H / a.G);
   const int64_t n = (rows + kPaRows - 1) / kPaRows * a.G * a.B;
   SOCKET_REQUIRE(n < (1LL << 31), SOCKET_ERR_SHAPE);
   constexpr int lds = 2 * kPaKeys * (D + D2 + DV) * 2;
-  auto kern = prompt_attend_kernel<DT, D, D2, DV, SPLIT, CAPPED, POS>;
+  auto kern = prompt_attend_kernel<DT, D, D2, DV, TERMS, CAPPED, POS>;
   if constexpr (lds > 65536) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
       return SOCKET_ERR_LAUNCH;
@@ -277,22 +283,26 @@ int pa_launch(const socket_chunk_attention& a, const int64_t* positions, hipStre
   return SOCKET_OK;
 }
 
+template <class DT, int D, int TERMS>
+int pa_terms(const socket_chunk_attention& a, const int64_t* positions, hipStream_t s) {
+  return positions ? pa_launch<DT, D, 0, D, TERMS, false, true>(a, positions, s) : pa_launch<DT, D, 0, D, TERMS, false>(a, nullptr, s);
+}
+
 template <class DT, int D>
-int pa_plain(const socket_chunk_attention& a, const int64_t* positions, bool weights16, hipStream_t s) {
+int pa_plain(const socket_chunk_attention& a, const int64_t* positions, int terms, hipStream_t s) {
   if constexpr (DT::kEnum == SOCKET_BF16) {
-    if (a.softcap > 0.f) return pa_launch<DT, D, 0, D, true, true>(a, nullptr, s);
+    if (a.softcap > 0.f) return pa_launch<DT, D, 0, D, 2, true>(a, nullptr, s);
+    if (terms == 2) return pa_launch<DT, D, 0, D, 2, false>(a, nullptr, s);
   }
-  if (weights16)
-    return positions ? pa_launch<DT, D, 0, D, false, false, true>(a, positions, s) : pa_launch<DT, D, 0, D, false, false>(a, nullptr, s);
-  return positions ? pa_launch<DT, D, 0, D, true, false, true>(a, positions, s) : pa_launch<DT, D, 0, D, true, false>(a, nullptr, s);
+  return terms == 1 ? pa_terms<DT, D, 1>(a, positions, s) : pa_terms<DT, D, 3>(a, positions, s);
 }
 
 template <class DT>
-int pa_run(const socket_chunk_attention& a, const int64_t* positions, bool weights16, hipStream_t s) {
+int pa_run(const socket_chunk_attention& a, const int64_t* positions, int terms, hipStream_t s) {
   if constexpr (DT::kEnum == SOCKET_BF16) {
-    if (a.k2) return pa_launch<DT, 128, 64, 128, true, false>(a, nullptr, s);
+    if (a.k2) return pa_launch<DT, 128, 64, 128, 2, false>(a, nullptr, s);
   }
-  return a.D == 64 ? pa_plain<DT, 64>(a, positions, weights16, s) : pa_plain<DT, 128>(a, positions, weights16, s);
+  return a.D == 64 ? pa_plain<DT, 64>(a, positions, terms, s) : pa_plain<DT, 128>(a, positions, terms, s);
 }
 
 }  // namespace
@@ -309,6 +319,8 @@ bool prompt_attend_fits(const socket_chunk_attention& a) {
   return (a.D == 64 || a.D == 128) && a.Dv == a.D && !a.gate;
 }
 
-int prompt_attend_launch(const socket_chunk_attention& a, const int64_t* positions, bool weights16, hipStream_t s) {
-  return a.dtype == SOCKET_F16 ? pa_run<DType_f16>(a, positions, weights16, s) : pa_run<DType_bf16>(a, positions, weights16, s);
+// terms: 1 or 3, or 2 as chunk_attend.hip's kernel has them (bf16, no positions); a capped score or a shared segment
+// always takes 2.
+int prompt_attend_launch(const socket_chunk_attention& a, const int64_t* positions, int terms, hipStream_t s) {
+  return a.dtype == SOCKET_F16 ? pa_run<DType_f16>(a, positions, terms, s) : pa_run<DType_bf16>(a, positions, terms, s);
 }

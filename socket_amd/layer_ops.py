@@ -352,7 +352,7 @@ def prompt_attend(q: Tensor, k: Tensor, v: Tensor, pos0: int, scale: float, posi
     """Causal attention of queries q [B,T,H,D] at positions pos0 .. over k / v [B,S,G,D], S = pos0 + T, of every
     position (any strides): [B,T,H,D].  `positions` (int64 [T], on the device): token t sees the keys up to
     positions[t] instead.  `weights16`: the weights enter the second product rounded to the inputs' type, as flash
-    attention kernels have it, instead of in two terms."""
+    attention kernels have it, instead of in 32 bits (three terms of that type)."""
     B, T, H, D = q.shape
     assert k.shape[1] == v.shape[1] == pos0 + T
     out = torch.empty(B, T, H, D, dtype=q.dtype, device=q.device)

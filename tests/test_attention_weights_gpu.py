@@ -1,5 +1,5 @@
-"""What the attention kernels' softmax weights keep: the largest weight of a row is exact, and a row's result depends on
-that row alone."""
+"""What the attention kernels' softmax weights keep: the largest weight of a row is exact, a row's result depends on that
+row alone, and over a cache the weights have 32 bits."""
 import math
 
 import pytest
@@ -59,3 +59,41 @@ def test_a_prompt_row_does_not_depend_on_its_neighbours(w16, gain):
     beside[:, :, 1::2] *= gain
     a, b = (layer_ops.prompt_attend(x, k, v, 0, 128 ** -0.5, weights16=w16) for x in (q, beside))
     assert torch.equal(a[:, ::2, ::2], b[:, ::2, ::2])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("counted", [True, False])
+def test_weights_over_a_cache_hold_32_bits(D, counted):
+    """Row r has in column r the value 1 under a weight p in [1/2, 1) and, under weights of 1, the first two bfloat16 terms of
+    -p: what is left is p's last eight bits, at most 2^-18, to the 2^-22 of the exponential's and the sums' 32 bits."""
+    x = torch.linspace(0.1, 0.69, D, device=DEV).bfloat16()
+    p = torch.exp(-x.double())
+    first = p.bfloat16().double()
+    second = (p - first).bfloat16().double()
+    T, S = D, D + 500
+    k = few_keys(S, D, torch.bfloat16, {70: (0.0, 0.0), 150: (0.0, 0.0), 200: (0.0, -1.0)})
+    v = torch.zeros(S, D, device=DEV, dtype=torch.bfloat16)
+    v[70], v[150], v[200] = -first.bfloat16(), -second.bfloat16(), 1.0
+    pos = None if counted else torch.arange(S - T, S, device=DEV)
+    got = layer_ops.prompt_attend(queries(x.float(), D, torch.bfloat16)[None, :, None], k[None, :, None], v[None, :, None], S - T,
+                                  1.0, pos)[0, :, 0].diagonal().double()
+    left = p - first - second
+    assert left.abs().max() > 2.0 ** -19
+    assert (got * (2 + p) - left).abs().max() < 2.0 ** -21
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_many_small_weights_over_a_cache(dt):
+    """4096 weights of about 1.3 x 2^-18 beside one of 1, whose value is 0: small ones keep their bits in fp16 too."""
+    S, D = 4097, 64
+    c = torch.tensor(math.log(1.3 * 2.0 ** -18)).to(dt)
+    k = torch.zeros(S, D, device=DEV, dtype=dt)
+    k[1:, 0] = c.to(DEV)
+    v = torch.ones(S, D, device=DEV, dtype=dt)
+    v[0] = 0
+    q = torch.zeros(1, 1, 1, D, device=DEV, dtype=dt)
+    q[..., 0] = 1
+    got = layer_ops.prompt_attend(q, k[None, :, None], v[None, :, None], S - 1, 1.0).double()
+    p = 4096 * math.exp(float(c.double()))
+    # (the score in base 2 is rounded to 2^-20 of a unit, which is 2^-20 of the weight)
+    assert (got / (p / (1 + p)) - 1).abs().max() < HALF_UNIT[dt] * 2 * 1.01
