@@ -121,10 +121,11 @@ __device__ __forceinline__ void bs_place(int num_rows, int& start_m, int& bh) {
 // into LDS (mma_tiles.h) and V^T fragments by transposing reads, so that no lane spends registers or
 // vector operations on staging.  A workgroup holds one tile of each at a time (32 KB); four of them
 // share a CU, and while one waits for its tiles the others work.  32700 tokens x 32 heads x 8 random
-// blocks: 450 us, 41 us per listed block (the register-staged form: 498), the same with every block
+// blocks: 459 us, 42 us per listed block (the register-staged form: 498), the same with every block
 // in the L2, so what bounds it is the chain of a tile -- copy, product, softmax, product -- at four waves
 // a SIMD.  Slower: 32x32 products with two waves sharing rows and merging key halves (505), a ring of
-// five tiles ahead (550), persistent workgroups that prefetch the next row block (580).
+// five tiles ahead (550), persistent workgroups that prefetch the next row block (580).  A rescale that waits until
+// a maximum has grown by 2^8 takes 448, but rounds a row's largest weight (error 2.22e-3 instead of 2.14e-3).
 template <class DT, int D>
 __global__ __launch_bounds__(kBsThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void block_sparse_tiles_kernel(
     const uint16_t* __restrict__ q_, const uint16_t* __restrict__ k_, const uint16_t* __restrict__ v_,
@@ -201,9 +202,9 @@ __global__ __launch_bounds__(kBsThreads) __attribute__((amdgpu_waves_per_eu(4, 4
       for (int r = 0; r < 4; ++r) mb = fmaxf(mb, s[nb][r]);
     mb = fmaxf(mb, lane_xor16(mb));
     mb = fmaxf(mb, lane_xor32(mb)) * scale_log2;
-    // (accumulators rescaled when a maximum has grown by more than 2^8, and large scores: see prompt_attend.hip)
-    if (__builtin_amdgcn_ballot_w64(mb > m + 8.f || (m == -INFINITY && mb > m)) != 0) {
-      const float mn = fmaxf(m, mb);
+    // (the row's own maximum, and large scores: see prompt_attend.hip)
+    const float mn = fmaxf(m, mb);
+    if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {
       const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
       m = mn;
       l *= alpha;
@@ -213,23 +214,23 @@ __global__ __launch_bounds__(kBsThreads) __attribute__((amdgpu_waves_per_eu(4, 4
         for (int r = 0; r < 4; ++r) o[db][r] *= alpha;
     }
     const float shift = m == -INFINITY ? 0.f : m;
-    if (__builtin_amdgcn_ballot_w64(fabsf(shift) > 1048576.f) == 0) {
+    const bool large = fabsf(shift) > 1048576.f;
+    if (__builtin_amdgcn_ballot_w64(large) == 0) {
 #pragma unroll
       for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[nb][r] = __builtin_amdgcn_exp2f(fmaf(s[nb][r], scale_log2, -shift));
-          l += s[nb][r];
-        }
+        for (int r = 0; r < 4; ++r) s[nb][r] = __builtin_amdgcn_exp2f(fmaf(s[nb][r], scale_log2, -shift));
     } else {
 #pragma unroll
       for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          s[nb][r] = __builtin_amdgcn_exp2f(pa_scaled_minus(s[nb][r], scale_log2, shift));
-          l += s[nb][r];
-        }
+        for (int r = 0; r < 4; ++r)
+          s[nb][r] = __builtin_amdgcn_exp2f(large ? pa_scaled_minus(s[nb][r], scale_log2, shift) : fmaf(s[nb][r], scale_log2, -shift));
     }
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) l += s[nb][r];
     // O^T += V^T . P^T, slots 0..3: keys 32c + 4q + r, slots 4..7: keys 32c + 16 + 4q + r
 #pragma unroll
     for (int c = 0; c < 2; ++c) {

@@ -5,6 +5,7 @@ import math
 import pytest
 import torch
 
+from socket_amd import block_sparse_flash_attention as bsa
 from socket_amd import layer_ops
 
 pytestmark = pytest.mark.gpu
@@ -59,6 +60,49 @@ def test_a_prompt_row_does_not_depend_on_its_neighbours(w16, gain):
     beside[:, :, 1::2] *= gain
     a, b = (layer_ops.prompt_attend(x, k, v, 0, 128 ** -0.5, weights16=w16) for x in (q, beside))
     assert torch.equal(a[:, ::2, ::2], b[:, ::2, ::2])
+
+
+def blocks_of(r):
+    """A list per row block: the first, three between, the two before the diagonal, the diagonal."""
+    return sorted({0, r // 4, r // 3, r // 2, max(r - 2, 0), max(r - 1, 0), r})
+
+
+def block_lists(H, R):
+    idx = torch.full((1, H, R, 7), R - 1, dtype=torch.int32)      # (padded with a block past the row: nothing visible)
+    for r in range(R - 1):
+        b = blocks_of(r)
+        idx[:, :, r, :len(b)] = torch.tensor(b, dtype=torch.int32)
+    idx[:, :, R - 1, :] = torch.arange(R - 7, R, dtype=torch.int32)
+    return idx.to(DEV)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+def test_the_largest_weight_of_a_block_sparse_row_is_exact(dt, D):
+    """Row block 9 lists blocks 0 and 8 (keys 3 and 512 are live)."""
+    T = 640
+    q, k, v, want = late_maximum(dt, 64, 512, T, D)
+    rows = torch.zeros(T, D, device=DEV, dtype=dt)
+    rows[576:] = q
+    idx = torch.zeros(1, 1, 10, 2, dtype=torch.int32, device=DEV)
+    idx[..., 1] = 8
+    # (scores are divided by sqrt(D))
+    got = bsa.random_walk_sparse_attention(rows[None, None], (k.float() * 8).to(dt)[None, None], v[None, None],
+                                           torch.tensor([T], dtype=torch.int32, device=DEV), idx)[0, 0, 576:, 1]
+    want = want if D == 64 else torch.sigmoid(q[:, 1].double() * 4 / D ** 0.5)
+    assert (got.double() - want).abs().max() < 1.01 * HALF_UNIT[dt]
+
+
+@pytest.mark.parametrize("gain", [3.0, 1e7])
+@pytest.mark.parametrize("D", [64, 128])
+def test_a_block_sparse_row_does_not_depend_on_its_neighbours(D, gain):
+    g = torch.Generator(device=DEV).manual_seed(2)
+    q, k, v = (torch.randn(1, 2, 700, D, generator=g, device=DEV).bfloat16() for _ in range(3))
+    beside = q.clone()
+    beside[:, :, 1::2] *= gain
+    lens = torch.tensor([700], dtype=torch.int32, device=DEV)
+    a, b = (bsa.random_walk_sparse_attention(x, k, v, lens, block_lists(2, 11)) for x in (q, beside))
+    assert torch.equal(a[:, :, ::2], b[:, :, ::2])
 
 
 @pytest.mark.parametrize("D", [64, 128])
