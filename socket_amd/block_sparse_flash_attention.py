@@ -56,10 +56,12 @@ def _most_forced(R: int, C: int, block_m: int, block_n: int, Tq: int, causal: bo
 def _lists(scores: torch.Tensor, K: int, block_m: int, block_n: int, Tq: int, causal: bool, diagonal: bool,
            window: Optional[int]) -> Optional[torch.Tensor]:
     """`_assemble` as one launch, for float32 scores on the device; None for what it does not take."""
+    if not plain_tensors(scores):
+        return None
     B, R, C = scores.shape
     k = min(K, C)
-    if not (scores.is_cuda and scores.dtype == torch.float32 and 0 < C <= LIST_MAX_BLOCKS and k <= LIST_MAX_PICKS and 0 < B <= 65535
-            and R > 0 and (R + 1) * block_m < 2 ** 31 and plain_tensors(scores)):
+    if not (scores.dtype == torch.float32 and 0 < C <= LIST_MAX_BLOCKS and k <= LIST_MAX_PICKS and 0 < B <= 65535
+            and R > 0 and (R + 1) * block_m < 2 ** 31):
         return None
     w = 0 if window is None else max(0, int(window))
     scores = scores if scores.stride(2) == 1 else scores.contiguous()

@@ -47,9 +47,11 @@ def rope_append(qkv: torch.Tensor, freqs_cis: torch.Tensor, input_pos: torch.Ten
 
 def rope_rows_fits(qkv: torch.Tensor, freqs: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor) -> bool:
     """Whether `rope_rows` takes the projected rows qkv [B,S,N] and these caches."""
+    if not plain_tensors(qkv, freqs, k_cache, v_cache):
+        return False
     per = 16 // qkv.element_size()
     D = k_cache.shape[-1]
-    return (qkv.is_cuda and plain_tensors(qkv, freqs, k_cache, v_cache) and qkv.dtype in (torch.bfloat16, torch.float16, torch.float32)
+    return (qkv.dtype in (torch.bfloat16, torch.float16, torch.float32)
             and k_cache.dtype == v_cache.dtype == qkv.dtype and k_cache.shape[0] == qkv.shape[0] <= 65535 and 0 < qkv.shape[1] <= 65535 * 8
             and k_cache.stride() == v_cache.stride() and k_cache.stride(-1) == qkv.stride(-1) == 1 and D % per == 0 and D % 2 == 0
             and all(st % per == 0 for st in qkv.stride()[:2] + k_cache.stride()[:3])

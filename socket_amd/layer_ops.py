@@ -334,8 +334,10 @@ def causal_attend(q: Tensor, k: Tensor, k_shared: Tensor, v: Tensor, pos0: int, 
 def prompt_attend_fits(q: Tensor, k: Tensor, v: Tensor) -> bool:
     """Whether `prompt_attend` takes q [B,T,H,D], k / v [B,S,G,D]: plain 16-bit device tensors of 64 or 128
     dims in rows a 16-byte load can read."""
+    if not plain_tensors(q, k, v):
+        return False
     D = q.shape[-1]
-    if not q.is_cuda or q.dtype not in (torch.bfloat16, torch.float16) or D not in (64, 128) or q.shape[1] < 1 or not plain_tensors(q, k, v):
+    if q.dtype not in (torch.bfloat16, torch.float16) or D not in (64, 128) or q.shape[1] < 1:
         return False
     for t in (q, k, v):
         if t.dtype != q.dtype or t.device != q.device or t.shape[-1] != D or t.stride(-1) != 1:

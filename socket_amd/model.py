@@ -623,8 +623,9 @@ class FeedForward(nn.Module):
 
     def forward(self, x: Tensor) -> Tensor:
         a, b = self.w1(x), self.w3(x)
-        if a.is_cuda and a.numel() > 0 and decode_ops.pointwise_fits(a, b) and a.shape == b.shape:
-            return self.w2(decode_ops.silu_mul(a, b))
+        if not torch.jit.is_scripting():
+            if decode_ops.pointwise_fits(a, b) and a.numel() > 0 and a.shape == b.shape:
+                return self.w2(decode_ops.silu_mul(a, b))
         return self.w2(F.silu(a) * b)
 
 
@@ -635,8 +636,9 @@ class RMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(dim))
 
     def forward(self, x: Tensor) -> Tensor:
-        if x.is_cuda and x.numel() > 0 and decode_ops.pointwise_fits(x, self.weight) and x.shape[-1] == self.weight.numel():
-            return decode_ops.add_rmsnorm(x, self.weight, self.eps)[1]
+        if not torch.jit.is_scripting():
+            if decode_ops.pointwise_fits(x, self.weight) and x.numel() > 0 and x.shape[-1] == self.weight.numel():
+                return decode_ops.add_rmsnorm(x, self.weight, self.eps)[1]
         xf = x.float()
         return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps)).type_as(x) * self.weight
 
@@ -644,8 +646,8 @@ class RMSNorm(nn.Module):
         """(x + residual, its norm), the add and the norm by one launch where the kernel takes both."""
         if residual is None:
             return x, self(x)
-        if (x.is_cuda and x.numel() > 0 and x.shape == residual.shape and x.shape[-1] == self.weight.numel()
-                and decode_ops.pointwise_fits(x, residual) and decode_ops.pointwise_fits(x, self.weight)
+        if (decode_ops.pointwise_fits(x, residual) and decode_ops.pointwise_fits(x, self.weight)
+                and x.numel() > 0 and x.shape == residual.shape and x.shape[-1] == self.weight.numel()
                 and type(self) is RMSNorm and not self._forward_hooks and not self._forward_pre_hooks
                 and not nn.modules.module._has_any_global_hook()):
             return tuple(decode_ops.add_rmsnorm(x, self.weight, self.eps, residual=residual))
