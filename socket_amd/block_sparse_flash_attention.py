@@ -23,7 +23,6 @@ sorted ascending (tests check it against a literal restatement of the pipeline).
 """
 from __future__ import annotations
 
-import functools
 from typing import Optional
 
 import torch
@@ -40,13 +39,17 @@ __all__ = [
 LIST_MAX_BLOCKS, LIST_MAX_PICKS = 4096, 256      # what one launch takes; longer lists are sorted by torch
 
 
-@functools.lru_cache(maxsize=256)
 def _most_forced(R: int, C: int, block_m: int, block_n: int, Tq: int, causal: bool, diagonal: bool, window: int) -> int:
-    """The largest number of forced blocks any row has (a function of the shape alone)."""
+    """The largest number of forced blocks any row has (a function of the shape alone).  Let d be the block of a row's
+    first query and `end` the last block any row may list.  While d <= end the count does not fall with the row (the
+    window fills up, block 0 and the diagonal leave each other); past it the window slides out of the list and the count
+    does not rise: the last row of the first kind or the first of the second has it."""
+    end = min(C - 1, (Tq - 1) // block_n) if causal else C - 1
+    inside = min(R - 1, ((end + 1) * block_n - 1) // block_m)
     most = 0
-    for r in range(R):
+    for r in (inside, min(inside + 1, R - 1)):
         d = r * block_m // block_n
-        last = min(C - 1, min((r + 1) * block_m - 1, Tq - 1) // block_n) if causal else C - 1
+        last = min(end, ((r + 1) * block_m - 1) // block_n) if causal else end
         lo, hi = (max(0, d - (window - 1)), min(d, last)) if window > 0 else (1, 0)
         rest = {0} | ({min(d, C - 1)} if diagonal else set())
         most = max(most, max(0, hi - lo + 1) + sum(c <= last and not lo <= c <= hi for c in rest))
