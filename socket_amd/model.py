@@ -594,7 +594,7 @@ class Attention(nn.Module):
             # (a block by itself is attended to as the library's flash kernels do it, weights in the model's
             # type; over the cache the masked form kept them in 32 bits, and a token sees what its position says)
             return layer_ops.prompt_attend(q, kt, vt, 0 if alone else pos0, self.head_dim ** -0.5,
-                                           positions=None if alone else input_pos, weights16=alone)
+                                           positions=None if alone else input_pos.contiguous(), weights16=alone)
         if alone:
             y = F.scaled_dot_product_attention(qh, k.transpose(1, 2), v.transpose(1, 2), is_causal=True,
                                                enable_gqa=gqa)

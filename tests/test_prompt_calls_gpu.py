@@ -1,0 +1,27 @@
+"""Prompt passes in the forms that callers may give them."""
+import pytest
+import torch
+
+from socket_amd.model import ModelArgs, Transformer
+
+pytestmark = pytest.mark.gpu
+
+
+def decoder(dtype=torch.bfloat16, batch=1):
+    torch.manual_seed(1)
+    model = Transformer(ModelArgs(block_size=64, vocab_size=96, n_layer=2, n_head=2, dim=128, intermediate_size=128,
+                                  L=4, K=4, R=16)).to("cuda", dtype).eval()
+    with torch.device("cuda"):
+        model.setup_caches(batch, 64)
+    return model
+
+
+@torch.no_grad()
+def test_a_portion_with_positions_of_any_stride():
+    model = decoder()
+    ids = torch.randint(0, 96, (1, 30), device="cuda")
+    pos = torch.arange(30, device="cuda")
+    column = torch.stack([pos, pos + 7], 1)[:, 0]
+    want = [model(ids[:, :11], pos[:11], pos0=0), model(ids[:, 11:], pos[11:], pos0=11)]
+    got = [model(ids[:, :11], column[:11], pos0=0), model(ids[:, 11:], column[11:], pos0=11)]
+    assert not column.is_contiguous() and all(torch.equal(a, b) for a, b in zip(got, want))
