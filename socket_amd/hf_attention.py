@@ -216,7 +216,8 @@ class SocketLlamaAttention(nn.Module):
             if attention_mask is not None:
                 y = F.scaled_dot_product_attention(q, k, v, attn_mask=attention_mask, scale=self.scaling,
                                                    enable_gqa=H != Hkv)
-            elif T_q > 1 and T_q == T_k and layer_ops.prompt_attend_fits(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)):
+            elif T_q > 1 and T_q == T_k and layer_ops.prompt_attend_fits(q.transpose(1, 2), k.transpose(1, 2),
+                                                                         v.transpose(1, 2), self.scaling):
                 y = layer_ops.prompt_attend(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), 0, self.scaling,
                                             weights16=True).transpose(1, 2)
             else:

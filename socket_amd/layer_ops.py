@@ -331,13 +331,13 @@ def causal_attend(q: Tensor, k: Tensor, k_shared: Tensor, v: Tensor, pos0: int, 
     return out
 
 
-def prompt_attend_fits(q: Tensor, k: Tensor, v: Tensor) -> bool:
-    """Whether `prompt_attend` takes q [B,T,H,D], k / v [B,S,G,D]: plain 16-bit device tensors of 64 or 128
-    dims in rows a 16-byte load can read."""
+def prompt_attend_fits(q: Tensor, k: Tensor, v: Tensor, scale: float = 1.0) -> bool:
+    """Whether `prompt_attend` takes q [B,T,H,D], k / v [B,S,G,D] and a scale: plain 16-bit device tensors of 64 or
+    128 dims in rows a 16-byte load can read, none empty, and a scale above zero (the kernel takes maxima before it)."""
     if not plain_tensors(q, k, v):
         return False
     D = q.shape[-1]
-    if q.dtype not in (torch.bfloat16, torch.float16) or D not in (64, 128) or q.shape[1] < 1:
+    if q.dtype not in (torch.bfloat16, torch.float16) or D not in (64, 128) or 0 in (q.numel(), k.numel()) or not scale > 0.0:
         return False
     for t in (q, k, v):
         if t.dtype != q.dtype or t.device != q.device or t.shape[-1] != D or t.stride(-1) != 1:

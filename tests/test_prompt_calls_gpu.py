@@ -2,7 +2,8 @@
 import pytest
 import torch
 
-from socket_amd.model import ModelArgs, Transformer
+from socket_amd import layer_ops
+from socket_amd.model import Attention, ModelArgs, Transformer
 
 pytestmark = pytest.mark.gpu
 
@@ -25,3 +26,19 @@ def test_a_portion_with_positions_of_any_stride():
     want = [model(ids[:, :11], pos[:11], pos0=0), model(ids[:, 11:], pos[11:], pos0=11)]
     got = [model(ids[:, :11], column[:11], pos0=0), model(ids[:, 11:], column[11:], pos0=11)]
     assert not column.is_contiguous() and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@torch.no_grad()
+def test_an_empty_batch():
+    att = Attention(ModelArgs(n_head=2, dim=128, L=4, K=4, R=16)).to("cuda", torch.bfloat16)
+    x = torch.zeros(0, 5, 128, device="cuda", dtype=torch.bfloat16)
+    freqs = torch.zeros(5, 32, 2, device="cuda", dtype=torch.bfloat16)
+    assert att._run(x, freqs, torch.arange(5, device="cuda"), False, 0).shape == (0, 5, 128)
+
+
+def test_scales_the_kernel_does_not_take():
+    """Zero (a mean over the keys) and below are left to torch's attention."""
+    q = torch.randn(1, 9, 2, 64, device="cuda").bfloat16()
+    assert layer_ops.prompt_attend_fits(q, q, q, 0.1)
+    for scale in (0.0, -0.1, float("nan")):
+        assert not layer_ops.prompt_attend_fits(q, q, q, scale)
