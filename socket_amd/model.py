@@ -379,7 +379,7 @@ class Transformer(nn.Module):
         pick = list(rows) if rows is not None else slice(-1, None) if last_only else slice(None)
         if rows is not None or last_only:           # (the last sum only where it is wanted)
             x, ffn = x[:, pick], None if ffn is None else ffn[:, pick]
-        return self.output(self.norm.add(x, ffn)[1])
+        return self.output(_add_norm(self.norm, x, ffn)[1])
 
     def forward(self, idx: Tensor, input_pos: Optional[Tensor] = None, *, pos0: Optional[int] = None,
                 last_only: bool = False, rows: Optional[Sequence[int]] = None) -> Tensor:
@@ -412,8 +412,8 @@ class TransformerBlock(nn.Module):
 
     def _run_pending(self, x, pending, input_pos, freqs_cis, sparse: bool, pos0):
         """The block on x + pending (None: x); returns its residual stream and its feed-forward output, not yet added."""
-        x, n = self.attention_norm.add(x, pending)
-        h, n = self.ffn_norm.add(x, self.attention._run(n, freqs_cis, input_pos, sparse, pos0))
+        x, n = _add_norm(self.attention_norm, x, pending)
+        h, n = _add_norm(self.ffn_norm, x, self.attention._run(n, freqs_cis, input_pos, sparse, pos0))
         return h, self.feed_forward(n)
 
     def _run_fused(self, x, pending, input_pos, sparse: bool, step: "DecodeStep"):
@@ -648,11 +648,19 @@ class RMSNorm(nn.Module):
             return x, self(x)
         if (decode_ops.pointwise_fits(x, residual) and decode_ops.pointwise_fits(x, self.weight)
                 and x.numel() > 0 and x.shape == residual.shape and x.shape[-1] == self.weight.numel()
-                and type(self) is RMSNorm and not self._forward_hooks and not self._forward_pre_hooks
+                and type(self) is RMSNorm and "forward" not in self.__dict__ and not self._forward_hooks and not self._forward_pre_hooks
                 and not nn.modules.module._has_any_global_hook()):
             return tuple(decode_ops.add_rmsnorm(x, self.weight, self.eps, residual=residual))
         h = x + residual
         return h, self(h)
+
+
+def _add_norm(norm: nn.Module, x: Tensor, residual: Optional[Tensor]) -> Tuple[Tensor, Tensor]:
+    """(x + residual, its norm); residual None: x.  `norm` may be any module that a caller has put there."""
+    if isinstance(norm, RMSNorm):
+        return norm.add(x, residual)
+    h = x if residual is None else x + residual
+    return h, norm(h)
 
 
 def precompute_freqs_cis(seq_len: int, n_elem: int, base: float = 10000, dtype=torch.bfloat16) -> Tensor:
