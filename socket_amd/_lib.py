@@ -13,6 +13,7 @@ import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p, POINTER
 
 import torch
+from torch import _C
 from torch.utils._device import DeviceContext
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -206,6 +207,8 @@ SIGNATURES = {
 _lib = None
 _core = None
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
 
 class SocketHipError(RuntimeError):
     """A libsocket_hip entry point returned a non-zero status."""
@@ -276,18 +279,31 @@ def require_device(*tensors) -> None:
 def observed() -> bool:
     """Whether torch operations are being recorded, transformed or replaced just now (torch.compile, jit.trace, make_fx,
     vmap, forward-mode differentiation, a dispatch or function mode): a launch by address would escape that."""
-    if (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._functorch.maybe_current_level() is not None or torch._C._len_torch_dispatch_stack() > 0):
+    if (torch.compiler.is_compiling() or _C._is_tracing() or torch.autograd.forward_ad._current_level >= 0
+            or _C._functorch.maybe_current_level() is not None or _C._len_torch_dispatch_stack() > 0):
         return True
+    modes = _C._len_torch_function_stack()
     # (a default device is a function mode too, which only sets where new tensors are made)
-    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+    return modes > 0 and any(type(_C._get_function_stack_at(i)) is not DeviceContext for i in range(modes))
+
+
+def one_device(tensors) -> bool:
+    """Whether the tensors lie on the same device, as torch's operations ask of theirs."""
+    device = tensors[0].device
+    for t in tensors:
+        if t.device != device:
+            return False
+    return True
 
 
 def plain_tensors(*tensors) -> bool:
-    """True for device tensors that nothing differentiates, transforms or traces, which a kernel may
+    """True for tensors of one HIP device that nothing differentiates, transforms or traces, which a kernel may
     therefore read and write by address in place of torch operations.  (Asked before any of their attributes:
     a tracer's stand-in for a tensor is no plain one.)"""
-    if observed() or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in tensors):
+    if observed():
         return False
     grad = torch.is_grad_enabled()
-    return all(t.is_cuda and not (grad and t.requires_grad) for t in tensors)
+    for t in tensors:
+        if type(t) not in _PLAIN or not t.is_cuda or (grad and t.requires_grad):
+            return False
+    return one_device(tensors)

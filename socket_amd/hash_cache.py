@@ -504,7 +504,7 @@ class SocketHashCache:
         """Whether one call of the library copies and hashes these rows (else: torch's copies, then the hash)."""
         kc, per = self.k_cache, 16 // self.k_cache.element_size()
         own = (kc, self.v_cache, self.codes, self.v_norm, self.lens, self.planes_words)
-        return (plain_tensors(k, v, *own) and k.dtype == v.dtype == kc.dtype == self.v_cache.dtype and k.device == v.device == kc.device
+        return (plain_tensors(k, v, *own) and k.dtype == v.dtype == kc.dtype == self.v_cache.dtype
                 and kc.dtype in (torch.bfloat16, torch.float16, torch.float32)
                 and k.shape == v.shape and tuple(k.shape[2:]) == (kc.shape[1], kc.shape[3]) and k.shape[1] > 0
                 and k.shape[3] % 8 == 0 and k.shape[3] <= HASH_DIM and self.planes_words.shape[1] == HASH_DIM and kc.shape[0] * kc.shape[1] <= 65535

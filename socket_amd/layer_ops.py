@@ -340,7 +340,7 @@ def prompt_attend_fits(q: Tensor, k: Tensor, v: Tensor, scale: float = 1.0) -> b
     if q.dtype not in (torch.bfloat16, torch.float16) or D not in (64, 128) or 0 in (q.numel(), k.numel()) or not scale > 0.0:
         return False
     for t in (q, k, v):
-        if t.dtype != q.dtype or t.device != q.device or t.shape[-1] != D or t.stride(-1) != 1:
+        if t.dtype != q.dtype or t.shape[-1] != D or t.stride(-1) != 1:
             return False
         if t.data_ptr() % 16 != 0 or any(st % 8 != 0 for st in t.stride()[:3]):
             return False

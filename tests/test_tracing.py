@@ -77,6 +77,17 @@ def test_every_tracer_is_seen(name):
         assert not _lib.observed()
 
 
+def test_tensors_of_two_devices_are_told_apart():
+    a, b = torch.ones(2), torch.ones(2, device="meta")
+    assert _lib.one_device((a, a)) and _lib.one_device((b,)) and not _lib.one_device((a, b))
+
+
+@pytest.mark.gpu
+def test_a_kernel_takes_no_operand_of_another_device():
+    x = torch.ones(4, 64, device="cuda")
+    assert decode_ops.pointwise_fits(x, x) and not decode_ops.pointwise_fits(x, x.cpu())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("make", [norm, feed_forward])
 @pytest.mark.parametrize("name", ["jit", "make_fx", "make_fx_pre_dispatch", "compile", "fx", "script"])
