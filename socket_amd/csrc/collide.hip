@@ -205,18 +205,30 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
   }
   const size_t lds = (size_t)ct * per_table;
   const bool vec = T % 8 == 0 && (((uintptr_t)key_buckets | (uintptr_t)allowed | (uintptr_t)v_hist | (uintptr_t)out) & 15) == 0;
-  // The widest workgroup that still leaves one to every CU (each pulls the whole table through LDS, and its
-  // waves are all that a CU has in flight): 32 heads x 32768 tokens, L60 x R1024, 1024 lanes on half the CUs with
-  // an fp32 table in two slices 43.6 us, 512 lanes with the bf16 table in one 33.7.  Short rows take a quarter, so
-  // that a tile is not mostly idle lanes.
+  // Lanes of a workgroup.  It pulls its row's whole table through LDS with them, which is quicker the more there are, and
+  // the chip has at most CUs x (tables that fit a CU's LDS) workgroups at work.  While all workgroups are at work at
+  // once narrower ones leave fewer CUs idle; past that each further round costs what the first did, and 1024 lanes need
+  // the fewest.  us at 256 / 512 / 1024 lanes, rows of 16-byte code loads (T % 8 == 0) | of 2-byte ones:
+  //   32 rows, L60 x R1024 fp32    4088: 32 / 24 / 23     8192: 34 / 29 / 36     32768: 66 / 35 / 40    48000: 99 / 61 / 44
+  //                              | 2051: 73 / 57 / 56     9003: 81 / 99 / 145    24001: 159 / 101 / 145 32771: 228 / 193 / 146
+  //   the same, bf16               4088: 23 / 22 / 22     5000: 25 / 25 / 27     32768: 51 / 28 / 36    65536: 93 / 58 / 50
+  //                              | 2051: 54 / 51 / 51     9003: 69 / 88 / 126    24001: 134 / 89 / 126  32771: 199 / 172 / 126
+  //   32 rows, L32 x R256 fp32     4088: 11 / 12 / 12    12000: 13 / 13 / 18     24000: 16 / 15 / 19
+  //                              | 4093: 30 / 40 / 40    12003: 37 / 48 / 75     24001: 52 / 51 / 76
+  // Just past 4096 tokens 512 lanes make a second, nearly empty workgroup of what 1024 hold in one.  A table in one
+  // slice (bf16) and few workgroups: 28 rows, L48, 5000 tokens 18.6 / 20.3 us at 256 / 512 lanes; 8 rows, L60, 16384: 21 / 23.
+  // 2-byte loads bound a lane more than the table does, so that 256 lanes pay from 2800 tokens on; there a few 512-lane
+  // workgroups over the CUs (264) still take 128 us where 1024 lanes take 145.
   auto tiles_of = [&](int th) { return (T + th * kTokensPerThread - 1) / (th * kTokensPerThread); };
-  int threads = 256;
-  if (T > 256 * kTokensPerThread)
-    for (int th : {1024, 512})
-      if ((int64_t)tiles_of(th) * B * H >= lim.cu_count) {
-        threads = th;
-        break;
-      }
+  auto fit = [&](int th, int workgroups) { return (int64_t)tiles_of(th) * B * H <= workgroups; };
+  const bool shares = 2 * lds <= budget;      // a CU holds several workgroups' tables
+  const int cus = lim.cu_count;
+  int threads = 1024;
+  if (T <= 256 * kTokensPerThread || (shares && fit(256, cus))) threads = 256;
+  else if (vec && ct >= L && T > 4096 && fit(256, cus * 3 / 8)) threads = 256;
+  else if (vec && T > 4608 && fit(512, cus)) threads = 512;
+  else if (!vec && T > 2816 && fit(256, cus)) threads = 256;
+  else if (!vec && T > 4096 && fit(512, cus + cus / 32)) threads = 512;
   const int tiles = tiles_of(threads);
   // tiles per workgroup: as many as leave two workgroups per CU (they amortise the
   // slices a workgroup pulls through LDS), at most 8
