@@ -1027,7 +1027,14 @@ extern "C" int socket_cache_append(const void* k, const void* v, int dtype, int6
 #undef SOCKET_COPY
     SOCKET_LAUNCH_CHECK();
   }
-  if (!streamed) return launch_staged(a, lim, s);
+  if (!streamed) {
+    // (from the rows just written: whole heads in order, partly still in the memory-side cache.  float32, 8 x 30000 rows of
+    // 128, 32 x 8 planes: 75 us against 85 from the caller's rows, which lie a token apart)
+    const int64_t first = (int64_t)t0 * cache_stride_s * (16 / per16);
+    a.k = (const char*)k_cache + first, a.v = (const char*)v_cache + first;
+    a.k_sb = a.v_sb = cache_stride_b, a.k_sh = a.v_sh = cache_stride_h, a.k_ss = a.v_ss = cache_stride_s;
+    return launch_staged(a, lim, s);
+  }
   return D == 64 ? launch_stream<64, true>(a, lim, s) : launch_stream<128, true>(a, lim, s);
 }
 
