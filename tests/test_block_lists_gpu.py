@@ -9,10 +9,12 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-# (columns around the 64 of a lane's bits and a register per lane, the 256 and 1024 of the launch's variants; more picks than columns)
+# (columns around the 64 of a lane's bits and a register per lane, the 256 and 1024 of the launch's variants, its last
+# column and most picks, one column more, which torch sorts; more picks than columns)
 @pytest.mark.parametrize("R,C,K,window,causal,diag", [(1, 1, 1, None, True, True), (5, 5, 9, 2, True, True), (64, 64, 8, 4, True, False),
                                                       (65, 65, 12, None, False, True), (256, 257, 8, 300, True, True),
-                                                      (70, 1024, 16, 1, False, False), (1030, 1030, 8, 4, True, True), (90, 31, 5, 3, True, True)])
+                                                      (70, 1024, 16, 1, False, False), (1030, 1030, 8, 4, True, True), (90, 31, 5, 3, True, True),
+                                                      (20, 4096, 256, 3, False, True), (20, 4097, 8, 3, False, True)])
 def test_block_level_lists(R, C, K, window, causal, diag):
     g = torch.Generator().manual_seed(R + K)
     for scores in (torch.rand(2, R, C, generator=g), torch.zeros(2, R, C),
@@ -20,11 +22,11 @@ def test_block_level_lists(R, C, K, window, causal, diag):
         kw = dict(enforce_causal_blocks=causal, force_include_diagonal=diag, window_blocks=window)
         want = bsa.random_walk_indices_from_block_probs(scores, K, **kw)
         got = bsa.random_walk_indices_from_block_probs(scores.to(DEV), K, **kw)
-        assert torch.equal(got.cpu(), want)
+        assert torch.equal(got.cpu(), want) and torch.equal(want, bso.random_walk_indices_from_block_probs(scores, K, causal, diag, window))
+        assert (bsa._lists(scores.to(DEV), K, 1, 1, R, causal, diag, window) is None) == (C > 4096)
         view = torch.zeros(2, R, C + 3, device=DEV)[..., :C]
         view.copy_(scores)
         assert torch.equal(bsa.random_walk_indices_from_block_probs(view, K, **kw).cpu(), want)
-    assert torch.equal(want, bso.random_walk_indices_from_block_probs(scores, K, **kw)) or not (causal and diag)
 
 
 @pytest.mark.parametrize("Tq,Tk,bm,bn,K,window", [(130, 130, 64, 64, 2, 1), (300, 200, 64, 32, 6, 3), (129, 700, 32, 64, 4, None)])
