@@ -219,7 +219,7 @@ class SocketLlamaAttention(nn.Module):
             elif T_q > 1 and T_q == T_k and layer_ops.prompt_attend_fits(q.transpose(1, 2), k.transpose(1, 2),
                                                                          v.transpose(1, 2), self.scaling):
                 y = layer_ops.prompt_attend(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), 0, self.scaling,
-                                            weights16=True).transpose(1, 2)
+                                            weights16=layer_ops.flash_weights()).transpose(1, 2)
             else:
                 y = F.scaled_dot_product_attention(q, k, v, is_causal=T_q > 1 and T_q == T_k, scale=self.scaling,
                                                    enable_gqa=H != Hkv)

@@ -348,6 +348,12 @@ def prompt_attend_fits(q: Tensor, k: Tensor, v: Tensor, scale: float = 1.0) -> b
             and k.shape[1] < 2 ** 30 and max(k.stride(1), v.stride(1)) < 2 ** 24 and min(k.stride() + v.stride()) >= 0)
 
 
+def flash_weights() -> bool:
+    """Whether a prompt by itself may round its attention weights to the inputs' type, as torch's flash kernels do:
+    unless the caller has them switched off (torch.nn.attention.sdpa_kernel, enable_flash_sdp)."""
+    return torch.backends.cuda.flash_sdp_enabled()
+
+
 @torch.no_grad()
 def prompt_attend(q: Tensor, k: Tensor, v: Tensor, pos0: int, scale: float, positions: Optional[Tensor] = None,
                   weights16: bool = False) -> Tensor:

@@ -592,9 +592,11 @@ class Attention(nn.Module):
         kt, vt = (k, v) if alone else (kc.transpose(1, 2), vc.transpose(1, 2))
         if layer_ops.prompt_attend_fits(q, kt, vt):
             # (a block by itself is attended to as the library's flash kernels do it, weights in the model's
-            # type; over the cache the masked form kept them in 32 bits, and a token sees what its position says)
+            # type unless these are switched off; over the cache the masked form kept them in 32 bits, and a token
+            # sees what its position says)
             return layer_ops.prompt_attend(q, kt, vt, 0 if alone else pos0, self.head_dim ** -0.5,
-                                           positions=None if alone else input_pos.contiguous(), weights16=alone)
+                                           positions=None if alone else input_pos.contiguous(),
+                                           weights16=alone and layer_ops.flash_weights())
         if alone:
             y = F.scaled_dot_product_attention(qh, k.transpose(1, 2), v.transpose(1, 2), is_causal=True,
                                                enable_gqa=gqa)

@@ -39,3 +39,19 @@ def test_scales_the_kernel_does_not_take():
     assert layer_ops.prompt_attend_fits(q, q, q, 0.1)
     for scale in (0.0, -0.1, float("nan")):
         assert not layer_ops.prompt_attend_fits(q, q, q, scale)
+
+
+@torch.no_grad()
+def test_weights_keep_32_bits_where_flash_kernels_are_switched_off():
+    """As torch's attention then does.  Values of +1 and -1 under weights 1 and p leave (1 - p) / (1 + p), of which weights
+    in bfloat16 leave a multiple of 2^-9."""
+    att = decoder().layers[0].attention
+    q, k, v = (torch.zeros(1, 2, 2, 64, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    q[..., 0], k[:, 0, :, 0] = 1.0, -0.01171875
+    v[:, 0], v[:, 1] = -1.0, 1.0
+    want = torch.tanh(torch.tensor(0.01171875 / 8 / 2, dtype=torch.float64)).item()
+    pos = torch.arange(2, device="cuda")
+    with torch.nn.attention.sdpa_kernel(torch.nn.attention.SDPBackend.MATH):
+        exact = att._prefill_attention(q, k, v, pos, 0)[0, 1, 0, 0].item()
+    flash = att._prefill_attention(q, k, v, pos, 0)[0, 1, 0, 0].item()
+    assert abs(exact / want - 1) < 2.0 ** -8 and abs(flash / want - 1) > 2.0 ** -3
