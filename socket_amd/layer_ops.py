@@ -348,6 +348,19 @@ def prompt_attend_fits(q: Tensor, k: Tensor, v: Tensor, scale: float = 1.0) -> b
             and k.shape[1] < 2 ** 30 and max(k.stride(1), v.stride(1)) < 2 ** 24 and min(k.stride() + v.stride()) >= 0)
 
 
+def portion_pays(B: int, H: int, G: int, D: int, T: int, S: int) -> bool:
+    """Whether `prompt_attend` is the quicker way for T tokens over a cache of S keys, B sequences of H heads over G.
+    A workgroup of it walks all keys of its rows: 8.2 + 0.148 D us per 1000 keys, however few workgroups there are.  Torch's
+    masked form spreads a grouped portion over the chip in some 20 launches: at least 150 us; 75 us and, per 1000
+    keys and head, 0.0066 D + 0.0125 T us.  Both sides of the line, kernel / torch, us: 4 heads of 64, 100000 keys, 16 tokens 1804 / 470, 200
+    tokens 1822 / 1474, 300 tokens level; 16 of 128, 32000 keys, 16 tokens 893 / 602, 64 tokens 903 / 896; 28 of 128, 100000
+    keys, 2 tokens 2713 / 2326; 32 of 128, 32000 keys, 2 tokens 878 / 973, 1024 tokens 1013 / 13223; 8 of 128, 6000 keys, 16
+    tokens 177 / 167.  (Without groups torch takes a slower form: the kernel was ahead everywhere.)"""
+    if H == G:
+        return True
+    return S * (8.2 + 0.148 * D) < max(150e3, 75e3 + S * B * H * (0.0066 * D + 0.0125 * T))
+
+
 def flash_weights() -> bool:
     """Whether a prompt by itself may round its attention weights to the inputs' type, as torch's flash kernels do:
     unless the caller has them switched off (torch.nn.attention.sdpa_kernel, enable_flash_sdp)."""

@@ -590,7 +590,8 @@ class Attention(nn.Module):
             end = pos0 + q.shape[1]
             kc, vc = self.kv_cache.k_cache[:, :, :end], self.kv_cache.v_cache[:, :, :end]
         kt, vt = (k, v) if alone else (kc.transpose(1, 2), vc.transpose(1, 2))
-        if layer_ops.prompt_attend_fits(q, kt, vt):
+        if layer_ops.prompt_attend_fits(q, kt, vt) and (
+                alone or layer_ops.portion_pays(q.shape[0], self.n_head, self.n_local_heads, self.head_dim, q.shape[1], kt.shape[1])):
             # (a block by itself is attended to as the library's flash kernels do it, weights in the model's
             # type unless these are switched off; over the cache the masked form kept them in 32 bits, and a token
             # sees what its position says)
