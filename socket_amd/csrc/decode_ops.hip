@@ -585,10 +585,11 @@ extern "C" int socket_rope_rows(const void* qkv, int dtype, int64_t qkv_stride_b
 namespace {
 
 // The first index of a row's greatest value (a NaN counts as the greatest, as in torch.argmax), one workgroup to a
-// row; workgroup 0 also advances the position.  The row comes from L2 (the product before has just written it) and
-// one CU reads 128 KB of it in about a microsecond, so splitting it over workgroups would only add a pass: 32000
-// logits take 5 us with the launch, where torch's reduction, its cast to int, the copy to the token
-// buffer and the position's add took 26 us in four launches.
+// row; workgroup 0 also advances the position.  The row comes from L2 (the product before has just written it), and
+// past some 50000 logits the compares of its one CU bound it: four vector operations an element, NaNs told by one compare
+// for two elements and taken care of aside.  us in a replayed graph, bf16, this / torch's argmax, its cast, the copy to
+// the token buffer and the position's add (four launches): 32000 logits 4.7 / 16, 128256 9.1 / 36, 256000 15.8 / 17
+// (torch splits a single row that long over workgroups; four rows 16.1 / 64).
 constexpr int kGreedyThreads = 1024;
 
 template <class DT, bool VEC>
@@ -597,20 +598,31 @@ __global__ __launch_bounds__(kGreedyThreads) void greedy_kernel(const void* __re
   constexpr int E = VEC ? DT::kPer16B : 1, U = 8;      // elements of a load, loads in flight
   __shared__ uint64_t red[kGreedyThreads / 64];
   const int64_t row = blockIdx.x * stride;
-  uint32_t best = 0;
-  int at = 0;
   const int pieces = V / E;
-  auto take = [&](uint32_t key, int i) {
-    if (key > best) best = key, at = i;                // (a lane's indices rise: the first of equals stays)
+  float best = -INFINITY;                               // (a lane's indices rise: the first of equals, or of NaNs, stays)
+  int at = (int)threadIdx.x < pieces ? threadIdx.x * E : INT32_MAX;
+  auto take = [&](const float (&f)[E], int first) {
+    bool nan = false;
+#pragma unroll
+    for (int e = 0; e < E; e += 2) nan |= __builtin_isunordered(f[e], f[E > 1 ? e + 1 : e]);
+    if (nan) {                                          // (rare)
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (best == best && !(f[e] <= best)) best = f[e], at = first + e;
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (f[e] > best) best = f[e], at = first + e;
+    }
   };
   for (int p0 = 0; p0 < pieces; p0 += U * kGreedyThreads) {
     uint4 w[VEC ? U : 1];
-    float x[U];
+    float x[U][1];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int p = min(p0 + u * kGreedyThreads + (int)threadIdx.x, pieces - 1);
       if constexpr (VEC) w[u] = *reinterpret_cast<const uint4*>((const typename DT::storage*)logits + row + (int64_t)p * E);
-      else x[u] = ld<DT>(logits, row + p);
+      else x[u][0] = ld<DT>(logits, row + p);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -619,18 +631,18 @@ __global__ __launch_bounds__(kGreedyThreads) void greedy_kernel(const void* __re
       if constexpr (VEC) {
         float f[E];
         unpack16<DT>(w[u], f);
-#pragma unroll
-        for (int e = 0; e < E; ++e) take(score_to_key(f[e]), p * E + e);
+        take(f, p * E);
       } else {
-        take(score_to_key(x[u]), p);
+        take(x[u], p);
       }
     }
   }
   if (VEC && (int)threadIdx.x < V - pieces * E) {
     const int i = pieces * E + threadIdx.x;
-    take(score_to_key(ld<DT>(logits, row + i)), i);
+    const float x = ld<DT>(logits, row + i);
+    if (best == best && !(x <= best)) best = x, at = i;
   }
-  uint64_t m = ((uint64_t)best << 32) | (0xffffffffu - (uint32_t)at);
+  uint64_t m = ((uint64_t)score_to_key(best) << 32) | (0xffffffffu - (uint32_t)at);
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
     const uint64_t o = __shfl_xor(m, d, 64);

@@ -34,3 +34,17 @@ def test_columns_and_other_types_take_the_general_way():
     assert torch.equal(decode_ops.greedy_tokens(x.t()), x.argmax(0, keepdim=True).t().int())
     y = torch.randn(3, 50, device="cuda", dtype=torch.float64)
     assert torch.equal(decode_ops.greedy_tokens(y), y.argmax(-1, keepdim=True).int())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V", [17, 30000, 256001])
+def test_many_nans_and_infinities(V, dtype):
+    """Among the elements of one load too: the first NaN whatever stands before and after it."""
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(8, V + 7, generator=g).to(dtype)[:, :V]
+    for row, share in enumerate((0.0, 1e-4, 0.01, 0.3, 1.0)):
+        x[row, torch.rand(V, generator=g) < share] = float("nan")
+    x[5:, torch.rand(V, generator=g) < 0.2] = float("inf")
+    x[6, V // 2:] = float("nan")
+    x[7] = -x[7]
+    assert torch.equal(decode_ops.greedy_tokens(x.cuda()).cpu(), x.float().argmax(-1, keepdim=True).int())
