@@ -19,10 +19,10 @@
 // 256 registers) let one's softmax run beside the other's products.  32 rows per wave: a K fragment
 // of 1 KB feeds one 32-cycle product, which is what the LDS delivers.  Measured (causal, bf16, repeated calls; in
 // brackets chunk_attend.hip's kernel): 32 heads over 8 kv heads of 128, cap 30, 8000 tokens 795 (1017) us, 660 TFLOP/s;
-// 32 heads of 128 + 64 shared dims, 8000 tokens 798 (1538) us, 821; without a cap 6001 tokens 307 us (961) with weights
-// rounded to 16 bits (385 within a prompt pass), 399 (740) in two terms, 495 (596) in three.  A rescale that waits until a maximum has grown by 2^8
-// takes 297 us instead of 307, but then a row's largest weight is rounded (error against float64 2.08e-3 instead of
-// 2.02e-3) and depends on the wave's other rows.
+// 32 heads of 128 + 64 shared dims, 8000 tokens 798 (1538) us, 821; without a cap 6001 tokens 307 us (961 TFLOP/s; 385 us
+// within a prompt pass) with weights rounded to 16 bits, 399 (740) in two terms, 495 (596) in three.  A rescale that
+// waits until a maximum has grown by 2^8 takes 297 us instead of 307, but then a row's largest weight is rounded (error
+// against float64 2.08e-3 instead of 2.02e-3) and depends on the wave's other rows.
 #include "mma_tiles.h"
 
 namespace {
