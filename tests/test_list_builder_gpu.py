@@ -14,7 +14,8 @@ DEV = "cuda"
 @pytest.mark.parametrize("qdt,vdt", [(torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16), (torch.float32, torch.float32),
                                      (torch.bfloat16, torch.bfloat16)])
 @pytest.mark.parametrize("B,H,T,L,P,sink,window,M", [(1, 2, 5, 3, 4, 2, 2, 9), (2, 3, 2056, 12, 6, 4, 64, 100), (1, 2, 4099, 9, 8, 0, 0, 33),
-                                                     (1, 40, 30000, 4, 7, 4, 128, 64), (2, 130, 8200, 3, 5, 30, 9000, 50)])
+                                                     (1, 40, 30000, 4, 7, 4, 128, 64), (2, 130, 8200, 3, 5, 30, 9000, 50),
+                                                      (1, 3, 20000, 3, 5, 3000, 12000, 300), (2, 2, 9000, 3, 5, 0, 4095, 1)])
 def test_against_the_oracle(B, H, T, L, P, sink, window, M, qdt, vdt):
     g = torch.Generator().manual_seed(T)
     q = torch.rand(B, H, L, 1 << P, generator=g).to(qdt)
