@@ -22,11 +22,12 @@ def separate(cache, pos0, k, v):
 
 # (S of 4100 in 8 rows is past a 128-key tile per CU, the streamed launch; 40 dims are three whole MFMA steps less a
 # half, 20 are no whole 16-byte pieces in 16 bits and stay with torch's copies; from some 3300 rows on, up to 13000, the
-# launch without LDS takes 64 of them at a time, 64-row tiles that cross from head to head among them)
+# launch without LDS takes 64 of them at a time, 64-row tiles that cross from head to head among them; 160004 float32
+# rows of 128 are past the 128 MB from which the hash reads the cache)
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("B,S,H,D,pos0", [(2, 1, 3, 128, 7), (1, 63, 2, 64, 0), (3, 129, 2, 40, 5), (1, 4100, 8, 128, 3),
                                           (2, 4097, 4, 64, 1), (2, 70, 2, 20, 2), (2, 777, 8, 64, 1003), (3, 401, 3, 40, 2),
-                                          (2, 401, 7, 128, 3)])
+                                          (2, 401, 7, 128, 3), (1, 40001, 4, 128, 5)])
 def test_append_equals_copies_and_hash(B, S, H, D, pos0, dt):
     g = torch.Generator(device=DEV).manual_seed(S + D)
     cache = hash_cache.SocketHashCache(B, pos0 + S + 9, H, D, 60, 10, dtype=dt, device=DEV)
