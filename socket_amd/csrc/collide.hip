@@ -14,8 +14,8 @@
 // tile of THREADS x 8 tokens of one (b, h) row and walks the tables in LDS-sized
 // slices (two slices of 30 fp32 tables at L60 x R1024; one slice for fp16), and
 // serves several such tiles under each slice; a thread fetches the codes of its
-// eight consecutive tokens with one 16-byte load per table, six tables ahead of
-// their use, and gathers without branches.
+// eight consecutive tokens with one 16-byte load per table (wherever the row
+// starts), six tables ahead of their use, and gathers without branches.
 #include <atomic>
 
 #include "socket_common.h"
@@ -40,16 +40,27 @@ __device__ __forceinline__ float norm_at(const void* v, int dtype, int64_t i) {
   return dtype == SOCKET_F16 ? f16_bits_to_f32(u) : bf16_bits_to_f32(u);
 }
 
+// Vectors of a thread's eight tokens.  Rows of the reference's layout start wherever T puts them, odd rows of an odd T on an
+// odd pair of bytes; global loads take such addresses as they are, and a wave's 1024 contiguous bytes touch nine 128-byte
+// lines instead of eight.  (32 rows, L60 x R1024, us against a code at a time: fp32 tables at 2051 / 4135 / 9003 / 20881 / 32771
+// tokens 26 / 32 / 31 / 33 / 50 against 71 / 80 / 79 / 101 / 168, bf16 24 / 29 / 26 / 28 / 41 against 60 / 69 / 68 / 88 / 147;
+// rows on 16-byte boundaries are as fast as before.)
+typedef uint32_t codes8 __attribute__((ext_vector_type(4), aligned(2)));     // eight 16-bit codes or norms
+typedef uint32_t bytes8 __attribute__((ext_vector_type(2), aligned(1)));     // eight mask bytes
+typedef float floats4 __attribute__((ext_vector_type(4), aligned(4)));
+
 // ct: tables per LDS slice.  INLDS false: a single table exceeds LDS, gather from global memory.
-// VEC: rows are 16-byte aligned (T % 8 == 0 and aligned bases): 16-byte code loads.
 // A workgroup serves `chunks` consecutive tiles of THREADS x 8 tokens under every
 // slice it brings into LDS; with more than one slice the running sums of a tile
 // wait in `out` between slices (each thread re-reads what it wrote itself), which
 // costs 8 bytes per token and slice against the 2 L + 9 of the stream and keeps
 // the order of the fp32 adds.
+// The thread at a row's end whose eight tokens would run past it takes the row's last eight (its loads stay inside the row)
+// and leaves those that its neighbour owns alone: it neither stores their sums nor their scores.
+// WIDE false: rows of fewer than eight tokens, element by element.
 // STREAM: the codes are loaded with the streaming hint (a code array too large to
-// stay in the memory-side cache from one call to the next; VEC only).
-template <typename QT, int THREADS, bool VEC, bool INLDS, bool STREAM>
+// stay in the memory-side cache from one call to the next; WIDE only).
+template <typename QT, int THREADS, bool WIDE, bool INLDS, bool STREAM>
 __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
     const QT* __restrict__ q_probs, const int16_t* __restrict__ key_buckets,
     const uint8_t* __restrict__ allowed, const void* __restrict__ v_hist, int v_dtype, float* __restrict__ out,
@@ -61,72 +72,70 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
   const QT* qp = q_probs + (int64_t)bh * L * R;
   const int16_t* kb = key_buckets + (int64_t)bh * L * T;
 
-  // the eight codes of a thread's tokens for table l, as loaded (two per word; -1 where no token is)
-  auto codes_of = [&](int l, int t0) -> uint4 {
+  // the codes of tokens t0 .. t0 + 7 for table l, as loaded (two per word; WIDE: all eight exist; else -1 where no token is)
+  auto codes_of = [&](int l, int t0) -> codes8 {
     const int16_t* row = kb + (int64_t)l * T + t0;
-    if (VEC && !STREAM) return *reinterpret_cast<const uint4*>(row);
-    if (VEC) {
-      typedef uint32_t u32x4_stream __attribute__((ext_vector_type(4)));
-      const u32x4_stream v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_stream*>(row));
-      return make_uint4(v.x, v.y, v.z, v.w);
-    }
-    uint32_t u[4];
+    if (WIDE && !STREAM) return *reinterpret_cast<const codes8*>(row);
+    if (WIDE) return __builtin_nontemporal_load(reinterpret_cast<const codes8*>(row));
+    codes8 u;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint32_t lo = (t0 + 2 * i < T) ? (uint16_t)row[2 * i] : 0xffffu;
       const uint32_t hi = (t0 + 2 * i + 1 < T) ? (uint16_t)row[2 * i + 1] : 0xffffu;
       u[i] = lo | (hi << 16);
     }
-    return make_uint4(u[0], u[1], u[2], u[3]);
+    return u;
   };
-  auto load_partial = [&](int64_t o, int t0, float (&sum)[TPT]) {
-    if (VEC) {
-      const float4 a = *reinterpret_cast<const float4*>(out + o);
-      const float4 b = *reinterpret_cast<const float4*>(out + o + 4);
-      sum[0] = a.x, sum[1] = a.y, sum[2] = a.z, sum[3] = a.w;
-      sum[4] = b.x, sum[5] = b.y, sum[6] = b.z, sum[7] = b.w;
+  // `skip`: how many of the eight belong to the thread before (only ever above zero at a row's end)
+  auto load_partial = [&](int64_t o, int t0, int skip, float (&sum)[TPT]) {
+    if (WIDE && skip == 0) {
+      const floats4 a = *reinterpret_cast<const floats4*>(out + o);
+      const floats4 b = *reinterpret_cast<const floats4*>(out + o + 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[i] = a[i], sum[4 + i] = b[i];
     } else {
 #pragma unroll
-      for (int i = 0; i < TPT; ++i) sum[i] = (t0 + i < T) ? out[o + i] : 0.f;
+      for (int i = 0; i < TPT; ++i) sum[i] = (i >= skip && t0 + i < T) ? out[o + i] : 0.f;
     }
   };
-  auto store_partial = [&](int64_t o, int t0, const float (&sum)[TPT]) {
-    if (VEC) {
-      *reinterpret_cast<float4*>(out + o) = make_float4(sum[0], sum[1], sum[2], sum[3]);
-      *reinterpret_cast<float4*>(out + o + 4) = make_float4(sum[4], sum[5], sum[6], sum[7]);
+  auto store_row = [&](int64_t o, int t0, int skip, const float (&x)[TPT]) {
+    if (WIDE && skip == 0) {
+      floats4 a, b;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] = x[i], b[i] = x[4 + i];
+      *reinterpret_cast<floats4*>(out + o) = a;
+      *reinterpret_cast<floats4*>(out + o + 4) = b;
     } else {
 #pragma unroll
       for (int i = 0; i < TPT; ++i)
-        if (t0 + i < T) out[o + i] = sum[i];
+        if (i >= skip && t0 + i < T) out[o + i] = x[i];
     }
   };
-  auto finish = [&](int64_t o, int t0, const float (&sum)[TPT]) {
-    if (VEC) {   // all eight tokens exist and every operand row is 16-byte aligned at o
-      const uint2 aw = *reinterpret_cast<const uint2*>(allowed + o);
-      const uint32_t ab[2] = {aw.x, aw.y};
+  auto finish = [&](int64_t o, int t0, int skip, const float (&sum)[TPT]) {
+    float res[TPT];
+    if (WIDE) {
+      const bytes8 aw = *reinterpret_cast<const bytes8*>(allowed + o);
       float vh[TPT];
       if (v_dtype == SOCKET_F32) {      // (uniform)
-        const float4 v0 = *reinterpret_cast<const float4*>((const float*)v_hist + o);
-        const float4 v1 = *reinterpret_cast<const float4*>((const float*)v_hist + o + 4);
-        vh[0] = v0.x, vh[1] = v0.y, vh[2] = v0.z, vh[3] = v0.w;
-        vh[4] = v1.x, vh[5] = v1.y, vh[6] = v1.z, vh[7] = v1.w;
+        const floats4 v0 = *reinterpret_cast<const floats4*>((const float*)v_hist + o);
+        const floats4 v1 = *reinterpret_cast<const floats4*>((const float*)v_hist + o + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vh[i] = v0[i], vh[4 + i] = v1[i];
       } else {
-        const uint4 w = *reinterpret_cast<const uint4*>((const uint16_t*)v_hist + o);
+        const codes8 c = *reinterpret_cast<const codes8*>((const uint16_t*)v_hist + o);
+        const uint4 w = make_uint4(c.x, c.y, c.z, c.w);
         if (v_dtype == SOCKET_F16) unpack16<DType_f16>(w, vh);
         else unpack16<DType_bf16>(w, vh);
       }
-      float res[TPT];
 #pragma unroll
       for (int i = 0; i < TPT; ++i)
-        res[i] = ((ab[i >> 2] >> (8 * (i & 3))) & 0xffu) ? sum[i] * vh[i] : -INFINITY;
-      *reinterpret_cast<float4*>(out + o) = make_float4(res[0], res[1], res[2], res[3]);
-      *reinterpret_cast<float4*>(out + o + 4) = make_float4(res[4], res[5], res[6], res[7]);
+        res[i] = (((i < 4 ? aw.x : aw.y) >> (8 * (i & 3))) & 0xffu) ? sum[i] * vh[i] : -INFINITY;
     } else {
 #pragma unroll
-      for (int i = 0; i < TPT; ++i) {
-        if (t0 + i < T) out[o + i] = allowed[o + i] ? sum[i] * norm_at(v_hist, v_dtype, o + i) : -INFINITY;
-      }
+      for (int i = 0; i < TPT; ++i)
+        res[i] = t0 + i < T && allowed[o + i] ? sum[i] * norm_at(v_hist, v_dtype, o + i) : -INFINITY;
     }
+    store_row(o, t0, skip, res);
   };
 
   const int step = INLDS ? ct : L;   // (without LDS: one pass over all tables)
@@ -146,21 +155,22 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
       __syncthreads();
     }
     for (int c = 0; c < chunks; ++c) {
-      const int t0 = ((blockIdx.x * chunks + c) * THREADS + threadIdx.x) * TPT;
-      if (t0 >= T) continue;
+      const int own = ((blockIdx.x * chunks + c) * THREADS + threadIdx.x) * TPT;
+      if (own >= T) continue;
+      const int t0 = WIDE ? min(own, T - TPT) : own, skip = own - t0;
       const int64_t o = (int64_t)bh * T + t0;
       float sum[TPT];
       if (l0 == 0) {
 #pragma unroll
         for (int i = 0; i < TPT; ++i) sum[i] = 0.f;
       } else {
-        load_partial(o, t0, sum);
+        load_partial(o, t0, skip, sum);
       }
       // A ring of kAhead code words per lane stays in flight (one 16-byte load per lane
       // would leave the stream waiting on latency): slot a always holds table lb + a;
       // the loop is unrolled by the ring's depth, so a slot is a fixed set of registers
       // and the wait before its use counts exactly the loads behind it.
-      uint4 ring[kAhead];
+      codes8 ring[kAhead];
 #pragma unroll
       for (int a = 0; a < kAhead; ++a) ring[a] = codes_of(l0 + min(a, nt - 1), t0);
       for (int lb = 0; lb < nt; lb += kAhead) {
@@ -168,15 +178,14 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
         for (int a = 0; a < kAhead; ++a) {
           const int l = lb + a;
           if (l >= nt) break;
-          const uint4 cur = ring[a];
+          const codes8 cur = ring[a];
           ring[a] = codes_of(l0 + min(l + kAhead, nt - 1), t0);   // (past the slice: its last table again, unused)
-          const uint32_t u[4] = {cur.x, cur.y, cur.z, cur.w};
           // branch-free: a stray code reads entry 0 and adds +0.0 instead (x + 0.0 == x;
           // the sums start at +0.0, so no -0.0 can be lost), and the LDS variant has no
           // global load in here for the compiler to wait on with the ring in flight
 #pragma unroll
           for (int i = 0; i < TPT; ++i) {
-            const int r = (int)(int16_t)((i & 1) ? (u[i >> 1] >> 16) : (u[i >> 1] & 0xffffu));
+            const int r = (int)(int16_t)((i & 1) ? (cur[i >> 1] >> 16) : (cur[i >> 1] & 0xffffu));
             const bool hit = r >= 0 && r < R;
             const int rr = hit ? r : 0;
             const float e = entry_to_f32(INLDS ? table[l * R + rr] : qp[(int64_t)(l0 + l) * R + rr]);
@@ -184,8 +193,8 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
           }
         }
       }
-      if (l0 + nt >= L) finish(o, t0, sum);
-      else store_partial(o, t0, sum);
+      if (l0 + nt >= L) finish(o, t0, skip, sum);
+      else store_row(o, t0, skip, sum);
     }
   }
 }
@@ -204,31 +213,24 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
     ct = (L + slices - 1) / slices;
   }
   const size_t lds = (size_t)ct * per_table;
-  const bool vec = T % 8 == 0 && (((uintptr_t)key_buckets | (uintptr_t)allowed | (uintptr_t)v_hist | (uintptr_t)out) & 15) == 0;
+  const bool wide = T >= kTokensPerThread;
   // Lanes of a workgroup.  It pulls its row's whole table through LDS with them, which is quicker the more there are, and
   // the chip has at most CUs x (tables that fit a CU's LDS) workgroups at work.  While all workgroups are at work at
   // once narrower ones leave fewer CUs idle; past that each further round costs what the first did, and 1024 lanes need
-  // the fewest.  us at 256 / 512 / 1024 lanes, rows of 16-byte code loads (T % 8 == 0) | of 2-byte ones:
+  // the fewest.  us at 256 / 512 / 1024 lanes:
   //   32 rows, L60 x R1024 fp32    4088: 32 / 24 / 23     8192: 34 / 29 / 36     32768: 66 / 35 / 40    48000: 99 / 61 / 44
-  //                              | 2051: 73 / 57 / 56     9003: 81 / 99 / 145    24001: 159 / 101 / 145 32771: 228 / 193 / 146
   //   the same, bf16               4088: 23 / 22 / 22     5000: 25 / 25 / 27     32768: 51 / 28 / 36    65536: 93 / 58 / 50
-  //                              | 2051: 54 / 51 / 51     9003: 69 / 88 / 126    24001: 134 / 89 / 126  32771: 199 / 172 / 126
   //   32 rows, L32 x R256 fp32     4088: 11 / 12 / 12    12000: 13 / 13 / 18     24000: 16 / 15 / 19
-  //                              | 4093: 30 / 40 / 40    12003: 37 / 48 / 75     24001: 52 / 51 / 76
   // Just past 4096 tokens 512 lanes make a second, nearly empty workgroup of what 1024 hold in one.  A table in one
   // slice (bf16) and few workgroups: 28 rows, L48, 5000 tokens 18.6 / 20.3 us at 256 / 512 lanes; 8 rows, L60, 16384: 21 / 23.
-  // 2-byte loads bound a lane more than the table does, so that 256 lanes pay from 2800 tokens on; there a few 512-lane
-  // workgroups over the CUs (264) still take 128 us where 1024 lanes take 145.
   auto tiles_of = [&](int th) { return (T + th * kTokensPerThread - 1) / (th * kTokensPerThread); };
   auto fit = [&](int th, int workgroups) { return (int64_t)tiles_of(th) * B * H <= workgroups; };
   const bool shares = 2 * lds <= budget;      // a CU holds several workgroups' tables
   const int cus = lim.cu_count;
   int threads = 1024;
   if (T <= 256 * kTokensPerThread || (shares && fit(256, cus))) threads = 256;
-  else if (vec && ct >= L && T > 4096 && fit(256, cus * 3 / 8)) threads = 256;
-  else if (vec && T > 4608 && fit(512, cus)) threads = 512;
-  else if (!vec && T > 2816 && fit(256, cus)) threads = 256;
-  else if (!vec && T > 4096 && fit(512, cus + cus / 32)) threads = 512;
+  else if (ct >= L && T > 4096 && fit(256, cus * 3 / 8)) threads = 256;
+  else if (T > 4608 && fit(512, cus)) threads = 512;
   const int tiles = tiles_of(threads);
   // tiles per workgroup: as many as leave two workgroups per CU (they amortise the
   // slices a workgroup pulls through LDS), at most 8
@@ -252,22 +254,24 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
     }                                                                                                 \
     hipLaunchKernelGGL(kern, grid, dim3(TH), lds, stream, q_probs, key_buckets, allowed, v_hist, v_dtype, out, L, R, T, ct, chunks); \
   } while (0)
-#define SOCKET_COLLIDE_V(TH, LD)         \
-  do {                                   \
-    if (vec && stream_codes) SOCKET_COLLIDE(TH, true, LD, true); \
-    else if (vec) SOCKET_COLLIDE(TH, true, LD, false); \
-    else SOCKET_COLLIDE(TH, false, LD, false);  \
+#define SOCKET_COLLIDE_W(TH, LD)                                   \
+  do {                                                             \
+    if (stream_codes) SOCKET_COLLIDE(TH, true, LD, true);          \
+    else SOCKET_COLLIDE(TH, true, LD, false);                      \
   } while (0)
-  if (ct > 0) {
-    if (threads == 256) SOCKET_COLLIDE_V(256, true);
-    else if (threads == 512) SOCKET_COLLIDE_V(512, true);
-    else SOCKET_COLLIDE_V(1024, true);
+  if (!wide) {      // (fewer than eight tokens: one narrow workgroup a row)
+    if (ct > 0) SOCKET_COLLIDE(256, false, true, false);
+    else SOCKET_COLLIDE(256, false, false, false);
+  } else if (ct > 0) {
+    if (threads == 256) SOCKET_COLLIDE_W(256, true);
+    else if (threads == 512) SOCKET_COLLIDE_W(512, true);
+    else SOCKET_COLLIDE_W(1024, true);
   } else {
-    if (threads == 256) SOCKET_COLLIDE_V(256, false);
-    else if (threads == 512) SOCKET_COLLIDE_V(512, false);
-    else SOCKET_COLLIDE_V(1024, false);
+    if (threads == 256) SOCKET_COLLIDE_W(256, false);
+    else if (threads == 512) SOCKET_COLLIDE_W(512, false);
+    else SOCKET_COLLIDE_W(1024, false);
   }
-#undef SOCKET_COLLIDE_V
+#undef SOCKET_COLLIDE_W
 #undef SOCKET_COLLIDE
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;

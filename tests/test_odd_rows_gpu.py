@@ -1,0 +1,52 @@
+"""Rows that start on any element: the reference's operand layout at contexts that are a multiple of nothing."""
+import pytest
+import torch
+
+from socket_amd._lib import check, dtype_enum, lib, ptr, stream_ptr
+
+pytestmark = pytest.mark.gpu
+
+
+def _collide(q, codes, allowed, v, out):
+    B, H, L, R = q.shape
+    check("socket_soft_hash_collision", lib().socket_soft_hash_collision_typed(
+        ptr(q), dtype_enum(q.dtype), ptr(codes), ptr(allowed), ptr(v), dtype_enum(v.dtype), ptr(out), B, H, L, R, codes.shape[3],
+        stream_ptr(q.device)))
+
+
+@pytest.mark.parametrize("B,H,L,R,T,qt,vt,shift", [
+    (1, 2, 5, 64, 1, torch.float32, torch.float16, 0),           # fewer tokens than a thread's eight
+    (1, 3, 5, 64, 7, torch.bfloat16, torch.float32, 0),
+    (2, 3, 7, 256, 8, torch.float16, torch.float16, 0),          # exactly eight, odd bases
+    (1, 3, 7, 256, 9, torch.float32, torch.bfloat16, 1),         # the second thread owns one
+    (2, 5, 60, 1024, 2051, torch.float32, torch.float16, 3),     # two table slices: sums wait in the output between them
+    (1, 32, 60, 1024, 8195, torch.float32, torch.float32, 0),    # several tiles to a workgroup
+    (2, 28, 48, 1024, 20881, torch.bfloat16, torch.float16, 5),  # codes loaded past the caches
+    (1, 2, 3, 65536, 4101, torch.float32, torch.float16, 0),     # a table that exceeds LDS
+])
+def test_collision_scores_of_odd_rows(B, H, L, R, T, qt, vt, shift):
+    """Bit for bit the sequential fp32 sum, masked, for rows and bases on no boundary; codes outside [0, R) add nothing;
+    nothing is written outside the scores."""
+    dev = "cuda"
+    g = torch.Generator(device=dev).manual_seed(T)
+    q = torch.rand(B, H, L, R, generator=g, device=dev).to(qt)
+    n = B * H * T
+
+    def at(flat, shape):      # (the values `shift` elements into an allocation)
+        whole = torch.empty(flat.numel() + shift, dtype=flat.dtype, device=dev)
+        whole[shift:] = flat
+        return whole[shift:].view(shape)
+
+    codes = at(torch.randint(-2, min(R + 2, 32767), (n * L,), generator=g, device=dev).to(torch.int16), (B, H, L, T))
+    allowed = at(torch.rand(n, generator=g, device=dev) < 0.8, (B, H, T))
+    v = at((torch.rand(n, generator=g, device=dev) * 4).to(vt), (B, H, T))
+    buf = torch.full((n + shift + 16,), 7.0, device=dev)
+    out = buf[shift:shift + n].view(B, H, T)
+    _collide(q, codes, allowed, v, out)
+    want = torch.zeros(B, H, T, device=dev)
+    for l in range(L):
+        c = codes[:, :, l].long()
+        want += torch.gather(q[:, :, l].float(), 2, c.clamp(0, R - 1)).masked_fill((c < 0) | (c >= R), 0.0)
+    want = (want * v.float()).masked_fill(~allowed, float("-inf"))
+    assert torch.equal(out, want)
+    assert (buf[:shift] == 7.0).all() and (buf[shift + n:] == 7.0).all()
