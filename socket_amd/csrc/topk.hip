@@ -56,6 +56,12 @@ constexpr int kMaxParts = 16;          // workgroups that share one row at most
 
 typedef unsigned long long u64;
 
+// Four consecutive scores.  Rows start on any multiple of four bytes (a row pitch of odd length is what a caller's
+// [B,Hq,T] tensor has); the hardware takes 16-byte loads at such addresses, and a wave's 1024 bytes then touch nine
+// 128-byte lines instead of eight (32 rows of 20881 / 32771 scores, us against a score at a time: 13.5 / 13.6 against
+// 15.9 / 17.9).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 template <bool B>
 struct BoolTag {
   static constexpr bool value = B;
@@ -160,44 +166,32 @@ __device__ __forceinline__ void find_bin(uint32_t* hist, int need, int descendin
 
 // Visit row[begin:n) once, 16 bytes per lane per load and eight loads in flight
 // per lane (a lone workgroup per row has to cover the memory latency itself).
-template <bool VEC, int THREADS, class F>
+template <int THREADS, class F>
 __device__ __forceinline__ void for_each_in(const float* row, int begin, int n, int tid, F&& f) {
   constexpr int U = 8;
-  if (VEC) {  // begin is a multiple of 4
-    const int n4 = n & ~3;
-    constexpr int kStride = THREADS * 4;
-    int i = begin + tid * 4;
-    for (; i + (U - 1) * kStride < n4; i += U * kStride) {
-      float4 x[U];
+  const int n4 = n & ~3;   // begin is a multiple of 4
+  constexpr int kStride = THREADS * 4;
+  int i = begin + tid * 4;
+  for (; i + (U - 1) * kStride < n4; i += U * kStride) {
+    f32x4_any x[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) x[u] = *reinterpret_cast<const float4*>(row + i + u * kStride);
+    for (int u = 0; u < U; ++u) x[u] = *reinterpret_cast<const f32x4_any*>(row + i + u * kStride);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        f(i + u * kStride, x[u].x);
-        f(i + u * kStride + 1, x[u].y);
-        f(i + u * kStride + 2, x[u].z);
-        f(i + u * kStride + 3, x[u].w);
-      }
+    for (int u = 0; u < U; ++u) {
+      f(i + u * kStride, x[u].x);
+      f(i + u * kStride + 1, x[u].y);
+      f(i + u * kStride + 2, x[u].z);
+      f(i + u * kStride + 3, x[u].w);
     }
-    for (; i < n4; i += kStride) {
-      const float4 x = *reinterpret_cast<const float4*>(row + i);
-      f(i, x.x);
-      f(i + 1, x.y);
-      f(i + 2, x.z);
-      f(i + 3, x.w);
-    }
-    for (int t = max(n4, begin) + tid; t < n; t += THREADS) f(t, row[t]);
-  } else {
-    int i = begin + tid;
-    for (; i + (U - 1) * THREADS < n; i += U * THREADS) {
-      float x[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) x[u] = row[i + u * THREADS];
-#pragma unroll
-      for (int u = 0; u < U; ++u) f(i + u * THREADS, x[u]);
-    }
-    for (; i < n; i += THREADS) f(i, row[i]);
   }
+  for (; i < n4; i += kStride) {
+    const f32x4_any x = *reinterpret_cast<const f32x4_any*>(row + i);
+    f(i, x.x);
+    f(i + 1, x.y);
+    f(i + 2, x.z);
+    f(i + 3, x.w);
+  }
+  for (int t = max(n4, begin) + tid; t < n; t += THREADS) f(t, row[t]);
 }
 
 // Append `value` to a list if `take`: one LDS atomic per wave, positions handed
@@ -464,7 +458,7 @@ __host__ __device__ __forceinline__ bool sampling_ok(int m) {
 // the lower edge of its bin.  Every workgroup that calls this for a row gets the
 // same tau.  Needs n > kPoolCap; clears hist itself (nobody may be using it).  When
 // it returns every lane has passed the barrier that follows the last read of hist.
-template <int THREADS, bool VEC>
+template <int THREADS>
 __device__ __forceinline__ uint32_t sample_threshold(const float* row, int n, int m, uint32_t* hist,
                                                      SelectShared& sh, int tid) {
   constexpr int kMaxQ = 16384 / 4 / THREADS;  // float4 groups per lane at most
@@ -480,17 +474,7 @@ __device__ __forceinline__ uint32_t sample_threshold(const float* row, int n, in
       const int q = j * THREADS + tid;
       const int chunk = q >> 4;
       const int at = (int)(((int64_t)chunk * n / nchunk) & ~3ll) + (q & 15) * 4;
-      float x[4];
-      if (VEC) {
-        const float4 v = *reinterpret_cast<const float4*>(row + at);
-        x[0] = v.x;
-        x[1] = v.y;
-        x[2] = v.z;
-        x[3] = v.w;
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) x[c] = row[at + c];
-      }
+      const f32x4_any x = *reinterpret_cast<const f32x4_any*>(row + at);
 #pragma unroll
       for (int c = 0; c < 4; ++c) key[j * 4 + c] = score_to_key(x[c]);
     }
@@ -575,7 +559,6 @@ __device__ __forceinline__ u64 load_coherent(const u64* p) {
 // row_count and row_done are zero on entry and zero again on exit.
 // The pooled composites are held in registers, eight per lane, from the moment
 // the pool is complete; LDS holds them only while they are being compacted.
-template <bool VEC>
 __global__ __launch_bounds__(kThreads) void select_list_kernel(
     const float* __restrict__ scores, int64_t score_stride, const int32_t* __restrict__ lens,
     const int32_t* __restrict__ budgets, const uint32_t* __restrict__ row_range, int range_parts,
@@ -642,109 +625,100 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
       const int chunk = (((n + parts - 1) / parts) + 3) & ~3;
       const int begin = min(part * chunk, n4), e4 = min(begin + chunk, n4);
       const int tail_end = (part == parts - 1) ? n : e4;
-      if (VEC) {
-        // In batches of 16 scores per lane (four 16-byte loads, all in flight
-        // together); the first two batches are requested before the threshold is
-        // worked out, each further one two batches ahead of the one being filtered.  A
-        // wave counts what passes in its batch, reserves a stretch of the pool with
-        // one LDS atomic and writes its entries there: no barrier in the loop.
-        constexpr int kLoads = 4, kStep = kThreads * 4 * kLoads;
-        static_assert(kStep == kBatch, "batch size");
-        auto fetch = [&](int base, float4 (&x)[kLoads]) {
+      // In batches of 16 scores per lane (four 16-byte loads, all in flight
+      // together); the first two batches are requested before the threshold is
+      // worked out, each further one two batches ahead of the one being filtered.  A
+      // wave counts what passes in its batch, reserves a stretch of the pool with
+      // one LDS atomic and writes its entries there: no barrier in the loop.
+      constexpr int kLoads = 4, kStep = kThreads * 4 * kLoads;
+      static_assert(kStep == kBatch, "batch size");
+      auto fetch = [&](int base, float4 (&x)[kLoads]) {
 #pragma unroll
-          for (int u = 0; u < kLoads; ++u) {
-            // (past the end: the share's last four, fetched and ignored -- a load under
-            // a condition would make every wait in the loop a wait for all loads)
-            const int i0 = max(min(base + (u * kThreads + tid) * 4, e4 - 4), 0);
-            typedef float f32x4 __attribute__((ext_vector_type(4)));
-            const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(row + i0));
-            x[u] = make_float4(v.x, v.y, v.z, v.w);
-          }
-        };
-        // One batch of one wave.  Each of a lane's 16 scores is tested on the float (one
-        // compare per score; keys only for the pool): x passes when it is not below the
-        // float whose key is tau.  A tau above +inf's key or below -inf's is no float's
-        // key and is widened to that infinity (the pool only has to hold everything at
-        // or above tau; more is allowed).  A compare leaves a wave-wide mask in scalar
-        // registers; the 16 masks' population is the stretch of the pool that one LDS
-        // atomic reserves for the wave, and an entry's place in it is the count of its
-        // mask's bits below its lane, on top of a scalar running base -- no per-lane
-        // bookkeeping, no cross-lane traffic.  A batch that would run past the pool is
-        // counted but not written (the row is then redone from scratch anyway).
-        auto filter_batch = [&](auto full, int base, const float4 (&x)[kLoads], float tau_f) {
-          constexpr bool FULL = decltype(full)::value;   // every lane's 16 scores are inside the share
-          int total = 0;
-          u64 mask[kLoads * 4];   // (scalar registers)
-#pragma unroll
-          for (int u = 0; u < kLoads; ++u) {
-            const float xs[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
-            const bool in = FULL || base + (u * kThreads + tid) * 4 < e4;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              mask[u * 4 + c] = __builtin_amdgcn_ballot_w64(in && !(xs[c] < tau_f));
-              total += __popcll(mask[u * 4 + c]);
-            }
-          }
-          if (total == 0) return;  // uniform
-          int at = 0;
-          if (lane == 0) at = atomicAdd(&sh.fill_pool, total);
-          at = __builtin_amdgcn_readfirstlane(at);
-          if (at + total > kPoolCap) return;  // uniform
-          const uint32_t cidx = 0xffffffffu - (uint32_t)(base + tid * 4);
-#pragma unroll
-          for (int u = 0; u < kLoads; ++u) {
-            const float xs[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
-            const bool in = FULL || base + (u * kThreads + tid) * 4 < e4;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const bool pass = in && !(xs[c] < tau_f);
-              const u64 mk = mask[u * 4 + c];
-              const int slot = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32),
-                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)mk, (uint32_t)at));
-              if (pass) {
-                // the two halves of the entry from wherever they are, in one write
-                // (a 64-bit store would first copy them into a register pair)
-                const uint32_t addr = (uint32_t)(uintptr_t)(pool + slot);
-                asm volatile("ds_write2_b32 %0, %1, %2 offset1:1"
-                             :: "v"(addr), "v"(cidx - (uint32_t)(u * kThreads * 4 + c)), "v"(__float_as_uint(xs[c]))
-                             : "memory");
-              }
-              at += __popcll(mk);
-            }
-          }
-        };
-        auto filter = [&](int base, const float4 (&x)[kLoads], float tau_f) {
-          if (base >= e4) return;  // uniform
-          if (base + kStep <= e4) filter_batch(BoolTag<true>{}, base, x, tau_f);
-          else filter_batch(BoolTag<false>{}, base, x, tau_f);
-        };
-        float4 b0[kLoads], b1[kLoads], b2[kLoads];
-        fetch(begin, b0);
-        fetch(begin + kStep, b1);
-        const uint32_t tau = sample_threshold<kThreads, VEC>(row, n, m, hist, sh, tid);
-        for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;   // for the first refinement pass
-        const float tau_f = tau >= 0xff800000u ? INFINITY : tau <= 0x007fffffu ? -INFINITY
-                            : __uint_as_float((tau & 0x80000000u) ? (tau & 0x7fffffffu) : ~tau);
-        for (int base = begin; base < e4; base += 3 * kStep) {
-          fetch(base + 2 * kStep, b2);
-          filter(base, b0, tau_f);
-          fetch(base + 3 * kStep, b0);
-          filter(base + kStep, b1, tau_f);
-          fetch(base + 4 * kStep, b1);
-          filter(base + 2 * kStep, b2, tau_f);
+        for (int u = 0; u < kLoads; ++u) {
+          // (past the end: the share's last four, fetched and ignored -- a load under
+          // a condition would make every wait in the loop a wait for all loads)
+          const int i0 = max(min(base + (u * kThreads + tid) * 4, e4 - 4), 0);
+          const f32x4_any v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(row + i0));
+          x[u] = make_float4(v.x, v.y, v.z, v.w);
         }
-        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the pool writes above are not the compiler's to wait for
-        if (wave == 0) {
-          const int i = e4 + lane;
-          const float x = i < tail_end ? row[i] : 0.f;
-          wave_append(i < tail_end && !(x < tau_f), composite(__float_as_uint(x), i), &sh.fill_pool, pool, kPoolCap);
+      };
+      // One batch of one wave.  Each of a lane's 16 scores is tested on the float (one
+      // compare per score; keys only for the pool): x passes when it is not below the
+      // float whose key is tau.  A tau above +inf's key or below -inf's is no float's
+      // key and is widened to that infinity (the pool only has to hold everything at
+      // or above tau; more is allowed).  A compare leaves a wave-wide mask in scalar
+      // registers; the 16 masks' population is the stretch of the pool that one LDS
+      // atomic reserves for the wave, and an entry's place in it is the count of its
+      // mask's bits below its lane, on top of a scalar running base -- no per-lane
+      // bookkeeping, no cross-lane traffic.  A batch that would run past the pool is
+      // counted but not written (the row is then redone from scratch anyway).
+      auto filter_batch = [&](auto full, int base, const float4 (&x)[kLoads], float tau_f) {
+        constexpr bool FULL = decltype(full)::value;   // every lane's 16 scores are inside the share
+        int total = 0;
+        u64 mask[kLoads * 4];   // (scalar registers)
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+          const float xs[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
+          const bool in = FULL || base + (u * kThreads + tid) * 4 < e4;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            mask[u * 4 + c] = __builtin_amdgcn_ballot_w64(in && !(xs[c] < tau_f));
+            total += __popcll(mask[u * 4 + c]);
+          }
         }
-      } else {
-        const uint32_t tau = sample_threshold<kThreads, VEC>(row, n, m, hist, sh, tid);
-        for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;   // for the first refinement pass
-        for_each_in<VEC, kThreads>(row, begin, tail_end, tid, [&](int i, float x) {
-          wave_append(score_to_key(x) >= tau, composite(__float_as_uint(x), i), &sh.fill_pool, pool, kPoolCap);
-        });
+        if (total == 0) return;  // uniform
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&sh.fill_pool, total);
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (at + total > kPoolCap) return;  // uniform
+        const uint32_t cidx = 0xffffffffu - (uint32_t)(base + tid * 4);
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+          const float xs[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
+          const bool in = FULL || base + (u * kThreads + tid) * 4 < e4;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const bool pass = in && !(xs[c] < tau_f);
+            const u64 mk = mask[u * 4 + c];
+            const int slot = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)mk, (uint32_t)at));
+            if (pass) {
+              // the two halves of the entry from wherever they are, in one write
+              // (a 64-bit store would first copy them into a register pair)
+              const uint32_t addr = (uint32_t)(uintptr_t)(pool + slot);
+              asm volatile("ds_write2_b32 %0, %1, %2 offset1:1"
+                           :: "v"(addr), "v"(cidx - (uint32_t)(u * kThreads * 4 + c)), "v"(__float_as_uint(xs[c]))
+                           : "memory");
+            }
+            at += __popcll(mk);
+          }
+        }
+      };
+      auto filter = [&](int base, const float4 (&x)[kLoads], float tau_f) {
+        if (base >= e4) return;  // uniform
+        if (base + kStep <= e4) filter_batch(BoolTag<true>{}, base, x, tau_f);
+        else filter_batch(BoolTag<false>{}, base, x, tau_f);
+      };
+      float4 b0[kLoads], b1[kLoads], b2[kLoads];
+      fetch(begin, b0);
+      fetch(begin + kStep, b1);
+      const uint32_t tau = sample_threshold<kThreads>(row, n, m, hist, sh, tid);
+      for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;   // for the first refinement pass
+      const float tau_f = tau >= 0xff800000u ? INFINITY : tau <= 0x007fffffu ? -INFINITY
+                          : __uint_as_float((tau & 0x80000000u) ? (tau & 0x7fffffffu) : ~tau);
+      for (int base = begin; base < e4; base += 3 * kStep) {
+        fetch(base + 2 * kStep, b2);
+        filter(base, b0, tau_f);
+        fetch(base + 3 * kStep, b0);
+        filter(base + kStep, b1, tau_f);
+        fetch(base + 4 * kStep, b1);
+        filter(base + 2 * kStep, b2, tau_f);
+      }
+      __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the pool writes above are not the compiler's to wait for
+      if (wave == 0) {
+        const int i = e4 + lane;
+        const float x = i < tail_end ? row[i] : 0.f;
+        wave_append(i < tail_end && !(x < tau_f), composite(__float_as_uint(x), i), &sh.fill_pool, pool, kPoolCap);
       }
       __syncthreads();
       // (an entry of the pool: the score's bits over the complemented index)
@@ -906,7 +880,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         kmax = max(kmax, rr[2 * i + 1]);
       }
     } else {
-      for_each_in<VEC, kThreads>(row, 0, n, tid, [&](int, float x) {
+      for_each_in<kThreads>(row, 0, n, tid, [&](int, float x) {
         const uint32_t k = score_to_key(x);
         kmin = min(kmin, k);
         kmax = max(kmax, k);
@@ -945,7 +919,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
     const int shift = range_shift(lo, hi);
     for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;
     __syncthreads();
-    for_each_in<VEC, kThreads>(row, 0, n, tid, [&](int, float x) {
+    for_each_in<kThreads>(row, 0, n, tid, [&](int, float x) {
       const uint32_t k = score_to_key(x);
       if (k >= lo && k <= hi) atomicAdd(&hist[(k - lo) >> shift], 1u);
     });
@@ -975,7 +949,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
     const int binw = (n + kBins - 1) / kBins;
     for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;
     __syncthreads();
-    for_each_in<VEC, kThreads>(row, 0, n, tid, [&](int i, float x) {
+    for_each_in<kThreads>(row, 0, n, tid, [&](int i, float x) {
       if (score_to_key(x) == blo) atomicAdd(&hist[i / binw], 1u);
     });
     __syncthreads();
@@ -1005,7 +979,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
 
   // ---- collect ------------------------------------------------------------------
   const int idx_star = sh.idx_star;
-  for_each_in<VEC, kThreads>(row, 0, n, tid, [&](int i, float x) {
+  for_each_in<kThreads>(row, 0, n, tid, [&](int i, float x) {
     const uint32_t k = score_to_key(x);
     const u64 v = composite(k, i);
     const bool in_bin = k >= blo && k <= bhi;
@@ -1099,7 +1073,6 @@ extern "C" int socket_select_list(const float* scores, int64_t score_stride, con
   const size_t lds_static = kBins * 4 + sizeof(SelectShared) + 256;
   size_t lds = (size_t)(cap_above + kCandCap) * sizeof(u64);
   SOCKET_REQUIRE(lds + lds_static <= lds_max, SOCKET_ERR_UNSUPPORTED);
-  const bool vec = socket_aligned16(scores) && (score_stride % 4 == 0);
   hipStream_t s = (hipStream_t)stream;
 
   // extras as LDS allows: the pool (where a pooled select can apply at all), then
@@ -1134,12 +1107,11 @@ extern "C" int socket_select_list(const float* scores, int64_t score_stride, con
   }
   SOCKET_REQUIRE((int64_t)rows * parts <= 0x7fffffff, SOCKET_ERR_SHAPE);
 
-  auto kern = vec ? select_list_kernel<true> : select_list_kernel<false>;
   if (lds > 32 * 1024 &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(select_list_kernel),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return SOCKET_ERR_LAUNCH;
-  hipLaunchKernelGGL(kern, dim3(rows * parts), dim3(kThreads), lds, s, scores, score_stride, lens, budgets,
+  hipLaunchKernelGGL(select_list_kernel, dim3(rows * parts), dim3(kThreads), lds, s, scores, score_stride, lens, budgets,
                      row_range, range_parts, Hq, T, M, sink, window, write_base, sparse_list,
                      list_stride, list_width, sparse_len, cap_above, counting_ok, use_pool, pool_slots, parts,
                      loc, row_count, row_done);

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from socket_amd import sparse
 from socket_amd._lib import check, dtype_enum, lib, ptr, stream_ptr
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +51,17 @@ def test_collision_scores_of_odd_rows(B, H, L, R, T, qt, vt, shift):
     want = (want * v.float()).masked_fill(~allowed, float("-inf"))
     assert torch.equal(out, want)
     assert (buf[:shift] == 7.0).all() and (buf[shift + n:] == 7.0).all()
+
+
+@pytest.mark.parametrize("T,M,shift", [(5, 3, 1), (4135, 129, 0), (8193, 300, 3), (20881, 652, 0), (49157, 1024, 2), (131075, 2048, 1)])
+def test_selection_from_odd_rows(T, M, shift):
+    """The list of a stable descending sort, from rows of odd pitch that start on any float, some scores minus infinity."""
+    dev, H = "cuda", 5
+    g = torch.Generator(device=dev).manual_seed(T)
+    whole = torch.randn(H * T + shift, generator=g, device=dev).exp_()
+    scores = whole[shift:].view(1, H, T)
+    scores[:, 1:3].masked_fill_(torch.rand(1, 2, T, generator=g, device=dev) < 0.5, float("-inf"))
+    scores[:, 3, :] = scores[:, 3, :].round()      # (many equal ones)
+    lists, lens = sparse.select_list(scores, 0, 0, M, write_base=False)
+    assert (lens == M).all()
+    assert torch.equal(lists.long(), torch.sort(scores, dim=-1, descending=True, stable=True).indices[..., :M])
