@@ -202,6 +202,12 @@ int socket_score_range_parts_grouped(int B, int Hq, int Hkv, int T, int q_dtype,
  * converting it with socket_group_q_probs first pays (socket_score_packed itself
  * never takes the persistent launch: its table slices need an interleaving pass). */
 int socket_score_persistent_serves(int B, int Hq, int Hkv, int T, int q_dtype, int L, int P, int R);
+/* socket_score_lanes_serve: 1 if socket_score_packed_grouped would serve a call of this
+ * shape (without row_range) with its launch for few tokens per CU, one or two tokens to a
+ * lane, 0 if not, -1 for an invalid shape.  Where it is 1 a producer does best to write the
+ * grouped table, whatever socket_score_prefers_grouped, which compares the other launches,
+ * says. */
+int socket_score_lanes_serve(int B, int Hq, int Hkv, int T, int q_dtype, int L, int P, int R);
 int socket_group_q_probs(const void* q_probs, int q_dtype, void* q_table, int B, int Hq, int Hkv,
                          int L, int R, void* stream);
 int socket_score_packed_grouped(const void* q_table, int q_dtype, const uint32_t* codes,

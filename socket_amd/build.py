@@ -22,7 +22,7 @@ LIB_PATH = os.path.join(HERE, "libsocket_hip.so")
 CORE_PATH = os.path.join(HERE, "libsocket_core.so")
 CORE_SOURCES = ["common.hip", "attend.hip", "decode_ops.hip", "rows.hip", "chunk_attend.hip", "prompt_attend.hip", "latent.hip",
                 "recurrence.hip"]
-SOURCES = ["score.hip", "collide.hip", "topk.hip", "hash.hip", "softhash.hip", "block_sparse.hip"]
+SOURCES = ["score.hip", "score_short.hip", "collide.hip", "topk.hip", "hash.hip", "softhash.hip", "block_sparse.hip"]
 ARCH = "gfx950"
 # Packed-FP32 VALU ops are switched off for every device translation unit.
 FLAGS = [

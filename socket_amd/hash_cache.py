@@ -150,7 +150,8 @@ def _prefers_grouped(B: int, Hq: int, Hkv: int, T: int, dtype_code: int, L: int,
     r = lib().socket_score_prefers_grouped(B, Hq, Hkv, T, dtype_code, L, P, R)
     if r < 0:
         raise ValueError(f"socket_score_prefers_grouped: invalid shape B={B} Hq={Hq} Hkv={Hkv} T={T} L={L} P={P} R={R}")
-    return bool(r)
+    # (calls with few tokens per CU have a launch of their own, which wants the grouped table)
+    return bool(r) or lib().socket_score_lanes_serve(B, Hq, Hkv, T, dtype_code, L, P, R) == 1
 
 
 @functools.lru_cache(maxsize=4096)
@@ -161,8 +162,8 @@ def _persistent_serves(B: int, Hq: int, Hkv: int, T: int, dtype_code: int, L: in
 def prefers_grouped(q_bhd: torch.Tensor, planes: torch.Tensor, protos_T: torch.Tensor, n_kv_heads: int,
                     context_len: int, out_dtype: Optional[torch.dtype] = None) -> bool:
     """Which table layout `soft_hash` should write for a scorer call over
-    `context_len` cached tokens: True = grouped, False = [B,Hq,L,R] (short
-    contexts with few kv heads, which the scorer serves one head per workgroup)."""
+    `context_len` cached tokens: True = grouped, False = [B,Hq,L,R] (shapes that the
+    scorer serves best with one head per workgroup)."""
     B, Hq = int(q_bhd.shape[0]), int(q_bhd.shape[1])
     L, P = int(planes.shape[0]), int(planes.shape[1])
     if out_dtype is None:
