@@ -466,6 +466,17 @@ int socket_decode_prologue(const void* qkv, int dtype, int64_t qkv_stride_b, con
                            void* v_norm, const void* planes, const void* protos_T, void* q_table, int out_dtype,
                            int grouped, int B, int Hq, int Hkv, int D, int L, int K, int R, int64_t Tcap,
                            float tanh_scale, float inv_temperature, void* stream);
+/* The same for more operands: dtype = SOCKET_BF16 or SOCKET_F32 (of the projection, the
+ * caches, planes, prototypes; the new key is hashed in bf16 as socket_hash_keys does it),
+ * D = 128, and K = 10 as above (fp32: R = 1024 and out_dtype SOCKET_F32) or any other
+ * K <= 16 with R <= 256. */
+int socket_decode_prologue_typed(const void* qkv, int dtype, int64_t qkv_stride_b, const void* freqs_cis,
+                                 int freqs_dtype, int64_t n_pos, const int64_t* pos, int pos_stride, void* q_out,
+                                 void* k_cache, void* v_cache, int64_t cache_stride_b, int64_t cache_stride_h,
+                                 int64_t cache_stride_s, int32_t* lens, const void* planes_words, void* codes,
+                                 void* v_norm, const void* planes, const void* protos_T, void* q_table, int out_dtype,
+                                 int grouped, int B, int Hq, int Hkv, int D, int L, int K, int R, int64_t Tcap,
+                                 float tanh_scale, float inv_temperature, void* stream);
 
 /* h = x + residual (residual may be NULL: h = x), rounded to `dtype`;
  * y = round(h * rsqrt(mean(h^2) + eps)) * weight.  x, residual, h_out (may be

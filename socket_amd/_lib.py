@@ -200,6 +200,8 @@ SIGNATURES = {
     "socket_select_list": (_I, [_P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _L, _I, _P, _P, _Z, _P]),
     "socket_decode_prologue": (_I, [_P, _I, _L, _P, _I, _L, _P, _I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _P, _P, _P, _P,
                                     _I, _I, _I, _I, _I, _I, _I, _I, _I, _L, c_float, c_float, _P]),
+    "socket_decode_prologue_typed": (_I, [_P, _I, _L, _P, _I, _L, _P, _I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _P, _P, _P, _P,
+                                    _I, _I, _I, _I, _I, _I, _I, _I, _I, _L, c_float, c_float, _P]),
     "socket_block_sparse_attention": (_I, [_P, _P, _P, _I] + [_L] * 9 + [_P, _P, _P] + [_L] * 3 + [_I] * 8 + [_P]),
     "socket_block_sparse_attention_cleared": (_I, [_P, _P, _P, _I] + [_L] * 9 + [_P, _P, _P] + [_L] * 3 + [_I] * 8 + [_P]),
     "socket_block_lists": (_I, [_P, _L, _L, _P] + [_I] * 11 + [_P]),

@@ -348,6 +348,180 @@ __host__ __device__ __forceinline__ float mx_scale(float tanh_scale, float inv_t
   return tanh_scale * inv_temperature * 1.4426950408889634f;
 }
 
+// The same for fp32 queries, planes and prototypes: v_mfma_f32_16x16x4_f32, which multiplies and adds in fp32 throughout, so
+// nothing is split.  Lane x holds column (or row) x % 16 and one k of four; which k that is is free as long as both operands
+// agree: for the projections quarter q takes dims 32 q .. + 31, a run, and for the logits step r takes plane 4 q + r,
+// which is what the lane's own projections are.
+// One sequence of 16 heads, 60 tables: 8.9 us as a launch of the scalar form below, 11.1 us with the rest of the prologue,
+// which took 9.3 us more, in one launch: a chain of trips to memory and of matrix products, on 80 workgroups.
+// Against float64 (2-norm, queries and planes N(0, 1)): 2.1e-7, the scalar form 2.5e-7.
+// OutDT: the table's type (bf16: the fp32 value rounded once).
+template <class FT, int W, class OutDT>
+__device__ __forceinline__ void soft_hash_mx32_block(const int l, const int group, const MxUnits& units, const float* __restrict__ q,
+                                                     int64_t q_sb, int64_t q_sh, const float* __restrict__ planes,
+                                                     const float* __restrict__ protos_T, void* __restrict__ out, int L, float scale,
+                                                     const void* __restrict__ freqs, const int64_t* __restrict__ pos, int pos_stride,
+                                                     int64_t n_pos, float* __restrict__ q_out) {
+  constexpr bool kRope = !std::is_void<FT>::value;
+  __shared__ float red[2][kSHWaves][kMxHeads];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 15, quarter = lane >> 4;
+  const int unit = group * (kMxHeads / W) + n / W;
+  const bool in_units = unit < units.count;
+  const int u = in_units ? unit : 0;
+  const int per_seq = units.parts > 0 ? units.Hkv * units.parts : units.Hq;
+  const int b = u / per_seq, at = u % per_seq;
+  const int member = units.parts > 0 ? at % units.parts * W + n % W : 0;       // of the kv head's group
+  const bool live = in_units && (units.parts == 0 || member < units.G);
+  const int head = units.parts > 0 ? at / units.parts * units.G + (live ? member : 0) : at;
+
+  const float* qrow = q + b * q_sb + head * q_sh + 32 * quarter;
+  const float* prow = planes + ((int64_t)l * kMxK + min(n, kMxK - 1)) * kMxD + 32 * quarter;
+  int64_t p = 0;
+  bool turn = false;
+  if constexpr (kRope) {
+    p = pos[(int64_t)b * pos_stride];
+    turn = p >= 0 && p < n_pos;
+  }
+  float x[32], pl[32], pr[4][4][4];
+#pragma unroll
+  for (int i = 0; i < 32; i += 4) {
+    float t[4];
+    sh_load4<DType_f32>(qrow, i, t);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[i + e] = t[e];
+    sh_load4<DType_f32>(prow, i, t);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) pl[i + e] = t[e];
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      sh_load4<DType_f32>(protos_T, min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c + 4 * n, pr[c][r]);
+  if constexpr (kRope) {
+    // (angles of row 0 for a position outside the table: a load under a condition is waited for at once)
+    float f[4][8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sh_load8<FT>(freqs, (turn ? p : 0) * kMxD + 32 * quarter + 8 * i, f[i]);
+    if (turn) {
+#pragma unroll
+      for (int i = 0; i < 32; i += 2) {
+        float re, im;
+        rotate_pair(x[i], x[i + 1], f[i / 8][i % 8], f[i / 8][i % 8 + 1], re, im);
+        x[i] = re, x[i + 1] = im;
+      }
+    }
+    if (l == 0 && wave == 0 && live) {
+#pragma unroll
+      for (int i = 0; i < 32; i += 4) {
+        const float t[4] = {x[i], x[i + 1], x[i + 2], x[i + 3]};
+        sh_store4<DType_f32>(q_out, ((int64_t)b * units.Hq + head) * kMxD + 32 * quarter + i, t);
+      }
+    }
+  }
+
+  // register r: plane 4 quarter + r of head n (planes past the tenth repeat it and are dropped).  Eight sums of sixteen
+  // products, added in pairs: one of 128 loses more than the scalar form's.
+  constexpr int kChains = 8;
+  sh_f32x4 proj[kChains];
+#pragma unroll
+  for (int j = 0; j < kChains; ++j) proj[j] = sh_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 32; ++i) proj[i % kChains] = __builtin_amdgcn_mfma_f32_16x16x4f32(pl[i], x[i], proj[i % kChains], 0, 0, 0);
+#pragma unroll
+  for (int j = kChains / 2; j > 0; j /= 2)
+#pragma unroll
+    for (int i = 0; i < j; ++i) proj[i] += proj[i + j];
+  float t[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) t[r] = 4 * quarter + r < kMxK ? tanhf(proj[0][r]) * scale : 0.f;
+
+  // lg[c][ii][r]: bucket 256 wave + 64 c + 4 (4 quarter + r) + ii of head n
+  sh_f32x4 lg[4][4];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) lg[c][ii] = sh_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii)
+        // (no prototype past the tenth: zeros, whatever the tenth is)
+        lg[c][ii] = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * quarter + r < kMxK ? pr[c][r][ii] : 0.f, t[r], lg[c][ii], 0, 0, 0);
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, lg[c][ii][r]);
+  mx = fmaxf(mx, lane_xor16(mx));
+  mx = fmaxf(mx, lane_xor32(mx));
+  if (quarter == 0) red[0][wave][n] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(red[0][0][n], red[0][1][n]), fmaxf(red[0][2][n], red[0][3][n]));
+  float sum = 0.f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        lg[c][ii][r] = __builtin_amdgcn_exp2f(lg[c][ii][r] - mx);
+        sum += lg[c][ii][r];
+      }
+  sum += lane_xor16(sum);
+  sum += lane_xor32(sum);
+  if (quarter == 0) red[1][wave][n] = sum;
+  __syncthreads();
+  sum = (red[1][0][n] + red[1][1][n]) + (red[1][2][n] + red[1][3][n]);
+  const float inv = live ? 1.f / sum : 0.f;          // (heads that only fill a unit up are zero)
+  if (!in_units) return;      // (whole groups of W lanes)
+  typename OutDT::storage* base = (typename OutDT::storage*)out + ((int64_t)unit * L + l) * kMxR * W;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float v[4];
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) v[ii] = lg[c][ii][r] * inv;
+      const int bucket = wave * 256 + 64 * c + 16 * quarter + 4 * r;
+      if constexpr (W == 4) {
+        // a quad of lanes holds four heads of four buckets: transposed, lane j has the heads of bucket j
+        const bool up2 = lane & 2, up1 = lane & 1;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const float got = __uint_as_float(sh_dpp_xor2(__float_as_uint(up2 ? v[i] : v[i + 2])));
+          v[i] = up2 ? got : v[i];
+          v[i + 2] = up2 ? v[i + 2] : got;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          const float got = __uint_as_float(sh_dpp_xor1(__float_as_uint(up1 ? v[i] : v[i + 1])));
+          v[i] = up1 ? got : v[i];
+          v[i + 1] = up1 ? v[i + 1] : got;
+        }
+        sh_store4<OutDT>(base, (bucket + (lane & 3)) * 4, v);
+      } else if constexpr (W == 1) {
+        sh_store4<OutDT>(base, bucket, v);
+      } else {
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) store_elem<OutDT>(base, (bucket + ii) * W + n % W, v[ii]);
+      }
+    }
+}
+
+template <int W, class OutDT>
+__global__ __launch_bounds__(kSHThreads) void soft_hash_mx32_kernel(const float* __restrict__ q, int64_t q_sb, int64_t q_sh,
+                                                                    const float* __restrict__ planes, const float* __restrict__ protos_T,
+                                                                    void* __restrict__ out, MxUnits units, int L, float scale) {
+  soft_hash_mx32_block<void, W, OutDT>(blockIdx.x, blockIdx.y, units, q, q_sb, q_sh, planes, protos_T, out, L, scale, nullptr, nullptr, 0, 0,
+                                nullptr);
+}
+
 template <int W, class OT>
 __global__ __launch_bounds__(kSHThreads) void soft_hash_mx_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_sh,
                                                                   const uint16_t* __restrict__ planes,
@@ -685,14 +859,18 @@ __device__ __forceinline__ void soft_hash_block(
 // the query and of every plane, and four buckets; the K sums, the maximum and the sum of exponentials are lane
 // reductions, lane k makes plane k's tanh.  The kernel above leaves three of its four waves without a bucket here and
 // goes through LDS and six barriers, and is bound by that chain: 7.9 us for 32 heads, 32 tables of 8 float32 planes of
-// 128 dims, where this one takes 4.2.
+// 128 dims, where this one takes 4.2 (and 6.5 with the rotation, the append and the key's hash of a decode step, which
+// are 7.3 us in two launches of their own).
 constexpr int kSmallR = 4 * SOCKET_WAVE;
 
-template <class DT, int KM>
-__global__ __launch_bounds__(kSHThreads) void soft_hash_small_kernel(
-    const void* __restrict__ q, int64_t q_sb, int64_t q_sh, const void* __restrict__ planes, const void* __restrict__ protos_T,
-    void* __restrict__ out, int out_dtype, int Hq, int Hkv, int G, int D, int L, int K, int R, float scale, int parts, int width) {
-  const int l = blockIdx.x, pair = blockIdx.y, b = pair / Hkv, kvh = pair % Hkv;
+// FT, freqs, rope_pos, rope_on, q_out: as in soft_hash_block.
+template <class DT, int KM, class FT>
+__device__ __forceinline__ void soft_hash_small_block(
+    const int l, const int pair, const void* __restrict__ q, int64_t q_sb, int64_t q_sh, const void* __restrict__ planes,
+    const void* __restrict__ protos_T, void* __restrict__ out, int out_dtype, int Hq, int Hkv, int G, int D, int L, int K, int R,
+    float scale, int parts, int width, const void* __restrict__ freqs, int64_t rope_pos, bool rope_on, void* __restrict__ q_out) {
+  constexpr bool kRope = !std::is_void<FT>::value;
+  const int b = pair / Hkv, kvh = pair % Hkv;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bool in_d = 4 * lane < D, in_r = 4 * lane < R;
   const int d0 = min(4 * lane, D - 4), r0 = min(4 * lane, R - 4);
@@ -702,11 +880,24 @@ __global__ __launch_bounds__(kSHThreads) void soft_hash_small_kernel(
   for (int k = 0; k < KM; ++k) sh_load4<DT>(planes, ((int64_t)l * K + min(k, K - 1)) * D + d0, pl[k]);
 #pragma unroll
   for (int k = 0; k < KM; ++k) sh_load4<DT>(protos_T, (int64_t)min(k, K - 1) * R + r0, pr[k]);
+  float f[4];
+  // (angles of row 0 for a position outside the table: a load under a condition is waited for at once)
+  if constexpr (kRope) sh_load4<FT>(freqs, (rope_on ? rope_pos : 0) * D + d0, f);
   for (int m = wave; m < members; m += kSHWaves) {
     float lg[4] = {0.f, 0.f, 0.f, 0.f};
     if (m < G) {                                    // (heads that only fill a unit up are zero)
       float x[4], z = 0.f;
       sh_load4<DT>(q, b * q_sb + (int64_t)(kvh * G + m) * q_sh + d0, x);
+      if constexpr (kRope) {
+        if (rope_on) {
+          float re, im;
+          rotate_pair(x[0], x[1], f[0], f[1], re, im);
+          x[0] = sh_round<DT>(re), x[1] = sh_round<DT>(im);
+          rotate_pair(x[2], x[3], f[2], f[3], re, im);
+          x[2] = sh_round<DT>(re), x[3] = sh_round<DT>(im);
+        }
+        if (l == 0 && in_d) sh_store4<DT>(q_out, ((int64_t)b * Hq + kvh * G + m) * D + d0, x);
+      }
 #pragma unroll
       for (int k = 0; k < KM; ++k) {
         float s = x[0] * pl[k][0];
@@ -751,6 +942,14 @@ __global__ __launch_bounds__(kSHThreads) void soft_hash_small_kernel(
   }
 }
 
+template <class DT, int KM>
+__global__ __launch_bounds__(kSHThreads) void soft_hash_small_kernel(
+    const void* __restrict__ q, int64_t q_sb, int64_t q_sh, const void* __restrict__ planes, const void* __restrict__ protos_T,
+    void* __restrict__ out, int out_dtype, int Hq, int Hkv, int G, int D, int L, int K, int R, float scale, int parts, int width) {
+  soft_hash_small_block<DT, KM, void>(blockIdx.x, blockIdx.y, q, q_sb, q_sh, planes, protos_T, out, out_dtype, Hq, Hkv, G, D, L, K, R,
+                                      scale, parts, width, nullptr, 0, false, nullptr);
+}
+
 template <class DT, int GC, int KC>
 __global__ __launch_bounds__(kSHThreads) void soft_hash_kernel(
     const void* __restrict__ q, int64_t q_sb, int64_t q_sh, const void* __restrict__ planes,
@@ -763,8 +962,8 @@ __global__ __launch_bounds__(kSHThreads) void soft_hash_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// The head of a single-token decode step in one launch (bf16, head dimension
-// 128): rotary embedding of the new token's query and key, append of the key and
+// The head of a single-token decode step in one launch (bf16 or fp32, head
+// dimension 128): rotary embedding of the new token's query and key, append of the key and
 // value to the cache, hash of the new key with the value norm, and the soft hash
 // of the rotated query (GPT-FAST/model.py:433-451 and :392-401).  Each of these
 // is a few microseconds of dependent latency on its own, so as three launches
@@ -781,33 +980,80 @@ __global__ __launch_bounds__(kSHThreads) void soft_hash_kernel(
 // k-steps in the same order), so both give the same bits for the same key.
 constexpr int kPrologueD = 128;
 
-// GC: as in soft_hash_block, or 0: soft_hash_mx_block with units of W heads, OT the output's elements.
-template <int GC, class FT, int W, class OT>
+// Eight elements of a row, loaded and stored as they are.
+template <class DT>
+struct alignas(16) sh_row8 {
+  uint4 w[DT::kPer16B == 8 ? 1 : 2];
+};
+template <class DT>
+__device__ __forceinline__ void sh_unpack8(const sh_row8<DT>& r, float (&x)[8]) {
+  if constexpr (DT::kPer16B == 8) {
+    unpack16<DT>(r.w[0], x);
+  } else {
+    __builtin_memcpy(x, r.w, 32);
+  }
+}
+template <class DT>
+__device__ __forceinline__ sh_row8<DT> sh_pack8(const float (&x)[8]) {
+  sh_row8<DT> r;
+  if constexpr (DT::kPer16B == 8) {
+    r.w[0] = make_uint4(f32x2_to_bf16_bits(x[0], x[1]), f32x2_to_bf16_bits(x[2], x[3]), f32x2_to_bf16_bits(x[4], x[5]),
+                        f32x2_to_bf16_bits(x[6], x[7]));
+  } else {
+    __builtin_memcpy(r.w, x, 32);
+  }
+  return r;
+}
+// The eight as bf16, which is what keys are hashed in.
+template <class DT>
+__device__ __forceinline__ uint4 sh_bf16_of8(const sh_row8<DT>& r) {
+  if constexpr (DT::kPer16B == 8) {
+    return r.w[0];
+  } else {
+    float x[8];
+    sh_unpack8<DT>(r, x);
+    return sh_pack8<DType_bf16>(x).w[0];
+  }
+}
+
+// DT: type of the projection, the caches, planes and prototypes.
+// GC: as in soft_hash_block (bf16 only), or 0: soft_hash_mx_block or soft_hash_mx32_block with units of W heads, OT the
+// output's elements; below zero: soft_hash_small_block for at most -GC planes.
+template <class DT, int GC, class FT, int W, class OT>
 __global__ __launch_bounds__(kSHThreads) void decode_prologue_kernel(
-    const uint16_t* __restrict__ qkv, int64_t qkv_sb, const void* __restrict__ freqs,
-    const int64_t* __restrict__ pos, int pos_stride, int64_t n_pos, uint16_t* __restrict__ q_out,
-    uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache, int64_t c_sb, int64_t c_sh, int64_t c_ss,
+    const typename DT::storage* __restrict__ qkv, int64_t qkv_sb, const void* __restrict__ freqs,
+    const int64_t* __restrict__ pos, int pos_stride, int64_t n_pos, typename DT::storage* __restrict__ q_out,
+    typename DT::storage* __restrict__ k_cache, typename DT::storage* __restrict__ v_cache, int64_t c_sb, int64_t c_sh, int64_t c_ss,
     int32_t* __restrict__ lens, const uint16_t* __restrict__ planes_words, uint32_t* __restrict__ codes,
     uint16_t* __restrict__ v_norm, int NW, int64_t Tcap, const void* __restrict__ planes,
     const void* __restrict__ protos_T, void* __restrict__ q_table, int out_dtype, int Hq, int Hkv, int G, int L,
     int K, int R, float tanh_scale, float inv_temperature, int parts, int width, int word_blocks,
     int n_key_blocks, MxUnits units) {
+  typedef typename DT::storage ST;
   constexpr int D = kPrologueD;
+  constexpr bool kF32 = DT::kEnum == SOCKET_F32;
   const int bx = blockIdx.x;
   if (bx >= n_key_blocks) {
     const int i = bx - n_key_blocks;
     const int l = i % L, pair = i / L;
-    if constexpr (GC == 0) {
+    const float mx = mx_scale(tanh_scale, inv_temperature);
+    if constexpr (GC == 0 && kF32) {
+      soft_hash_mx32_block<FT, W, DType_f32>(l, pair, units, qkv, qkv_sb, D, (const float*)planes, (const float*)protos_T, q_table, L, mx,
+                                  freqs, pos, pos_stride, n_pos, q_out);
+    } else if constexpr (GC == 0) {
       soft_hash_mx_block<FT, W, OT>(l, pair, units, qkv, qkv_sb, D, (const uint16_t*)planes, (const uint16_t*)protos_T, (OT*)q_table, L,
-                                    mx_scale(tanh_scale, inv_temperature), freqs, pos, pos_stride, n_pos, q_out);
-      return;
+                                    mx, freqs, pos, pos_stride, n_pos, q_out);
     } else {
-    const int64_t p = pos[(int64_t)(pair / Hkv) * pos_stride];
-    soft_hash_block<DType_bf16, GC, 10, FT>(l, pair, qkv, qkv_sb, D, planes, protos_T, q_table, out_dtype, Hq, Hkv,
-                                            G, D, L, K, R, tanh_scale, inv_temperature, parts, width, 0, 1, freqs, p,
-                                            p >= 0 && p < n_pos, q_out);
-    return;
+      const int64_t p = pos[(int64_t)(pair / Hkv) * pos_stride];
+      const bool turn = p >= 0 && p < n_pos;
+      if constexpr (GC < 0)
+        soft_hash_small_block<DT, -GC, FT>(l, pair, qkv, qkv_sb, D, planes, protos_T, q_table, out_dtype, Hq, Hkv, G, D, L, K, R,
+                                           tanh_scale * inv_temperature, parts, width, freqs, p, turn, q_out);
+      else
+        soft_hash_block<DT, GC, 10, FT>(l, pair, qkv, qkv_sb, D, planes, protos_T, q_table, out_dtype, Hq, Hkv, G, D, L, K, R,
+                                        tanh_scale, inv_temperature, parts, width, 0, 1, freqs, p, turn, q_out);
     }
+    return;
   }
   const int pair = bx / word_blocks, part = bx % word_blocks;
   const int b = pair / Hkv, kvh = pair % Hkv;
@@ -836,62 +1082,70 @@ __global__ __launch_bounds__(kSHThreads) void decode_prologue_kernel(
   }
   // the new key as column 0 of the N operand: lane 16 * quarter holds elements
   // 32 * ks + 8 * quarter .. + 7 of k-step ks, every other column is zero
-  const uint16_t* krow = qkv + b * qkv_sb + (int64_t)(Hq + kvh) * D;
-  const uint16_t* vrow = qkv + b * qkv_sb + (int64_t)(Hq + Hkv + kvh) * D;
-  ShFrag kf[4], vf[4];
+  const ST* krow = qkv + b * qkv_sb + (int64_t)(Hq + kvh) * D;
+  const ST* vrow = qkv + b * qkv_sb + (int64_t)(Hq + Hkv + kvh) * D;
+  typedef sh_row8<DT> Row8;                               // eight elements as they lie in memory
+  ShFrag kf[4];
+  Row8 vr[4];
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
     kf[ks].u = make_uint4(0, 0, 0, 0);
-    vf[ks].u = make_uint4(0, 0, 0, 0);
+    vr[ks] = Row8{};
   }
   if (prow == 0) {
-    uint4 raw[4];
+    Row8 raw[4];
     float f[4][8];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const int e0 = ks * 32 + quarter * 8;
       // (all three fetched whether needed or not -- the angles from row 0 for a position outside
       // the table, the value row by every wave: loads under a condition are waited for one by one)
-      raw[ks] = *reinterpret_cast<const uint4*>(krow + e0);
+      raw[ks] = *reinterpret_cast<const Row8*>(krow + e0);
       sh_load8<FT>(freqs, (rope_on ? p : 0) * D + e0, f[ks]);   // ((p * D/2) + e0/2) * 2
-      vf[ks].u = *reinterpret_cast<const uint4*>(vrow + e0);
+      vr[ks] = *reinterpret_cast<const Row8*>(vrow + e0);
     }
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       if (rope_on) {
-        float x[8];
-        unpack16<DType_bf16>(raw[ks], x);
-        uint32_t o[4];
+        float x[8], o[8];
+        sh_unpack8<DT>(raw[ks], x);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float re, im;
-          rotate_pair(x[2 * j], x[2 * j + 1], f[ks][2 * j], f[ks][2 * j + 1], re, im);
-          o[j] = f32x2_to_bf16_bits(re, im);
-        }
-        kf[ks].u = make_uint4(o[0], o[1], o[2], o[3]);
-      } else {
-        kf[ks].u = raw[ks];
+        for (int j = 0; j < 8; j += 2) rotate_pair(x[j], x[j + 1], f[ks][j], f[ks][j + 1], o[j], o[j + 1]);
+        raw[ks] = sh_pack8<DT>(o);
       }
+      kf[ks].u = sh_bf16_of8<DT>(raw[ks]);
     }
     if (first && rows_ok) {
-      uint16_t* kdst = k_cache + b * c_sb + kvh * c_sh + p * c_ss;
-      uint16_t* vdst = v_cache + b * c_sb + kvh * c_sh + p * c_ss;
+      ST* kdst = k_cache + b * c_sb + kvh * c_sh + p * c_ss;
+      ST* vdst = v_cache + b * c_sb + kvh * c_sh + p * c_ss;
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
         const int e0 = ks * 32 + quarter * 8;
-        *reinterpret_cast<uint4*>(kdst + e0) = kf[ks].u;
-        *reinterpret_cast<uint4*>(vdst + e0) = vf[ks].u;
+        *reinterpret_cast<Row8*>(kdst + e0) = raw[ks];
+        *reinterpret_cast<Row8*>(vdst + e0) = vr[ks];
       }
     }
   }
   if (first) {
     // the cached length follows the position
     if (kvh == 0 && lane == 0 && rows_ok && lens) lens[b] = (int32_t)p + 1;
-    // ||v||^2 = element (0, 0) of the value column against itself: register 0 of lane 0
-    sh_f32x4 g = sh_f32x4{0.f, 0.f, 0.f, 0.f};
+    float norm2;
+    if constexpr (kF32) {
+      // (sixteen lanes of eight elements each, added up as the hash's launch adds them)
+      float x[8];
+      sh_unpack8<DT>(*reinterpret_cast<const Row8*>(vrow + 8 * prow), x);
+      norm2 = 0.f;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) g = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[ks].v, vf[ks].v, g, 0, 0, 0);
-    if (lane == 0 && cached) v_norm[(int64_t)pair * Tcap + p] = f32_to_f16_bits(sqrtf(g[0]));
+      for (int i = 0; i < 8; ++i) norm2 += x[i] * x[i];
+      norm2 = group_sum<16>(norm2);
+    } else {
+      // ||v||^2 = element (0, 0) of the value column against itself: register 0 of lane 0
+      sh_f32x4 g = sh_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) g = sh_mfma(sh_bf16_of8<DT>(vr[ks]), sh_bf16_of8<DT>(vr[ks]), g);
+      norm2 = g[0];
+    }
+    if (lane == 0 && cached) v_norm[(int64_t)pair * Tcap + p] = f32_to_f16_bits(sqrtf(norm2));
   }
   if (w < NW) {
     sh_f32x4 acc[2] = {sh_f32x4{0.f, 0.f, 0.f, 0.f}, sh_f32x4{0.f, 0.f, 0.f, 0.f}};
@@ -975,6 +1229,21 @@ int soft_hash_entry(const void* q, int dtype, int64_t q_stride_b, int64_t q_stri
     SOCKET_LAUNCH_CHECK();
     return SOCKET_OK;
   }
+  if (dtype == SOCKET_F32 && mx_serves(D, K, R) && vec_ok) {
+    const MxUnits units = mx_units(B, Hq, Hkv, parts);
+    const int W = grouped ? width : 1, per = kMxHeads / W;
+    const dim3 mx_grid(L, (units.count + per - 1) / per);
+    SOCKET_REQUIRE(mx_grid.y <= 65535, SOCKET_ERR_SHAPE);
+    auto of_type = [&](auto dt) {
+      typedef decltype(dt) OutDT;
+      return W == 4 ? soft_hash_mx32_kernel<4, OutDT> : W == 2 ? soft_hash_mx32_kernel<2, OutDT> : soft_hash_mx32_kernel<1, OutDT>;
+    };
+    auto kern = out_dtype == SOCKET_F32 ? of_type(DType_f32{}) : of_type(DType_bf16{});
+    hipLaunchKernelGGL(kern, mx_grid, dim3(kSHThreads), 0, s, (const float*)q, q_stride_b, q_stride_h, (const float*)planes,
+                       (const float*)protos_T, out, units, L, mx_scale(tanh_scale, inv_temperature));
+    SOCKET_LAUNCH_CHECK();
+    return SOCKET_OK;
+  }
   // K = 10 with a single sweep (R <= 4 buckets per lane) and vector loads: the
   // prototypes go from global memory straight into registers.  Otherwise they go
   // to LDS as fp32 when they fit in 64 KB, else they are read from global memory
@@ -1052,7 +1321,9 @@ extern "C" int socket_soft_hash_grouped(const void* q, int dtype, int64_t q_stri
                          L, K, R, tanh_scale, inv_temperature, stream, 1);
 }
 
-extern "C" int socket_decode_prologue(const void* qkv, int dtype, int64_t qkv_stride_b, const void* freqs_cis,
+namespace {
+
+int decode_prologue_entry(const void* qkv, int dtype, int64_t qkv_stride_b, const void* freqs_cis,
                                       int freqs_dtype, int64_t n_pos, const int64_t* pos, int pos_stride,
                                       void* q_out, void* k_cache, void* v_cache, int64_t cache_stride_b,
                                       int64_t cache_stride_h, int64_t cache_stride_s, int32_t* lens,
@@ -1064,7 +1335,9 @@ extern "C" int socket_decode_prologue(const void* qkv, int dtype, int64_t qkv_st
                      planes && protos_T && q_table,
                  SOCKET_ERR_NULL);
   // the shapes the fused launch is written for; anything else takes the separate entry points
-  SOCKET_REQUIRE(dtype == SOCKET_BF16 && D == kPrologueD && K == 10, SOCKET_ERR_UNSUPPORTED);
+  const bool mx = mx_serves(D, K, R), small = K != 10 && R <= kSmallR;
+  SOCKET_REQUIRE((dtype == SOCKET_BF16 || dtype == SOCKET_F32) && D == kPrologueD && K >= 1 && K <= kSHMaxK, SOCKET_ERR_UNSUPPORTED);
+  SOCKET_REQUIRE(small || (dtype == SOCKET_BF16 ? K == 10 : mx && out_dtype == SOCKET_F32), SOCKET_ERR_UNSUPPORTED);
   SOCKET_REQUIRE(freqs_dtype == SOCKET_F32 || freqs_dtype == SOCKET_BF16, SOCKET_ERR_UNSUPPORTED);
   SOCKET_REQUIRE(out_dtype == SOCKET_F32 || out_dtype == SOCKET_BF16, SOCKET_ERR_UNSUPPORTED);
   SOCKET_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && L > 0 && Tcap > 0 && n_pos > 0, SOCKET_ERR_SHAPE);
@@ -1093,41 +1366,68 @@ extern "C" int socket_decode_prologue(const void* qkv, int dtype, int64_t qkv_st
                                kSHWaves * GC + 3) / 4) * 4;
   const size_t dyn_lds = head_floats * sizeof(float);
   hipStream_t s = (hipStream_t)stream;
-  const bool mx = mx_serves(D, K, R);
   const MxUnits units = mx_units(B, Hq, Hkv, parts);
   const int W = grouped ? width : 1, per = kMxHeads / W;
   const int64_t blocks = mx ? n_key_blocks + (int64_t)((units.count + per - 1) / per) * L : n_blocks;
-#define SOCKET_DP(GCV, FT, WV, OT)                                                                              \
-  hipLaunchKernelGGL((decode_prologue_kernel<GCV, FT, WV, OT>), dim3((unsigned)blocks), dim3(kSHThreads), mx ? 0 : dyn_lds, s, \
-                     (const uint16_t*)qkv, qkv_stride_b, freqs_cis, pos, pos_stride, n_pos, (uint16_t*)q_out,   \
-                     (uint16_t*)k_cache, (uint16_t*)v_cache, cache_stride_b, cache_stride_h, cache_stride_s,    \
-                     lens, (const uint16_t*)planes_words, (uint32_t*)codes, (uint16_t*)v_norm, NW, Tcap,        \
-                     planes, protos_T, q_table, out_dtype, Hq, Hkv, G, L, K, R, tanh_scale, inv_temperature,    \
-                     parts, width, word_blocks, (int)n_key_blocks, units)
-#define SOCKET_DP_MX(FT)                                                     \
-  do {                                                                       \
-    if (out_dtype == SOCKET_F32) {                                           \
-      if (W == 4) SOCKET_DP(0, FT, 4, float);                                \
-      else if (W == 2) SOCKET_DP(0, FT, 2, float);                           \
-      else SOCKET_DP(0, FT, 1, float);                                       \
-    } else {                                                                 \
-      if (W == 4) SOCKET_DP(0, FT, 4, uint16_t);                             \
-      else if (W == 2) SOCKET_DP(0, FT, 2, uint16_t);                        \
-      else SOCKET_DP(0, FT, 1, uint16_t);                                    \
-    }                                                                        \
+#define SOCKET_DP(DT, GCV, FT, WV, OT)                                                                                        \
+  hipLaunchKernelGGL((decode_prologue_kernel<DT, GCV, FT, WV, OT>), dim3((unsigned)blocks), dim3(kSHThreads), GCV > 0 ? dyn_lds : 0, s, \
+                     (const DT::storage*)qkv, qkv_stride_b, freqs_cis, pos, pos_stride, n_pos, (DT::storage*)q_out,            \
+                     (DT::storage*)k_cache, (DT::storage*)v_cache, cache_stride_b, cache_stride_h, cache_stride_s, lens,       \
+                     (const uint16_t*)planes_words, (uint32_t*)codes, (uint16_t*)v_norm, NW, Tcap, planes, protos_T, q_table,  \
+                     out_dtype, Hq, Hkv, G, L, K, R, tanh_scale, inv_temperature, parts, width, word_blocks,                   \
+                     (int)n_key_blocks, units)
+#define SOCKET_DP_MX(DT, FT, OT)                  \
+  do {                                            \
+    if (W == 4) SOCKET_DP(DT, 0, FT, 4, OT);      \
+    else if (W == 2) SOCKET_DP(DT, 0, FT, 2, OT); \
+    else SOCKET_DP(DT, 0, FT, 1, OT);             \
   } while (0)
-  if (mx) {
-    if (freqs_dtype == SOCKET_F32) SOCKET_DP_MX(DType_f32);
-    else SOCKET_DP_MX(DType_bf16);
-  } else if (GC == 4) {
-    if (freqs_dtype == SOCKET_F32) SOCKET_DP(4, DType_f32, 1, float);
-    else SOCKET_DP(4, DType_bf16, 1, float);
-  } else {
-    if (freqs_dtype == SOCKET_F32) SOCKET_DP(8, DType_f32, 1, float);
-    else SOCKET_DP(8, DType_bf16, 1, float);
-  }
+#define SOCKET_DP_FT(FT)                                                                  \
+  do {                                                                                    \
+    if (small && dtype == SOCKET_F32) {                                                   \
+      if (K <= 8) SOCKET_DP(DType_f32, -8, FT, 1, float);                                 \
+      else SOCKET_DP(DType_f32, -kSHMaxK, FT, 1, float);                                  \
+    } else if (small) {                                                                   \
+      if (K <= 8) SOCKET_DP(DType_bf16, -8, FT, 1, float);                                \
+      else SOCKET_DP(DType_bf16, -kSHMaxK, FT, 1, float);                                 \
+    } else if (dtype == SOCKET_F32) SOCKET_DP_MX(DType_f32, FT, float);                   \
+    else if (mx && out_dtype == SOCKET_F32) SOCKET_DP_MX(DType_bf16, FT, float);          \
+    else if (mx) SOCKET_DP_MX(DType_bf16, FT, uint16_t);                                  \
+    else if (GC == 4) SOCKET_DP(DType_bf16, 4, FT, 1, float);                             \
+    else SOCKET_DP(DType_bf16, 8, FT, 1, float);                                          \
+  } while (0)
+  if (freqs_dtype == SOCKET_F32) SOCKET_DP_FT(DType_f32);
+  else SOCKET_DP_FT(DType_bf16);
+#undef SOCKET_DP_FT
 #undef SOCKET_DP_MX
 #undef SOCKET_DP
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
+}
+
+}  // namespace
+
+extern "C" int socket_decode_prologue(const void* qkv, int dtype, int64_t qkv_stride_b, const void* freqs_cis,
+                                      int freqs_dtype, int64_t n_pos, const int64_t* pos, int pos_stride,
+                                      void* q_out, void* k_cache, void* v_cache, int64_t cache_stride_b,
+                                      int64_t cache_stride_h, int64_t cache_stride_s, int32_t* lens,
+                                      const void* planes_words, void* codes, void* v_norm, const void* planes,
+                                      const void* protos_T, void* q_table, int out_dtype, int grouped, int B,
+                                      int Hq, int Hkv, int D, int L, int K, int R, int64_t Tcap,
+                                      float tanh_scale, float inv_temperature, void* stream) {
+  // (what this entry has always taken: bf16, ten planes)
+  SOCKET_REQUIRE(qkv && freqs_cis && pos && q_out && k_cache && v_cache && planes_words && codes && v_norm && planes && protos_T && q_table, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(dtype == SOCKET_BF16 && K == 10, SOCKET_ERR_UNSUPPORTED);
+  return decode_prologue_entry(qkv, dtype, qkv_stride_b, freqs_cis, freqs_dtype, n_pos, pos, pos_stride, q_out, k_cache, v_cache, cache_stride_b, cache_stride_h, cache_stride_s, lens, planes_words, codes, v_norm, planes, protos_T, q_table, out_dtype, grouped, B, Hq, Hkv, D, L, K, R, Tcap, tanh_scale, inv_temperature, stream);
+}
+
+extern "C" int socket_decode_prologue_typed(const void* qkv, int dtype, int64_t qkv_stride_b, const void* freqs_cis,
+                                      int freqs_dtype, int64_t n_pos, const int64_t* pos, int pos_stride,
+                                      void* q_out, void* k_cache, void* v_cache, int64_t cache_stride_b,
+                                      int64_t cache_stride_h, int64_t cache_stride_s, int32_t* lens,
+                                      const void* planes_words, void* codes, void* v_norm, const void* planes,
+                                      const void* protos_T, void* q_table, int out_dtype, int grouped, int B,
+                                      int Hq, int Hkv, int D, int L, int K, int R, int64_t Tcap,
+                                      float tanh_scale, float inv_temperature, void* stream) {
+  return decode_prologue_entry(qkv, dtype, qkv_stride_b, freqs_cis, freqs_dtype, n_pos, pos, pos_stride, q_out, k_cache, v_cache, cache_stride_b, cache_stride_h, cache_stride_s, lens, planes_words, codes, v_norm, planes, protos_T, q_table, out_dtype, grouped, B, Hq, Hkv, D, L, K, R, Tcap, tanh_scale, inv_temperature, stream);
 }

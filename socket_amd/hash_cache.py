@@ -232,8 +232,13 @@ def soft_hash(queries_bhd: torch.Tensor, planes_lkd: torch.Tensor, protos_T: tor
 def decode_prologue_fits(qkv: torch.Tensor, head_dim: int, K: int, R: int, n_heads: int, n_kv_heads: int) -> bool:
     """Whether `decode_prologue` takes these operands (else: rope_append, hash_keys_into
     and soft_hash, three launches with the same results)."""
-    return (qkv.is_cuda and qkv.dtype == torch.bfloat16 and head_dim == HASH_DIM and K == 10 and R % 4 == 0 and
-            4 <= R <= 1024 and n_heads % n_kv_heads == 0 and n_heads // n_kv_heads <= 8)
+    if not (qkv.is_cuda and head_dim == HASH_DIM and R % 4 == 0 and 4 <= R <= 1024 and n_heads % n_kv_heads == 0
+            and n_heads // n_kv_heads <= 8):
+        return False
+    if qkv.dtype == torch.bfloat16 and K == 10:
+        return True
+    return (qkv.dtype in (torch.bfloat16, torch.float32) and (R <= 256 if K != 10 else R == 1024) and 1 <= K <= 16
+            and qkv.data_ptr() % 16 == 0 and (qkv.shape[0] == 1 or qkv.stride(0) % 8 == 0))
 
 
 @torch.no_grad()
@@ -274,7 +279,7 @@ def decode_prologue(qkv: torch.Tensor, freqs_cis: torch.Tensor, input_pos: torch
         table = torch.empty((B, n_kv_heads * parts, L, R, width), dtype=q2.dtype, device=q2.device)
     else:
         table = torch.empty((B, n_heads, L, R), dtype=q2.dtype, device=q2.device)
-    check("socket_decode_prologue", lib().socket_decode_prologue(
+    check("socket_decode_prologue", lib().socket_decode_prologue_typed(
         ptr(q2), dtype_enum(q2.dtype), q2.stride(0), ptr(freqs_cis), dtype_enum(freqs_cis.dtype), freqs_cis.shape[0],
         ptr(input_pos), 0 if input_pos.numel() == 1 else 1, ptr(q_out), ptr(k_cache), ptr(v_cache),
         k_cache.stride(0), k_cache.stride(1), k_cache.stride(2), ptr(lens), ptr(planes_words), ptr(codes),
