@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
 }
 
 // ---------------------------------------------------------------------------
-// Streamed variant for large bf16 launches (prefill).
+// Streamed variant for large launches (prefill).
 //
 // The roles are turned round: the PLANES are stationary in registers and the
 // keys stream through LDS.  Wave i of the eight owns packed words i, i + 8 and
@@ -337,26 +337,37 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
 // chunk s ^ (r & 15), so the image needs no pass of its own, and the sixteen
 // lanes of a fragment read (sixteen consecutive rows, one chunk) hit sixteen
 // different slots.
-constexpr int kStreamTile = 128;                       // keys per tile
-constexpr int stream_stage_bytes(int D) { return 2 * kStreamTile * D * 2; }   // keys | values
+constexpr int kStreamTile = 128;                       // keys per tile, at most
+// LDS of a stage: bf16 keys, and the values where they come straight into LDS
+constexpr int stream_stage_bytes(int dtype, int D, int tile) { return (dtype == SOCKET_BF16 ? 2 : 1) * tile * D * 2; }
 constexpr int kStreamWordsPerWave = 3;
 constexpr int kStreamMaxWords = kStreamWordsPerWave * kHashWaves;
 
-// D: 128, or 64 (half the contraction: the planes' other half is zero).  STORE: the tile's rows also go on
-// into k_cache / v_cache (element strides c_sb, c_sh, c_ss) at their positions, from LDS: an append then
+// Keys of other types have to be rounded to bf16 on the way, and their value norms are fp32 sums: their tiles (64 keys of
+// 128 dims, so that the registers suffice) are loaded into registers a tile ahead, eight elements of a row to a lane, and
+// from there go on into the caches, into the norms and, rounded, into the same LDS image.
+// The whole append of 8 pairs, 20 words, us before (staged, the copy a launch of its own): 128 dims, 3000 / 12000 / 50000 tokens
+// fp16 27.6 / 59.9 / 211 -> 15.8 / 36.5 / 118, fp32 36 / 86 / 312 -> 20.8 / 55 / 196 (89 % of a copy's rate);
+// 64 dims fp16 24 / 45 / 153 -> 9.7 / 20 / 65, fp32 26 / 58 / 200 -> 12.6 / 31 / 107.  bf16, whose lengths were a launch of
+// their own and whose tiles were 128 keys always: 20.8 / 35.8 / 118 -> 14.7 / 33.9 / 115.
+//
+// D: 128, or 64 (half the contraction: the planes' other half is zero).  kTile: 128 or 64 keys.  STORE: the tile's rows also go on
+// into k_cache / v_cache (element strides c_sb, c_sh, c_ss) at their positions: an append then
 // reads its keys and values once.
-template <int D, bool STORE>
+template <class DT, int D, int kTile, bool STORE>
 __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void hash_keys_stream_kernel(
-    const uint16_t* __restrict__ k_, const uint16_t* __restrict__ v_, int64_t k_sb, int64_t k_sh,
+    const typename DT::storage* __restrict__ k_, const typename DT::storage* __restrict__ v_, int64_t k_sb, int64_t k_sh,
     int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
     const uint16_t* __restrict__ planes_words,  // bf16 [NW*32, 128]
     uint32_t* __restrict__ codes, uint16_t* __restrict__ v_norm,
     const int32_t* __restrict__ pos_b, int t0, int Hkv, int S, int L, int P, int NW, int64_t Tcap,
-    int tiles_per_row, int n_tiles, uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache, int64_t c_sb,
-    int64_t c_sh, int64_t c_ss) {
-  constexpr int kKSteps = D / 32, CH = D / 8, kRows = 64 / CH;      // k-steps; 16-byte pieces of a row; rows of a 1 KB copy
-  constexpr int kStreamTileBytes = kStreamTile * D * 2, kStreamStageBytes = stream_stage_bytes(D);
-  constexpr int kPieces = kStreamTile / kRows / kHashWaves;
+    int tiles_per_row, int n_tiles, typename DT::storage* __restrict__ k_cache, typename DT::storage* __restrict__ v_cache,
+    int64_t c_sb, int64_t c_sh, int64_t c_ss, int32_t* __restrict__ lens, int B) {
+  typedef typename DT::storage ST;
+  constexpr bool kDma = DT::kEnum == SOCKET_BF16;
+  constexpr int kKSteps = D / 32, CH = D / 8, kRows = 64 / CH;      // k-steps; 8-element pieces of a row; rows of a wave's copy
+  constexpr int kStreamTileBytes = kTile * D * 2, kStreamStageBytes = stream_stage_bytes(DT::kEnum, D, kTile);
+  constexpr int kPieces = kTile / kRows / kHashWaves;
   // where piece c of row r goes: sixteen consecutive rows at one piece must hit sixteen different 16-byte
   // slots of the banks (rows of 128 bytes start half a bank line apart by the row's parity)
   auto place = [](int r, int c) { return c ^ (CH == 16 ? (r & 15) : ((r >> 1) & 7)); };
@@ -394,46 +405,89 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
   // (a copy's rows are all the same modulo 16, so a lane's piece is too)
   const int lane_at = lane / CH * (int)(c_ss / 8) + place(kRows * wave + lane / CH, lane % CH);
 
-  // this wave's four 1 KB pieces of a tile (rows 4p .. 4p+3 of piece p), keys and values
-  auto issue_tile = [&](int tile, int stage) {
+  // eight elements of a row as they lie in memory
+  struct alignas(16) Row8 {
+    uint4 w[DT::kPer16B == 8 ? 1 : 2];
+  };
+  Row8 kreg[kDma ? 1 : kPieces], vreg[kDma ? 1 : kPieces];
+  auto load_row8 = [&](const ST* p) __attribute__((always_inline)) {
+    typedef uint32_t u32x4_s __attribute__((ext_vector_type(4)));
+    Row8 r;
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(Row8) / 16); ++i) {
+      const u32x4_s v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_s*>(p) + i);
+      r.w[i] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+    return r;
+  };
+  // this wave's pieces of a tile (rows kRows p .. of piece p), keys and values: into LDS, or into registers
+  auto issue_tile = [&](int tile, int stage) __attribute__((always_inline)) {
     const int pair = tile / tiles_per_row;
-    const int s0 = (tile % tiles_per_row) * kStreamTile;
+    const int s0 = (tile % tiles_per_row) * kTile;
     const int b = pair / Hkv, h = pair % Hkv;
-    const uint16_t* kbase = k_ + b * k_sb + h * k_sh;
-    const uint16_t* vbase = with_values ? v_ + b * v_sb + h * v_sh : nullptr;
+    const ST* kbase = k_ + b * k_sb + h * k_sh;
+    const ST* vbase = with_values ? v_ + b * v_sb + h * v_sh : nullptr;
     unsigned char* dst = lds_raw + (size_t)stage * kStreamStageBytes;
 #pragma unroll
     for (int q = 0; q < kPieces; ++q) {
       const int p = wave + kHashWaves * q;
       const int row = kRows * p + lane / CH;
       const int srow = min(s0 + row, S - 1);  // rows past the end re-read the last one; never stored
-      const int chunk = place(kRows * wave + lane / CH, lane % CH);
-      lds_dma16_stream(kbase + (int64_t)srow * k_ss + chunk * 8, dst + p * 1024);
-      if (with_values) lds_dma16_stream(vbase + (int64_t)srow * v_ss + chunk * 8, dst + kStreamTileBytes + p * 1024);
+      if constexpr (kDma) {
+        const int chunk = place(kRows * wave + lane / CH, lane % CH);
+        lds_dma16_stream(kbase + (int64_t)srow * k_ss + chunk * 8, dst + p * 1024);
+        if (with_values) lds_dma16_stream(vbase + (int64_t)srow * v_ss + chunk * 8, dst + kStreamTileBytes + p * 1024);
+      } else {
+        kreg[q] = load_row8(kbase + (int64_t)srow * k_ss + lane % CH * 8);
+        if (with_values) vreg[q] = load_row8(vbase + (int64_t)srow * v_ss + lane % CH * 8);
+      }
     }
   };
 
   int tile = blockIdx.x;
   if (tile < n_tiles) issue_tile(tile, 0);
+  if (STORE && lens && blockIdx.x == 0)
+    for (int b = tid; b < B; b += kHashThreads) lens[b] = t0 + S;
   for (int it = 0; tile < n_tiles; tile += gridDim.x, ++it) {
     const int stage = it & 1;
     const int next = tile + gridDim.x;
+    const int pair = tile / tiles_per_row;
+    const int s0 = (tile % tiles_per_row) * kTile;
+    const int pos0 = pos_b ? pos_b[pair / Hkv] : t0;
+    if constexpr (!kDma) {
+      // out of the registers: rounded keys into the stage (left by every wave before the last barrier), rows into the
+      // caches, norms
+      uint4* image = reinterpret_cast<uint4*>(lds_raw + (size_t)stage * kStreamStageBytes);
+#pragma unroll
+      for (int q = 0; q < kPieces; ++q) {
+        const int r = kRows * (wave + kHashWaves * q) + lane / CH, c = lane % CH;
+        image[r * CH + place(r, c)] = load_frag8<DT>(reinterpret_cast<const ST*>(kreg[q].w));
+        if constexpr (STORE) {
+          if (s0 + r < S) {
+            const int64_t at = (int64_t)(pair / Hkv) * c_sb + (pair % Hkv) * c_sh + (int64_t)(pos0 + s0 + r) * c_ss + c * 8;
+            *reinterpret_cast<Row8*>(k_cache + at) = kreg[q];
+            *reinterpret_cast<Row8*>(v_cache + at) = vreg[q];
+          }
+        }
+        if (with_values) {
+          const float t = group_sum<CH>(sumsq8<DT>(reinterpret_cast<const ST*>(vreg[q].w)));
+          if (c == 0 && s0 + r < S && in_cache(pos0 + s0 + r, Tcap)) v_norm[(int64_t)pair * Tcap + pos0 + s0 + r] = f32_to_f16_bits(sqrtf(t));
+        }
+      }
+    }
     // One barrier per tile: behind it every wave's pieces of this tile are in place
     // AND every wave is done with the previous tile, whose stage the next tile's
     // loads may therefore overwrite while this one is contracted.
-    wait_vmcnt(0);
+    if constexpr (kDma) wait_vmcnt(0);
     __syncthreads();
     if (next < n_tiles) issue_tile(next, stage ^ 1);
 
-    const int pair = tile / tiles_per_row;
-    const int s0 = (tile % tiles_per_row) * kStreamTile;
-    const int pos0 = pos_b ? pos_b[pair / Hkv] : t0;
     const uint4* ktile = reinterpret_cast<const uint4*>(lds_raw + (size_t)stage * kStreamStageBytes);
     const uint4* vtile = ktile + kStreamTileBytes / 16;
     // chunk c of row r of a tile (r & 15 == prow for every row this lane reads)
     auto frag_at = [&](const uint4* t, int r, int c) { return t[r * CH + place(prow, c)]; };
 
-    if constexpr (STORE) {
+    if constexpr (STORE && kDma) {
       // this wave's pieces of the tile on into the caches, whole rows of 256 (128) bytes
       const int64_t c0 = (int64_t)(pair / Hkv) * c_sb + (pair % Hkv) * c_sh + (int64_t)(pos0 + s0 + kRows * wave) * c_ss;
 #pragma unroll
@@ -445,7 +499,7 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
         }
     }
 
-    if (with_values) {
+    if (kDma && with_values && wave < kTile / 16) {
       // ||v||^2 = diagonal of V V^T (see hash_keys_kernel), key block `wave` of the tile
       Frag vf[kKSteps];
 #pragma unroll
@@ -461,7 +515,7 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
     }
 
     uint32_t* codes_pair = codes + (int64_t)pair * NW * Tcap;
-    // The tile's eight 16-key blocks go through in pairs, the next pair's
+    // The tile's 16-key blocks go through in pairs, the next pair's
     // fragments on their way from LDS while the current pair is contracted.  A
     // 64-key group is taken high blocks first, (3,2) then (1,0), so that the sign
     // bits shift into `neg` in the byte order the transpose expects.
@@ -519,10 +573,10 @@ __global__ __launch_bounds__(kHashThreads) __attribute__((amdgpu_waves_per_eu(2,
       Frag kfa[2][kKSteps], kfb[2][kKSteps];
       load_pair(0, kfa);
 #pragma unroll
-      for (int pp = 0; pp < kStreamTile / 32; pp += 2) {
+      for (int pp = 0; pp < kTile / 32; pp += 2) {
         load_pair(pp + 1, kfb);
         do_pair(pp, kfa);
-        if (pp + 2 < kStreamTile / 32) load_pair(pp + 2, kfa);
+        if (pp + 2 < kTile / 32) load_pair(pp + 2, kfa);
         do_pair(pp + 1, kfb);
       }
     };
@@ -699,12 +753,11 @@ __global__ __launch_bounds__(256) void copy_rows_kernel(const void* __restrict__
                                                         int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss,
                                                         void* __restrict__ k_cache, void* __restrict__ v_cache, int64_t c_sb,
                                                         int64_t c_sh, int64_t c_ss, int32_t* __restrict__ lens, int t0, int B,
-                                                        int Hkv, int S, int D, int copy) {
+                                                        int Hkv, int S, int D) {
   typedef typename DT::storage ST;
   constexpr int E = DT::kPer16B;
   if (lens && blockIdx.x == 0 && blockIdx.y == 0)
     for (int b = threadIdx.x; b < B; b += 256) lens[b] = t0 + S;
-  if (!copy) return;
   const int b = blockIdx.y / Hkv, h = blockIdx.y % Hkv, per = D / E;
   const ST* kp = (const ST*)k + b * k_sb + h * k_sh;
   const ST* vp = (const ST*)v + b * v_sb + h * v_sh;
@@ -837,39 +890,80 @@ struct HashRows {
   int64_t c_sb, c_sh, c_ss;
 };
 
-// Enough 128-key tiles to keep every CU streaming: the variant with the planes in registers.
-bool streams(const HashRows& a, const SocketDeviceLimits& lim) {
-  const int64_t tiles = (int64_t)a.B * a.Hkv * ((a.S + kStreamTile - 1) / kStreamTile);
-  return a.dtype == SOCKET_BF16 && (a.D == 128 || a.D == 64) && a.NW <= kStreamMaxWords && tiles >= lim.cu_count &&
-         2 * stream_stage_bytes(a.D) <= lim.max_lds_per_block;
+int64_t stream_tiles(const HashRows& a, int tile) { return (int64_t)a.B * a.Hkv * ((a.S + tile - 1) / tile); }
+
+// Keys of a tile: 128, halves where that leaves CUs idle or (rows of 128 dims that go through the registers) is more than
+// the registers hold.
+int stream_tile(const HashRows& a, const SocketDeviceLimits& lim) {
+  if (a.dtype != SOCKET_BF16 && a.D == 128) return kStreamTile / 2;
+  return stream_tiles(a, kStreamTile) >= lim.cu_count ? kStreamTile : kStreamTile / 2;
 }
 
-template <int D, bool STORE>
-int launch_stream(const HashRows& a, const SocketDeviceLimits& lim, hipStream_t s) {
-  const int tiles_per_row = (a.S + kStreamTile - 1) / kStreamTile;
-  const int64_t n_tiles64 = (int64_t)a.B * a.Hkv * tiles_per_row;
-  const size_t lds = 2 * (size_t)stream_stage_bytes(D);
-  auto kern = hash_keys_stream_kernel<D, STORE>;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+
+// Whether the variant with the planes in registers serves: rows of 128 or 64 dims, up to 24 words, and so many rows that what
+// a workgroup fetches once, all planes (160 KB at 20 words), no longer outweighs what the direct variant fetches for
+// every tile and word.  The whole append of 8 pairs, us, direct / streamed: 128 dims, 20 words, bf16 4000 rows 8.7 / 9.3, 6216
+// 10.4 / 9.8, 8800 13.1 / 10.4; fp16 2400 7.1 / 9.7, 4000 10.2 / 9.9, 8800 13.0 / 10.7; fp32 2400 8.8 / 11.2, 4000 12.5 / 12.2;
+// 8 words, bf16 2400 5.4 / 6.0, 4000 6.5 / 6.2, 6216 9.3 / 6.4.  64 dims, 20 words, 2400 rows: 6.4 / 6.0, 6.4 / 6.2, 7.3 / 6.7;
+// 6216: 7.5 / 6.4, 8.3 / 6.4, 10.1 / 7.5.  (The staged variant is behind from 5000 rows on: 24000 rows, 128 dims, 20 words,
+// with the copy 21.0 / 14.7, 27.5 / 15.7, 35.5 / 20.8.)  Many pairs of few rows each leave most of a tile empty: not
+// unless every CU has a tile of 128 all the same.
+bool streams(const HashRows& a, const SocketDeviceLimits& lim) {
+  if ((a.D != 128 && a.D != 64) || a.NW > kStreamMaxWords) return false;
+  const int tile = stream_tile(a, lim);
+  if (2 * stream_stage_bytes(a.dtype, a.D, tile) > lim.max_lds_per_block) return false;
+  const int64_t rows = (int64_t)a.B * a.Hkv * a.S;
+  return stream_tiles(a, kStreamTile) >= lim.cu_count ||
+         (rows >= (a.D == 64 ? 2048 : 4096 + 128 * a.NW) && 2 * rows >= stream_tiles(a, tile) * tile);
+}
+
+template <class DT, int D, int kTile, bool STORE>
+int launch_stream_of(const HashRows& a, const SocketDeviceLimits& lim, int32_t* lens, hipStream_t s) {
+  typedef typename DT::storage ST;
+  const int tiles_per_row = (a.S + kTile - 1) / kTile;
+  const int64_t n_tiles = (int64_t)a.B * a.Hkv * tiles_per_row;
+  const size_t lds = 2 * (size_t)stream_stage_bytes(DT::kEnum, D, kTile);
+  auto kern = hash_keys_stream_kernel<DT, D, kTile, STORE>;
+  if (lds > 48 * 1024 &&
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return SOCKET_ERR_LAUNCH;
-  const int n_wg = (int)(n_tiles64 < lim.cu_count ? n_tiles64 : lim.cu_count);
-  hipLaunchKernelGGL(kern, dim3(n_wg), dim3(kHashThreads), lds, s, (const uint16_t*)a.k, (const uint16_t*)a.v, a.k_sb, a.k_sh,
-                     a.k_ss, a.v_sb, a.v_sh, a.v_ss, (const uint16_t*)a.planes_words, a.codes, a.v_norm, a.pos_b, a.t0, a.Hkv,
-                     a.S, a.L, a.P, a.NW, a.Tcap, tiles_per_row, (int)n_tiles64, (uint16_t*)a.k_cache, (uint16_t*)a.v_cache,
-                     a.c_sb, a.c_sh, a.c_ss);
+  const int n_wg = (int)(n_tiles < lim.cu_count ? n_tiles : lim.cu_count);
+  hipLaunchKernelGGL(kern, dim3(n_wg), dim3(kHashThreads), lds, s, (const ST*)a.k, (const ST*)a.v, a.k_sb, a.k_sh, a.k_ss, a.v_sb,
+                     a.v_sh, a.v_ss, (const uint16_t*)a.planes_words, a.codes, a.v_norm, a.pos_b, a.t0, a.Hkv, a.S, a.L, a.P, a.NW,
+                     a.Tcap, tiles_per_row, (int)n_tiles, (ST*)a.k_cache, (ST*)a.v_cache, a.c_sb, a.c_sh, a.c_ss, lens, a.B);
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
 }
 
+template <bool STORE>
+int launch_stream(const HashRows& a, const SocketDeviceLimits& lim, int32_t* lens, hipStream_t s) {
+  const bool half = stream_tile(a, lim) < kStreamTile;
+#define SOCKET_STREAM(DT, D)                                                                             \
+  return half ? launch_stream_of<DT, D, kStreamTile / 2, STORE>(a, lim, lens, s)                         \
+              : launch_stream_of<DT, D, kStreamTile, STORE>(a, lim, lens, s)
+  if (a.D == 64) {
+    if (a.dtype == SOCKET_BF16) SOCKET_STREAM(DType_bf16, 64);
+    if (a.dtype == SOCKET_F16) SOCKET_STREAM(DType_f16, 64);
+    SOCKET_STREAM(DType_f32, 64);
+  }
+  if (a.dtype == SOCKET_BF16) SOCKET_STREAM(DType_bf16, 128);
+  if (a.dtype == SOCKET_F16) return launch_stream_of<DType_f16, 128, kStreamTile / 2, STORE>(a, lim, lens, s);
+  return launch_stream_of<DType_f32, 128, kStreamTile / 2, STORE>(a, lim, lens, s);
+#undef SOCKET_STREAM
+}
+
 // Few enough rows for the direct variant.  Its time grows with rows x words, since a wave fetches its tile's keys and
-// its word's planes for itself; the others' hardly does below a few tiles per CU.  Hashing 8 pairs' rows with 20
+// its word's planes for itself; the staged variant's hardly does below a few tiles per CU.  Hashing 8 pairs' rows with 20
 // words, bf16 of 128 dims, direct / staged: 8192 rows 10.4 / 11.8 us, 12288 13.5 / 12.1; with 8 words 24576 rows 11.3 / 12.0.
 // The lines cross between 180k (float32) and 260k words; with the copy in the same launch (one fewer) between 270k and
-// 400k: 12288 rows of 64 dims in 16 bits 12.1 / 15.6 us, 16384 of 128 bf16 dims 18.5 / 17.4.  Where the streamed kernel
-// has at least half of every tile it is ahead of both (32768 rows, 8 words: 7.0 against 14.5 direct).
-bool goes_direct(const HashRows& a, bool streamed) {
-  const int64_t rows = (int64_t)a.B * a.Hkv * a.S, tiles = (int64_t)a.B * a.Hkv * ((a.S + kStreamTile - 1) / kStreamTile);
-  if (streamed && 2 * rows >= tiles * kStreamTile) return false;
+// 400k.  Where the streamed kernel serves and has at least half of every tile it is ahead of both (32768 rows, 8 words:
+// 7.0 against 14.5 direct).
+bool goes_direct(const HashRows& a, const SocketDeviceLimits& lim, bool streamed) {
+  const int64_t rows = (int64_t)a.B * a.Hkv * a.S;
+  if (streamed) {
+    const int tile = stream_tile(a, lim);
+    if (2 * rows >= stream_tiles(a, tile) * tile) return false;
+  }
   return rows * a.NW <= (a.k_cache ? 256 : 176) * 1024 && a.NW <= 65536;      // (a grid's y)
 }
 
@@ -952,7 +1046,7 @@ int check_hash_rows(const HashRows& a) {
   if (a.v)
     SOCKET_REQUIRE(socket_aligned16(a.v) && a.v_sb % per16 == 0 && a.v_sh % per16 == 0 && a.v_ss % per16 == 0, SOCKET_ERR_ALIGN);
   // (tile + grid size stays an int)
-  SOCKET_REQUIRE((int64_t)a.B * a.Hkv * ((a.S + kStreamTile - 1) / kStreamTile) < (1LL << 30), SOCKET_ERR_SHAPE);
+  SOCKET_REQUIRE((int64_t)a.B * a.Hkv * ((a.S + kStreamTile / 2 - 1) / (kStreamTile / 2)) < (1LL << 30), SOCKET_ERR_SHAPE);
   return SOCKET_OK;
 }
 
@@ -973,8 +1067,8 @@ extern "C" int socket_hash_keys(const void* k, const void* v, int dtype, int64_t
   if (st != SOCKET_OK) return st;
   const SocketDeviceLimits& lim = socket_device_limits();
   const bool streamed = streams(a, lim);
-  if (goes_direct(a, streamed)) return launch_direct(a, lim, nullptr, (hipStream_t)stream);
-  return streamed ? launch_stream<kD, false>(a, lim, (hipStream_t)stream) : launch_staged(a, lim, (hipStream_t)stream);
+  if (goes_direct(a, lim, streamed)) return launch_direct(a, lim, nullptr, (hipStream_t)stream);
+  return streamed ? launch_stream<false>(a, lim, nullptr, (hipStream_t)stream) : launch_staged(a, lim, (hipStream_t)stream);
 }
 
 extern "C" int socket_hash_rows(const void* k, const void* v, int dtype, int64_t k_stride_b, int64_t k_stride_h,
@@ -989,9 +1083,9 @@ extern "C" int socket_hash_rows(const void* k, const void* v, int dtype, int64_t
   hipStream_t s = (hipStream_t)stream;
   const SocketDeviceLimits& lim = socket_device_limits();
   const bool streamed = streams(a, lim);
-  if (goes_direct(a, streamed)) return launch_direct(a, lim, nullptr, s);
+  if (goes_direct(a, lim, streamed)) return launch_direct(a, lim, nullptr, s);
   if (!streamed) return launch_staged(a, lim, s);
-  return D == 64 ? launch_stream<64, false>(a, lim, s) : launch_stream<128, false>(a, lim, s);
+  return launch_stream<false>(a, lim, nullptr, s);
 }
 
 extern "C" int socket_cache_append(const void* k, const void* v, int dtype, int64_t k_stride_b, int64_t k_stride_h,
@@ -1015,33 +1109,29 @@ extern "C" int socket_cache_append(const void* k, const void* v, int dtype, int6
   hipStream_t s = (hipStream_t)stream;
   const SocketDeviceLimits& lim = socket_device_limits();
   const bool streamed = streams(a, lim);
-  if (goes_direct(a, streamed)) return launch_direct(a, lim, lens, s);
-  // the rows' copy (all of it where the hash does not pass them on) and the lengths
-  if (!streamed || lens) {
-    const int64_t pieces = streamed ? 1 : (int64_t)S * (D / per16);
-    const dim3 grid((unsigned)((pieces + 256 * kCopyPieces - 1) / (256 * kCopyPieces)), (unsigned)(streamed ? 1 : B * Hkv));
+  if (goes_direct(a, lim, streamed)) return launch_direct(a, lim, lens, s);
+  if (streamed) return launch_stream<true>(a, lim, lens, s);
+  // the rows' copy and the lengths
+  const int64_t pieces = (int64_t)S * (D / per16);
+  const dim3 grid((unsigned)((pieces + 256 * kCopyPieces - 1) / (256 * kCopyPieces)), (unsigned)(B * Hkv));
 #define SOCKET_COPY(DT)                                                                                                    \
   hipLaunchKernelGGL((copy_rows_kernel<DT>), grid, dim3(256), 0, s, k, v, k_stride_b, k_stride_h, k_stride_s, v_stride_b,  \
                      v_stride_h, v_stride_s, k_cache, v_cache, cache_stride_b, cache_stride_h, cache_stride_s, lens, t0, B, \
-                     Hkv, S, D, streamed ? 0 : 1)
-    if (dtype == SOCKET_F32) SOCKET_COPY(DType_f32);
-    else SOCKET_COPY(DType_bf16);      // (16-bit rows are moved as they are)
+                     Hkv, S, D)
+  if (dtype == SOCKET_F32) SOCKET_COPY(DType_f32);
+  else SOCKET_COPY(DType_bf16);      // (16-bit rows are moved as they are)
 #undef SOCKET_COPY
-    SOCKET_LAUNCH_CHECK();
+  SOCKET_LAUNCH_CHECK();
+  // Rows past what the caches of the chip hold are read back from where the copy has put them, whole heads in order,
+  // rather than a token apart; fewer are nearer where they came from.  float32, 128 dims, 60 x 10 planes, the whole
+  // append, caller's rows / cache: 8 x 2500 rows (20 MB) 31.3 / 32.5 us, 8 x 10000 62.7 / 61.9, 8 x 24000 147 / 142,
+  // 8 x 60000 382 / 358.
+  if ((int64_t)B * Hkv * S * D * (16 / per16) * 2 > (128ll << 20)) {
+    const int64_t first = (int64_t)t0 * cache_stride_s * (16 / per16);
+    a.k = (const char*)k_cache + first, a.v = (const char*)v_cache + first;
+    a.k_sb = a.v_sb = cache_stride_b, a.k_sh = a.v_sh = cache_stride_h, a.k_ss = a.v_ss = cache_stride_s;
   }
-  if (!streamed) {
-    // Rows past what the caches of the chip hold are read back from where the copy has put them, whole heads in order,
-    // rather than a token apart; fewer are nearer where they came from.  float32, 128 dims, 60 x 10 planes, the whole
-    // append, caller's rows / cache: 8 x 2500 rows (20 MB) 31.3 / 32.5 us, 8 x 10000 62.7 / 61.9, 8 x 24000 147 / 142,
-    // 8 x 60000 382 / 358.
-    if ((int64_t)B * Hkv * S * D * (16 / per16) * 2 > (128ll << 20)) {
-      const int64_t first = (int64_t)t0 * cache_stride_s * (16 / per16);
-      a.k = (const char*)k_cache + first, a.v = (const char*)v_cache + first;
-      a.k_sb = a.v_sb = cache_stride_b, a.k_sh = a.v_sh = cache_stride_h, a.k_ss = a.v_ss = cache_stride_s;
-    }
-    return launch_staged(a, lim, s);
-  }
-  return D == 64 ? launch_stream<64, true>(a, lim, s) : launch_stream<128, true>(a, lim, s);
+  return launch_staged(a, lim, s);
 }
 
 extern "C" int socket_unpack_codes(const uint32_t* codes, int16_t* out, int B, int Hkv, int L, int P,
