@@ -263,14 +263,17 @@ def dtype_enum(dt: torch.dtype) -> int:
         raise RuntimeError(f"unsupported dtype {dt}: expected float32, bfloat16 or float16") from None
 
 
-def ptr(t) -> c_void_p:
-    return c_void_p(0 if t is None else t.data_ptr())
+def ptr(t):
+    """A tensor's address (None: NULL) as the entry points' pointer arguments take it."""
+    return None if t is None else t.data_ptr()
 
 
-def stream_ptr(device=None) -> c_void_p:
+def stream_ptr(device=None):
     """The HIP stream torch is currently issuing work on, as the reference's
-    kernels (Triton and load_inline launches) do."""
-    return c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    kernels (Triton and load_inline launches) do.  (Its handle straight from torch's binding: a
+    Stream object costs 2 us a call, a launch some 4.)"""
+    index = None if device is None else device.index
+    return _C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def require_device(*tensors) -> None:
@@ -299,13 +302,15 @@ def one_device(tensors) -> bool:
     return True
 
 
-def plain_tensors(*tensors) -> bool:
+def plain_tensors(*tensors, grad=None) -> bool:
     """True for tensors of one HIP device that nothing differentiates, transforms or traces, which a kernel may
     therefore read and write by address in place of torch operations.  (Asked before any of their attributes:
-    a tracer's stand-in for a tensor is no plain one.)"""
+    a tracer's stand-in for a tensor is no plain one.)  `grad`: whether the operations would be differentiated, by
+    default whether gradients are enabled."""
     if observed():
         return False
-    grad = torch.is_grad_enabled()
+    if grad is None:
+        grad = torch.is_grad_enabled()
     for t in tensors:
         if type(t) not in _PLAIN or not t.is_cuda or (grad and t.requires_grad):
             return False

@@ -481,7 +481,6 @@ class SocketHashCache:
         assert tuple(planes_lpd.shape[:2]) == (self.L, self.P)
         self.planes_words = permute_planes(planes_lpd.to(self.k_cache.device))
 
-    @torch.no_grad()
     def append(self, pos0: int, k_bshd: torch.Tensor, v_bshd: torch.Tensor) -> None:
         """Write S new tokens at positions [pos0, pos0+S) for every sequence:
         K/V rows, packed codes and value norms (KVCache.update,
@@ -493,27 +492,36 @@ class SocketHashCache:
             raise RuntimeError(
                 f"KVCache.update out-of-bounds: positions [{pos0},{pos0 + S - 1}] but cache T={self.Tcap}")
         if self._append_fits(k_bshd, v_bshd):
-            kc = self.k_cache
+            kc, ks, vs = self.k_cache, k_bshd.stride(), v_bshd.stride()
+            cs = kc.stride()
             check("socket_cache_append", lib().socket_cache_append(
-                ptr(k_bshd), ptr(v_bshd), dtype_enum(kc.dtype), k_bshd.stride(0), k_bshd.stride(2), k_bshd.stride(1),
-                v_bshd.stride(0), v_bshd.stride(2), v_bshd.stride(1), ptr(self.planes_words), ptr(kc), ptr(self.v_cache),
-                kc.stride(0), kc.stride(1), kc.stride(2), ptr(self.codes), ptr(self.v_norm), ptr(self.lens), int(pos0), B, H, S, D,
-                self.L, self.P, self.Tcap, stream_ptr(kc.device)))
+                k_bshd.data_ptr(), v_bshd.data_ptr(), dtype_enum(kc.dtype), ks[0], ks[2], ks[1], vs[0], vs[2], vs[1],
+                self.planes_words.data_ptr(), kc.data_ptr(), self.v_cache.data_ptr(), cs[0], cs[1], cs[2], self.codes.data_ptr(),
+                self.v_norm.data_ptr(), self.lens.data_ptr(), int(pos0), B, H, S, D, self.L, self.P, self.Tcap,
+                stream_ptr(kc.device)))
             return
-        self.k_cache[:, :, pos0:pos0 + S].copy_(k_bshd.permute(0, 2, 1, 3))
-        self.v_cache[:, :, pos0:pos0 + S].copy_(v_bshd.permute(0, 2, 1, 3))
-        hash_keys_into(self.k_cache[:, :, pos0:pos0 + S], self.v_cache[:, :, pos0:pos0 + S],
-                       self.planes_words, self.codes, self.v_norm, self.L, self.P, t0=pos0)
-        self.lens.fill_(pos0 + S)      # the cached length follows the position
+        with torch.no_grad():
+            self.k_cache[:, :, pos0:pos0 + S].copy_(k_bshd.permute(0, 2, 1, 3))
+            self.v_cache[:, :, pos0:pos0 + S].copy_(v_bshd.permute(0, 2, 1, 3))
+            hash_keys_into(self.k_cache[:, :, pos0:pos0 + S], self.v_cache[:, :, pos0:pos0 + S],
+                           self.planes_words, self.codes, self.v_norm, self.L, self.P, t0=pos0)
+            self.lens.fill_(pos0 + S)      # the cached length follows the position
 
     def _append_fits(self, k: torch.Tensor, v: torch.Tensor) -> bool:
         """Whether one call of the library copies and hashes these rows (else: torch's copies, then the hash)."""
-        kc, per = self.k_cache, 16 // self.k_cache.element_size()
-        own = (kc, self.v_cache, self.codes, self.v_norm, self.lens, self.planes_words)
-        return (plain_tensors(k, v, *own) and k.dtype == v.dtype == kc.dtype == self.v_cache.dtype
-                and kc.dtype in (torch.bfloat16, torch.float16, torch.float32)
-                and k.shape == v.shape and tuple(k.shape[2:]) == (kc.shape[1], kc.shape[3]) and k.shape[1] > 0
-                and k.shape[3] % 8 == 0 and k.shape[3] <= HASH_DIM and self.planes_words.shape[1] == HASH_DIM and kc.shape[0] * kc.shape[1] <= 65535
-                and all(t.is_contiguous() for t in own) and k.stride(3) == v.stride(3) == 1
-                and all(st % per == 0 for st in k.stride()[:3] + v.stride()[:3])
-                and all(t.data_ptr() % 16 == 0 for t in (k, v, kc, self.v_cache)))
+        kc, vc, codes, norms, lens, words = self.k_cache, self.v_cache, self.codes, self.v_norm, self.lens, self.planes_words
+        # (an append is never differentiated)
+        if not plain_tensors(k, v, kc, vc, codes, norms, lens, words, grad=False):
+            return False
+        dt, shape = kc.dtype, k.shape
+        if not (k.dtype == v.dtype == dt == vc.dtype and dt in (torch.bfloat16, torch.float16, torch.float32) and shape == v.shape):
+            return False
+        B, S, H, D = shape
+        cb, ch, _, cd = kc.shape
+        if not (H == ch and D == cd and S > 0 and D % 8 == 0 and D <= HASH_DIM and words.shape[1] == HASH_DIM and cb * ch <= 65535
+                and kc.is_contiguous() and vc.is_contiguous() and codes.is_contiguous() and norms.is_contiguous()
+                and lens.is_contiguous() and words.is_contiguous()):
+            return False
+        ks, vs = k.stride(), v.stride()
+        return (ks[3] == vs[3] == 1 and (ks[0] | ks[1] | ks[2] | vs[0] | vs[1] | vs[2]) % (16 // kc.element_size()) == 0
+                and (k.data_ptr() | v.data_ptr() | kc.data_ptr() | vc.data_ptr()) % 16 == 0)

@@ -106,7 +106,6 @@ def sparse_decode_stage2(
         B, H, D, mid_out.shape[2], int(block_seq), stream_ptr(out.device)))
 
 
-@torch.no_grad()
 def sparse_attention_fwd(
     query: torch.Tensor,        # [B,H,D]
     key: torch.Tensor,          # [B,Kv,S,D]
@@ -135,14 +134,13 @@ def sparse_attention_fwd(
     L = lib()
     nbytes = L.socket_sparse_attention_workspace_bytes(B, H, D, width)
     ws = torch.empty(nbytes // 4, dtype=torch.float32, device=query.device)
+    ks, vs = key.stride(), value.stride()
     check("socket_sparse_attention", L.socket_sparse_attention(
         ptr(query), ptr(key), ptr(value), dtype_enum(query.dtype),
-        query.stride(0), query.stride(1),
-        key.stride(0), key.stride(1), key.stride(2),
-        value.stride(0), value.stride(1), value.stride(2),
+        query.stride(0), query.stride(1), ks[0], ks[1], ks[2], vs[0], vs[1], vs[2],
         ptr(sparse_list), sparse_list.stride(0), sparse_list.stride(1),
         ptr(sparse_len), sparse_len.stride(0), sparse_len.stride(1),
-        ptr(out), out.stride(0), out.stride(1),
+        ptr(out), H * D, D,
         ptr(ws), nbytes,
         B, H, key.shape[1], D, key.shape[2], width, stream_ptr(query.device)))
     return out

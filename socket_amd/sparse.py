@@ -67,7 +67,7 @@ def _select_workspace(device: torch.device, nbytes: int, zero_bytes: int) -> tor
             return _new_workspace(device, nbytes, zero_bytes)
         _SELECT_WS.move_to_end(graph_key)
         return ws[0]
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream, nbytes)
+    key = (device.index, stream_ptr(device), nbytes)
     for k in (key, graph_key):
         if k not in _SELECT_WS:
             _SELECT_WS[k] = (_new_workspace(device, nbytes, zero_bytes), zero_bytes)
@@ -167,7 +167,6 @@ def _build_in_place(q_probs, k_hard, v_norm, allowed, sink: int, window: int, M:
     return sparse_list, sparse_len
 
 
-@torch.no_grad()
 def build_sparse_list_decode(
     q_probs: torch.Tensor,       # [B,H,L,R] fp16/bf16/fp32
     k_hard_bhlt: torch.Tensor,   # [B,H,L,T] int16/int32
@@ -186,15 +185,22 @@ def build_sparse_list_decode(
     assert q_probs.is_cuda and k_hard_bhlt.is_cuda and v_norm_bht.is_cuda and allowed_bht.is_cuda
     assert q_probs.dtype in (torch.float16, torch.bfloat16, torch.float32)
     assert allowed_bht.dtype == torch.bool
-    B, H, L, R = q_probs.shape
+    _, _, L, _ = q_probs.shape
     _, _, L2, T = k_hard_bhlt.shape
     assert L2 == L
-    device = q_probs.device
     M_eff = min(M, T)
     built = _build_in_place(q_probs, k_hard_bhlt if k_hard_bhlt.dtype == torch.int16 else k_hard_bhlt.to(torch.int16),
                             v_norm_bht, allowed_bht, int(sink), int(window), int(M_eff))
     if built is not None:
         return built
+    with torch.no_grad():
+        return _build_with_torch(q_probs, k_hard_bhlt, v_norm_bht, allowed_bht, sink, window, M_eff)
+
+
+def _build_with_torch(q_probs, k_hard_bhlt, v_norm_bht, allowed_bht, sink: int, window: int, M_eff: int):
+    """The same with torch's operations around the scorer and the top-k, for operands `_build_in_place` does not take."""
+    B, H = q_probs.shape[:2]
+    T, device = k_hard_bhlt.shape[3], q_probs.device
     if M_eff > 0:
         ext = _get_soft_hash_ext()
         q_probs_f32 = q_probs.float().unsqueeze(2).contiguous()

@@ -43,3 +43,22 @@ def test_streamed_append_equals_small_ones(B, S, H, D, L, P, pos0, dt):
     norms = torch.zeros_like(whole.v_norm)
     hash_cache.hash_keys_into(whole.k_cache[:, :, pos0:pos0 + S], None, whole.planes_words, codes, norms, L, P, t0=pos0)
     assert torch.equal(codes, whole.codes) and not norms.any()
+
+
+def test_launches_follow_the_current_stream():
+    """The handle the launches are given is that of torch's current stream, by tensor device, by bare device and by default;
+    rows that require gradients are appended like any others."""
+    from socket_amd._lib import stream_ptr
+    side = torch.cuda.Stream()
+    for s in (torch.cuda.current_stream(), side):
+        with torch.cuda.stream(s):
+            for d in (torch.zeros(1, device=DEV).device, torch.device(DEV), None):
+                assert (stream_ptr(d) or 0) == s.cuda_stream
+    k, v = (torch.randn(2, 9, 3, 64, device=DEV) for _ in range(2))
+    caches = [hash_cache.SocketHashCache(2, 16, 3, 64, 12, 4, dtype=torch.float32, device=DEV) for _ in range(2)]
+    planes = torch.randn(12, 4, 64, device=DEV)
+    for cache, grad in zip(caches, (False, True)):
+        cache.set_planes(planes)
+        cache.append(2, k.clone().requires_grad_(grad), v)
+    for name in ("k_cache", "v_cache", "codes", "v_norm", "lens"):
+        assert torch.equal(getattr(caches[0], name), getattr(caches[1], name)) and not getattr(caches[1], name).requires_grad
