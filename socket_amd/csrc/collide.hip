@@ -11,19 +11,24 @@
 // This layout costs 2 L + 9 bytes of HBM per (head, token) -- eight times the
 // packed per-kv-head cache of score.hip at G = 4 -- and the launch is bound by
 // that stream if the tables stay out of its way.  A workgroup therefore keeps a
-// tile of THREADS x 8 tokens of one (b, h) row and walks the tables in LDS-sized
-// slices (two slices of 30 fp32 tables at L60 x R1024; one slice for fp16), and
+// tile of tokens of one (b, h) row and walks the tables in LDS-sized
+// slices (two slices of 30 fp32 tables at L60 x R1024; one slice for fp16), copied
+// straight from memory into LDS while the first codes are on their way, and
 // serves several such tiles under each slice; a thread fetches the codes of its
 // eight consecutive tokens with one 16-byte load per table (wherever the row
-// starts), six tables ahead of their use, and gathers without branches.
+// starts), six tables ahead of their use, and gathers without branches.  Short rows
+// are dealt out two or four tokens to a thread.
 #include <atomic>
 
 #include "socket_common.h"
 
 namespace {
 
+// Consecutive tokens of a thread: eight where rows are long, four or two where a row's tokens have to be dealt out wide to
+// occupy the chip.
 constexpr int kTokensPerThread = 8;
-constexpr int kAhead = 6;   // tables whose codes are in flight per lane
+// tables whose codes are in flight per lane: 96 bytes of them either way
+constexpr int ahead(int tpt) { return 48 / tpt; }
 constexpr size_t kCollideLdsSlack = 1024;
 
 struct Bf16Entry {
@@ -45,54 +50,88 @@ __device__ __forceinline__ float norm_at(const void* v, int dtype, int64_t i) {
 // lines instead of eight.  (32 rows, L60 x R1024, us against a code at a time: fp32 tables at 2051 / 4135 / 9003 / 20881 / 32771
 // tokens 26 / 32 / 31 / 33 / 50 against 71 / 80 / 79 / 101 / 168, bf16 24 / 29 / 26 / 28 / 41 against 60 / 69 / 68 / 88 / 147;
 // rows on 16-byte boundaries are as fast as before.)
-typedef uint32_t codes8 __attribute__((ext_vector_type(4), aligned(2)));     // eight 16-bit codes or norms
-typedef uint32_t bytes8 __attribute__((ext_vector_type(2), aligned(1)));     // eight mask bytes
-typedef float floats4 __attribute__((ext_vector_type(4), aligned(4)));
+template <int TPT>
+struct Vectors;
+template <>
+struct Vectors<8> {
+  typedef uint32_t codes __attribute__((ext_vector_type(4), aligned(2)));      // 16-bit codes or norms
+  typedef uint32_t bytes __attribute__((ext_vector_type(2), aligned(1)));      // mask bytes
+  typedef float floats __attribute__((ext_vector_type(4), aligned(4)));
+  static __device__ __forceinline__ uint32_t word(const codes& c, int i) { return c[i]; }
+  static __device__ __forceinline__ uint32_t mask(const bytes& b, int i) { return (i < 4 ? b.x : b.y) >> (8 * (i & 3)); }
+};
+template <>
+struct Vectors<4> {
+  typedef uint32_t codes __attribute__((ext_vector_type(2), aligned(2)));
+  typedef uint32_t bytes __attribute__((aligned(1)));
+  typedef float floats __attribute__((ext_vector_type(4), aligned(4)));
+  static __device__ __forceinline__ uint32_t word(const codes& c, int i) { return c[i]; }
+  static __device__ __forceinline__ uint32_t mask(bytes b, int i) { return b >> (8 * i); }
+};
+template <>
+struct Vectors<2> {
+  typedef uint32_t codes __attribute__((aligned(2)));
+  typedef uint16_t bytes __attribute__((aligned(1)));
+  typedef float floats __attribute__((ext_vector_type(2), aligned(4)));
+  static __device__ __forceinline__ uint32_t word(codes c, int) { return c; }
+  static __device__ __forceinline__ uint32_t mask(bytes b, int i) { return (uint32_t)b >> (8 * i); }
+};
 
 // ct: tables per LDS slice.  INLDS false: a single table exceeds LDS, gather from global memory.
-// A workgroup serves `chunks` consecutive tiles of THREADS x 8 tokens under every
+// A workgroup serves `chunks` consecutive tiles of `tile` <= THREADS x TPT tokens under every
 // slice it brings into LDS; with more than one slice the running sums of a tile
 // wait in `out` between slices (each thread re-reads what it wrote itself), which
 // costs 8 bytes per token and slice against the 2 L + 9 of the stream and keeps
 // the order of the fp32 adds.
-// The thread at a row's end whose eight tokens would run past it takes the row's last eight (its loads stay inside the row)
+// The thread at a row's end whose tokens would run past it takes the row's last TPT (its loads stay inside the row)
 // and leaves those that its neighbour owns alone: it neither stores their sums nor their scores.
 // WIDE false: rows of fewer than eight tokens, element by element.
 // STREAM: the codes are loaded with the streaming hint (a code array too large to
 // stay in the memory-side cache from one call to the next; WIDE only).
-template <typename QT, int THREADS, bool WIDE, bool INLDS, bool STREAM>
+template <typename QT, int THREADS, int TPT, bool WIDE, bool INLDS, bool STREAM>
 __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
     const QT* __restrict__ q_probs, const int16_t* __restrict__ key_buckets,
     const uint8_t* __restrict__ allowed, const void* __restrict__ v_hist, int v_dtype, float* __restrict__ out,
-    int L, int R, int T, int ct, int chunks) {
+    int rows, int L, int R, int T, int tile, int ct, int chunks) {
   extern __shared__ __attribute__((aligned(16))) unsigned char collide_lds[];
   QT* table = reinterpret_cast<QT*>(collide_lds);
-  constexpr int TPT = kTokensPerThread;
-  const int bh = blockIdx.y;
+  typedef Vectors<TPT> V;
+  typedef typename V::codes codes_t;
+  typedef typename V::floats floats_t;
+  constexpr int F = sizeof(floats_t) / sizeof(float);
+  // row r is workgroups r, r + rows, ...: on one XCD, or few, whose L2 then fetches its table once for all its tiles
+  // (with the tiles of a row next to each other every XCD fetched every table: 32 rows, L60 x R1024, fp32, 32768 tokens
+  // 42.6 us against 38.5, 1000 tokens 20.9 against 13.8, both with the copy into LDS, which is the smaller part)
+  const int bh = blockIdx.x % rows, part = blockIdx.x / rows;
   const QT* qp = q_probs + (int64_t)bh * L * R;
   const int16_t* kb = key_buckets + (int64_t)bh * L * T;
 
-  // the codes of tokens t0 .. t0 + 7 for table l, as loaded (two per word; WIDE: all eight exist; else -1 where no token is)
-  auto codes_of = [&](int l, int t0) -> codes8 {
+  // the codes of a thread's tokens from t0 on for table l, as loaded (two per word; WIDE: all of them exist; else -1 where no
+  // token is)
+  auto codes_of = [&](int l, int t0) -> codes_t {
     const int16_t* row = kb + (int64_t)l * T + t0;
-    if (WIDE && !STREAM) return *reinterpret_cast<const codes8*>(row);
-    if (WIDE) return __builtin_nontemporal_load(reinterpret_cast<const codes8*>(row));
-    codes8 u;
+    if (WIDE && !STREAM) return *reinterpret_cast<const codes_t*>(row);
+    if (WIDE) return __builtin_nontemporal_load(reinterpret_cast<const codes_t*>(row));
+    uint32_t u[TPT / 2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < TPT / 2; ++i) {
       const uint32_t lo = (t0 + 2 * i < T) ? (uint16_t)row[2 * i] : 0xffffu;
       const uint32_t hi = (t0 + 2 * i + 1 < T) ? (uint16_t)row[2 * i + 1] : 0xffffu;
       u[i] = lo | (hi << 16);
     }
-    return u;
+    codes_t c;
+    __builtin_memcpy(&c, u, sizeof(c));
+    return c;
   };
-  // `skip`: how many of the eight belong to the thread before (only ever above zero at a row's end)
+  // `skip`: how many of the tokens belong to the thread before (only ever above zero at a row's end)
   auto load_partial = [&](int64_t o, int t0, int skip, float (&sum)[TPT]) {
     if (WIDE && skip == 0) {
-      const floats4 a = *reinterpret_cast<const floats4*>(out + o);
-      const floats4 b = *reinterpret_cast<const floats4*>(out + o + 4);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sum[i] = a[i], sum[4 + i] = b[i];
+      for (int v = 0; v < TPT; v += F) {
+        const floats_t a = *reinterpret_cast<const floats_t*>(out + o + v);
+#pragma unroll
+        for (int i = 0; i < F; ++i) sum[v + i] = a[i];
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < TPT; ++i) sum[i] = (i >= skip && t0 + i < T) ? out[o + i] : 0.f;
@@ -100,11 +139,13 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
   };
   auto store_row = [&](int64_t o, int t0, int skip, const float (&x)[TPT]) {
     if (WIDE && skip == 0) {
-      floats4 a, b;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = x[i], b[i] = x[4 + i];
-      *reinterpret_cast<floats4*>(out + o) = a;
-      *reinterpret_cast<floats4*>(out + o + 4) = b;
+      for (int v = 0; v < TPT; v += F) {
+        floats_t a;
+#pragma unroll
+        for (int i = 0; i < F; ++i) a[i] = x[v + i];
+        *reinterpret_cast<floats_t*>(out + o + v) = a;
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < TPT; ++i)
@@ -114,22 +155,25 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
   auto finish = [&](int64_t o, int t0, int skip, const float (&sum)[TPT]) {
     float res[TPT];
     if (WIDE) {
-      const bytes8 aw = *reinterpret_cast<const bytes8*>(allowed + o);
+      const typename V::bytes ok = *reinterpret_cast<const typename V::bytes*>(allowed + o);
       float vh[TPT];
       if (v_dtype == SOCKET_F32) {      // (uniform)
-        const floats4 v0 = *reinterpret_cast<const floats4*>((const float*)v_hist + o);
-        const floats4 v1 = *reinterpret_cast<const floats4*>((const float*)v_hist + o + 4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) vh[i] = v0[i], vh[4 + i] = v1[i];
+        for (int v = 0; v < TPT; v += F) {
+          const floats_t a = *reinterpret_cast<const floats_t*>((const float*)v_hist + o + v);
+#pragma unroll
+          for (int i = 0; i < F; ++i) vh[v + i] = a[i];
+        }
       } else {
-        const codes8 c = *reinterpret_cast<const codes8*>((const uint16_t*)v_hist + o);
-        const uint4 w = make_uint4(c.x, c.y, c.z, c.w);
-        if (v_dtype == SOCKET_F16) unpack16<DType_f16>(w, vh);
-        else unpack16<DType_bf16>(w, vh);
+        const codes_t c = *reinterpret_cast<const codes_t*>((const uint16_t*)v_hist + o);
+#pragma unroll
+        for (int i = 0; i < TPT; ++i) {
+          const uint16_t bits = (uint16_t)(V::word(c, i >> 1) >> (16 * (i & 1)));
+          vh[i] = v_dtype == SOCKET_F16 ? f16_bits_to_f32(bits) : bf16_bits_to_f32(bits);
+        }
       }
 #pragma unroll
-      for (int i = 0; i < TPT; ++i)
-        res[i] = (((i < 4 ? aw.x : aw.y) >> (8 * (i & 3))) & 0xffu) ? sum[i] * vh[i] : -INFINITY;
+      for (int i = 0; i < TPT; ++i) res[i] = (V::mask(ok, i) & 0xffu) ? sum[i] * vh[i] : -INFINITY;
     } else {
 #pragma unroll
       for (int i = 0; i < TPT; ++i)
@@ -138,26 +182,44 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
     store_row(o, t0, skip, res);
   };
 
+  constexpr int kAhead = ahead(TPT);
+  codes_t ring[kAhead];
+  auto fill_ring = [&](int l0, int nt, int t0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a) ring[a] = codes_of(l0 + min(a, nt - 1), t0);
+  };
+  struct Where {
+    int own, t0;      // the thread's first token of a tile, and where its loads start; own < 0: it has none
+  };
+  auto where = [&](int c) __attribute__((always_inline)) {
+    const int first = (part * chunks + c) * tile, own = first + (int)threadIdx.x * TPT;
+    if (own >= min(first + tile, T)) return Where{-1, 0};
+    return Where{own, WIDE ? min(own, T - TPT) : own};
+  };
   const int step = INLDS ? ct : L;   // (without LDS: one pass over all tables)
   for (int l0 = 0; l0 < L; l0 += step) {
     const int nt = min(step, L - l0);
+    const Where w0 = where(0);
+    if (w0.own >= 0) fill_ring(l0, nt, w0.t0);     // (on their way while the slice comes)
     if (INLDS) {
       __syncthreads();   // the previous slice has been consumed
-      // 16 bytes per lane where the slice starts and ends on 16-byte boundaries
-      const int n16 = nt * R * (int)sizeof(QT) / 16;
-      const uint4* src = reinterpret_cast<const uint4*>(qp + (int64_t)l0 * R);
-      uint4* dst = reinterpret_cast<uint4*>(table);
-      if (((uintptr_t)src & 15) == 0 && (nt * R * (int)sizeof(QT)) % 16 == 0) {
-        for (int i = threadIdx.x; i < n16; i += THREADS) dst[i] = src[i];
+      const int bytes = nt * R * (int)sizeof(QT);
+      const char* src = reinterpret_cast<const char*>(qp + (int64_t)l0 * R);
+      if (((uintptr_t)src & 15) == 0 && bytes % 16 == 0) {
+        // straight into LDS, all of it under way at once (through registers every 16 KB were a trip to memory)
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+        for (int o = wave * 1024; o < bytes; o += THREADS * 16)
+          if (o + lane * 16 < bytes) lds_dma16(src + o + lane * 16, collide_lds + o);
+        wait_vmcnt(0);
       } else {
         for (int i = threadIdx.x; i < nt * R; i += THREADS) table[i] = qp[(int64_t)l0 * R + i];
       }
       __syncthreads();
     }
     for (int c = 0; c < chunks; ++c) {
-      const int own = ((blockIdx.x * chunks + c) * THREADS + threadIdx.x) * TPT;
-      if (own >= T) continue;
-      const int t0 = WIDE ? min(own, T - TPT) : own, skip = own - t0;
+      const Where at = c ? where(c) : w0;
+      if (at.own < 0) continue;
+      const int t0 = at.t0, skip = at.own - t0;
       const int64_t o = (int64_t)bh * T + t0;
       float sum[TPT];
       if (l0 == 0) {
@@ -170,22 +232,20 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
       // would leave the stream waiting on latency): slot a always holds table lb + a;
       // the loop is unrolled by the ring's depth, so a slot is a fixed set of registers
       // and the wait before its use counts exactly the loads behind it.
-      codes8 ring[kAhead];
-#pragma unroll
-      for (int a = 0; a < kAhead; ++a) ring[a] = codes_of(l0 + min(a, nt - 1), t0);
+      if (c) fill_ring(l0, nt, t0);
       for (int lb = 0; lb < nt; lb += kAhead) {
 #pragma unroll
         for (int a = 0; a < kAhead; ++a) {
           const int l = lb + a;
           if (l >= nt) break;
-          const codes8 cur = ring[a];
+          const codes_t cur = ring[a];
           ring[a] = codes_of(l0 + min(l + kAhead, nt - 1), t0);   // (past the slice: its last table again, unused)
           // branch-free: a stray code reads entry 0 and adds +0.0 instead (x + 0.0 == x;
           // the sums start at +0.0, so no -0.0 can be lost), and the LDS variant has no
           // global load in here for the compiler to wait on with the ring in flight
 #pragma unroll
           for (int i = 0; i < TPT; ++i) {
-            const int r = (int)(int16_t)((i & 1) ? (cur[i >> 1] >> 16) : (cur[i >> 1] & 0xffffu));
+            const int r = (int)(int16_t)((i & 1) ? (V::word(cur, i >> 1) >> 16) : (V::word(cur, i >> 1) & 0xffffu));
             const bool hit = r >= 0 && r < R;
             const int rr = hit ? r : 0;
             const float e = entry_to_f32(INLDS ? table[l * R + rr] : qp[(int64_t)(l0 + l) * R + rr]);
@@ -213,36 +273,38 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
     ct = (L + slices - 1) / slices;
   }
   const size_t lds = (size_t)ct * per_table;
-  const bool wide = T >= kTokensPerThread;
-  // Lanes of a workgroup.  It pulls its row's whole table through LDS with them, which is quicker the more there are, and
-  // the chip has at most CUs x (tables that fit a CU's LDS) workgroups at work.  While all workgroups are at work at
-  // once narrower ones leave fewer CUs idle; past that each further round costs what the first did, and 1024 lanes need
-  // the fewest.  us at 256 / 512 / 1024 lanes:
-  //   32 rows, L60 x R1024 fp32    4088: 32 / 24 / 23     8192: 34 / 29 / 36     32768: 66 / 35 / 40    48000: 99 / 61 / 44
-  //   the same, bf16               4088: 23 / 22 / 22     5000: 25 / 25 / 27     32768: 51 / 28 / 36    65536: 93 / 58 / 50
-  //   32 rows, L32 x R256 fp32     4088: 11 / 12 / 12    12000: 13 / 13 / 18     24000: 16 / 15 / 19
-  // Just past 4096 tokens 512 lanes make a second, nearly empty workgroup of what 1024 hold in one.  A table in one
-  // slice (bf16) and few workgroups: 28 rows, L48, 5000 tokens 18.6 / 20.3 us at 256 / 512 lanes; 8 rows, L60, 16384: 21 / 23.
-  auto tiles_of = [&](int th) { return (T + th * kTokensPerThread - 1) / (th * kTokensPerThread); };
-  auto fit = [&](int th, int workgroups) { return (int64_t)tiles_of(th) * B * H <= workgroups; };
-  const bool shares = 2 * lds <= budget;      // a CU holds several workgroups' tables
   const int cus = lim.cu_count;
+  const bool wide = T >= kTokensPerThread;
+  // Rows short enough that two (or four) tokens to a lane hold them in one round of workgroups, each row in as many equal
+  // tiles as there are CUs for it: with eight to a lane most waves would have no token and the rest a long chain of lookups.
+  // 32 rows, L60 x R1024, us at two to a lane / at eight: fp32 1000 tokens 13.8 / 25, 4135 16.5 / 30, 16384 23.2 / 33.6; bf16
+  // 12.0 / 22, 13.4 / 27, 19.4 / 29; 56 rows, L48, fp32 6001 18.3 / 26; 28 rows, L32 x R256, fp32 4135 8.6 / 13.2, 16384 12.9 /
+  // 15.  Four to a lane pay while a quarter of the lanes is spare (32 rows, 20000 tokens: fp32 32.0 / 35.7, bf16 27.6 / 30.8)
+  // and not with every lane in use (32768 bf16 33.8 / 32.8; 64 rows, L32 x R256, 16384: 20.6 / 19.1).
+  const int64_t per_row = cus / ((int64_t)B * H);
+  const int few = !wide || ct == 0 ? 0 : per_row * 1024 * 2 >= T ? 2 : per_row * 1024 * 3 >= T ? 4 : 0;
+  // Lanes of a workgroup of eight tokens each.  It pulls its row's whole table through LDS with them, which is quicker the
+  // more there are, but while all workgroups are at work at once narrower ones leave fewer CUs idle (us at 512 / 1024 lanes,
+  // 32 rows, L60 x R1024: fp32 32768 tokens 35 / 40, 48000 61 / 44; bf16 32768 28 / 36, 65536 58 / 50).
+  auto tiles_of = [&](int th) { return (T + th * kTokensPerThread - 1) / (th * kTokensPerThread); };
   int threads = 1024;
-  if (T <= 256 * kTokensPerThread || (shares && fit(256, cus))) threads = 256;
-  else if (ct >= L && T > 4096 && fit(256, cus * 3 / 8)) threads = 256;
-  else if (T > 4608 && fit(512, cus)) threads = 512;
-  const int tiles = tiles_of(threads);
+  if (T <= 256 * kTokensPerThread) threads = 256;
+  else if (T > 4608 && (int64_t)tiles_of(512) * B * H <= cus) threads = 512;
+  const int tile = few ? (int)((T + per_row - 1) / per_row + 127) / 128 * 128 : threads * kTokensPerThread;
+  const int tiles = (T + tile - 1) / tile;
   // tiles per workgroup: as many as leave two workgroups per CU (they amortise the
   // slices a workgroup pulls through LDS), at most 8
   int chunks = (int)((int64_t)tiles * B * H / (2 * (int64_t)lim.cu_count));
-  chunks = chunks < 1 ? 1 : chunks > 8 ? 8 : chunks;
+  chunks = chunks < 1 || few ? 1 : chunks > 8 ? 8 : chunks;
   if (chunks > tiles) chunks = tiles;
-  dim3 grid((tiles + chunks - 1) / chunks, B * H);
+  const int64_t n_wg = (int64_t)((tiles + chunks - 1) / chunks) * B * H;
+  SOCKET_REQUIRE(n_wg < (1LL << 31), SOCKET_ERR_SHAPE);
+  dim3 grid((unsigned)n_wg);
   // (measured: 2 GB of codes gain 10 % from the hint, 135 MB that the cache still holds from the last call lose 7 %)
   const bool stream_codes = (int64_t)B * H * L * T * (int64_t)sizeof(int16_t) > (192ll << 20);
-#define SOCKET_COLLIDE(TH, V, LD, ST)                                                                     \
+#define SOCKET_COLLIDE(TH, N, V, LD, ST)                                                                     \
   do {                                                                                                \
-    auto kern = collision_i16_kernel<QT, TH, V, LD, ST>;                                                 \
+    auto kern = collision_i16_kernel<QT, TH, N, V, LD, ST>;                                                 \
     if (lds > 64 * 1024) {                                                                            \
       static std::atomic<size_t> granted{0};                                                          \
       if (granted.load(std::memory_order_acquire) < lds) {                                            \
@@ -252,16 +314,21 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
         granted.store(budget, std::memory_order_release);                                             \
       }                                                                                               \
     }                                                                                                 \
-    hipLaunchKernelGGL(kern, grid, dim3(TH), lds, stream, q_probs, key_buckets, allowed, v_hist, v_dtype, out, L, R, T, ct, chunks); \
+    hipLaunchKernelGGL(kern, grid, dim3(TH), lds, stream, q_probs, key_buckets, allowed, v_hist, v_dtype, out, B * H, L, R, T, tile, ct, chunks); \
   } while (0)
-#define SOCKET_COLLIDE_W(TH, LD)                                   \
-  do {                                                             \
-    if (stream_codes) SOCKET_COLLIDE(TH, true, LD, true);          \
-    else SOCKET_COLLIDE(TH, true, LD, false);                      \
+#define SOCKET_COLLIDE_W(TH, LD)                                                      \
+  do {                                                                                \
+    if (stream_codes) SOCKET_COLLIDE(TH, kTokensPerThread, true, LD, true);           \
+    else SOCKET_COLLIDE(TH, kTokensPerThread, true, LD, false);                       \
   } while (0)
   if (!wide) {      // (fewer than eight tokens: one narrow workgroup a row)
-    if (ct > 0) SOCKET_COLLIDE(256, false, true, false);
-    else SOCKET_COLLIDE(256, false, false, false);
+    if (ct > 0) SOCKET_COLLIDE(256, kTokensPerThread, false, true, false);
+    else SOCKET_COLLIDE(256, kTokensPerThread, false, false, false);
+  } else if (few == 2) {
+    SOCKET_COLLIDE(1024, 2, true, true, false);
+  } else if (few == 4) {
+    if (stream_codes) SOCKET_COLLIDE(1024, 4, true, true, true);
+    else SOCKET_COLLIDE(1024, 4, true, true, false);
   } else if (ct > 0) {
     if (threads == 256) SOCKET_COLLIDE_W(256, true);
     else if (threads == 512) SOCKET_COLLIDE_W(512, true);

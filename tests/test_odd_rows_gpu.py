@@ -23,6 +23,10 @@ def _collide(q, codes, allowed, v, out):
     (2, 5, 60, 1024, 2051, torch.float32, torch.float16, 3),     # two table slices: sums wait in the output between them
     (1, 32, 60, 1024, 8195, torch.float32, torch.float32, 0),    # several tiles to a workgroup
     (2, 28, 48, 1024, 20881, torch.bfloat16, torch.float16, 5),  # codes loaded past the caches
+    (1, 32, 60, 1024, 16383, torch.bfloat16, torch.float16, 1),  # two tokens to a lane, one short of every lane's two
+    (1, 32, 7, 1024, 16385, torch.float32, torch.bfloat16, 0),   # ... one more: four to a lane
+    (1, 32, 60, 1024, 24577, torch.float32, torch.float16, 1),   # ... and one past the last of those
+    (3, 7, 3, 16, 131, torch.bfloat16, torch.bfloat16, 0),       # a tile and three tokens
     (1, 2, 3, 65536, 4101, torch.float32, torch.float16, 0),     # a table that exceeds LDS
 ])
 def test_collision_scores_of_odd_rows(B, H, L, R, T, qt, vt, shift):
