@@ -233,6 +233,13 @@ int socket_soft_hash_collision_typed(const void* q_probs, int q_dtype, const int
  * (T - 1 if that is none), -1 wherever allowed [rows,T] is false; list_len [rows] becomes the row's width. */
 int socket_finish_list(int32_t* list, int32_t* list_len, const uint8_t* allowed, int rows, int T, int sink, int window,
                        int heavy, void* stream);
+/* socket_select_list over whole rows (no lens, budgets or ranges) with the sink and window part written, where `allowed`
+ * [B,Hq,T] (a byte each) says which positions may be listed: the others become -1 wherever the list has them.  Scores of
+ * positions that are not allowed are expected to be minus infinity.  The same list as socket_select_list without the base
+ * and socket_finish_list after it, in one launch. */
+int socket_select_list_allowed(const float* scores, int64_t score_stride, const uint8_t* allowed, int B, int Hq, int T, int M,
+                               int sink, int window, int32_t* sparse_list, int64_t list_stride, int list_width,
+                               int32_t* sparse_len, void* workspace, size_t workspace_bytes, void* stream);
 
 
 /* fp16 variant: q_probs f16 [B,H,L,R], v_norm f16 [B,H,T], any L.

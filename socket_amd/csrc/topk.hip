@@ -62,6 +62,9 @@ typedef unsigned long long u64;
 // 15.9 / 17.9).
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
+// The key of minus infinity, which scores of masked positions are.
+constexpr uint32_t kMaskedKey = 0x007fffffu;
+
 template <bool B>
 struct BoolTag {
   static constexpr bool value = B;
@@ -314,19 +317,27 @@ __device__ __forceinline__ void row_shape(const int32_t* lens, const int32_t* bu
   m = max(0, min(nbase + m, list_width) - nbase);
 }
 
+// What the list holds for a position.
+template <bool MASKED>
+__device__ __forceinline__ int32_t listed(int32_t at, const uint8_t* ok) {
+  if constexpr (MASKED) return at >= 0 && ok[at] ? at : -1;
+  else return at;
+}
+
 // Sink / window part of a list row, its length and the -1 padding.
+template <bool MASKED>
 __device__ __forceinline__ void write_list_base(int32_t* out, int n, int m, int nbase, int sink,
                                                 int window, int write_base, int list_width,
-                                                int32_t* len_out, int tid, int nthreads) {
+                                                int32_t* len_out, const uint8_t* ok, int tid, int nthreads) {
   if (write_base) {
     const int s_e = max(0, min(sink, n));
     const int w_e = max(0, min(window, n));
     const int win_start = max(n - w_e, s_e);
     if (s_e + ((w_e > 0 && win_start < n) ? n - win_start : 0) == 0) {
-      if (tid == 0 && list_width > 0) out[0] = n - 1;
+      if (tid == 0 && list_width > 0) out[0] = listed<MASKED>(n - 1, ok);
     } else {
       for (int i = tid; i < nbase && i < list_width; i += nthreads)
-        out[i] = i < s_e ? i : win_start + (i - s_e);
+        out[i] = listed<MASKED>(i < s_e ? i : win_start + (i - s_e), ok);
     }
   }
   const int total = min(nbase + m, list_width);
@@ -352,10 +363,11 @@ __device__ __forceinline__ int range_shift(u64 lo, u64 hi) {
 // when `counting_ok` (tmp then has 2 * cap_above slots) and no bin is crowded,
 // else by the bitonic sort.  All 1024 lanes; callers sync before; no barrier at
 // the end.
+template <bool MASKED>
 __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand, int ncand, int need,
                                                 u64 lo0, int shift0, u64* tmp, uint32_t* hist,
                                                 SelectShared& sh, bool counting_ok, int32_t* out,
-                                                int tid, bool placed = false) {
+                                                const uint8_t* ok, int tid, bool placed = false) {
   const int lane = tid & 63, wave = tid >> 6;
   // ---- the k-th bin: rank its entries, the best `need` follow the winners ----------
   if (ncand <= kMaxBinForCounting || need == ncand) {
@@ -363,14 +375,14 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
       const u64 v = cand[i];
       int r = 0;
       for (int j = 0; j < ncand; ++j) r += cand[j] > v;
-      if (r < need) out[n_above + r] = composite_index(v);
+      if (r < need) out[n_above + r] = listed<MASKED>(composite_index(v), ok);
     }
   } else {
     const int npc = next_pow2_dev(ncand);
     for (int i = ncand + tid; i < npc; i += kThreads) cand[i] = 0ull;
     __syncthreads();
     sort_desc(cand, npc, tid);
-    for (int i = tid; i < need; i += kThreads) out[n_above + i] = composite_index(cand[i]);
+    for (int i = tid; i < need; i += kThreads) out[n_above + i] = listed<MASKED>(composite_index(cand[i]), ok);
   }
   if (n_above == 0) return;
 
@@ -383,7 +395,7 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
       const int s0 = (int)(h & 0xffffu), c = (int)(h >> 16);
       int r = 0;
       for (int q = s0; q < s0 + c; ++q) r += buf[q] > v;
-      out[s0 + r] = composite_index(v);
+      out[s0 + r] = listed<MASKED>(composite_index(v), ok);
     }
     return;
   }
@@ -428,7 +440,7 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
         const int s0 = (int)(h & 0xffffu), c = (int)(h >> 16);
         int r = 0;
         for (int q = s0; q < s0 + c; ++q) r += grouped[q] > v;
-        out[s0 + r] = composite_index(v);
+        out[s0 + r] = listed<MASKED>(composite_index(v), ok);
       }
       return;
     }
@@ -437,7 +449,7 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
   for (int i = n_above + tid; i < np; i += kThreads) buf[i] = 0ull;
   __syncthreads();
   sort_desc(buf, np, tid);
-  for (int j = tid; j < n_above; j += kThreads) out[j] = composite_index(buf[j]);
+  for (int j = tid; j < n_above; j += kThreads) out[j] = listed<MASKED>(composite_index(buf[j]), ok);
 }
 
 // ---------------------------------------------------------------------------
@@ -458,7 +470,7 @@ __host__ __device__ __forceinline__ bool sampling_ok(int m) {
 // the lower edge of its bin.  Every workgroup that calls this for a row gets the
 // same tau.  Needs n > kPoolCap; clears hist itself (nobody may be using it).  When
 // it returns every lane has passed the barrier that follows the last read of hist.
-template <int THREADS>
+template <int THREADS, bool MASKED>
 __device__ __forceinline__ uint32_t sample_threshold(const float* row, int n, int m, uint32_t* hist,
                                                      SelectShared& sh, int tid) {
   constexpr int kMaxQ = 16384 / 4 / THREADS;  // float4 groups per lane at most
@@ -485,7 +497,7 @@ __device__ __forceinline__ uint32_t sample_threshold(const float* row, int n, in
     if (j < nq) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        kmin = min(kmin, key[j * 4 + c]);
+        if (!MASKED || key[j * 4 + c] > kMaskedKey) kmin = min(kmin, key[j * 4 + c]);
         kmax = max(kmax, key[j * 4 + c]);
       }
     }
@@ -500,8 +512,8 @@ __device__ __forceinline__ uint32_t sample_threshold(const float* row, int n, in
   kmin = (uint32_t)sh.wmin[lane & (THREADS / SOCKET_WAVE - 1)];
   kmax = (uint32_t)sh.wmax[lane & (THREADS / SOCKET_WAVE - 1)];
   wave_minmax_to_last(kmin, kmax);
-  const uint32_t smin = (uint32_t)__builtin_amdgcn_readlane((int)kmin, 63);
-  const uint32_t smax = max(smin, (uint32_t)__builtin_amdgcn_readlane((int)kmax, 63));
+  const uint32_t smax = (uint32_t)__builtin_amdgcn_readlane((int)kmax, 63);
+  const uint32_t smin = min((uint32_t)__builtin_amdgcn_readlane((int)kmin, 63), smax);
   const int target = max(2 * m, 1024);
   const int r = (int)min((int64_t)nsample, ((int64_t)target * nsample + n - 1) / n);
   const int fine = max(4, r / 8);  // a bin this small pins tau well enough
@@ -520,7 +532,7 @@ __device__ __forceinline__ uint32_t sample_threshold(const float* row, int n, in
       if (j < nq) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          const uint32_t k = key[j * 4 + c];
+          const uint32_t k = MASKED ? max(key[j * 4 + c], smin) : key[j * 4 + c];
           if (k >= lo && k <= hi) atomicAdd(&hist[(k - lo) >> shift], 1u);
         }
       }
@@ -559,8 +571,13 @@ __device__ __forceinline__ u64 load_coherent(const u64* p) {
 // row_count and row_done are zero on entry and zero again on exit.
 // The pooled composites are held in registers, eight per lane, from the moment
 // the pool is complete; LDS holds them only while they are being compacted.
+// MASKED: a byte per score says whether its position may be listed; positions that may not become -1 in the list, and
+// their scores are minus infinity.  Those are kept out of the ranges that the histograms are laid over (they count in
+// the lowest bin): with them in, half the bins lie between minus infinity and the lowest score, and rows with a masked end
+// took two passes more (56 rows of 4135, part of each masked: 19.1 us against 8.9).
+template <bool MASKED>
 __global__ __launch_bounds__(kThreads) void select_list_kernel(
-    const float* __restrict__ scores, int64_t score_stride, const int32_t* __restrict__ lens,
+    const float* __restrict__ scores, const uint8_t* __restrict__ allowed, int64_t score_stride, const int32_t* __restrict__ lens,
     const int32_t* __restrict__ budgets, const uint32_t* __restrict__ row_range, int range_parts,
     int Hq, int T, int M, int sink, int window, int write_base, int32_t* __restrict__ sparse_list,
     int64_t list_stride, int list_width, int32_t* __restrict__ sparse_len, int cap_above,
@@ -583,9 +600,10 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
   row_shape(lens, budgets, b, T, M, sink, window, write_base, list_width, n, m, nbase);
   const float* row = scores + (int64_t)rowi * score_stride;
   int32_t* out = sparse_list + (int64_t)rowi * list_stride;
+  const uint8_t* ok = MASKED ? allowed + (int64_t)rowi * T : nullptr;
   if (part == 0)
-    write_list_base(out, n, m, nbase, sink, window, write_base, list_width,
-                    sparse_len ? sparse_len + rowi : nullptr, tid, kThreads);
+    write_list_base<MASKED>(out, n, m, nbase, sink, window, write_base, list_width,
+                            sparse_len ? sparse_len + rowi : nullptr, ok, tid, kThreads);
   if (m == 0) return;
   int32_t* heavy = out + nbase;
 
@@ -610,7 +628,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         const int i = tid + u * kThreads;
         const uint32_t k = score_to_key(i < n ? row[i] : 0.f);
         if (i < n) {
-          kmin = min(kmin, k);
+          if (!MASKED || k > kMaskedKey) kmin = min(kmin, k);
           kmax = max(kmax, k);
         }
         pv[u] = composite(k, i);
@@ -702,7 +720,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
       float4 b0[kLoads], b1[kLoads], b2[kLoads];
       fetch(begin, b0);
       fetch(begin + kStep, b1);
-      const uint32_t tau = sample_threshold<kThreads>(row, n, m, hist, sh, tid);
+      const uint32_t tau = sample_threshold<kThreads, MASKED>(row, n, m, hist, sh, tid);
       for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;   // for the first refinement pass
       const float tau_f = tau >= 0xff800000u ? INFINITY : tau <= 0x007fffffu ? -INFINITY
                           : __uint_as_float((tau & 0x80000000u) ? (tau & 0x7fffffffu) : ~tau);
@@ -764,7 +782,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         for (int u = 0; u < U; ++u)
           if (tid + u * kThreads < total) {
             const uint32_t k = (uint32_t)(pv[u] >> 32);
-            kmin = min(kmin, k);
+            if (!MASKED || k > kMaskedKey) kmin = min(kmin, k);
             kmax = max(kmax, k);
           }
       }
@@ -780,8 +798,9 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         atomicMax(&sh.kmax, kmax);
       }
       __syncthreads();
-      const u64 lo0 = (u64)sh.kmin << 32, hi0 = ((u64)sh.kmax << 32) | 0xffffffffull;
+      const u64 lo0 = (u64)(MASKED ? min(sh.kmin, sh.kmax) : sh.kmin) << 32, hi0 = ((u64)sh.kmax << 32) | 0xffffffffull;
       const int shift0 = range_shift(lo0, hi0);
+      auto bin0 = [&](u64 v) { return MASKED && v < lo0 ? 0 : (int)((v - lo0) >> shift0); };
       // refinement on the composites; they are distinct, so it ends with a bin of
       // at most kCandCap entries (ties need no special case here).
       // The first pass covers every entry, and every entry keeps the slot that its
@@ -796,7 +815,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           if (tid + u * kThreads < total) {
-            const uint32_t sl = atomicAdd(&hist[(int)((pv[u] - lo0) >> shift0)], 1u);
+            const uint32_t sl = atomicAdd(&hist[bin0(pv[u])], 1u);
             slot2[u >> 1] |= sl << (16 * (u & 1));
           }
         }
@@ -804,7 +823,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         find_bin<kThreads, true>(hist, m, 1, sh, tid, [&](int bin, int before, int count) {
           const u64 blo = lo0 + ((u64)bin << shift0);
           const u64 bspan = (shift0 == 0) ? 0ull : ((1ull << shift0) - 1ull);
-          sh.lo = blo;
+          sh.lo = MASKED && bin == 0 ? 0ull : blo;
           sh.hi = (hi0 - blo < bspan) ? hi0 : blo + bspan;
           sh.need = m - before;
           sh.done = (count <= kCandCap || shift0 == 0) ? 1 : 0;
@@ -815,15 +834,15 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
           for (int u = 0; u < U; ++u) {
             if (tid + u * kThreads < total) {
               const u64 v = pv[u];
-              const int bin = (int)((v - lo0) >> shift0);
+              const int bin = bin0(v);
               const int sl = (int)((slot2[u >> 1] >> (16 * (u & 1))) & 0xffffu);
               if (bin > fb) buf[(int)(hist[bin] & 0xffffu) + sl] = v;
               else if (bin == fb && sl < kCandCap) cand[sl] = v;
             }
           }
           __syncthreads();
-          order_and_write(buf, m - need, cand, ncand, need, lo0, shift0, tmp, hist, sh, counting_ok != 0, heavy,
-                          tid, true);
+          order_and_write<MASKED>(buf, m - need, cand, ncand, need, lo0, shift0, tmp, hist, sh, counting_ok != 0, heavy,
+                          ok, tid, true);
           return;
         }
       }
@@ -861,8 +880,8 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         wave_append(have && v >= blo && v <= bhi, v, &sh.fill_cand, cand, kCandCap);
       }
       __syncthreads();
-      order_and_write(buf, m - need, cand, min(sh.fill_cand, kCandCap), need, lo0, shift0, tmp, hist, sh,
-                      counting_ok != 0, heavy, tid);
+      order_and_write<MASKED>(buf, m - need, cand, min(sh.fill_cand, kCandCap), need, lo0, shift0, tmp, hist, sh,
+                      counting_ok != 0, heavy, ok, tid);
       return;
     }
   } else if (part != 0) {
@@ -992,8 +1011,8 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
   // mass ties: all m winners are in buf and there are no candidates
   const int ncand = mass_ties ? 0 : min(sh.fill_cand, kCandCap);
   const int n_above = mass_ties ? m : m - need;
-  order_and_write(buf, n_above, cand, ncand, mass_ties ? 0 : need, (u64)lo0 << 32, shift0 + 32, tmp, hist,
-                  sh, counting_ok != 0, heavy, tid);
+  order_and_write<MASKED>(buf, n_above, cand, ncand, mass_ties ? 0 : need, (u64)lo0 << 32, shift0 + 32, tmp, hist,
+                  sh, counting_ok != 0, heavy, ok, tid);
 }
 
 int next_pow2(int x) {
@@ -1053,7 +1072,9 @@ extern "C" size_t socket_select_workspace_zero_bytes(int B, int Hq, int T, int M
   return split_layout(B * Hq).off_loc;
 }
 
-extern "C" int socket_select_list(const float* scores, int64_t score_stride, const int32_t* lens,
+namespace {
+
+int select_entry(const float* scores, const uint8_t* allowed, int64_t score_stride, const int32_t* lens,
                                   const int32_t* budgets, const uint32_t* row_range, int range_parts,
                                   int B, int Hq, int T, int M, int sink, int window, int write_base,
                                   int32_t* sparse_list, int64_t list_stride, int list_width,
@@ -1107,14 +1128,35 @@ extern "C" int socket_select_list(const float* scores, int64_t score_stride, con
   }
   SOCKET_REQUIRE((int64_t)rows * parts <= 0x7fffffff, SOCKET_ERR_SHAPE);
 
+  auto kern = allowed ? select_list_kernel<true> : select_list_kernel<false>;
   if (lds > 32 * 1024 &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(select_list_kernel),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return SOCKET_ERR_LAUNCH;
-  hipLaunchKernelGGL(select_list_kernel, dim3(rows * parts), dim3(kThreads), lds, s, scores, score_stride, lens, budgets,
+  hipLaunchKernelGGL(kern, dim3(rows * parts), dim3(kThreads), lds, s, scores, allowed, score_stride, lens, budgets,
                      row_range, range_parts, Hq, T, M, sink, window, write_base, sparse_list,
                      list_stride, list_width, sparse_len, cap_above, counting_ok, use_pool, pool_slots, parts,
                      loc, row_count, row_done);
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
+}
+
+}  // namespace
+
+extern "C" int socket_select_list(const float* scores, int64_t score_stride, const int32_t* lens,
+                                  const int32_t* budgets, const uint32_t* row_range, int range_parts,
+                                  int B, int Hq, int T, int M, int sink, int window, int write_base,
+                                  int32_t* sparse_list, int64_t list_stride, int list_width,
+                                  int32_t* sparse_len, void* workspace, size_t workspace_bytes,
+                                  void* stream) {
+  return select_entry(scores, nullptr, score_stride, lens, budgets, row_range, range_parts, B, Hq, T, M, sink, window, write_base,
+                      sparse_list, list_stride, list_width, sparse_len, workspace, workspace_bytes, stream);
+}
+
+extern "C" int socket_select_list_allowed(const float* scores, int64_t score_stride, const uint8_t* allowed, int B, int Hq, int T, int M,
+                                          int sink, int window, int32_t* sparse_list, int64_t list_stride, int list_width,
+                                          int32_t* sparse_len, void* workspace, size_t workspace_bytes, void* stream) {
+  SOCKET_REQUIRE(allowed, SOCKET_ERR_NULL);
+  return select_entry(scores, allowed, score_stride, nullptr, nullptr, nullptr, 0, B, Hq, T, M, sink, window, 1, sparse_list,
+                      list_stride, list_width, sparse_len, workspace, workspace_bytes, stream);
 }

@@ -118,18 +118,22 @@ def select_list(scores: torch.Tensor, sink: int, window: int, M: int, *, lens=No
     return sparse_list, sparse_len
 
 
+def _workspace_of(device, B: int, H: int, T: int, M: int):
+    """(workspace, its bytes) of a selection: (None, 0) where every row is one workgroup's."""
+    L = lib()
+    nbytes = L.socket_select_workspace_bytes(B, H, T, M)
+    return (_select_workspace(device, nbytes, L.socket_select_workspace_zero_bytes(B, H, T, M)) if nbytes else None), nbytes
+
+
 def _select_into(scores, sink: int, window: int, M: int, lens, budgets, write_base: bool, row_range, split: bool,
                  sparse_list: torch.Tensor, sparse_len: torch.Tensor) -> None:
     """The selection's launch into the rows of `sparse_list` [B,H,width] (any stride between rows)."""
     B, H, T = scores.shape
     width = sparse_list.shape[2]
     assert sparse_list.stride(2) == 1 and sparse_list.stride(0) == H * sparse_list.stride(1)
-    L = lib()
-    ws, ws_bytes = None, L.socket_select_workspace_bytes(B, H, T, M) if split else 0
-    if ws_bytes:
-        ws = _select_workspace(scores.device, ws_bytes, L.socket_select_workspace_zero_bytes(B, H, T, M))
+    ws, ws_bytes = _workspace_of(scores.device, B, H, T, M) if split else (None, 0)
     try:
-        check("socket_select_list", L.socket_select_list(
+        check("socket_select_list", lib().socket_select_list(
             ptr(scores), scores.stride(1), ptr(lens), ptr(budgets), ptr(row_range),
             0 if row_range is None else row_range.shape[2], B, H, T, M, int(sink), int(window),
             1 if write_base else 0, ptr(sparse_list), sparse_list.stride(1), width, ptr(sparse_len),
@@ -141,8 +145,8 @@ def _select_into(scores, sink: int, window: int, M: int, lens, budgets, write_ba
 
 
 def _build_in_place(q_probs, k_hard, v_norm, allowed, sink: int, window: int, M: int):
-    """`build_sparse_list_decode` in three launches: scores from the operands in their own types, the top-k straight
-    into the list, and the positions and -1 entries around it.  None for operands it does not take."""
+    """`build_sparse_list_decode` in two launches: scores from the operands in their own types, and the list.  None for
+    operands it does not take."""
     B, H, L, R = q_probs.shape
     T = k_hard.shape[3]
     types = (torch.float16, torch.bfloat16, torch.float32)
@@ -162,8 +166,15 @@ def _build_in_place(q_probs, k_hard, v_norm, allowed, sink: int, window: int, M:
     check("socket_soft_hash_collision", lib().socket_soft_hash_collision_typed(
         ptr(q_probs), dtype_enum(q_probs.dtype), ptr(k_hard), ptr(allowed), ptr(v_norm), dtype_enum(v_norm.dtype), ptr(scores),
         B, H, L, R, T, s))
-    _select_into(scores, 0, 0, M, None, None, False, None, True, sparse_list[:, :, base:], sparse_len)
-    check("socket_finish_list", lib().socket_finish_list(ptr(sparse_list), ptr(sparse_len), ptr(allowed), B * H, T, sink, window, M, s))
+    ws, ws_bytes = _workspace_of(scores.device, B, H, T, M)
+    try:
+        check("socket_select_list", lib().socket_select_list_allowed(
+            ptr(scores), T, ptr(allowed), B, H, T, M, sink, window, ptr(sparse_list), base + M, base + M, ptr(sparse_len),
+            ptr(ws), ws_bytes, s))
+    except RuntimeError:
+        if ws is not None:
+            reset_select_workspaces()
+        raise
     return sparse_list, sparse_len
 
 

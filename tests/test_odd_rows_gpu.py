@@ -69,3 +69,28 @@ def test_selection_from_odd_rows(T, M, shift):
     lists, lens = sparse.select_list(scores, 0, 0, M, write_base=False)
     assert (lens == M).all()
     assert torch.equal(lists.long(), torch.sort(scores, dim=-1, descending=True, stable=True).indices[..., :M])
+
+
+@pytest.mark.parametrize("B,H,T,M,sink,window,kept", [
+    (1, 4, 5, 5, 2, 2, 0.5),                # more asked for than are allowed
+    (2, 7, 4135, 129, 20, 20, 0.5),
+    (1, 8, 8192, 700, 0, 0, 0.05),          # fewer allowed than are asked for: masked ones fill the list
+    (1, 8, 8193, 300, 4, 64, 0.9),          # threshold from a sample
+    (2, 5, 20881, 652, 4, 64, 0.02),        # ... of which little is allowed
+    (1, 6, 49157, 1024, 4, 64, 0.6),        # a row shared between workgroups
+    (1, 3, 9000, 128, 3, 9000, 0.7),        # a window that is the whole row
+])
+def test_masked_lists(B, H, T, M, sink, window, kept):
+    """The list builder's masked selection against the unmasked one with torch's masking around it; the second row of every
+    sequence has nothing allowed, the third everything."""
+    dev, L, R = "cuda", 4, 64
+    g = torch.Generator(device=dev).manual_seed(T + M)
+    q = torch.rand(B, H, L, R, generator=g, device=dev)
+    codes = torch.randint(0, R, (B, H, L, T), generator=g, device=dev).to(torch.int16)
+    norms = (torch.rand(B, H, T, generator=g, device=dev) + 0.1).half()
+    allowed = torch.rand(B, H, T, generator=g, device=dev) < kept
+    allowed[:, 0, T // 2:] = False
+    allowed[:, 1], allowed[:, 2] = False, True
+    got, got_len = sparse.build_sparse_list_decode(q, codes, norms, allowed, sink, window, M)
+    want, want_len = sparse._build_with_torch(q, codes, norms, allowed, sink, window, min(M, T))
+    assert torch.equal(got, want) and torch.equal(got_len, want_len)
