@@ -36,7 +36,7 @@ constexpr float kPaMaxCap = 60.f;   // exp(60) * 2^31 keys < 3.4e38, exp(-60) > 
 // maximum: p = exp(cap - 2 cap / (exp(2 s / cap) + 1)).  POS: token t sees the keys up to positions[t]
 // instead of pos0 + t (one endless chunk, a.k_from = 0).
 template <class DT, int D, int D2, int DV, int TERMS, bool CAPPED, bool POS>
-__global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_chunk_attention a, const int64_t* positions) {
+__global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_chunk_attention a, const int64_t* positions, int first_round) {
   constexpr int CK = D / 8, CK2 = D2 / 8, CV = DV / 8;            // 16-byte pieces per row
   constexpr int KS = D / 16, KS2 = D2 / 16, DB = DV / 32;
   constexpr int kK2 = kPaKeys * D * 2, kV = kK2 + kPaKeys * D2 * 2, kStage = kV + kPaKeys * DV * 2;   // places in a stage
@@ -44,9 +44,13 @@ __global__ __launch_bounds__(64 * kPaWaves, 2) void prompt_attend_kernel(socket_
 
   const int Gq = a.H / a.G;
   // kv heads are neighbours in the launch order: with eight of them each XCD's L2 serves one head's
-  // keys.  Later tiles see more keys and come first.
+  // keys.  Later tiles see more keys and come first.  Where every workgroup is at work at once, two to a CU (first_round: the
+  // tiles that make one for every CU; 0: more or fewer than that), the second ones come shortest first: the CU with the
+  // longest tile has the shortest as well, and all end together (2 x 2048 tokens of 16 heads over caches of 4096 to 8192
+  // keys, weights in three terms: 335 us with the longest first throughout, 296).
   const int heads = a.G * a.B, tiles = gridDim.x / heads;
-  const int hb = blockIdx.x % heads, tile = tiles - 1 - blockIdx.x / heads;
+  const int hb = blockIdx.x % heads, nth = blockIdx.x / heads;
+  const int tile = first_round > 0 && nth >= first_round ? nth - first_round : tiles - 1 - nth;
   const int g = hb % a.G, b = hb / a.G;
   const int64_t R = (int64_t)a.T * Gq, r0 = (int64_t)tile * kPaRows;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -278,7 +282,9 @@ int pa_launch(const socket_chunk_attention& a, const int64_t* positions, hipStre
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
       return SOCKET_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64 * kPaWaves), lds, s, a, positions);
+  const int cus = socket_device_limits().cu_count, heads = a.G * a.B;
+  const int first_round = n > cus && n <= 2 * (int64_t)cus ? (cus + heads - 1) / heads : 0;
+  hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64 * kPaWaves), lds, s, a, positions, first_round);
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
 }
