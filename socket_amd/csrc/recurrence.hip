@@ -17,14 +17,16 @@
 // strong decay.  Tokens are grouped in blocks of 16 with sums pl local to the block and
 // block totals tot; for s in an earlier block the exponent splits at the start of t's
 // block into two parts that are both <= 0.  Inside a block the split at the block's
-// start is used while its total stays above kMildDecay, else the exponent is taken per
-// pair on the vector ALU.
+// start is used while its total stays above kMildDecay, else those at the middle of ever smaller
+// groups of rows, where both parts are <= 0 again.
 //
 // All products are v_mfma_f32_16x16x4_f32 (fp32 operands).  Its operands hold one k index
 // per lane quarter; a step r of four takes k = 4 * quarter + r of a 16-wide tile, so that
 // a lane's four values are one 16-byte vector ("fragment order": lane (quarter, x) holds row x,
 // columns 4 quarter .. + 3 of a tile), and an accumulator (rows 4 quarter + r, column x) is
 // directly the second operand of the next product.
+#include <type_traits>
+
 #include "elem.h"
 
 namespace {
@@ -431,85 +433,239 @@ __device__ __forceinline__ void invert_diagonal(float* d, int x16, int quarter) 
     for (int r = 0; r < 16; ++r) d[((x16 >> 2) * 16 + r) * 4 + (x16 & 3)] = x[r];
 }
 
-template <class DT, int NB>
-__global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_recurrence a, int vec) {
+// Eight channels of N inputs of token t (q, k and v of one head: columns `col` of the projected row, channels `ch`
+// of the convolution) after the convolution and its activation, as conv_input gives them, every tap of every input
+// requested before the first is used.  No load stands under a condition: rows before the portion come from another
+// address, and rows that are nowhere are cleared where a chunk can have them.
+template <class DT, int N, int TAPS>
+__device__ __forceinline__ void conv_inputs(const socket_recurrence& a, int b, int t, bool at_start, const int (&col)[N],
+                                            const int (&ch)[N], float (&out)[N][8]) {
+  const int64_t row = b * a.proj_stride_b;
+  if (a.taps < 1) {
+    Raw8<DT> x[N];
+#pragma unroll
+    for (int s = 0; s < N; ++s) x[s].load(a.proj, row + t * a.proj_stride_t + col[s]);
+#pragma unroll
+    for (int s = 0; s < N; ++s) x[s].get(out[s]);
+    return;
+  }
+  const int n1 = a.taps - 1, C = conv_channels(a);
+#pragma unroll
+  for (int s = 0; s < N; ++s)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out[s][e] = 0.f;
+  for (int m0 = 0; m0 < a.taps; m0 += TAPS) {
+    Raw8<DT> x[N][TAPS];
+#pragma unroll
+    for (int i = 0; i < TAPS; ++i) {
+      const int tt = t - n1 + min(m0 + i, n1);
+      const bool stored = at_start && tt < 0 && !a.fresh;
+      const void* from = stored ? a.conv_state : a.proj;
+      const int64_t at = stored ? (((int64_t)(a.pos0 & 1) * a.B + b) * n1 + (tt + n1)) * C : row + max(tt, 0) * a.proj_stride_t;
+#pragma unroll
+      for (int s = 0; s < N; ++s) x[s][i].load(from, at + (stored ? ch[s] : col[s]));
+    }
+    if (at_start && a.fresh) {
+#pragma unroll
+      for (int i = 0; i < TAPS; ++i)
+        if (t - n1 + m0 + i < 0)
+#pragma unroll
+          for (int s = 0; s < N; ++s) x[s][i].zero();
+    }
+#pragma unroll
+    for (int s = 0; s < N; ++s) {
+#pragma unroll
+      for (int i0 = 0; i0 < TAPS; i0 += 2) {
+        float w[2][8];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) load_vec<DType_f32, 8>(a.conv_w, (int64_t)min(m0 + i0 + i, n1) * C + ch[s], w[i]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          if (m0 + i0 + i < a.taps) {
+            float y[8];
+            x[s][i0 + i].get(y);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) out[s][e] = fmaf(y[e], w[i][e], out[s][e]);
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < N; ++s)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out[s][e] *= sigmoid_f32(out[s][e]);
+}
+
+// Lane j of every four lanes gives x[c] of lane c: x[c] becomes what lane c held at j.
+__device__ __forceinline__ void transpose_quad(rc_f32x4& x, int lane) {
+  const bool odd = lane & 1, high = lane & 2;
+#pragma unroll
+  for (int p = 0; p < 4; p += 2) {
+    const float got = butterfly_partner<1>(odd ? x[p] : x[p + 1]);
+    x[p] = odd ? got : x[p];
+    x[p + 1] = odd ? x[p + 1] : got;
+  }
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const float got = butterfly_partner<2>(high ? x[p] : x[p + 2]);
+    x[p] = high ? got : x[p];
+    x[p + 2] = high ? x[p + 2] : got;
+  }
+}
+
+// One workgroup per (chunk, head, sequence).  With 16 waves on a CU and one such workgroup (three operands and the
+// tiles in LDS) nothing but the waves themselves hides a wait, so each phase asks for all it reads before it uses any:
+//  * a lane's eight channels of q, k and v with all their taps, and its eight decays, in one trip to memory; unit
+//    norms from those registers, running sums of the decays over 8 rows of a lane and a lane 32 further on;
+//  * the tiles of Aqk and L (a diagonal tile inverted by its own wave) and the fragments of Q^ and K^T are dealt out
+//    by a counter, the long ones first;
+//  * the forward substitution has its tiles in registers before it starts, and W leaves in 16-byte stores.
+// A workgroup of 128 key channels with the delta rule / of 64 without, in clock cycles: 63000 / 29000 -> 47000 / 21000
+// (18000 of the 47000 the first trip and its arithmetic, 13000 the tiles, 5000 the substitution); 5000 tokens of 16 heads
+// of either kind 294 -> 238 us.  A chunk writes 144 KB for the scan, which 256 of them drain in about 8 us.  Holding
+// the second kind to 64 registers for two workgroups a CU spilled: 63 us a pass instead of 53.
+template <class DT, int NB, bool DELTA>
+__global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_recurrence a, int vec, int own_v) {
   constexpr int C = 16 * NB;
+  constexpr int LPR = kPrepThreads / C;          // lanes to a token: 8 channels each
   extern __shared__ __attribute__((aligned(16))) float rp_lds[];
-  const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ int next_item;
+  const int h = blockIdx.x, chunk = blockIdx.y, b = blockIdx.z;   // (a head on one XCD, where its scan will be)
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int x16 = lane & 15, quarter = lane >> 4;
   const int dk = a.dk, dv = a.dv, hk = h / (a.H / a.Hk);
-  const bool delta = a.beta_off >= 0;
   const ChunkSpace sp{(dk + 15) / 16, (dv + 15) / 16, NB};
   const int dkp = sp.kt * 16, dvp = sp.vt * 16;
   const int kp = dkp + 4, vp = dvp + 4;          // LDS pitches
   const int t_first = a.t0 + chunk * C;          // token of the portion
   const int n_rows = min(C, a.t0 + a.n - t_first);
 
-  float* qs = rp_lds;                            // C x kp; later V, C x vp
-  float* ks = qs + C * (kp > vp ? kp : vp);      // C x kp
-  float* pl = ks + C * kp;                       // C x kp: log2 decay, then its running sum inside the block
+  float* pl = rp_lds;                            // C x kp: running sum of the log2 decay inside the block
   float* tot = pl + C * kp;                      // NB x dkp
-  float* lk = tot + NB * dkp;                    // NB x NB tiles in fragment order: -L, inverses on the diagonal
-  float* beta = lk + NB * NB * 256;              // C
+  float* beta = tot + NB * dkp;                  // C
+  float* lk = beta + C;                          // DELTA: NB x NB tiles in fragment order: -L, inverses on the diagonal
+  float* ks = lk + (DELTA ? NB * NB * 256 : 0);  // C x kp
+  float* qs = ks + C * kp;                       // C x kp
+  // C x vp; by itself where LDS allows it, else over q (without the delta rule over k as well) once that has been used
+  float* vs = DELTA && own_v ? qs + C * kp : DELTA ? qs : ks;
 
-  float* ws = (float*)a.workspace + (((int64_t)b * a.H + h) * gridDim.x + chunk) * sp.size();
+  float* ws = (float*)a.workspace + (((int64_t)b * a.H + h) * gridDim.y + chunk) * sp.size();
 
-  // ---- inputs
-  stage_rows<DT>(a, b, t_first, n_rows, C, a.q_off + hk * dk, hk * dk, dk, dkp, qs, kp, vec);
-  stage_rows<DT>(a, b, t_first, n_rows, C, a.k_off + hk * dk, a.Hk * dk + hk * dk, dk, dkp, ks, kp, vec);
-  const float a_exp = a.decay_kind == 0 ? exp_f32(a.a_log[h]) : 0.f;
-#pragma unroll 4
-  for (int w = tid; w < C * dkp; w += kPrepThreads) {
-    const int r = w / dkp, c = w % dkp;
-    float g = 0.f;
-    if (r < n_rows && c < dk) {
-      const int64_t zi = ((int64_t)b * a.T + t_first + r) * a.H * dk + h * dk + c;
-      g = log2_decay(a, a_exp, (a.decay_z_f32 ? ((const float*)a.decay_z)[zi] : load_elem<DT>(a.decay_z, zi)) +
-                                   (a.decay_bias ? a.decay_bias[h * dk + c] : 0.f));
+  // ---- inputs.  Decays: lane x of 32 (and x + 32) takes a channel over rows 0 .. 7 (and 8 .. 15) of a block
+  const int spans = (dkp + 31) / 32;
+  float z[8];
+  auto request_decays = [&](int g) __attribute__((always_inline)) {
+    const int blk = g / spans, c = (g - blk * spans) * 32 + (lane & 31), r0 = 16 * blk + 8 * (lane >> 5);
+    const int64_t zc = (int64_t)h * dk + min(c, dk - 1);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int64_t zi = ((int64_t)b * a.T + t_first + min(r0 + r, n_rows - 1)) * a.H * dk + zc;
+      z[r] = a.decay_z_f32 ? ((const float*)a.decay_z)[zi] : load_elem<DT>(a.decay_z, zi);
     }
-    pl[r * kp + c] = g;
+  };
+  if (wave < NB * spans) request_decays(wave);
+  {
+    const int r = tid / LPR, c = tid % LPR * 8;
+    const bool row_ok = r < n_rows;
+    const int t = t_first + min(r, n_rows - 1);
+    constexpr int N = 3;
+    const int width[N] = {dk, dk, dv};
+    const int col0[N] = {a.q_off + hk * dk, a.k_off + hk * dk, a.v_off + h * dv};
+    const int ch0[N] = {hk * dk, a.Hk * dk + hk * dk, 2 * a.Hk * dk + h * dv};
+    float x[N][8];
+    if (vec) {
+      int col[N], ch[N];
+#pragma unroll
+      for (int s = 0; s < N; ++s) {
+        const int in = c < width[s] ? c : 0;
+        col[s] = col0[s] + in;
+        ch[s] = ch0[s] + in;
+      }
+      const bool at_start = t_first < a.taps - 1;
+      if (DELTA && own_v) {
+        conv_inputs<DT, 3, DT::kPer16B == 8 ? 4 : 2>(a, b, t, at_start, col, ch, x);
+      } else {
+        const int col2[2] = {col[0], col[1]}, ch2[2] = {ch[0], ch[1]};
+        float y[2][8];
+        conv_inputs<DT, 2, 2>(a, b, t, at_start, col2, ch2, y);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          x[0][e] = y[0][e];
+          x[1][e] = y[1][e];
+          x[2][e] = 0.f;
+        }
+      }
+    } else {
+      stage_rows<DT>(a, b, t_first, n_rows, C, col0[0], ch0[0], dk, dkp, qs, kp, false);
+      stage_rows<DT>(a, b, t_first, n_rows, C, col0[1], ch0[1], dk, dkp, ks, kp, false);
+      if (DELTA && own_v) stage_rows<DT>(a, b, t_first, n_rows, C, col0[2], ch0[2], dv, dvp, vs, vp, false);
+      __syncthreads();
+      // (a lane's own eight channels, which it writes again below; those past the width are zero)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        x[0][e] = c < dkp ? qs[r * kp + c + e] : 0.f;
+        x[1][e] = c < dkp ? ks[r * kp + c + e] : 0.f;
+        x[2][e] = DELTA && own_v && c < dvp ? vs[r * vp + c + e] : 0.f;
+      }
+    }
+    float sq[2] = {0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < N; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        x[s][e] = row_ok && c < width[s] ? x[s][e] : 0.f;
+        if (s < 2) sq[s] = fmaf(x[s][e], x[s][e], sq[s]);
+      }
+    float mul[2] = {a.q_scale, 1.f};
+    if (a.unit_qk) {
+      mul[0] *= rsqrt_f32(group_sum<LPR>(sq[0]) + 1e-6f);
+      mul[1] = rsqrt_f32(group_sum<LPR>(sq[1]) + 1e-6f);
+    }
+    auto put = [&](float* to, const float* y, float m) __attribute__((always_inline)) {
+      *reinterpret_cast<float4*>(to) = make_float4(y[0] * m, y[1] * m, y[2] * m, y[3] * m);
+      *reinterpret_cast<float4*>(to + 4) = make_float4(y[4] * m, y[5] * m, y[6] * m, y[7] * m);
+    };
+    if (c < dkp) {
+      put(qs + r * kp + c, x[0], mul[0]);
+      put(ks + r * kp + c, x[1], mul[1]);
+    }
+    if (DELTA && own_v && c < dvp) put(vs + r * vp + c, x[2], 1.f);
+  }
+  const float a_exp = a.decay_kind == 0 ? exp_f32(a.a_log[h]) : 0.f;
+  for (int g = wave; g < NB * spans; g += kPrepWaves) {
+    if (g != wave) request_decays(g);
+    const int blk = g / spans, c = (g - blk * spans) * 32 + (lane & 31), r0 = 16 * blk + 8 * (lane >> 5);
+    const float bias = a.decay_bias && c < dk ? a.decay_bias[h * dk + c] : 0.f;
+    float sum = 0.f;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      sum += r0 + r < n_rows && c < dk ? log2_decay(a, a_exp, z[r] + bias) : 0.f;
+      z[r] = sum;
+    }
+    const float first = lane_xor32(sum), before = lane < 32 ? 0.f : first;
+    if (c < dkp) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) pl[(r0 + r) * kp + c] = z[r] + before;
+      if (lane >= 32) tot[blk * dkp + c] = sum + before;
+    }
   }
   if (tid < C)
-    beta[tid] = (delta && tid < n_rows)
+    beta[tid] = (DELTA && tid < n_rows)
                     ? sigmoid_f32(load_elem<DT>(a.proj, b * a.proj_stride_b + (t_first + tid) * a.proj_stride_t + a.beta_off + h))
                     : 0.f;
+  if (tid == 0) next_item = 0;
   __syncthreads();
 
-  // ---- unit vectors and the scale of q; running sums of the log2 decay inside each block
-  for (int r = wave; r < C; r += kPrepWaves) {
-    float qm = a.q_scale, km = 1.f;
-    if (a.unit_qk) {
-      float sq = 0.f, sk = 0.f;
-      for (int c = lane; c < dkp; c += 64) {
-        sq = fmaf(qs[r * kp + c], qs[r * kp + c], sq);
-        sk = fmaf(ks[r * kp + c], ks[r * kp + c], sk);
-      }
-      qm *= rsqrt_f32(group_sum<64>(sq) + 1e-6f);
-      km = rsqrt_f32(group_sum<64>(sk) + 1e-6f);
-    }
-    for (int c = lane; c < dkp; c += 64) {
-      qs[r * kp + c] *= qm;
-      ks[r * kp + c] *= km;
-    }
-  }
-  for (int w = tid; w < NB * dkp; w += kPrepThreads) {
-    const int blk = w / dkp, c = w % dkp;
+  for (int c = tid; c < dkp; c += kPrepThreads) {
     float s = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s += pl[(blk * 16 + r) * kp + c];
-      pl[(blk * 16 + r) * kp + c] = s;
-    }
-    tot[blk * dkp + c] = s;
+    for (int m = 0; m < NB; ++m) s += tot[m * dkp + c];
+    ws[sp.gamma() + c] = exp2_fast(s);
   }
-  __syncthreads();
 
-  // ---- Aqk and -L, tile (I, J): lane (quarter, x) holds row x of block I against keys
+  // Aqk and -L, tile (I, J): lane (quarter, x) holds row x of block I against keys
   // 4 quarter + r of block J (the transposed product, which leaves fragment order)
-  for (int unit = wave; unit < NB * (NB + 1) / 2; unit += kPrepWaves) {
-    int I = 0, J = unit;
-    while (J > I) J -= ++I;
+  auto pair_tile = [&](int I, int J) __attribute__((always_inline)) {
     const int t = 16 * I + x16, s = 16 * J + x16;
     rc_f32x4 aq = {0.f, 0.f, 0.f, 0.f}, ak = {0.f, 0.f, 0.f, 0.f};
     bool mild = true;
@@ -519,13 +675,19 @@ __global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_re
       mild = __builtin_amdgcn_ballot_w64(low) == 0;
     }
     if (mild) {
+#pragma unroll 2
       for (int j = 0; j < sp.kt; ++j) {
         const int c = 16 * j + 4 * quarter;
         float4 kk = *reinterpret_cast<const float4*>(ks + s * kp + c);
         const float4 ps = *reinterpret_cast<const float4*>(pl + s * kp + c);
+        const float4 pt = *reinterpret_cast<const float4*>(pl + t * kp + c);
+        const float4 qt = *reinterpret_cast<const float4*>(qs + t * kp + c);
+        float4 kt = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (DELTA) kt = *reinterpret_cast<const float4*>(ks + t * kp + c);
         float4 e = make_float4(-ps.x, -ps.y, -ps.z, -ps.w);
-        if (I != J) {
-          for (int m = J; m < I; ++m) {
+#pragma unroll
+        for (int m = 0; m < NB - 1; ++m) {
+          if (m >= J && m < I) {
             const float4 tm = *reinterpret_cast<const float4*>(tot + m * dkp + c);
             e.x += tm.x;
             e.y += tm.y;
@@ -537,28 +699,51 @@ __global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_re
         kk.y *= exp2_fast(e.y);
         kk.z *= exp2_fast(e.z);
         kk.w *= exp2_fast(e.w);
-        const float4 pt = *reinterpret_cast<const float4*>(pl + t * kp + c);
         const float4 f = make_float4(exp2_fast(pt.x), exp2_fast(pt.y), exp2_fast(pt.z), exp2_fast(pt.w));
-        const float4 qt = *reinterpret_cast<const float4*>(qs + t * kp + c);
         aq = mfma4(kk, rc_f32x4{qt.x * f.x, qt.y * f.y, qt.z * f.z, qt.w * f.w}, aq);
-        if (delta) {
-          const float4 kt = *reinterpret_cast<const float4*>(ks + t * kp + c);
-          ak = mfma4(kk, rc_f32x4{kt.x * f.x, kt.y * f.y, kt.z * f.z, kt.w * f.w}, ak);
-        }
+        if (DELTA) ak = mfma4(kk, rc_f32x4{kt.x * f.x, kt.y * f.y, kt.z * f.z, kt.w * f.w}, ak);
       }
     } else {
-      for (int c = 0; c < dkp; ++c) {
-        const float pt = pl[t * kp + c], qt = qs[t * kp + c], kt = ks[t * kp + c];
+      // Strong decay inside the block: rows in groups of 2 n (n = 8, 4, 2, 1), the exponent split at the last row of
+      // a group's first half.  Both parts are <= 0 for a token of the second half and a key of the first; the others
+      // are taken as zero.  Token t and key s are in different halves of one group for the n that is the highest bit
+      // of t ^ s, and that product is the one kept; t = s has no exponent.  (A pair at a time on the vector ALU took the
+      // workgroup 26000 cycles more than mild tiles; this 11000.)
+      rc_f32x4 lq[5], lkk[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int sr = 16 * J + 4 * quarter + r;
-          const float w = ks[sr * kp + c] * exp2_fast(fminf(pt - pl[sr * kp + c], 0.f));
-          aq[r] = fmaf(qt, w, aq[r]);
-          ak[r] = fmaf(kt, w, ak[r]);
+      for (int v = 0; v < 5; ++v) {
+        lq[v] = rc_f32x4{0.f, 0.f, 0.f, 0.f};
+        if (v < 4) lkk[v] = rc_f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      for (int j = 0; j < sp.kt; ++j) {
+        const int c = 16 * j + 4 * quarter;
+        const float4 k = *reinterpret_cast<const float4*>(ks + t * kp + c);
+        const float4 q = *reinterpret_cast<const float4*>(qs + t * kp + c);
+        const float4 p = *reinterpret_cast<const float4*>(pl + t * kp + c);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int n = 1 << v;
+          const bool second = x16 & n;
+          const float4 ref = *reinterpret_cast<const float4*>(pl + (16 * I + (x16 & ~(2 * n - 1)) + n - 1) * kp + c);
+          const float sign = second ? 1.f : -1.f;
+          const float4 f = make_float4(exp2_fast(fminf(sign * (p.x - ref.x), 0.f)), exp2_fast(fminf(sign * (p.y - ref.y), 0.f)),
+                                       exp2_fast(fminf(sign * (p.z - ref.z), 0.f)), exp2_fast(fminf(sign * (p.w - ref.w), 0.f)));
+          const float4 key = second ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(k.x * f.x, k.y * f.y, k.z * f.z, k.w * f.w);
+          const float one = second ? 1.f : 0.f;
+          const rc_f32x4 g = {f.x * one, f.y * one, f.z * one, f.w * one};
+          lq[v] = mfma4(key, rc_f32x4{q.x * g[0], q.y * g[1], q.z * g[2], q.w * g[3]}, lq[v]);
+          if (DELTA) lkk[v] = mfma4(key, rc_f32x4{k.x * g[0], k.y * g[1], k.z * g[2], k.w * g[3]}, lkk[v]);
         }
+        lq[4] = mfma4(k, rc_f32x4{q.x, q.y, q.z, q.w}, lq[4]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int apart = x16 ^ (4 * quarter + r);
+        aq[r] = apart >= 8 ? lq[3][r] : apart >= 4 ? lq[2][r] : apart >= 2 ? lq[1][r] : apart ? lq[0][r] : lq[4][r];
+        ak[r] = apart >= 8 ? lkk[3][r] : apart >= 4 ? lkk[2][r] : apart >= 2 ? lkk[1][r] : lkk[0][r];
       }
     }
-    const float bt = beta[t];
+    const float bt = DELTA ? beta[t] : 0.f;
     float4 q4, k4;
     float* q4p = &q4.x;
     float* k4p = &k4.x;
@@ -569,87 +754,129 @@ __global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_re
       k4p[r] = sr < t ? -bt * ak[r] : 0.f;
     }
     *reinterpret_cast<float4*>(ws + sp.aqk() + (I * NB + J) * 256 + lane * 4) = q4;
-    if (delta) *reinterpret_cast<float4*>(lk + (I * NB + J) * 256 + lane * 4) = k4;
-  }
-
-  // ---- Q^ and K^T (for the update) fragments, the chunk's total decay
-  for (int item = wave; item < 2 * NB * sp.kt; item += kPrepWaves) {
-    const bool is_q = item < NB * sp.kt;
-    const int w = is_q ? item : item - NB * sp.kt;
-    if (is_q) {
-      const int rt = w / sp.kt, ct = w % sp.kt;
-      const int t = 16 * rt + x16, c = 16 * ct + 4 * quarter;
-      float4 e = *reinterpret_cast<const float4*>(pl + t * kp + c);
-      for (int m = 0; m < rt; ++m) {
+    if (DELTA) {
+      float* d = lk + (I * NB + J) * 256;
+      *reinterpret_cast<float4*>(d + lane * 4) = k4;
+      if (I == J) {
+        // (I + L_II)^{-1}, a column per lane; the tile is this wave's own until the barrier
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        invert_diagonal(d, x16, quarter);
+      }
+    }
+  };
+  auto q_fragment = [&](int w) __attribute__((always_inline)) {
+    const int ct = w / NB, rt = w % NB;
+    const int t = 16 * rt + x16, c = 16 * ct + 4 * quarter;
+    float4 e = *reinterpret_cast<const float4*>(pl + t * kp + c);
+    const float4 q = *reinterpret_cast<const float4*>(qs + t * kp + c);
+#pragma unroll
+    for (int m = 0; m < NB - 1; ++m) {
+      if (m < rt) {
         const float4 tm = *reinterpret_cast<const float4*>(tot + m * dkp + c);
         e.x += tm.x;
         e.y += tm.y;
         e.z += tm.z;
         e.w += tm.w;
       }
-      const float4 q = *reinterpret_cast<const float4*>(qs + t * kp + c);
-      *reinterpret_cast<float4*>(ws + sp.q() + (rt * sp.kt + ct) * 256 + lane * 4) =
-          make_float4(q.x * exp2_fast(e.x), q.y * exp2_fast(e.y), q.z * exp2_fast(e.z), q.w * exp2_fast(e.w));
-    } else {
-      const int ct = w / NB, rt = w % NB;
-      const int c = 16 * ct + x16;
-      float after = 0.f;
-      for (int m = rt; m < NB; ++m) after += tot[m * dkp + c];
-      float4 o;
-      float* op = &o.x;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * rt + 4 * quarter + r;
-        op[r] = ks[t * kp + c] * exp2_fast(after - pl[t * kp + c]);
-      }
-      *reinterpret_cast<float4*>(ws + sp.kT() + (ct * NB + rt) * 256 + lane * 4) = o;
     }
-  }
-  for (int c = tid; c < dkp; c += kPrepThreads) {
-    float s = 0.f;
-    for (int m = 0; m < NB; ++m) s += tot[m * dkp + c];
-    ws[sp.gamma() + c] = exp2_fast(s);
-  }
-  __syncthreads();
+    *reinterpret_cast<float4*>(ws + sp.q() + (rt * sp.kt + ct) * 256 + lane * 4) =
+        make_float4(q.x * exp2_fast(e.x), q.y * exp2_fast(e.y), q.z * exp2_fast(e.z), q.w * exp2_fast(e.w));
+  };
+  auto k_fragment = [&](int w) __attribute__((always_inline)) {
+    const int ct = w / NB, rt = w % NB;
+    const int c = 16 * ct + x16;
+    float after = 0.f;
+#pragma unroll
+    for (int m = 0; m < NB; ++m) after += m >= rt ? tot[m * dkp + c] : 0.f;
+    float4 o;
+    float* op = &o.x;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int t = 16 * rt + 4 * quarter + r;
+      op[r] = ks[t * kp + c] * exp2_fast(after - pl[t * kp + c]);
+    }
+    *reinterpret_cast<float4*>(ws + sp.kT() + (ct * NB + rt) * 256 + lane * 4) = o;
+  };
 
-  // ---- (I + L_II)^{-1} of the diagonal tiles, a column per lane; V over q's rows meanwhile
-  if (delta && wave < NB) invert_diagonal(lk + (wave * NB + wave) * 256, x16, quarter);
-  stage_rows<DT>(a, b, t_first, n_rows, C, a.v_off + h * dv, 2 * a.Hk * dk + h * dv, dv, dvp, qs, vp, vec);
+  // ---- tiles (the diagonal ones first), then fragments of Q^ and K^T (for the update), one of each to an item
+  constexpr int kTiles = NB * (NB + 1) / 2;
+  const int items = kTiles + NB * sp.kt;
+  for (int item = wave;;) {
+    if (item >= items) break;   // (an item past the end is the wave's last)
+    if (item < kTiles) {
+      int I = item, J = item;
+      if (item >= NB) {
+        I = 1;
+        J = item - NB;
+        while (J >= I) J -= I++;
+      }
+      pair_tile(I, J);
+    } else {
+      q_fragment(item - kTiles);
+      k_fragment(item - kTiles);
+    }
+    int got = 0;
+    if (lane == 0) got = atomicAdd(&next_item, 1);
+    item = kPrepWaves + __builtin_amdgcn_readfirstlane(got);
+  }
   __syncthreads();
+  if (!DELTA || !own_v) {
+    stage_rows<DT>(a, b, t_first, n_rows, C, a.v_off + h * dv, 2 * a.Hk * dk + h * dv, dv, dvp, vs, vp, vec);
+    __syncthreads();
+  }
 
   // ---- Ubar = T beta V and W = T beta K^, a 16-column tile per wave: forward substitution over
   // the blocks; a finished block's accumulator is the next product's operand
-  const int n_tiles = delta ? sp.vt + sp.kt : sp.vt;
+  const int n_tiles = DELTA ? sp.vt + sp.kt : sp.vt;
   for (int tile = wave; tile < n_tiles; tile += kPrepWaves) {
-    const bool is_v = tile < sp.vt;
+    const bool is_v = !DELTA || tile < sp.vt;
     const int ct = is_v ? tile : tile - sp.vt;
     const int c = 16 * ct + x16;
     rc_f32x4 X[NB];
-    float before = 0.f;
+    float4 m[DELTA ? kTiles : 1];
+    if constexpr (DELTA) {
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int J = 0; J <= I; ++J)
+          m[I * (I + 1) / 2 + J] = *reinterpret_cast<const float4*>(lk + (I * NB + J) * 256 + lane * 4);
+    }
+    if (is_v) {
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) X[I][r] = vs[(16 * I + 4 * quarter + r) * vp + c];
+    } else {
+      float before = 0.f;
+#pragma unroll
+      for (int I = 0; I < NB; ++I) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = 16 * I + 4 * quarter + r;
+          X[I][r] = ks[t * kp + c] * exp2_fast(before + pl[t * kp + c]);
+        }
+        before += tot[I * dkp + c];
+      }
+    }
 #pragma unroll
     for (int I = 0; I < NB; ++I) {
-      rc_f32x4 acc;
+      if constexpr (DELTA) {
+        rc_f32x4 acc;
+        const float4 bt = *reinterpret_cast<const float4*>(beta + 16 * I + 4 * quarter);
+        acc[0] = bt.x * X[I][0];
+        acc[1] = bt.y * X[I][1];
+        acc[2] = bt.z * X[I][2];
+        acc[3] = bt.w * X[I][3];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 16 * I + 4 * quarter + r;
-        const float v = is_v ? qs[t * vp + c] : ks[t * kp + c] * exp2_fast(before + pl[t * kp + c]);
-        acc[r] = delta ? beta[t] * v : v;
-      }
-      if (!is_v) before += tot[I * dkp + c];
-      if (delta) {
-#pragma unroll
-        for (int J = 0; J < I; ++J)
-          acc = mfma4(*reinterpret_cast<const float4*>(lk + (I * NB + J) * 256 + lane * 4), X[J], acc);
-        X[I] = mfma4(*reinterpret_cast<const float4*>(lk + (I * NB + I) * 256 + lane * 4), acc, rc_f32x4{0.f, 0.f, 0.f, 0.f});
-      } else {
-        X[I] = acc;
+        for (int J = 0; J < I; ++J) acc = mfma4(m[I * (I + 1) / 2 + J], X[J], acc);
+        X[I] = mfma4(m[I * (I + 1) / 2 + I], acc, rc_f32x4{0.f, 0.f, 0.f, 0.f});
       }
       if (is_v) {
         *reinterpret_cast<rc_f32x4*>(ws + sp.u() + (I * sp.vt + ct) * 256 + lane * 4) = X[I];
       } else {
-        float* w = ws + sp.w() + (I * sp.kt + ct) * 256;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) w[((x16 >> 2) * 16 + 4 * quarter + r) * 4 + (x16 & 3)] = X[I][r];
+        rc_f32x4 y = X[I];
+        transpose_quad(y, lane);
+        *reinterpret_cast<rc_f32x4*>(ws + sp.w() + (I * sp.kt + ct) * 256 + ((x16 >> 2) * 16 + 4 * quarter + (x16 & 3)) * 4) = y;
       }
     }
   }
@@ -910,33 +1137,115 @@ __global__ __launch_bounds__(kPrepThreads) void general_prep_kernel(socket_recur
   }
 }
 
-constexpr int kScanThreads = 256;
-constexpr int kScanWaves = 4;
+constexpr int kScanThreads = 512;
+constexpr int kScanWaves = 4;     // of either kind
 
-// The chunks of one (16 value columns, head, sequence) in order.  Wave w takes row block w of
-// U and O and state tiles w, w + 4, ...; U and S pass through LDS.  KT: 16-row state tiles.
+// The chunks of one (16 value columns, head, sequence) in order, by two kinds of waves, one of each on a SIMD:
+//  * wave w of the first four has state tiles w, w + 4, ... and, with the delta rule, row block w of U = Ubar - W S;
+//  * wave w of the others reads row block w out, O = Q^ S + Aqk U, which nothing later waits for.
+// S and (DELTA) U pass through LDS, S in two copies so that one is read while the next is written; without the delta
+// rule U is what the preparation left, and a chunk has one barrier instead of two.  KT: 16-row state tiles.
 // EXTRA: rule 1's additions to the read-outs and the state.
+// The chain state -> U -> state bounds it: its products are dependent, with an LDS exchange after each half.  Four waves
+// that did both, fragments one chunk ahead, took 245 us for 5000 tokens x 16 heads x 128 key channels with the delta rule and
+// 116 for 64 without; these 204 and 108 (eight waves alone 229 and 127, with fragments two chunks ahead 212 and 109, with a
+// chunk's state tiles asked for together and the first kind's products first the rest).  Two accumulators in turn for
+// every chain changed nothing.
 template <int KT, int NB, bool DELTA, bool EXTRA>
-__global__ __launch_bounds__(kScanThreads, 1) void recurrence_scan_kernel(socket_recurrence a, int n_chunks, int slices) {
+__global__ __launch_bounds__(kScanThreads, 2) void recurrence_scan_kernel(socket_recurrence a, int n_chunks) {
   constexpr int C = 16 * NB;
   constexpr int OWN = (KT + kScanWaves - 1) / kScanWaves;
-  __shared__ __attribute__((aligned(16))) float s_lds[KT * 256];
-  __shared__ __attribute__((aligned(16))) float u_lds[NB * 256];
+  __shared__ __attribute__((aligned(16))) float s_lds[2][KT * 256];
+  __shared__ __attribute__((aligned(16))) float u_lds[DELTA ? 1 : 2][NB * 256];
   // workgroups go to the XCDs round-robin by id: the slices of one (sequence, head) share an
   // XCD (whose L2 then serves their common W, Q^ and K^T) when the heads are a multiple of 8
   const int bh_n = a.B * a.H;
   const int slice = blockIdx.x / bh_n, bh = blockIdx.x % bh_n;
   const int h = bh % a.H, b = bh / a.H;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = id & (kScanWaves - 1);
+  const bool reads_out = id >= kScanWaves;
   const int x16 = lane & 15, quarter = lane >> 4;
   const ChunkSpace sp{(a.dk + 15) / 16, (a.dv + 15) / 16, NB, EXTRA};
   const int kt = sp.kt;
   const int col = 16 * slice + x16;
   const bool col_ok = col < a.dv;
-  float* Sg = a.state + (int64_t)bh * a.dk * a.dv;
+  const bool rows_mine = wave < NB;
+  const int wb = rows_mine ? wave : 0;
   const float* ws = (const float*)a.workspace + (int64_t)bh * n_chunks * sp.size();
-  (void)slices;
+  const uint32_t l4 = lane * 4;
+  auto tile = [&](const float* at) __attribute__((always_inline)) { return *reinterpret_cast<const float4*>(at + l4); };
+  auto acc_tile = [&](const float* at) __attribute__((always_inline)) { return *reinterpret_cast<const rc_f32x4*>(at + l4); };
+  // Loads return in the order of their requests, and a wait counts those made since: the first chunks' are made in the
+  // order in which the loop makes them (the compiler, left to itself, mixed them and waited in the loop for all).
+  auto in_order = [] __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
+  auto chunk_at = [&](int n) __attribute__((always_inline)) { return ws + (int64_t)min(n, n_chunks - 1) * sp.size(); };
+  // A fragment's registers take a later chunk's as soon as it has been used: every load has the time of two chunks to
+  // arrive (where registers hold two, one chunk otherwise).
+  constexpr int SETS = NB == 4 ? 2 : 1;
 
+  if (reads_out) {
+    float4 fq[SETS][KT], fa[SETS][NB];
+    rc_f32x4 fo[SETS] = {};
+    auto q_tile = [&](const float* c, int j) __attribute__((always_inline)) {
+      return tile(c + sp.q() + (wb * kt + (j < kt ? j : kt - 1)) * 256);     // (tiles past dk meet zero state)
+    };
+    auto a_tile = [&](const float* c, int J) __attribute__((always_inline)) {
+      return tile(c + sp.aqk() + (wb * NB + (J <= wb ? J : wb)) * 256);
+    };
+#pragma unroll
+    for (int p = 0; p < SETS; ++p) {
+      const float* c = chunk_at(p);
+#pragma unroll
+      for (int j = 0; j < KT; ++j) fq[p][j] = q_tile(c, j);
+      in_order();
+      if (EXTRA) fo[p] = acc_tile(c + sp.o() + (wb * sp.vt + slice) * 256);
+#pragma unroll
+      for (int J = 0; J < NB; ++J) fa[p][J] = a_tile(c, J);
+      in_order();
+    }
+    __syncthreads();   // the first state
+    auto chunk = [&](int n, auto half) __attribute__((always_inline)) {
+      constexpr int at = decltype(half)::value, p = at % SETS;
+      const float* nx = chunk_at(n + SETS);
+      const float* S = s_lds[at];
+      rc_f32x4 o = fo[p];
+      if (rows_mine) {
+        rc_f32x4 x[KT];
+#pragma unroll
+        for (int j = 0; j < KT; ++j) x[j] = acc_tile(S + j * 256);
+        __builtin_amdgcn_sched_barrier(0);     // (every tile asked for before the first product)
+#pragma unroll
+        for (int j = 0; j < KT; ++j) {
+          o = mfma4(fq[p][j], x[j], o);
+          fq[p][j] = q_tile(nx, j);
+        }
+        if (EXTRA) fo[p] = acc_tile(nx + sp.o() + (wb * sp.vt + slice) * 256);
+      }
+      if (DELTA) __syncthreads();   // U complete
+      if (rows_mine) {
+#pragma unroll
+        for (int J = 0; J < NB; ++J) {
+          if (J <= wave) o = mfma4(fa[p][J], acc_tile(u_lds[DELTA ? 0 : at] + J * 256), o);
+          fa[p][J] = a_tile(nx, J);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = n * C + 16 * wave + 4 * quarter + r;
+          if (t < a.n && col_ok) a.o_buf[(((int64_t)b * a.n + t) * a.H + h) * a.dv + col] = o[r];
+        }
+      }
+      __syncthreads();   // the next state complete, U and this one read
+    };
+    for (int n = 0; n + 1 < n_chunks; n += 2) {
+      chunk(n, std::integral_constant<int, 0>{});
+      chunk(n + 1, std::integral_constant<int, 1>{});
+    }
+    if (n_chunks & 1) chunk(n_chunks - 1, std::integral_constant<int, 0>{});
+    return;
+  }
+
+  float* Sg = a.state + (int64_t)bh * a.dk * a.dv;
   rc_f32x4 S[OWN];
 #pragma unroll
   for (int i = 0; i < OWN; ++i) {
@@ -949,96 +1258,111 @@ __global__ __launch_bounds__(kScanThreads, 1) void recurrence_scan_kernel(socket
         if (row < a.dk) S[i][r] = Sg[(int64_t)row * a.dv + col];
       }
     }
-    if (j < KT) *reinterpret_cast<rc_f32x4*>(s_lds + j * 256 + lane * 4) = S[i];
+    if (j < KT) {
+      *reinterpret_cast<rc_f32x4*>(s_lds[0] + j * 256 + lane * 4) = S[i];
+      if (j >= kt) *reinterpret_cast<rc_f32x4*>(s_lds[1] + j * 256 + lane * 4) = S[i];   // (zero, and written by nobody later)
+    }
   }
-  const bool rows_mine = wave < NB;
-  const int wb = rows_mine ? wave : 0;
-  float4 fw[DELTA ? KT : 1], fq[KT], fk[OWN][NB], fa[NB], fg[OWN];
-  rc_f32x4 fu, fo = {0.f, 0.f, 0.f, 0.f}, fs[EXTRA ? OWN : 1];
-  auto fetch = [&](int n) __attribute__((always_inline)) {
-    const float* c = ws + (int64_t)n * sp.size() + lane * 4;
-#pragma unroll
-    for (int j = 0; j < KT; ++j) {
-      const int jj = j < kt ? j : kt - 1;   // (tiles past dk meet zero state)
-      if (DELTA) fw[j] = *reinterpret_cast<const float4*>(c + sp.w() + (wb * kt + jj) * 256);
-      fq[j] = *reinterpret_cast<const float4*>(c + sp.q() + (wb * kt + jj) * 256);
-    }
-    fu = *reinterpret_cast<const rc_f32x4*>(c + sp.u() + (wb * sp.vt + slice) * 256);
-    if (EXTRA) fo = *reinterpret_cast<const rc_f32x4*>(c + sp.o() + (wb * sp.vt + slice) * 256);
-#pragma unroll
-    for (int J = 0; J < NB; ++J) fa[J] = *reinterpret_cast<const float4*>(c + sp.aqk() + (wb * NB + (J <= wb ? J : wb)) * 256);
-#pragma unroll
-    for (int i = 0; i < OWN; ++i) {
-      const int j = wave + i * kScanWaves, jj = j < kt ? j : kt - 1;
-#pragma unroll
-      for (int I = 0; I < NB; ++I) fk[i][I] = *reinterpret_cast<const float4*>(c + sp.kT() + (jj * NB + I) * 256);
-      fg[i] = *reinterpret_cast<const float4*>(ws + (int64_t)n * sp.size() + sp.gamma() + 16 * jj + 4 * quarter);
-      if (EXTRA) fs[i] = *reinterpret_cast<const rc_f32x4*>(c + sp.s() + (jj * sp.vt + slice) * 256);
-    }
+  float4 fw[SETS][DELTA ? KT : 1], fk[SETS][OWN][NB], fg[SETS][OWN];
+  rc_f32x4 fu[2], fs[SETS][EXTRA ? OWN : 1];
+  auto w_tile = [&](const float* c, int j) __attribute__((always_inline)) {
+    return tile(c + sp.w() + (wb * kt + (j < kt ? j : kt - 1)) * 256);
   };
-  fetch(0);
-  __syncthreads();
-  for (int n = 0; n < n_chunks; ++n) {
-    // a fragment's registers take the next chunk's as soon as it has been used: every load has
-    // about one chunk's time to arrive
-    const float* nx = ws + (int64_t)min(n + 1, n_chunks - 1) * sp.size() + lane * 4;
-    rc_f32x4 u = fu, o = fo, y = {0.f, 0.f, 0.f, 0.f};
+  auto own = [&](int i) __attribute__((always_inline)) { return min(wave + i * kScanWaves, kt - 1); };
+  auto k_tile = [&](const float* c, int i, int I) __attribute__((always_inline)) { return tile(c + sp.kT() + (own(i) * NB + I) * 256); };
+  auto gammas = [&](const float* c, int i) __attribute__((always_inline)) {
+    return *reinterpret_cast<const float4*>(c + sp.gamma() + 16 * own(i) + (uint32_t)(4 * quarter));
+  };
+  auto u_tile = [&](const float* c) __attribute__((always_inline)) { return acc_tile(c + sp.u() + (wb * sp.vt + slice) * 256); };
+  auto publish = [&](float* to, const rc_f32x4& u) __attribute__((always_inline)) {
+    if (rows_mine) *reinterpret_cast<rc_f32x4*>(to + wave * 256 + lane * 4) = u;
+  };
+  auto s_tile = [&](const float* c, int i) __attribute__((always_inline)) { return acc_tile(c + sp.s() + (own(i) * sp.vt + slice) * 256); };
 #pragma unroll
-    for (int j = 0; j < KT; ++j) {
-      const int jj = j < kt ? j : kt - 1;
-      const rc_f32x4 s = *reinterpret_cast<const rc_f32x4*>(s_lds + j * 256 + lane * 4);
-      if (DELTA) {
-        y = mfma4(fw[j], s, y);
-        fw[j] = *reinterpret_cast<const float4*>(nx + sp.w() + (wb * kt + jj) * 256);
-      }
-      o = mfma4(fq[j], s, o);
-      fq[j] = *reinterpret_cast<const float4*>(nx + sp.q() + (wb * kt + jj) * 256);
-    }
+  for (int p = 0; p < SETS; ++p) {
+    const float* c = chunk_at(p);
     if (DELTA) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) u[r] -= y[r];
+      for (int j = 0; j < KT; ++j) fw[p][j] = w_tile(c, j);
+      in_order();
     }
-    fu = *reinterpret_cast<const rc_f32x4*>(nx + sp.u() + (wb * sp.vt + slice) * 256);
-    if (EXTRA) fo = *reinterpret_cast<const rc_f32x4*>(nx + sp.o() + (wb * sp.vt + slice) * 256);
-    if (rows_mine) *reinterpret_cast<rc_f32x4*>(u_lds + wave * 256 + lane * 4) = u;
-    __syncthreads();   // U complete, S read by everyone
-    rc_f32x4 ub[NB];
-#pragma unroll
-    for (int I = 0; I < NB; ++I) ub[I] = *reinterpret_cast<const rc_f32x4*>(u_lds + I * 256 + lane * 4);
+    if (DELTA) fu[p] = u_tile(c);
+    in_order();
 #pragma unroll
     for (int i = 0; i < OWN; ++i) {
-      const int j = wave + i * kScanWaves, jj = j < kt ? j : kt - 1;
-      S[i][0] *= fg[i].x;
-      S[i][1] *= fg[i].y;
-      S[i][2] *= fg[i].z;
-      S[i][3] *= fg[i].w;
-      fg[i] = *reinterpret_cast<const float4*>(nx - lane * 4 + sp.gamma() + 16 * jj + 4 * quarter);
+      fg[p][i] = gammas(c, i);
+      if (EXTRA) fs[p][i] = s_tile(c, i);
+#pragma unroll
+      for (int I = 0; I < NB; ++I) fk[p][i][I] = k_tile(c, i, I);
+      in_order();
+    }
+  }
+  if (!DELTA) {
+    publish(u_lds[0], u_tile(ws));
+    fu[1] = u_tile(chunk_at(1));
+    fu[0] = u_tile(chunk_at(2));
+  }
+  __syncthreads();   // the first state
+  __builtin_amdgcn_s_setprio(1);   // (the other kind's products go where these leave the matrix core free)
+  auto chunk = [&](int n, auto half) __attribute__((always_inline)) {
+    constexpr int at = decltype(half)::value, p = at % SETS;
+    const float* nx = chunk_at(n + SETS);
+    const float* Sn = s_lds[at];
+    rc_f32x4 ub[NB];
+    if constexpr (DELTA) {
+      if (rows_mine) {
+        rc_f32x4 y = {0.f, 0.f, 0.f, 0.f}, x[KT];
+#pragma unroll
+        for (int j = 0; j < KT; ++j) x[j] = acc_tile(Sn + j * 256);
+        __builtin_amdgcn_sched_barrier(0);     // (every tile asked for before the first product)
+#pragma unroll
+        for (int j = 0; j < KT; ++j) {
+          y = mfma4(fw[p][j], x[j], y);
+          fw[p][j] = w_tile(nx, j);
+        }
+        rc_f32x4 u = fu[p];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) u[r] -= y[r];
+        publish(u_lds[0], u);
+        in_order();
+        fu[p] = u_tile(nx);
+      }
+      __syncthreads();   // U complete
+    } else {
+      // (U comes from memory: the next chunk's is laid down beside this one's)
+      publish(u_lds[DELTA ? 0 : at ^ 1], fu[at ^ 1]);
+      in_order();
+      fu[at ^ 1] = u_tile(chunk_at(n + 3));
+    }
+#pragma unroll
+    for (int I = 0; I < NB; ++I) ub[I] = acc_tile(u_lds[DELTA ? 0 : at] + I * 256);
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      const int j = wave + i * kScanWaves;
+      S[i][0] *= fg[p][i].x;
+      S[i][1] *= fg[p][i].y;
+      S[i][2] *= fg[p][i].z;
+      S[i][3] *= fg[p][i].w;
+      fg[p][i] = gammas(nx, i);
       if (EXTRA) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) S[i][r] += fs[i][r];
-        fs[i] = *reinterpret_cast<const rc_f32x4*>(nx + sp.s() + (jj * sp.vt + slice) * 256);
+        for (int r = 0; r < 4; ++r) S[i][r] += fs[p][i][r];
+        fs[p][i] = s_tile(nx, i);
       }
 #pragma unroll
       for (int I = 0; I < NB; ++I) {
-        S[i] = mfma4(fk[i][I], ub[I], S[i]);
-        fk[i][I] = *reinterpret_cast<const float4*>(nx + sp.kT() + (jj * NB + I) * 256);
+        S[i] = mfma4(fk[p][i][I], ub[I], S[i]);
+        fk[p][i][I] = k_tile(nx, i, I);
       }
-      if (j < kt) *reinterpret_cast<rc_f32x4*>(s_lds + j * 256 + lane * 4) = S[i];
+      if (j < kt) *reinterpret_cast<rc_f32x4*>(s_lds[at ^ 1] + j * 256 + lane * 4) = S[i];
     }
-    if (rows_mine) {
-#pragma unroll
-      for (int J = 0; J < NB; ++J) {
-        if (J <= wave) o = mfma4(fa[J], ub[J], o);
-        fa[J] = *reinterpret_cast<const float4*>(nx + sp.aqk() + (wb * NB + (J <= wb ? J : wb)) * 256);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = n * C + 16 * wave + 4 * quarter + r;
-        if (t < a.n && col_ok) a.o_buf[(((int64_t)b * a.n + t) * a.H + h) * a.dv + col] = o[r];
-      }
-    }
-    __syncthreads();   // S complete, U read by everyone
+    __syncthreads();   // the next state complete, U and this one read
+  };
+  for (int n = 0; n + 1 < n_chunks; n += 2) {
+    chunk(n, std::integral_constant<int, 0>{});
+    chunk(n + 1, std::integral_constant<int, 1>{});
   }
+  if (n_chunks & 1) chunk(n_chunks - 1, std::integral_constant<int, 0>{});
 #pragma unroll
   for (int i = 0; i < OWN; ++i) {
     const int j = wave + i * kScanWaves;
@@ -1171,19 +1495,30 @@ int launch_step(const socket_recurrence& a, hipStream_t s) {
   return SOCKET_OK;
 }
 
-template <class DT, int NB>
+template <class DT, int NB, bool DELTA>
 int launch_prep(const socket_recurrence& a, int n_chunks, bool vec, hipStream_t s) {
   constexpr int C = 16 * NB;
+  constexpr size_t kStatic = 64;
   const ChunkSpace sp{(a.dk + 15) / 16, (a.dv + 15) / 16, NB};
-  const int dkp = sp.kt * 16, kp = dkp + 4, vp = sp.vt * 16 + 4;
-  const size_t lds = (size_t)(C * (kp > vp ? kp : vp) + 2 * C * kp + NB * dkp + NB * NB * 256 + C) * 4;
-  SOCKET_REQUIRE(lds <= (size_t)socket_device_limits().max_lds_per_block, SOCKET_ERR_UNSUPPORTED);
-  auto kern = recurrence_prep_kernel<DT, NB>;
+  const int dkp = sp.kt * 16, dvp = sp.vt * 16, kp = dkp + 4, vp = dvp + 4;
+  const size_t limit = (size_t)socket_device_limits().max_lds_per_block;
+  const size_t fixed = (size_t)(C * kp + NB * dkp + C + (DELTA ? NB * NB * 256 : 0)) * 4, qk = (size_t)2 * C * kp * 4;
+  // what shares LDS with V once it is through: q, or q and k where nothing reads k after the fragments
+  const size_t over = (size_t)(DELTA ? C * kp : 2 * C * kp) * 4, v = (size_t)C * vp * 4;
+  const int own_v = DELTA && dvp <= kPrepThreads / C * 8 && fixed + qk + v + kStatic <= limit ? 1 : 0;
+  const size_t lds = fixed + qk + (own_v ? v : v > over ? v - over : 0);
+  SOCKET_REQUIRE(lds + kStatic <= limit, SOCKET_ERR_UNSUPPORTED);
+  auto kern = recurrence_prep_kernel<DT, NB, DELTA>;
   if (lds > 48 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return SOCKET_ERR_LAUNCH;
-  hipLaunchKernelGGL(kern, dim3((unsigned)n_chunks, (unsigned)a.H, (unsigned)a.B), dim3(kPrepThreads), lds, s, a, vec ? 1 : 0);
+  hipLaunchKernelGGL(kern, dim3((unsigned)a.H, (unsigned)n_chunks, (unsigned)a.B), dim3(kPrepThreads), lds, s, a, vec ? 1 : 0, own_v);
   return SOCKET_OK;
+}
+
+template <class DT, int NB>
+int launch_prep(const socket_recurrence& a, int n_chunks, bool vec, bool delta, hipStream_t s) {
+  return delta ? launch_prep<DT, NB, true>(a, n_chunks, vec, s) : launch_prep<DT, NB, false>(a, n_chunks, vec, s);
 }
 
 template <class DT, int NB>
@@ -1209,7 +1544,7 @@ template <int NB, bool DELTA, bool EXTRA = false>
 int launch_scan(const socket_recurrence& a, int n_chunks, hipStream_t s) {
   const int kt = (a.dk + 15) / 16, slices = (a.dv + 15) / 16;
   const dim3 grid((unsigned)((int64_t)slices * a.B * a.H)), block(kScanThreads);
-#define SOCKET_SCAN(KT) hipLaunchKernelGGL((recurrence_scan_kernel<KT, NB, DELTA, EXTRA>), grid, block, 0, s, a, n_chunks, slices)
+#define SOCKET_SCAN(KT) hipLaunchKernelGGL((recurrence_scan_kernel<KT, NB, DELTA, EXTRA>), grid, block, 0, s, a, n_chunks)
   if constexpr (NB == 4) {
     if (kt <= 2) SOCKET_SCAN(2);
     else if (kt <= 4) SOCKET_SCAN(4);
@@ -1271,9 +1606,9 @@ extern "C" int socket_recurrence_scan(const socket_recurrence* args, void* strea
       st = a.dtype == SOCKET_F32 ? launch_general_prep<DType_f32, 2>(a, n_chunks, vec, s)
                                  : launch_general_prep<DType_bf16, 2>(a, n_chunks, vec, s);
   } else if (nb == 4)
-    st = a.dtype == SOCKET_F32 ? launch_prep<DType_f32, 4>(a, n_chunks, vec, s) : launch_prep<DType_bf16, 4>(a, n_chunks, vec, s);
+    st = a.dtype == SOCKET_F32 ? launch_prep<DType_f32, 4>(a, n_chunks, vec, delta, s) : launch_prep<DType_bf16, 4>(a, n_chunks, vec, delta, s);
   else
-    st = a.dtype == SOCKET_F32 ? launch_prep<DType_f32, 2>(a, n_chunks, vec, s) : launch_prep<DType_bf16, 2>(a, n_chunks, vec, s);
+    st = a.dtype == SOCKET_F32 ? launch_prep<DType_f32, 2>(a, n_chunks, vec, delta, s) : launch_prep<DType_bf16, 2>(a, n_chunks, vec, delta, s);
   if (st != SOCKET_OK) return st;
   SOCKET_LAUNCH_CHECK();
   if (a.rule == 1) st = nb == 4 ? launch_scan<4, true, true>(a, n_chunks, s) : launch_scan<2, true, true>(a, n_chunks, s);
