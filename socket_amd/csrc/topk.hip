@@ -7,7 +7,7 @@
 // composite" is exactly "higher score, then lower index" and all composites of a
 // row are distinct.
 //
-// select_list_kernel, workgroups of 1024 lanes, selects in two ways:
+// select_list_kernel, workgroups of 1024 lanes (512 where rows outnumber the CUs), selects in two ways:
 //  * pooled: a superset of the row's m winners, at most kPoolCap composites, is
 //    formed and the m-th largest located in it by range refinement -- a 2048-bin
 //    LDS histogram over [lo, hi] (initially the pool's min / max, so the bins
@@ -214,11 +214,11 @@ __device__ __forceinline__ void wave_append(bool take, u64 value, int* cursor, u
 }
 
 // Bitonic sort of buf[0:np] (np a power of two) into descending order by the
-// whole 1024-lane workgroup.  Lane t owns elements [t*E, (t+1)*E): exchange
+// whole workgroup.  Lane t owns elements [t*E, (t+1)*E): exchange
 // distances below E stay in registers, below 64*E go through wave shuffles, and
 // only the longer ones through LDS with a barrier.  Callers sync before and get
 // a synced buffer back.
-template <int E>
+template <int E, int THREADS>
 __device__ __forceinline__ void sort_desc_impl(u64* buf, int np, int tid) {
   const bool active = tid * E < np;
   u64 r[E];
@@ -266,7 +266,7 @@ __device__ __forceinline__ void sort_desc_impl(u64* buf, int np, int tid) {
   __syncthreads();
   for (int k = 2 * span; k <= np; k <<= 1) {
     for (int j = k >> 1; j >= span; j >>= 1) {
-      for (int i = tid; i < np; i += kThreads) {
+      for (int i = tid; i < np; i += THREADS) {
         const int p = i ^ j;
         if (p > i) {
           const u64 a = buf[i], c = buf[p];
@@ -286,12 +286,13 @@ __device__ __forceinline__ void sort_desc_impl(u64* buf, int np, int tid) {
   }
 }
 
+template <int THREADS>
 __device__ __forceinline__ void sort_desc(u64* buf, int np, int tid) {
-  if (np <= kThreads) sort_desc_impl<1>(buf, np, tid);
-  else if (np == 2 * kThreads) sort_desc_impl<2>(buf, np, tid);
-  else if (np == 4 * kThreads) sort_desc_impl<4>(buf, np, tid);
-  else if (np == 8 * kThreads) sort_desc_impl<8>(buf, np, tid);
-  else sort_desc_impl<16>(buf, np, tid);
+  if (np <= THREADS) sort_desc_impl<1, THREADS>(buf, np, tid);
+  else if (np == 2 * THREADS) sort_desc_impl<2, THREADS>(buf, np, tid);
+  else if (np == 4 * THREADS) sort_desc_impl<4, THREADS>(buf, np, tid);
+  else if (np == 8 * THREADS) sort_desc_impl<8, THREADS>(buf, np, tid);
+  else sort_desc_impl<16, THREADS>(buf, np, tid);
 }
 
 __device__ __forceinline__ int next_pow2_dev(int x) {
@@ -361,9 +362,9 @@ __device__ __forceinline__ int range_shift(u64 lo, u64 hi) {
 // n_above + need winners are written in descending order at out[0:...).
 // Winners are placed by their level-0 bin (c - lo0) >> shift0 with counting ranks
 // when `counting_ok` (tmp then has 2 * cap_above slots) and no bin is crowded,
-// else by the bitonic sort.  All 1024 lanes; callers sync before; no barrier at
+// else by the bitonic sort.  All lanes; callers sync before; no barrier at
 // the end.
-template <bool MASKED>
+template <bool MASKED, int THREADS>
 __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand, int ncand, int need,
                                                 u64 lo0, int shift0, u64* tmp, uint32_t* hist,
                                                 SelectShared& sh, bool counting_ok, int32_t* out,
@@ -371,7 +372,7 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
   const int lane = tid & 63, wave = tid >> 6;
   // ---- the k-th bin: rank its entries, the best `need` follow the winners ----------
   if (ncand <= kMaxBinForCounting || need == ncand) {
-    for (int i = tid; i < ncand; i += kThreads) {
+    for (int i = tid; i < ncand; i += THREADS) {
       const u64 v = cand[i];
       int r = 0;
       for (int j = 0; j < ncand; ++j) r += cand[j] > v;
@@ -379,17 +380,17 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
     }
   } else {
     const int npc = next_pow2_dev(ncand);
-    for (int i = ncand + tid; i < npc; i += kThreads) cand[i] = 0ull;
+    for (int i = ncand + tid; i < npc; i += THREADS) cand[i] = 0ull;
     __syncthreads();
-    sort_desc(cand, npc, tid);
-    for (int i = tid; i < need; i += kThreads) out[n_above + i] = listed<MASKED>(composite_index(cand[i]), ok);
+    sort_desc<THREADS>(cand, npc, tid);
+    for (int i = tid; i < need; i += THREADS) out[n_above + i] = listed<MASKED>(composite_index(cand[i]), ok);
   }
   if (n_above == 0) return;
 
   // ---- winners above the bin ----------------------------------------------------------
   if (placed) {
     // `buf` holds them grouped by level-0 bin already, hist[bin] = offset | population << 16
-    for (int p = tid; p < n_above; p += kThreads) {
+    for (int p = tid; p < n_above; p += THREADS) {
       const u64 v = buf[p];
       const uint32_t h = hist[(int)((v - lo0) >> shift0)];
       const int s0 = (int)(h & 0xffffu), c = (int)(h >> 16);
@@ -400,41 +401,50 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
     return;
   }
   if (counting_ok) {
-    for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;
+    for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;
     __syncthreads();
-    for (int i = tid; i < n_above; i += kThreads) {
+    for (int i = tid; i < n_above; i += THREADS) {
       const int bin = (int)((buf[i] - lo0) >> shift0);
       const uint32_t slot = atomicAdd(&hist[bin], 1u);
       tmp[i] = ((u64)bin << 32) | slot;  // parked until the offsets are known
     }
     __syncthreads();
-    // descending exclusive scan over the bins, two per lane; crowded-bin check
-    const int b0 = kBins - 1 - 2 * tid, b1 = b0 - 1;
-    const int c0 = (int)hist[b0], c1 = (int)hist[b1];
-    const int incl_w = wave_incl_scan(c0 + c1, lane);
-    const int crowded = __any((c0 > kMaxBinForCounting || c1 > kMaxBinForCounting) ? 1 : 0);
+    // descending exclusive scan over the bins, PER per lane; crowded-bin check
+    constexpr int PER = kBins / THREADS;
+    int c[PER], mine = 0, full = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      c[i] = (int)hist[kBins - 1 - PER * tid - i];
+      mine += c[i];
+      full |= c[i] > kMaxBinForCounting;
+    }
+    const int incl_w = wave_incl_scan(mine, lane);
+    const int crowded = __any(full);
     if (lane == 63) sh.wsum[wave] = incl_w;
     if (lane == 0) sh.wflag[wave] = crowded;
     __syncthreads();
     int base = 0, any_crowded = 0;
-    for (int w = 0; w < kWaves; ++w) {
+    for (int w = 0; w < (THREADS / SOCKET_WAVE); ++w) {
       if (w < wave) base += sh.wsum[w];
       any_crowded |= sh.wflag[w];
     }
-    const int excl = base + incl_w - (c0 + c1);
+    int excl = base + incl_w - mine;
     __syncthreads();
     if (!any_crowded) {
-      hist[b0] = (uint32_t)excl | ((uint32_t)c0 << 16);  // offset | population << 16
-      hist[b1] = (uint32_t)(excl + c0) | ((uint32_t)c1 << 16);
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        hist[kBins - 1 - PER * tid - i] = (uint32_t)excl | ((uint32_t)c[i] << 16);  // offset | population << 16
+        excl += c[i];
+      }
       __syncthreads();
       u64* grouped = tmp + n_above;
-      for (int i = tid; i < n_above; i += kThreads) {
+      for (int i = tid; i < n_above; i += THREADS) {
         const int bin = (int)(tmp[i] >> 32);
         const int slot = (int)(tmp[i] & 0xffffffffull);
         grouped[(hist[bin] & 0xffffu) + slot] = buf[i];
       }
       __syncthreads();
-      for (int p = tid; p < n_above; p += kThreads) {
+      for (int p = tid; p < n_above; p += THREADS) {
         const u64 v = grouped[p];
         const uint32_t h = hist[(int)((v - lo0) >> shift0)];
         const int s0 = (int)(h & 0xffffu), c = (int)(h >> 16);
@@ -446,10 +456,10 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
     }
   }
   const int np = next_pow2_dev(n_above);
-  for (int i = n_above + tid; i < np; i += kThreads) buf[i] = 0ull;
+  for (int i = n_above + tid; i < np; i += THREADS) buf[i] = 0ull;
   __syncthreads();
-  sort_desc(buf, np, tid);
-  for (int j = tid; j < n_above; j += kThreads) out[j] = listed<MASKED>(composite_index(buf[j]), ok);
+  sort_desc<THREADS>(buf, np, tid);
+  for (int j = tid; j < n_above; j += THREADS) out[j] = listed<MASKED>(composite_index(buf[j]), ok);
 }
 
 // ---------------------------------------------------------------------------
@@ -569,14 +579,14 @@ __device__ __forceinline__ u64 load_coherent(const u64* p) {
 // row's list in `loc` (a stretch reserved with one atomic add on row_count), and
 // the last part to arrive (row_done) selects from that list; the others leave.
 // row_count and row_done are zero on entry and zero again on exit.
-// The pooled composites are held in registers, eight per lane, from the moment
+// The pooled composites are held in registers, kPoolCap / THREADS per lane, from the moment
 // the pool is complete; LDS holds them only while they are being compacted.
 // MASKED: a byte per score says whether its position may be listed; positions that may not become -1 in the list, and
 // their scores are minus infinity.  Those are kept out of the ranges that the histograms are laid over (they count in
 // the lowest bin): with them in, half the bins lie between minus infinity and the lowest score, and rows with a masked end
 // took two passes more (56 rows of 4135, part of each masked: 19.1 us against 8.9).
-template <bool MASKED>
-__global__ __launch_bounds__(kThreads) void select_list_kernel(
+template <bool MASKED, int THREADS>
+__global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
     const float* __restrict__ scores, const uint8_t* __restrict__ allowed, int64_t score_stride, const int32_t* __restrict__ lens,
     const int32_t* __restrict__ budgets, const uint32_t* __restrict__ row_range, int range_parts,
     int Hq, int T, int M, int sink, int window, int write_base, int32_t* __restrict__ sparse_list,
@@ -588,8 +598,11 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   u64* buf = reinterpret_cast<u64*>(lds_raw);  // winners                  [cap_above]
   u64* cand = buf + cap_above;                 // entries of the k-th bin  [kCandCap]
-  u64* pool = cand + kCandCap;                 // what passes the filter   [pool_slots]: kPoolCap for rows beyond that
-  u64* tmp = pool + pool_slots;                // counting placement       [2*cap_above] if counting_ok
+  // What passes the filter [pool_slots]: kPoolCap for rows beyond that.  In the half workgroup it lies over the rest,
+  // which nothing writes before every lane holds its entries of the pool in registers.
+  constexpr bool kPoolOver = THREADS < kThreads;
+  u64* pool = kPoolOver ? buf : cand + kCandCap;
+  u64* tmp = kPoolOver ? cand + kCandCap : pool + pool_slots;   // counting placement [2*cap_above] if counting_ok
 
   const int rowi = blockIdx.x / parts, part = blockIdx.x % parts;
   const int b = rowi / Hq;
@@ -603,7 +616,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
   const uint8_t* ok = MASKED ? allowed + (int64_t)rowi * T : nullptr;
   if (part == 0)
     write_list_base<MASKED>(out, n, m, nbase, sink, window, write_base, list_width,
-                            sparse_len ? sparse_len + rowi : nullptr, ok, tid, kThreads);
+                            sparse_len ? sparse_len + rowi : nullptr, ok, tid, THREADS);
   if (m == 0) return;
   int32_t* heavy = out + nbase;
 
@@ -619,13 +632,13 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
     }
     int total = -1;  // uniform; stays -1 when no pool could be formed
     uint32_t kmin = 0xffffffffu, kmax = 0u;  // key range of what this lane holds
-    constexpr int U = kPoolCap / kThreads;
-    u64 pv[U];                               // entry tid + u * kThreads of the pool
+    constexpr int U = kPoolCap / THREADS;
+    u64 pv[U];                               // entry tid + u * THREADS of the pool
     if (n <= kPoolCap) {  // the whole row, by one workgroup
       if (part != 0) return;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int i = tid + u * kThreads;
+        const int i = tid + u * THREADS;
         const uint32_t k = score_to_key(i < n ? row[i] : 0.f);
         if (i < n) {
           if (!MASKED || k > kMaskedKey) kmin = min(kmin, k);
@@ -634,7 +647,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         pv[u] = composite(k, i);
       }
       total = n;
-      for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;   // for the first refinement pass
+      for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;   // for the first refinement pass
       __syncthreads();
     } else if (sampling_ok(m)) {
       // This part's share of the row; the last part also takes the one to three
@@ -648,14 +661,13 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
       // worked out, each further one two batches ahead of the one being filtered.  A
       // wave counts what passes in its batch, reserves a stretch of the pool with
       // one LDS atomic and writes its entries there: no barrier in the loop.
-      constexpr int kLoads = 4, kStep = kThreads * 4 * kLoads;
-      static_assert(kStep == kBatch, "batch size");
+      constexpr int kLoads = 4, kStep = THREADS * 4 * kLoads;
       auto fetch = [&](int base, float4 (&x)[kLoads]) {
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
           // (past the end: the share's last four, fetched and ignored -- a load under
           // a condition would make every wait in the loop a wait for all loads)
-          const int i0 = max(min(base + (u * kThreads + tid) * 4, e4 - 4), 0);
+          const int i0 = max(min(base + (u * THREADS + tid) * 4, e4 - 4), 0);
           const f32x4_any v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_any*>(row + i0));
           x[u] = make_float4(v.x, v.y, v.z, v.w);
         }
@@ -677,7 +689,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
           const float xs[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
-          const bool in = FULL || base + (u * kThreads + tid) * 4 < e4;
+          const bool in = FULL || base + (u * THREADS + tid) * 4 < e4;
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
             mask[u * 4 + c] = __builtin_amdgcn_ballot_w64(in && !(xs[c] < tau_f));
@@ -693,7 +705,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
           const float xs[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
-          const bool in = FULL || base + (u * kThreads + tid) * 4 < e4;
+          const bool in = FULL || base + (u * THREADS + tid) * 4 < e4;
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
             const bool pass = in && !(xs[c] < tau_f);
@@ -705,7 +717,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
               // (a 64-bit store would first copy them into a register pair)
               const uint32_t addr = (uint32_t)(uintptr_t)(pool + slot);
               asm volatile("ds_write2_b32 %0, %1, %2 offset1:1"
-                           :: "v"(addr), "v"(cidx - (uint32_t)(u * kThreads * 4 + c)), "v"(__float_as_uint(xs[c]))
+                           :: "v"(addr), "v"(cidx - (uint32_t)(u * THREADS * 4 + c)), "v"(__float_as_uint(xs[c]))
                            : "memory");
             }
             at += __popcll(mk);
@@ -720,8 +732,8 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
       float4 b0[kLoads], b1[kLoads], b2[kLoads];
       fetch(begin, b0);
       fetch(begin + kStep, b1);
-      const uint32_t tau = sample_threshold<kThreads, MASKED>(row, n, m, hist, sh, tid);
-      for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;   // for the first refinement pass
+      const uint32_t tau = sample_threshold<THREADS, MASKED>(row, n, m, hist, sh, tid);
+      for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;   // for the first refinement pass
       const float tau_f = tau >= 0xff800000u ? INFINITY : tau <= 0x007fffffu ? -INFINITY
                           : __uint_as_float((tau & 0x80000000u) ? (tau & 0x7fffffffu) : ~tau);
       for (int base = begin; base < e4; base += 3 * kStep) {
@@ -748,7 +760,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         if (got >= m && got <= kPoolCap) {
 #pragma unroll
           for (int u = 0; u < U; ++u)
-            if (tid + u * kThreads < got) pv[u] = keyed(pool[tid + u * kThreads]);
+            if (tid + u * THREADS < got) pv[u] = keyed(pool[tid + u * THREADS]);
           total = got;
         }
       } else {
@@ -757,7 +769,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         const int at = sh.base;
         u64* mine = loc + (int64_t)rowi * kPoolCap;
         if (at + got <= kPoolCap) {   // (a row whose parts pass more than the list holds is redone from scratch)
-          for (int i = tid; i < got; i += kThreads) store_coherent(mine + at + i, keyed(pool[i]));
+          for (int i = tid; i < got; i += THREADS) store_coherent(mine + at + i, keyed(pool[i]));
         }
         // Every lane waits until its written-through stores have been acknowledged,
         // the barrier collects the lanes, and only then is the ticket drawn: whoever
@@ -773,14 +785,14 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         if (sum >= m && sum <= kPoolCap) {
 #pragma unroll
           for (int u = 0; u < U; ++u)
-            if (tid + u * kThreads < sum) pv[u] = load_coherent(mine + tid + u * kThreads);
+            if (tid + u * THREADS < sum) pv[u] = load_coherent(mine + tid + u * THREADS);
           total = sum;
         }
       }
       if (total >= 0) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          if (tid + u * kThreads < total) {
+          if (tid + u * THREADS < total) {
             const uint32_t k = (uint32_t)(pv[u] >> 32);
             if (!MASKED || k > kMaskedKey) kmin = min(kmin, k);
             kmax = max(kmax, k);
@@ -814,13 +826,13 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         for (int u = 0; u < U / 2; ++u) slot2[u] = 0;   // (hist is zero: cleared ahead of the pool)
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          if (tid + u * kThreads < total) {
+          if (tid + u * THREADS < total) {
             const uint32_t sl = atomicAdd(&hist[bin0(pv[u])], 1u);
             slot2[u >> 1] |= sl << (16 * (u & 1));
           }
         }
         __syncthreads();
-        find_bin<kThreads, true>(hist, m, 1, sh, tid, [&](int bin, int before, int count) {
+        find_bin<THREADS, true>(hist, m, 1, sh, tid, [&](int bin, int before, int count) {
           const u64 blo = lo0 + ((u64)bin << shift0);
           const u64 bspan = (shift0 == 0) ? 0ull : ((1ull << shift0) - 1ull);
           sh.lo = MASKED && bin == 0 ? 0ull : blo;
@@ -832,7 +844,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
           const int fb = sh.found_bin, need = sh.need, ncand = min(sh.found_count, kCandCap);
 #pragma unroll
           for (int u = 0; u < U; ++u) {
-            if (tid + u * kThreads < total) {
+            if (tid + u * THREADS < total) {
               const u64 v = pv[u];
               const int bin = bin0(v);
               const int sl = (int)((slot2[u >> 1] >> (16 * (u & 1))) & 0xffffu);
@@ -841,7 +853,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
             }
           }
           __syncthreads();
-          order_and_write<MASKED>(buf, m - need, cand, ncand, need, lo0, shift0, tmp, hist, sh, counting_ok != 0, heavy,
+          order_and_write<MASKED, THREADS>(buf, m - need, cand, ncand, need, lo0, shift0, tmp, hist, sh, counting_ok != 0, heavy,
                           ok, tid, true);
           return;
         }
@@ -850,15 +862,15 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
         const u64 lo = sh.lo, hi = sh.hi;
         const int need_in = sh.need;
         const int shift = range_shift(lo, hi);
-        for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;
+        for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const u64 v = pv[u];
-          if (tid + u * kThreads < total && v >= lo && v <= hi) atomicAdd(&hist[(int)((v - lo) >> shift)], 1u);
+          if (tid + u * THREADS < total && v >= lo && v <= hi) atomicAdd(&hist[(int)((v - lo) >> shift)], 1u);
         }
         __syncthreads();
-        find_bin<kThreads>(hist, need_in, 1, sh, tid);
+        find_bin<THREADS>(hist, need_in, 1, sh, tid);
         if (tid == 0) {
           const u64 blo = lo + ((u64)sh.found_bin << shift);
           const u64 bspan = (shift == 0) ? 0ull : ((1ull << shift) - 1ull);
@@ -875,12 +887,12 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const u64 v = pv[u];
-        const bool have = tid + u * kThreads < total;
+        const bool have = tid + u * THREADS < total;
         wave_append(have && v > bhi, v, &sh.fill_above, buf, cap_above);
         wave_append(have && v >= blo && v <= bhi, v, &sh.fill_cand, cand, kCandCap);
       }
       __syncthreads();
-      order_and_write<MASKED>(buf, m - need, cand, min(sh.fill_cand, kCandCap), need, lo0, shift0, tmp, hist, sh,
+      order_and_write<MASKED, THREADS>(buf, m - need, cand, min(sh.fill_cand, kCandCap), need, lo0, shift0, tmp, hist, sh,
                       counting_ok != 0, heavy, ok, tid);
       return;
     }
@@ -894,12 +906,12 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
     uint32_t kmin = 0xffffffffu, kmax = 0u;
     if (row_range) {
       const uint32_t* rr = row_range + (int64_t)rowi * range_parts * 2;
-      for (int i = tid; i < range_parts; i += kThreads) {
+      for (int i = tid; i < range_parts; i += THREADS) {
         kmin = min(kmin, rr[2 * i]);
         kmax = max(kmax, rr[2 * i + 1]);
       }
     } else {
-      for_each_in<kThreads>(row, 0, n, tid, [&](int, float x) {
+      for_each_in<THREADS>(row, 0, n, tid, [&](int, float x) {
         const uint32_t k = score_to_key(x);
         kmin = min(kmin, k);
         kmax = max(kmax, k);
@@ -914,7 +926,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
     if (tid == 0) {
       kmin = 0xffffffffu;
       kmax = 0u;
-      for (int w = 0; w < kWaves; ++w) {
+      for (int w = 0; w < (THREADS / SOCKET_WAVE); ++w) {
         kmin = min(kmin, (uint32_t)sh.wmin[w]);
         kmax = max(kmax, (uint32_t)sh.wmax[w]);
       }
@@ -936,14 +948,14 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
     const uint32_t lo = (uint32_t)sh.lo, hi = (uint32_t)sh.hi;
     const int need_in = sh.need;
     const int shift = range_shift(lo, hi);
-    for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;
+    for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;
     __syncthreads();
-    for_each_in<kThreads>(row, 0, n, tid, [&](int, float x) {
+    for_each_in<THREADS>(row, 0, n, tid, [&](int, float x) {
       const uint32_t k = score_to_key(x);
       if (k >= lo && k <= hi) atomicAdd(&hist[(k - lo) >> shift], 1u);
     });
     __syncthreads();
-    find_bin<kThreads>(hist, need_in, 1, sh, tid);
+    find_bin<THREADS>(hist, need_in, 1, sh, tid);
     if (tid == 0) {
       const uint32_t blo = lo + ((uint32_t)sh.found_bin << shift);
       const uint32_t bspan = (shift == 0) ? 0u : ((1u << shift) - 1u);
@@ -966,13 +978,13 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
     // Take the `need` lowest indices among the keys equal to blo: histogram over
     // index ranges, then an in-order walk of the one range that straddles.
     const int binw = (n + kBins - 1) / kBins;
-    for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;
+    for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;
     __syncthreads();
-    for_each_in<kThreads>(row, 0, n, tid, [&](int i, float x) {
+    for_each_in<THREADS>(row, 0, n, tid, [&](int i, float x) {
       if (score_to_key(x) == blo) atomicAdd(&hist[i / binw], 1u);
     });
     __syncthreads();
-    find_bin<kThreads>(hist, need, 0, sh, tid);
+    find_bin<THREADS>(hist, need, 0, sh, tid);
     if (wave == 0) {
       int rest = need - sh.found_before;  // >= 1 ties to take inside this index range
       const int i0 = sh.found_bin * binw, i1 = min(n, i0 + binw);
@@ -998,7 +1010,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
 
   // ---- collect ------------------------------------------------------------------
   const int idx_star = sh.idx_star;
-  for_each_in<kThreads>(row, 0, n, tid, [&](int i, float x) {
+  for_each_in<THREADS>(row, 0, n, tid, [&](int i, float x) {
     const uint32_t k = score_to_key(x);
     const u64 v = composite(k, i);
     const bool in_bin = k >= blo && k <= bhi;
@@ -1011,7 +1023,7 @@ __global__ __launch_bounds__(kThreads) void select_list_kernel(
   // mass ties: all m winners are in buf and there are no candidates
   const int ncand = mass_ties ? 0 : min(sh.fill_cand, kCandCap);
   const int n_above = mass_ties ? m : m - need;
-  order_and_write<MASKED>(buf, n_above, cand, ncand, mass_ties ? 0 : need, (u64)lo0 << 32, shift0 + 32, tmp, hist,
+  order_and_write<MASKED, THREADS>(buf, n_above, cand, ncand, mass_ties ? 0 : need, (u64)lo0 << 32, shift0 + 32, tmp, hist,
                   sh, counting_ok != 0, heavy, ok, tid);
 }
 
@@ -1128,12 +1140,20 @@ int select_entry(const float* scores, const uint8_t* allowed, int64_t score_stri
   }
   SOCKET_REQUIRE((int64_t)rows * parts <= 0x7fffffff, SOCKET_ERR_SHAPE);
 
-  auto kern = allowed ? select_list_kernel<true> : select_list_kernel<false>;
+  // More rows than CUs: workgroups of half the lanes, and so little LDS that a CU holds two of them, so that one's
+  // barriers and waits are the other's work and no last round leaves most CUs idle.  Whole / half workgroups, us: 260 rows
+  // of 65536 33.1 / 26.9, 264 of 131072 53.0 / 47.0, 288 of 12000 21.3 / 14.9, 320 of 32768 25.7 / 19.7, 448 of 16384 to
+  // 98304 40.3 / 36.6, 512 of 32768 28.3 / 20.2, 2048 of up to 20000 81.3 / 54.8.  Rows that all have a CU to themselves
+  // keep its 16 waves; budgets past 2048 need more LDS than half of a CU's.
+  const bool half = pool_slots > 0 && parts == 1 && rows > lim.cu_count && 3 * cap_above + kCandCap <= kPoolCap;
+  if (half) lds = (size_t)kPoolCap * sizeof(u64);
+  auto kern = half ? (allowed ? select_list_kernel<true, kThreads / 2> : select_list_kernel<false, kThreads / 2>)
+                   : (allowed ? select_list_kernel<true, kThreads> : select_list_kernel<false, kThreads>);
   if (lds > 32 * 1024 &&
       hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return SOCKET_ERR_LAUNCH;
-  hipLaunchKernelGGL(kern, dim3(rows * parts), dim3(kThreads), lds, s, scores, allowed, score_stride, lens, budgets,
+  hipLaunchKernelGGL(kern, dim3(rows * parts), dim3(half ? kThreads / 2 : kThreads), lds, s, scores, allowed, score_stride, lens, budgets,
                      row_range, range_parts, Hq, T, M, sink, window, write_base, sparse_list,
                      list_stride, list_width, sparse_len, cap_above, counting_ok, use_pool, pool_slots, parts,
                      loc, row_count, row_done);
