@@ -1143,10 +1143,11 @@ int select_entry(const float* scores, const uint8_t* allowed, int64_t score_stri
   // More rows than CUs: workgroups of half the lanes, and so little LDS that a CU holds two of them, so that one's
   // barriers and waits are the other's work and no last round leaves most CUs idle.  Whole / half workgroups, us: 260 rows
   // of 65536 33.1 / 26.9, 264 of 131072 53.0 / 47.0, 288 of 12000 21.3 / 14.9, 320 of 32768 25.7 / 19.7, 448 of 16384 to
-  // 98304 40.3 / 36.6, 512 of 32768 28.3 / 20.2, 2048 of up to 20000 81.3 / 54.8.  Rows that all have a CU to themselves
-  // keep its 16 waves; budgets past 2048 need more LDS than half of a CU's.
-  const bool half = pool_slots > 0 && parts == 1 && rows > lim.cu_count && 3 * cap_above + kCandCap <= kPoolCap;
-  if (half) lds = (size_t)kPoolCap * sizeof(u64);
+  // 98304 40.3 / 36.6, 512 of 32768 28.3 / 20.2, 2048 of up to 20000 81.3 / 54.8; rows pooled whole, 448 of 3000 12.6 / 9.0,
+  // 512 of 4096 13.2 / 9.4, 512 of 8192 16.6 / 12.7, 1280 of 2000 28.2 / 18.8.  Rows that all have a CU to themselves keep
+  // its 16 waves (32 to 256 of 4096: 7.0 to 7.3 / 7.3 to 7.5); budgets past 2048 need more LDS than half of a CU's.
+  const bool half = use_pool && parts == 1 && rows > lim.cu_count && 3 * cap_above + kCandCap <= kPoolCap;
+  if (half && pool_slots > 0) lds = (size_t)kPoolCap * sizeof(u64);
   auto kern = half ? (allowed ? select_list_kernel<true, kThreads / 2> : select_list_kernel<false, kThreads / 2>)
                    : (allowed ? select_list_kernel<true, kThreads> : select_list_kernel<false, kThreads>);
   if (lds > 32 * 1024 &&

@@ -23,7 +23,7 @@ def _scores(kind, rows, T, g, dev):
 
 
 @pytest.mark.parametrize("extra", [1, 300])
-@pytest.mark.parametrize("T,M", [(8193, 1), (8200, 2048), (9001, 129), (20003, 2048), (20000, 2049), (33333, 700)])
+@pytest.mark.parametrize("T,M", [(37, 5), (4096, 300), (8192, 2048), (8193, 1), (8200, 2048), (9001, 129), (20003, 2048), (20000, 2049), (33333, 700)])
 @pytest.mark.parametrize("kind", ["plain", "ties", "one_value", "misled", "extremes"])
 def test_more_rows_than_cus(dev, kind, T, M, extra):
     from socket_amd import sparse
