@@ -17,8 +17,8 @@
 // strong decay.  Tokens are grouped in blocks of 16 with sums pl local to the block and
 // block totals tot; for s in an earlier block the exponent splits at the start of t's
 // block into two parts that are both <= 0.  Inside a block the split at the block's
-// start is used while its total stays above kMildDecay, else those at the middle of ever smaller
-// groups of rows, where both parts are <= 0 again.
+// start is used while its total stays above kMildDecay, else the exponent is taken per
+// pair on the vector ALU.
 //
 // All products are v_mfma_f32_16x16x4_f32 (fp32 operands).  Its operands hold one k index
 // per lane quarter; a step r of four takes k = 4 * quarter + r of a 16-wide tile, so that
@@ -497,6 +497,29 @@ __device__ __forceinline__ void conv_inputs(const socket_recurrence& a, int b, i
     for (int e = 0; e < 8; ++e) out[s][e] *= sigmoid_f32(out[s][e]);
 }
 
+// Sum of the squares of a token's channels, eight consecutive ones in each of its LPR lanes, in the order in which a wave
+// of one channel a lane adds them: channels 64 apart one after the other, then the butterfly, whose first three steps are
+// inside a lane.
+template <int LPR>
+__device__ __forceinline__ float sum_of_squares(const float (&x)[8], int lane) {
+  static_assert(LPR == 16 || LPR == 32, "128 or 256 channels");
+  float s[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float other = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x[e]), 0x128, 0xf, 0xf, false));   // row_ror:8
+    const float low = lane & 8 ? other : x[e], high = lane & 8 ? x[e] : other;
+    if constexpr (LPR == 16) {
+      s[e] = fmaf(high, high, low * low);
+    } else {
+      const float low2 = lane_xor16(low), high2 = lane_xor16(high);
+      const bool upper = lane & 16;
+      const float c0 = upper ? low2 : low, c1 = upper ? high2 : high, c2 = upper ? low : low2, c3 = upper ? high : high2;
+      s[e] = fmaf(c3, c3, fmaf(c2, c2, fmaf(c1, c1, c0 * c0)));
+    }
+  }
+  return group_sum<8>(((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])));
+}
+
 // Lane j of every four lanes gives x[c] of lane c: x[c] becomes what lane c held at j.
 __device__ __forceinline__ void transpose_quad(rc_f32x4& x, int lane) {
   const bool odd = lane & 1, high = lane & 2;
@@ -517,7 +540,9 @@ __device__ __forceinline__ void transpose_quad(rc_f32x4& x, int lane) {
 // One workgroup per (chunk, head, sequence).  With 16 waves on a CU and one such workgroup (three operands and the
 // tiles in LDS) nothing but the waves themselves hides a wait, so each phase asks for all it reads before it uses any:
 //  * a lane's eight channels of q, k and v with all their taps, and its eight decays, in one trip to memory; unit
-//    norms from those registers, running sums of the decays over 8 rows of a lane and a lane 32 further on;
+//    norms from those registers, running sums of the decays over 8 rows of a lane and, from its sum on, a lane 32 further
+//    on.  (Both halves summed from zero and the first one's sum added to each entry of the second rounds every entry at the
+//    full sum's magnitude twice: states up to four times as far from float64, 6.8e-7 where this gives 1.7e-7.);
 //  * the tiles of Aqk and L (a diagonal tile inverted by its own wave) and the fragments of Q^ and K^T are dealt out
 //    by a counter, the long ones first;
 //  * the forward substitution has its tiles in registers before it starts, and W leaves in 16-byte stores.
@@ -609,18 +634,14 @@ __global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_re
         x[2][e] = DELTA && own_v && c < dvp ? vs[r * vp + c + e] : 0.f;
       }
     }
-    float sq[2] = {0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < N; ++s)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        x[s][e] = row_ok && c < width[s] ? x[s][e] : 0.f;
-        if (s < 2) sq[s] = fmaf(x[s][e], x[s][e], sq[s]);
-      }
+      for (int e = 0; e < 8; ++e) x[s][e] = row_ok && c < width[s] ? x[s][e] : 0.f;
     float mul[2] = {a.q_scale, 1.f};
     if (a.unit_qk) {
-      mul[0] *= rsqrt_f32(group_sum<LPR>(sq[0]) + 1e-6f);
-      mul[1] = rsqrt_f32(group_sum<LPR>(sq[1]) + 1e-6f);
+      mul[0] *= rsqrt_f32(sum_of_squares<LPR>(x[0], lane) + 1e-6f);
+      mul[1] = rsqrt_f32(sum_of_squares<LPR>(x[1], lane) + 1e-6f);
     }
     auto put = [&](float* to, const float* y, float m) __attribute__((always_inline)) {
       *reinterpret_cast<float4*>(to) = make_float4(y[0] * m, y[1] * m, y[2] * m, y[3] * m);
@@ -637,17 +658,22 @@ __global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_re
     if (g != wave) request_decays(g);
     const int blk = g / spans, c = (g - blk * spans) * 32 + (lane & 31), r0 = 16 * blk + 8 * (lane >> 5);
     const float bias = a.decay_bias && c < dk ? a.decay_bias[h * dk + c] : 0.f;
-    float sum = 0.f;
+    // (a block's sixteen rows are summed one after the other: the upper half's lanes go on from the lower half's sum)
+    float half = 0.f;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      sum += r0 + r < n_rows && c < dk ? log2_decay(a, a_exp, z[r] + bias) : 0.f;
-      z[r] = sum;
+      z[r] = r0 + r < n_rows && c < dk ? log2_decay(a, a_exp, z[r] + bias) : 0.f;
+      half += z[r];
     }
-    const float first = lane_xor32(sum), before = lane < 32 ? 0.f : first;
+    const float before = lane_xor32(half);
+    float sum = lane < 32 ? 0.f : before;
     if (c < dkp) {
 #pragma unroll
-      for (int r = 0; r < 8; ++r) pl[(r0 + r) * kp + c] = z[r] + before;
-      if (lane >= 32) tot[blk * dkp + c] = sum + before;
+      for (int r = 0; r < 8; ++r) {
+        sum += z[r];
+        pl[(r0 + r) * kp + c] = sum;
+      }
+      if (lane >= 32) tot[blk * dkp + c] = sum;
     }
   }
   if (tid < C)
@@ -704,43 +730,28 @@ __global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_re
         if (DELTA) ak = mfma4(kk, rc_f32x4{kt.x * f.x, kt.y * f.y, kt.z * f.z, kt.w * f.w}, ak);
       }
     } else {
-      // Strong decay inside the block: rows in groups of 2 n (n = 8, 4, 2, 1), the exponent split at the last row of
-      // a group's first half.  Both parts are <= 0 for a token of the second half and a key of the first; the others
-      // are taken as zero.  Token t and key s are in different halves of one group for the n that is the highest bit
-      // of t ^ s, and that product is the one kept; t = s has no exponent.  (A pair at a time on the vector ALU took the
-      // workgroup 26000 cycles more than mild tiles; this 11000.)
-      rc_f32x4 lq[5], lkk[4];
-#pragma unroll
-      for (int v = 0; v < 5; ++v) {
-        lq[v] = rc_f32x4{0.f, 0.f, 0.f, 0.f};
-        if (v < 4) lkk[v] = rc_f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-      for (int j = 0; j < sp.kt; ++j) {
-        const int c = 16 * j + 4 * quarter;
-        const float4 k = *reinterpret_cast<const float4*>(ks + t * kp + c);
-        const float4 q = *reinterpret_cast<const float4*>(qs + t * kp + c);
+      // Strong decay inside the block: four channels of the rows at a time.  (16 heads x 5000 tokens with every tile such a
+      // one: 393 us for the branch, 390 with mild tiles; five matrix products split at the middle of ever smaller groups of
+      // rows are no faster.)
+      for (int c = 0; c < dkp; c += 4) {
         const float4 p = *reinterpret_cast<const float4*>(pl + t * kp + c);
+        const float4 q = *reinterpret_cast<const float4*>(qs + t * kp + c);
+        float4 kt = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (DELTA) kt = *reinterpret_cast<const float4*>(ks + t * kp + c);
+        float4 k[4], ps[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int n = 1 << v;
-          const bool second = x16 & n;
-          const float4 ref = *reinterpret_cast<const float4*>(pl + (16 * I + (x16 & ~(2 * n - 1)) + n - 1) * kp + c);
-          const float sign = second ? 1.f : -1.f;
-          const float4 f = make_float4(exp2_fast(fminf(sign * (p.x - ref.x), 0.f)), exp2_fast(fminf(sign * (p.y - ref.y), 0.f)),
-                                       exp2_fast(fminf(sign * (p.z - ref.z), 0.f)), exp2_fast(fminf(sign * (p.w - ref.w), 0.f)));
-          const float4 key = second ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(k.x * f.x, k.y * f.y, k.z * f.z, k.w * f.w);
-          const float one = second ? 1.f : 0.f;
-          const rc_f32x4 g = {f.x * one, f.y * one, f.z * one, f.w * one};
-          lq[v] = mfma4(key, rc_f32x4{q.x * g[0], q.y * g[1], q.z * g[2], q.w * g[3]}, lq[v]);
-          if (DELTA) lkk[v] = mfma4(key, rc_f32x4{k.x * g[0], k.y * g[1], k.z * g[2], k.w * g[3]}, lkk[v]);
+        for (int r = 0; r < 4; ++r) {
+          k[r] = *reinterpret_cast<const float4*>(ks + (16 * J + 4 * quarter + r) * kp + c);
+          ps[r] = *reinterpret_cast<const float4*>(pl + (16 * J + 4 * quarter + r) * kp + c);
         }
-        lq[4] = mfma4(k, rc_f32x4{q.x, q.y, q.z, q.w}, lq[4]);
-      }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int apart = x16 ^ (4 * quarter + r);
-        aq[r] = apart >= 8 ? lq[3][r] : apart >= 4 ? lq[2][r] : apart >= 2 ? lq[1][r] : apart ? lq[0][r] : lq[4][r];
-        ak[r] = apart >= 8 ? lkk[3][r] : apart >= 4 ? lkk[2][r] : apart >= 2 ? lkk[1][r] : lkk[0][r];
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float w = (&k[r].x)[e] * exp2_fast(fminf((&p.x)[e] - (&ps[r].x)[e], 0.f));
+            aq[r] = fmaf((&q.x)[e], w, aq[r]);
+            if (DELTA) ak[r] = fmaf((&kt.x)[e], w, ak[r]);
+          }
       }
     }
     const float bt = DELTA ? beta[t] : 0.f;

@@ -1,6 +1,6 @@
 """Chunked recurrences where the preparation and the scan take another branch: odd and even numbers of chunks and a rest
-beside full ones, V in LDS by itself or over what has been used, decays so strong that a diagonal tile is split at every
-level, an odd number of state tiles."""
+beside full ones, V in LDS by itself or over what has been used, decays so strong that a diagonal tile takes its
+exponents pair by pair, an odd number of state tiles."""
 import pytest
 import torch
 
