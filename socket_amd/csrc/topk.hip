@@ -357,10 +357,18 @@ __device__ __forceinline__ int range_shift(u64 lo, u64 hi) {
   return bits > 11 ? bits - 11 : 0;
 }
 
+// Bin of a composite in the histogram that starts at lo0.  Where positions may be masked it starts at the lowest one
+// that is not: the others lie below it, and every place that bins counts them in the lowest bin (a difference that wraps is
+// no bin, and there can be thousands of them above the m-th entry of a row that has fewer allowed positions than m).
+template <bool MASKED>
+__device__ __forceinline__ int level0_bin(u64 v, u64 lo0, int shift0) {
+  return MASKED && v < lo0 ? 0 : (int)((v - lo0) >> shift0);
+}
+
 // Final step of both paths.  buf[0:n_above) holds the winners above the k-th
 // bin, cand[0:ncand) the k-th bin's entries of which the best `need` win; the
 // n_above + need winners are written in descending order at out[0:...).
-// Winners are placed by their level-0 bin (c - lo0) >> shift0 with counting ranks
+// Winners are placed by their level-0 bin with counting ranks
 // when `counting_ok` (tmp then has 2 * cap_above slots) and no bin is crowded,
 // else by the bitonic sort.  All lanes; callers sync before; no barrier at
 // the end.
@@ -392,7 +400,7 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
     // `buf` holds them grouped by level-0 bin already, hist[bin] = offset | population << 16
     for (int p = tid; p < n_above; p += THREADS) {
       const u64 v = buf[p];
-      const uint32_t h = hist[(int)((v - lo0) >> shift0)];
+      const uint32_t h = hist[level0_bin<MASKED>(v, lo0, shift0)];
       const int s0 = (int)(h & 0xffffu), c = (int)(h >> 16);
       int r = 0;
       for (int q = s0; q < s0 + c; ++q) r += buf[q] > v;
@@ -404,7 +412,7 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
     for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;
     __syncthreads();
     for (int i = tid; i < n_above; i += THREADS) {
-      const int bin = (int)((buf[i] - lo0) >> shift0);
+      const int bin = level0_bin<MASKED>(buf[i], lo0, shift0);
       const uint32_t slot = atomicAdd(&hist[bin], 1u);
       tmp[i] = ((u64)bin << 32) | slot;  // parked until the offsets are known
     }
@@ -446,7 +454,7 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
       __syncthreads();
       for (int p = tid; p < n_above; p += THREADS) {
         const u64 v = grouped[p];
-        const uint32_t h = hist[(int)((v - lo0) >> shift0)];
+        const uint32_t h = hist[level0_bin<MASKED>(v, lo0, shift0)];
         const int s0 = (int)(h & 0xffffu), c = (int)(h >> 16);
         int r = 0;
         for (int q = s0; q < s0 + c; ++q) r += grouped[q] > v;
@@ -812,7 +820,6 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
       __syncthreads();
       const u64 lo0 = (u64)(MASKED ? min(sh.kmin, sh.kmax) : sh.kmin) << 32, hi0 = ((u64)sh.kmax << 32) | 0xffffffffull;
       const int shift0 = range_shift(lo0, hi0);
-      auto bin0 = [&](u64 v) { return MASKED && v < lo0 ? 0 : (int)((v - lo0) >> shift0); };
       // refinement on the composites; they are distinct, so it ends with a bin of
       // at most kCandCap entries (ties need no special case here).
       // The first pass covers every entry, and every entry keeps the slot that its
@@ -827,7 +834,7 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           if (tid + u * THREADS < total) {
-            const uint32_t sl = atomicAdd(&hist[bin0(pv[u])], 1u);
+            const uint32_t sl = atomicAdd(&hist[level0_bin<MASKED>(pv[u], lo0, shift0)], 1u);
             slot2[u >> 1] |= sl << (16 * (u & 1));
           }
         }
@@ -846,7 +853,7 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
           for (int u = 0; u < U; ++u) {
             if (tid + u * THREADS < total) {
               const u64 v = pv[u];
-              const int bin = bin0(v);
+              const int bin = level0_bin<MASKED>(v, lo0, shift0);
               const int sl = (int)((slot2[u >> 1] >> (16 * (u & 1))) & 0xffffu);
               if (bin > fb) buf[(int)(hist[bin] & 0xffffu) + sl] = v;
               else if (bin == fb && sl < kCandCap) cand[sl] = v;
