@@ -345,9 +345,9 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
 }
 
 // The rest of a row [sink | window | heavy] whose heavy entries are in place: the sink and window positions
-// (the last position if there are none), -1 for every position that is not allowed, and the length.  A workgroup takes
-// kFinishEntries of a row: lists are seldom longer, but a window may be (100000 positions x 32 rows, the whole operator:
-// 46 us, 190 with a workgroup to a row, where torch's arange, gather and concatenation make it 128).
+// (the last position if there are none), -1 for every position that is not allowed, and the length.  For rows whose
+// window is long (the others are written by the selection's launch): a workgroup takes kFinishEntries of a row.  100000
+// positions x 32 rows, the whole operator over four small tables: 39 us, 61 with one workgroup of the selection's launch to a row.
 constexpr int kFinishEntries = 4096;
 
 __global__ __launch_bounds__(256) void finish_list_kernel(int32_t* __restrict__ list, int32_t* __restrict__ list_len,

@@ -144,9 +144,16 @@ def _select_into(scores, sink: int, window: int, M: int, lens, budgets, write_ba
         raise
 
 
+# Entries of a row's sink and window from which they are a launch of their own, dealt out over several workgroups.  In
+# the selection's launch one workgroup of a row writes them: no launch more, but 25 us per 100000 entries.  The whole operator
+# over four small tables, us, in the selection's launch / in its own: 32 rows, 16000 entries 21.3 / 22.4, 32768 25.1 / 23.0, 100000 61
+# / 39; 4 rows, 16000 20.1 / 21.7, 32768 23.8 / 21.2, 100000 41 / 25; 128 rows, 16000 33.6 / 36.2, 32768 39.6 / 37.8.
+_LONG_BASE = 24576
+
+
 def _build_in_place(q_probs, k_hard, v_norm, allowed, sink: int, window: int, M: int):
-    """`build_sparse_list_decode` in two launches: scores from the operands in their own types, and the list.  None for
-    operands it does not take."""
+    """`build_sparse_list_decode` in two launches: scores from the operands in their own types, and the list (three where
+    the window is long).  None for operands it does not take."""
     B, H, L, R = q_probs.shape
     T = k_hard.shape[3]
     types = (torch.float16, torch.bfloat16, torch.float32)
@@ -166,6 +173,11 @@ def _build_in_place(q_probs, k_hard, v_norm, allowed, sink: int, window: int, M:
     check("socket_soft_hash_collision", lib().socket_soft_hash_collision_typed(
         ptr(q_probs), dtype_enum(q_probs.dtype), ptr(k_hard), ptr(allowed), ptr(v_norm), dtype_enum(v_norm.dtype), ptr(scores),
         B, H, L, R, T, s))
+    if base > _LONG_BASE:
+        _select_into(scores, 0, 0, M, None, None, False, None, True, sparse_list[:, :, base:], sparse_len)
+        check("socket_finish_list", lib().socket_finish_list(ptr(sparse_list), ptr(sparse_len), ptr(allowed), B * H, T, sink,
+                                                             window, M, s))
+        return sparse_list, sparse_len
     ws, ws_bytes = _workspace_of(scores.device, B, H, T, M)
     try:
         check("socket_select_list", lib().socket_select_list_allowed(
