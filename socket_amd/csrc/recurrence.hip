@@ -369,6 +369,7 @@ __global__ __launch_bounds__(1024) void recurrence_step_kernel(socket_recurrence
 
 constexpr int kPrepThreads = 1024;
 constexpr int kPrepWaves = kPrepThreads / 64;
+constexpr int kPrepHeadsFirst = 65535;   // chunks up to which they are the grid's y, whose limit this is
 constexpr float kMildDecay = -60.f;   // a block's total log2 decay above which 2^{-pl} is safe in fp32
 
 // Workspace of one (chunk, head, sequence), in floats.  kt / vt: 16-wide tiles of dk / dv.
@@ -551,12 +552,14 @@ __device__ __forceinline__ void transpose_quad(rc_f32x4& x, int lane) {
 // of either kind 294 -> 238 us.  A chunk writes 144 KB for the scan, which 256 of them drain in about 8 us.  Holding
 // the second kind to 64 registers for two workgroups a CU spilled: 63 us a pass instead of 53.
 template <class DT, int NB, bool DELTA>
-__global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_recurrence a, int vec, int own_v) {
+__global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_recurrence a, int n_chunks, int vec, int own_v) {
   constexpr int C = 16 * NB;
   constexpr int LPR = kPrepThreads / C;          // lanes to a token: 8 channels each
   extern __shared__ __attribute__((aligned(16))) float rp_lds[];
   __shared__ int next_item;
-  const int h = blockIdx.x, chunk = blockIdx.y, b = blockIdx.z;   // (a head on one XCD, where its scan will be)
+  // (a head on one XCD, where its scan will be, while the chunks fit the grid's y)
+  const bool heads_first = n_chunks <= kPrepHeadsFirst;
+  const int h = heads_first ? blockIdx.x : blockIdx.y, chunk = heads_first ? blockIdx.y : blockIdx.x, b = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int x16 = lane & 15, quarter = lane >> 4;
   const int dk = a.dk, dv = a.dv, hk = h / (a.H / a.Hk);
@@ -575,7 +578,7 @@ __global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_re
   // C x vp; by itself where LDS allows it, else over q (without the delta rule over k as well) once that has been used
   float* vs = DELTA && own_v ? qs + C * kp : DELTA ? qs : ks;
 
-  float* ws = (float*)a.workspace + (((int64_t)b * a.H + h) * gridDim.y + chunk) * sp.size();
+  float* ws = (float*)a.workspace + (((int64_t)b * a.H + h) * n_chunks + chunk) * sp.size();
 
   // ---- inputs.  Decays: lane x of 32 (and x + 32) takes a channel over rows 0 .. 7 (and 8 .. 15) of a block
   const int spans = (dkp + 31) / 32;
@@ -1523,7 +1526,10 @@ int launch_prep(const socket_recurrence& a, int n_chunks, bool vec, hipStream_t 
   if (lds > 48 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
     return SOCKET_ERR_LAUNCH;
-  hipLaunchKernelGGL(kern, dim3((unsigned)a.H, (unsigned)n_chunks, (unsigned)a.B), dim3(kPrepThreads), lds, s, a, vec ? 1 : 0, own_v);
+  const unsigned heads = (unsigned)a.H, chunks = (unsigned)n_chunks;
+  const bool heads_first = n_chunks <= kPrepHeadsFirst;
+  const dim3 grid(heads_first ? heads : chunks, heads_first ? chunks : heads, (unsigned)a.B);
+  hipLaunchKernelGGL(kern, grid, dim3(kPrepThreads), lds, s, a, n_chunks, vec ? 1 : 0, own_v);
   return SOCKET_OK;
 }
 
