@@ -229,9 +229,12 @@ def soft_hash(queries_bhd: torch.Tensor, planes_lkd: torch.Tensor, protos_T: tor
     return out
 
 
-def decode_prologue_fits(qkv: torch.Tensor, head_dim: int, K: int, R: int, n_heads: int, n_kv_heads: int) -> bool:
+def decode_prologue_fits(qkv: torch.Tensor, head_dim: int, K: int, R: int, n_heads: int, n_kv_heads: int, operands=()) -> bool:
     """Whether `decode_prologue` takes these operands (else: rope_append, hash_keys_into
-    and soft_hash, three launches with the same results)."""
+    and soft_hash, three launches with the same results).  `operands`: the other tensors of the call that have to start on
+    a 16-byte boundary (views that a program has made of its own buffers may not)."""
+    if any(t.data_ptr() % 16 for t in operands):
+        return False
     if not (qkv.is_cuda and head_dim == HASH_DIM and R % 4 == 0 and 4 <= R <= 1024 and n_heads % n_kv_heads == 0
             and n_heads // n_kv_heads <= 8):
         return False

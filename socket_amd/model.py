@@ -277,9 +277,9 @@ def _decode_prologue(qkv: Tensor, freqs_table: Tensor, input_pos: Tensor, cache:
     """Rotary + append + hash of the new key + soft hash of the new query in one
     launch; None when the shapes are not the ones that launch is written for."""
     D = cache.k_cache.size(-1)
-    if cache.planes_words is None or not hash_cache.decode_prologue_fits(qkv, D, cache.K, protos_T.shape[1], n_heads,
-                                                                         n_kv_heads) \
-            or freqs_table.dtype not in (torch.bfloat16, torch.float32):
+    if cache.planes_words is None or freqs_table.dtype not in (torch.bfloat16, torch.float32) \
+            or not hash_cache.decode_prologue_fits(qkv, D, cache.K, protos_T.shape[1], n_heads, n_kv_heads,
+                                                   (freqs_table, cache.k_cache, cache.v_cache, planes, protos_T)):
         return None
     T = cache.k_cache.size(2)
     grouped = hash_cache._prefers_grouped(qkv.shape[0], n_heads, n_kv_heads, T, hash_cache.dtype_enum(qkv.dtype),

@@ -58,3 +58,34 @@ def test_prologue_of_other_types_equals_the_three_launches(dt, Hq, Hkv, L, K, R,
     of_logit = ((of_proj + (K + 2) * u) @ protos_T.double().abs()).amax(-1, keepdim=True) * scale
     bound = 2 * of_logit + 16 * u + (0 if dt == torch.float32 else 2.0 ** -8)
     assert (((plain.double() - want).abs() / want) <= bound).all()
+
+
+@pytest.mark.parametrize("moved", ["planes", "protos_T"])
+@pytest.mark.parametrize("dt,K,R", [(torch.float32, 8, 256), (torch.float32, 10, 1024), (torch.bfloat16, 4, 16)])
+def test_operands_that_start_on_no_boundary(dt, K, R, moved):
+    """Views one element into an allocation: such a step is answered by the three launches."""
+    dev, B, D, Hq, Hkv, L = "cuda", 2, 128, 8, 4, 6
+    cfg = M.ModelArgs(block_size=64, vocab_size=64, n_layer=1, n_head=Hq, n_local_heads=Hkv, dim=Hq * D, intermediate_size=256,
+                      head_dim=D, L=L, K=K, R=R)
+    steps = []
+    for shift in (0, 1):
+        torch.manual_seed(1)
+        att = M.Attention(cfg).to(device=dev, dtype=dt)
+        att.kv_cache = M.KVCache(B, 64, Hkv, D, L=L, R=R, dtype=dt, K=K, device=dev)
+        att.sync_planes()
+        t = getattr(att, moved)
+        whole = torch.empty(t.numel() + shift, dtype=t.dtype, device=dev)
+        view = whole[shift:].view(t.shape)
+        view.copy_(t)
+        setattr(att, moved, view)
+        assert (view.data_ptr() % 16 == 0) == (shift == 0)
+        qkv = torch.randn(B, 1, (Hq + 2 * Hkv) * D, generator=torch.Generator().manual_seed(3)).to(dt).to(dev)
+        freqs = M.precompute_freqs_cis(64, D, 10000).to(torch.float32).to(dev)
+        pos = torch.tensor([5], device=dev)
+        fused = M._decode_prologue(qkv, freqs, pos, att.kv_cache, att.planes, att.protos_T, Hq, Hkv)
+        assert (fused is None) == (shift == 1)
+        steps.append(att._run_fused_qkv(qkv, pos, True, M.DecodeStep(freqs, pos.to(torch.int32).expand(B).contiguous())))
+    # (every cached token is attended to: the table decides their order alone, and 32-bit sums over 64 of them and 1024
+    # columns, or their rounding to bfloat16, are what differs)
+    assert torch.isfinite(steps[0]).all()
+    assert (steps[0] - steps[1]).float().norm() <= (1e-6 if dt == torch.float32 else 2.0 ** -8) * steps[0].float().norm()
