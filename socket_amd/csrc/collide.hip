@@ -15,9 +15,9 @@
 // slices (two slices of 30 fp32 tables at L60 x R1024; one slice for fp16), copied
 // straight from memory into LDS while the first codes are on their way, and
 // serves several such tiles under each slice; a thread fetches the codes of its
-// eight consecutive tokens with one 16-byte load per table (wherever the row
-// starts), six tables ahead of their use, and gathers without branches.  Short rows
-// are dealt out two or four tokens to a thread.
+// consecutive tokens with one load per table (wherever the row starts) and gathers
+// without branches.  It has eight tokens, 16-byte loads, six tables ahead of their use;
+// four or two where rows are short, 8- or 4-byte loads, 12 or 24 tables ahead.
 #include <atomic>
 
 #include "socket_common.h"
@@ -285,7 +285,11 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
   const int few = !wide || ct == 0 ? 0 : per_row * 1024 * 2 >= T ? 2 : per_row * 1024 * 3 >= T ? 4 : 0;
   // Lanes of a workgroup of eight tokens each.  It pulls its row's whole table through LDS with them, which is quicker the
   // more there are, but while all workgroups are at work at once narrower ones leave fewer CUs idle (us at 512 / 1024 lanes,
-  // 32 rows, L60 x R1024: fp32 32768 tokens 35 / 40, 48000 61 / 44; bf16 32768 28 / 36, 65536 58 / 50).
+  // 32 rows, L60 x R1024: fp32 32768 tokens 35 / 40, 48000 61 / 44; bf16 32768 28 / 36, 65536 58 / 50).  A row of at most 4608
+  // tokens has no use for 512: one workgroup of 1024 holds it, or all but nothing (200 rows of 4096, L60 x R1024, fp32 30.6 /
+  // 29.3).  Rows of at most 2048 tokens come here where they outnumber the CUs; 256 lanes hold each of them, which pays where
+  // tables share a CU's LDS (us at 256 / 1024 lanes, L32 x R256, fp32: 448 rows x 1000 14.8 / 15.4, 1024 rows x 1000 18.8 / 23.4)
+  // and does not where one fills it (L60 x R1024, fp32: 257 rows x 1000 62 / 47, 1024 x 1000 183 / 121).
   auto tiles_of = [&](int th) { return (T + th * kTokensPerThread - 1) / (th * kTokensPerThread); };
   int threads = 1024;
   if (T <= 256 * kTokensPerThread) threads = 256;

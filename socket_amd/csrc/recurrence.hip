@@ -542,14 +542,14 @@ __device__ __forceinline__ void transpose_quad(rc_f32x4& x, int lane) {
 // tiles in LDS) nothing but the waves themselves hides a wait, so each phase asks for all it reads before it uses any:
 //  * a lane's eight channels of q, k and v with all their taps, and its eight decays, in one trip to memory; unit
 //    norms from those registers, running sums of the decays over 8 rows of a lane and, from its sum on, a lane 32 further
-//    on.  (Both halves summed from zero and the first one's sum added to each entry of the second rounds every entry at the
-//    full sum's magnitude twice: states up to four times as far from float64, 6.8e-7 where this gives 1.7e-7.);
+//    on (with both halves summed from zero and put together afterwards neighbours are rounded apart at the full sum's
+//    magnitude: states up to four times as far from float64, 6.8e-7 where this gives 1.7e-7);
 //  * the tiles of Aqk and L (a diagonal tile inverted by its own wave) and the fragments of Q^ and K^T are dealt out
 //    by a counter, the long ones first;
 //  * the forward substitution has its tiles in registers before it starts, and W leaves in 16-byte stores.
 // A workgroup of 128 key channels with the delta rule / of 64 without, in clock cycles: 63000 / 29000 -> 47000 / 21000
 // (18000 of the 47000 the first trip and its arithmetic, 13000 the tiles, 5000 the substitution); 5000 tokens of 16 heads
-// of either kind 294 -> 238 us.  A chunk writes 144 KB for the scan, which 256 of them drain in about 8 us.  Holding
+// of either kind 294 -> 245 us.  A chunk writes 144 KB for the scan, which 256 of them drain in about 8 us.  Holding
 // the second kind to 64 registers for two workgroups a CU spilled: 63 us a pass instead of 53.
 template <class DT, int NB, bool DELTA>
 __global__ __launch_bounds__(kPrepThreads) void recurrence_prep_kernel(socket_recurrence a, int n_chunks, int vec, int own_v) {

@@ -142,7 +142,8 @@ __global__ __launch_bounds__(kShortLanes) void score_short_kernel(
 #pragma unroll
     for (int g = 0; g < GP; ++g) {
       if (g >= geff) break;
-      __builtin_nontemporal_store(tok + i * kShortLanes < len ? acc[i][g] * vn[i] : -INFINITY, out + (int64_t)g * score_stride + tok + i * kShortLanes);
+      __builtin_nontemporal_store(tok + i * kShortLanes < len ? acc[i][g] * vn[i] : -INFINITY,
+                                  out + (int64_t)g * score_stride + tok + i * kShortLanes);
     }
   }
 }

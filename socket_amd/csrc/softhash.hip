@@ -1416,9 +1416,14 @@ extern "C" int socket_decode_prologue(const void* qkv, int dtype, int64_t qkv_st
                                       int Hq, int Hkv, int D, int L, int K, int R, int64_t Tcap,
                                       float tanh_scale, float inv_temperature, void* stream) {
   // (what this entry has always taken: bf16, ten planes)
-  SOCKET_REQUIRE(qkv && freqs_cis && pos && q_out && k_cache && v_cache && planes_words && codes && v_norm && planes && protos_T && q_table, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(qkv && freqs_cis && pos && q_out && k_cache && v_cache && planes_words && codes && v_norm &&
+                     planes && protos_T && q_table,
+                 SOCKET_ERR_NULL);
   SOCKET_REQUIRE(dtype == SOCKET_BF16 && K == 10, SOCKET_ERR_UNSUPPORTED);
-  return decode_prologue_entry(qkv, dtype, qkv_stride_b, freqs_cis, freqs_dtype, n_pos, pos, pos_stride, q_out, k_cache, v_cache, cache_stride_b, cache_stride_h, cache_stride_s, lens, planes_words, codes, v_norm, planes, protos_T, q_table, out_dtype, grouped, B, Hq, Hkv, D, L, K, R, Tcap, tanh_scale, inv_temperature, stream);
+  return decode_prologue_entry(qkv, dtype, qkv_stride_b, freqs_cis, freqs_dtype, n_pos, pos, pos_stride, q_out, k_cache,
+                               v_cache, cache_stride_b, cache_stride_h, cache_stride_s, lens, planes_words, codes, v_norm,
+                               planes, protos_T, q_table, out_dtype, grouped, B, Hq, Hkv, D, L, K, R, Tcap, tanh_scale,
+                               inv_temperature, stream);
 }
 
 extern "C" int socket_decode_prologue_typed(const void* qkv, int dtype, int64_t qkv_stride_b, const void* freqs_cis,
@@ -1429,5 +1434,8 @@ extern "C" int socket_decode_prologue_typed(const void* qkv, int dtype, int64_t 
                                       const void* protos_T, void* q_table, int out_dtype, int grouped, int B,
                                       int Hq, int Hkv, int D, int L, int K, int R, int64_t Tcap,
                                       float tanh_scale, float inv_temperature, void* stream) {
-  return decode_prologue_entry(qkv, dtype, qkv_stride_b, freqs_cis, freqs_dtype, n_pos, pos, pos_stride, q_out, k_cache, v_cache, cache_stride_b, cache_stride_h, cache_stride_s, lens, planes_words, codes, v_norm, planes, protos_T, q_table, out_dtype, grouped, B, Hq, Hkv, D, L, K, R, Tcap, tanh_scale, inv_temperature, stream);
+  return decode_prologue_entry(qkv, dtype, qkv_stride_b, freqs_cis, freqs_dtype, n_pos, pos, pos_stride, q_out, k_cache,
+                               v_cache, cache_stride_b, cache_stride_h, cache_stride_s, lens, planes_words, codes, v_norm,
+                               planes, protos_T, q_table, out_dtype, grouped, B, Hq, Hkv, D, L, K, R, Tcap, tanh_scale,
+                               inv_temperature, stream);
 }

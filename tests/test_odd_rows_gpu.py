@@ -74,7 +74,7 @@ def test_selection_from_odd_rows(T, M, shift):
 @pytest.mark.parametrize("B,H,T,M,sink,window,kept", [
     (1, 4, 5, 5, 2, 2, 0.5),                # more asked for than are allowed
     (2, 7, 4135, 129, 20, 20, 0.5),
-    (1, 8, 8192, 700, 0, 0, 0.05),          # fewer allowed than are asked for: masked ones fill the list
+    (1, 8, 8192, 700, 0, 0, 0.05),          # fewer allowed than are asked for: masked ones, mostly of one run, fill the list
     (1, 8, 8193, 300, 4, 64, 0.9),          # threshold from a sample
     (2, 5, 20881, 652, 4, 64, 0.02),        # ... of which little is allowed
     (1, 6, 49157, 1024, 4, 64, 0.6),        # a row shared between workgroups
