@@ -115,6 +115,21 @@ __device__ __forceinline__ u64 shfl_xor_u64(u64 v, int mask) {
   return ((u64)hi << 32) | lo;
 }
 
+// Sum of sums[0, wave) of W <= 16 waves: every wave scans all of them, one to a lane.  (One LDS read a wave; each lane reading
+// them one after another was 256 reads a workgroup, 0.4 us of each of the two or three calls of a selection.)
+template <int W>
+__device__ __forceinline__ int earlier_waves(const int* sums, int lane, int wave) {
+  static_assert(W <= 16 && (W & (W - 1)) == 0, "a row of 16 lanes");
+  int v = sums[lane & (W - 1)];
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);   // row_shr:8
+  const int w = __builtin_amdgcn_readfirstlane(wave);
+  const int s = __builtin_amdgcn_readlane(v, (w + 63) & 63);        // (lane w - 1)
+  return w > 0 ? s : 0;
+}
+
 // All THREADS lanes.  Ranks the bins from the top (descending != 0) or from the
 // bottom, kBins / THREADS per lane, and publishes in `sh` the bin where the
 // running count first reaches `need`, the count ranked before it and its own.
@@ -142,12 +157,7 @@ __device__ __forceinline__ void find_bin(uint32_t* hist, int need, int descendin
   const int incl_w = wave_incl_scan(mine, lane);
   if (lane == 63) sh.wsum[wave] = incl_w;
   __syncthreads();
-  int run = incl_w - mine;
-#pragma unroll
-  for (int w = 0; w < THREADS / SOCKET_WAVE; ++w) {   // (all entries read at once, the later waves' discarded)
-    const int v = sh.wsum[w];
-    run += (w < wave) ? v : 0;
-  }
+  int run = incl_w - mine + earlier_waves<THREADS / SOCKET_WAVE>(sh.wsum, lane, wave);
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     if (run < need && need <= run + c[i]) {
@@ -380,9 +390,11 @@ __device__ __forceinline__ void order_and_write(u64* buf, int n_above, u64* cand
   const int lane = tid & 63, wave = tid >> 6;
   // ---- the k-th bin: rank its entries, the best `need` follow the winners ----------
   if (ncand <= kMaxBinForCounting || need == ncand) {
-    for (int i = tid; i < ncand; i += THREADS) {
+    // (by the last lanes: the first have most of the winners)
+    for (int i = THREADS - 1 - tid; i < ncand; i += THREADS) {
       const u64 v = cand[i];
       int r = 0;
+#pragma unroll 4
       for (int j = 0; j < ncand; ++j) r += cand[j] > v;
       if (r < need) out[n_above + r] = listed<MASKED>(composite_index(v), ok);
     }
@@ -488,25 +500,40 @@ __host__ __device__ __forceinline__ bool sampling_ok(int m) {
 // the lower edge of its bin.  Every workgroup that calls this for a row gets the
 // same tau.  Needs n > kPoolCap; clears hist itself (nobody may be using it).  When
 // it returns every lane has passed the barrier that follows the last read of hist.
+constexpr int kSample = 4096, kLongSample = 16384;
+template <int THREADS>
+constexpr int kSampleVecs = kLongSample / 4 / THREADS;   // groups of four per lane at most
+
+// The sample's scores, requested ahead of the row's first batches: what is asked for first arrives first.
+template <int THREADS>
+__device__ __forceinline__ void request_sample(const float* row, int n, f32x4_any (&x)[kSampleVecs<THREADS>], int tid) {
+  const int nsample = n <= 262144 ? kSample : kLongSample;
+  const int nq = nsample / 4 / THREADS;  // 1 or 4 (1024 lanes), 2 or 8 (512 lanes)
+  const int shift = nsample == kSample ? 6 : 8;          // runs of 64 scores, 2^shift of them
+#pragma unroll
+  for (int j = 0; j < kSampleVecs<THREADS>; ++j) {
+    if (j < nq) {
+      const int q = j * THREADS + tid;
+      const int at = (int)(((int64_t)(q >> 4) * n >> shift) & ~3ll) + (q & 15) * 4;
+      x[j] = *reinterpret_cast<const f32x4_any*>(row + at);
+    }
+  }
+}
+
 template <int THREADS, bool MASKED>
-__device__ __forceinline__ uint32_t sample_threshold(const float* row, int n, int m, uint32_t* hist,
+__device__ __forceinline__ uint32_t sample_threshold(const f32x4_any (&x)[kSampleVecs<THREADS>], int n, int m, uint32_t* hist,
                                                      SelectShared& sh, int tid) {
-  constexpr int kMaxQ = 16384 / 4 / THREADS;  // float4 groups per lane at most
+  constexpr int kMaxQ = kSampleVecs<THREADS>;
   const int lane = tid & 63, wave = tid >> 6;
-  const int nsample = n <= 262144 ? 4096 : 16384;
-  const int nchunk = nsample / 64;
-  const int nq = nsample / 4 / THREADS;  // 1 or 4 (1024 lanes), 4 or 16 (256 lanes)
+  const int nsample = n <= 262144 ? kSample : kLongSample;
+  const int nq = nsample / 4 / THREADS;
   uint32_t key[kMaxQ * 4];
   for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;   // (no one uses hist before this call)
 #pragma unroll
   for (int j = 0; j < kMaxQ; ++j) {
     if (j < nq) {
-      const int q = j * THREADS + tid;
-      const int chunk = q >> 4;
-      const int at = (int)(((int64_t)chunk * n / nchunk) & ~3ll) + (q & 15) * 4;
-      const f32x4_any x = *reinterpret_cast<const f32x4_any*>(row + at);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) key[j * 4 + c] = score_to_key(x[c]);
+      for (int c = 0; c < 4; ++c) key[j * 4 + c] = score_to_key(x[j][c]);
     }
   }
   uint32_t kmin = 0xffffffffu, kmax = 0u;
@@ -581,6 +608,137 @@ __device__ __forceinline__ u64 load_coherent(const u64* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// ---------------------------------------------------------------------------
+// from a pool in registers, kPoolCap / THREADS entries per lane
+// ---------------------------------------------------------------------------
+// A row of at most kPoolCap scores, all of it (past its end: zeros, which no load asks the memory for).
+template <int THREADS>
+__device__ __forceinline__ void request_row(const float* row, int n, f32x4_any (&x)[kPoolCap / THREADS / 4], int tid) {
+  const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(row), 0, n * 4, 0x00027000);
+#pragma unroll
+  for (int u = 0; u < kPoolCap / THREADS / 4; ++u)
+    x[u] = __builtin_bit_cast(f32x4_any, __builtin_amdgcn_raw_buffer_load_b128(src, (u * THREADS + tid) * 16, 0, 0));
+}
+
+// Its entries, four neighbours to a lane and group, and the range of the keys that this lane holds.
+template <bool MASKED, int THREADS>
+__device__ __forceinline__ void pool_row(const f32x4_any (&x)[kPoolCap / THREADS / 4], int n, u64 (&pv)[kPoolCap / THREADS],
+                                         uint32_t& have, uint32_t& kmin, uint32_t& kmax, int tid) {
+#pragma unroll
+  for (int u = 0; u < kPoolCap / THREADS; ++u) {
+    const int i = ((u >> 2) * THREADS + tid) * 4 + (u & 3);
+    const uint32_t k = score_to_key(x[u >> 2][u & 3]);
+    if (i < n) {
+      if (!MASKED || k > kMaskedKey) kmin = min(kmin, k);
+      kmax = max(kmax, k);
+      have |= 1u << u;
+    }
+    pv[u] = composite(k, i);
+  }
+}
+
+// All lanes: the m best of the pool's entries, in order, at heavy[0:m).  have: bit u where pv[u] is one; kmin / kmax: the
+// range of this lane's keys; hist is zero, sh's counters and range are as select_list_kernel sets them, and a barrier lies behind both.
+template <bool MASKED, int THREADS>
+__device__ __forceinline__ void select_from_pool(const u64 (&pv)[kPoolCap / THREADS], uint32_t have, uint32_t kmin, uint32_t kmax, int m,
+                                                 uint32_t* hist, SelectShared& sh, u64* buf, u64* cand, u64* tmp, int cap_above,
+                                                 bool counting_ok, int32_t* heavy, const uint8_t* ok, int tid) {
+  constexpr int U = kPoolCap / THREADS;
+  static_assert(U <= 32, "a bit each");
+  const int lane = tid & (SOCKET_WAVE - 1);
+  // range of the pooled composites, from their keys (the high halves): any range
+  // that holds them all serves the refinement
+  wave_minmax_to_last(kmin, kmax);
+  if (lane == 63) {
+    atomicMin(&sh.kmin, kmin);
+    atomicMax(&sh.kmax, kmax);
+  }
+  __syncthreads();
+  const u64 lo0 = (u64)(MASKED ? min(sh.kmin, sh.kmax) : sh.kmin) << 32, hi0 = ((u64)sh.kmax << 32) | 0xffffffffull;
+  const int shift0 = range_shift(lo0, hi0);
+  // refinement on the composites; they are distinct, so it ends with a bin of
+  // at most kCandCap entries (ties need no special case here).
+  // The first pass covers every entry, and every entry keeps the slot that its
+  // bin's counter hands out.  When that pass already isolates the k-th bin (the
+  // usual case) the bins' counters, turned into offsets by the same scan that
+  // finds the bin, and those slots place every winner next to the others of its
+  // bin and the k-th bin's entries in their list with no further counting.
+  {
+    uint32_t slot2[U / 2];   // 16 bits per entry
+#pragma unroll
+    for (int u = 0; u < U / 2; ++u) slot2[u] = 0;   // (hist is zero: cleared ahead of the pool)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (have >> u & 1) {
+        const uint32_t sl = atomicAdd(&hist[level0_bin<MASKED>(pv[u], lo0, shift0)], 1u);
+        slot2[u >> 1] |= sl << (16 * (u & 1));
+      }
+    }
+    __syncthreads();
+    find_bin<THREADS, true>(hist, m, 1, sh, tid, [&](int bin, int before, int count) {
+      const u64 blo = lo0 + ((u64)bin << shift0);
+      const u64 bspan = (shift0 == 0) ? 0ull : ((1ull << shift0) - 1ull);
+      sh.lo = MASKED && bin == 0 ? 0ull : blo;
+      sh.hi = (hi0 - blo < bspan) ? hi0 : blo + bspan;
+      sh.need = m - before;
+      sh.done = (count <= kCandCap || shift0 == 0) ? 1 : 0;
+    });
+    if (sh.done && !sh.crowded) {
+      const int fb = sh.found_bin, need = sh.need, ncand = min(sh.found_count, kCandCap);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (have >> u & 1) {
+          const u64 v = pv[u];
+          const int bin = level0_bin<MASKED>(v, lo0, shift0);
+          const int sl = (int)((slot2[u >> 1] >> (16 * (u & 1))) & 0xffffu);
+          if (bin > fb) buf[(int)(hist[bin] & 0xffffu) + sl] = v;
+          else if (bin == fb && sl < kCandCap) cand[sl] = v;
+        }
+      }
+      __syncthreads();
+      order_and_write<MASKED, THREADS>(buf, m - need, cand, ncand, need, lo0, shift0, tmp, hist, sh, counting_ok, heavy,
+                                       ok, tid, true);
+      return;
+    }
+  }
+  for (int iter = 1; iter < 8 && !sh.done; ++iter) {
+    const u64 lo = sh.lo, hi = sh.hi;
+    const int need_in = sh.need;
+    const int shift = range_shift(lo, hi);
+    for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const u64 v = pv[u];
+      if ((have >> u & 1) && v >= lo && v <= hi) atomicAdd(&hist[(int)((v - lo) >> shift)], 1u);
+    }
+    __syncthreads();
+    find_bin<THREADS>(hist, need_in, 1, sh, tid);
+    if (tid == 0) {
+      const u64 blo = lo + ((u64)sh.found_bin << shift);
+      const u64 bspan = (shift == 0) ? 0ull : ((1ull << shift) - 1ull);
+      sh.lo = blo;
+      sh.hi = (hi - blo < bspan) ? hi : blo + bspan;
+      sh.need = need_in - sh.found_before;
+      sh.done = (sh.found_count <= kCandCap || shift == 0) ? 1 : 0;
+    }
+    __syncthreads();
+    if (sh.done) break;
+  }
+  const u64 blo = sh.lo, bhi = sh.hi;
+  const int need = sh.need;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const u64 v = pv[u];
+    const bool in = have >> u & 1;
+    wave_append(in && v > bhi, v, &sh.fill_above, buf, cap_above);
+    wave_append(in && v >= blo && v <= bhi, v, &sh.fill_cand, cand, kCandCap);
+  }
+  __syncthreads();
+  order_and_write<MASKED, THREADS>(buf, m - need, cand, min(sh.fill_cand, kCandCap), need, lo0, shift0, tmp, hist, sh,
+                                   counting_ok, heavy, ok, tid);
+}
+
 // `parts` workgroups per row (blockIdx.x = row * parts + part).  With parts > 1
 // each filters its share of the row against the same sampled threshold (every
 // part works it out for itself from the same sample), appends what passes to the
@@ -622,10 +780,15 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
   const float* row = scores + (int64_t)rowi * score_stride;
   int32_t* out = sparse_list + (int64_t)rowi * list_stride;
   const uint8_t* ok = MASKED ? allowed + (int64_t)rowi * T : nullptr;
-  if (part == 0)
-    write_list_base<MASKED>(out, n, m, nbase, sink, window, write_base, list_width,
-                            sparse_len ? sparse_len + rowi : nullptr, ok, tid, THREADS);
-  if (m == 0) return;
+  auto list_base = [&]() __attribute__((always_inline)) {
+    if (part == 0)
+      write_list_base<MASKED>(out, n, m, nbase, sink, window, write_base, list_width,
+                              sparse_len ? sparse_len + rowi : nullptr, ok, tid, THREADS);
+  };
+  if (m == 0) {
+    list_base();
+    return;
+  }
   int32_t* heavy = out + nbase;
 
   // ================================ pooled select ======================================
@@ -641,19 +804,14 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
     int total = -1;  // uniform; stays -1 when no pool could be formed
     uint32_t kmin = 0xffffffffu, kmax = 0u;  // key range of what this lane holds
     constexpr int U = kPoolCap / THREADS;
-    u64 pv[U];                               // entry tid + u * THREADS of the pool
+    u64 pv[U];                               // of the pool, this lane's
+    uint32_t have = 0;                       // bit u: pv[u] is an entry
     if (n <= kPoolCap) {  // the whole row, by one workgroup
       if (part != 0) return;
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = tid + u * THREADS;
-        const uint32_t k = score_to_key(i < n ? row[i] : 0.f);
-        if (i < n) {
-          if (!MASKED || k > kMaskedKey) kmin = min(kmin, k);
-          kmax = max(kmax, k);
-        }
-        pv[u] = composite(k, i);
-      }
+      f32x4_any x[U / 4];
+      request_row<THREADS>(row, n, x, tid);
+      list_base();
+      pool_row<MASKED, THREADS>(x, n, pv, have, kmin, kmax, tid);
       total = n;
       for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;   // for the first refinement pass
       __syncthreads();
@@ -680,55 +838,46 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
           x[u] = make_float4(v.x, v.y, v.z, v.w);
         }
       };
-      // One batch of one wave.  Each of a lane's 16 scores is tested on the float (one
-      // compare per score; keys only for the pool): x passes when it is not below the
-      // float whose key is tau.  A tau above +inf's key or below -inf's is no float's
-      // key and is widened to that infinity (the pool only has to hold everything at
-      // or above tau; more is allowed).  A compare leaves a wave-wide mask in scalar
-      // registers; the 16 masks' population is the stretch of the pool that one LDS
-      // atomic reserves for the wave, and an entry's place in it is the count of its
-      // mask's bits below its lane, on top of a scalar running base -- no per-lane
-      // bookkeeping, no cross-lane traffic.  A batch that would run past the pool is
-      // counted but not written (the row is then redone from scratch anyway).
+      // One batch of one wave.  Each of a lane's 16 scores is tested on the float (keys only for the pool): x passes when
+      // it is not below the float whose key is tau.  A tau above +inf's key or below -inf's is no float's key and is
+      // widened to that infinity (the pool only has to hold everything at or above tau; more is allowed).  A lane counts
+      // its own; a scan over the lanes and one LDS atomic give it its stretch of the pool, which it fills in order: some
+      // nine vector instructions a score, where ranking the lanes of every score's ballot took twenty (us, before / now: 32
+      // rows of 32771 11.8 / 11.4, 256 of 65536 18.1 / 17.9, 448 of 98304 39.7 / 37.8).  A batch that would run past the
+      // pool is counted but not written (the row is then redone from scratch anyway).
       auto filter_batch = [&](auto full, int base, const float4 (&x)[kLoads], float tau_f) {
         constexpr bool FULL = decltype(full)::value;   // every lane's 16 scores are inside the share
-        int total = 0;
-        u64 mask[kLoads * 4];   // (scalar registers)
+        int mine = 0;
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
           const float xs[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
           const bool in = FULL || base + (u * THREADS + tid) * 4 < e4;
 #pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            mask[u * 4 + c] = __builtin_amdgcn_ballot_w64(in && !(xs[c] < tau_f));
-            total += __popcll(mask[u * 4 + c]);
-          }
+          for (int c = 0; c < 4; ++c) mine += in && !(xs[c] < tau_f) ? 1 : 0;
         }
+        const int upto = wave_incl_scan(mine, lane);
+        const int total = __builtin_amdgcn_readlane(upto, 63);
         if (total == 0) return;  // uniform
         int at = 0;
         if (lane == 0) at = atomicAdd(&sh.fill_pool, total);
         at = __builtin_amdgcn_readfirstlane(at);
         if (at + total > kPoolCap) return;  // uniform
         const uint32_t cidx = 0xffffffffu - (uint32_t)(base + tid * 4);
+        uint32_t addr = (uint32_t)(uintptr_t)(pool + at + upto - mine);
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) {
           const float xs[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
           const bool in = FULL || base + (u * THREADS + tid) * 4 < e4;
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
-            const bool pass = in && !(xs[c] < tau_f);
-            const u64 mk = mask[u * 4 + c];
-            const int slot = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32),
-                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)mk, (uint32_t)at));
-            if (pass) {
+            if (in && !(xs[c] < tau_f)) {
               // the two halves of the entry from wherever they are, in one write
               // (a 64-bit store would first copy them into a register pair)
-              const uint32_t addr = (uint32_t)(uintptr_t)(pool + slot);
               asm volatile("ds_write2_b32 %0, %1, %2 offset1:1"
                            :: "v"(addr), "v"(cidx - (uint32_t)(u * THREADS * 4 + c)), "v"(__float_as_uint(xs[c]))
                            : "memory");
+              addr += 8;
             }
-            at += __popcll(mk);
           }
         }
       };
@@ -738,9 +887,14 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
         else filter_batch(BoolTag<false>{}, base, x, tau_f);
       };
       float4 b0[kLoads], b1[kLoads], b2[kLoads];
+      f32x4_any sample[kSampleVecs<THREADS>];
+      request_sample<THREADS>(row, n, sample, tid);
+      const float tail = e4 + lane < tail_end ? row[e4 + lane] : 0.f;     // (of wave 0)
+      __builtin_amdgcn_sched_barrier(0);
       fetch(begin, b0);
       fetch(begin + kStep, b1);
-      const uint32_t tau = sample_threshold<THREADS, MASKED>(row, n, m, hist, sh, tid);
+      list_base();
+      const uint32_t tau = sample_threshold<THREADS, MASKED>(sample, n, m, hist, sh, tid);
       for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;   // for the first refinement pass
       const float tau_f = tau >= 0xff800000u ? INFINITY : tau <= 0x007fffffu ? -INFINITY
                           : __uint_as_float((tau & 0x80000000u) ? (tau & 0x7fffffffu) : ~tau);
@@ -755,8 +909,7 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
       __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the pool writes above are not the compiler's to wait for
       if (wave == 0) {
         const int i = e4 + lane;
-        const float x = i < tail_end ? row[i] : 0.f;
-        wave_append(i < tail_end && !(x < tau_f), composite(__float_as_uint(x), i), &sh.fill_pool, pool, kPoolCap);
+        wave_append(i < tail_end && !(tail < tau_f), composite(__float_as_uint(tail), i), &sh.fill_pool, pool, kPoolCap);
       }
       __syncthreads();
       // (an entry of the pool: the score's bits over the complemented index)
@@ -801,110 +954,23 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
 #pragma unroll
         for (int u = 0; u < U; ++u)
           if (tid + u * THREADS < total) {
+            have |= 1u << u;
             const uint32_t k = (uint32_t)(pv[u] >> 32);
             if (!MASKED || k > kMaskedKey) kmin = min(kmin, k);
             kmax = max(kmax, k);
           }
       }
-    } else if (part != 0) {
-      return;   // no threshold can be relied on: one workgroup selects from scratch
+    } else {
+      if (part != 0) return;   // no threshold can be relied on: one workgroup selects from scratch
+      list_base();
     }
     if (total >= 0) {
-      // range of the pooled composites, from their keys (the high halves): any range
-      // that holds them all serves the refinement
-      wave_minmax_to_last(kmin, kmax);
-      if (lane == 63) {
-        atomicMin(&sh.kmin, kmin);
-        atomicMax(&sh.kmax, kmax);
-      }
-      __syncthreads();
-      const u64 lo0 = (u64)(MASKED ? min(sh.kmin, sh.kmax) : sh.kmin) << 32, hi0 = ((u64)sh.kmax << 32) | 0xffffffffull;
-      const int shift0 = range_shift(lo0, hi0);
-      // refinement on the composites; they are distinct, so it ends with a bin of
-      // at most kCandCap entries (ties need no special case here).
-      // The first pass covers every entry, and every entry keeps the slot that its
-      // bin's counter hands out.  When that pass already isolates the k-th bin (the
-      // usual case) the bins' counters, turned into offsets by the same scan that
-      // finds the bin, and those slots place every winner next to the others of its
-      // bin and the k-th bin's entries in their list with no further counting.
-      {
-        uint32_t slot2[U / 2];   // 16 bits per entry
-#pragma unroll
-        for (int u = 0; u < U / 2; ++u) slot2[u] = 0;   // (hist is zero: cleared ahead of the pool)
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          if (tid + u * THREADS < total) {
-            const uint32_t sl = atomicAdd(&hist[level0_bin<MASKED>(pv[u], lo0, shift0)], 1u);
-            slot2[u >> 1] |= sl << (16 * (u & 1));
-          }
-        }
-        __syncthreads();
-        find_bin<THREADS, true>(hist, m, 1, sh, tid, [&](int bin, int before, int count) {
-          const u64 blo = lo0 + ((u64)bin << shift0);
-          const u64 bspan = (shift0 == 0) ? 0ull : ((1ull << shift0) - 1ull);
-          sh.lo = MASKED && bin == 0 ? 0ull : blo;
-          sh.hi = (hi0 - blo < bspan) ? hi0 : blo + bspan;
-          sh.need = m - before;
-          sh.done = (count <= kCandCap || shift0 == 0) ? 1 : 0;
-        });
-        if (sh.done && !sh.crowded) {
-          const int fb = sh.found_bin, need = sh.need, ncand = min(sh.found_count, kCandCap);
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            if (tid + u * THREADS < total) {
-              const u64 v = pv[u];
-              const int bin = level0_bin<MASKED>(v, lo0, shift0);
-              const int sl = (int)((slot2[u >> 1] >> (16 * (u & 1))) & 0xffffu);
-              if (bin > fb) buf[(int)(hist[bin] & 0xffffu) + sl] = v;
-              else if (bin == fb && sl < kCandCap) cand[sl] = v;
-            }
-          }
-          __syncthreads();
-          order_and_write<MASKED, THREADS>(buf, m - need, cand, ncand, need, lo0, shift0, tmp, hist, sh, counting_ok != 0, heavy,
-                          ok, tid, true);
-          return;
-        }
-      }
-      for (int iter = 1; iter < 8 && !sh.done; ++iter) {
-        const u64 lo = sh.lo, hi = sh.hi;
-        const int need_in = sh.need;
-        const int shift = range_shift(lo, hi);
-        for (int i = tid; i < kBins; i += THREADS) hist[i] = 0;
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const u64 v = pv[u];
-          if (tid + u * THREADS < total && v >= lo && v <= hi) atomicAdd(&hist[(int)((v - lo) >> shift)], 1u);
-        }
-        __syncthreads();
-        find_bin<THREADS>(hist, need_in, 1, sh, tid);
-        if (tid == 0) {
-          const u64 blo = lo + ((u64)sh.found_bin << shift);
-          const u64 bspan = (shift == 0) ? 0ull : ((1ull << shift) - 1ull);
-          sh.lo = blo;
-          sh.hi = (hi - blo < bspan) ? hi : blo + bspan;
-          sh.need = need_in - sh.found_before;
-          sh.done = (sh.found_count <= kCandCap || shift == 0) ? 1 : 0;
-        }
-        __syncthreads();
-        if (sh.done) break;
-      }
-      const u64 blo = sh.lo, bhi = sh.hi;
-      const int need = sh.need;
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const u64 v = pv[u];
-        const bool have = tid + u * THREADS < total;
-        wave_append(have && v > bhi, v, &sh.fill_above, buf, cap_above);
-        wave_append(have && v >= blo && v <= bhi, v, &sh.fill_cand, cand, kCandCap);
-      }
-      __syncthreads();
-      order_and_write<MASKED, THREADS>(buf, m - need, cand, min(sh.fill_cand, kCandCap), need, lo0, shift0, tmp, hist, sh,
-                      counting_ok != 0, heavy, ok, tid);
+      select_from_pool<MASKED, THREADS>(pv, have, kmin, kmax, m, hist, sh, buf, cand, tmp, cap_above, counting_ok != 0, heavy, ok, tid);
       return;
     }
-  } else if (part != 0) {
-    return;
+  } else {
+    if (part != 0) return;
+    list_base();
   }
 
   // ================================ from scratch ======================================
