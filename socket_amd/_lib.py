@@ -199,6 +199,8 @@ SIGNATURES = {
     "socket_select_workspace_bytes": (_Z, [_I, _I, _I, _I]),
     "socket_select_workspace_zero_bytes": (_Z, [_I, _I, _I, _I]),
     "socket_select_list": (_I, [_P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P, _L, _I, _P, _P, _Z, _P]),
+    "socket_select_attend_fits": (_I, [_I, _I, _I, _I, _I, _I]),
+    "socket_select_attend": (_I, [_P, _L, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P, _I] + [_L] * 8 + [_P, _L, _L] + [_I] * 5 + [_P]),
     "socket_decode_prologue": (_I, [_P, _I, _L, _P, _I, _L, _P, _I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _P, _P, _P, _P,
                                     _I, _I, _I, _I, _I, _I, _I, _I, _I, _L, c_float, c_float, _P]),
     "socket_decode_prologue_typed": (_I, [_P, _I, _L, _P, _I, _L, _P, _I, _P, _P, _P, _L, _L, _L, _P, _P, _P, _P, _P, _P, _P,

@@ -17,15 +17,13 @@
 
 #include <atomic>
 
-#include "socket_common.h"
+#include "attend_row.h"
 
 namespace {
 
 constexpr int kAttThreads = 256;
 constexpr int kAttWaves = kAttThreads / SOCKET_WAVE;
 constexpr int kUnroll = 4;
-
-__device__ __forceinline__ float fast_exp(float x) { return __expf(x); }
 
 // Stores and loads that are coherent across the whole GPU without a fence: the
 // store is written through to where every compute die sees it, the load does not
@@ -37,19 +35,6 @@ __device__ __forceinline__ void store_coherent(float* p, float v) {
 }
 __device__ __forceinline__ float load_coherent(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Merge (m, l, acc) pairs of an online softmax.
-template <int E>
-__device__ __forceinline__ void merge_state(float& m, float& l, float* acc, float m2, float l2,
-                                            const float* acc2) {
-  const float nm = fmaxf(m, m2);
-  const float s1 = (m == nm) ? 1.f : fast_exp(m - nm);
-  const float s2 = (m2 == nm) ? 1.f : fast_exp(m2 - nm);
-  l = l * s1 + l2 * s2;
-#pragma unroll
-  for (int i = 0; i < E; ++i) acc[i] = acc[i] * s1 + acc2[i] * s2;
-  m = nm;
 }
 
 // The split's output from the waves' states in LDS, records [wave][head] of D
@@ -382,92 +367,23 @@ __global__ __launch_bounds__(kAttThreads) void sparse_stage1_kernel(
   }
 }
 
-// fp32 rows with short lists (at most row_entries(D)): a workgroup of sixteen waves takes a (b, h) row's whole list in one
+// fp32 rows with short lists (at most row_entries<DType_f32>(D)): a workgroup of sixteen waves takes a (b, h) row's whole list in one
 // pass, every entry requested at once, and writes the output itself.  The list's few hundred KB come through one CU at its
 // L2 rate in about the time a second launch takes: 32 rows x 196 entries of 128 dims 6.3 us where splits and their merge
 // take 7.4 (8 rows 5.4 / 6.2, 256 rows 11.3 / 14.3).  Past one pass a lone CU is behind (32 rows x 400: 10.1 / 8.4), and
 // 16-bit rows gain nothing (196 entries 6.8 / 6.1).
-constexpr int kRowWaves = 16, kRowUnroll = 8;
-constexpr int row_entries(int D) { return kRowWaves * (SOCKET_WAVE / (D / 4)) * kRowUnroll; }
-
 template <int D>
 __global__ __launch_bounds__(kRowWaves * SOCKET_WAVE) void sparse_row_kernel(
     const float* __restrict__ q_, const float* __restrict__ k_, const float* __restrict__ v_, int64_t q_sb, int64_t q_sh,
     int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, const int32_t* __restrict__ sparse_list,
     int64_t list_sb, int64_t list_sh, const int32_t* __restrict__ sparse_len, int64_t len_sb, int64_t len_sh, int G, int kv_rows,
     int list_width, float sm_scale, float* __restrict__ out, int64_t out_sb, int64_t out_sh) {
-  constexpr int LPR = D / 4, RPW = SOCKET_WAVE / LPR;
   __shared__ float lds[kRowWaves][D + 2];
   const int h = blockIdx.x, b = blockIdx.y, kvh = h / G;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int slot = lane / LPR, chunk = lane % LPR;
-  const float* kbase = k_ + b * k_sb + kvh * k_sh + chunk * 4;
-  const float* vbase = v_ + b * v_sb + kvh * v_sh + chunk * 4;
   const int32_t* list = sparse_list + b * list_sb + h * list_sh;
-  const int len = min(sparse_len[b * len_sb + h * len_sh], list_width);
-  const float4 qf = *reinterpret_cast<const float4*>(q_ + b * q_sb + h * q_sh + chunk * 4);
-  int idx[kRowUnroll];
-#pragma unroll
-  for (int u = 0; u < kRowUnroll; ++u) {         // (past the list: its last entry, not live)
-    const int e = (u * kRowWaves + wave) * RPW + slot;
-    idx[u] = list[min(e, list_width - 1)];
-    if (e >= len || idx[u] >= kv_rows) idx[u] = -1;
-  }
-  float4 kr[kRowUnroll], vr[kRowUnroll];
-#pragma unroll
-  for (int u = 0; u < kRowUnroll; ++u) {
-    kr[u] = vr[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (idx[u] >= 0) {
-      kr[u] = *reinterpret_cast<const float4*>(kbase + (int64_t)idx[u] * k_ss);
-      vr[u] = *reinterpret_cast<const float4*>(vbase + (int64_t)idx[u] * v_ss);
-    }
-  }
-  float sc[kRowUnroll], m[1] = {-INFINITY}, l[1] = {0.f}, acc[1][4] = {{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-  for (int u = 0; u < kRowUnroll; ++u) {
-    const float d = group_sum<LPR>(qf.x * kr[u].x + qf.y * kr[u].y + qf.z * kr[u].z + qf.w * kr[u].w);
-    sc[u] = idx[u] >= 0 ? d * sm_scale : -INFINITY;
-    m[0] = fmaxf(m[0], sc[u]);
-  }
-#pragma unroll
-  for (int u = 0; u < kRowUnroll; ++u) {
-    const float p = idx[u] >= 0 ? fast_exp(sc[u] - m[0]) : 0.f;
-    l[0] += p;
-    acc[0][0] += p * vr[u].x;
-    acc[0][1] += p * vr[u].y;
-    acc[0][2] += p * vr[u].z;
-    acc[0][3] += p * vr[u].w;
-  }
-  // row slots inside the wave, then the waves through LDS
-#pragma unroll
-  for (int d = LPR; d < SOCKET_WAVE; d <<= 1) {
-    auto partner = [&](float x) { return d == 16 ? lane_xor16(x) : d == 32 ? lane_xor32(x) : __shfl_xor(x, d, SOCKET_WAVE); };
-    const float m2 = partner(m[0]), l2 = partner(l[0]);
-    float a2[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) a2[i] = partner(acc[0][i]);
-    merge_state<4>(m[0], l[0], acc[0], m2, l2, a2);
-  }
-  if (lane < LPR) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) lds[wave][chunk * 4 + i] = acc[0][i];
-    if (chunk == 0) {
-      lds[wave][D] = m[0];
-      lds[wave][D + 1] = l[0];
-    }
-  }
-  __syncthreads();
-  if (tid >= D) return;
-  float M = -INFINITY, sum = 0.f, val = 0.f;
-#pragma unroll
-  for (int w = 0; w < kRowWaves; ++w) M = fmaxf(M, lds[w][D]);
-#pragma unroll
-  for (int w = 0; w < kRowWaves; ++w) {
-    const float f = lds[w][D] == M ? 1.f : fast_exp(lds[w][D] - M);
-    sum += lds[w][D + 1] * f;
-    val += lds[w][tid] * f;
-  }
-  out[b * out_sb + h * out_sh + tid] = val / sum;      // (0/0 -> NaN when nothing was attended, as the reference)
+  row_attend<DType_f32, D>(q_ + b * q_sb + h * q_sh, k_ + b * k_sb + kvh * k_sh, k_ss, v_ + b * v_sb + kvh * v_sh, v_ss, list,
+                           min(sparse_len[b * len_sb + h * len_sh], list_width), list_width, kv_rows, sm_scale, lds,
+                           out + b * out_sb + h * out_sh);
 }
 
 // Dense flash-decode: rows [s*rows_per_split, ...) of one kv head, all G heads
@@ -1141,7 +1057,7 @@ namespace {
 
 // A workgroup to a row (sparse_row_kernel, where both sides' times are): fp32, lists of one pass, no more rows than CUs.
 bool one_row_each(int B, int Hq, int D, int max_len, int dtype) {
-  return dtype == SOCKET_F32 && (D == 16 || D == 32 || D == 64 || D == 128) && max_len <= row_entries(D) &&
+  return dtype == SOCKET_F32 && (D == 16 || D == 32 || D == 64 || D == 128) && max_len <= row_entries<DType_f32>(D) &&
          (int64_t)B * Hq <= socket_device_limits().cu_count;
 }
 

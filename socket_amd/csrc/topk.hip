@@ -39,7 +39,7 @@
 // bin's counter handed it, the scan that finds the m-th bin turns the counters
 // into offsets, and when that one pass isolates the bin (the usual case) the
 // winners are grouped by bin with no second count.
-#include "socket_common.h"
+#include "attend_row.h"
 
 
 namespace {
@@ -1100,6 +1100,54 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
                   sh, counting_ok != 0, heavy, ok, tid);
 }
 
+// A short row's selection and its attention in one launch, a workgroup to a (b, h) row: the list stays in LDS.  Rows of at
+// most kPoolCap scores whose list is one pass of row_attend, no more rows than CUs.  What bounds it is a chain of short
+// phases on one CU; what it saves is a launch, and the list's way to memory and back.  Two launches / one, us: fp32, 32 rows
+// of 4096, 196 entries 14.5 / 11.8, 128 rows 15.4 / 12.3, 256 rows of 2000, 168 entries 17.2 / 13.5; bf16, 32 rows of 8000, 504
+// entries 17.5 / 15.8, 256 rows of 8192 27.2 / 20.9.
+constexpr int kFuseList = 512;      // entries of a list at most
+template <class DT, int D>
+__global__ __launch_bounds__(kThreads, 4) void select_attend_kernel(
+    const float* __restrict__ scores, int64_t score_stride, const int32_t* __restrict__ lens, const int32_t* __restrict__ budgets,
+    int Hq, int T, int M, int sink, int window, int list_width, const typename DT::storage* __restrict__ q_,
+    const typename DT::storage* __restrict__ k_, const typename DT::storage* __restrict__ v_, int64_t q_sb, int64_t q_sh, int64_t k_sb,
+    int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, int G, int kv_rows, float sm_scale,
+    typename DT::storage* __restrict__ out, int64_t out_sb, int64_t out_sh) {
+  static_assert(kRowWaves * SOCKET_WAVE == kThreads, "one workgroup serves both parts");
+  __shared__ uint32_t hist[kBins];
+  __shared__ SelectShared sh;
+  __shared__ u64 buf[kFuseList], cand[kCandCap], tmp[2 * kFuseList];
+  __shared__ int32_t list[kFuseList];
+  __shared__ float waves[kRowWaves][D + 2];
+  const int b = blockIdx.x / Hq, h = blockIdx.x % Hq, kvh = h / G, tid = threadIdx.x;
+  int n, m, nbase;
+  row_shape(lens, budgets, b, T, M, sink, window, 1, list_width, n, m, nbase);
+  if (m > 0) {
+    const float* row = scores + (int64_t)blockIdx.x * score_stride;
+    if (tid == 0) {
+      sh.fill_above = 0;
+      sh.fill_cand = 0;
+      sh.kmin = 0xffffffffu;
+      sh.kmax = 0u;
+      sh.crowded = 0;
+    }
+    u64 pv[kPoolCap / kThreads];
+    uint32_t have = 0, kmin = 0xffffffffu, kmax = 0u;
+    f32x4_any x[kPoolCap / kThreads / 4];
+    request_row<kThreads>(row, n, x, tid);
+    for (int i = tid; i < kBins; i += kThreads) hist[i] = 0;
+    write_list_base<false>(list, n, m, nbase, sink, window, 1, list_width, nullptr, nullptr, tid, kThreads);
+    pool_row<false, kThreads>(x, n, pv, have, kmin, kmax, tid);
+    __syncthreads();
+    select_from_pool<false, kThreads>(pv, have, kmin, kmax, m, hist, sh, buf, cand, tmp, kFuseList, true, list + nbase, nullptr, tid);
+  } else {
+    write_list_base<false>(list, n, m, nbase, sink, window, 1, list_width, nullptr, nullptr, tid, kThreads);
+  }
+  __syncthreads();
+  row_attend<DT, D>(q_ + b * q_sb + h * q_sh, k_ + b * k_sb + kvh * k_sh, k_ss, v_ + b * v_sb + kvh * v_sh, v_ss, list,
+                    min(nbase + m, list_width), list_width, kv_rows, sm_scale, waves, out + b * out_sb + h * out_sh);
+}
+
 int next_pow2(int x) {
   int p = 1;
   while (p < x) p <<= 1;
@@ -1253,4 +1301,45 @@ extern "C" int socket_select_list_allowed(const float* scores, int64_t score_str
   SOCKET_REQUIRE(allowed, SOCKET_ERR_NULL);
   return select_entry(scores, allowed, score_stride, nullptr, nullptr, nullptr, 0, B, Hq, T, M, sink, window, 1, sparse_list,
                       list_stride, list_width, sparse_len, workspace, workspace_bytes, stream);
+}
+
+extern "C" int socket_select_attend_fits(int B, int Hq, int D, int T, int list_width, int dtype) {
+  const int eb = socket_dtype_bytes(dtype);
+  if (eb == 0 || B <= 0 || Hq <= 0 || T <= 0 || list_width <= 0 || (D != 64 && D != 128)) return 0;
+  const int most = eb == 4 ? row_entries<DType_f32>(D) : row_entries<DType_bf16>(D);
+  return T <= kPoolCap && list_width <= most && list_width <= kFuseList && (int64_t)B * Hq <= socket_device_limits().cu_count;
+}
+
+extern "C" int socket_select_attend(const float* scores, int64_t score_stride, const int32_t* lens, const int32_t* budgets, int T,
+                                    int M, int sink, int window, int list_width, const void* q, const void* k, const void* v,
+                                    int dtype, int64_t q_stride_b, int64_t q_stride_h, int64_t k_stride_b, int64_t k_stride_h,
+                                    int64_t k_stride_s, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_s, void* out,
+                                    int64_t out_stride_b, int64_t out_stride_h, int B, int Hq, int Hkv, int D, int kv_rows,
+                                    void* stream) {
+  SOCKET_REQUIRE(scores && q && k && v && out, SOCKET_ERR_NULL);
+  SOCKET_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && T > 0 && kv_rows > 0, SOCKET_ERR_SHAPE);
+  SOCKET_REQUIRE(M >= 0 && sink >= 0 && window >= 0, SOCKET_ERR_SHAPE);
+  SOCKET_REQUIRE(score_stride >= T && list_width > 0, SOCKET_ERR_SHAPE);
+  SOCKET_REQUIRE(socket_select_attend_fits(B, Hq, D, T, list_width, dtype), SOCKET_ERR_UNSUPPORTED);
+  const int per16 = 16 / socket_dtype_bytes(dtype);
+  SOCKET_REQUIRE(socket_aligned16(q) && socket_aligned16(k) && socket_aligned16(v), SOCKET_ERR_ALIGN);
+  for (int64_t st : {q_stride_b, q_stride_h, k_stride_b, k_stride_h, k_stride_s, v_stride_b, v_stride_h, v_stride_s})
+    SOCKET_REQUIRE(st % per16 == 0, SOCKET_ERR_ALIGN);
+#define SOCKET_SA(DT, DD)                                                                                                          \
+  hipLaunchKernelGGL((select_attend_kernel<DT, DD>), dim3(B * Hq), dim3(kThreads), 0, (hipStream_t)stream, scores, score_stride, lens, \
+                     budgets, Hq, T, M, sink, window, list_width, (const DT::storage*)q, (const DT::storage*)k, (const DT::storage*)v, \
+                     q_stride_b, q_stride_h, k_stride_b, k_stride_h, k_stride_s, v_stride_b, v_stride_h, v_stride_s, Hq / Hkv,      \
+                     kv_rows, 1.0f / sqrtf((float)D), (DT::storage*)out, out_stride_b, out_stride_h)
+#define SOCKET_SA_D(DT)             \
+  do {                              \
+    if (D == 128) SOCKET_SA(DT, 128); \
+    else SOCKET_SA(DT, 64);         \
+  } while (0)
+  if (dtype == SOCKET_F32) SOCKET_SA_D(DType_f32);
+  else if (dtype == SOCKET_F16) SOCKET_SA_D(DType_f16);
+  else SOCKET_SA_D(DType_bf16);
+#undef SOCKET_SA_D
+#undef SOCKET_SA
+  SOCKET_LAUNCH_CHECK();
+  return SOCKET_OK;
 }

@@ -24,7 +24,7 @@ import torch
 
 from ._lib import check, dtype_enum, lib, plain_tensors, ptr, stream_ptr
 from .socket_kernels import prefers_one_launch, sparse_attention_fwd, sparse_attention_fwd_static
-from .sparse import select_list
+from .sparse import select_attend, select_list
 
 
 HASH_DIM = 128     # coordinates the hashing kernel contracts over
@@ -419,6 +419,10 @@ def sparse_decode_step(q: torch.Tensor, q_probs: torch.Tensor, k_cache: torch.Te
     # the selection reads a row up to the same `lens`)
     scores = score_packed(q_probs, codes, v_norm, T, P, lens=lens, n_heads=q.shape[1], out=scores_buf,
                           skip_masked=not return_details)
+    if not return_details:
+        out = select_attend(scores, q, k_cache, v_cache, sink, window, M, lens=lens, budgets=budgets)
+        if out is not None:
+            return out
     sparse_list, sparse_len = select_list(scores, sink, window, M, lens=lens, budgets=budgets)
     B, Hq, D = q.shape
     if _use_one_launch(q, sparse_list.shape[-1], one_launch):

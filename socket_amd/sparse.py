@@ -13,11 +13,14 @@ use `socket_amd.hash_cache`.
 from __future__ import annotations
 
 import collections
+import functools
+from typing import Optional
 
 import torch
 
 from ._lib import SOCKET_TOPK_MAX_M, check, dtype_enum, lib, ptr, stream_ptr
 from .socket_kernels import (  # noqa: F401  (re-exported, as in the reference module)
+    _check_qkv,
     attention_mask_to_allowed_prob,
     sparse_attention_fwd,
     sparse_decode_stage1,
@@ -88,6 +91,39 @@ def reset_select_workspaces() -> None:
         ws[:zero_bytes].zero_()
 
 
+def _base_width(T: int, sink: int, window: int) -> int:
+    """Entries of a list's sink and window part over T positions."""
+    s_e, w_e = max(0, min(sink, T)), max(0, min(window, T))
+    return max(1, s_e + (T - max(T - w_e, s_e) if w_e > 0 else 0))
+
+
+@functools.lru_cache(maxsize=1024)
+def _select_attend_fits(B: int, H: int, D: int, T: int, width: int, dtype: torch.dtype) -> bool:
+    return dtype in (torch.float32, torch.bfloat16, torch.float16) and bool(
+        lib().socket_select_attend_fits(B, H, D, T, width, dtype_enum(dtype)))
+
+
+def select_attend(scores: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sink: int, window: int, M: int, *,
+                  lens=None, budgets=None) -> Optional[torch.Tensor]:
+    """`select_list` and the attention of q [B,H,D] over its list of rows of k / v [B,Kv,S,D] as one launch: [B,H,D], or None
+    where the two are launches of their own (long rows or lists, more rows than CUs, operands one of them would refuse)."""
+    B, H, T = scores.shape
+    D = q.shape[-1]
+    width = _base_width(T, sink, window) + min(int(M), T)
+    if M < 0 or sink < 0 or window < 0 or not _select_attend_fits(B, H, D, T, width, q.dtype):
+        return None
+    _check_qkv(q, k, v)
+    assert scores.is_cuda and scores.dtype == torch.float32
+    assert scores.stride(2) == 1 and scores.stride(0) == H * scores.stride(1)
+    out = torch.empty((B, H, D), dtype=q.dtype, device=q.device)
+    ks, vs = k.stride(), v.stride()
+    check("socket_select_attend", lib().socket_select_attend(
+        ptr(scores), scores.stride(1), ptr(lens), ptr(budgets), T, int(M), int(sink), int(window), width, ptr(q), ptr(k), ptr(v),
+        dtype_enum(q.dtype), q.stride(0), q.stride(1), ks[0], ks[1], ks[2], vs[0], vs[1], vs[2], ptr(out), H * D, D,
+        B, H, k.shape[1], D, k.shape[2], stream_ptr(q.device)))
+    return out
+
+
 def select_list(scores: torch.Tensor, sink: int, window: int, M: int, *, lens=None, budgets=None,
                 write_base: bool = True, list_width=None, row_range=None, split: bool = True):
     """Top-M + [sink | window | heavy] assembly on fp32 score rows [B,H,T]
@@ -104,12 +140,7 @@ def select_list(scores: torch.Tensor, sink: int, window: int, M: int, *, lens=No
     if M > SOCKET_TOPK_MAX_M:
         raise RuntimeError(f"top-k budget {M} exceeds the supported maximum {SOCKET_TOPK_MAX_M}")
     if list_width is None:
-        s_e, w_e = max(0, min(sink, T)), max(0, min(window, T))
-        nbase = 0
-        if write_base:
-            nbase = s_e + (T - max(T - w_e, s_e) if w_e > 0 else 0)
-            nbase = max(nbase, 1)
-        list_width = nbase + min(M, T)
+        list_width = (_base_width(T, sink, window) if write_base else 0) + min(M, T)
     sparse_list = torch.empty((B, H, list_width), dtype=torch.int32, device=scores.device)
     sparse_len = torch.empty((B, H), dtype=torch.int32, device=scores.device)
     if list_width == 0:
