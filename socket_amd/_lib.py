@@ -9,6 +9,7 @@ raises at first use with the build command to run.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p, POINTER
 
@@ -18,6 +19,7 @@ from torch.utils._device import DeviceContext
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsocket_hip.so")
+HOST_PATH = os.path.join(_HERE, "_host.so")
 CORE_PATH = os.path.join(_HERE, "libsocket_core.so")
 
 SOCKET_OK = 0
@@ -212,6 +214,7 @@ SIGNATURES = {
 
 _lib = None
 _core = None
+_host = None
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
@@ -251,6 +254,18 @@ def core() -> ctypes.CDLL:
     if _core is None:
         _core = _load(CORE_PATH, CORE_SIGNATURES, "python -m socket_amd.build --core")
     return _core
+
+
+def host():
+    """The native module that hands tensors to the library (csrc/host.cpp); raises if it is not built."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            _host = importlib.import_module("._host", __package__)
+        except ModuleNotFoundError as e:
+            raise RuntimeError("socket_amd/_host.so is missing: build it with `python -m socket_amd.build`. There is no fallback path.") from e
+    return _host
 
 
 def check(fn: str, status: int) -> None:

@@ -6,7 +6,8 @@ linked into two libraries next to this file: libsocket_core.so (what every model
 family uses: decode-step helpers, dense attention, chunked and latent attention,
 gated recurrences) and libsocket_hip.so (hashing, scoring, selection and block-sparse
 attention of the SOCKET path), which depends on it.  `build_core()` makes the first
-alone.
+alone.  _host.so is a Python module (csrc/host.cpp, host code only) that hands tensors to
+libsocket_hip.so.
 """
 from __future__ import annotations
 
@@ -20,6 +21,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libsocket_hip.so")
 CORE_PATH = os.path.join(HERE, "libsocket_core.so")
+HOST_PATH = os.path.join(HERE, "_host.so")
 CORE_SOURCES = ["common.hip", "attend.hip", "decode_ops.hip", "rows.hip", "chunk_attend.hip", "prompt_attend.hip", "latent.hip",
                 "recurrence.hip"]
 SOURCES = ["score.hip", "score_short.hip", "collide.hip", "topk.hip", "hash.hip", "softhash.hip", "block_sparse.hip"]
@@ -101,13 +103,34 @@ def build_core(verbose: bool = False, extra_flags=(), only_changed: bool = False
     return CORE_PATH
 
 
+def build_host(only_changed: bool = False) -> str:
+    """Compile _host.so against this interpreter and this torch; libsocket_hip.so must be there."""
+    src = os.path.join(CSRC, "host.cpp")
+    if only_changed and not _stale(src, HOST_PATH):
+        return HOST_PATH
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    tmp = "%s.%d.tmp" % (HOST_PATH, os.getpid())
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
+          "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I" + sysconfig.get_paths()["include"],
+          *["-I" + d for d in cpp_extension.include_paths()], src, "-L" + lib, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+          "-L" + HERE, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN", "-o", tmp])
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
 def build(verbose: bool = False, extra_flags=(), only_changed: bool = False) -> str:
     """Compile every source (or, with only_changed, those newer than their
-    object) and link both libraries."""
+    object) and link both libraries and the Python module."""
     n = len(CORE_SOURCES)
     objs = _compile(CORE_SOURCES + SOURCES, verbose, extra_flags, only_changed)
     _link(objs[:n], CORE_PATH)
     _link(objs[n:], LIB_PATH, CORE_PATH, "-Wl,-rpath,$ORIGIN")
+    build_host(only_changed)
     return LIB_PATH
 
 

@@ -22,7 +22,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from ._lib import check, dtype_enum, lib, plain_tensors, ptr, stream_ptr
+from ._lib import check, dtype_enum, host, lib, observed, ptr, stream_ptr
 from .socket_kernels import prefers_one_launch, sparse_attention_fwd, sparse_attention_fwd_static
 from .sparse import select_attend, select_list
 
@@ -498,15 +498,9 @@ class SocketHashCache:
         if pos0 < 0 or pos0 + S > self.Tcap:
             raise RuntimeError(
                 f"KVCache.update out-of-bounds: positions [{pos0},{pos0 + S - 1}] but cache T={self.Tcap}")
-        if self._append_fits(k_bshd, v_bshd):
-            kc, ks, vs = self.k_cache, k_bshd.stride(), v_bshd.stride()
-            cs = kc.stride()
-            check("socket_cache_append", lib().socket_cache_append(
-                k_bshd.data_ptr(), v_bshd.data_ptr(), dtype_enum(kc.dtype), ks[0], ks[2], ks[1], vs[0], vs[2], vs[1],
-                self.planes_words.data_ptr(), kc.data_ptr(), self.v_cache.data_ptr(), cs[0], cs[1], cs[2], self.codes.data_ptr(),
-                self.v_norm.data_ptr(), self.lens.data_ptr(), int(pos0), B, H, S, D, self.L, self.P, self.Tcap,
-                stream_ptr(kc.device)))
-            return
+        status = self._native_append(k_bshd, v_bshd, int(pos0), True)
+        if status >= 0:
+            return check("socket_cache_append", status)
         with torch.no_grad():
             self.k_cache[:, :, pos0:pos0 + S].copy_(k_bshd.permute(0, 2, 1, 3))
             self.v_cache[:, :, pos0:pos0 + S].copy_(v_bshd.permute(0, 2, 1, 3))
@@ -514,21 +508,13 @@ class SocketHashCache:
                            self.planes_words, self.codes, self.v_norm, self.L, self.P, t0=pos0)
             self.lens.fill_(pos0 + S)      # the cached length follows the position
 
+    def _native_append(self, k: torch.Tensor, v: torch.Tensor, pos0: int, run: bool) -> int:
+        """Whether one call of the library copies and hashes these rows (-1: no, torch's copies and then the hash; an
+        append is never differentiated), and with `run` that call's status."""
+        if observed() or not self.k_cache.is_cuda:
+            return -1
+        return host().cache_append(k, v, self.k_cache, self.v_cache, self.codes, self.v_norm, self.lens, self.planes_words, pos0,
+                                   self.L, self.P, self.Tcap, stream_ptr(self.k_cache.device), run)
+
     def _append_fits(self, k: torch.Tensor, v: torch.Tensor) -> bool:
-        """Whether one call of the library copies and hashes these rows (else: torch's copies, then the hash)."""
-        kc, vc, codes, norms, lens, words = self.k_cache, self.v_cache, self.codes, self.v_norm, self.lens, self.planes_words
-        # (an append is never differentiated)
-        if not plain_tensors(k, v, kc, vc, codes, norms, lens, words, grad=False):
-            return False
-        dt, shape = kc.dtype, k.shape
-        if not (k.dtype == v.dtype == dt == vc.dtype and dt in (torch.bfloat16, torch.float16, torch.float32) and shape == v.shape):
-            return False
-        B, S, H, D = shape
-        cb, ch, _, cd = kc.shape
-        if not (H == ch and D == cd and S > 0 and D % 8 == 0 and D <= HASH_DIM and words.shape[1] == HASH_DIM and cb * ch <= 65535
-                and kc.is_contiguous() and vc.is_contiguous() and codes.is_contiguous() and norms.is_contiguous()
-                and lens.is_contiguous() and words.is_contiguous()):
-            return False
-        ks, vs = k.stride(), v.stride()
-        return (ks[3] == vs[3] == 1 and (ks[0] | ks[1] | ks[2] | vs[0] | vs[1] | vs[2]) % (16 // kc.element_size()) == 0
-                and (k.data_ptr() | v.data_ptr() | kc.data_ptr() | vc.data_ptr()) % 16 == 0)
+        return self._native_append(k, v, 0, False) == 0
