@@ -22,6 +22,7 @@
 // collide.hip.)
 
 #include "score_entry.h"
+#include "score_deal.h"
 
 namespace {
 
@@ -681,71 +682,9 @@ __global__ __launch_bounds__(1024) void score_flat_kernel(
   const int chunk_elems = chunk_words * CPW * R * GP;
   const int offl = wave * kFlatUnit + lane * 4;      // the lane's first token in a tile (group j: + 256 j)
 
-  // ---- this workgroup's stretch of the flattened unit space -----------------------------
-  int len_l = 0;                                     // lane l: cached length of sequence l
-  if (lane < B) len_l = lens ? max(0, min(lens[lane], T)) : T;
-  const int u_l = (len_l + kFlatUnit - 1) / kFlatUnit;
-  const int incl = wave_incl_scan(u_l);
-  // Rows are (sequence, kv head) pairs, each as long as its sequence, laid end to end in
-  // units.  The row space is cut into equal stretches, and the tiles of a stretch -- every
-  // row segment in ceil(n / 16) tiles of equal size, the head parts of a tile next to each
-  // other -- are dealt in turn to the workgroups that share the stretch:
-  //   spread == 0: a stretch per workgroup (it walks consecutive tiles of one row); workgroup
-  //     n of N takes stretch (n % 8) * N / 8 + n / 8, so that neighbouring stretches, the
-  //     tiles of one row, sit on one XCD (workgroup n runs on XCD n % 8) and share its L2;
-  //   spread == 1: a stretch per XCD, its tiles dealt round to its workgroups.  They then work
-  //     on neighbouring tiles at any moment: few tables are live in the XCD's L2 however many
-  //     rows its stretch holds, and the parts of a wide head group, which read the same
-  //     codes, read them at the same time -- the second read is served by the L2.
-  const int nwg = gridDim.x;
-  const bool by_xcd = (nwg & 7) == 0;
-  const int ngroups = spread ? (by_xcd ? 8 : 1) : nwg, gsize = nwg / ngroups;
-  const int xcd = by_xcd ? (int)(blockIdx.x & 7) : 0, slot = by_xcd ? (int)(blockIdx.x >> 3) : (int)blockIdx.x;
-  const int group = spread ? xcd : (by_xcd ? xcd * (nwg >> 3) + slot : slot);
-  const int64_t total = (int64_t)__builtin_amdgcn_readlane(incl, 63) * Hkv;
-  const int64_t x0 = total * group / ngroups, x1 = total * (group + 1) / ngroups;
-  int wk_b = 0, wk_kvh = 0, wk_a = 0, wk_left = (int)(x1 - x0);
-  int wk_skip = spread ? slot : 0;   // tiles of the stretch before this workgroup's next
-  if (wk_left > 0) {
-    wk_b = __popcll(__builtin_amdgcn_ballot_w64((int64_t)incl * Hkv <= x0));
-    const int ub = __builtin_amdgcn_readlane(u_l, wk_b);
-    const int rem = (int)(x0 - (int64_t)(__builtin_amdgcn_readlane(incl, wk_b) - ub) * Hkv);
-    wk_kvh = rem / ub;
-    wk_a = rem % ub;
-  }
-  struct Tile {   // tokens [start, end) of row (b, vp); end <= the sequence's length; start == end: none
-    int b, vp, start, end;
-  };
-  auto next_tile = [&]() __attribute__((always_inline)) {
-    Tile t{0, 0, 0, 0};
-    while (wk_left > 0) {
-      const int ub = __builtin_amdgcn_readlane(u_l, wk_b);
-      const int n = min(ub - wk_a, wk_left);               // units of this row inside the stretch
-      const int k = (n + kFlatTileUnits - 1) / kFlatTileUnits;
-      const int sz = (n + k - 1) / k;
-      const int cnt = k * hsplit;
-      if (wk_skip < cnt) {
-        const int j = wk_skip / hsplit;
-        t.b = wk_b;
-        t.vp = wk_kvh * hsplit + wk_skip % hsplit;
-        t.start = (wk_a + j * sz) * kFlatUnit;
-        t.end = min((wk_a + min((j + 1) * sz, n)) * kFlatUnit, __builtin_amdgcn_readlane(len_l, wk_b));
-        wk_skip += gsize;
-        return t;
-      }
-      wk_skip -= cnt;
-      wk_left -= n;
-      wk_a = 0;
-      if (++wk_kvh == Hkv) {
-        wk_kvh = 0;
-        do ++wk_b;
-        while (wk_b < B && __builtin_amdgcn_readlane(u_l, wk_b) == 0);
-      }
-    }
-    return t;
-  };
-  auto codes_of = [&](const Tile& t) __attribute__((always_inline)) { return codes + (int64_t)(t.b * Hkv + t.vp / hsplit) * NW * Tcap; };
-  auto table_of = [&](const Tile& t) __attribute__((always_inline)) { return q_table + (int64_t)(t.b * VS + t.vp) * L * R * GP; };
+  ScoreDeal<kFlatUnit, kFlatTileUnits> deal(lens, B, Hkv, hsplit, T, spread);
+  auto codes_of = [&](const ScoreTile& t) __attribute__((always_inline)) { return codes + (int64_t)(t.b * Hkv + (t.vp >> (hsplit - 1))) * NW * Tcap; };
+  auto table_of = [&](const ScoreTile& t) __attribute__((always_inline)) { return q_table + (int64_t)(t.b * VS + t.vp) * L * R * GP; };
 
   float acc[KT4][4][GP];
   uint4 ring[kPrefetch][KT4];
@@ -772,16 +711,16 @@ __global__ __launch_bounds__(1024) void score_flat_kernel(
     const int t = start + offl + j * 256;
     return t < end ? t : start;
   };
-  auto load_norms = [&](const Tile& t) __attribute__((always_inline)) {
-    const uint16_t* vn = v_norm + (int64_t)(t.b * Hkv + t.vp / hsplit) * Tcap;
+  auto load_norms = [&](const ScoreTile& t) __attribute__((always_inline)) {
+    const uint16_t* vn = v_norm + (int64_t)(t.b * Hkv + (t.vp >> (hsplit - 1))) * Tcap;
 #pragma unroll
     for (int j = 0; j < KT4; ++j) vn_raw[j] = *reinterpret_cast<const uint2*>(vn + token_of(t.start, t.end, j));
   };
   // sums of a finished tile -> scores
-  auto flush = [&](const Tile& t) __attribute__((always_inline)) {
-    const int part = t.vp % hsplit, kvh = t.vp / hsplit;
+  auto flush = [&](const ScoreTile& t) __attribute__((always_inline)) {
+    const int part = (t.vp & (hsplit - 1)), kvh = (t.vp >> (hsplit - 1));
     const int geff = min(GP, G - part * GP);
-    const int len = __builtin_amdgcn_readlane(len_l, t.b);
+    const int len = deal.length(t.b);
     float* row0 = scores + (int64_t)(t.b * Hq + kvh * G + part * GP) * score_stride;
 #pragma unroll
     for (int j = 0; j < KT4; ++j) {
@@ -809,11 +748,11 @@ __global__ __launch_bounds__(1024) void score_flat_kernel(
     }
   };
 
-  Tile cur = next_tile();
+  ScoreTile cur = deal.next();
   if (cur.end > cur.start) {
-    Tile nxt = next_tile();
+    ScoreTile nxt = deal.next();
     bool more = nxt.end > nxt.start;
-    Tile prev = cur;
+    ScoreTile prev = cur;
     // what the ring fetches: the tile being scored and the one after it (itself when it is the last)
     const uint32_t* cur_codes = codes_of(cur);
     const uint32_t* nxt_codes = more ? codes_of(nxt) : cur_codes;
@@ -912,7 +851,7 @@ __global__ __launch_bounds__(1024) void score_flat_kernel(
     while (more) {
       prev = cur;
       cur = nxt;
-      nxt = next_tile();
+      nxt = deal.next();
       more = nxt.end > nxt.start;
       cur_codes = nxt_codes;
       nxt_codes = more ? codes_of(nxt) : cur_codes;
@@ -927,22 +866,7 @@ __global__ __launch_bounds__(1024) void score_flat_kernel(
     flush(cur);
   }
 
-  // ---- positions past a sequence's cached length ------------------------------------------------
-  if (fill_masked) {
-    for (int row = blockIdx.x; row < B * Hq; row += gridDim.x) {
-      const int len = __builtin_amdgcn_readlane(len_l, row / Hq);
-      float* dst = scores + (int64_t)row * score_stride;
-      // the scored tiles wrote -inf up to the next multiple of four past the length
-      const int from = (len + 3) & ~3;
-      for (int t = from + tid * 4; t < T; t += THREADS * 4) {
-        if (t + 4 <= T) {
-          store_stream16(dst + t, -INFINITY, -INFINITY, -INFINITY, -INFINITY);
-        } else {
-          for (int i = t; i < T; ++i) dst[i] = -INFINITY;
-        }
-      }
-    }
-  }
+  if (fill_masked) score_fill_past(scores, score_stride, deal.len_l, B, Hq, T);      // (positions past a sequence's cached length)
 }
 
 // How a workgroup's table passes through LDS: buffers, packed words per slice.

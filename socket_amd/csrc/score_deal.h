@@ -1,0 +1,149 @@
+// How the persistent scorer (score.hip) shares the cached tokens out among its workgroups.
+#pragma once
+#include "socket_common.h"
+
+namespace {
+
+// Tokens [start, end) of row (b, vp); end <= the sequence's length; start == end: none.
+struct ScoreTile {
+  int b, vp, start, end;
+};
+
+// Tokens are counted in units of UNIT, tiles have up to UNITS units.  Rows are (sequence, kv head) pairs, each as long as
+// its sequence, laid end to end in units.  The row space is cut into equal stretches, and the tiles of a stretch -- every
+// row segment in ceil(n / UNITS) tiles of equal size, the head parts of a tile next to each other -- are dealt in turn to
+// the workgroups that share the stretch:
+//   spread == 0: a stretch per workgroup (it walks consecutive tiles of one row); workgroup
+//     n of N takes stretch (n % 8) * N / 8 + n / 8, so that neighbouring stretches, the
+//     tiles of one row, sit on one XCD (workgroup n runs on XCD n % 8) and share its L2;
+//   spread == 1: a stretch per XCD, its tiles dealt round to its workgroups.  They then work
+//     on neighbouring tiles at any moment: few tables are live in the XCD's L2 however many
+//     rows its stretch holds, and the parts of a wide head group, which read the same
+//     codes, read them at the same time -- the second read is served by the L2.
+//     The tiles are then as small as the rounds they take allow (even_out below): dealt at their full size, a little
+//     more than one round took two, and all but a few workgroups stood idle in the last.  us of the scorer, full
+//     tiles / even ones: 8 sequences x 28 heads of 4, 60 tables x 1024, 40000 tokens 67.8 / 52.4, 81920: 101.5 / 95.0,
+//     32768 and 65536 (whole rounds) 39.0 / 38.8 and 72.4 / 72.1, ragged 57344: 65.4 / 49.8; 4 x 28 heads, 48 tables,
+//     131072 ragged 56.5 / 42.5; 8 x 32 heads, 65536 ragged 70.1 / 55.7; 32 tables x 256, 8 x 28 heads, 16384 tokens 13.8 / 13.5,
+//     65536 ragged 31.3 / 27.9.
+// (One wave ranks the lengths of up to 64 sequences.)
+template <int UNIT, int UNITS>
+struct ScoreDeal {
+  int B, Hkv, hsplit, gsize;
+  int len_l, u_l;                  // lane l: cached length of sequence l, and its units
+  int row_b, row_kvh, row_a, left; // where the stretch stands: sequence, kv head, unit; units left
+  int skip;                        // tiles of the stretch before this workgroup's next
+  int units;                       // of a tile at most
+
+  __device__ __forceinline__ ScoreDeal(const int32_t* lens, int B_, int Hkv_, int hsplit_, int T, int spread)
+      : B(B_), Hkv(Hkv_), hsplit(hsplit_), len_l(0), row_b(0), row_kvh(0), row_a(0) {
+    const int lane = threadIdx.x & 63;
+    if (lane < B) len_l = lens ? max(0, min(lens[lane], T)) : T;
+    u_l = (len_l + UNIT - 1) / UNIT;
+    const int incl = wave_incl_scan(u_l);
+    const int nwg = gridDim.x;
+    const bool by_xcd = (nwg & 7) == 0;
+    const int slot = by_xcd ? (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+    const int group = !spread ? (by_xcd ? (int)(blockIdx.x & 7) * (nwg >> 3) + slot : slot) : by_xcd ? (int)(blockIdx.x & 7) : 0;
+    gsize = !spread ? 1 : by_xcd ? nwg >> 3 : nwg;
+    // Stretches of total / groups units, the first of them with one of the remainder each.  (What comes before the first
+    // copy is a chain of scalar instructions that nothing hides, a 64-bit division some 150 of them; with two of those, and
+    // divisions by the one or two parts, a launch took 0.3 to 0.9 us longer.)
+    const uint32_t total = (uint32_t)(__builtin_amdgcn_readlane(incl, 63) * Hkv);
+    const uint32_t each = !spread ? total / (uint32_t)nwg : by_xcd ? total >> 3 : total;
+    const uint32_t more = !spread ? total - each * nwg : by_xcd ? total & 7 : 0;
+    const int x0 = (int)(each * group + min((uint32_t)group, more));
+    left = (int)(each + ((uint32_t)group < more ? 1 : 0));
+    skip = spread ? slot : 0;
+    if (left > 0) {
+      row_b = __popcll(__builtin_amdgcn_ballot_w64(incl * Hkv <= x0));
+      const uint32_t ub = (uint32_t)__builtin_amdgcn_readlane(u_l, row_b);
+      const uint32_t rem = (uint32_t)(x0 - (__builtin_amdgcn_readlane(incl, row_b) - (int)ub) * Hkv);
+      row_kvh = (int)(rem / ub);
+      row_a = (int)(rem - row_kvh * ub);
+    }
+    units = UNITS;
+    if (spread) even_out();
+  }
+
+  // The fewest units to a tile that need no more rounds than full tiles do, where at least an eighth of these would stand
+  // idle: lane l counts the tiles of up to l + 1 units.  (A few rows only: the count takes 0.15 us a row, which nothing hides,
+  // and many rows make many rounds: 16 sequences x 8 kv heads, 16384 tokens 57.0 us without it, 59.4 with.)
+  __device__ __forceinline__ void even_out() {
+    if (B * Hkv > 64 || left <= 0 || left >= 1 << 16 || left * hsplit % (UNITS * gsize) == 0) return;
+    const int most = min((int)(threadIdx.x & 63), UNITS - 1) + 1;
+    int b = row_b, kvh = row_kvh, a = row_a, rest = left, tiles = 0;
+    for (int r = 0; rest > 0; ++r) {
+      if (r == 12) return;
+      const int ub = __builtin_amdgcn_readlane(u_l, b), n = min(ub - a, rest);
+      tiles += tiles_of(n, most);
+      rest -= n;
+      a = 0;
+      if (++kvh == Hkv) {
+        kvh = 0;
+        do ++b;
+        while (b < B && __builtin_amdgcn_readlane(u_l, b) == 0);
+      }
+    }
+    const int full = __builtin_amdgcn_readlane(tiles, UNITS - 1) * hsplit;
+    const int fit = (full + gsize - 1) / gsize * gsize;
+    if (full * 8 <= fit * 7) units = (int)__ffsll((unsigned long long)__builtin_amdgcn_ballot_w64(tiles * hsplit <= fit));
+  }
+
+  // n / most rounded up (exact below 2^16: the half keeps the quotient 1 / 32 and more from a whole number)
+  static __device__ __forceinline__ int tiles_of(int n, int most) {
+    return (int)(((float)(n + most - 1) + 0.5f) * __builtin_amdgcn_rcpf((float)most));
+  }
+
+  __device__ __forceinline__ int length(int b) const { return __builtin_amdgcn_readlane(len_l, b); }
+
+  __device__ __forceinline__ ScoreTile next() {
+    ScoreTile t{0, 0, 0, 0};
+    while (left > 0) {
+      const int ub = __builtin_amdgcn_readlane(u_l, row_b);
+      const int n = min(ub - row_a, left);               // units of this row inside the stretch
+      int k = (n + UNITS - 1) / UNITS;
+      if (units != UNITS) {
+        asm volatile("");      // (a branch, not a choice between two results: a workgroup walks past many rows)
+        k = __builtin_amdgcn_readfirstlane(tiles_of(n, units));
+      }
+      const int cnt = k * hsplit;
+      if (skip < cnt) {
+        const int sz = (n + k - 1) / k;
+        const int j = skip >> (hsplit - 1);      // (one part or two)
+        t.b = row_b;
+        t.vp = row_kvh * hsplit + (skip & (hsplit - 1));
+        t.start = (row_a + j * sz) * UNIT;
+        t.end = min((row_a + min((j + 1) * sz, n)) * UNIT, __builtin_amdgcn_readlane(len_l, row_b));
+        skip += gsize;
+        return t;
+      }
+      skip -= cnt;
+      left -= n;
+      row_a = 0;
+      if (++row_kvh == Hkv) {
+        row_kvh = 0;
+        do ++row_b;
+        while (row_b < B && __builtin_amdgcn_readlane(u_l, row_b) == 0);
+      }
+    }
+    return t;
+  }
+};
+
+// Positions past each sequence's cached length: -inf.  (The scored tiles wrote it up to the next multiple of four.)
+__device__ __forceinline__ void score_fill_past(float* scores, int64_t score_stride, int len_l, int B, int Hq, int T) {
+  for (int row = blockIdx.x; row < B * Hq; row += gridDim.x) {
+    const int len = __builtin_amdgcn_readlane(len_l, row / Hq);
+    float* dst = scores + (int64_t)row * score_stride;
+    for (int t = ((len + 3) & ~3) + (int)threadIdx.x * 4; t < T; t += (int)blockDim.x * 4) {
+      if (t + 4 <= T) {
+        store_stream16(dst + t, -INFINITY, -INFINITY, -INFINITY, -INFINITY);
+      } else {
+        for (int i = t; i < T; ++i) dst[i] = -INFINITY;
+      }
+    }
+  }
+}
+
+}  // namespace
