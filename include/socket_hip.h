@@ -314,7 +314,7 @@ int socket_select_list(const float* scores, int64_t score_stride, const int32_t*
 /* socket_select_list (with write_base) and socket_sparse_attention over its list in one launch that needs no workspace and
  * leaves no list behind: out [B,Hq,D] as the two calls give it.  list_width as there.  For rows that
  * socket_select_attend_fits(B, Hq, D, T, list_width, dtype) names (SOCKET_ERR_UNSUPPORTED for others): at most 8192
- * scores, short lists, D of 64 or 128, no more rows than CUs. */
+ * scores, short lists, D of 64 or 128, no more rows than CUs.  M as there. */
 int socket_select_attend_fits(int B, int Hq, int D, int T, int list_width, int dtype);
 int socket_select_attend(const float* scores, int64_t score_stride, const int32_t* lens, const int32_t* budgets, int T, int M,
                          int sink, int window, int list_width, const void* q, const void* k, const void* v, int dtype,

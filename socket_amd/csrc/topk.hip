@@ -1320,6 +1320,7 @@ extern "C" int socket_select_attend(const float* scores, int64_t score_stride, c
   SOCKET_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && T > 0 && kv_rows > 0, SOCKET_ERR_SHAPE);
   SOCKET_REQUIRE(M >= 0 && sink >= 0 && window >= 0, SOCKET_ERR_SHAPE);
   SOCKET_REQUIRE(score_stride >= T && list_width > 0, SOCKET_ERR_SHAPE);
+  SOCKET_REQUIRE(M <= SOCKET_TOPK_MAX_M, SOCKET_ERR_UNSUPPORTED);
   SOCKET_REQUIRE(socket_select_attend_fits(B, Hq, D, T, list_width, dtype), SOCKET_ERR_UNSUPPORTED);
   const int per16 = 16 / socket_dtype_bytes(dtype);
   SOCKET_REQUIRE(socket_aligned16(q) && socket_aligned16(k) && socket_aligned16(v), SOCKET_ERR_ALIGN);

@@ -91,6 +91,11 @@ def reset_select_workspaces() -> None:
         ws[:zero_bytes].zero_()
 
 
+def _check_budget(M: int) -> None:
+    if M > SOCKET_TOPK_MAX_M:
+        raise RuntimeError(f"top-k budget {M} exceeds the supported maximum {SOCKET_TOPK_MAX_M}")
+
+
 def _base_width(T: int, sink: int, window: int) -> int:
     """Entries of a list's sink and window part over T positions."""
     s_e, w_e = max(0, min(sink, T)), max(0, min(window, T))
@@ -103,14 +108,26 @@ def _select_attend_fits(B: int, H: int, D: int, T: int, width: int, dtype: torch
         lib().socket_select_attend_fits(B, H, D, T, width, dtype_enum(dtype)))
 
 
+def _rows_agree(scores: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lens, budgets) -> bool:
+    """Whether each row of the scores has a query of its own, rows of k / v and, where given, an int32 length and budget, all
+    on one device: the one launch reads them by address, row by row of the scores."""
+    B, H, _ = scores.shape
+    return (q.dim() == 3 and tuple(q.shape[:2]) == (B, H) and k.dim() == 4 and k.shape == v.shape and k.shape[0] >= B
+            and all(t.device == scores.device for t in (q, k, v))
+            and all(t is None or (t.dtype == torch.int32 and t.device == scores.device and t.numel() == B and t.is_contiguous())
+                    for t in (lens, budgets)))
+
+
 def select_attend(scores: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sink: int, window: int, M: int, *,
                   lens=None, budgets=None) -> Optional[torch.Tensor]:
     """`select_list` and the attention of q [B,H,D] over its list of rows of k / v [B,Kv,S,D] as one launch: [B,H,D], or None
-    where the two are launches of their own (long rows or lists, more rows than CUs, operands one of them would refuse)."""
+    where the two are launches of their own (long rows or lists, more rows than CUs, operands that do not agree)."""
+    _check_budget(int(M))
     B, H, T = scores.shape
     D = q.shape[-1]
     width = _base_width(T, sink, window) + min(int(M), T)
-    if M < 0 or sink < 0 or window < 0 or not _select_attend_fits(B, H, D, T, width, q.dtype):
+    if (M < 0 or sink < 0 or window < 0 or not _select_attend_fits(B, H, D, T, width, q.dtype)
+            or not _rows_agree(scores, q, k, v, lens, budgets)):
         return None
     _check_qkv(q, k, v)
     assert scores.is_cuda and scores.dtype == torch.float32
@@ -137,8 +154,7 @@ def select_list(scores: torch.Tensor, sink: int, window: int, M: int, *, lens=No
     assert scores.stride(2) == 1 and scores.stride(0) == scores.shape[1] * scores.stride(1)
     B, H, T = scores.shape
     M = int(M)
-    if M > SOCKET_TOPK_MAX_M:
-        raise RuntimeError(f"top-k budget {M} exceeds the supported maximum {SOCKET_TOPK_MAX_M}")
+    _check_budget(M)
     if list_width is None:
         list_width = (_base_width(T, sink, window) if write_base else 0) + min(M, T)
     sparse_list = torch.empty((B, H, list_width), dtype=torch.int32, device=scores.device)
@@ -192,8 +208,7 @@ def _build_in_place(q_probs, k_hard, v_norm, allowed, sink: int, window: int, M:
             or tuple(k_hard.shape[:2]) != (B, H) or tuple(v_norm.shape) != (B, H, T) or tuple(allowed.shape) != (B, H, T)
             or not all(t.device == q_probs.device for t in (k_hard, v_norm, allowed))):
         return None
-    if M > SOCKET_TOPK_MAX_M:
-        raise RuntimeError(f"top-k budget {M} exceeds the supported maximum {SOCKET_TOPK_MAX_M}")
+    _check_budget(M)
     q_probs, k_hard, v_norm, allowed = (t.contiguous() for t in (q_probs, k_hard, v_norm, allowed))
     sink, window = max(0, min(sink, T)), max(0, min(window, T))
     base = max(1, sink + (T - max(T - window, sink) if window > 0 else 0))
