@@ -39,6 +39,8 @@
 // bin's counter handed it, the scan that finds the m-th bin turns the counters
 // into offsets, and when that one pass isolates the bin (the usual case) the
 // winners are grouped by bin with no second count.
+#include <utility>
+
 #include "attend_row.h"
 
 
@@ -64,6 +66,23 @@ typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 // The key of minus infinity, which scores of masked positions are.
 constexpr uint32_t kMaskedKey = 0x007fffffu;
+
+// f(0) to f(N - 1), each index a constant from the start.  (An array that an unrolled loop indexes may still be one vector
+// when registers are given out.  The slots of select_from_pool were one of eight registers, which the half workgroup moved to
+// scratch and back around every entry, 80 spilled registers in all.  us, that loop / this: masked rows, 512 of 8192 23.2 / 10.5,
+// 512 of 32768 29.2 / 20.7, 700 of 9000 32.6 / 21.3, 448 of 98304 48.7 / 41.1; unmasked, 448 of 98304 38.1 / 37.7.)
+template <int I>
+struct IntTag {
+  static constexpr int value = I;
+};
+template <int... I, class F>
+__device__ __forceinline__ void for_indices(std::integer_sequence<int, I...>, F&& f) {
+  (f(IntTag<I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void for_constant(F&& f) {
+  for_indices(std::make_integer_sequence<int, N>{}, f);
+}
 
 template <bool B>
 struct BoolTag {
@@ -664,16 +683,14 @@ __device__ __forceinline__ void select_from_pool(const u64 (&pv)[kPoolCap / THRE
   // finds the bin, and those slots place every winner next to the others of its
   // bin and the k-th bin's entries in their list with no further counting.
   {
-    uint32_t slot2[U / 2];   // 16 bits per entry
-#pragma unroll
-    for (int u = 0; u < U / 2; ++u) slot2[u] = 0;   // (hist is zero: cleared ahead of the pool)
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
+    uint32_t slot2[U / 2] = {};   // 16 bits per entry  (hist is zero: cleared ahead of the pool)
+    for_constant<U>([&](auto i) __attribute__((always_inline)) {
+      constexpr int u = decltype(i)::value;
       if (have >> u & 1) {
         const uint32_t sl = atomicAdd(&hist[level0_bin<MASKED>(pv[u], lo0, shift0)], 1u);
         slot2[u >> 1] |= sl << (16 * (u & 1));
       }
-    }
+    });
     __syncthreads();
     find_bin<THREADS, true>(hist, m, 1, sh, tid, [&](int bin, int before, int count) {
       const u64 blo = lo0 + ((u64)bin << shift0);
@@ -685,8 +702,8 @@ __device__ __forceinline__ void select_from_pool(const u64 (&pv)[kPoolCap / THRE
     });
     if (sh.done && !sh.crowded) {
       const int fb = sh.found_bin, need = sh.need, ncand = min(sh.found_count, kCandCap);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for_constant<U>([&](auto i) __attribute__((always_inline)) {
+        constexpr int u = decltype(i)::value;
         if (have >> u & 1) {
           const u64 v = pv[u];
           const int bin = level0_bin<MASKED>(v, lo0, shift0);
@@ -694,7 +711,7 @@ __device__ __forceinline__ void select_from_pool(const u64 (&pv)[kPoolCap / THRE
           if (bin > fb) buf[(int)(hist[bin] & 0xffffu) + sl] = v;
           else if (bin == fb && sl < kCandCap) cand[sl] = v;
         }
-      }
+      });
       __syncthreads();
       order_and_write<MASKED, THREADS>(buf, m - need, cand, ncand, need, lo0, shift0, tmp, hist, sh, counting_ok, heavy,
                                        ok, tid, true);
