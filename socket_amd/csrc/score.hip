@@ -644,7 +644,7 @@ __global__ __launch_bounds__(THREADS) void score_packed_kernel(
 // row as long as its sequence's cached length, are laid end to end and cut into equal
 // stretches, whose tiles -- up to 16 units of one row for one part of the head group;
 // the waves past a short tile's end skip the lookups and only join the copies and
-// barriers -- are dealt to the workgroups (how: at `spread` below).  Across a tile
+// barriers -- are dealt to the workgroups (how: score_deal.h).  Across a tile
 // boundary nothing drains: the last LDS slice of a tile is gathered from while
 // the first slice of the next tile's table is being copied, the code ring fetches
 // the next tile's first words where it would run past the current tile's last, and

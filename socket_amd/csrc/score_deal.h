@@ -1,5 +1,6 @@
 // How the persistent scorer (score.hip) shares the cached tokens out among its workgroups.
 #pragma once
+#include "score_stretch.h"
 #include "socket_common.h"
 
 namespace {
@@ -46,14 +47,12 @@ struct ScoreDeal {
     const int slot = by_xcd ? (int)(blockIdx.x >> 3) : (int)blockIdx.x;
     const int group = !spread ? (by_xcd ? (int)(blockIdx.x & 7) * (nwg >> 3) + slot : slot) : by_xcd ? (int)(blockIdx.x & 7) : 0;
     gsize = !spread ? 1 : by_xcd ? nwg >> 3 : nwg;
-    // Stretches of total / groups units, the first of them with one of the remainder each.  (What comes before the first
-    // copy is a chain of scalar instructions that nothing hides, a 64-bit division some 150 of them; with two of those, and
-    // divisions by the one or two parts, a launch took 0.3 to 0.9 us longer.)
+    // (What comes before the first copy is a chain of scalar instructions that nothing hides, a 64-bit division some 150 of
+    // them; with two of those, and divisions by the one or two parts, a launch took 0.3 to 0.9 us longer.)
     const uint32_t total = (uint32_t)(__builtin_amdgcn_readlane(incl, 63) * Hkv);
-    const uint32_t each = !spread ? total / (uint32_t)nwg : by_xcd ? total >> 3 : total;
-    const uint32_t more = !spread ? total - each * nwg : by_xcd ? total & 7 : 0;
-    const int x0 = (int)(each * group + min((uint32_t)group, more));
-    left = (int)(each + ((uint32_t)group < more ? 1 : 0));
+    const ScoreStretch mine = score_stretch(total, (uint32_t)group, (uint32_t)(!spread ? nwg : by_xcd ? 8 : 1));
+    const int x0 = (int)mine.start;
+    left = (int)mine.size;
     skip = spread ? slot : 0;
     if (left > 0) {
       row_b = __popcll(__builtin_amdgcn_ballot_w64(incl * Hkv <= x0));

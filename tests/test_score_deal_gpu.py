@@ -1,5 +1,6 @@
-"""The persistent scorer's dealing of a wide head group's tiles (evened out over the rounds they take, or full where a
-stretch has more rows than a wave has lanes): every token of every row scored, bit for bit the definition's sum."""
+"""The persistent scorer's dealing of its tiles: of a wide head group, dealt round (evened out over the rounds they take, or full
+past 64 rows in all or 12 in a stretch), and of a group in one part, a stretch to a workgroup.  Every token of every row scored,
+bit for bit the definition's sum."""
 import pytest
 import torch
 
@@ -22,6 +23,27 @@ DEV, L, P, G = "cuda", 16, 8, 7
     (40, 1, 30000, "short"),      # rows of very different lengths: a stretch of many, one of a few
 ])
 def test_every_token_is_scored(B, Hkv, T, lengths):
+    _check(B, Hkv, G, T, lengths)
+
+
+@pytest.mark.parametrize("group", [2, 4])
+@pytest.mark.parametrize("B,Hkv,T,lengths", [
+    (1, 8, 131072, 12000),        # one and a half units of 256 a workgroup, rows and stretches ending together
+    (1, 8, 131072, 4000),         # fewer units than workgroups
+    (1, 8, 131072, 1),            # one a row
+    (2, 5, 131072, "ragged"),
+    (1, 8, 131072, "full"),
+    (9, 8, 8192, "short"),        # rows of no, one and a few units, empty ones first and last
+    (64, 1, 9000, "one"),
+    (7, 5, 30001, "short"),
+])
+def test_a_stretch_to_a_workgroup(B, Hkv, T, lengths, group):
+    assert hash_cache.lib().socket_score_persistent_serves(B, Hkv * group, Hkv, T, 0, L, P, 1 << P) == 1
+    assert hash_cache.lib().socket_score_lanes_serve(B, Hkv * group, Hkv, T, 0, L, P, 1 << P) == 0
+    _check(B, Hkv, group, T, lengths)
+
+
+def _check(B, Hkv, G, T, lengths):
     g = torch.Generator(device=DEV).manual_seed(B + T)
     table = torch.rand(B, Hkv * G, L, 1 << P, generator=g, device=DEV)
     codes = torch.randint(0, 1 << P, (B, Hkv, L, T), generator=g, device=DEV, dtype=torch.int16)
@@ -34,6 +56,8 @@ def test_every_token_is_scored(B, Hkv, T, lengths):
         lens = torch.randint(0, T + 1, (B,), generator=g, device=DEV, dtype=torch.int32)
     elif lengths == "short":
         lens = torch.tensor(([0, 1, 255, 256, 257, 511, 512, 513, 1024, 8192, 8193, T, 0] * 4)[:B], dtype=torch.int32, device=DEV)
+    elif isinstance(lengths, int):
+        lens = torch.full((B,), lengths, dtype=torch.int32, device=DEV)
     elif lengths == "one":
         lens = torch.zeros_like(lens)
         lens[B // 2] = T - 1
