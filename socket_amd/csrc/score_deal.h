@@ -62,36 +62,75 @@ struct ScoreDeal {
       row_a = (int)(rem - row_kvh * ub);
     }
     units = UNITS;
-    if (spread) even_out();
+    if (spread) even_out(incl, x0);
   }
 
   // The fewest units to a tile that need no more rounds than full tiles do, where at least an eighth of these would stand
-  // idle: lane l counts the tiles of up to l + 1 units.  (A few rows only: the count takes 0.15 us a row, which nothing hides,
-  // and many rows make many rounds: 16 sequences x 8 kv heads, 16384 tokens 57.0 us without it, 59.4 with.)
-  __device__ __forceinline__ void even_out() {
-    if (B * Hkv > 64 || left <= 0 || left >= 1 << 16 || left * hsplit % (UNITS * gsize) == 0) return;
-    const int most = min((int)(threadIdx.x & 63), UNITS - 1) + 1;
-    int b = row_b, kvh = row_kvh, a = row_a, rest = left, tiles = 0;
-    for (int r = 0; rest > 0; ++r) {
-      if (r == 12) return;
-      const int ub = __builtin_amdgcn_readlane(u_l, b), n = min(ub - a, rest);
-      tiles += tiles_of(n, most);
-      rest -= n;
-      a = 0;
-      if (++kvh == Hkv) {
-        kvh = 0;
-        do ++b;
-        while (b < B && __builtin_amdgcn_readlane(u_l, b) == 0);
-      }
+  // idle.  The count is 0.2 to 0.9 us that nothing hides: a few sequences one after another with a size to each lane, more of
+  // them a lane each and the size found by halves.  (Row after row, 0.15 us a row, it was left out past 64 rows in all and
+  // given up after 12 of a stretch.)  us of the scorer, full tiles / row after row / this, 60 tables x 1024 unless stated:
+  // 32 x 4 kv heads of 7, 12000 ragged 67.9 / 67.1 / 53.2, 20000 ragged 87 / 90 / 79, 6000 full 38.0 / 37.7 / 38.6; 20 x 4, 12000 57.5 /
+  // 57.7 / 47.1; 9 x 8, 20000 ragged 65.8 / 66.0 / 48.0, 12000 ragged 38.9 / 38.7 / 39.6; 16 x 4, most of 20000 short 41.4 / 46.7 /
+  // 38.5, 64 x 1 the same way 43.6 / 33.1 / 38.7; 16 x 8, 6000 full 37.6 / 37.4 / 38.4; 1 x 4, 8000 cached of 131072 22.1 / 15.9 / 16.2.
+  // Tiles of up to kPassage tokens cost the passage of the table and little else, and a stretch without longer sequences is
+  // not counted: 8 x 8 kv heads of 4 with 300 / 2000 / 4000 cached of 16384, full tiles 18.0 / 19.0 / 25.3, even ones with the
+  // count 19.2 / 19.8 / 20.4; 16 x 4 of 7, 48 tables, of 98304: 19.0 / 19.8 / 23.1 and 20.4 / 20.8 / 22.1.
+  static constexpr int kPassage = 2048;
+  static constexpr int kFewSequences = 4;
+  __device__ __forceinline__ void even_out(int incl, int x0) {
+    if (left <= 0 || left >= 1 << 16 || left * hsplit % (UNITS * gsize) == 0) return;
+    // lane l: the rows of sequence l in the stretch: units of the first, whole ones, units of the last
+    const int base = (incl - u_l) * Hkv;
+    const int p = max(x0 - base, 0), q = min(x0 + left - base, u_l * Hkv);
+    if (__builtin_amdgcn_ballot_w64(p < q && len_l > kPassage) == 0) return;
+    int head = 0, whole = 0, tail = 0;
+    if (p < q) {
+      const int first = quotient(p, u_l), last = quotient(q, u_l);
+      tail = q - last * u_l;
+      head = first == last ? q - p : (first + 1) * u_l - p;
+      whole = last - first - 1;
+      if (first == last) whole = tail = 0;
     }
-    const int full = __builtin_amdgcn_readlane(tiles, UNITS - 1) * hsplit;
-    const int fit = (full + gsize - 1) / gsize * gsize;
-    if (full * 8 <= fit * 7) units = (int)__ffsll((unsigned long long)__builtin_amdgcn_ballot_w64(tiles * hsplit <= fit));
+    const float headf = (float)head, rowf = (float)u_l, tailf = (float)tail;
+    const auto fits = [&](int full) __attribute__((always_inline)) { return (full + gsize - 1) / gsize * gsize; };
+    unsigned long long here = __builtin_amdgcn_ballot_w64(p < q);
+    if (__popcll(here) <= kFewSequences) {
+      // sequence after sequence, a size to each lane
+      const int most = min((int)(threadIdx.x & 63), UNITS - 1) + 1;
+      int n = 0;
+      for (; here; here &= here - 1) {
+        const int l = __ffsll(here) - 1;
+        auto of = [&](float v) __attribute__((always_inline)) {
+          return tiles_of(__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l)), most);
+        };
+        n += of(headf) + __builtin_amdgcn_readlane(whole, l) * of(rowf) + of(tailf);
+      }
+      const int full = __builtin_amdgcn_readlane(n, UNITS - 1) * hsplit, fit = fits(full);
+      if (full * 8 <= fit * 7) units = (int)__ffsll((unsigned long long)__builtin_amdgcn_ballot_w64(n * hsplit <= fit));
+      return;
+    }
+    // all sequences at once, the size found by halves
+    auto tiles = [&](int most) __attribute__((always_inline)) {
+      const int n = tiles_of(headf, most) + whole * tiles_of(rowf, most) + tiles_of(tailf, most);
+      return __builtin_amdgcn_readlane(wave_incl_scan(n), 63) * hsplit;
+    };
+    const int full = tiles(UNITS), fit = fits(full);
+    if (full * 8 > fit * 7) return;
+    static_assert((UNITS & (UNITS - 1)) == 0, "halves");
+#pragma unroll
+    for (int step = UNITS / 2; step > 0; step >>= 1)
+      if (tiles(units - step) <= fit) units -= step;
   }
 
   // n / most rounded up (exact below 2^16: the half keeps the quotient 1 / 32 and more from a whole number)
-  static __device__ __forceinline__ int tiles_of(int n, int most) {
-    return (int)(((float)(n + most - 1) + 0.5f) * __builtin_amdgcn_rcpf((float)most));
+  static __device__ __forceinline__ int tiles_of(float n, int most) {
+    const float r = __builtin_amdgcn_rcpf((float)most);
+    return (int)fmaf(n, r, ((float)most - 0.5f) * r);
+  }
+  // a / b for small quotients (the float's is one off at most)
+  static __device__ __forceinline__ int quotient(int a, int b) {
+    const int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b)), r = a - q * b;
+    return q + (r >= b ? 1 : 0) - (r < 0 ? 1 : 0);
   }
 
   __device__ __forceinline__ int length(int b) const { return __builtin_amdgcn_readlane(len_l, b); }
@@ -104,7 +143,7 @@ struct ScoreDeal {
       int k = (n + UNITS - 1) / UNITS;
       if (units != UNITS) {
         asm volatile("");      // (a branch, not a choice between two results: a workgroup walks past many rows)
-        k = __builtin_amdgcn_readfirstlane(tiles_of(n, units));
+        k = __builtin_amdgcn_readfirstlane(tiles_of((float)n, units));
       }
       const int cnt = k * hsplit;
       if (skip < cnt) {

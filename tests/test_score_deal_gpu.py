@@ -1,5 +1,5 @@
 """The persistent scorer's dealing of its tiles: of a wide head group, dealt round (evened out over the rounds they take, or full
-past 64 rows in all or 12 in a stretch), and of a group in one part, a stretch to a workgroup.  Every token of every row scored,
+where all sequences of a stretch are short), and of a group in one part, a stretch to a workgroup.  Every token of every row scored,
 bit for bit the definition's sum."""
 import pytest
 import torch
@@ -16,7 +16,10 @@ DEV, L, P, G = "cuda", 16, 8, 7
     (1, 1, 131072, "full"),       # a row over all XCDs, fewer tiles than workgroups
     (1, 3, 33000, "full"),
     (13, 5, 40000, "short"),      # rows of no, one and a few units
-    (64, 9, 1501, "full"),        # more rows than are counted
+    (64, 9, 1501, "full"),        # short rows, and many
+    (20, 4, 12000, "full"),       # 80 rows, three sequences to a stretch
+    (52, 2, 20000, "short"),      # stretches of many sequences, all lengths among them
+    (64, 1, 5000, "ragged"),      # eight sequences to a stretch
     (64, 9, 1501, "one"),         # all but one of them empty
     (64, 1, 9000, "ragged"),      # about eight rows
     (64, 1, 3001, "one"),
