@@ -52,9 +52,10 @@ def warmup_sparse_decode(model: Transformer, device: torch.device, *, T: int = 4
     k = torch.randn((B, Hl, Tcap, D), device=device, dtype=dtype)
     v = torch.randn((B, Hl, Tcap, D), device=device, dtype=dtype)
     cfg = attn.config
-    for _ in range(2):
-        hash_cache.sparse_decode_step(q, q_probs, k, v, codes, v_norm, T, P, int(cfg.sink_size),
-                                      int(cfg.window_size), int(attn.heavy_const))
+    for details in (False, True):      # (short rows have selection and attention in one launch; with details, and for long rows, two)
+        for _ in range(2):
+            hash_cache.sparse_decode_step(q, q_probs, k, v, codes, v_norm, T, P, int(cfg.sink_size),
+                                          int(cfg.window_size), int(attn.heavy_const), return_details=details)
     # the library's fixed scratch array is looked up here, outside any capture
     hash_cache.prepare_one_launch_attention(device)
     torch.cuda.synchronize()

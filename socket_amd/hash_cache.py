@@ -405,7 +405,8 @@ def sparse_decode_step(q: torch.Tensor, q_probs: torch.Tensor, k_cache: torch.Te
     step takes the re-entrant two-launch form with a workspace per call (same
     output, bit for bit).  Replays of graphs that hold this step must not overlap
     on one GPU.  True forces the one-launch form (the caller answers for the
-    serialisation), False forbids it.
+    serialisation), False forbids it.  It has no bearing on short rows whose selection and
+    attention are one launch (`sparse.select_attend`): that one shares nothing.
 
     `scores_buf`: an fp32 [B, Hq, T rounded up to 4] tensor to score into (67 MB at
     4 x 32 heads x 131072 tokens); without it the step allocates one per call, which an
@@ -422,6 +423,8 @@ def sparse_decode_step(q: torch.Tensor, q_probs: torch.Tensor, k_cache: torch.Te
     if not return_details:
         out = select_attend(scores, q, k_cache, v_cache, sink, window, M, lens=lens, budgets=budgets)
         if out is not None:
+            if one_launch is not False:      # (for a longer step that is recorded after this one)
+                prepare_one_launch_attention(q.device)
             return out
     sparse_list, sparse_len = select_list(scores, sink, window, M, lens=lens, budgets=budgets)
     B, Hq, D = q.shape
