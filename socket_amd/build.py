@@ -103,23 +103,37 @@ def build_core(verbose: bool = False, extra_flags=(), only_changed: bool = False
     return CORE_PATH
 
 
+def _host_made_for() -> str:
+    """The interpreter and the torch that _host.so is compiled against."""
+    import torch
+
+    return "python %s torch %s" % (sys.version, torch.__version__)
+
+
 def build_host(only_changed: bool = False) -> str:
-    """Compile _host.so against this interpreter and this torch; libsocket_hip.so must be there."""
-    src = os.path.join(CSRC, "host.cpp")
-    if only_changed and not _stale(src, HOST_PATH):
+    """Compile _host.so against this interpreter and this torch, whose headers it needs (`only_changed`: if it was made for
+    others, or is older than its source); libsocket_hip.so must be there."""
+    src, made_for = os.path.join(CSRC, "host.cpp"), os.path.join(HERE, "build", "host.txt")
+    if only_changed and not _stale(src, HOST_PATH) and os.path.exists(made_for) and open(made_for).read() == _host_made_for():
         return HOST_PATH
     import sysconfig
 
     import torch
     from torch.utils import cpp_extension
 
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        raise RuntimeError("Python.h not found in %s: _host.so needs the interpreter's headers (the libraries are built)" % include)
     tmp = "%s.%d.tmp" % (HOST_PATH, os.getpid())
     lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared",
-          "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I" + sysconfig.get_paths()["include"],
-          *["-I" + d for d in cpp_extension.include_paths()], src, "-L" + lib, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
-          "-L" + HERE, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN", "-o", tmp])
+    _run([_hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared",
+          "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I" + include,
+          *["-I" + d for d in cpp_extension.include_paths()], src, "-x", "none", "-L" + lib, "-ltorch_python", "-ltorch",
+          "-ltorch_cpu", "-lc10", "-L" + HERE, "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN", "-o", tmp])
     os.replace(tmp, HOST_PATH)
+    os.makedirs(os.path.dirname(made_for), exist_ok=True)
+    with open(made_for, "w") as f:
+        f.write(_host_made_for())
     return HOST_PATH
 
 
