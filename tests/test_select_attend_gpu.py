@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from socket_amd import hash_cache
 from socket_amd.sparse import select_attend, select_list
 
 pytestmark = pytest.mark.gpu
@@ -16,8 +17,17 @@ def _operands(dev, B, H, Hkv, T, D, dtype, seed):
     return scores, q, k, v
 
 
-def _check(got, scores, q, k, v, sink, window, M, lens=None, budgets=None):
-    lists, n = select_list(scores, sink, window, M, lens=lens, budgets=budgets)
+def _sorted_list(scores, sink, window, M):
+    """Sink, window and the M largest (NaN first, equal scores by index) of full rows, without the library."""
+    B, H, T = scores.shape
+    base = torch.tensor([i for i in range(T) if i < sink or i >= T - window], dtype=torch.int32, device=scores.device)
+    best = torch.sort(scores, dim=-1, descending=True, stable=True)[1][..., :M].to(torch.int32)
+    lists = torch.cat([base.expand(B, H, -1), best], -1)
+    return lists, torch.full((B, H), lists.shape[-1], dtype=torch.int32, device=scores.device)
+
+
+def _check(got, scores, q, k, v, sink, window, M, lens=None, budgets=None, listed=None):
+    lists, n = listed or select_list(scores, sink, window, M, lens=lens, budgets=budgets)
     B, H, D = q.shape
     G = H // k.shape[1]
     unit = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[q.dtype]
@@ -48,6 +58,55 @@ def test_against_float64(dev, dtype, T, M, window, D):
     got = select_attend(*ops, 4, window, M)
     assert got is not None
     _check(got, *ops, 4, window, M)
+
+
+# Rows whose m-th bin or bins of winners are full: more entries than are ranked or kept at once, a second pass over them, the
+# sort in place of counting.
+HARD = {
+    "equal": lambda s: s * 0 + 1.25,
+    "two values": lambda s: (s > 1).float(),
+    "three values": lambda s: (s > 0.5).float() + (s > 6).float(),
+    "a crowd above": lambda s: torch.where(s > 4, torch.full_like(s, 1e30), s),        # some 1400 winners in one bin
+    "two crowds": lambda s: torch.where(s > 25, torch.full_like(s, 1e30), torch.where(s > 12, torch.full_like(s, 9e29), s)),
+    "mostly masked": lambda s: torch.where(s > 12, s, torch.full_like(s, float("-inf"))),
+    "all masked": lambda s: torch.full_like(s, float("-inf")),
+    "extremes": lambda s: torch.where(s > 20, torch.full_like(s, float("inf")), torch.where(s < 0.1, torch.full_like(s, float("nan")), s)),
+    "tiny range": lambda s: 1 + (s * 3).floor() * 2.0 ** -23,
+    "wide range": lambda s: torch.where(s > 1, s * 1e30, s * 1e-30),
+}
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("T", [511, 4099, 8192])
+@pytest.mark.parametrize("kind", HARD)
+def test_hard_rows_against_a_stable_sort(dev, kind, T, dtype, D):
+    _, q, k, v = _operands(dev, 1, 4, 2, T, D, dtype, T)
+    g = torch.Generator(dev).manual_seed(T + 1)
+    scores = HARD[kind](torch.exp(1.5 * torch.randn(1, 4, T, generator=g, device=dev)))
+    for M in (1, 129, 400, 476):
+        got = select_attend(scores, q, k, v, 4, 32, M)
+        assert got is not None
+        _check(got, scores, q, k, v, 4, 32, M, listed=_sorted_list(scores, 4, 32, M))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [100, 4100, 8192])
+def test_a_step_without_details_is_the_step_with_them(dev, T, dtype):
+    L, P, B, H, Hkv, D, M = 12, 8, 2, 8, 2, 128, 150
+    _, q, k, v = _operands(dev, B, H, Hkv, T, D, dtype, T)
+    q, k, v = q.contiguous(), k[:, :, :T].contiguous(), v[:, :, :T].contiguous()
+    g = torch.Generator(dev).manual_seed(T)
+    words = torch.randint(0, 2 ** 31 - 1, (B, Hkv, hash_cache.words_per_key(L, P), T), generator=g, device=dev, dtype=torch.int32)
+    probs = torch.rand(B, H, L, 1 << P, generator=g, device=dev)
+    args = (q, probs, k, v, words, torch.rand(B, Hkv, T, generator=g, device=dev).half(), T, P, 4, 32, M)
+    lens = torch.tensor([T, T // 3], dtype=torch.int32, device=dev)
+    for more in ({}, {"lens": lens}, {"lens": lens, "budgets": torch.tensor([M, 17], dtype=torch.int32, device=dev)}):
+        want, scores, lists, n = hash_cache.sparse_decode_step(*args, return_details=True, **more)
+        got = hash_cache.sparse_decode_step(*args, **more)
+        if "lens" not in more:
+            assert torch.equal(lists.sort(-1)[0], _sorted_list(scores, 4, 32, min(M, T))[0].sort(-1)[0])
+        _check(want, scores, q, k, v, 4, 32, M, listed=(lists, n))
+        _check(got, scores, q, k, v, 4, 32, M, listed=(lists, n))
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
