@@ -1120,8 +1120,9 @@ __global__ __launch_bounds__(THREADS, 4) void select_list_kernel(
 // A short row's selection and its attention in one launch, a workgroup to a (b, h) row: the list stays in LDS.  Rows of at
 // most kPoolCap scores whose list is one pass of row_attend, no more rows than CUs.  What bounds it is a chain of short
 // phases on one CU; what it saves is a launch, and the list's way to memory and back.  Two launches / one, us: fp32, 32 rows
-// of 4096, 196 entries 14.5 / 11.8, 128 rows 15.4 / 12.3, 256 rows of 2000, 168 entries 17.2 / 13.5; bf16, 32 rows of 8000, 504
-// entries 17.5 / 15.8, 256 rows of 8192 27.2 / 20.9.
+// of 4096, 196 entries 13.0 / 10.7, 128 rows 15.4 / 12.3, 256 rows of 2000, 168 entries 17.2 / 13.5; bf16, 32 rows of 8000, 504
+// entries 15.7 / 13.9, 256 rows of 8192 27.2 / 20.9.  From one row up, where the two spread a row over many CUs: fp32, 1 / 8 rows of
+// 4096 11.7 / 9.9 and 12.6 / 10.4; bf16, 1 / 8 rows of 8000, 504 entries 13.9 / 12.7 and 14.5 / 12.9, of 8192, 508 entries of 64 dims 16.4 / 14.8.
 constexpr int kFuseList = 512;      // entries of a list at most
 template <class DT, int D>
 __global__ __launch_bounds__(kThreads, 4) void select_attend_kernel(
