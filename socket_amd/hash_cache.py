@@ -374,13 +374,10 @@ def _use_one_launch(q: torch.Tensor, width: int, one_launch: Optional[bool]) -> 
     if one_launch is False or not prefers_one_launch(B, Hq, D, width):
         return False
     idx = q.device.index if q.device.index is not None else torch.cuda.current_device()
-    capturing = torch.cuda.is_current_stream_capturing()
-    if not capturing:
-        prepare_one_launch_attention(q.device)
     if one_launch is True:
         return idx in _STATIC_READY
     # default: only inside a graph capture, whose replays the caller issues one after another
-    return capturing and idx in _STATIC_READY
+    return torch.cuda.is_current_stream_capturing() and idx in _STATIC_READY
 
 
 @torch.no_grad()
@@ -420,11 +417,11 @@ def sparse_decode_step(q: torch.Tensor, q_probs: torch.Tensor, k_cache: torch.Te
     # the selection reads a row up to the same `lens`)
     scores = score_packed(q_probs, codes, v_norm, T, P, lens=lens, n_heads=q.shape[1], out=scores_buf,
                           skip_masked=not return_details)
+    if one_launch is not False:      # (whichever form this step takes: one that is recorded later may need it)
+        prepare_one_launch_attention(q.device)
     if not return_details:
         out = select_attend(scores, q, k_cache, v_cache, sink, window, M, lens=lens, budgets=budgets)
         if out is not None:
-            if one_launch is not False:      # (for a longer step that is recorded after this one)
-                prepare_one_launch_attention(q.device)
             return out
     sparse_list, sparse_len = select_list(scores, sink, window, M, lens=lens, budgets=budgets)
     B, Hq, D = q.shape

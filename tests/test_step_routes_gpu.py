@@ -23,10 +23,11 @@ def _step(*operands, **more):
     return hash_cache.sparse_decode_step(*operands, **more)
 
 
+@pytest.mark.parametrize("T", [512, 9000])
 @pytest.mark.parametrize("rows", [32, 128])
-def test_a_short_eager_step_looks_the_scratch_array_up(dev, monkeypatch, rows):
+def test_an_eager_step_looks_the_scratch_array_up(dev, monkeypatch, rows, T):
     monkeypatch.setattr(hash_cache, "_STATIC_READY", set())
-    ops = _operands(dev, rows // 32, 512)
+    ops = _operands(dev, rows // 32, T)
     assert torch.isfinite(_step(*ops, one_launch=False)).all()
     assert hash_cache._STATIC_READY == set()
     _step(*ops)
