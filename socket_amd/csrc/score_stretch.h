@@ -5,10 +5,10 @@
 // Units [start, start + size) of `total` for stretch `group` of `groups`: start is total * group / groups rounded down, so
 // that the remainder is spread evenly over the groups and stretches end where rows do wherever the two divide.  In 32 bits
 // (group < groups <= 65535): total * g / n = each * g + more * g / n, with each = total / n and more = total % n.
-// (The remainder given to the first groups instead, a unit each, was 0.3 to 0.6 us shorter where few units are scored, and
-// lost far more: groups follow one another by XCD, so it left whole XCDs idle or with twice the work, and stretches over the
-// ends of rows, two tables where one would do.  us, that / this: 1 x 8 kv heads, 60 tables x 1024, capacity 131072, 12000 cached
-// tokens 25.9 / 15.2, 40000 26.6 / 16.3.)
+// (The remainder given to the first groups instead, a unit each: no faster where a workgroup has no more than a unit, and
+// groups follow one another by XCD, so it left whole XCDs idle or with twice the work, and stretches over the ends of rows,
+// two tables where one would do.  us, that / this: 8 kv heads of 4, 60 tables x 1024, capacity 131072, 4000 cached tokens 14.8 / 14.7,
+// 12000 26.0 / 14.7, 40000 26.8 / 16.0.)
 struct ScoreStretch {
   uint32_t start, size;
 };
