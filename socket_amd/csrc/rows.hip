@@ -8,6 +8,8 @@
 //    as an optional prologue, and a gated unit, a second scaled term, or the residual sum
 //    and the average over depth as epilogue.
 //  * gated_unit_kernel: the gated unit alone, for prompts.
+#include <algorithm>
+
 #include "elem.h"
 
 namespace {
@@ -137,56 +139,206 @@ __global__ __launch_bounds__(256) void gated_unit_kernel(const void* __restrict_
 }
 
 constexpr int kVec = 8;                    // weights per lane and load
-constexpr int kDepth = 4;                  // loads in flight per matrix
+constexpr int kDepth = 4;                  // loads of a chunk of a row
 constexpr int kChunkElems = 64 * kVec * kDepth;
-constexpr int kWgPerCu = 4;                // workgroups per CU of the persistent (NORM) launch
+constexpr int kWgPerCu = 4;                // workgroups per CU of a persistent launch
+constexpr int most_slots(int two) { return two == 1 ? 2 : 4; }      // chunks of a wave in flight: 16 KB
+constexpr int kInputVecs = 8;              // 16-byte vectors of a lane that wait in registers on their way to LDS
+
+__host__ __device__ __forceinline__ int chunks_of(int K) { return (K + kChunkElems - 1) / kChunkElems; }
 
 typedef uint32_t rl_u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-// kDepth weight vectors of row n, elements [kc * kChunkElems, ...), zero past K (FULL: K is a
-// multiple of kChunkElems, no element is past it).
-template <bool FULL>
-__device__ __forceinline__ void fetch_row(rl_u32x4 (&v)[kDepth], const uint16_t* w, int64_t n, int K, int kc, int lane) {
-#pragma unroll
-  for (int u = 0; u < kDepth; ++u) {
-    const int k = kc * kChunkElems + (u * 64 + lane) * kVec;
-    v[u] = (FULL || k < K) ? __builtin_nontemporal_load(reinterpret_cast<const rl_u32x4*>(w + n * K + k)) : rl_u32x4{0, 0, 0, 0};
-  }
+// Where the input rows come from.
+enum RowsInput {
+  kFromMemory,      // x1 (and x2), read from memory as they are used: rows that do not fit into LDS
+  kFromLds,         // x1 (and x2), brought into LDS
+  kNormRows,        // residual_row's, one row after the other, behind the first weights
+  kNormEarly2,      // residual_row's for one row of up to 2 float4 vectors a lane, its operands requested ahead of the weights
+  kNormEarly4,      // the same, up to 4
+};
+
+// A row of weights as a buffer: loads past its end give zeros and ask the memory for nothing, so that whether there is a
+// row at all is no branch (behind one, the compiler's wait for a chunk would be a wait for everything in flight).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(const uint16_t* w, int64_t n, int K, bool there) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w + (there ? n * K : 0)), 0, there ? K * 2 : 0, 0x00027000);
 }
 
-template <int M, bool FULL>
+constexpr int kStreaming = 2;              // cache policy of a buffer load: nt
+
+// Chunk kc of a row, kDepth vectors a lane.
+__device__ __forceinline__ void fetch_chunk(rl_u32x4 (&v)[kDepth], __amdgpu_buffer_rsrc_t row, int kc, int lane) {
+  const int at = kc * (kChunkElems * 2) + lane * 16;
+#pragma unroll
+  for (int u = 0; u < kDepth; ++u)
+    v[u] = __builtin_bit_cast(rl_u32x4, __builtin_amdgcn_raw_buffer_load_b128(row, at + u * 1024, 0, kStreaming));
+}
+
+// acc + the two products of bf16 pairs (an element of a vector has to be a value of its own here: a bit cast of the element
+// itself takes the vector's first)
+__device__ __forceinline__ float dot2(uint32_t w, uint32_t x, float acc) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), __builtin_bit_cast(bf16x2, x), acc, false);
+}
+
+// A chunk of a row with the M input rows.  Lanes past the rows' end have zero weights; ZEROS: and find zeros in place of the
+// input, else take them, for what they would read might be an infinity.
+template <int M, bool ZEROS>
 __device__ __forceinline__ void mul_chunk(float (&acc)[M], const rl_u32x4 (&v)[kDepth], const uint16_t* x, int64_t xs, int K,
                                           int kc, int lane) {
+  auto mul = [&](auto whole) __attribute__((always_inline)) {
 #pragma unroll
-  for (int u = 0; u < kDepth; ++u) {
-    const int k = kc * kChunkElems + (u * 64 + lane) * kVec;
-    if (!FULL && k >= K) continue;
+    for (int u = 0; u < kDepth; ++u) {
+      const int k = kc * kChunkElems + (u * 64 + lane) * kVec;
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-      const uint4 xv = *reinterpret_cast<const uint4*>(x + m * xs + k);
-      const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
+      for (int m = 0; m < M; ++m) {
+        constexpr bool kWhole = decltype(whole)::value;
+        const rl_u32x4 xv = *reinterpret_cast<const rl_u32x4*>(x + m * xs + (kWhole ? k : min(k, K - kVec)));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        acc[m] = fmaf(__uint_as_float(v[u][i] << 16), __uint_as_float(xw[i] << 16), acc[m]);
-        acc[m] = fmaf(__uint_as_float(v[u][i] & 0xffff0000u), __uint_as_float(xw[i] & 0xffff0000u), acc[m]);
+        for (int i = 0; i < 4; ++i) acc[m] = dot2(v[u][i], kWhole || k < K ? xv[i] : 0u, acc[m]);
       }
     }
-  }
+  };
+  if (ZEROS || (kc + 1) * kChunkElems <= K) mul(std::true_type{});
+  else mul(std::false_type{});
 }
 
+// Zeros behind a row of K elements in LDS, up to the end of its last chunk.
+__device__ __forceinline__ void zeros_behind(uint16_t* row, int K) {
+  const int at = K + (int)threadIdx.x * kVec;
+  if (at < chunks_of(K) * kChunkElems) *reinterpret_cast<rl_u32x4*>(row + at) = rl_u32x4{0, 0, 0, 0};
+}
+
+// M input rows of K elements on their way to LDS: N vectors of every lane's wait in registers (zeros past the rows' end, by
+// the same means as the weights'), what is left goes there at once.
+template <int M, int N>
+__device__ __forceinline__ void request_input(rl_u32x4 (&v)[N], uint16_t* lds, const uint16_t* x, int K) {
+  const __amdgpu_buffer_rsrc_t rows = row_buffer(x, 0, M * K, true);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if (i * kRowThreads * kVec >= M * K) break;     // (uniform)
+    v[i] = __builtin_bit_cast(rl_u32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, (i * kRowThreads + (int)threadIdx.x) * 16, 0, 0));
+  }
+#pragma unroll 1
+  for (int at = N * kRowThreads; at < M * K / kVec; at += N * kRowThreads) {
+    rl_u32x4 r[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      r[i] = __builtin_bit_cast(rl_u32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, (at + i * kRowThreads + (int)threadIdx.x) * 16, 0, 0));
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (at + i * kRowThreads + (int)threadIdx.x < M * K / kVec)
+        reinterpret_cast<rl_u32x4*>(lds)[at + i * kRowThreads + threadIdx.x] = r[i];
+  }
+}
+template <int M, int N>
+__device__ __forceinline__ void place_input(const rl_u32x4 (&v)[N], uint16_t* lds, int K) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (i * kRowThreads + (int)threadIdx.x < M * K / kVec) reinterpret_cast<rl_u32x4*>(lds)[i * kRowThreads + threadIdx.x] = v[i];
+}
+
+// residual_row for a row of at most kRowThreads * 4 * NV elements without a second pending term, in two parts: the
+// operands' requests, and the rest, which finds them on their way.  The same sums in the same order.
+template <int NV>
+struct EarlyNorm {
+  float4 x[NV], w[NV], y[NV], pw[NV];
+
+  static __host__ bool serves(const socket_residual& a) { return a.dim % 4 == 0 && a.dim <= kRowThreads * 4 * NV && !a.b; }
+
+  __device__ __forceinline__ void request(const socket_residual& a) {
+    const bool pending = a.a != nullptr, post = pending && a.post_w;
+    int64_t src = 0;
+    if (!a.x) {
+      const int64_t id = a.ids64 ? ((const int64_t*)a.ids)[0] : (int64_t)((const int32_t*)a.ids)[0];
+      src = (id < 0 ? 0 : (id >= a.vocab ? a.vocab - 1 : id)) * a.dim;
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int i = (v * kRowThreads + (int)threadIdx.x) * 4;
+      if (i >= a.dim) break;
+      if (a.x) x[v] = *reinterpret_cast<const float4*>(a.x + i);
+      else load_vec<DType_bf16, 4>(a.embed, src + i, &x[v].x);
+      if (pending) {
+        if (a.pending_f32) y[v] = *reinterpret_cast<const float4*>((const float*)a.a + i);
+        else load_vec<DType_bf16, 4>(a.a, i, &y[v].x);
+      }
+      if (post) pw[v] = *reinterpret_cast<const float4*>(a.post_w + i);
+      w[v] = *reinterpret_cast<const float4*>(a.pre_w + i);
+    }
+  }
+
+  template <class Emit>
+  __device__ __forceinline__ void finish(const socket_residual& a, float (*red)[4], bool store_x, Emit emit) {
+    float rs_y = 1.f;
+    if (a.a) {
+      float ss = 0.f;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        if ((v * kRowThreads + (int)threadIdx.x) * 4 >= a.dim) break;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float& t = (&y[v].x)[e];
+          t *= a.scale_a;
+          ss = fmaf(t, t, ss);
+        }
+      }
+      if (a.post_w) rs_y = rsqrt_f32(block_sum(ss, red[0]) / (float)a.dim + a.eps);
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int i = (v * kRowThreads + (int)threadIdx.x) * 4;
+      if (i >= a.dim) break;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float& t = (&x[v].x)[e];
+        if (!a.x) t *= a.embed_scale;
+        if (a.a) {
+          float u = (&y[v].x)[e];
+          if (a.post_w) u = u * rs_y * (&pw[v].x)[e];
+          t += u;
+        }
+        ss = fmaf(t, t, ss);
+      }
+      if (store_x && a.x_out) *reinterpret_cast<float4*>(a.x_out + i) = x[v];
+    }
+    const float rs = rsqrt_f32(block_sum(ss, red[1]) / (float)a.dim + a.eps);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int i = (v * kRowThreads + (int)threadIdx.x) * 4;
+      if (i >= a.dim) break;
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (&x[v].x)[e] * rs * (&w[v].x)[e];
+      emit(i, o);
+    }
+  }
+};
+
 // One wave per output feature; wave g of the launch takes features g, g + waves, ...
-// TWO: 0 one product, 1 the gated unit (w1 and w2 share the input row), 2 a second scaled
-// product (x2 . w2).  NORM: the input row is residual_row's, in LDS (M rows of K1), and the
-// launch is persistent so that few workgroups pay for it; the first weights are requested
-// before it starts, and a wave's weight vectors run through two register buffers, so that
-// it streams without a gap from its first row to its last.  RES: the residual sum and the
-// average over depth in the epilogue; a wave takes one feature, whose earlier results its lanes
-// gather (one each) before the weights arrive.
-template <int M, bool NORM, int TWO, bool FULL, bool RES>
+// TWO: 0 one product, 1 the gated unit (w1 and w2 share the input row), 2 a second scaled product (x2 . w2).  RES: the
+// residual sum and the average over depth in the epilogue; a wave takes one feature, whose earlier results its lanes gather
+// (one each) before the weights arrive.
+//
+// Bound by the stream of weights, and a launch is so short (5 to 20 us) that what counts is how soon all of it is asked
+// for.  The input's operands are requested first, behind them up to 16 KB of weights a wave (its next SLOTS chunks, each
+// register refilled right after its use); loads return in order, so an input requested behind the weights would arrive
+// behind them.  `row_buffer` keeps every wait a wait for one chunk.  The products are the pairwise dot instruction's: with
+// a conversion of each operand in front of a multiply-add the vector ALUs took 4 of the 14 us of the first line.
+// us a launch, weights that no cache holds, before (weights first, two chunks in flight, inputs without a norm read from
+// memory behind them) / now, beside a launch that only reads as many bytes:
+//   norm, gated 2 x 8192 x 2048       14.25 / 12.3 (10.8)     one row; 2 rows 19.9 / 16.0; 4 rows 26.4 / 20.8
+//   norm, 32000 x 2048                23.4 / 22.0 (20.2)      norm, 3392 x 2048   5.8 / 5.1
+//   sum and average, 2048 x 8192       8.45 / 7.75 (6.2)      2048 x 2048         3.46 / 3.27 (2.8)
+//   norm, gated 2 x 14336 x 4096      40.7 / 38.3             4096 x 14336       21.9 / 19.9
+template <int M, RowsInput IN, int TWO, bool RES, int SLOTS>
 __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_linear a, socket_residual nrm) {
   extern __shared__ __attribute__((aligned(16))) float rl_lds[];
   __shared__ float red[2][4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr bool EARLY = IN == kNormEarly2 || IN == kNormEarly4;
+  constexpr bool ZEROS = M == 1 && (EARLY || IN == kFromLds);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int waves = gridDim.x * (kRowThreads / 64);
   int n = blockIdx.x * (kRowThreads / 64) + wave;   // (wave-uniform)
   const uint16_t* w1 = (const uint16_t*)a.w1;
@@ -194,56 +346,113 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
   const uint16_t* x1 = (const uint16_t*)a.x1;
   const uint16_t* x2 = TWO == 2 ? (const uint16_t*)a.x2 : x1;
   const int K1 = a.K1, K2 = TWO == 2 ? a.K2 : K1;
-  const int nk1 = (K1 + kChunkElems - 1) / kChunkElems;
-  const int nk = TWO == 2 ? nk1 + (K2 + kChunkElems - 1) / kChunkElems : nk1;
-  rl_u32x4 wa[kDepth], ga[TWO == 1 ? kDepth : 1], wb[kDepth], gb[TWO == 1 ? kDepth : 1];
-  float bias1 = 0.f, bias2 = 0.f;          // of the row whose first chunk was requested last
-  auto fetch = [&](rl_u32x4 (&v)[kDepth], auto& g, int row, int kc) __attribute__((always_inline)) {
-    if (kc == 0) {
-      if (a.b1) bias1 = load_elem<DType_bf16>(a.b1, row);
-      if (TWO == 1 && a.b2) bias2 = load_elem<DType_bf16>(a.b2, row);
-    }
-    if (TWO == 2 && kc >= nk1) fetch_row<FULL>(v, w2, row, K2, kc - nk1, lane);
-    else fetch_row<FULL>(v, w1, row, K1, kc, lane);
-    if constexpr (TWO == 1) fetch_row<FULL>(g, w2, row, K1, kc, lane);
-  };
-  if (n < a.N) fetch(wa, ga, n, 0);
-  float before[M], mixed[M], own = 1.f;    // RES: the stream, this lane's share of the average
+  const int nk1 = chunks_of(K1), nk = TWO == 2 ? nk1 + chunks_of(K2) : nk1;
+  const int rows1 = ZEROS ? nk1 * kChunkElems : M * K1;     // elements of LDS in front of the second input's
+
+  // ---- the input's requests ----
+  uint16_t* xs = reinterpret_cast<uint16_t*>(rl_lds) + (IN == kNormRows ? 2 * K1 : 0);    // (behind residual_row's floats)
+  constexpr int kIn = TWO == 2 ? kInputVecs / 2 : kInputVecs;      // vectors a lane requests of either input
+  rl_u32x4 in1[IN == kFromLds ? kIn : 1], in2[IN == kFromLds && TWO == 2 ? kIn : 1];
+  EarlyNorm<IN == kNormEarly4 ? 4 : 2> early;
+  if constexpr (EARLY) early.request(nrm);
+  if constexpr (IN == kFromLds) {
+    request_input<M, kIn>(in1, xs, x1, K1);
+    if constexpr (TWO == 2) request_input<M, kIn>(in2, xs + rows1, x2, K2);
+  }
+  // RES: the stream, the share of the result in the average, and this lane's earlier result with its share
+  float before[M], past[M], own = 1.f, share = 0.f;
   if constexpr (RES) {
     const socket_depth_mix& d = a.depth;
+    const bool averaged = d.w && n < a.N && lane < d.n;
     if (d.w) own = d.w[d.n];
+    if (averaged) share = d.w[lane];
 #pragma unroll
     for (int m = 0; m < M; ++m) {
-      before[m] = mixed[m] = 0.f;
-      if (n >= a.N) continue;
-      const int64_t at = (int64_t)m * a.N + n;
+      const int64_t at = (int64_t)m * a.N + min(n, a.N - 1);
       before[m] = a.res[at];
-      if (d.w)
-        for (int j = lane; j < d.n; j += 64) mixed[m] = fmaf(d.w[j], d.past[j * d.past_stride + at], mixed[m]);
+      past[m] = averaged ? d.past[lane * d.past_stride + at] : 0.f;
     }
   }
-  if constexpr (NORM) {
-    uint16_t* xs = reinterpret_cast<uint16_t*>(rl_lds + K1);
+
+  // ---- the first weights' ----
+  rl_u32x4 wv[SLOTS][kDepth], gv[TWO == 1 ? SLOTS : 1][kDepth];
+  uint16_t bias1[SLOTS], bias2[TWO == 1 ? SLOTS : 1];
+  const __amdgpu_buffer_rsrc_t b1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.b1), 0, a.b1 ? a.N * 2 : 0, 0x00027000);
+  const __amdgpu_buffer_rsrc_t b2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.b2), 0, a.b2 ? a.N * 2 : 0, 0x00027000);
+  int fn = n, fkc = 0;                     // the next chunk to request
+  auto fetch = [&](auto slot) __attribute__((always_inline)) {
+    constexpr int i = decltype(slot)::value;
+    const bool there = fn < a.N;
+    const bool second = TWO == 2 && fkc >= nk1;
+    fetch_chunk(wv[i], row_buffer(second ? w2 : w1, fn, second ? K2 : K1, there), second ? fkc - nk1 : fkc, lane);
+    bias1[i] = __builtin_amdgcn_raw_buffer_load_b16(b1, there ? fn * 2 : 0, 0, 0);
+    if constexpr (TWO == 1) {
+      fetch_chunk(gv[i], row_buffer(w2, fn, K1, there), fkc, lane);
+      bias2[i] = __builtin_amdgcn_raw_buffer_load_b16(b2, there ? fn * 2 : 0, 0, 0);
+    }
+    const bool row_ends = ++fkc == nk;
+    fn = row_ends ? fn + waves : fn;
+    fkc = row_ends ? 0 : fkc;
+  };
+  static_for<SLOTS>(fetch);
+
+  // ---- the input ----
+  if constexpr (EARLY) {
+    early.finish(nrm, red, blockIdx.x == 0, [&](int i, const float* v) { store_vec<DType_bf16, 4>(xs, i, v); });
+    zeros_behind(xs, K1);
+    __syncthreads();
+  } else if constexpr (IN == kNormRows) {
     for (int m = 0; m < M; ++m) {
       residual_row<DType_bf16, 4, false>(nrm, m, rl_lds, red, blockIdx.x == 0,
                                   [&](int i, const float* v) { store_vec<DType_bf16, 4>(xs, (int64_t)m * K1 + i, v); });
       __syncthreads();
     }
-    x1 = x2 = xs;
+  } else if constexpr (IN == kFromLds) {
+    place_input<M, kIn>(in1, xs, K1);
+    if constexpr (TWO == 2) place_input<M, kIn>(in2, xs + rows1, K2);
+    if constexpr (ZEROS) zeros_behind(xs, K1);
+    if constexpr (ZEROS && TWO == 2) zeros_behind(xs + rows1, K2);
+    __syncthreads();
   }
+  if constexpr (IN != kFromMemory) {
+    x1 = xs;
+    x2 = IN == kFromLds ? xs + rows1 : xs;
+  }
+
+  float mixed[M];
+  if constexpr (RES) {
+    const socket_depth_mix& d = a.depth;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      mixed[m] = share * past[m];
+      if (d.w && n < a.N)
+#pragma unroll 1
+        for (int j = lane + 64; j < d.n; j += 64) mixed[m] = fmaf(d.w[j], d.past[j * d.past_stride + (int64_t)m * a.N + n], mixed[m]);
+    }
+  }
+
+  // ---- the products ----
   float acc[M], acc2[M];
 #pragma unroll
   for (int m = 0; m < M; ++m) acc[m] = acc2[m] = 0.f;
   int kc = 0;
-  auto step = [&](rl_u32x4 (&cv)[kDepth], auto& cg, rl_u32x4 (&nv)[kDepth], auto& ng) __attribute__((always_inline)) {
+  auto step = [&](auto slot, auto refill) __attribute__((always_inline)) {
+    constexpr int i = decltype(slot)::value;
     const bool row_ends = kc + 1 == nk;
-    const int n2 = row_ends ? n + waves : n, kc2 = row_ends ? 0 : kc + 1;
-    const float c1 = bias1, c2 = bias2;
-    if (n2 < a.N) fetch(nv, ng, n2, kc2);
-    if (TWO == 2 && kc >= nk1) mul_chunk<M, FULL>(acc2, cv, x2, K2, K2, kc - nk1, lane);
-    else mul_chunk<M, FULL>(acc, cv, x1, K1, K1, kc, lane);
-    if constexpr (TWO == 1) mul_chunk<M, FULL>(acc2, cg, x1, K1, K1, kc, lane);
-    if (row_ends) {
+    if (n < a.N) {
+      if (TWO == 2 && kc >= nk1) mul_chunk<M, ZEROS>(acc2, wv[i], x2, K2, K2, kc - nk1, lane);
+      else mul_chunk<M, ZEROS>(acc, wv[i], x1, K1, K1, kc, lane);
+      if constexpr (TWO == 1) mul_chunk<M, ZEROS>(acc2, gv[i], x1, K1, K1, kc, lane);
+    }
+    float c1 = bf16_bits_to_f32(bias1[i]), c2 = TWO == 1 ? bf16_bits_to_f32(bias2[TWO == 1 ? i : 0]) : 0.f;
+    if constexpr (decltype(refill)::value) {
+      // (all of the slot has been read by here, or its refill would take other registers and have to be copied, which
+      // waits for it)
+      asm volatile("" : "+v"(c1), "+v"(c2));
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(slot);
+    }
+    if (row_ends && n < a.N) {
 #pragma unroll
       for (int m = 0; m < M; ++m) {
         float o = wave_reduce_to_last<false>(acc[m]);
@@ -255,9 +464,9 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
         }
         if constexpr (RES) {
           o += before[m];
-          const float past = wave_reduce_to_last<false>(mixed[m]);
+          const float earlier = wave_reduce_to_last<false>(mixed[m]);
           if (lane == 63 && a.depth.w) a.depth.result[(int64_t)m * a.N + n] = o;
-          o = fmaf(own, o, past);
+          o = fmaf(own, o, earlier);
         }
         if (lane == 63) {
           if (a.y_f32) ((float*)a.y)[(int64_t)m * a.N + n] = o;
@@ -266,49 +475,74 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
         acc[m] = acc2[m] = 0.f;
       }
     }
-    n = n2;
-    kc = kc2;
+    n = row_ends ? n + waves : n;
+    kc = row_ends ? 0 : kc + 1;
   };
-  while (n < a.N) {
-    step(wa, ga, wb, gb);
-    if (n >= a.N) break;
-    step(wb, gb, wa, ga);
-  }
+  // (all slots in every turn: to leave in the middle of one would make the waits of the next for everything, too)
+  if constexpr (SLOTS == most_slots(TWO))
+    while (fn < a.N) static_for<SLOTS>([&](auto slot) __attribute__((always_inline)) { step(slot, std::true_type{}); });
+  static_for<SLOTS>([&](auto slot) __attribute__((always_inline)) { step(slot, std::false_type{}); });
 }
 
-template <int M, bool NORM, int TWO, bool FULL, bool RES = false>
-int launch_rows_linear(const socket_rows_linear& a, hipStream_t s) {
-  const SocketDeviceLimits& lim = socket_device_limits();
-  size_t lds = 0;
-  int n_wg = (a.N + kRowThreads / 64 - 1) / (kRowThreads / 64);
-  auto kern = rows_linear_kernel<M, NORM, TWO, FULL, RES>;
-  socket_residual nrm{};
-  if (NORM) {
-    nrm = *a.norm;
-    lds = (size_t)a.K1 * 4 + (size_t)M * a.K1 * 2;
-    if (lds + 256 > (size_t)lim.max_lds_per_block) return SOCKET_ERR_UNSUPPORTED;
-    if (lds > 48 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-      return SOCKET_ERR_LAUNCH;
-    n_wg = n_wg < lim.cu_count * kWgPerCu ? n_wg : lim.cu_count * kWgPerCu;
-  }
-  hipLaunchKernelGGL(kern, dim3((unsigned)n_wg), dim3(kRowThreads), lds, s, a, nrm);
+template <int M, RowsInput IN, int TWO, bool RES, int SLOTS>
+int launch_rows_linear(const socket_rows_linear& a, int n_wg, size_t lds, hipStream_t s) {
+  auto kern = rows_linear_kernel<M, IN, TWO, RES, SLOTS>;
+  if (lds > 48 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)lds) != hipSuccess)
+    return SOCKET_ERR_LAUNCH;
+  hipLaunchKernelGGL(kern, dim3((unsigned)n_wg), dim3(kRowThreads), lds, s, a, a.norm ? *a.norm : socket_residual{});
   return SOCKET_OK;
 }
 
-template <int M, bool FULL>
-int dispatch_form(const socket_rows_linear& a, hipStream_t s) {
-  const int two = a.kind != 0 ? 1 : (a.x2 ? 2 : 0);
-  if (a.res) return launch_rows_linear<M, false, 0, FULL, true>(a, s);
-  if (a.norm) return two == 1 ? launch_rows_linear<M, true, 1, FULL>(a, s) : launch_rows_linear<M, true, 0, FULL>(a, s);
-  if (two == 1) return launch_rows_linear<M, false, 1, FULL>(a, s);
-  return two == 2 ? launch_rows_linear<M, false, 2, FULL>(a, s) : launch_rows_linear<M, false, 0, FULL>(a, s);
+// A wave's slots: as many as it has chunks, up to 16 KB of weights (a load that finds no row left brings nothing, but takes
+// its turn).
+template <int M, RowsInput IN, int TWO, bool RES>
+int dispatch_slots(const socket_rows_linear& a, size_t lds, hipStream_t s) {
+  constexpr int kWaves = kRowThreads / 64;
+  int n_wg = (a.N + kWaves - 1) / kWaves;
+  // (few workgroups pay for the input's passage: each keeps its waves streaming from row to row)
+  if (!RES && IN != kFromMemory) n_wg = std::min(n_wg, socket_device_limits().cu_count * kWgPerCu);
+  const int nk = chunks_of(a.K1) + (TWO == 2 ? chunks_of(a.K2) : 0);
+  const int64_t chunks = (int64_t)((a.N + n_wg * kWaves - 1) / (n_wg * kWaves)) * nk;
+  if constexpr (TWO != 2 && IN != kFromMemory) {
+    if (chunks == 1) return launch_rows_linear<M, IN, TWO, RES, 1>(a, n_wg, lds, s);
+    if (chunks == 2) return launch_rows_linear<M, IN, TWO, RES, 2>(a, n_wg, lds, s);
+  }
+  return launch_rows_linear<M, IN, TWO, RES, most_slots(TWO)>(a, n_wg, lds, s);
+}
+
+template <int M, RowsInput IN, int TWO>
+int dispatch_res(const socket_rows_linear& a, size_t lds, hipStream_t s) {
+  if constexpr (TWO == 0 && (IN == kFromMemory || IN == kFromLds))
+    if (a.res) return dispatch_slots<M, IN, TWO, true>(a, lds, s);
+  return dispatch_slots<M, IN, TWO, false>(a, lds, s);
+}
+
+template <int M, int TWO>
+int dispatch_input(const socket_rows_linear& a, hipStream_t s) {
+  const size_t room = (size_t)socket_device_limits().max_lds_per_block - 256;
+  auto in_lds = [](int K) { return M == 1 ? ((size_t)K + kChunkElems - 1) / kChunkElems * kChunkElems * 2 : (size_t)M * K * 2; };
+  if (!a.norm) {
+    const size_t lds = in_lds(a.K1) + (TWO == 2 ? in_lds(a.K2) : 0);
+    return lds <= room ? dispatch_res<M, kFromLds, TWO>(a, lds, s) : dispatch_res<M, kFromMemory, TWO>(a, 0, s);
+  }
+  if constexpr (TWO == 2) {
+    return SOCKET_ERR_UNSUPPORTED;
+  } else {
+    const size_t rows = (size_t)a.K1 * (4 + 2 * M);
+    if (rows > room) return SOCKET_ERR_UNSUPPORTED;
+    if constexpr (M == 1) {
+      if (EarlyNorm<2>::serves(*a.norm)) return dispatch_res<M, kNormEarly2, TWO>(a, in_lds(a.K1), s);
+      if (EarlyNorm<4>::serves(*a.norm)) return dispatch_res<M, kNormEarly4, TWO>(a, in_lds(a.K1), s);
+    }
+    return dispatch_res<M, kNormRows, TWO>(a, rows, s);
+  }
 }
 
 template <int M>
 int dispatch_rows_linear(const socket_rows_linear& a, hipStream_t s) {
-  const bool full = a.K1 % kChunkElems == 0 && (!a.x2 || a.K2 % kChunkElems == 0);
-  return full ? dispatch_form<M, true>(a, s) : dispatch_form<M, false>(a, s);
+  if (a.kind != 0) return dispatch_input<M, 1>(a, s);
+  return a.x2 ? dispatch_input<M, 2>(a, s) : dispatch_input<M, 0>(a, s);
 }
 
 int check_residual(const socket_residual* a) {

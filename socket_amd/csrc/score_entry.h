@@ -136,15 +136,6 @@ __device__ __forceinline__ void accumulate(float* acc, const RawEntry<GP * 2>& e
   }
 }
 
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>), in order
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, I + 1>(f);
-  }
-}
-
 // LDS past the table buffers in every launch: scratch of the key-range reduction
 constexpr size_t kScoreScratchBytes = 1024;
 

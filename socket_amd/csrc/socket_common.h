@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 #include "../../include/socket_hip.h"
 
 #define SOCKET_WAVE 64
@@ -24,6 +25,15 @@ static inline int socket_dtype_bytes(int dt) {
 }
 
 static inline bool socket_aligned16(const void* p) { return (((uintptr_t)p) & 15u) == 0; }
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>), in order
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(f);
+  }
+}
 
 // ---- element conversions -------------------------------------------------
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
