@@ -77,6 +77,19 @@ struct Vectors<2> {
   static __device__ __forceinline__ uint32_t mask(bytes b, int i) { return (uint32_t)b >> (8 * i); }
 };
 
+// an entry as it is read from LDS
+template <class QT>
+using entry_bits_t = std::conditional_t<sizeof(QT) == 4, uint32_t, uint16_t>;
+
+// Byte address of entry `code` of the table at `base` in LDS: the low or high code of a word, one instruction.
+template <int EB>
+__device__ __forceinline__ uint32_t entry_address(uint32_t codes, bool high, uint32_t base) {
+  uint32_t a;
+  if (high) asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(a) : "v"(codes), "n"(EB), "s"(base));
+  else asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(a) : "v"(codes), "n"(EB), "s"(base));
+  return a;
+}
+
 // ct: tables per LDS slice.  INLDS false: a single table exceeds LDS, gather from global memory.
 // A workgroup serves `chunks` consecutive tiles of `tile` <= THREADS x TPT tokens under every
 // slice it brings into LDS; with more than one slice the running sums of a tile
@@ -197,6 +210,9 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
     return Where{own, WIDE ? min(own, T - TPT) : own};
   };
   const int step = INLDS ? ct : L;   // (without LDS: one pass over all tables)
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  const uint16_t last_code = (uint16_t)(min(R, 32768) - 1);      // (as 16 bits without a sign, anything above is no code)
+  const uint32_t table_at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) QT*)table;
   for (int l0 = 0; l0 < L; l0 += step) {
     const int nt = min(step, L - l0);
     const Where w0 = where(0);
@@ -227,6 +243,9 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
         for (int i = 0; i < TPT; ++i) sum[i] = 0.f;
       } else {
         load_partial(o, t0, skip, sum);
+        // (waited for here: left to the first use in the loop, the wait is there in every turn, for nearly all codes in flight)
+#pragma unroll
+        for (int i = 0; i < TPT; ++i) asm volatile("" : "+v"(sum[i]));
       }
       // A ring of kAhead code words per lane stays in flight (one 16-byte load per lane
       // would leave the stream waiting on latency): slot a always holds table lb + a;
@@ -239,17 +258,51 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
           const int l = lb + a;
           if (l >= nt) break;
           const codes_t cur = ring[a];
-          ring[a] = codes_of(l0 + min(l + kAhead, nt - 1), t0);   // (past the slice: its last table again, unused)
-          // branch-free: a stray code reads entry 0 and adds +0.0 instead (x + 0.0 == x;
-          // the sums start at +0.0, so no -0.0 can be lost), and the LDS variant has no
-          // global load in here for the compiler to wait on with the ring in flight
+          // (past the slice: its last table again, unused)
+          auto refill = [&]() __attribute__((always_inline)) { ring[a] = codes_of(l0 + min(l + kAhead, nt - 1), t0); };
+          // Without a branch: a stray code reads entry 0 and adds +0.0 instead (x + 0.0 == x; the sums start at +0.0, so no
+          // -0.0 can be lost).
+          auto add_any = [&]() __attribute__((always_inline)) {
 #pragma unroll
-          for (int i = 0; i < TPT; ++i) {
-            const int r = (int)(int16_t)((i & 1) ? (V::word(cur, i >> 1) >> 16) : (V::word(cur, i >> 1) & 0xffffu));
-            const bool hit = r >= 0 && r < R;
-            const int rr = hit ? r : 0;
-            const float e = entry_to_f32(INLDS ? table[l * R + rr] : qp[(int64_t)(l0 + l) * R + rr]);
-            sum[i] += hit ? e : 0.f;
+            for (int i = 0; i < TPT; ++i) {
+              const int r = (int)(int16_t)((i & 1) ? (V::word(cur, i >> 1) >> 16) : (V::word(cur, i >> 1) & 0xffffu));
+              const bool hit = r >= 0 && r < R;
+              const int rr = hit ? r : 0;
+              const float e = entry_to_f32(INLDS ? table[l * R + rr] : qp[(int64_t)(l0 + l) * R + rr]);
+              sum[i] += hit ? e : 0.f;
+            }
+          };
+          if constexpr (INLDS && WIDE) {
+            // One test for all codes of the wave: the sums of codes that are all inside take less than five vector
+            // instructions a code, where a test of each took nine and 1.8 times the code.  The vector ALUs were what the
+            // launch waited for, two waves to each of them at 512 lanes (us before / now, with the wait below: 32 rows of
+            // 32768 tokens, L60 x R1024, bf16 35.6 / 30.5, fp32 43.0 / 33.7; 9001 tokens, bf16 17.1 / 15.1).
+            const uint32_t base = table_at + (uint32_t)(l * R) * (uint32_t)sizeof(QT);
+            u16x2 most = {0, 0};
+            uint32_t at[TPT];
+#pragma unroll
+            for (int i = 0; i < TPT; i += 2) {
+              const uint32_t w = V::word(cur, i >> 1);
+              most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, w));
+              at[i] = entry_address<sizeof(QT)>(w, false, base);
+              at[i + 1] = entry_address<sizeof(QT)>(w, true, base);
+            }
+            const u16x2 outside = __builtin_elementwise_sub_sat(most, u16x2{last_code, last_code});
+            if (__builtin_expect(__ballot(__builtin_bit_cast(uint32_t, outside) != 0) != 0, 0)) {
+              add_any();
+              refill();
+            } else {
+              __builtin_amdgcn_sched_barrier(0);     // (the codes have been used: their registers take the next)
+              refill();
+              entry_bits_t<QT> e[TPT];
+#pragma unroll
+              for (int i = 0; i < TPT; ++i) e[i] = *(const __attribute__((address_space(3))) entry_bits_t<QT>*)(uintptr_t)at[i];
+#pragma unroll
+              for (int i = 0; i < TPT; ++i) sum[i] += entry_to_f32(__builtin_bit_cast(QT, e[i]));
+            }
+          } else {
+            refill();
+            add_any();
           }
         }
       }
@@ -277,24 +330,33 @@ int launch_collision_i16(const QT* q_probs, const int16_t* key_buckets, const ui
   const bool wide = T >= kTokensPerThread;
   // Rows short enough that two (or four) tokens to a lane hold them in one round of workgroups, each row in as many equal
   // tiles as there are CUs for it: with eight to a lane most waves would have no token and the rest a long chain of lookups.
-  // 32 rows, L60 x R1024, us at two to a lane / at eight: fp32 1000 tokens 13.8 / 25, 4135 16.5 / 30, 16384 23.2 / 33.6; bf16
-  // 12.0 / 22, 13.4 / 27, 19.4 / 29; 56 rows, L48, fp32 6001 18.3 / 26; 28 rows, L32 x R256, fp32 4135 8.6 / 13.2, 16384 12.9 /
-  // 15.  Four to a lane pay while a quarter of the lanes is spare (32 rows, 20000 tokens: fp32 32.0 / 35.7, bf16 27.6 / 30.8)
-  // and not with every lane in use (32768 bf16 33.8 / 32.8; 64 rows, L32 x R256, 16384: 20.6 / 19.1).
+  // us at two / four / eight tokens to a lane, L60 x R1024:
+  //   32 rows   fp32  1000 tokens 14.9 / 15.3 / 20.2   4135 16.7 / 16.7 / 20.9   9001 20.0 / 18.3 / 22.0   16384 24.6 / 22.3 / 23.8
+  //             bf16              10.4 / 11.5 / 16.9        12.7 / 13.8 / 20.2        15.5 / 15.1 / 20.7         19.6 / 18.5 / 23.1
+  //   28 rows, L32 x R256, fp32: 4135 tokens 7.5 / 7.6 / 9.2, 16384 13.0 / 11.6 / 12.5
+  // Two pay while half of the lanes at most have a token, four while a quarter of the lanes is spare (32 rows, 24576 tokens:
+  // 24.8 / 26.4 at four / eight, bf16; 32768: 30.9 / 30.5, fp32 35.2 / 33.6).
   const int64_t per_row = cus / ((int64_t)B * H);
-  const int few = !wide || ct == 0 ? 0 : per_row * 1024 * 2 >= T ? 2 : per_row * 1024 * 3 >= T ? 4 : 0;
+  const int few = !wide || ct == 0 ? 0 : per_row * 1024 >= T ? 2 : per_row * 1024 * 3 >= T ? 4 : 0;
   // Lanes of a workgroup of eight tokens each.  It pulls its row's whole table through LDS with them, which is quicker the
-  // more there are, but while all workgroups are at work at once narrower ones leave fewer CUs idle (us at 512 / 1024 lanes,
-  // 32 rows, L60 x R1024: fp32 32768 tokens 35 / 40, 48000 61 / 44; bf16 32768 28 / 36, 65536 58 / 50).  A row of at most 4608
-  // tokens has no use for 512: one workgroup of 1024 holds it, or all but nothing (200 rows of 4096, L60 x R1024, fp32 30.6 /
-  // 29.3).  Rows of at most 2048 tokens come here where they outnumber the CUs; 256 lanes hold each of them, which pays where
+  // more there are; 512 of them hold a tile of 4096 tokens and run its lookups as fast (32 rows of 32768, L60 x R1024, at 512 /
+  // 1024 lanes of eight / four tokens: bf16 30.5 / 30.9, fp32 33.6 / 35.2).  A row of at most 4608
+  // tokens has no use for 512: one workgroup of 1024 holds it, or all but nothing.  Rows of at most 2048 tokens come here where
+  // they outnumber the CUs; 256 lanes hold each of them, which pays where
   // tables share a CU's LDS (us at 256 / 1024 lanes, L32 x R256, fp32: 448 rows x 1000 14.8 / 15.4, 1024 rows x 1000 18.8 / 23.4)
   // and does not where one fills it (L60 x R1024, fp32: 257 rows x 1000 62 / 47, 1024 x 1000 183 / 121).
+  // Rows that a workgroup of 1024 lanes to each of their CUs holds are cut into that many equal tiles, whole waves of them, or
+  // CUs go without (56 rows of 20001, L48 x R1024, bf16: 28.8 us against 39.3 with tiles of as many tokens as the lanes hold).
+  const bool even = wide && ct > 0 && !few && per_row > 0 && T > 256 * kTokensPerThread && T <= per_row * 1024 * kTokensPerThread;
+  const int wave_tokens = SOCKET_WAVE * kTokensPerThread;
   auto tiles_of = [&](int th) { return (T + th * kTokensPerThread - 1) / (th * kTokensPerThread); };
   int threads = 1024;
+  int tile = threads * kTokensPerThread;
+  if (few) tile = (int)((T + per_row - 1) / per_row + 127) / 128 * 128;
+  else if (even) tile = (int)((T + per_row - 1) / per_row + wave_tokens - 1) / wave_tokens * wave_tokens;
   if (T <= 256 * kTokensPerThread) threads = 256;
-  else if (T > 4608 && (int64_t)tiles_of(512) * B * H <= cus) threads = 512;
-  const int tile = few ? (int)((T + per_row - 1) / per_row + 127) / 128 * 128 : threads * kTokensPerThread;
+  else if (T > 4608 && (even ? tile <= 512 * kTokensPerThread : (int64_t)tiles_of(512) * B * H <= cus)) threads = 512;
+  if (!few && !even) tile = threads * kTokensPerThread;
   const int tiles = (T + tile - 1) / tile;
   // tiles per workgroup: as many as leave two workgroups per CU (they amortise the
   // slices a workgroup pulls through LDS), at most 8
