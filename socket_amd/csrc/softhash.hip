@@ -102,21 +102,24 @@ __device__ __forceinline__ void sh_store4<DType_f16>(void* p, int64_t i, const f
 // matrix cores, sixteen heads of one table to a workgroup.
 //
 //   proj^T[plane, head] = planes . q^T          v_mfma_f32_16x16x32_bf16, exact products, fp32 sums
-//   logit^T[bucket, head] = protos . t          t in three bf16 terms (hi, mid, lo: all 24 bits), so that
+//   logit[head, bucket] = t . protos            t in three bf16 terms (hi, mid, lo: all 24 bits), so that
 //                                               two products of 16 x 16 x 32 keep what fp32 keeps
-// In both the head is the N index: lane x holds head x % 16 in all its registers, the planes of lane
-// quarter q are 4 q .. + 3, and the terms a lane splits off its own projections are the operand it
-// has to supply.  Bucket order inside a product is free: block ii of a 64-bucket chunk takes buckets
-// 4 m + ii for row m, so that a lane's prototypes are runs of four (8-byte loads) and its results runs of
-// sixteen.  A wave has 256 buckets; maxima and sums meet in 512 bytes of LDS.  Logits are made in
-// base-2 units (log2 e goes into t) for the hardware's exponential.
-// The scalar form below spends ten multiply-adds and a library exponential per (head, bucket) and is bound by
-// the vector ALU: with it the decode prologue takes 23 us for 4 x 32 heads x 60 tables and 56 us for
-// 16 x 28 x 48; with this one 13 us and 25 us, and 7.7 us instead of 10.4 us for one sequence of 32 x 60
-// (dependent trips to memory and a launch).
+// The head is the N index of the first: lane x holds head x % 16, and the planes of lane quarter q are 4 q .. + 3; the terms a
+// lane splits off are the operand it has to supply to the second, where the head is the M index: register r of quarter q is head 4 q + r,
+// so that the heads of a unit lie in one lane and an entry of the table is stored as it is.  Bucket order inside a product is free:
+// block ii of a 64-bucket chunk takes buckets 4 n + ii for column n, so that a lane's prototypes are runs of four (8-byte
+// loads) and its results runs of four entries.  A wave has 256 buckets.  Of what all four waves need, each works out a share: a
+// quarter of the dims of the rotation and the projections, one plane of four of the tanh.  Logits are made in base-2 units
+// (log2 e goes into t) for the hardware's exponential, and nothing is taken off them first where all of a head's are small,
+// which they are with +-1 prototypes (tanh / sqrt(D) / temperature: at most 4.3); it is seen from the logits themselves.
+// What bounds it are vector instructions, about 600 a wave at 64 logits a lane, and at few heads dependent trips to memory.
+// Before (head as the N index of both products: entries put together by lane exchanges; every wave rotated and projected
+// everything; maxima exchanged and taken off) and now, the decode prologue with the rest of its roles: one sequence of 32 heads x
+// 60 tables 7.7 / 6.3 us, four 13.4 / 10.9, sixteen of 28 x 48 27.2 / 23.4.  (The scalar form below spends ten multiply-adds
+// and a library exponential per head and bucket: 10.4, 23 and 56 us.)
 //
 // W: heads of a unit (the scorer's grouped layout [unit, L, R, W]; 1 for the reference's [B,Hq,L,R], whose
-// units are heads).  OT: float or uint16_t (bf16).  FT: void, or the element type of a rotary table, as above.
+// units are heads).  OutDT: the table's type.  FT: void, or the element type of a rotary table, as above.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 sh_bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float sh_f32x4;
 union ShFrag {
@@ -129,8 +132,6 @@ __device__ __forceinline__ sh_f32x4 sh_mfma(const uint4& a, const uint4& b, sh_f
   y.u = b;
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x.v, y.v, c, 0, 0, 0);
 }
-__device__ __forceinline__ uint32_t sh_dpp_xor1(uint32_t x) { return __builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, false); }
-__device__ __forceinline__ uint32_t sh_dpp_xor2(uint32_t x) { return __builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, false); }
 
 // eight consecutive table entries (cos, sin of four pairs) as floats
 template <class FT>
@@ -147,201 +148,269 @@ __device__ __forceinline__ void sh_load8<DType_f32>(const void* p, int64_t i, fl
 }
 
 constexpr int kMxHeads = 16, kMxD = 128, kMxK = 10, kMxR = 1024;
+constexpr float kMxPlain = 32.f;      // base-2 logits up to which nothing is taken off before the exponential
 
 // Which heads the units are: `parts` units of W heads to a kv head's G (0: a unit is a head of Hq).
+// per_seq: units of a sequence; the reciprocals are for mx_div.
 struct MxUnits {
-  int count, parts, Hq, Hkv, G;
+  int count, parts, Hq, Hkv, G, per_seq;
+  float inv_per_seq, inv_parts;
 };
 
-template <class FT, int W, class OT>
+// x / d of x >= 0 and 0 < d with inv = 1 / d in fp32: the rounded quotient is off by at most one while it is below 2^22.
+__device__ __forceinline__ int mx_div(int x, int d, float inv) {
+  int k = (int)((float)x * inv);
+  k -= k * d > x ? 1 : 0;
+  return k + ((k + 1) * d <= x ? 1 : 0);
+}
+
+// Sum or maximum over the sixteen lanes of a row, in every lane of it.
+template <bool MAX>
+__device__ __forceinline__ float mx_row(float x) {
+#define SOCKET_STEP(ctrl)                                                                                               \
+  {                                                                                                                     \
+    const float o = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xf, 0xf, false));           \
+    x = MAX ? fmaxf(x, o) : x + o;                                                                                      \
+  }
+  SOCKET_STEP(0x128)      // row_ror: 8, 4, 2, 1
+  SOCKET_STEP(0x124)
+  SOCKET_STEP(0x122)
+  SOCKET_STEP(0x121)
+#undef SOCKET_STEP
+  return x;
+}
+
+// What the matrix-core forms share: where a lane's head is, the waves' shares of the projections put together, and the
+// softmax and the write of one table.
+struct MxHead {
+  int b, head;
+  bool live;
+};
+template <int W>
+__device__ __forceinline__ MxHead mx_head(const int group, const MxUnits& units, int n) {
+  const int first = group * (kMxHeads / W), b0 = first / units.per_seq;         // (uniform)
+  const bool in_units = first + n / W < units.count;
+  const int at0 = first - b0 * units.per_seq + (in_units ? n / W : 0), over = mx_div(at0, units.per_seq, units.inv_per_seq);
+  const int at = at0 - over * units.per_seq;
+  MxHead h{b0 + over, at, in_units};
+  if (units.parts > 0) {
+    const int kvh = mx_div(at, units.parts, units.inv_parts), member = (at - kvh * units.parts) * W + n % W;     // (of the kv head's group)
+    h.live = in_units && member < units.G;
+    h.head = kvh * units.G + (h.live ? member : 0);
+  }
+  return h;
+}
+
+// part: register r is this wave's share of plane 4 quarter + r of head n.  Returns t of those planes, each wave having worked out
+// one register's (planes past the tenth: zero).
+__device__ __forceinline__ sh_f32x4 mx_angles(const sh_f32x4& part, float scale, int wave, int lane) {
+  __shared__ __attribute__((aligned(16))) sh_f32x4 shares[kSHWaves][SOCKET_WAVE];
+  __shared__ __attribute__((aligned(16))) float angles[SOCKET_WAVE][4];
+  shares[wave][lane] = part;
+  __syncthreads();
+  const float* at = (const float*)shares + 4 * lane + wave;
+  constexpr int kStep = 4 * SOCKET_WAVE;
+  const float proj = (at[0] + at[2 * kStep]) + (at[kStep] + at[3 * kStep]);
+  angles[lane][wave] = 4 * (lane >> 4) + wave < kMxK ? tanhf(proj) * scale : 0.f;
+  __syncthreads();
+  return *reinterpret_cast<const sh_f32x4*>(angles[lane]);
+}
+
+// logits(c, lg): lg[ii][r] is bucket 256 wave + 64 c + 4 n + ii of head 4 quarter + r, in base-2 units, from prototypes that
+// reload() fetches again.
+template <int W, class OutDT, class LOGITS, class RELOAD>
+__device__ __forceinline__ void mx_table(const LOGITS& logits, const RELOAD& reload, bool live, void* __restrict__ out, int l, int group, int n_units, int L,
+                                         int wave, int lane) {
+  __shared__ __attribute__((aligned(16))) float red[4][kSHWaves][kMxHeads];
+  __shared__ __attribute__((aligned(16))) float alive[kMxHeads];
+  __shared__ int wide[kSHWaves];
+  const int n = lane & 15, quarter = lane >> 4;
+  sh_f32x4 lg[4][4];
+  auto total = [&](int k) {      // of a head, over the table: the sums (or the maxima) of the four waves
+    sh_f32x4 w[kSHWaves];
+#pragma unroll
+    for (int i = 0; i < kSHWaves; ++i) w[i] = *reinterpret_cast<const sh_f32x4*>(&red[k][i][4 * quarter]);
+    if (k % 2 == 0) return (w[0] + w[1]) + (w[2] + w[3]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w[0][r] = fmaxf(fmaxf(w[0][r], w[1][r]), fmaxf(w[2][r], w[3][r]));
+    return w[0];
+  };
+  float top = 0.f;
+  sh_f32x4 sum = sh_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) logits(c, lg[c]);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) top = fmaxf(top, fabsf(lg[c][i][r]));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) lg[c][i][r] = __builtin_amdgcn_exp2f(lg[c][i][r]);
+      sum += lg[c][i];
+    }
+  }
+  const bool far = __builtin_amdgcn_ballot_w64(top > kMxPlain) != 0;
+  auto sum_up = [&](int k) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sum[r] = mx_row<false>(sum[r]);
+    if (n == 0) *reinterpret_cast<sh_f32x4*>(&red[k][wave][4 * quarter]) = sum;
+  };
+  sum_up(0);
+  if (quarter == 0) alive[n] = live ? 1.f : 0.f;
+  if (lane == 0) wide[wave] = far ? 1 : 0;
+  __syncthreads();
+  auto write = [&](const sh_f32x4& sum) __attribute__((always_inline)) {
+    const sh_f32x4 real = *reinterpret_cast<const sh_f32x4*>(&alive[4 * quarter]);
+    sh_f32x4 inv;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) inv[r] = real[r] != 0.f ? 1.f / sum[r] : 0.f;      // (heads that only fill a unit up are zero)
+    typedef typename OutDT::storage OT;
+#pragma unroll
+    for (int g = 0; g < 4; g += W) {      // the lane's units: heads 4 quarter + g .. + W - 1
+      const int unit = group * (kMxHeads / W) + (4 * quarter + g) / W;
+      if (unit >= n_units) break;
+      OT* base = (OT*)out + (((int64_t)unit * L + l) * kMxR + wave * 256 + 4 * n) * W;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        float v[4 * W];                   // four buckets of W heads: a run
+#pragma unroll
+        for (int i = 0; i < 4 * W; ++i) v[i] = lg[c][i / W][g + i % W] * inv[g + i % W];
+#pragma unroll
+        for (int i = 0; i < 4 * W; i += 16 / (int)sizeof(OT)) {
+          OT* to = base + 64 * c * W + i;
+          if constexpr (sizeof(OT) == 4) *reinterpret_cast<float4*>(to) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
+          else if constexpr (W == 1) *reinterpret_cast<uint2*>(to) = make_uint2(f32x2_to_bf16_bits(v[0], v[1]), f32x2_to_bf16_bits(v[2], v[3]));
+          else
+            *reinterpret_cast<uint4*>(to) = make_uint4(f32x2_to_bf16_bits(v[i], v[i + 1]), f32x2_to_bf16_bits(v[i + 2], v[i + 3]),
+                                                       f32x2_to_bf16_bits(v[i + 4], v[i + 5]), f32x2_to_bf16_bits(v[i + 6], v[i + 7]));
+        }
+      }
+    }
+  };
+  if (__builtin_amdgcn_readfirstlane(wide[0] | wide[1] | wide[2] | wide[3]) == 0) {
+    write(total(0));
+    return;
+  }
+  // a large logit somewhere (the same answer in all waves): from the start, with the largest taken off in the heads that have one
+  reload();
+#pragma unroll
+  for (int c = 0; c < 4; ++c) logits(c, lg[c]);
+  sh_f32x4 mx = lg[0][0], size = sh_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      mx[r] = fmaxf(mx[r], lg[i >> 2][i & 3][r]);
+      size[r] = fmaxf(size[r], fabsf(lg[i >> 2][i & 3][r]));
+    }
+    mx[r] = mx_row<true>(mx[r]);
+    size[r] = mx_row<true>(size[r]);
+  }
+  if (n == 0) {
+    *reinterpret_cast<sh_f32x4*>(&red[1][wave][4 * quarter]) = mx;
+    *reinterpret_cast<sh_f32x4*>(&red[3][wave][4 * quarter]) = size;
+  }
+  __syncthreads();
+  mx = total(1);
+  size = total(3);
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (!(size[r] > kMxPlain)) mx[r] = 0.f;       // (what the head has when it is with others)
+  sum = sh_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) lg[i >> 2][i & 3][r] = __builtin_amdgcn_exp2f(lg[i >> 2][i & 3][r] - mx[r]);
+    sum += lg[i >> 2][i & 3];
+  }
+  sum_up(2);
+  __syncthreads();
+  write(total(2));
+}
+
+template <class FT, int W, class OutDT>
 __device__ __forceinline__ void soft_hash_mx_block(const int l, const int group, const MxUnits& units, const uint16_t* __restrict__ q,
                                                    int64_t q_sb, int64_t q_sh, const uint16_t* __restrict__ planes,
-                                                   const uint16_t* __restrict__ protos_T, OT* __restrict__ out, int L, float scale,
+                                                   const uint16_t* __restrict__ protos_T, void* __restrict__ out, int L, float scale,
                                                    const void* __restrict__ freqs, const int64_t* __restrict__ pos, int pos_stride,
                                                    int64_t n_pos, uint16_t* __restrict__ q_out) {
   constexpr bool kRope = !std::is_void<FT>::value;
-  __shared__ float red[2][kSHWaves][kMxHeads];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, quarter = lane >> 4;
-  const int unit = group * (kMxHeads / W) + n / W;
-  const bool in_units = unit < units.count;
-  const int u = in_units ? unit : 0;
-  const int per_seq = units.parts > 0 ? units.Hkv * units.parts : units.Hq;
-  const int b = u / per_seq, at = u % per_seq;
-  const int member = units.parts > 0 ? at % units.parts * W + n % W : 0;       // of the kv head's group
-  const bool live = in_units && (units.parts == 0 || member < units.G);
-  const int head = units.parts > 0 ? at / units.parts * units.G + (live ? member : 0) : at;
+  const MxHead at = mx_head<W>(group, units, n);
 
-  // everything is asked for first: queries, angles, planes, prototypes
-  const uint16_t* qrow = q + b * q_sb + head * q_sh;
+  // everything is asked for first: the wave's quarter of the queries, angles and planes, prototypes
+  const int d0 = 32 * wave + 8 * quarter;
   int64_t p = 0;
-  bool turn = false;
-  if constexpr (kRope) {
-    p = pos[(int64_t)b * pos_stride];
-    turn = p >= 0 && p < n_pos;
-  }
-  uint4 qf[4], pl[4];
+  if constexpr (kRope) p = pos[(int64_t)at.b * pos_stride];
+  uint4 qf = *reinterpret_cast<const uint4*>(q + at.b * q_sb + at.head * q_sh + d0);
+  const uint4 pl = *reinterpret_cast<const uint4*>(planes + ((int64_t)l * kMxK + min(n, kMxK - 1)) * kMxD + d0);
   uint2 pr[4][4];
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    qf[ks] = *reinterpret_cast<const uint4*>(qrow + 32 * ks + 8 * quarter);
-    pl[ks] = *reinterpret_cast<const uint4*>(planes + ((int64_t)l * kMxK + min(n, kMxK - 1)) * kMxD + 32 * ks + 8 * quarter);
-  }
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      pr[c][r] = *reinterpret_cast<const uint2*>(protos_T + min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c + 4 * n);
-  if (quarter >= 2) {         // (no prototype past the tenth: zeros, whatever the tenth is)
+  uint32_t protos_at = 0;
+  auto load_protos = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (4 * quarter + r >= kMxK) pr[c][r] = make_uint2(0, 0);
-  }
-  if constexpr (kRope) {
-    // (angles of row 0 for a position outside the table: a load under a condition is waited for at once)
-    float f[4][8];
+        pr[c][r] = *reinterpret_cast<const uint2*>(protos_T + (protos_at + min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c + 4 * n));
+    if (quarter >= 2) {         // (no prototype past the tenth: zeros, whatever the tenth is)
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) sh_load8<FT>(freqs, (turn ? p : 0) * kMxD + 32 * ks + 8 * quarter, f[ks]);
+      for (int c = 0; c < 4; ++c)
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (turn) {
-        float x[8];
-        unpack16<DType_bf16>(qf[ks], x);
-        uint32_t w[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float re, im;
-          rotate_pair(x[2 * j], x[2 * j + 1], f[ks][2 * j], f[ks][2 * j + 1], re, im);
-          w[j] = f32x2_to_bf16_bits(re, im);
-        }
-        qf[ks] = make_uint4(w[0], w[1], w[2], w[3]);
-      }
-      if (l == 0 && wave == 0 && live)
-        *reinterpret_cast<uint4*>(q_out + ((int64_t)b * units.Hq + head) * kMxD + 32 * ks + 8 * quarter) = qf[ks];
+        for (int r = 0; r < 4; ++r)
+          if (4 * quarter + r >= kMxK) pr[c][r] = make_uint2(0, 0);
     }
+  };
+  load_protos();
+  if constexpr (kRope) {
+    const bool turn = p >= 0 && p < n_pos;
+    // (angles of row 0 for a position outside the table: a load under a condition is waited for at once)
+    float f[8];
+    sh_load8<FT>(freqs, (turn ? p : 0) * kMxD + d0, f);
+    if (turn) {
+      float x[8];
+      unpack16<DType_bf16>(qf, x);
+      uint32_t w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float re, im;
+        rotate_pair(x[2 * j], x[2 * j + 1], f[2 * j], f[2 * j + 1], re, im);
+        w[j] = f32x2_to_bf16_bits(re, im);
+      }
+      qf = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    if (l == 0 && at.live) *reinterpret_cast<uint4*>(q_out + ((int64_t)at.b * units.Hq + at.head) * kMxD + d0) = qf;
   }
 
-  // register r: plane 4 quarter + r of head n (planes past the tenth repeat it and are dropped)
-  sh_f32x4 proj = sh_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) proj = sh_mfma(pl[ks], qf[ks], proj);
+  const sh_f32x4 t = mx_angles(sh_mfma(pl, qf, sh_f32x4{0.f, 0.f, 0.f, 0.f}), scale, wave, lane);
   float hi[4], mid[4], lo[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const float t = 4 * quarter + r < kMxK ? tanhf(proj[r]) * scale : 0.f;
-    hi[r] = sh_round<DType_bf16>(t);
-    mid[r] = sh_round<DType_bf16>(t - hi[r]);
-    lo[r] = t - hi[r] - mid[r];
+    hi[r] = sh_round<DType_bf16>(t[r]);
+    mid[r] = sh_round<DType_bf16>(t[r] - hi[r]);
+    lo[r] = t[r] - hi[r] - mid[r];
   }
   const uint4 t_high = make_uint4(f32x2_to_bf16_bits(hi[0], hi[1]), f32x2_to_bf16_bits(hi[2], hi[3]),
                                   f32x2_to_bf16_bits(mid[0], mid[1]), f32x2_to_bf16_bits(mid[2], mid[3]));
   const uint4 t_low = make_uint4(f32x2_to_bf16_bits(lo[0], lo[1]), f32x2_to_bf16_bits(lo[2], lo[3]), 0, 0);
-
-  // lg[c][ii][r]: bucket 256 wave + 64 c + 4 (4 quarter + r) + ii of head n
-  sh_f32x4 lg[4][4];
-  float mx = -INFINITY;
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
+  auto logits = [&](int c, sh_f32x4 (&lg)[4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int ii = 0; ii < 4; ++ii) {
       const uint32_t sel = (ii & 1) ? 0x07060302u : 0x05040100u;
       auto word = [&](int r) { return ii < 2 ? pr[c][r].x : pr[c][r].y; };
       const uint32_t a0 = __builtin_amdgcn_perm(word(1), word(0), sel), a1 = __builtin_amdgcn_perm(word(3), word(2), sel);
-      lg[c][ii] = sh_mfma(make_uint4(a0, a1, 0, 0), t_low, sh_f32x4{0.f, 0.f, 0.f, 0.f});
-      lg[c][ii] = sh_mfma(make_uint4(a0, a1, a0, a1), t_high, lg[c][ii]);
+      lg[ii] = sh_mfma(t_low, make_uint4(a0, a1, 0, 0), sh_f32x4{0.f, 0.f, 0.f, 0.f});
+      lg[ii] = sh_mfma(t_high, make_uint4(a0, a1, a0, a1), lg[ii]);
     }
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, lg[c][ii][r]);
-  mx = fmaxf(mx, lane_xor16(mx));
-  mx = fmaxf(mx, lane_xor32(mx));
-  if (quarter == 0) red[0][wave][n] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(red[0][0][n], red[0][1][n]), fmaxf(red[0][2][n], red[0][3][n]));
-  float sum = 0.f;
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        lg[c][ii][r] = __builtin_amdgcn_exp2f(lg[c][ii][r] - mx);
-        sum += lg[c][ii][r];
-      }
-  sum += lane_xor16(sum);
-  sum += lane_xor32(sum);
-  if (quarter == 0) red[1][wave][n] = sum;
-  __syncthreads();
-  sum = (red[1][0][n] + red[1][1][n]) + (red[1][2][n] + red[1][3][n]);
-  const float inv = live ? 1.f / sum : 0.f;          // (heads that only fill a unit up are zero)
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) lg[c][ii][r] *= inv;
-  if (!in_units) return;      // (whole groups of W lanes)
-
-  OT* base = out + ((int64_t)unit * L + l) * kMxR * W;
-  if constexpr (std::is_same<OT, float>::value) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) base[(wave * 256 + 64 * c + 16 * quarter + 4 * r + ii) * W + n % W] = lg[c][ii][r];
-  } else if constexpr (W == 1) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      uint32_t w[8];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        w[2 * r] = f32x2_to_bf16_bits(lg[c][0][r], lg[c][1][r]);
-        w[2 * r + 1] = f32x2_to_bf16_bits(lg[c][2][r], lg[c][3][r]);
-      }
-      uint4* to = reinterpret_cast<uint4*>(base + wave * 256 + 64 * c + 16 * quarter);
-      to[0] = make_uint4(w[0], w[1], w[2], w[3]);
-      to[1] = make_uint4(w[4], w[5], w[6], w[7]);
-    }
-  } else {
-    // heads of a unit lie on neighbouring lanes: exchanges between lanes x ^ 1 (and x ^ 2) leave lane j of the
-    // unit with the heads of bucket j (and j + 2) of four, a run of four buckets over ii
-    const uint32_t sel = (lane & 1) ? 0x03020706u : 0x05040100u;
-    const bool upper = (lane >> 1) & 1;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      uint32_t x[4], y[4];
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) {
-        const uint32_t w0 = f32x2_to_bf16_bits(lg[c][ii][0], lg[c][ii][1]);
-        const uint32_t w1 = f32x2_to_bf16_bits(lg[c][ii][2], lg[c][ii][3]);
-        const uint32_t a = __builtin_amdgcn_perm(sh_dpp_xor1(w0), w0, sel);       // two heads of bucket row (lane & 1)
-        const uint32_t d = __builtin_amdgcn_perm(sh_dpp_xor1(w1), w1, sel);       // ... and of row 2 + (lane & 1)
-        if constexpr (W == 2) {
-          x[ii] = a;
-          y[ii] = d;
-        } else {
-          const uint32_t got = sh_dpp_xor2(upper ? a : d), own = upper ? d : a;
-          x[ii] = upper ? got : own;
-          y[ii] = upper ? own : got;
-        }
-      }
-      const int row = wave * 256 + 64 * c + 16 * quarter;
-      if constexpr (W == 2) {
-        *reinterpret_cast<uint4*>(base + (row + 4 * (lane & 1)) * 2) = make_uint4(x[0], x[1], x[2], x[3]);
-        *reinterpret_cast<uint4*>(base + (row + 8 + 4 * (lane & 1)) * 2) = make_uint4(y[0], y[1], y[2], y[3]);
-      } else {
-        uint4* to = reinterpret_cast<uint4*>(base + (row + 4 * (lane & 3)) * 4);
-        to[0] = make_uint4(x[0], y[0], x[1], y[1]);
-        to[1] = make_uint4(x[2], y[2], x[3], y[3]);
-      }
-    }
-  }
+  };
+  auto reload = [&]() __attribute__((always_inline)) {
+    asm volatile("" : "+v"(protos_at));       // (fetched again, not kept in registers for a case that is rare)
+    load_protos();
+  };
+  mx_table<W, OutDT>(logits, reload, at.live, out, l, group, units.count, L, wave, lane);
 }
 
 __host__ __device__ __forceinline__ float mx_scale(float tanh_scale, float inv_temperature) {
@@ -350,7 +419,7 @@ __host__ __device__ __forceinline__ float mx_scale(float tanh_scale, float inv_t
 
 // The same for fp32 queries, planes and prototypes: v_mfma_f32_16x16x4_f32, which multiplies and adds in fp32 throughout, so
 // nothing is split.  Lane x holds column (or row) x % 16 and one k of four; which k that is is free as long as both operands
-// agree: for the projections quarter q takes dims 32 q .. + 31, a run, and for the logits step r takes plane 4 q + r,
+// agree: for the projections quarter q of wave w takes dims 32 q + 8 w .. + 7, a run, and for the logits step r takes plane 4 q + r,
 // which is what the lane's own projections are.
 // One sequence of 16 heads, 60 tables: 8.9 us as a launch of the scalar form below, 11.1 us with the rest of the prologue,
 // which took 9.3 us more, in one launch: a chain of trips to memory and of matrix products, on 80 workgroups.
@@ -363,29 +432,26 @@ __device__ __forceinline__ void soft_hash_mx32_block(const int l, const int grou
                                                      const void* __restrict__ freqs, const int64_t* __restrict__ pos, int pos_stride,
                                                      int64_t n_pos, float* __restrict__ q_out) {
   constexpr bool kRope = !std::is_void<FT>::value;
-  __shared__ float red[2][kSHWaves][kMxHeads];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, quarter = lane >> 4;
-  const int unit = group * (kMxHeads / W) + n / W;
-  const bool in_units = unit < units.count;
-  const int u = in_units ? unit : 0;
-  const int per_seq = units.parts > 0 ? units.Hkv * units.parts : units.Hq;
-  const int b = u / per_seq, at = u % per_seq;
-  const int member = units.parts > 0 ? at % units.parts * W + n % W : 0;       // of the kv head's group
-  const bool live = in_units && (units.parts == 0 || member < units.G);
-  const int head = units.parts > 0 ? at / units.parts * units.G + (live ? member : 0) : at;
+  const MxHead at = mx_head<W>(group, units, n);
 
-  const float* qrow = q + b * q_sb + head * q_sh + 32 * quarter;
-  const float* prow = planes + ((int64_t)l * kMxK + min(n, kMxK - 1)) * kMxD + 32 * quarter;
+  const int d0 = 32 * quarter + 8 * wave;
+  const float* qrow = q + at.b * q_sb + at.head * q_sh + d0;
+  const float* prow = planes + ((int64_t)l * kMxK + min(n, kMxK - 1)) * kMxD + d0;
   int64_t p = 0;
-  bool turn = false;
-  if constexpr (kRope) {
-    p = pos[(int64_t)b * pos_stride];
-    turn = p >= 0 && p < n_pos;
-  }
-  float x[32], pl[32], pr[4][4][4];
+  if constexpr (kRope) p = pos[(int64_t)at.b * pos_stride];
+  float x[8], pl[8], pr[4][4][4];
+  uint32_t protos_at = 0;
+  auto load_protos = [&]() __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < 32; i += 4) {
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sh_load4<DType_f32>(protos_T, protos_at + min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c + 4 * n, pr[c][r]);
+  };
+#pragma unroll
+  for (int i = 0; i < 8; i += 4) {
     float t[4];
     sh_load4<DType_f32>(qrow, i, t);
 #pragma unroll
@@ -394,124 +460,50 @@ __device__ __forceinline__ void soft_hash_mx32_block(const int l, const int grou
 #pragma unroll
     for (int e = 0; e < 4; ++e) pl[i + e] = t[e];
   }
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      sh_load4<DType_f32>(protos_T, min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c + 4 * n, pr[c][r]);
+  load_protos();
   if constexpr (kRope) {
+    const bool turn = p >= 0 && p < n_pos;
     // (angles of row 0 for a position outside the table: a load under a condition is waited for at once)
-    float f[4][8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sh_load8<FT>(freqs, (turn ? p : 0) * kMxD + 32 * quarter + 8 * i, f[i]);
+    float f[8];
+    sh_load8<FT>(freqs, (turn ? p : 0) * kMxD + d0, f);
     if (turn) {
 #pragma unroll
-      for (int i = 0; i < 32; i += 2) {
+      for (int i = 0; i < 8; i += 2) {
         float re, im;
-        rotate_pair(x[i], x[i + 1], f[i / 8][i % 8], f[i / 8][i % 8 + 1], re, im);
+        rotate_pair(x[i], x[i + 1], f[i], f[i + 1], re, im);
         x[i] = re, x[i + 1] = im;
       }
     }
-    if (l == 0 && wave == 0 && live) {
+    if (l == 0 && at.live) {
 #pragma unroll
-      for (int i = 0; i < 32; i += 4) {
+      for (int i = 0; i < 8; i += 4) {
         const float t[4] = {x[i], x[i + 1], x[i + 2], x[i + 3]};
-        sh_store4<DType_f32>(q_out, ((int64_t)b * units.Hq + head) * kMxD + 32 * quarter + i, t);
+        sh_store4<DType_f32>(q_out, ((int64_t)at.b * units.Hq + at.head) * kMxD + d0 + i, t);
       }
     }
   }
 
   // register r: plane 4 quarter + r of head n (planes past the tenth repeat it and are dropped).  Eight sums of sixteen
-  // products, added in pairs: one of 128 loses more than the scalar form's.
-  constexpr int kChains = 8;
-  sh_f32x4 proj[kChains];
+  // products over the four waves, added in pairs: one of 128 loses more than the scalar form's.
+  sh_f32x4 proj[2] = {sh_f32x4{0.f, 0.f, 0.f, 0.f}, sh_f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-  for (int j = 0; j < kChains; ++j) proj[j] = sh_f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < 8; ++i) proj[i % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(pl[i], x[i], proj[i % 2], 0, 0, 0);
+  const sh_f32x4 t = mx_angles(proj[0] + proj[1], scale, wave, lane);
+  auto logits = [&](int c, sh_f32x4 (&lg)[4]) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < 32; ++i) proj[i % kChains] = __builtin_amdgcn_mfma_f32_16x16x4f32(pl[i], x[i], proj[i % kChains], 0, 0, 0);
+    for (int ii = 0; ii < 4; ++ii) lg[ii] = sh_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int j = kChains / 2; j > 0; j /= 2)
-#pragma unroll
-    for (int i = 0; i < j; ++i) proj[i] += proj[i + j];
-  float t[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) t[r] = 4 * quarter + r < kMxK ? tanhf(proj[0][r]) * scale : 0.f;
-
-  // lg[c][ii][r]: bucket 256 wave + 64 c + 4 (4 quarter + r) + ii of head n
-  sh_f32x4 lg[4][4];
-  float mx = -INFINITY;
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii) lg[c][ii] = sh_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii)
         // (no prototype past the tenth: zeros, whatever the tenth is)
-        lg[c][ii] = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * quarter + r < kMxK ? pr[c][r][ii] : 0.f, t[r], lg[c][ii], 0, 0, 0);
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, lg[c][ii][r]);
-  mx = fmaxf(mx, lane_xor16(mx));
-  mx = fmaxf(mx, lane_xor32(mx));
-  if (quarter == 0) red[0][wave][n] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(red[0][0][n], red[0][1][n]), fmaxf(red[0][2][n], red[0][3][n]));
-  float sum = 0.f;
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        lg[c][ii][r] = __builtin_amdgcn_exp2f(lg[c][ii][r] - mx);
-        sum += lg[c][ii][r];
-      }
-  sum += lane_xor16(sum);
-  sum += lane_xor32(sum);
-  if (quarter == 0) red[1][wave][n] = sum;
-  __syncthreads();
-  sum = (red[1][0][n] + red[1][1][n]) + (red[1][2][n] + red[1][3][n]);
-  const float inv = live ? 1.f / sum : 0.f;          // (heads that only fill a unit up are zero)
-  if (!in_units) return;      // (whole groups of W lanes)
-  typename OutDT::storage* base = (typename OutDT::storage*)out + ((int64_t)unit * L + l) * kMxR * W;
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float v[4];
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) v[ii] = lg[c][ii][r] * inv;
-      const int bucket = wave * 256 + 64 * c + 16 * quarter + 4 * r;
-      if constexpr (W == 4) {
-        // a quad of lanes holds four heads of four buckets: transposed, lane j has the heads of bucket j
-        const bool up2 = lane & 2, up1 = lane & 1;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const float got = __uint_as_float(sh_dpp_xor2(__float_as_uint(up2 ? v[i] : v[i + 2])));
-          v[i] = up2 ? got : v[i];
-          v[i + 2] = up2 ? v[i + 2] : got;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i += 2) {
-          const float got = __uint_as_float(sh_dpp_xor1(__float_as_uint(up1 ? v[i] : v[i + 1])));
-          v[i] = up1 ? got : v[i];
-          v[i + 1] = up1 ? v[i + 1] : got;
-        }
-        sh_store4<OutDT>(base, (bucket + (lane & 3)) * 4, v);
-      } else if constexpr (W == 1) {
-        sh_store4<OutDT>(base, bucket, v);
-      } else {
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii) store_elem<OutDT>(base, (bucket + ii) * W + n % W, v[ii]);
-      }
-    }
+        lg[ii] = __builtin_amdgcn_mfma_f32_16x16x4f32(t[r], 4 * quarter + r < kMxK ? pr[c][r][ii] : 0.f, lg[ii], 0, 0, 0);
+  };
+  auto reload = [&]() __attribute__((always_inline)) {
+    asm volatile("" : "+v"(protos_at));       // (fetched again, not kept in registers for a case that is rare)
+    load_protos();
+  };
+  mx_table<W, OutDT>(logits, reload, at.live, out, l, group, units.count, L, wave, lane);
 }
 
 template <int W, class OutDT>
@@ -522,12 +514,12 @@ __global__ __launch_bounds__(kSHThreads) void soft_hash_mx32_kernel(const float*
                                 nullptr);
 }
 
-template <int W, class OT>
+template <int W, class OutDT>
 __global__ __launch_bounds__(kSHThreads) void soft_hash_mx_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_sh,
                                                                   const uint16_t* __restrict__ planes,
-                                                                  const uint16_t* __restrict__ protos_T, OT* __restrict__ out,
+                                                                  const uint16_t* __restrict__ protos_T, void* __restrict__ out,
                                                                   MxUnits units, int L, float scale) {
-  soft_hash_mx_block<void, W, OT>(blockIdx.x, blockIdx.y, units, q, q_sb, q_sh, planes, protos_T, out, L, scale, nullptr, nullptr, 0, 0,
+  soft_hash_mx_block<void, W, OutDT>(blockIdx.x, blockIdx.y, units, q, q_sb, q_sh, planes, protos_T, out, L, scale, nullptr, nullptr, 0, 0,
                                   nullptr);
 }
 
@@ -1041,8 +1033,8 @@ __global__ __launch_bounds__(kSHThreads) void decode_prologue_kernel(
       soft_hash_mx32_block<FT, W, DType_f32>(l, pair, units, qkv, qkv_sb, D, (const float*)planes, (const float*)protos_T, q_table, L, mx,
                                   freqs, pos, pos_stride, n_pos, q_out);
     } else if constexpr (GC == 0) {
-      soft_hash_mx_block<FT, W, OT>(l, pair, units, qkv, qkv_sb, D, (const uint16_t*)planes, (const uint16_t*)protos_T, (OT*)q_table, L,
-                                    mx, freqs, pos, pos_stride, n_pos, q_out);
+      soft_hash_mx_block<FT, W, std::conditional_t<sizeof(OT) == 4, DType_f32, DType_bf16>>(
+          l, pair, units, qkv, qkv_sb, D, (const uint16_t*)planes, (const uint16_t*)protos_T, q_table, L, mx, freqs, pos, pos_stride, n_pos, q_out);
     } else {
       const int64_t p = pos[(int64_t)(pair / Hkv) * pos_stride];
       const bool turn = p >= 0 && p < n_pos;
@@ -1179,7 +1171,8 @@ namespace {
 bool mx_serves(int D, int K, int R) { return D == kMxD && K == kMxK && R == kMxR; }
 
 MxUnits mx_units(int B, int Hq, int Hkv, int parts) {
-  return {parts > 0 ? B * Hkv * parts : B * Hq, parts, Hq, Hkv, Hq / Hkv};
+  const int per_seq = parts > 0 ? Hkv * parts : Hq;
+  return {B * per_seq, parts, Hq, Hkv, Hq / Hkv, per_seq, 1.f / (float)per_seq, parts > 0 ? 1.f / (float)parts : 0.f};
 }
 
 int soft_hash_entry(const void* q, int dtype, int64_t q_stride_b, int64_t q_stride_h, const void* planes,
@@ -1216,11 +1209,11 @@ int soft_hash_entry(const void* q, int dtype, int64_t q_stride_b, int64_t q_stri
 #define SOCKET_MX(WV)                                                                                                         \
   do {                                                                                                                        \
     if (out_dtype == SOCKET_F32)                                                                                              \
-      hipLaunchKernelGGL((soft_hash_mx_kernel<WV, float>), mx_grid, dim3(kSHThreads), 0, s, (const uint16_t*)q, q_stride_b,   \
-                         q_stride_h, (const uint16_t*)planes, (const uint16_t*)protos_T, (float*)out, units, L, scale);       \
+      hipLaunchKernelGGL((soft_hash_mx_kernel<WV, DType_f32>), mx_grid, dim3(kSHThreads), 0, s, (const uint16_t*)q, q_stride_b,  \
+                         q_stride_h, (const uint16_t*)planes, (const uint16_t*)protos_T, out, units, L, scale);               \
     else                                                                                                                      \
-      hipLaunchKernelGGL((soft_hash_mx_kernel<WV, uint16_t>), mx_grid, dim3(kSHThreads), 0, s, (const uint16_t*)q, q_stride_b, \
-                         q_stride_h, (const uint16_t*)planes, (const uint16_t*)protos_T, (uint16_t*)out, units, L, scale);    \
+      hipLaunchKernelGGL((soft_hash_mx_kernel<WV, DType_bf16>), mx_grid, dim3(kSHThreads), 0, s, (const uint16_t*)q, q_stride_b, \
+                         q_stride_h, (const uint16_t*)planes, (const uint16_t*)protos_T, out, units, L, scale);               \
   } while (0)
     if (W == 4) SOCKET_MX(4);
     else if (W == 2) SOCKET_MX(2);

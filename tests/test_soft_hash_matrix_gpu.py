@@ -60,3 +60,47 @@ def test_a_head_of_nan_stays_alone():
     assert torch.equal(got[keep], clean[keep]) and got[1, 3].isnan().all()
     # an infinite coordinate saturates every plane it meets
     assert torch.allclose(got[0, 2].double(), exact(q, planes, protos, 0.3)[0, 2], rtol=2 ** -8)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("G", [1, 2, 4])
+def test_large_logits_in_some_heads(dtype, G):
+    """Logits up to thousands in one head of sixteen: nothing overflows, and the heads beside it have what they have without it."""
+    Hq, L, temp = 4 * G, 3, 0.3
+    q, planes, protos = inputs(3, Hq, L, G, True)
+    q, planes, protos = q.to(dtype), (0.02 * planes).to(dtype), protos.to(dtype) * 16
+    planes[1, 4:] *= 1000                                  # (table 1 saturates: logits of up to 16 * 10 / sqrt(128) / 0.3 = 47)
+    q[0] *= 0.01
+    small = hash_cache.soft_hash(q, planes, protos, temp, 4, out_dtype=torch.float32)
+    q2 = q.clone()
+    q2[1, 0] *= 100
+    got = hash_cache.soft_hash(q2, planes, protos, temp, 4, out_dtype=torch.float32)
+    keep = torch.ones(3, Hq, dtype=torch.bool, device=DEV)
+    keep[1, 0] = False
+    assert torch.equal(got[keep], small[keep])
+    want = exact(q2, planes, protos, temp)
+    # (logits up to 68 in base 2: sixteen roundings of that size, and where the largest is taken off one more; the projections'
+    # 128 products, added up in fp32, are off by 128 * 2^-24 of 128 * 0.02 * 4 in front of a slope of 16 * 10 / sqrt(128) / 0.3)
+    bound = 2 ** -23 * (16 + 17 * 68 + 64 * 10 * 47)
+    assert ((got.double() - want).abs() <= bound * want + 1e-37).all()
+    assert torch.equal(hash_cache.soft_hash(q2, planes, protos, temp, 4, out_dtype=torch.float32, grouped=True)[:, 2, :, :, 0], got[:, 2 * G])
+    # far past what an exponential holds: one bucket has it all, and the sums stay finite
+    far = hash_cache.soft_hash(q2, planes * 1000, protos * 64, temp, 4, out_dtype=torch.float32)
+    assert far.isfinite().all() and torch.allclose(far.sum(-1), torch.ones_like(far[..., 0]), atol=1e-4)
+
+
+@pytest.mark.parametrize("Hq,Hkv,B", [(8, 8, 3), (28, 4, 5), (6, 3, 7), (16, 4, 1)])
+def test_float32_tables_of_every_layout(Hq, Hkv, B):
+    """fp32 operands, units that do not fill a workgroup's sixteen heads or cross sequences, padded groups."""
+    q, planes, protos = (x.float() for x in inputs(B, Hq, 5, Hq, False))
+    parts, width = hash_cache.group_shape(Hq, Hkv)
+    G = Hq // Hkv
+    want = exact(q, planes, protos, 0.3)
+    flat = hash_cache.soft_hash(q, planes, protos, 0.3, Hkv)
+    assert ((flat.double() - want).abs() <= 2 ** -23 * (16 + 16 * 0.9 * 4 / 0.3) * want).all()
+    got = hash_cache.soft_hash(q, planes, protos, 0.3, Hkv, grouped=True)
+    for h in range(Hq):
+        kv, g = h // G, h % G
+        assert torch.equal(got[:, kv * parts + g // width, :, :, g % width], flat[:, h])
+    for g in range(G, parts * width):
+        assert (got.view(B, Hkv, parts, 5, 1024, width)[:, :, g // width, :, :, g % width] == 0).all()
