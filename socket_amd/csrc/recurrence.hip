@@ -1156,15 +1156,18 @@ constexpr int kScanWaves = 4;     // of either kind
 
 // The chunks of one (16 value columns, head, sequence) in order, by two kinds of waves, one of each on a SIMD:
 //  * wave w of the first four has state tiles w, w + 4, ... and, with the delta rule, row block w of U = Ubar - W S;
-//  * wave w of the others reads row block w out, O = Q^ S + Aqk U, which nothing later waits for.
+//  * wave w of the others reads row block w out, O = Q^ S + Aqk U, which nothing later waits for: it takes S and U into
+//    registers as soon as they are there and works a barrier behind the first kind, whose waits its products fill.
 // S and (DELTA) U pass through LDS, S in two copies so that one is read while the next is written; without the delta
 // rule U is what the preparation left, and a chunk has one barrier instead of two.  KT: 16-row state tiles.
 // EXTRA: rule 1's additions to the read-outs and the state.
 // The chain state -> U -> state bounds it: its products are dependent, with an LDS exchange after each half.  Four waves
 // that did both, fragments one chunk ahead, took 245 us for 5000 tokens x 16 heads x 128 key channels with the delta rule and
 // 116 for 64 without; these 204 and 108 (eight waves alone 229 and 127, with fragments two chunks ahead 212 and 109, with a
-// chunk's state tiles asked for together and the first kind's products first the rest).  Two accumulators in turn for
-// every chain changed nothing.
+// chunk's state tiles asked for together and the first kind's products first the rest).  Read-outs a barrier behind: 32
+// chunks of 16 heads of 128 x 128 with the delta rule 70.8 -> 66.9 us, of 64 x 128 without 40.0 -> 39.0.  Two accumulators in turn
+// for every chain: 69.3.  Without its matrix products such a launch takes 56, without its loads 69: the fragments of a
+// chunk, 116 KB, come at 31 bytes a cycle.
 template <int KT, int NB, bool DELTA, bool EXTRA>
 __global__ __launch_bounds__(kScanThreads, 2) void recurrence_scan_kernel(socket_recurrence a, int n_chunks) {
   constexpr int C = 16 * NB;
@@ -1218,30 +1221,47 @@ __global__ __launch_bounds__(kScanThreads, 2) void recurrence_scan_kernel(socket
       for (int J = 0; J < NB; ++J) fa[p][J] = a_tile(c, J);
       in_order();
     }
+    rc_f32x4 x[KT], u[NB];
+    auto take_state = [&](const float* from) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < KT; ++j) x[j] = acc_tile(from + j * 256);
+    };
+    auto take_u = [&](const float* from) __attribute__((always_inline)) {
+#pragma unroll
+      for (int J = 0; J < NB; ++J) u[J] = acc_tile(from + J * 256);
+    };
     __syncthreads();   // the first state
+    if (rows_mine) {
+      take_state(s_lds[0]);
+      if (!DELTA) take_u(u_lds[0]);
+    }
+    __syncthreads();   // the first U; without the delta rule the second state
     auto chunk = [&](int n, auto half) __attribute__((always_inline)) {
-      constexpr int at = decltype(half)::value, p = at % SETS;
+      constexpr int at = decltype(half)::value, p = at % SETS, next = DELTA ? 0 : at ^ 1;
       const float* nx = chunk_at(n + SETS);
-      const float* S = s_lds[at];
+      const bool more = n + 1 < n_chunks;
       rc_f32x4 o = fo[p];
       if (rows_mine) {
-        rc_f32x4 x[KT];
-#pragma unroll
-        for (int j = 0; j < KT; ++j) x[j] = acc_tile(S + j * 256);
-        __builtin_amdgcn_sched_barrier(0);     // (every tile asked for before the first product)
 #pragma unroll
         for (int j = 0; j < KT; ++j) {
           o = mfma4(fq[p][j], x[j], o);
           fq[p][j] = q_tile(nx, j);
         }
         if (EXTRA) fo[p] = acc_tile(nx + sp.o() + (wb * sp.vt + slice) * 256);
+        in_order();
+        if (DELTA) take_u(u_lds[0]);
       }
-      if (DELTA) __syncthreads();   // U complete
+      if (DELTA) __syncthreads();   // the next state complete, this U read
       if (rows_mine) {
 #pragma unroll
         for (int J = 0; J < NB; ++J) {
-          if (J <= wave) o = mfma4(fa[p][J], acc_tile(u_lds[DELTA ? 0 : at] + J * 256), o);
+          if (J <= wave) o = mfma4(fa[p][J], u[J], o);
           fa[p][J] = a_tile(nx, J);
+        }
+        in_order();
+        if (more) {
+          take_state(s_lds[at ^ 1]);
+          if (!DELTA) take_u(u_lds[next]);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -1249,7 +1269,7 @@ __global__ __launch_bounds__(kScanThreads, 2) void recurrence_scan_kernel(socket
           if (t < a.n && col_ok) a.o_buf[(((int64_t)b * a.n + t) * a.H + h) * a.dv + col] = o[r];
         }
       }
-      __syncthreads();   // the next state complete, U and this one read
+      if (more) __syncthreads();   // the next U complete, without the delta rule the state after the next; those taken read
     };
     for (int n = 0; n + 1 < n_chunks; n += 2) {
       chunk(n, std::integral_constant<int, 0>{});
