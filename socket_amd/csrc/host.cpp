@@ -6,8 +6,11 @@
 // 4.6 of the host's under it.
 #include <Python.h>
 
+#include <ATen/ops/empty.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <exception>
 
 #include "../../include/socket_hip.h"
@@ -105,7 +108,146 @@ PyObject* cache_append(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return PyLong_FromLong(status);
 }
 
+// ---- the list builder and the attention over its list -------------------------------------------
+//
+// Over 4448 tokens of 32 heads (32 tables x 256) the two are some 20 us on the GPU, and their Python took the host 37.5: looking
+// operands over, five allocations and four calls through ctypes.  Now 18 to 21, and such a stream of calls 38.5 / 20.5 to 22 us each.
+// Operands in another form than these take go the way through Python, which also says what is wrong with them.
+int type_of(at::ScalarType t) {
+  return t == at::kFloat ? SOCKET_F32 : t == at::kBFloat16 ? SOCKET_BF16 : t == at::kHalf ? SOCKET_F16 : -1;
+}
+
+// The first n arguments as tensors of one HIP device.
+template <int N>
+bool tensors(PyObject* const* args, const at::Tensor* (&t)[N]) {
+  for (int i = 0; i < N; ++i) {
+    if (!plain(args[i])) return false;
+    t[i] = &THPVariable_Unpack(args[i]);
+    if (!t[i]->is_cuda() || t[i]->device() != t[0]->device() || t[i]->layout() != at::kStrided) return false;
+  }
+  return true;
+}
+
+PyObject* none() { Py_RETURN_NONE; }
+
+// What a call that did not return 0 is answered with: its name and its status.
+PyObject* failed(const char* name, int status) { return Py_BuildValue("si", name, status); }
+
+// build_list(q_probs, k_hard, v_norm, allowed, sink, window, M, max_base, max_M, workspace, stream): (list, lengths), None if
+// the operands do not fit, (name, status) of a call that failed.  workspace(device, bytes, zero bytes) is asked where one is needed.
+PyObject* build_list(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 11) {
+    PyErr_SetString(PyExc_TypeError, "build_list takes 11 arguments");
+    return nullptr;
+  }
+  const at::Tensor* t[4];
+  if (!tensors(args, t)) return none();
+  long long num[6];      // sink, window, M, max_base, max_M, stream
+  for (int i = 0; i < 6; ++i) {
+    PyObject* o = args[i < 5 ? 4 + i : 10];
+    if (!PyLong_CheckExact(o)) return none();
+    num[i] = PyLong_AsLongLong(o);
+    if (num[i] == -1 && PyErr_Occurred()) {
+      PyErr_Clear();
+      return none();
+    }
+  }
+  const at::Tensor &q = *t[0], &k = *t[1], &norms = *t[2], &allowed = *t[3];
+  if (q.dim() != 4 || k.dim() != 4 || norms.dim() != 3 || allowed.dim() != 3) return none();
+  const int64_t B = q.size(0), H = q.size(1), L = q.size(2), R = q.size(3), T = k.size(3);
+  const int64_t M = std::min<int64_t>(num[2], T), rows[3] = {B, H, T};
+  if (std::min({B, H, L, R, T, M}) < 1 || B * H > 65535 || std::max({L, R, T}) > INT32_MAX || M > num[4] || k.size(0) != B ||
+      k.size(1) != H || k.size(2) != L || norms.sizes() != at::IntArrayRef(rows) || allowed.sizes() != at::IntArrayRef(rows) ||
+      k.scalar_type() != at::kShort || allowed.scalar_type() != at::kBool || type_of(q.scalar_type()) < 0 ||
+      type_of(norms.scalar_type()) < 0)
+    return none();
+  for (const at::Tensor* x : t)
+    if (!x->is_contiguous()) return none();
+  const int64_t sink = std::clamp<int64_t>(num[0], 0, T), window = std::clamp<int64_t>(num[1], 0, T);
+  const int64_t base = std::max<int64_t>(1, sink + (window > 0 ? T - std::max(T - window, sink) : 0)), width = base + M;
+  if (base > num[3]) return none();
+  const size_t bytes = socket_select_workspace_bytes((int)B, (int)H, (int)T, (int)M);
+  at::Tensor ws;
+  if (bytes > 0) {
+    PyObject* device = PyObject_GetAttrString(args[0], "device");
+    if (!device) return nullptr;
+    PyObject* got = PyObject_CallFunction(args[9], "OKK", device, (unsigned long long)bytes,
+                                          (unsigned long long)socket_select_workspace_zero_bytes((int)B, (int)H, (int)T, (int)M));
+    Py_DECREF(device);
+    if (!got) return nullptr;
+    if (THPVariable_Check(got)) ws = THPVariable_Unpack(got);
+    Py_DECREF(got);
+    if (!ws.defined()) return none();
+  }
+  const auto on = at::TensorOptions().device(q.device());
+  at::Tensor scores = at::empty({B, H, T}, on.dtype(at::kFloat)), list = at::empty({B, H, width}, on.dtype(at::kInt)),
+             lengths = at::empty({B, H}, on.dtype(at::kInt));
+  const void *pq = q.data_ptr(), *pk = k.data_ptr(), *pn = norms.data_ptr(), *pa = allowed.data_ptr();
+  void *ps = scores.data_ptr(), *pl = list.data_ptr(), *pc = lengths.data_ptr(), *pw = bytes > 0 ? ws.data_ptr() : nullptr;
+  const int q_type = type_of(q.scalar_type()), norm_type = type_of(norms.scalar_type());
+  int scored = 0, selected = 0;
+  Py_BEGIN_ALLOW_THREADS
+  scored = socket_soft_hash_collision_typed(pq, q_type, (const int16_t*)pk, (const uint8_t*)pa, pn, norm_type, (float*)ps, (int)B, (int)H,
+                                            (int)L, (int)R, (int)T, (void*)num[5]);
+  if (scored == SOCKET_OK)
+    selected = socket_select_list_allowed((const float*)ps, T, (const uint8_t*)pa, (int)B, (int)H, (int)T, (int)M, (int)sink, (int)window,
+                                          (int32_t*)pl, width, (int)width, (int32_t*)pc, pw, bytes, (void*)num[5]);
+  Py_END_ALLOW_THREADS
+  if (scored != SOCKET_OK) return failed("socket_soft_hash_collision", scored);
+  if (selected != SOCKET_OK) return failed("socket_select_list", selected);
+  PyObject* out[2] = {THPVariable_Wrap(std::move(list)), THPVariable_Wrap(std::move(lengths))};
+  PyObject* both = out[0] && out[1] ? PyTuple_Pack(2, out[0], out[1]) : nullptr;
+  Py_XDECREF(out[0]);
+  Py_XDECREF(out[1]);
+  return both;
+  END_HANDLE_TH_ERRORS
+}
+
+// sparse_attention(query, key, value, list, lengths, stream): the output, None if the operands do not fit, (name, status) of
+// a call that failed.
+PyObject* sparse_attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 6) {
+    PyErr_SetString(PyExc_TypeError, "sparse_attention takes 6 arguments");
+    return nullptr;
+  }
+  const at::Tensor* t[5];
+  if (!tensors(args, t)) return none();
+  const long long stream = PyLong_AsLongLong(args[5]);
+  if (stream == -1 && PyErr_Occurred()) return nullptr;
+  const at::Tensor &q = *t[0], &k = *t[1], &v = *t[2], &list = *t[3], &lengths = *t[4];
+  if (q.dim() != 3 || k.dim() != 4 || v.dim() != 4 || list.dim() != 3 || lengths.dim() != 2) return none();
+  const int64_t B = q.size(0), H = q.size(1), D = q.size(2), Hkv = k.size(1), rows = k.size(2), width = list.size(2);
+  const int type = type_of(q.scalar_type());
+  if (type < 0 || k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() || (D != 16 && D != 32 && D != 64 && D != 128) ||
+      k.size(3) != D || v.size(3) != D || q.stride(2) != 1 || k.stride(3) != 1 || v.stride(3) != 1 || std::min({B, H, Hkv, rows, width}) < 1 ||
+      H % Hkv != 0 || std::max({B, H, rows, width}) > INT32_MAX || list.scalar_type() != at::kInt || lengths.scalar_type() != at::kInt ||
+      list.stride(2) != 1 || k.size(0) != B || v.sizes() != k.sizes() || list.size(0) != B || list.size(1) != H ||
+      lengths.sizes() != list.sizes().slice(0, 2))
+    return none();
+  const size_t bytes = socket_sparse_attention_workspace_bytes((int)B, (int)H, (int)D, (int)width);
+  at::Tensor out = at::empty({B, H, D}, at::TensorOptions().device(q.device()).dtype(q.scalar_type())),
+             ws = at::empty({(int64_t)(bytes / 4)}, at::TensorOptions().device(q.device()).dtype(at::kFloat));
+  const void *pq = q.data_ptr(), *pk = k.data_ptr(), *pv = v.data_ptr(), *pl = list.data_ptr(), *pc = lengths.data_ptr();
+  void *po = out.data_ptr(), *pw = ws.data_ptr();
+  const int64_t s[10] = {q.stride(0), q.stride(1), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
+                         list.stride(0), list.stride(1)};
+  const int64_t c0 = lengths.stride(0), c1 = lengths.stride(1);
+  int status = 0;
+  Py_BEGIN_ALLOW_THREADS
+  status = socket_sparse_attention(pq, pk, pv, type, s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], (const int32_t*)pl, s[8], s[9],
+                                   (const int32_t*)pc, c0, c1, po, H * D, D, pw, bytes, (int)B, (int)H, (int)Hkv, (int)D, (int)rows,
+                                   (int)width, (void*)stream);
+  Py_END_ALLOW_THREADS
+  if (status != SOCKET_OK) return failed("socket_sparse_attention", status);
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"build_list", (PyCFunction)(void (*)())build_list, METH_FASTCALL, nullptr},
+    {"sparse_attention", (PyCFunction)(void (*)())sparse_attention, METH_FASTCALL, nullptr},
     {"cache_append", (PyCFunction)(void (*)())cache_append, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
