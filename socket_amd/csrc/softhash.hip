@@ -115,7 +115,7 @@ __device__ __forceinline__ void sh_store4<DType_f16>(void* p, int64_t i, const f
 // What bounds it are vector instructions, about 600 a wave at 64 logits a lane, and at few heads dependent trips to memory.
 // Before (head as the N index of both products: entries put together by lane exchanges; every wave rotated and projected
 // everything; maxima exchanged and taken off) and now, the decode prologue with the rest of its roles: one sequence of 32 heads x
-// 60 tables 7.7 / 6.3 us, four 13.4 / 10.9, sixteen of 28 x 48 27.2 / 23.4.  (The scalar form below spends ten multiply-adds
+// 60 tables 7.7 / 6.2 us, four 13.4 / 10.5, sixteen of 28 x 48 27.2 / 20.4.  (The scalar form below spends ten multiply-adds
 // and a library exponential per head and bucket: 10.4, 23 and 56 us.)
 //
 // W: heads of a unit (the scorer's grouped layout [unit, L, R, W]; 1 for the reference's [B,Hq,L,R], whose
@@ -290,7 +290,7 @@ __device__ __forceinline__ void mx_table(const LOGITS& logits, const RELOAD& rel
       }
     }
   };
-  if (__builtin_amdgcn_readfirstlane(wide[0] | wide[1] | wide[2] | wide[3]) == 0) {
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane(wide[0] | wide[1] | wide[2] | wide[3]) == 0, 1)) {
     write(total(0));
     return;
   }
@@ -351,11 +351,14 @@ __device__ __forceinline__ void soft_hash_mx_block(const int l, const int group,
   uint2 pr[4][4];
   uint32_t protos_at = 0;
   auto load_protos = [&]() __attribute__((always_inline)) {
+    // (byte offsets of 32 bits beside a common address)
+    const char* at0 = (const char*)protos_T + wave * 512;
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t off = protos_at + (uint32_t)min(4 * quarter + r, kMxK - 1) * (kMxR * 2) + 8 * n;
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        pr[c][r] = *reinterpret_cast<const uint2*>(protos_T + (protos_at + min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c + 4 * n));
+      for (int c = 0; c < 4; ++c) pr[c][r] = *reinterpret_cast<const uint2*>(at0 + off + 128 * c);
+    }
     if (quarter >= 2) {         // (no prototype past the tenth: zeros, whatever the tenth is)
 #pragma unroll
       for (int c = 0; c < 4; ++c)
@@ -515,7 +518,7 @@ __global__ __launch_bounds__(kSHThreads) void soft_hash_mx32_kernel(const float*
 }
 
 template <int W, class OutDT>
-__global__ __launch_bounds__(kSHThreads) void soft_hash_mx_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_sh,
+__global__ __launch_bounds__(kSHThreads, 4) void soft_hash_mx_kernel(const uint16_t* __restrict__ q, int64_t q_sb, int64_t q_sh,
                                                                   const uint16_t* __restrict__ planes,
                                                                   const uint16_t* __restrict__ protos_T, void* __restrict__ out,
                                                                   MxUnits units, int L, float scale) {
@@ -1011,8 +1014,11 @@ __device__ __forceinline__ uint4 sh_bf16_of8(const sh_row8<DT>& r) {
 // DT: type of the projection, the caches, planes and prototypes.
 // GC: as in soft_hash_block (bf16 only), or 0: soft_hash_mx_block or soft_hash_mx32_block with units of W heads, OT the
 // output's elements; below zero: soft_hash_small_block for at most -GC planes.
+// (bf16 operands on the matrix cores: four waves a SIMD, whose registers the usual path fits; what the rare one spills is its own.  At
+// the three that 164 registers leave, sixteen sequences of 28 heads x 48 tables take 23.4 us instead of 20.4, four of 32 x 60 11.0
+// instead of 10.5.)
 template <class DT, int GC, class FT, int W, class OT>
-__global__ __launch_bounds__(kSHThreads) void decode_prologue_kernel(
+__global__ __launch_bounds__(kSHThreads, GC == 0 && DT::kEnum == SOCKET_BF16 ? 4 : 1) void decode_prologue_kernel(
     const typename DT::storage* __restrict__ qkv, int64_t qkv_sb, const void* __restrict__ freqs,
     const int64_t* __restrict__ pos, int pos_stride, int64_t n_pos, typename DT::storage* __restrict__ q_out,
     typename DT::storage* __restrict__ k_cache, typename DT::storage* __restrict__ v_cache, int64_t c_sb, int64_t c_sh, int64_t c_ss,
