@@ -107,8 +107,7 @@ __device__ __forceinline__ void sh_store4<DType_f16>(void* p, int64_t i, const f
 // The head is the N index of the first: lane x holds head x % 16, and the planes of lane quarter q are 4 q .. + 3; the terms a
 // lane splits off are the operand it has to supply to the second, where the head is the M index: register r of quarter q is head 4 q + r,
 // so that the heads of a unit lie in one lane and an entry of the table is stored as it is.  Bucket order inside a product is free:
-// block ii of a 64-bucket chunk takes buckets 4 n + ii for column n, so that a lane's prototypes are runs of four (8-byte
-// loads) and its results runs of four entries.  A wave has 256 buckets.  Of what all four waves need, each works out a share: a
+// a lane's prototypes and its results are runs of kMxRun16 buckets.  A wave has 256 buckets.  Of what all four waves need, each works out a share: a
 // quarter of the dims of the rotation and the projections, one plane of four of the tanh.  Logits are made in base-2 units
 // (log2 e goes into t) for the hardware's exponential, and nothing is taken off them first where all of a head's are small,
 // which they are with +-1 prototypes (tanh / sqrt(D) / temperature: at most 4.3); it is seen from the logits themselves.
@@ -216,9 +215,42 @@ __device__ __forceinline__ sh_f32x4 mx_angles(const sh_f32x4& part, float scale,
   return *reinterpret_cast<const sh_f32x4*>(angles[lane]);
 }
 
-// logits(c, lg): lg[ii][r] is bucket 256 wave + 64 c + 4 n + ii of head 4 quarter + r, in base-2 units, from prototypes that
-// reload() fetches again.
-template <int W, class OutDT, class LOGITS, class RELOAD>
+// Buckets that follow one another in a lane, the same number for every layout and type of the table, whose sums are then the same:
+// block ii of a 64-bucket chunk takes bucket mx_bucket<RUN>(n, ii) of it for column n.  Four 16-bit prototypes are fetched at
+// once, 32-bit ones one by one: four at once would leave a lane's entry of four heads, 16 bytes, 64 bytes from the next lane's.  fp32
+// table of one / eight sequences of 32 heads x 60 tables, runs of two / one: grouped 7.6, 22.3 / 6.6, 19.3 us, plain 7.0, 19.7 / 6.7,
+// 19.4 (before, heads as columns: 8.1, 23.3 and 10.1, 34.2); steps over 15617 tokens of two sequences of 64 heads, four layers, runs of four
+// 270 us, two 257, one 252 (before 264).
+constexpr int kMxRun16 = 4, kMxRun32 = 1;
+template <int RUN>
+__device__ __forceinline__ int mx_bucket(int n, int ii) {
+  return 16 * RUN * (ii / RUN) + RUN * n + ii % RUN;
+}
+
+// N neighbouring elements, aligned to all of them (to 16 bytes where they are more).
+template <int N, class OT>
+__device__ __forceinline__ void mx_store(OT* to, const float* v) {
+  if constexpr (sizeof(OT) == 4) {
+    if constexpr (N == 1) *to = v[0];
+    else if constexpr (N == 2) *reinterpret_cast<float2*>(to) = make_float2(v[0], v[1]);
+    else
+#pragma unroll
+      for (int i = 0; i < N; i += 4) *reinterpret_cast<float4*>(to + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
+  } else {
+    if constexpr (N == 1) *to = f32_to_bf16_bits(v[0]);
+    else if constexpr (N == 2) *reinterpret_cast<uint32_t*>(to) = f32x2_to_bf16_bits(v[0], v[1]);
+    else if constexpr (N == 4) *reinterpret_cast<uint2*>(to) = make_uint2(f32x2_to_bf16_bits(v[0], v[1]), f32x2_to_bf16_bits(v[2], v[3]));
+    else
+#pragma unroll
+      for (int i = 0; i < N; i += 8)
+        *reinterpret_cast<uint4*>(to + i) = make_uint4(f32x2_to_bf16_bits(v[i], v[i + 1]), f32x2_to_bf16_bits(v[i + 2], v[i + 3]),
+                                                       f32x2_to_bf16_bits(v[i + 4], v[i + 5]), f32x2_to_bf16_bits(v[i + 6], v[i + 7]));
+  }
+}
+
+// logits(c, lg): lg[ii][r] is bucket 256 wave + 64 c + mx_bucket<RUN>(n, ii) of head 4 quarter + r, in base-2 units, from
+// prototypes that reload() fetches again.
+template <int W, class OutDT, int RUN, class LOGITS, class RELOAD>
 __device__ __forceinline__ void mx_table(const LOGITS& logits, const RELOAD& reload, bool live, void* __restrict__ out, int l, int group, int n_units, int L,
                                          int wave, int lane) {
   __shared__ __attribute__((aligned(16))) float red[4][kSHWaves][kMxHeads];
@@ -272,21 +304,14 @@ __device__ __forceinline__ void mx_table(const LOGITS& logits, const RELOAD& rel
     for (int g = 0; g < 4; g += W) {      // the lane's units: heads 4 quarter + g .. + W - 1
       const int unit = group * (kMxHeads / W) + (4 * quarter + g) / W;
       if (unit >= n_units) break;
-      OT* base = (OT*)out + (((int64_t)unit * L + l) * kMxR + wave * 256 + 4 * n) * W;
+      OT* base = (OT*)out + (((int64_t)unit * L + l) * kMxR + wave * 256) * W;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        float v[4 * W];                   // four buckets of W heads: a run
+        float v[4 * W];                   // four buckets of W heads, in runs
 #pragma unroll
         for (int i = 0; i < 4 * W; ++i) v[i] = lg[c][i / W][g + i % W] * inv[g + i % W];
 #pragma unroll
-        for (int i = 0; i < 4 * W; i += 16 / (int)sizeof(OT)) {
-          OT* to = base + 64 * c * W + i;
-          if constexpr (sizeof(OT) == 4) *reinterpret_cast<float4*>(to) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
-          else if constexpr (W == 1) *reinterpret_cast<uint2*>(to) = make_uint2(f32x2_to_bf16_bits(v[0], v[1]), f32x2_to_bf16_bits(v[2], v[3]));
-          else
-            *reinterpret_cast<uint4*>(to) = make_uint4(f32x2_to_bf16_bits(v[i], v[i + 1]), f32x2_to_bf16_bits(v[i + 2], v[i + 3]),
-                                                       f32x2_to_bf16_bits(v[i + 4], v[i + 5]), f32x2_to_bf16_bits(v[i + 6], v[i + 7]));
-        }
+        for (int ii = 0; ii < 4; ii += RUN) mx_store<RUN * W>(base + (64 * c + mx_bucket<RUN>(n, ii)) * W, v + ii * W);
       }
     }
   };
@@ -355,7 +380,7 @@ __device__ __forceinline__ void soft_hash_mx_block(const int l, const int group,
     const char* at0 = (const char*)protos_T + wave * 512;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const uint32_t off = protos_at + (uint32_t)min(4 * quarter + r, kMxK - 1) * (kMxR * 2) + 8 * n;
+      const uint32_t off = protos_at + (uint32_t)min(4 * quarter + r, kMxK - 1) * (kMxR * 2) + 2 * kMxRun16 * n;
 #pragma unroll
       for (int c = 0; c < 4; ++c) pr[c][r] = *reinterpret_cast<const uint2*>(at0 + off + 128 * c);
     }
@@ -413,7 +438,7 @@ __device__ __forceinline__ void soft_hash_mx_block(const int l, const int group,
     asm volatile("" : "+v"(protos_at));       // (fetched again, not kept in registers for a case that is rare)
     load_protos();
   };
-  mx_table<W, OutDT>(logits, reload, at.live, out, l, group, units.count, L, wave, lane);
+  mx_table<W, OutDT, kMxRun16>(logits, reload, at.live, out, l, group, units.count, L, wave, lane);
 }
 
 __host__ __device__ __forceinline__ float mx_scale(float tanh_scale, float inv_temperature) {
@@ -451,7 +476,11 @@ __device__ __forceinline__ void soft_hash_mx32_block(const int l, const int grou
     for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        sh_load4<DType_f32>(protos_T, protos_at + min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c + 4 * n, pr[c][r]);
+      {
+        const float* at = protos_T + protos_at + min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c;
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) pr[c][r][ii] = at[mx_bucket<kMxRun32>(n, ii)];
+      }
   };
 #pragma unroll
   for (int i = 0; i < 8; i += 4) {
@@ -506,7 +535,7 @@ __device__ __forceinline__ void soft_hash_mx32_block(const int l, const int grou
     asm volatile("" : "+v"(protos_at));       // (fetched again, not kept in registers for a case that is rare)
     load_protos();
   };
-  mx_table<W, OutDT>(logits, reload, at.live, out, l, group, units.count, L, wave, lane);
+  mx_table<W, OutDT, kMxRun32>(logits, reload, at.live, out, l, group, units.count, L, wave, lane);
 }
 
 template <int W, class OutDT>
