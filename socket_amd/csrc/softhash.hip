@@ -114,7 +114,7 @@ __device__ __forceinline__ void sh_store4<DType_f16>(void* p, int64_t i, const f
 // What bounds it are vector instructions, about 600 a wave at 64 logits a lane, and at few heads dependent trips to memory.
 // Before (head as the N index of both products: entries put together by lane exchanges; every wave rotated and projected
 // everything; maxima exchanged and taken off) and now, the decode prologue with the rest of its roles: one sequence of 32 heads x
-// 60 tables 7.7 / 6.2 us, four 13.4 / 10.5, sixteen of 28 x 48 27.2 / 20.4.  (The scalar form below spends ten multiply-adds
+// 60 tables 7.7 / 5.4 us, four 13.4 / 9.4, sixteen of 28 x 48 27.2 / 18.1.  (The scalar form below spends ten multiply-adds
 // and a library exponential per head and bucket: 10.4, 23 and 56 us.)
 //
 // W: heads of a unit (the scorer's grouped layout [unit, L, R, W]; 1 for the reference's [B,Hq,L,R], whose
@@ -216,12 +216,13 @@ __device__ __forceinline__ sh_f32x4 mx_angles(const sh_f32x4& part, float scale,
 }
 
 // Buckets that follow one another in a lane, the same number for every layout and type of the table, whose sums are then the same:
-// block ii of a 64-bucket chunk takes bucket mx_bucket<RUN>(n, ii) of it for column n.  Four 16-bit prototypes are fetched at
-// once, 32-bit ones one by one: four at once would leave a lane's entry of four heads, 16 bytes, 64 bytes from the next lane's.  fp32
-// table of one / eight sequences of 32 heads x 60 tables, runs of two / one: grouped 7.6, 22.3 / 6.6, 19.3 us, plain 7.0, 19.7 / 6.7,
-// 19.4 (before, heads as columns: 8.1, 23.3 and 10.1, 34.2); steps over 15617 tokens of two sequences of 64 heads, four layers, runs of four
-// 270 us, two 257, one 252 (before 264).
-constexpr int kMxRun16 = 4, kMxRun32 = 1;
+// block ii of a 64-bucket chunk takes bucket mx_bucket<RUN>(n, ii) of it for column n.  Two 16-bit
+// prototypes are fetched at once and 32-bit ones one by one, so that a lane's entries of four heads are 16 bytes in a row and its
+// quarter's 256: more at once would leave them further apart.  Decode prologue in bf16, runs of four / two: one sequence of 32 heads x 60
+// tables 6.0 / 5.4 us, four 10.7 / 9.4, sixteen of 28 x 48 20.9 / 18.1.  fp32 table of one / eight sequences of 32 heads x 60 by itself,
+// runs of two / one: grouped 7.6, 22.3 / 6.6, 19.3 us, plain 7.0, 19.7 / 6.7, 19.4 (before, heads as columns: 8.1, 23.3 and 10.1, 34.2);
+// steps over 15617 tokens of two sequences of 64 heads, four layers, runs of four 270 us, two 257, one 252 (before 264).
+constexpr int kMxRun16 = 2, kMxRun32 = 1;
 template <int RUN>
 __device__ __forceinline__ int mx_bucket(int n, int ii) {
   return 16 * RUN * (ii / RUN) + RUN * n + ii % RUN;
@@ -382,7 +383,8 @@ __device__ __forceinline__ void soft_hash_mx_block(const int l, const int group,
     for (int r = 0; r < 4; ++r) {
       const uint32_t off = protos_at + (uint32_t)min(4 * quarter + r, kMxK - 1) * (kMxR * 2) + 2 * kMxRun16 * n;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) pr[c][r] = *reinterpret_cast<const uint2*>(at0 + off + 128 * c);
+      for (int c = 0; c < 4; ++c)
+        pr[c][r] = make_uint2(*reinterpret_cast<const uint32_t*>(at0 + off + 128 * c), *reinterpret_cast<const uint32_t*>(at0 + off + 128 * c + 64));
     }
     if (quarter >= 2) {         // (no prototype past the tenth: zeros, whatever the tenth is)
 #pragma unroll
@@ -1044,7 +1046,7 @@ __device__ __forceinline__ uint4 sh_bf16_of8(const sh_row8<DT>& r) {
 // GC: as in soft_hash_block (bf16 only), or 0: soft_hash_mx_block or soft_hash_mx32_block with units of W heads, OT the
 // output's elements; below zero: soft_hash_small_block for at most -GC planes.
 // (bf16 operands on the matrix cores: four waves a SIMD, whose registers the usual path fits; what the rare one spills is its own.  At
-// the three that 164 registers leave, sixteen sequences of 28 heads x 48 tables take 23.4 us instead of 20.4, four of 32 x 60 11.0
+// the three that 164 registers leave (and runs of four buckets to a lane), sixteen sequences of 28 heads x 48 tables take 23.4 us instead of 20.4, four of 32 x 60 11.0
 // instead of 10.5.)
 template <class DT, int GC, class FT, int W, class OT>
 __global__ __launch_bounds__(kSHThreads, GC == 0 && DT::kEnum == SOCKET_BF16 ? 4 : 1) void decode_prologue_kernel(
