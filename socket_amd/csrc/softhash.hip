@@ -249,112 +249,99 @@ __device__ __forceinline__ void mx_store(OT* to, const float* v) {
   }
 }
 
-// logits(c, lg): lg[ii][r] is bucket 256 wave + 64 c + mx_bucket<RUN>(n, ii) of head 4 quarter + r, in base-2 units, from
-// prototypes that reload() fetches again.
-template <int W, class OutDT, int RUN, class LOGITS, class RELOAD>
-__device__ __forceinline__ void mx_table(const LOGITS& logits, const RELOAD& reload, bool live, void* __restrict__ out, int l, int group, int n_units, int L,
+// logits(c, lg): lg[ii][r] is bucket 256 wave + 64 c + mx_bucket<RUN>(n, ii) of head 4 quarter + r, in base-2 units.
+// A wave in which some logit is past kMxPlain takes the largest of its own off, in the heads that have one, and rounded to a
+// whole number, so that putting the waves' sums together multiplies by powers of two.  Logits of +-1 prototypes at a
+// temperature of 0.02, bf16, us with the maximum over all waves taken off everywhere / worked out again where a logit is large /
+// now: one sequence of 32 heads x 60 tables 6.3 / 16.0 / 6.0, four 9.7 / 27.9 / 9.2, sixteen of 28 x 48 19.3 / 66.7 / 17.0 (small logits:
+// 4.8, 7.7, 14.2).
+template <int W, class OutDT, int RUN, class LOGITS>
+__device__ __forceinline__ void mx_table(const LOGITS& logits, bool live, void* __restrict__ out, int l, int group, int n_units, int L,
                                          int wave, int lane) {
-  __shared__ __attribute__((aligned(16))) float red[4][kSHWaves][kMxHeads];
+  __shared__ __attribute__((aligned(16))) float sums[kSHWaves][kMxHeads], offs[kSHWaves][kMxHeads];
   __shared__ __attribute__((aligned(16))) float alive[kMxHeads];
   __shared__ int wide[kSHWaves];
   const int n = lane & 15, quarter = lane >> 4;
   sh_f32x4 lg[4][4];
-  auto total = [&](int k) {      // of a head, over the table: the sums (or the maxima) of the four waves
-    sh_f32x4 w[kSHWaves];
-#pragma unroll
-    for (int i = 0; i < kSHWaves; ++i) w[i] = *reinterpret_cast<const sh_f32x4*>(&red[k][i][4 * quarter]);
-    if (k % 2 == 0) return (w[0] + w[1]) + (w[2] + w[3]);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) w[0][r] = fmaxf(fmaxf(w[0][r], w[1][r]), fmaxf(w[2][r], w[3][r]));
-    return w[0];
-  };
   float top = 0.f;
-  sh_f32x4 sum = sh_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int c = 0; c < 4; ++c) logits(c, lg[c]);
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
+    logits(c, lg[c]);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) top = fmaxf(top, fabsf(lg[c][i][r]));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) lg[c][i][r] = __builtin_amdgcn_exp2f(lg[c][i][r]);
-      sum += lg[c][i];
-    }
   }
   const bool far = __builtin_amdgcn_ballot_w64(top > kMxPlain) != 0;
-  auto sum_up = [&](int k) {
+  if (__builtin_expect(far, 0)) {
+    sh_f32x4 off;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sum[r] = mx_row<false>(sum[r]);
-    if (n == 0) *reinterpret_cast<sh_f32x4*>(&red[k][wave][4 * quarter]) = sum;
-  };
-  sum_up(0);
-  if (quarter == 0) alive[n] = live ? 1.f : 0.f;
-  if (lane == 0) wide[wave] = far ? 1 : 0;
-  __syncthreads();
-  auto write = [&](const sh_f32x4& sum) __attribute__((always_inline)) {
-    const sh_f32x4 real = *reinterpret_cast<const sh_f32x4*>(&alive[4 * quarter]);
-    sh_f32x4 inv;
+    for (int r = 0; r < 4; ++r) {
+      float mx = -INFINITY, size = 0.f;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) inv[r] = real[r] != 0.f ? 1.f / sum[r] : 0.f;      // (heads that only fill a unit up are zero)
-    typedef typename OutDT::storage OT;
-#pragma unroll
-    for (int g = 0; g < 4; g += W) {      // the lane's units: heads 4 quarter + g .. + W - 1
-      const int unit = group * (kMxHeads / W) + (4 * quarter + g) / W;
-      if (unit >= n_units) break;
-      OT* base = (OT*)out + (((int64_t)unit * L + l) * kMxR + wave * 256) * W;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        float v[4 * W];                   // four buckets of W heads, in runs
-#pragma unroll
-        for (int i = 0; i < 4 * W; ++i) v[i] = lg[c][i / W][g + i % W] * inv[g + i % W];
-#pragma unroll
-        for (int ii = 0; ii < 4; ii += RUN) mx_store<RUN * W>(base + (64 * c + mx_bucket<RUN>(n, ii)) * W, v + ii * W);
+      for (int i = 0; i < 16; ++i) {
+        mx = fmaxf(mx, lg[i >> 2][i & 3][r]);
+        size = fmaxf(size, fabsf(lg[i >> 2][i & 3][r]));
       }
+      off[r] = mx_row<true>(size) > kMxPlain ? rintf(mx_row<true>(mx)) : 0.f;      // (0: what the head has when it is with others)
+      const float taken = off[r] == -INFINITY ? 0.f : off[r];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) lg[i >> 2][i & 3][r] -= taken;
     }
-  };
-  if (__builtin_expect(__builtin_amdgcn_readfirstlane(wide[0] | wide[1] | wide[2] | wide[3]) == 0, 1)) {
-    write(total(0));
-    return;
+    if (n == 0) *reinterpret_cast<sh_f32x4*>(&offs[wave][4 * quarter]) = off;
   }
-  // a large logit somewhere (the same answer in all waves): from the start, with the largest taken off in the heads that have one
-  reload();
-#pragma unroll
-  for (int c = 0; c < 4; ++c) logits(c, lg[c]);
-  sh_f32x4 mx = lg[0][0], size = sh_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      mx[r] = fmaxf(mx[r], lg[i >> 2][i & 3][r]);
-      size[r] = fmaxf(size[r], fabsf(lg[i >> 2][i & 3][r]));
-    }
-    mx[r] = mx_row<true>(mx[r]);
-    size[r] = mx_row<true>(size[r]);
-  }
-  if (n == 0) {
-    *reinterpret_cast<sh_f32x4*>(&red[1][wave][4 * quarter]) = mx;
-    *reinterpret_cast<sh_f32x4*>(&red[3][wave][4 * quarter]) = size;
-  }
-  __syncthreads();
-  mx = total(1);
-  size = total(3);
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-    if (!(size[r] > kMxPlain)) mx[r] = 0.f;       // (what the head has when it is with others)
-  sum = sh_f32x4{0.f, 0.f, 0.f, 0.f};
+  sh_f32x4 sum = sh_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) lg[i >> 2][i & 3][r] = __builtin_amdgcn_exp2f(lg[i >> 2][i & 3][r] - mx[r]);
+    for (int r = 0; r < 4; ++r) lg[i >> 2][i & 3][r] = __builtin_amdgcn_exp2f(lg[i >> 2][i & 3][r]);
     sum += lg[i >> 2][i & 3];
   }
-  sum_up(2);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) sum[r] = mx_row<false>(sum[r]);
+  if (n == 0) *reinterpret_cast<sh_f32x4*>(&sums[wave][4 * quarter]) = sum;
+  if (quarter == 0) alive[n] = live ? 1.f : 0.f;
+  if (lane == 0) wide[wave] = far ? 1 : 0;
   __syncthreads();
-  write(total(2));
+  sh_f32x4 part[kSHWaves], scale = sh_f32x4{1.f, 1.f, 1.f, 1.f};      // the waves' sums; this wave's entries times that
+#pragma unroll
+  for (int i = 0; i < kSHWaves; ++i) part[i] = *reinterpret_cast<const sh_f32x4*>(&sums[i][4 * quarter]);
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane(wide[0] | wide[1] | wide[2] | wide[3]) != 0, 0)) {
+    sh_f32x4 off[kSHWaves];
+#pragma unroll
+    for (int i = 0; i < kSHWaves; ++i)
+      off[i] = wide[i] ? *reinterpret_cast<const sh_f32x4*>(&offs[i][4 * quarter]) : sh_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float most = fmaxf(fmaxf(off[0][r], off[1][r]), fmaxf(off[2][r], off[3][r]));
+#pragma unroll
+      for (int i = 0; i < kSHWaves; ++i) {
+        const float f = ldexpf(1.f, (int)fmaxf(off[i][r] - most, -200.f));      // (0 from -150 down, and where all are infinite)
+        part[i][r] *= f;
+        scale[r] = wave == i ? f : scale[r];
+      }
+    }
+  }
+  sum = (part[0] + part[1]) + (part[2] + part[3]);
+  const sh_f32x4 real = *reinterpret_cast<const sh_f32x4*>(&alive[4 * quarter]);
+  sh_f32x4 inv;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) inv[r] = real[r] != 0.f ? scale[r] / sum[r] : 0.f;      // (heads that only fill a unit up are zero)
+  typedef typename OutDT::storage OT;
+#pragma unroll
+  for (int g = 0; g < 4; g += W) {      // the lane's units: heads 4 quarter + g .. + W - 1
+    const int unit = group * (kMxHeads / W) + (4 * quarter + g) / W;
+    if (unit >= n_units) break;
+    OT* base = (OT*)out + (((int64_t)unit * L + l) * kMxR + wave * 256) * W;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      float v[4 * W];                   // four buckets of W heads, in runs
+#pragma unroll
+      for (int i = 0; i < 4 * W; ++i) v[i] = lg[c][i / W][g + i % W] * inv[g + i % W];
+#pragma unroll
+      for (int ii = 0; ii < 4; ii += RUN) mx_store<RUN * W>(base + (64 * c + mx_bucket<RUN>(n, ii)) * W, v + ii * W);
+    }
+  }
 }
 
 template <class FT, int W, class OutDT>
@@ -375,26 +362,22 @@ __device__ __forceinline__ void soft_hash_mx_block(const int l, const int group,
   uint4 qf = *reinterpret_cast<const uint4*>(q + at.b * q_sb + at.head * q_sh + d0);
   const uint4 pl = *reinterpret_cast<const uint4*>(planes + ((int64_t)l * kMxK + min(n, kMxK - 1)) * kMxD + d0);
   uint2 pr[4][4];
-  uint32_t protos_at = 0;
-  auto load_protos = [&]() __attribute__((always_inline)) {
-    // (byte offsets of 32 bits beside a common address)
-    const char* at0 = (const char*)protos_T + wave * 512;
+  // (byte offsets of 32 bits beside a common address)
+  const char* at0 = (const char*)protos_T + wave * 512;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const uint32_t off = protos_at + (uint32_t)min(4 * quarter + r, kMxK - 1) * (kMxR * 2) + 2 * kMxRun16 * n;
+  for (int r = 0; r < 4; ++r) {
+    const uint32_t off = (uint32_t)min(4 * quarter + r, kMxK - 1) * (kMxR * 2) + 2 * kMxRun16 * n;
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
-        pr[c][r] = make_uint2(*reinterpret_cast<const uint32_t*>(at0 + off + 128 * c), *reinterpret_cast<const uint32_t*>(at0 + off + 128 * c + 64));
-    }
-    if (quarter >= 2) {         // (no prototype past the tenth: zeros, whatever the tenth is)
+    for (int c = 0; c < 4; ++c)
+      pr[c][r] = make_uint2(*reinterpret_cast<const uint32_t*>(at0 + off + 128 * c), *reinterpret_cast<const uint32_t*>(at0 + off + 128 * c + 64));
+  }
+  if (quarter >= 2) {         // (no prototype past the tenth: zeros, whatever the tenth is)
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (4 * quarter + r >= kMxK) pr[c][r] = make_uint2(0, 0);
-    }
-  };
-  load_protos();
+      for (int r = 0; r < 4; ++r)
+        if (4 * quarter + r >= kMxK) pr[c][r] = make_uint2(0, 0);
+  }
   if constexpr (kRope) {
     const bool turn = p >= 0 && p < n_pos;
     // (angles of row 0 for a position outside the table: a load under a condition is waited for at once)
@@ -436,11 +419,7 @@ __device__ __forceinline__ void soft_hash_mx_block(const int l, const int group,
       lg[ii] = sh_mfma(t_high, make_uint4(a0, a1, a0, a1), lg[ii]);
     }
   };
-  auto reload = [&]() __attribute__((always_inline)) {
-    asm volatile("" : "+v"(protos_at));       // (fetched again, not kept in registers for a case that is rare)
-    load_protos();
-  };
-  mx_table<W, OutDT, kMxRun16>(logits, reload, at.live, out, l, group, units.count, L, wave, lane);
+  mx_table<W, OutDT, kMxRun16>(logits, at.live, out, l, group, units.count, L, wave, lane);
 }
 
 __host__ __device__ __forceinline__ float mx_scale(float tanh_scale, float inv_temperature) {
@@ -472,18 +451,6 @@ __device__ __forceinline__ void soft_hash_mx32_block(const int l, const int grou
   int64_t p = 0;
   if constexpr (kRope) p = pos[(int64_t)at.b * pos_stride];
   float x[8], pl[8], pr[4][4][4];
-  uint32_t protos_at = 0;
-  auto load_protos = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-      {
-        const float* at = protos_T + protos_at + min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c;
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii) pr[c][r][ii] = at[mx_bucket<kMxRun32>(n, ii)];
-      }
-  };
 #pragma unroll
   for (int i = 0; i < 8; i += 4) {
     float t[4];
@@ -494,7 +461,14 @@ __device__ __forceinline__ void soft_hash_mx32_block(const int l, const int grou
 #pragma unroll
     for (int e = 0; e < 4; ++e) pl[i + e] = t[e];
   }
-  load_protos();
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float* from = protos_T + min(4 * quarter + r, kMxK - 1) * kMxR + wave * 256 + 64 * c;
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) pr[c][r][ii] = from[mx_bucket<kMxRun32>(n, ii)];
+    }
   if constexpr (kRope) {
     const bool turn = p >= 0 && p < n_pos;
     // (angles of row 0 for a position outside the table: a load under a condition is waited for at once)
@@ -533,11 +507,7 @@ __device__ __forceinline__ void soft_hash_mx32_block(const int l, const int grou
         // (no prototype past the tenth: zeros, whatever the tenth is)
         lg[ii] = __builtin_amdgcn_mfma_f32_16x16x4f32(t[r], 4 * quarter + r < kMxK ? pr[c][r][ii] : 0.f, lg[ii], 0, 0, 0);
   };
-  auto reload = [&]() __attribute__((always_inline)) {
-    asm volatile("" : "+v"(protos_at));       // (fetched again, not kept in registers for a case that is rare)
-    load_protos();
-  };
-  mx_table<W, OutDT, kMxRun32>(logits, reload, at.live, out, l, group, units.count, L, wave, lane);
+  mx_table<W, OutDT, kMxRun32>(logits, at.live, out, l, group, units.count, L, wave, lane);
 }
 
 template <int W, class OutDT>
@@ -1045,9 +1015,8 @@ __device__ __forceinline__ uint4 sh_bf16_of8(const sh_row8<DT>& r) {
 // DT: type of the projection, the caches, planes and prototypes.
 // GC: as in soft_hash_block (bf16 only), or 0: soft_hash_mx_block or soft_hash_mx32_block with units of W heads, OT the
 // output's elements; below zero: soft_hash_small_block for at most -GC planes.
-// (bf16 operands on the matrix cores: four waves a SIMD, whose registers the usual path fits; what the rare one spills is its own.  At
-// the three that 164 registers leave (and runs of four buckets to a lane), sixteen sequences of 28 heads x 48 tables take 23.4 us instead of 20.4, four of 32 x 60 11.0
-// instead of 10.5.)
+// (bf16 operands on the matrix cores: four waves a SIMD.  At the three that 164 registers leave (and runs of four buckets to a
+// lane), sixteen sequences of 28 heads x 48 tables took 23.4 us instead of 20.4, four of 32 x 60 11.0 instead of 10.5.)
 template <class DT, int GC, class FT, int W, class OT>
 __global__ __launch_bounds__(kSHThreads, GC == 0 && DT::kEnum == SOCKET_BF16 ? 4 : 1) void decode_prologue_kernel(
     const typename DT::storage* __restrict__ qkv, int64_t qkv_sb, const void* __restrict__ freqs,

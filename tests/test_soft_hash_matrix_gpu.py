@@ -104,3 +104,73 @@ def test_float32_tables_of_every_layout(Hq, Hkv, B):
         assert torch.equal(got[:, kv * parts + g // width, :, :, g % width], flat[:, h])
     for g in range(G, parts * width):
         assert (got.view(B, Hkv, parts, 5, 1024, width)[:, :, g // width, :, :, g % width] == 0).all()
+
+
+def single(B, Hq, L, seed, positive=False):
+    """Planes of one coordinate each, which fp32 projects without an error: t is tanh's alone."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    q = torch.randn(B, Hq, 128, generator=g, device=DEV).bfloat16()
+    planes = torch.zeros(L, 10, 128, device=DEV)
+    planes.view(-1, 128)[torch.arange(10 * L, device=DEV), torch.arange(10 * L, device=DEV) * 37 % 128] = 1.0
+    return (q.abs() if positive else q), planes.bfloat16()
+
+
+def assert_close(got, want, largest):
+    """(Logits up to `largest` in base 2: sixteen roundings of that size, and an exponential and a normalisation to an ulp or two.)"""
+    assert ((got.double() - want).abs() <= 2 ** -23 * (16 + 17 * largest) * want + 1e-37).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("sizes", [(64, 1, 1, 1), (1, 1, 1, 64), (0.01, 64, 1, 16), (4096, 4096, 4096, 4096), (1, 4096, 64, 0.01), (8, 7, 6, 5)])
+def test_large_logits_in_some_buckets(dtype, sizes):
+    """The four waves' buckets of different sizes: each takes its own largest logit off, or none."""
+    q, planes = single(3, 8, 3, 5)
+    r, k = torch.arange(1024, device=DEV)[None], torch.arange(10, device=DEV)[:, None]
+    protos = (((r >> (9 - k)) & 1) * 2.0 - 1) * torch.tensor(sizes, device=DEV, dtype=torch.float32).repeat_interleave(256)
+    protos = protos.to(dtype)
+    q[0] *= 0.01                                # (heads of small logits beside them)
+    got = hash_cache.soft_hash(q.to(dtype), planes.to(dtype), protos, 0.3, 4, out_dtype=torch.float32)
+    t = torch.tanh(torch.einsum("bhd,lkd->bhlk", q.double(), planes.double())) / math.sqrt(128)
+    logits = torch.einsum("bhlk,kr->bhlr", t, protos.double()) / 0.3 / math.log(2)
+    assert_close(got, torch.softmax(logits * math.log(2), -1), logits.abs().amax().item())
+    half = hash_cache.soft_hash(q.to(dtype), planes.to(dtype), protos, 0.3, 4, out_dtype=torch.bfloat16)
+    # (bfloat16 has eight significant bits: a rounding is off by up to 2^-8 of its result)
+    assert ((half.float() - got).abs() <= 2 ** -8 * got + 1e-37).all()
+
+
+def test_buckets_that_are_out_of_reach():
+    """Logits of minus infinity have no weight, also where they are all of a wave's and the other waves' are far below zero."""
+    q, planes = single(2, 4, 2, 6, positive=True)
+    protos = torch.full((10, 1024), -100.0, device=DEV) - torch.rand(10, 1024, generator=torch.Generator(device=DEV).manual_seed(1), device=DEV)
+    for out in (slice(5, 6), slice(256, 512), slice(0, 900)):
+        p = protos.clone()
+        p[:, out] = -math.inf
+        got = hash_cache.soft_hash(q.float(), planes.float(), p, 0.3, 4)
+        finite = torch.ones(1024, dtype=torch.bool, device=DEV)
+        finite[out] = False
+        assert (got[..., out] == 0).all()
+        assert_close(got[..., finite], exact(q, planes, protos[:, finite], 0.3), 10 * 101 / math.sqrt(128) / 0.3 / math.log(2))
+    assert hash_cache.soft_hash(q.float(), planes.float(), torch.full_like(protos, -math.inf), 0.3, 4).isnan().all()
+
+
+def test_large_logits_take_no_second_pass():
+    """Small and large logits are worked out once each: the launch takes about as long (made twice, 3.3 to 4.7 times as long)."""
+    q, planes, protos = inputs(16, 28, 48, 1, True)
+
+    def best(temperature):
+        hash_cache.soft_hash(q, planes, protos, temperature, 4)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(10):
+                hash_cache.soft_hash(q, planes, protos, temperature, 4)
+        times = []
+        for _ in range(12):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            graph.replay()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    assert best(0.01) < 2 * best(0.3)
