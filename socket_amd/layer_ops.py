@@ -136,6 +136,11 @@ def linear_f32(x: Tensor, weight: Tensor) -> Tensor:
     return torch.mm(x.reshape(rows, K), weight.t(), out_dtype=torch.float32).view(*x.shape[:-1], N)
 
 
+# What the matrix-vector kernel has of a CU's 160 KB for the rows that it norms itself, four bytes an element for the one in work
+# and two for each that is done.
+_NORMED_ROWS_LDS = 160 * 1024 - 256
+
+
 @torch.no_grad()
 def norm_linear(x: Optional[Tensor], pending: Optional[Pending], pre_w: Tensor, eps: float, weight: Tensor, *,
                 embed: Optional[Tensor] = None, ids: Optional[Tensor] = None, f32_out: bool = False,
@@ -156,11 +161,15 @@ def norm_linear(x: Optional[Tensor], pending: Optional[Pending], pre_w: Tensor, 
             return x_out, gated_unit(torch.cat([F.linear(h, weight, bias), F.linear(h, up_weight, up_bias)], dim=-1), act, limit)
         assert bias is None or not f32_out
         return x_out, linear_f32(h, weight) if f32_out else F.linear(h, weight, bias)
-    x_out = _stream_out(x, pending, lead, K, weight.device, x_out)
-    r = _residual(x, embed, ids, pending, pre_w, eps, dtype, None if x_out is x else x_out, None, embed_scale)
     y = torch.empty(*lead, N, dtype=torch.float32 if f32_out else dtype, device=weight.device)
-    a = RowsLinear(norm=ctypes.pointer(r), w1=weight.data_ptr(), s1=1.0, K1=K, y=y.data_ptr(), y_f32=int(f32_out),
-                   M=rows, N=N)
+    a = RowsLinear(w1=weight.data_ptr(), s1=1.0, K1=K, y=y.data_ptr(), y_f32=int(f32_out), M=rows, N=N)
+    if K * (4 + 2 * rows) <= _NORMED_ROWS_LDS:
+        x_out = _stream_out(x, pending, lead, K, weight.device, x_out)
+        r = _residual(x, embed, ids, pending, pre_w, eps, dtype, None if x_out is x else x_out, None, embed_scale)
+        a.norm = ctypes.pointer(r)
+    else:      # (the norm a launch of its own: the same rows, the same product)
+        x_out, h = residual_norm(x, pending, pre_w, eps, dtype, embed=embed, ids=ids, embed_scale=embed_scale, x_out=x_out)
+        a.x1 = h.data_ptr()
     if up_weight is not None:
         assert up_weight.shape == weight.shape and up_weight.is_contiguous() and up_weight.dtype == dtype
         a.w2, a.kind, a.limit = up_weight.data_ptr(), GATED_UNITS[act], limit
