@@ -142,7 +142,6 @@ constexpr int kVec = 8;                    // weights per lane and load
 constexpr int kDepth = 4;                  // loads of a chunk of a row
 constexpr int kChunkElems = 64 * kVec * kDepth;
 constexpr int kWgPerCu = 4;                // workgroups per CU of a persistent launch
-constexpr int most_slots(int two) { return two == 1 ? 2 : 4; }      // chunks of a wave in flight: 16 KB
 constexpr int kInputVecs = 8;              // 16-byte vectors of a lane that wait in registers on their way to LDS
 
 __host__ __device__ __forceinline__ int chunks_of(int K) { return (K + kChunkElems - 1) / kChunkElems; }
@@ -152,12 +151,15 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // Where the input rows come from.
 enum RowsInput {
-  kFromMemory,      // x1 (and x2), read from memory as they are used: rows that do not fit into LDS
+  kFromMemory,      // x1 (and x2), requested with the weights that they meet: rows that do not fit into LDS
   kFromLds,         // x1 (and x2), brought into LDS
   kNormRows,        // residual_row's, one row after the other, behind the first weights
   kNormEarly2,      // residual_row's for one row of up to 2 float4 vectors a lane, its operands requested ahead of the weights
   kNormEarly4,      // the same, up to 4
 };
+
+// Chunks of a wave in flight: 16 KB of weights, or two chunks and the inputs' beside them.
+constexpr int most_slots(RowsInput in, int two) { return in == kFromMemory || two == 1 ? 2 : 4; }
 
 // A row of weights as a buffer: loads past its end give zeros and ask the memory for nothing, so that whether there is a
 // row at all is no branch (behind one, the compiler's wait for a chunk would be a wait for everything in flight).
@@ -168,11 +170,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(const uint16_t* w, 
 constexpr int kStreaming = 2;              // cache policy of a buffer load: nt
 
 // Chunk kc of a row, kDepth vectors a lane.
+template <int POLICY = kStreaming>
 __device__ __forceinline__ void fetch_chunk(rl_u32x4 (&v)[kDepth], __amdgpu_buffer_rsrc_t row, int kc, int lane) {
   const int at = kc * (kChunkElems * 2) + lane * 16;
 #pragma unroll
   for (int u = 0; u < kDepth; ++u)
-    v[u] = __builtin_bit_cast(rl_u32x4, __builtin_amdgcn_raw_buffer_load_b128(row, at + u * 1024, 0, kStreaming));
+    v[u] = __builtin_bit_cast(rl_u32x4, __builtin_amdgcn_raw_buffer_load_b128(row, at + u * 1024, 0, POLICY));
 }
 
 // acc + the two products of bf16 pairs (an element of a vector has to be a value of its own here: a bit cast of the element
@@ -181,7 +184,7 @@ __device__ __forceinline__ float dot2(uint32_t w, uint32_t x, float acc) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), __builtin_bit_cast(bf16x2, x), acc, false);
 }
 
-// A chunk of a row with the M input rows.  Lanes past the rows' end have zero weights; ZEROS: and find zeros in place of the
+// A chunk of a row with the M input rows in LDS.  Lanes past the rows' end have zero weights; ZEROS: and find zeros in place of the
 // input, else take them, for what they would read might be an infinity.
 template <int M, bool ZEROS>
 __device__ __forceinline__ void mul_chunk(float (&acc)[M], const rl_u32x4 (&v)[kDepth], const uint16_t* x, int64_t xs, int K,
@@ -201,6 +204,17 @@ __device__ __forceinline__ void mul_chunk(float (&acc)[M], const rl_u32x4 (&v)[k
   };
   if (ZEROS || (kc + 1) * kChunkElems <= K) mul(std::true_type{});
   else mul(std::false_type{});
+}
+
+// The same with the input's chunk in registers, zeros where there is none.
+template <int M>
+__device__ __forceinline__ void mul_chunk(float (&acc)[M], const rl_u32x4 (&v)[kDepth], const rl_u32x4 (&x)[M][kDepth]) {
+#pragma unroll
+  for (int u = 0; u < kDepth; ++u)
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[m] = dot2(v[u][i], x[m][u][i], acc[m]);
 }
 
 // Zeros behind a row of K elements in LDS, up to the end of its last chunk.
@@ -332,12 +346,15 @@ struct EarlyNorm {
 //   norm, 32000 x 2048                23.4 / 22.0 (20.2)      norm, 3392 x 2048   5.8 / 5.1
 //   sum and average, 2048 x 8192       8.45 / 7.75 (6.2)      2048 x 2048         3.46 / 3.27 (2.8)
 //   norm, gated 2 x 14336 x 4096      40.7 / 38.3             4096 x 14336       21.9 / 19.9
+// Inputs that LDS does not hold ride with the weights (read from memory as before / as they are used, between requests for weights / now):
+//   4 rows: 1000 x 20480   17.0 / 25.0 / 12.6     5120 x 20480   62.6 / 78.5 / 55.8     1000 x 98304   75 / 208 / 58
+//           two terms of 14336: 1000 rows of each 22.0 / 34.5 / 18.9, 14336 231 / 224 / 221;  3 rows, 1000: 19.9 / 29.2 / 17.0
 template <int M, RowsInput IN, int TWO, bool RES, int SLOTS>
 __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_linear a, socket_residual nrm) {
   extern __shared__ __attribute__((aligned(16))) float rl_lds[];
   __shared__ float red[2][4];
   constexpr bool EARLY = IN == kNormEarly2 || IN == kNormEarly4;
-  constexpr bool ZEROS = M == 1 && (EARLY || IN == kFromLds);
+  constexpr bool ZEROS = M == 1 && (EARLY || IN == kFromLds), MEM = IN == kFromMemory;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int waves = gridDim.x * (kRowThreads / 64);
   int n = blockIdx.x * (kRowThreads / 64) + wave;   // (wave-uniform)
@@ -375,7 +392,7 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
   }
 
   // ---- the first weights' ----
-  rl_u32x4 wv[SLOTS][kDepth], gv[TWO == 1 ? SLOTS : 1][kDepth];
+  rl_u32x4 wv[SLOTS][kDepth], gv[TWO == 1 ? SLOTS : 1][kDepth], xv[MEM ? SLOTS : 1][M][kDepth];
   uint16_t bias1[SLOTS], bias2[TWO == 1 ? SLOTS : 1];
   const __amdgpu_buffer_rsrc_t b1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.b1), 0, a.b1 ? a.N * 2 : 0, 0x00027000);
   const __amdgpu_buffer_rsrc_t b2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.b2), 0, a.b2 ? a.N * 2 : 0, 0x00027000);
@@ -384,7 +401,11 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
     constexpr int i = decltype(slot)::value;
     const bool there = fn < a.N;
     const bool second = TWO == 2 && fkc >= nk1;
-    fetch_chunk(wv[i], row_buffer(second ? w2 : w1, fn, second ? K2 : K1, there), second ? fkc - nk1 : fkc, lane);
+    const int K = second ? K2 : K1, at = second ? fkc - nk1 : fkc;
+    if constexpr (MEM)
+#pragma unroll
+      for (int m = 0; m < M; ++m) fetch_chunk<0>(xv[i][m], row_buffer(second ? x2 : x1, m, K, there), at, lane);
+    fetch_chunk(wv[i], row_buffer(second ? w2 : w1, fn, K, there), at, lane);
     bias1[i] = __builtin_amdgcn_raw_buffer_load_b16(b1, there ? fn * 2 : 0, 0, 0);
     if constexpr (TWO == 1) {
       fetch_chunk(gv[i], row_buffer(w2, fn, K1, there), fkc, lane);
@@ -439,7 +460,11 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
   auto step = [&](auto slot, auto refill) __attribute__((always_inline)) {
     constexpr int i = decltype(slot)::value;
     const bool row_ends = kc + 1 == nk;
-    if (n < a.N) {
+    if constexpr (MEM) {
+      if (TWO == 2 && kc >= nk1) mul_chunk<M>(acc2, wv[i], xv[i]);
+      else mul_chunk<M>(acc, wv[i], xv[i]);
+      if constexpr (TWO == 1) mul_chunk<M>(acc2, gv[i], xv[i]);
+    } else if (n < a.N) {
       if (TWO == 2 && kc >= nk1) mul_chunk<M, ZEROS>(acc2, wv[i], x2, K2, K2, kc - nk1, lane);
       else mul_chunk<M, ZEROS>(acc, wv[i], x1, K1, K1, kc, lane);
       if constexpr (TWO == 1) mul_chunk<M, ZEROS>(acc2, gv[i], x1, K1, K1, kc, lane);
@@ -479,7 +504,7 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
     kc = row_ends ? 0 : kc + 1;
   };
   // (all slots in every turn: to leave in the middle of one would make the waits of the next for everything, too)
-  if constexpr (SLOTS == most_slots(TWO))
+  if constexpr (SLOTS == most_slots(IN, TWO))
     while (fn < a.N) static_for<SLOTS>([&](auto slot) __attribute__((always_inline)) { step(slot, std::true_type{}); });
   static_for<SLOTS>([&](auto slot) __attribute__((always_inline)) { step(slot, std::false_type{}); });
 }
@@ -508,7 +533,7 @@ int dispatch_slots(const socket_rows_linear& a, size_t lds, hipStream_t s) {
     if (chunks == 1) return launch_rows_linear<M, IN, TWO, RES, 1>(a, n_wg, lds, s);
     if (chunks == 2) return launch_rows_linear<M, IN, TWO, RES, 2>(a, n_wg, lds, s);
   }
-  return launch_rows_linear<M, IN, TWO, RES, most_slots(TWO)>(a, n_wg, lds, s);
+  return launch_rows_linear<M, IN, TWO, RES, most_slots(IN, TWO)>(a, n_wg, lds, s);
 }
 
 template <int M, RowsInput IN, int TWO>

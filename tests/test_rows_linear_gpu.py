@@ -80,7 +80,7 @@ def test_products_of_every_form(dev, rows, K, N):
     assert _rms(got_x, e) < 1e-6 and _rms(y, h @ w.double().t(), _spread(h, w)) < normed
 
 
-@pytest.mark.parametrize("K", [40, 2056])
+@pytest.mark.parametrize("K", [40, 2056, 41000])      # (the last past what LDS holds of two rows)
 def test_an_infinity_stays_in_its_row(dev, K):
     """Lanes past a row's end multiply zeros, not what lies behind the row."""
     from socket_amd import layer_ops
