@@ -140,11 +140,12 @@ __global__ __launch_bounds__(256) void gated_unit_kernel(const void* __restrict_
 
 constexpr int kVec = 8;                    // weights per lane and load
 constexpr int kDepth = 4;                  // loads of a chunk of a row
-constexpr int kChunkElems = 64 * kVec * kDepth;
+constexpr int kShortDepth = 2;             // the same of rows that are one short chunk, whose inputs the lanes keep
+constexpr int kChunkElems = 64 * kVec * kDepth, kShortElems = 64 * kVec * kShortDepth;
 constexpr int kWgPerCu = 4;                // workgroups per CU of a persistent launch
 constexpr int kInputVecs = 8;              // 16-byte vectors of a lane that wait in registers on their way to LDS
 
-__host__ __device__ __forceinline__ int chunks_of(int K) { return (K + kChunkElems - 1) / kChunkElems; }
+__host__ __device__ __forceinline__ int chunks_of(int K, int elems = kChunkElems) { return (K + elems - 1) / elems; }
 
 typedef uint32_t rl_u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -169,13 +170,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(const uint16_t* w, 
 
 constexpr int kStreaming = 2;              // cache policy of a buffer load: nt
 
-// Chunk kc of a row, kDepth vectors a lane.
-template <int POLICY = kStreaming>
-__device__ __forceinline__ void fetch_chunk(rl_u32x4 (&v)[kDepth], __amdgpu_buffer_rsrc_t row, int kc, int lane) {
-  const int at = kc * (kChunkElems * 2) + lane * 16;
+// Chunk kc of a row, DEPTH vectors a lane; `last`: of which those behind it are zeros without a load.
+template <int POLICY = kStreaming, int DEPTH>
+__device__ __forceinline__ void fetch_chunk(rl_u32x4 (&v)[DEPTH], __amdgpu_buffer_rsrc_t row, int kc, int lane, int last = DEPTH - 1) {
+  const int at = kc * (DEPTH * 1024) + lane * 16;
 #pragma unroll
-  for (int u = 0; u < kDepth; ++u)
-    v[u] = __builtin_bit_cast(rl_u32x4, __builtin_amdgcn_raw_buffer_load_b128(row, at + u * 1024, 0, POLICY));
+  for (int u = 0; u < DEPTH; ++u)
+    if (u > last) v[u] = rl_u32x4{0, 0, 0, 0};
+    else v[u] = __builtin_bit_cast(rl_u32x4, __builtin_amdgcn_raw_buffer_load_b128(row, at + u * 1024, 0, POLICY));
 }
 
 // acc + the two products of bf16 pairs (an element of a vector has to be a value of its own here: a bit cast of the element
@@ -207,12 +209,12 @@ __device__ __forceinline__ void mul_chunk(float (&acc)[M], const rl_u32x4 (&v)[k
 }
 
 // The same with the input's chunk in registers, zeros where there is none.
-template <int M>
-__device__ __forceinline__ void mul_chunk(float (&acc)[M], const rl_u32x4 (&v)[kDepth], const rl_u32x4 (&x)[M][kDepth]) {
+template <int M, int DEPTH>
+__device__ __forceinline__ void mul_chunk(float (&acc)[M], const rl_u32x4 (&v)[DEPTH], const rl_u32x4 (&x)[M][DEPTH], int last = DEPTH - 1) {
 #pragma unroll
-  for (int u = 0; u < kDepth; ++u)
+  for (int u = 0; u < DEPTH; ++u)
 #pragma unroll
-    for (int m = 0; m < M; ++m)
+    for (int m = 0; m < M && u <= last; ++m)
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[m] = dot2(v[u][i], x[m][u][i], acc[m]);
 }
@@ -349,12 +351,19 @@ struct EarlyNorm {
 // Inputs that LDS does not hold ride with the weights (read from memory as before / as they are used, between requests for weights / now):
 //   4 rows: 1000 x 20480   17.0 / 25.0 / 12.6     5120 x 20480   62.6 / 78.5 / 55.8     1000 x 98304   75 / 208 / 58
 //           two terms of 14336: 1000 rows of each 22.0 / 34.5 / 18.9, 14336 231 / 224 / 221;  3 rows, 1000: 19.9 / 29.2 / 17.0
-template <int M, RowsInput IN, int TWO, bool RES, int SLOTS>
+// SHORT: rows of at most kShortElems, whose inputs every lane takes into registers before the first product (from memory by
+// itself, IN == kFromMemory, or what a norm left in LDS), so that a row's work is two loads and two vectors' products, not four.
+// us a launch, loads past a row's end skipped by branches (as it was) / chunks of four vectors / now:
+//   one row   3392 x 256 2.64 / 3.04 / 2.52    32000 x 256 7.4 / 8.5 / 6.0    32000 x 1000 14.3 / 11.9 / 11.6    residual, 3392 x 256 2.67 / 3.01 / 2.67
+//   4 rows    3392 x 256 3.38 / 3.95 / 3.10    32000 x 256 12.3 / 18.5 / 10.4   32000 x 1000 20.9 / 20.8 / 14.7   norm, gated 2 x 32000 x 256 27 / 37 / 21
+// From 1032 elements on the chunks of four are ahead of what was: 4 rows of 1032, 3392 results 4.99 / 4.57, 1000 4.28 / 3.41.
+template <int M, RowsInput IN, int TWO, bool RES, int SLOTS, bool SHORT>
 __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_linear a, socket_residual nrm) {
   extern __shared__ __attribute__((aligned(16))) float rl_lds[];
   __shared__ float red[2][4];
   constexpr bool EARLY = IN == kNormEarly2 || IN == kNormEarly4;
-  constexpr bool ZEROS = M == 1 && (EARLY || IN == kFromLds), MEM = IN == kFromMemory;
+  constexpr bool ZEROS = M == 1 && (EARLY || IN == kFromLds), MEM = IN == kFromMemory && !SHORT;
+  constexpr int kLoads = SHORT ? kShortDepth : kDepth, kElems = SHORT ? kShortElems : kChunkElems;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int waves = gridDim.x * (kRowThreads / 64);
   int n = blockIdx.x * (kRowThreads / 64) + wave;   // (wave-uniform)
@@ -363,15 +372,27 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
   const uint16_t* x1 = (const uint16_t*)a.x1;
   const uint16_t* x2 = TWO == 2 ? (const uint16_t*)a.x2 : x1;
   const int K1 = a.K1, K2 = TWO == 2 ? a.K2 : K1;
-  const int nk1 = chunks_of(K1), nk = TWO == 2 ? nk1 + chunks_of(K2) : nk1;
+  const int nk1 = chunks_of(K1, kElems), nk = TWO == 2 ? nk1 + chunks_of(K2, kElems) : nk1;
   const int rows1 = ZEROS ? nk1 * kChunkElems : M * K1;     // elements of LDS in front of the second input's
+
+  // (which vectors of a short row hold any of it: a branch, which costs nothing where a wave has one row, but for the residual's
+  // single row, 2.67 us without and 2.75 with it for 3392 x 256)
+  const int last1 = SHORT && SLOTS == 1 && !(RES && M == 1) ? (K1 - 1) / (64 * kVec) : kLoads - 1;
 
   // ---- the input's requests ----
   uint16_t* xs = reinterpret_cast<uint16_t*>(rl_lds) + (IN == kNormRows ? 2 * K1 : 0);    // (behind residual_row's floats)
   constexpr int kIn = TWO == 2 ? kInputVecs / 2 : kInputVecs;      // vectors a lane requests of either input
   rl_u32x4 in1[IN == kFromLds ? kIn : 1], in2[IN == kFromLds && TWO == 2 ? kIn : 1];
   EarlyNorm<IN == kNormEarly4 ? 4 : 2> early;
+  rl_u32x4 held1[SHORT ? M : 1][kLoads], held2[SHORT ? M : 1][kLoads];
   if constexpr (EARLY) early.request(nrm);
+  if constexpr (SHORT && IN == kFromMemory) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      fetch_chunk<0>(held1[m], row_buffer(x1, m, K1, true), 0, lane, last1);
+      if constexpr (TWO == 2) fetch_chunk<0>(held2[m], row_buffer(x2, m, K2, true), 0, lane);
+    }
+  }
   if constexpr (IN == kFromLds) {
     request_input<M, kIn>(in1, xs, x1, K1);
     if constexpr (TWO == 2) request_input<M, kIn>(in2, xs + rows1, x2, K2);
@@ -392,7 +413,7 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
   }
 
   // ---- the first weights' ----
-  rl_u32x4 wv[SLOTS][kDepth], gv[TWO == 1 ? SLOTS : 1][kDepth], xv[MEM ? SLOTS : 1][M][kDepth];
+  rl_u32x4 wv[SLOTS][kLoads], gv[TWO == 1 ? SLOTS : 1][kLoads], xv[MEM ? SLOTS : 1][M][kLoads];
   uint16_t bias1[SLOTS], bias2[TWO == 1 ? SLOTS : 1];
   const __amdgpu_buffer_rsrc_t b1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.b1), 0, a.b1 ? a.N * 2 : 0, 0x00027000);
   const __amdgpu_buffer_rsrc_t b2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.b2), 0, a.b2 ? a.N * 2 : 0, 0x00027000);
@@ -405,10 +426,10 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
     if constexpr (MEM)
 #pragma unroll
       for (int m = 0; m < M; ++m) fetch_chunk<0>(xv[i][m], row_buffer(second ? x2 : x1, m, K, there), at, lane);
-    fetch_chunk(wv[i], row_buffer(second ? w2 : w1, fn, K, there), at, lane);
+    fetch_chunk(wv[i], row_buffer(second ? w2 : w1, fn, K, there), at, lane, last1);
     bias1[i] = __builtin_amdgcn_raw_buffer_load_b16(b1, there ? fn * 2 : 0, 0, 0);
     if constexpr (TWO == 1) {
-      fetch_chunk(gv[i], row_buffer(w2, fn, K1, there), fkc, lane);
+      fetch_chunk(gv[i], row_buffer(w2, fn, K1, there), fkc, lane, last1);
       bias2[i] = __builtin_amdgcn_raw_buffer_load_b16(b2, there ? fn * 2 : 0, 0, 0);
     }
     const bool row_ends = ++fkc == nk;
@@ -439,6 +460,16 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
     x1 = xs;
     x2 = IN == kFromLds ? xs + rows1 : xs;
   }
+  if constexpr (SHORT && IN != kFromMemory) {
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int u = 0; u < kLoads; ++u) {
+        const int k = (u * 64 + lane) * kVec;
+        held1[m][u] = *reinterpret_cast<const rl_u32x4*>(xs + m * K1 + (k < K1 ? k : 0));
+        if (k >= K1) held1[m][u] = rl_u32x4{0, 0, 0, 0};
+      }
+  }
 
   float mixed[M];
   if constexpr (RES) {
@@ -460,7 +491,11 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
   auto step = [&](auto slot, auto refill) __attribute__((always_inline)) {
     constexpr int i = decltype(slot)::value;
     const bool row_ends = kc + 1 == nk;
-    if constexpr (MEM) {
+    if constexpr (SHORT) {
+      if (TWO == 2 && kc >= nk1) mul_chunk<M>(acc2, wv[i], held2);
+      else mul_chunk<M>(acc, wv[i], held1, last1);
+      if constexpr (TWO == 1) mul_chunk<M>(acc2, gv[i], held1, last1);
+    } else if constexpr (MEM) {
       if (TWO == 2 && kc >= nk1) mul_chunk<M>(acc2, wv[i], xv[i]);
       else mul_chunk<M>(acc, wv[i], xv[i]);
       if constexpr (TWO == 1) mul_chunk<M>(acc2, gv[i], xv[i]);
@@ -504,14 +539,14 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
     kc = row_ends ? 0 : kc + 1;
   };
   // (all slots in every turn: to leave in the middle of one would make the waits of the next for everything, too)
-  if constexpr (SLOTS == most_slots(IN, TWO))
+  if constexpr (SHORT ? SLOTS > 1 : SLOTS == most_slots(IN, TWO))
     while (fn < a.N) static_for<SLOTS>([&](auto slot) __attribute__((always_inline)) { step(slot, std::true_type{}); });
   static_for<SLOTS>([&](auto slot) __attribute__((always_inline)) { step(slot, std::false_type{}); });
 }
 
-template <int M, RowsInput IN, int TWO, bool RES, int SLOTS>
+template <int M, RowsInput IN, int TWO, bool RES, int SLOTS, bool SHORT = false>
 int launch_rows_linear(const socket_rows_linear& a, int n_wg, size_t lds, hipStream_t s) {
-  auto kern = rows_linear_kernel<M, IN, TWO, RES, SLOTS>;
+  auto kern = rows_linear_kernel<M, IN, TWO, RES, SLOTS, SHORT>;
   if (lds > 48 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                              (int)lds) != hipSuccess)
     return SOCKET_ERR_LAUNCH;
@@ -521,33 +556,37 @@ int launch_rows_linear(const socket_rows_linear& a, int n_wg, size_t lds, hipStr
 
 // A wave's slots: as many as it has chunks, up to 16 KB of weights (a load that finds no row left brings nothing, but takes
 // its turn).
-template <int M, RowsInput IN, int TWO, bool RES>
+template <int M, RowsInput IN, int TWO, bool RES, bool SHORT = false>
 int dispatch_slots(const socket_rows_linear& a, size_t lds, hipStream_t s) {
   constexpr int kWaves = kRowThreads / 64;
   int n_wg = (a.N + kWaves - 1) / kWaves;
   // (few workgroups pay for the input's passage: each keeps its waves streaming from row to row)
-  if (!RES && IN != kFromMemory) n_wg = std::min(n_wg, socket_device_limits().cu_count * kWgPerCu);
-  const int nk = chunks_of(a.K1) + (TWO == 2 ? chunks_of(a.K2) : 0);
+  if (!RES && (SHORT || IN != kFromMemory)) n_wg = std::min(n_wg, socket_device_limits().cu_count * kWgPerCu);
+  constexpr int kElems = SHORT ? kShortElems : kChunkElems, kMost = SHORT && TWO != 1 ? 4 : most_slots(IN, TWO);
+  const int nk = chunks_of(a.K1, kElems) + (TWO == 2 ? chunks_of(a.K2, kElems) : 0);
   const int64_t chunks = (int64_t)((a.N + n_wg * kWaves - 1) / (n_wg * kWaves)) * nk;
-  if constexpr (TWO != 2 && IN != kFromMemory) {
-    if (chunks == 1) return launch_rows_linear<M, IN, TWO, RES, 1>(a, n_wg, lds, s);
-    if (chunks == 2) return launch_rows_linear<M, IN, TWO, RES, 2>(a, n_wg, lds, s);
+  if constexpr (RES && SHORT) return launch_rows_linear<M, IN, TWO, RES, 1, true>(a, n_wg, lds, s);      // (a wave, a row)
+  if constexpr (TWO != 2 && (SHORT || IN != kFromMemory)) {
+    if (chunks == 1) return launch_rows_linear<M, IN, TWO, RES, 1, SHORT>(a, n_wg, lds, s);
+    if (!SHORT && chunks == 2) return launch_rows_linear<M, IN, TWO, RES, 2>(a, n_wg, lds, s);
   }
-  return launch_rows_linear<M, IN, TWO, RES, most_slots(IN, TWO)>(a, n_wg, lds, s);
+  return launch_rows_linear<M, IN, TWO, RES, kMost, SHORT>(a, n_wg, lds, s);
 }
 
-template <int M, RowsInput IN, int TWO>
+template <int M, RowsInput IN, int TWO, bool SHORT = false>
 int dispatch_res(const socket_rows_linear& a, size_t lds, hipStream_t s) {
   if constexpr (TWO == 0 && (IN == kFromMemory || IN == kFromLds))
-    if (a.res) return dispatch_slots<M, IN, TWO, true>(a, lds, s);
-  return dispatch_slots<M, IN, TWO, false>(a, lds, s);
+    if (a.res) return dispatch_slots<M, IN, TWO, true, SHORT>(a, lds, s);
+  return dispatch_slots<M, IN, TWO, false, SHORT>(a, lds, s);
 }
 
 template <int M, int TWO>
 int dispatch_input(const socket_rows_linear& a, hipStream_t s) {
   const size_t room = (size_t)socket_device_limits().max_lds_per_block - 256;
   auto in_lds = [](int K) { return M == 1 ? ((size_t)K + kChunkElems - 1) / kChunkElems * kChunkElems * 2 : (size_t)M * K * 2; };
+  const bool is_short = a.K1 <= kShortElems && (TWO != 2 || a.K2 <= kShortElems);
   if (!a.norm) {
+    if (is_short) return dispatch_res<M, kFromMemory, TWO, true>(a, 0, s);
     const size_t lds = in_lds(a.K1) + (TWO == 2 ? in_lds(a.K2) : 0);
     return lds <= room ? dispatch_res<M, kFromLds, TWO>(a, lds, s) : dispatch_res<M, kFromMemory, TWO>(a, 0, s);
   }
@@ -560,6 +599,8 @@ int dispatch_input(const socket_rows_linear& a, hipStream_t s) {
       if (EarlyNorm<2>::serves(*a.norm)) return dispatch_res<M, kNormEarly2, TWO>(a, in_lds(a.K1), s);
       if (EarlyNorm<4>::serves(*a.norm)) return dispatch_res<M, kNormEarly4, TWO>(a, in_lds(a.K1), s);
     }
+    if constexpr (M > 1)
+      if (is_short) return dispatch_res<M, kNormRows, TWO, true>(a, rows, s);
     return dispatch_res<M, kNormRows, TWO>(a, rows, s);
   }
 }

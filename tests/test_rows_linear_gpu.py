@@ -32,12 +32,12 @@ def dev():
     return torch.device("cuda:0")
 
 
-# K: below, at and behind a chunk of 2048; four chunks in flight and more; inputs past the registers on their way to LDS, and
+# K: below, at and behind a vector of 512 and rows of 1024 that lanes hold; below, at and behind a chunk of 2048; four chunks in flight and more; inputs past the registers on their way to LDS, and
 # past LDS.  N: no full workgroup, one row too many for one, two and four rows a wave of the persistent launch.
 # Rows that are normed: past a CU's LDS with four at 13640, with three and four at 16384.
 @pytest.mark.parametrize("rows", [1, 2, 3, 4])
 @pytest.mark.parametrize("K,N", [(8, 1), (40, 4097), (2040, 5), (2048, 4099), (2056, 8200), (4096, 1030), (8192, 64), (10248, 33),
-                                 (13632, 6), (13640, 6), (14336, 40), (16352, 5), (16384, 24), (16392, 7), (20488, 9), (256, 16390), (64, 40000)])
+                                 (13632, 6), (13640, 6), (14336, 40), (16352, 5), (16384, 24), (16392, 7), (20488, 9), (256, 16390), (64, 40000), (512, 4099), (520, 3), (1024, 8200), (1032, 4090)])
 def test_products_of_every_form(dev, rows, K, N):
     from socket_amd import layer_ops
     g = torch.Generator().manual_seed(rows * 1000003 + K * 31 + N)
@@ -80,7 +80,7 @@ def test_products_of_every_form(dev, rows, K, N):
     assert _rms(got_x, e) < 1e-6 and _rms(y, h @ w.double().t(), _spread(h, w)) < normed
 
 
-@pytest.mark.parametrize("K", [40, 2056, 41000])      # (the last past what LDS holds of two rows)
+@pytest.mark.parametrize("K", [40, 520, 2056, 41000])      # (the last past what LDS holds of two rows)
 def test_an_infinity_stays_in_its_row(dev, K):
     """Lanes past a row's end multiply zeros, not what lies behind the row."""
     from socket_amd import layer_ops
