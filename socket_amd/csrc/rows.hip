@@ -154,7 +154,8 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 enum RowsInput {
   kFromMemory,      // x1 (and x2), requested with the weights that they meet: rows that do not fit into LDS
   kFromLds,         // x1 (and x2), brought into LDS
-  kNormRows,        // residual_row's, one row after the other, behind the first weights
+  kNormRows,        // residual_row's, one row after the other, behind the first weights: half of a wave's slots
+  kNormRowsLong,    // the same behind all of its slots, where a wave has more chunks than that
   kNormEarly2,      // residual_row's for one row of up to 2 float4 vectors a lane, its operands requested ahead of the weights
   kNormEarly4,      // the same, up to 4
 };
@@ -372,6 +373,7 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
   const uint16_t* x1 = (const uint16_t*)a.x1;
   const uint16_t* x2 = TWO == 2 ? (const uint16_t*)a.x2 : x1;
   const int K1 = a.K1, K2 = TWO == 2 ? a.K2 : K1;
+  constexpr bool NORM_ROWS = IN == kNormRows || IN == kNormRowsLong;
   const int nk1 = chunks_of(K1, kElems), nk = TWO == 2 ? nk1 + chunks_of(K2, kElems) : nk1;
   const int rows1 = ZEROS ? nk1 * kChunkElems : M * K1;     // elements of LDS in front of the second input's
 
@@ -380,7 +382,7 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
   const int last1 = SHORT && SLOTS == 1 && !(RES && M == 1) ? (K1 - 1) / (64 * kVec) : kLoads - 1;
 
   // ---- the input's requests ----
-  uint16_t* xs = reinterpret_cast<uint16_t*>(rl_lds) + (IN == kNormRows ? 2 * K1 : 0);    // (behind residual_row's floats)
+  uint16_t* xs = reinterpret_cast<uint16_t*>(rl_lds) + (NORM_ROWS ? 2 * K1 : 0);    // (behind residual_row's floats)
   constexpr int kIn = TWO == 2 ? kInputVecs / 2 : kInputVecs;      // vectors a lane requests of either input
   rl_u32x4 in1[IN == kFromLds ? kIn : 1], in2[IN == kFromLds && TWO == 2 ? kIn : 1];
   EarlyNorm<IN == kNormEarly4 ? 4 : 2> early;
@@ -436,19 +438,24 @@ __global__ __launch_bounds__(kRowThreads) void rows_linear_kernel(socket_rows_li
     fn = row_ends ? fn + waves : fn;
     fkc = row_ends ? 0 : fkc;
   };
-  static_for<SLOTS>(fetch);
+  // (Rows normed one after the other have trips to memory for each, which all of a wave's weights, requested first, would keep
+  // waiting to the last.  2 and 4 rows, us with all slots / half of them first: 14336 x 2048 15.7 / 14.7 and 20.3 / 18.9, gated
+  // 2 x 3392 x 4096 17.6 / 16.2 and 34.2 / 32.3; past as many chunks the stream counts, 32000 x 2048 24.4 / 25.0 and 30.2 / 29.8.)
+  constexpr int kFirst = IN == kNormRows && !SHORT && SLOTS > 1 ? SLOTS / 2 : SLOTS;
+  static_for<kFirst>(fetch);
 
   // ---- the input ----
   if constexpr (EARLY) {
     early.finish(nrm, red, blockIdx.x == 0, [&](int i, const float* v) { store_vec<DType_bf16, 4>(xs, i, v); });
     zeros_behind(xs, K1);
     __syncthreads();
-  } else if constexpr (IN == kNormRows) {
+  } else if constexpr (NORM_ROWS) {
     for (int m = 0; m < M; ++m) {
       residual_row<DType_bf16, 4, false>(nrm, m, rl_lds, red, blockIdx.x == 0,
                                   [&](int i, const float* v) { store_vec<DType_bf16, 4>(xs, (int64_t)m * K1 + i, v); });
       __syncthreads();
     }
+    static_for<SLOTS - kFirst>([&](auto slot) __attribute__((always_inline)) { fetch(std::integral_constant<int, decltype(slot)::value + kFirst>{}); });
   } else if constexpr (IN == kFromLds) {
     place_input<M, kIn>(in1, xs, K1);
     if constexpr (TWO == 2) place_input<M, kIn>(in2, xs + rows1, K2);
@@ -570,6 +577,8 @@ int dispatch_slots(const socket_rows_linear& a, size_t lds, hipStream_t s) {
     if (chunks == 1) return launch_rows_linear<M, IN, TWO, RES, 1, SHORT>(a, n_wg, lds, s);
     if (!SHORT && chunks == 2) return launch_rows_linear<M, IN, TWO, RES, 2>(a, n_wg, lds, s);
   }
+  if constexpr (IN == kNormRows && !SHORT)
+    if (chunks > kMost) return launch_rows_linear<M, kNormRowsLong, TWO, RES, kMost>(a, n_wg, lds, s);
   return launch_rows_linear<M, IN, TWO, RES, kMost, SHORT>(a, n_wg, lds, s);
 }
 
