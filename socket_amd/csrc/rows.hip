@@ -573,9 +573,9 @@ int dispatch_slots(const socket_rows_linear& a, size_t lds, hipStream_t s) {
   const int nk = chunks_of(a.K1, kElems) + (TWO == 2 ? chunks_of(a.K2, kElems) : 0);
   const int64_t chunks = (int64_t)((a.N + n_wg * kWaves - 1) / (n_wg * kWaves)) * nk;
   if constexpr (RES && SHORT) return launch_rows_linear<M, IN, TWO, RES, 1, true>(a, n_wg, lds, s);      // (a wave, a row)
-  if constexpr (TWO != 2 && (SHORT || IN != kFromMemory)) {
+  if constexpr (TWO != 2 && (SHORT || IN != kFromMemory || (RES && M < 4))) {
     if (chunks == 1) return launch_rows_linear<M, IN, TWO, RES, 1, SHORT>(a, n_wg, lds, s);
-    if (!SHORT && chunks == 2) return launch_rows_linear<M, IN, TWO, RES, 2>(a, n_wg, lds, s);
+    if (!SHORT && IN != kFromMemory && chunks == 2) return launch_rows_linear<M, IN, TWO, RES, 2>(a, n_wg, lds, s);
   }
   if constexpr (IN == kNormRows && !SHORT)
     if (chunks > kMost) return launch_rows_linear<M, kNormRowsLong, TWO, RES, kMost>(a, n_wg, lds, s);
@@ -596,6 +596,11 @@ int dispatch_input(const socket_rows_linear& a, hipStream_t s) {
   const bool is_short = a.K1 <= kShortElems && (TWO != 2 || a.K2 <= kShortElems);
   if (!a.norm) {
     if (is_short) return dispatch_res<M, kFromMemory, TWO, true>(a, 0, s);
+    // A residual's rows of one chunk while each CU has a workgroup at most: the way through LDS is on the chain of what the launch
+    // waits for.  2048 elements, us through LDS / from memory: one row, 64 results 2.45 / 2.16, 1000 2.88 / 2.76, two rows 3.17 / 3.07,
+    // three 3.41 / 3.36, four 3.60 / 3.68; one row, 3392 results 4.44 / 4.59; without a residual, one row, 1000 results 2.74 / 3.04.
+    if (M < 4 && a.res && chunks_of(a.K1) == 1 && a.N <= kRowThreads / 64 * socket_device_limits().cu_count)
+      return dispatch_res<M, kFromMemory, TWO>(a, 0, s);
     const size_t lds = in_lds(a.K1) + (TWO == 2 ? in_lds(a.K2) : 0);
     return lds <= room ? dispatch_res<M, kFromLds, TWO>(a, lds, s) : dispatch_res<M, kFromMemory, TWO>(a, 0, s);
   }

@@ -37,7 +37,8 @@ def dev():
 # Rows that are normed: past a CU's LDS with four at 13640, with three and four at 16384.
 @pytest.mark.parametrize("rows", [1, 2, 3, 4])
 @pytest.mark.parametrize("K,N", [(8, 1), (40, 4097), (2040, 5), (2048, 4099), (2056, 8200), (4096, 1030), (8192, 64), (10248, 33),
-                                 (13632, 6), (13640, 6), (14336, 40), (16352, 5), (16384, 24), (16392, 7), (20488, 9), (256, 16390), (64, 40000), (512, 4099), (520, 3), (1024, 8200), (1032, 4090)])
+                                 (13632, 6), (13640, 6), (14336, 40), (16352, 5), (16384, 24), (16392, 7), (20488, 9), (256, 16390), (64, 40000), (512, 4099), (520, 3), (1024, 8200), (1032, 4090),
+                                 (1032, 7), (2048, 1023), (2048, 1028)])
 def test_products_of_every_form(dev, rows, K, N):
     from socket_amd import layer_ops
     g = torch.Generator().manual_seed(rows * 1000003 + K * 31 + N)
