@@ -276,7 +276,9 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
             // One test for all codes of the wave: the sums of codes that are all inside take less than five vector
             // instructions a code, where a test of each took nine and 1.8 times the code.  The vector ALUs were what the
             // launch waited for, two waves to each of them at 512 lanes (us before / now, with the wait below: 32 rows of
-            // 32768 tokens, L60 x R1024, bf16 35.6 / 30.5, fp32 43.0 / 33.7; 9001 tokens, bf16 17.1 / 15.1).
+            // 32768 tokens, L60 x R1024, bf16 35.6 / 30.5, fp32 43.0 / 33.7; 9001 tokens, bf16 17.1 / 15.1).  Where one is outside
+            // each code is tested by one comparison more (a hundredth of the codes outside, us with a test of each / with the
+            // branch's old form / now: 32 rows of 4448, L32 x R256, fp32 8.1 / 9.6 / 8.2, 32768, L60 x R1024 31.6 / 32.6 / 27.4).
             const uint32_t base = table_at + (uint32_t)(l * R) * (uint32_t)sizeof(QT);
             u16x2 most = {0, 0};
             uint32_t at[TPT];
@@ -288,18 +290,23 @@ __global__ __launch_bounds__(THREADS) void collision_i16_kernel(
               at[i + 1] = entry_address<sizeof(QT)>(w, true, base);
             }
             const u16x2 outside = __builtin_elementwise_sub_sat(most, u16x2{last_code, last_code});
-            if (__builtin_expect(__ballot(__builtin_bit_cast(uint32_t, outside) != 0) != 0, 0)) {
-              add_any();
-              refill();
-            } else {
+            auto add = [&](auto all) __attribute__((always_inline)) {
+              bool hit[TPT];
+#pragma unroll
+              for (int i = 0; i < TPT; ++i) {
+                hit[i] = decltype(all)::value || (uint16_t)(V::word(cur, i >> 1) >> (16 * (i & 1))) <= last_code;
+                at[i] = hit[i] ? at[i] : base;
+              }
               __builtin_amdgcn_sched_barrier(0);     // (the codes have been used: their registers take the next)
               refill();
               entry_bits_t<QT> e[TPT];
 #pragma unroll
               for (int i = 0; i < TPT; ++i) e[i] = *(const __attribute__((address_space(3))) entry_bits_t<QT>*)(uintptr_t)at[i];
 #pragma unroll
-              for (int i = 0; i < TPT; ++i) sum[i] += entry_to_f32(__builtin_bit_cast(QT, e[i]));
-            }
+              for (int i = 0; i < TPT; ++i) sum[i] += hit[i] ? entry_to_f32(__builtin_bit_cast(QT, e[i])) : 0.f;
+            };
+            if (__builtin_expect(__ballot(__builtin_bit_cast(uint32_t, outside) != 0) != 0, 0)) add(std::false_type{});
+            else add(std::true_type{});
           } else {
             refill();
             add_any();
