@@ -62,3 +62,14 @@ def test_codes_outside_the_table_add_nothing(dtype, R, T):
 def test_tiles(dtype, B, H, L, T, R):
     probs, codes, allowed, norms = _operands(B, H, L, T, R, dtype, T)
     assert torch.equal(_run(probs, codes, allowed, norms), _scores(probs, codes, allowed, norms))
+
+
+# codes past what a cache keeps from call to call, four and eight tokens a lane, also with some outside the table
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,L,T,R", [(32, 130, 24575, 64), (56, 48, 40003, 256)])
+def test_streamed_codes(dtype, H, L, T, R):
+    probs, codes, allowed, norms = _operands(1, H, L, T, R, dtype, T)
+    assert codes.numel() * 2 > 192 << 20
+    assert torch.equal(_run(probs, codes, allowed, norms), _scores(probs, codes, allowed, norms))
+    codes[:, :, ::7, ::1013] = -1
+    assert torch.equal(_run(probs, codes, allowed, norms), _scores(probs, codes, allowed, norms))
