@@ -413,13 +413,20 @@ __global__ __launch_bounds__(kAttThreads, 1) void latent_attend_kernel(socket_la
 //
 // Grid (rows of w_uv in slices of 64, heads, tokens).  The first weights are requested before the
 // partial results are merged, which eight groups of lanes share.
+// FEW: 2 to 63 splits, rows that the groups share: every wave works all the shares out by itself, a lane a split, without a barrier,
+// while the partial results that it will add up are on their way (shares through LDS and the results asked for after them: 7.2 us a
+// launch of 16 heads x 128 x 512 over 12 splits, now 6.5).  It reads what splits without keys left, too, and with more workgroups
+// than three quarters of the CUs that is felt, so that these take it up to eight splits only.
+// us with the attention before it, without / with FEW: 16 heads, 24 splits full 12.9 / 11.9, a third full 12.0 / 11.5; 96 heads, 24 splits 16.8 /
+// 15.9 and 13.3 / 12.8, 32 splits a third full 14.5 / 15.0; 128 heads, 2 splits 13.1 / 12.8, 24 splits 20.4 / 19.8 and 15.0 / 16.3; 64 splits, whose loop without it has all of a group's results in
+// flight, 16 heads 14.2 / 14.4, 5 heads 9.4 / 9.8.
 constexpr int kValThreads = 1024, kValWaves = kValThreads / 64;
 constexpr int kValRows = 4;               // per wave
 constexpr int kValGroups = 8, kValLanes = kValThreads / kValGroups;
 constexpr int kMaxSplits = 256;
 constexpr int kMaxMerge = 4 * kValLanes;  // widest row whose merge the groups share
 
-template <class DT, bool VEC>
+template <class DT, bool VEC, bool FEW>
 __global__ __launch_bounds__(kValThreads) void latent_values_kernel(socket_latent_attention a) {
   extern __shared__ __attribute__((aligned(16))) float lv_lds[];   // rank_p, then kValGroups x rank_p
   __shared__ float share[kMaxSplits], red[kValWaves], red2[kValWaves];
@@ -451,11 +458,7 @@ __global__ __launch_bounds__(kValThreads) void latent_values_kernel(socket_laten
   if (a.gate && lane < kValRows && d0 + lane < a.vdim)
     gate = a.gate_f32 ? ((const float*)a.gate)[g0 + d0 + lane] : load_elem<DT>(a.gate, g0 + d0 + lane);
   const int64_t part = (int64_t)blockIdx.z * a.splits * a.H + h;
-  // Up to a wave's lanes of splits: every wave works all their shares out by itself, without a barrier, while the partial
-  // results that it will add up are on their way (shares through LDS and the results asked for after them: 7.2 us a launch of 16
-  // heads x 128 x 512 over 12 splits, now 6.5).
-  const bool few = a.ml && a.splits > 1 && a.splits <= 64 && rank_p <= kMaxMerge;
-  if (few) {
+  if constexpr (FEW) {
     constexpr int kAhead = 4;
     const int grp = __builtin_amdgcn_readfirstlane(tid / kValLanes), c = tid % kValLanes * 4;
     const float* o = a.o + part * rank_p + (c < rank_p ? c : 0);
@@ -495,10 +498,10 @@ __global__ __launch_bounds__(kValThreads) void latent_values_kernel(socket_laten
     if (tid == 0) share[0] = 1.f;
     __syncthreads();
   }
-  if (few || (a.splits > 1 && rank_p <= kMaxMerge)) {
+  if (FEW || (a.splits > 1 && rank_p <= kMaxMerge)) {
     const int grp = tid / kValLanes, c = tid % kValLanes * 4;
     float* mine = lv_lds + (1 + grp) * rank_p;
-    if (!few && c < rank_p) {
+    if (!FEW && c < rank_p) {
       float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 8
       for (int k = grp; k < a.splits; k += kValGroups) {
@@ -684,13 +687,21 @@ extern "C" int socket_latent_values(const socket_latent_attention* args, void* s
   const size_t lds = (size_t)rank_p * 4 * (rank_p <= kMaxMerge ? 1 + kValGroups : 1);
   hipStream_t s = (hipStream_t)stream;
   const bool vec = a.rank % 8 == 0 && socket_aligned16(a.w_uv);
+  const bool many = (int64_t)grid.x * grid.y * grid.z > socket_device_limits().cu_count * 3 / 4;
+  const bool few = a.ml && a.splits > 1 && a.splits < (many ? 9 : 64) && rank_p <= kMaxMerge;
+#define SOCKET_LV(DT, V)                                                                            \
+  do {                                                                                              \
+    if (few) hipLaunchKernelGGL((latent_values_kernel<DT, V, true>), grid, block, lds, s, a);       \
+    else hipLaunchKernelGGL((latent_values_kernel<DT, V, false>), grid, block, lds, s, a);          \
+  } while (0)
   if (a.dtype == SOCKET_F32) {
-    if (vec) hipLaunchKernelGGL((latent_values_kernel<DType_f32, true>), grid, block, lds, s, a);
-    else hipLaunchKernelGGL((latent_values_kernel<DType_f32, false>), grid, block, lds, s, a);
+    if (vec) SOCKET_LV(DType_f32, true);
+    else SOCKET_LV(DType_f32, false);
   } else {
-    if (vec) hipLaunchKernelGGL((latent_values_kernel<DType_bf16, true>), grid, block, lds, s, a);
-    else hipLaunchKernelGGL((latent_values_kernel<DType_bf16, false>), grid, block, lds, s, a);
+    if (vec) SOCKET_LV(DType_bf16, true);
+    else SOCKET_LV(DType_bf16, false);
   }
+#undef SOCKET_LV
   SOCKET_LAUNCH_CHECK();
   return SOCKET_OK;
 }
