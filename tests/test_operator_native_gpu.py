@@ -30,7 +30,16 @@ def operands(B, H, Hkv, L, R, T, D, dtype, norm_dtype, seed):
     return (probs, codes, norms, allowed), (q, k, v)
 
 
-def both(ops, qkv, sink, window, M):
+def natively(ops, qkv, sink, window, M):
+    """What the native step by itself makes of the operands: their list, its lengths and the attention, or None."""
+    from socket_amd import sparse
+    host, stream = _lib.host(), _lib.stream_ptr(qkv[0].device)
+    lists = host.build_list(*ops, sink, window, M, sparse._LONG_BASE, _lib.SOCKET_TOPK_MAX_M, sparse._select_workspace, stream)
+    return lists and (*lists, host.sparse_attention(*qkv, *lists, stream))
+
+
+def both(ops, qkv, sink, window, M, taken=True):
+    direct = natively(ops, qkv, sink, window, M)
     lists = build_sparse_list_decode(*ops, sink, window, M)
     out = sparse_attention_fwd(*qkv, *lists)
     with Watch():
@@ -39,16 +48,21 @@ def both(ops, qkv, sink, window, M):
     assert type(lists) is tuple and torch.equal(lists[0], want_lists[0]) and torch.equal(lists[1], want_lists[1])
     assert lists[0].dtype == lists[1].dtype == torch.int32 and out.dtype == qkv[0].dtype
     assert torch.equal(out, want)
+    assert (direct is not None) == taken
+    if taken:
+        assert type(direct[2]) is torch.Tensor
+        assert torch.equal(direct[0], want_lists[0]) and torch.equal(direct[1], want_lists[1]) and torch.equal(direct[2], want)
 
 
 @pytest.mark.parametrize("dtype,norm_dtype", [(torch.bfloat16, torch.float16), (torch.float32, torch.float32), (torch.float16, torch.bfloat16)])
 @pytest.mark.parametrize("B,H,Hkv,L,R,T,D,sink,window,M", [
     (1, 1, 1, 1, 4, 1, 16, 0, 0, 5), (2, 6, 2, 5, 32, 131, 64, 4, 16, 20), (1, 4, 4, 8, 256, 1000, 128, 1000, 7, 2000),
     (1, 2, 1, 3, 64, 70001, 32, 20, 0, 700), (3, 8, 4, 4, 128, 517, 128, 0, 600, 1),
-    (1, 2, 2, 2, 16, 5000, 64, 96, 4000, 9), (1, 2, 2, 2, 16, 5000, 64, 96, 4001, 9)])      # (at and past the entries that it takes)
+    (1, 2, 2, 2, 16, 5000, 64, 96, 4000, 9), (1, 2, 2, 2, 16, 5000, 64, 96, 4001, 9),
+    (1, 2, 2, 2, 16, 30000, 64, 96, 24480, 9), (1, 2, 2, 2, 16, 30000, 64, 96, 24481, 9)])      # (at and past the entries that it takes)
 def test_same_as_through_python(dtype, norm_dtype, B, H, Hkv, L, R, T, D, sink, window, M):
     ops, qkv = operands(B, H, Hkv, L, R, T, D, dtype, norm_dtype, T)
-    both(ops, qkv, sink, window, M)
+    both(ops, qkv, sink, window, M, taken=sink + window <= 24576)
 
 
 def test_strided_rows_and_lists():
@@ -91,3 +105,29 @@ def test_what_goes_through_python():
     with pytest.raises(RuntimeError):      # (the library wants rows on 16-byte boundaries)
         sparse_attention_fwd(torch.randn(1, 4 * 64 + 1, device=DEV).bfloat16()[:, 1:].view(1, 4, 64), k, v, *want)
     assert not sparse_attention_fwd(q.requires_grad_(), k, v, *want).requires_grad
+
+
+@pytest.mark.parametrize("T", [3000, 70001])      # (one workgroup to a row, and several, which need the workspace)
+def test_on_a_side_stream_and_captured(T):
+    ops, qkv = operands(1, 2, 1, 3, 64, T, 64, torch.bfloat16, torch.float16, 7)
+    want = natively(ops, qkv, 4, 64, 300)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = build_sparse_list_decode(*ops, 4, 64, 300)
+        got = (*got, sparse_attention_fwd(*qkv, *got))
+    torch.cuda.current_stream().wait_stream(side)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    q = qkv[0].clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        lists = build_sparse_list_decode(*ops, 4, 64, 300)
+        out = sparse_attention_fwd(q, *qkv[1:], *lists)
+    for turn in range(4):
+        ops[0].copy_(torch.roll(ops[0], 1, -1))
+        q.copy_(torch.roll(q, 1, -1))
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = natively(ops, (q, *qkv[1:]), 4, 64, 300)
+        assert torch.equal(lists[0], want[0]) and torch.equal(lists[1], want[1]) and torch.equal(out, want[2])
