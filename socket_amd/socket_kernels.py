@@ -122,7 +122,7 @@ def sparse_attention_fwd(
     on the split beyond fp32 rounding), and the list width bounds the lengths,
     so there is no `sparse_len.max().item()` device-to-host read.
     """
-    if type(query) is torch.Tensor and query.is_cuda and not observed():
+    if type(query) is torch.Tensor and query.is_cuda and sparse_list.dtype is torch.int32 and not observed():
         # (the usual operands in one step; what it does not take is looked over here)
         out = host().sparse_attention(query, key, value, sparse_list, sparse_len, stream_ptr(query.device))
         if out is not None:

@@ -252,7 +252,7 @@ def build_sparse_list_decode(
 ):
     """GPT-FAST/kernels/sparse.py:16-95.  KC, BLOCK_N, num_warps, num_stages are
     accepted and ignored, as in the reference (:38)."""
-    if type(q_probs) is torch.Tensor and q_probs.is_cuda and not observed():
+    if type(q_probs) is torch.Tensor and q_probs.is_cuda and k_hard_bhlt.dtype is torch.int16 and not observed():
         # (the usual operands in one step; what it does not take is looked over here)
         built = host().build_list(q_probs, k_hard_bhlt, v_norm_bht, allowed_bht, sink, window, M, _LONG_BASE, SOCKET_TOPK_MAX_M,
                                   _select_workspace, stream_ptr(q_probs.device))
