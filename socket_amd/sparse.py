@@ -195,7 +195,7 @@ def _select_into(scores, sink: int, window: int, M: int, lens, budgets, write_ba
 # the selection's launch one workgroup of a row writes them: no launch more, but 25 us per 100000 entries.  The whole operator
 # over four small tables, us, in the selection's launch / in its own: 32 rows, 16000 entries 21.3 / 22.4, 32768 25.1 / 23.0, 100000 61
 # / 39; 4 rows, 16000 20.1 / 21.7, 32768 23.8 / 21.2, 100000 41 / 25; 128 rows, 16000 33.6 / 36.2, 32768 39.6 / 37.8.
-# The native step knows the first alone, and takes calls up to here.
+# The native step knows the first alone, and takes calls below here.
 _LONG_BASE = 24576
 
 
@@ -254,7 +254,7 @@ def build_sparse_list_decode(
     accepted and ignored, as in the reference (:38)."""
     if type(q_probs) is torch.Tensor and q_probs.is_cuda and k_hard_bhlt.dtype is torch.int16 and not observed():
         # (the usual operands in one step; what it does not take is looked over here)
-        built = host().build_list(q_probs, k_hard_bhlt, v_norm_bht, allowed_bht, sink, window, M, _LONG_BASE, SOCKET_TOPK_MAX_M,
+        built = host().build_list(q_probs, k_hard_bhlt, v_norm_bht, allowed_bht, sink, window, M, _LONG_BASE - 1, SOCKET_TOPK_MAX_M,
                                   _select_workspace, stream_ptr(q_probs.device))
         if built is not None:
             if type(built[0]) is str:

@@ -34,7 +34,7 @@ def natively(ops, qkv, sink, window, M):
     """What the native step by itself makes of the operands: their list, its lengths and the attention, or None."""
     from socket_amd import sparse
     host, stream = _lib.host(), _lib.stream_ptr(qkv[0].device)
-    lists = host.build_list(*ops, sink, window, M, sparse._LONG_BASE, _lib.SOCKET_TOPK_MAX_M, sparse._select_workspace, stream)
+    lists = host.build_list(*ops, sink, window, M, sparse._LONG_BASE - 1, _lib.SOCKET_TOPK_MAX_M, sparse._select_workspace, stream)
     return lists and (*lists, host.sparse_attention(*qkv, *lists, stream))
 
 
@@ -59,10 +59,10 @@ def both(ops, qkv, sink, window, M, taken=True):
     (1, 1, 1, 1, 4, 1, 16, 0, 0, 5), (2, 6, 2, 5, 32, 131, 64, 4, 16, 20), (1, 4, 4, 8, 256, 1000, 128, 1000, 7, 2000),
     (1, 2, 1, 3, 64, 70001, 32, 20, 0, 700), (3, 8, 4, 4, 128, 517, 128, 0, 600, 1),
     (1, 2, 2, 2, 16, 5000, 64, 96, 4000, 9), (1, 2, 2, 2, 16, 5000, 64, 96, 4001, 9),
-    (1, 2, 2, 2, 16, 30000, 64, 96, 24480, 9), (1, 2, 2, 2, 16, 30000, 64, 96, 24481, 9)])      # (at and past the entries that it takes)
+    (1, 2, 2, 2, 16, 30000, 64, 96, 24479, 9), (1, 2, 2, 2, 16, 30000, 64, 96, 24480, 9)])      # (at and past the entries that it takes)
 def test_same_as_through_python(dtype, norm_dtype, B, H, Hkv, L, R, T, D, sink, window, M):
     ops, qkv = operands(B, H, Hkv, L, R, T, D, dtype, norm_dtype, T)
-    both(ops, qkv, sink, window, M, taken=sink + window <= 24576)
+    both(ops, qkv, sink, window, M, taken=sink + window < 24576)
 
 
 def test_strided_rows_and_lists():
