@@ -16,7 +16,7 @@
 // straight from memory into LDS while the first codes are on their way, and
 // serves several such tiles under each slice; a thread fetches the codes of its
 // consecutive tokens with one load per table (wherever the row starts) and gathers
-// without branches.  It has eight tokens, 16-byte loads, six tables ahead of their use;
+// with one branch a wave and table (is any of its codes outside?).  It has eight tokens, 16-byte loads, six tables ahead of their use;
 // four or two where rows are short, 8- or 4-byte loads, 12 or 24 tables ahead.
 #include <atomic>
 

@@ -1166,8 +1166,8 @@ constexpr int kScanWaves = 4;     // of either kind
 // 116 for 64 without; these 204 and 108 (eight waves alone 229 and 127, with fragments two chunks ahead 212 and 109, with a
 // chunk's state tiles asked for together and the first kind's products first the rest).  Read-outs a barrier behind: 32
 // chunks of 16 heads of 128 x 128 with the delta rule 70.8 -> 66.9 us, of 64 x 128 without 40.0 -> 39.0.  Two accumulators in turn
-// for every chain: 69.3.  Without its matrix products such a launch takes 56, without its loads 69: the fragments of a
-// chunk, 116 KB, come at 31 bytes a cycle.
+// for every chain: 69.3.  Parts of it left out, under a tracer and with one head of keys for all (70.8): without the matrix products 42,
+// without the fragments' loads 65, without the read-outs 44; without the delta rule 38.7: 23.8, 36.8, 18.5.
 template <int KT, int NB, bool DELTA, bool EXTRA>
 __global__ __launch_bounds__(kScanThreads, 2) void recurrence_scan_kernel(socket_recurrence a, int n_chunks) {
   constexpr int C = 16 * NB;

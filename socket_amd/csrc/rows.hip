@@ -182,7 +182,10 @@ __device__ __forceinline__ void fetch_chunk(rl_u32x4 (&v)[DEPTH], __amdgpu_buffe
 }
 
 // acc + the two products of bf16 pairs (an element of a vector has to be a value of its own here: a bit cast of the element
-// itself takes the vector's first)
+// itself takes the vector's first).  Products are exact in 32 bits; how the three are rounded is the instruction's own.  Error of
+// whole rows against float64 beside a chain of two multiply-adds, 300 draws each: N(0, 1) 7.48e-8 / 7.43e-8 at 2048 elements, 1.19e-7 /
+// 1.16e-7 at 14336, positive 4.23e-8 / 4.24e-8 (+- 0.1 %), heavy-tailed 2.45e-7 / 2.00e-7.  Subnormal operands and results are kept;
+// products past 2^128 are infinities, which of opposite signs in one pair give a NaN where the chain gives the infinity.
 __device__ __forceinline__ float dot2(uint32_t w, uint32_t x, float acc) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), __builtin_bit_cast(bf16x2, x), acc, false);
 }

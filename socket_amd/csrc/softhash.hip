@@ -430,9 +430,8 @@ __host__ __device__ __forceinline__ float mx_scale(float tanh_scale, float inv_t
 // nothing is split.  Lane x holds column (or row) x % 16 and one k of four; which k that is is free as long as both operands
 // agree: for the projections quarter q of wave w takes dims 32 q + 8 w .. + 7, a run, and for the logits step r takes plane 4 q + r,
 // which is what the lane's own projections are.
-// One sequence of 16 heads, 60 tables: 8.9 us as a launch of the scalar form below, 11.1 us with the rest of the prologue,
-// which took 9.3 us more, in one launch: a chain of trips to memory and of matrix products, on 80 workgroups.
-// Against float64 (2-norm, queries and planes N(0, 1)): 2.1e-7, the scalar form 2.5e-7.
+// One sequence of 16 heads, 60 tables, by itself: 6.0 us, 8.9 of the scalar form below; a chain of trips to memory and of matrix
+// products, on 60 workgroups.  Against float64 (2-norm, queries and planes N(0, 1)): 1.9e-7, the scalar form 2.5e-7.
 // OutDT: the table's type (bf16: the fp32 value rounded once).
 template <class FT, int W, class OutDT>
 __device__ __forceinline__ void soft_hash_mx32_block(const int l, const int group, const MxUnits& units, const float* __restrict__ q,

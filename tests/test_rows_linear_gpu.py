@@ -94,3 +94,18 @@ def test_an_infinity_stays_in_its_row(dev, K):
     w[3, K - 1] = float("nan")
     got = layer_ops.linear_f32(x[:1].to(dev), w.to(dev)).cpu()[0, 0]
     assert torch.isnan(got[3]) and torch.isfinite(got[torch.arange(9) != 3]).all()
+
+
+@pytest.mark.parametrize("K", [40, 2056, 4096])
+def test_subnormal_operands_and_results_are_kept(dev, K):
+    """One product a row, exact in 32 bits: bfloat16 and 32-bit subnormals go in and come out as they are."""
+    from socket_amd import layer_ops
+    exponents = [(-130, 100), (100, -130), (-133, 20), (-70, -65), (-60, -80), (-133, -10), (-126, 0), (-140, 0)]
+    x, w = torch.zeros(1, 1, K), torch.zeros(len(exponents), K)
+    for i, (p, q) in enumerate(exponents):
+        at = (i * 37 + 5) % K
+        x[0, 0, at], w[i, at] = 1.5 * 2.0 ** p if p > -130 else 2.0 ** p, 2.0 ** q
+    x, w = x.to(torch.bfloat16), w.to(torch.bfloat16)
+    got = layer_ops.linear_f32(x.to(dev), w.to(dev)).double().cpu()
+    want = x.double() @ w.double().t()
+    assert (want[0, 0, [0, 1, 2, 3, 6]] != 0).all() and torch.equal(got, want.float().double())
